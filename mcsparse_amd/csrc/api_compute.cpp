@@ -402,9 +402,8 @@ mcspStatus_t spmv_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
         mcsp::bucketed_products_shape(static_cast<idx_t>(v.n), &bucket_shift)) {
         mcsp::BucketedProducts b;
         mcsp::launch_bucketed_products(h->stream, static_cast<idx_t>(v.m), static_cast<idx_t>(v.n), nnz, v.val, v.ptr,
-                                       v.ind, x->values, t_val, sizeof(T), base, buf + l.csr2csc_ws, &b);
-        return mcsp::launch_bucket_sums<T>(h->stream, static_cast<idx_t>(v.n), nnz, b, static_cast<const T*>(t_val),
-                                           static_cast<T*>(y->values), h_alpha, h_beta)
+                                       v.ind, x->values, sizeof(T), base, buf + l.csr2csc_ws, l.narrow - l.csr2csc_ws, &b);
+        return mcsp::launch_bucket_sums<T>(h->stream, static_cast<idx_t>(v.n), b, static_cast<T*>(y->values), h_alpha, h_beta)
                    ? MCSP_STATUS_SUCCESS
                    : MCSP_STATUS_INTERNAL_ERROR;
     }

@@ -557,8 +557,7 @@ struct ValueOf<8> { typedef uint64_t type; };
 
 // AUX = false: (key, value) pairs, rows_out is not written.  TIMES_X (with FROM_CSR, without AUX): the
 // value that travels is value * x[row of the nonzero], in the floating-point type of VB bytes.
-// short_keys (TIMES_X only, shift <= 16): keys_out is an array of uint16_t that receives the bits of key - bias below
-// `shift`.  bias is subtracted from a key wherever a digit is taken from it (the index base, where that saves a bit).
+// bias is subtracted from a key wherever a digit is taken from it (the index base, where that saves a bit).
 template <int VB>
 struct RealOf { typedef float type; };
 template <>
@@ -569,7 +568,7 @@ __global__ __launch_bounds__(kSortBlock) void radix_scatter_kernel(
     const idx_t* __restrict__ keys_in, const idx_t* __restrict__ rows_in, const void* __restrict__ vals_in_v,
     idx_t* __restrict__ keys_out, idx_t* __restrict__ rows_out, void* __restrict__ vals_out_v, idx_t count,
     uint32_t shift, uint32_t bits, uint32_t tiles, const uint32_t* __restrict__ counters,
-    const idx_t* __restrict__ tile_rows, idx_t base, const void* __restrict__ x_v, bool short_keys, idx_t bias,
+    const idx_t* __restrict__ tile_rows, idx_t base, const void* __restrict__ x_v, idx_t bias,
     uint32_t xcds) {
     static_assert(AUX || VB != 0, "pairs carry a value");
     static_assert(!TIMES_X || (FROM_CSR && !AUX), "products are formed where the rows are worked out");
@@ -788,13 +787,7 @@ __global__ __launch_bounds__(kSortBlock) void radix_scatter_kernel(
             const idx_t k = s_keys[slot];
             const uint32_t d = ((k - bias) >> shift) & mask;
             const uint64_t out = static_cast<uint64_t>(s_dest[d]) + (slot - s_start[d]);
-            if constexpr (TIMES_X) {
-                // short_keys: the last pass of a sort on the top bits keeps only what lies below them, in 16 bits
-                if (short_keys) reinterpret_cast<uint16_t*>(keys_out)[out] = static_cast<uint16_t>((k - bias) & ((1u << shift) - 1u));
-                else keys_out[out] = k;
-            } else {
-                keys_out[out] = k;
-            }
+            keys_out[out] = k;
             if constexpr (AUX) rows_out[out] = s_rows[slot];
             if constexpr (VB != 0) vals_out[out] = s_vals[slot];
         }
@@ -831,30 +824,30 @@ template <int VB>
 void launch_scatter(hipStream_t stream, bool from_csr, uint32_t grid, const idx_t* keys_in, const idx_t* aux_in,
                     const void* vals_in, idx_t* keys_out, idx_t* aux_out, void* vals_out, idx_t count, uint32_t shift,
                     uint32_t bits, uint32_t tiles, const uint32_t* counters, const idx_t* tile_rows, idx_t base,
-                    bool pairs, const void* x, bool short_keys, idx_t bias, uint32_t xcds) {
+                    bool pairs, const void* x, idx_t bias, uint32_t xcds) {
     const void* none = nullptr;
     if constexpr (VB != 0) {
         if (pairs && from_csr) {
             hipLaunchKernelGGL((radix_scatter_kernel<VB, true, false, true>), dim3(grid), dim3(kSortBlock), 0, stream, keys_in,
                                aux_in, vals_in, keys_out, aux_out, vals_out, count, shift, bits, tiles, counters, tile_rows,
-                               base, x, short_keys, bias, xcds);
+                               base, x, bias, xcds);
             return;
         }
         if (pairs) {
             hipLaunchKernelGGL((radix_scatter_kernel<VB, false, false, false>), dim3(grid), dim3(kSortBlock), 0, stream, keys_in,
                                aux_in, vals_in, keys_out, aux_out, vals_out, count, shift, bits, tiles, counters, tile_rows,
-                               base, none, false, bias, xcds);
+                               base, none, bias, xcds);
             return;
         }
     }
     if (from_csr) {
         hipLaunchKernelGGL((radix_scatter_kernel<VB, true, true, false>), dim3(grid), dim3(kSortBlock), 0, stream, keys_in,
                            aux_in, vals_in, keys_out, aux_out, vals_out, count, shift, bits, tiles, counters, tile_rows, base,
-                           none, false, bias, xcds);
+                           none, bias, xcds);
     } else {
         hipLaunchKernelGGL((radix_scatter_kernel<VB, false, true, false>), dim3(grid), dim3(kSortBlock), 0, stream, keys_in,
                            aux_in, vals_in, keys_out, aux_out, vals_out, count, shift, bits, tiles, counters, tile_rows, base,
-                           none, false, bias, xcds);
+                           none, bias, xcds);
     }
 }
 
@@ -868,9 +861,6 @@ struct CsrSource {
     const void* times_x = nullptr;
     // lowest key bit the sort looks at: the keys are ordered by bits [first_bit, first_bit + key_bits)
     uint32_t first_bit = 0;
-    // with times_x, in a sort of one pass: keys_out is an array of uint16_t that receives the key bits below
-    // first_bit (<= 16 of them), which is all that tells the keys of one digit apart
-    bool short_keys = false;
     // subtracted from every key before its digits are taken (the keys themselves travel unchanged)
     idx_t bias = 0;
 };
@@ -905,7 +895,7 @@ void radix_sort_triples(hipStream_t stream, idx_t count, uint32_t key_bits, cons
         auto* launch = value_bytes == 0 ? launch_scatter<0> : value_bytes == 4 ? launch_scatter<4> : launch_scatter<8>;
         launch(stream, from_csr, scatter_grid, keys_in, aux_in, vals_in, k_out, a_out, v_out, count, shift, bits, tiles,
                t.counters, t.tile_rows, csr.base, csr.times_x != nullptr, csr.times_x,
-               csr.short_keys && last && from_csr, csr.bias, xcds);
+               csr.bias, xcds);
         keys_in = k_out;
         aux_in = a_out;
         vals_in = v_out;
@@ -1045,7 +1035,9 @@ size_t csr2csc_workspace_bytes(idx_t /*m*/, idx_t /*n*/, idx_t nnz, size_t value
 }
 
 size_t transposed_products_workspace_bytes(idx_t nnz, size_t value_bytes) {
-    return csr2csc_layout(nnz, value_bytes, true).total;
+    const size_t sort = csr2csc_layout(nnz, value_bytes, true).total;
+    const size_t buckets = bucketed_products_workspace_bytes(nnz, value_bytes);
+    return sort > buckets ? sort : buckets;
 }
 
 // The nonzeros are sorted by column where they lie: the first pass reads col / val in place and
@@ -1107,51 +1099,6 @@ void launch_transposed_products(hipStream_t stream, idx_t m, idx_t n, idx_t nnz,
     radix_sort_triples(stream, nnz, bit_length(n - 1), col, row_ptr, csr_val, sorted_keys, nullptr, products, value_bytes,
                        t, csr);
     launch_coo2csr(stream, nnz, n, sorted_keys, base, col_ptr);
-}
-
-bool bucketed_products_shape(idx_t n, uint32_t* shift) {
-    const uint32_t bits = bit_length(n - 1);  // of the columns without their index base
-    // fewer keys than that: the full sort is two short passes; more: a bucket's sums no longer fit in LDS
-    if (bits < kBucketMinKeyBits || bits > 8 + kBucketMaxShift) return false;
-    *shift = bits - 8;
-    return true;
-}
-
-// One pass of the same sort, for a transposing SpMV that may add the products of a column in any order:
-// (column, value * x[row]) pairs ordered by the top eight bits of the columns (index base taken off) only, that is
-// in up to 256 buckets of 2^shift neighbouring columns, inside a bucket in CSR order.  The sums over a bucket's
-// columns then fit in LDS.  Of a key only its place in the bucket is written, as 16 bits: a quarter fewer
-// bytes for this pass to write and the sums to read.  workspace as for launch_transposed_products.
-void launch_bucketed_products(hipStream_t stream, idx_t m, idx_t n, idx_t nnz, const void* csr_val, const idx_t* row_ptr,
-                              const idx_t* col, const void* x, void* products, size_t value_bytes, idx_t base,
-                              void* workspace, BucketedProducts* out) {
-    uint32_t shift = 0;
-    if (m == 0 || nnz == 0 || !bucketed_products_shape(n, &shift)) return;
-    const Csr2CscLayout l = csr2csc_layout(nnz, value_bytes, true);
-    char* w = static_cast<char*>(workspace);
-    idx_t* keys = reinterpret_cast<idx_t*>(w + l.sorted_keys);  // room for 32-bit keys, used for 16-bit ones
-    SortScratch t;  // one pass writes the outputs directly: no alternating sets
-    t.keys[0] = t.keys[1] = nullptr;
-    t.aux[0] = t.aux[1] = nullptr;
-    t.vals[0] = t.vals[1] = nullptr;
-    t.counters = reinterpret_cast<uint32_t*>(w + l.counters);
-    t.scan_ws = reinterpret_cast<uint32_t*>(w + l.scan_ws);
-    t.tile_rows = reinterpret_cast<idx_t*>(w + l.tile_rows);
-    CsrSource csr;
-    csr.rows = m;
-    csr.base = base;
-    csr.times_x = x;
-    csr.first_bit = shift;
-    csr.short_keys = true;
-    csr.bias = base;
-    radix_sort_triples(stream, nnz, 8, col, row_ptr, csr_val, keys, nullptr, products, value_bytes, t, csr);
-    out->keys = reinterpret_cast<const uint16_t*>(keys);
-    out->starts = t.counters;  // after the scan, counters[digit * tiles] is where the digit's keys begin
-    out->stride = sort_tiles(nnz);
-    out->shift = shift;
-    out->buckets = static_cast<uint32_t>((n - 1) >> shift) + 1;
-    out->spare = w + l.keys_a;  // the sets the passes of a full sort alternate between
-    out->spare_bytes = l.counters - l.keys_a;
 }
 
 // Scratch of launch_sort_by_column_band: the counters of one pass, their scan, the row starts per tile.

@@ -477,31 +477,35 @@ void launch_transposed_products(hipStream_t stream, idx_t m, idx_t n, idx_t nnz,
                                 const idx_t* col, const void* x, void* products, idx_t* col_ptr, size_t value_bytes,
                                 idx_t base, void* workspace);
 
-// The same products in up to 256 buckets of 2^shift neighbouring columns (index base taken off: bucket b
-// holds columns [b << shift, (b + 1) << shift)), bucket b starting at starts[b * stride] and ending where
-// the next begins (the last at nnz); inside a bucket the pairs are in CSR order, not sorted, and keys[]
-// holds a column's low `shift` bits, its place in the bucket.  Both arrays may be read up to the next even index past nnz.  One pass over the nonzeros instead of the three of a
-// full sort: for callers that then add the products of a column in any order.  The shape function says
-// whether the shape allows it (more than 2^14 and at most 2^22 columns: a bucket's sums must fit in LDS as
-// doubles).
+// The same products ordered by bucket of 2^shift neighbouring columns (index base taken off: bucket b holds columns
+// [b << shift, (b + 1) << shift), at most 256 of them), but only inside tiles of the CSR order: table[b * tiles + t] says
+// where in tile t, which begins at place t * tile_places, the run of bucket b lies (place | length << 16,
+// partition_device.h).  Runs begin at multiples of kBucketRunPad and are padded with products of 0 to such a length.
+// keys[] holds a column's place in its bucket (in its low `shift` bits).  One pass over the nonzeros instead of the three of a full sort, for
+// callers that then add the products of a column in any order.  The shape function says whether the shape allows it
+// (more than 2^14 and at most 2^22 columns: a bucket's sums must fit in LDS as doubles).
 constexpr uint32_t kBucketMinKeyBits = 15;
 constexpr uint32_t kBucketMaxShift = 14;
+constexpr uint32_t kBucketTileMin = 2048;  // nonzeros of the smallest tiles
+constexpr uint32_t kBucketRunPad = 4;
 struct BucketedProducts {
     const uint16_t* keys = nullptr;
-    const uint32_t* starts = nullptr;
-    uint32_t stride = 0, shift = 0, buckets = 0;
+    const void* products = nullptr;
+    const uint32_t* table = nullptr;
+    uint32_t* totals = nullptr;  // room for 256 words
+    uint32_t tiles = 0, tile_places = 0, shift = 0, buckets = 0;
     void* spare = nullptr;  // part of the workspace the pass did not use, for the sums of buckets that are split
     size_t spare_bytes = 0;
 };
 bool bucketed_products_shape(idx_t n, uint32_t* shift);
+size_t bucketed_products_workspace_bytes(idx_t nnz, size_t value_bytes);
 void launch_bucketed_products(hipStream_t stream, idx_t m, idx_t n, idx_t nnz, const void* csr_val, const idx_t* row_ptr,
-                              const idx_t* col, const void* x, void* products, size_t value_bytes, idx_t base,
-                              void* workspace, BucketedProducts* out);
+                              const idx_t* col, const void* x, size_t value_bytes, idx_t base, void* workspace,
+                              size_t workspace_bytes, BucketedProducts* out);
 // y[c] = alpha * (sum of the products of column c) + beta * y[c] for all n columns, from such buckets;
 // the sums are formed in LDS in the order the wavefronts reach the products.
 template <typename T>
-bool launch_bucket_sums(hipStream_t stream, idx_t n, idx_t nnz, const BucketedProducts& b, const T* products, T* y,
-                        T alpha, T beta);
+bool launch_bucket_sums(hipStream_t stream, idx_t n, const BucketedProducts& b, T* y, T alpha, T beta);
 
 // y = alpha * A^T x + beta * y for an m x n matrix with at most 2^14 columns and many nonzeros per
 // column, without sorting anything: shares of the nonzeros are summed into copies of y in LDS, the copies

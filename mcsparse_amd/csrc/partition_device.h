@@ -1,0 +1,371 @@
+// Building blocks of the kernels that partition entries by the bits of a key and read the parts back: partition.hip,
+// spmv_transposed.hip.
+#ifndef MCSPARSE_AMD_PARTITION_DEVICE_H_
+#define MCSPARSE_AMD_PARTITION_DEVICE_H_
+
+#include "device_util.h"
+#include "internal.h"
+
+namespace mcsp {
+namespace partition_detail {
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// ---- one wavefront ---------------------------------------------------------------------------------------------
+// Inclusive sum over the 64 lanes: four shifted adds inside each row of 16 lanes, then the last lane of rows 0 and 2
+// is added to rows 1 and 3, then lane 31 to rows 2 and 3.
+__device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t v) {
+    constexpr int kRowShr = 0x110, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+    int x = static_cast<int>(v);
+    x += __builtin_amdgcn_update_dpp(0, x, kRowShr + 1, 0xF, 0xF, false);
+    x += __builtin_amdgcn_update_dpp(0, x, kRowShr + 2, 0xF, 0xF, false);
+    x += __builtin_amdgcn_update_dpp(0, x, kRowShr + 4, 0xF, 0xF, false);
+    x += __builtin_amdgcn_update_dpp(0, x, kRowShr + 8, 0xF, 0xF, false);
+    x += __builtin_amdgcn_update_dpp(0, x, kRowBcast15, 0xA, 0xF, false);
+    x += __builtin_amdgcn_update_dpp(0, x, kRowBcast31, 0xC, 0xF, false);
+    return static_cast<uint32_t>(x);
+}
+
+// How many of the ascending values a[0 .. n) are <= g, with 64 probes per round.  Every lane of the wavefront must
+// call this; all lanes return the same value.
+__device__ __forceinline__ uint32_t wave_count_up_to(const uint32_t* __restrict__ a, uint32_t n, uint32_t base, uint32_t g) {
+    uint64_t lo = 0, hi = n;
+    const unsigned lane = lane_id();
+    while (lo < hi) {
+        const uint64_t step = (hi - lo + kWave - 1) / kWave;
+        const uint64_t probe = lo + lane * step;
+        const bool pred = probe < hi && a[probe] - base <= g;
+        const unsigned count = __popcll(__ballot(pred));
+        if (count == 0) {
+            hi = lo;
+        } else {
+            const uint64_t new_hi = lo + static_cast<uint64_t>(count) * step;
+            lo = lo + static_cast<uint64_t>(count - 1) * step + 1;
+            hi = new_hi < hi ? new_hi : hi;
+        }
+    }
+    return static_cast<uint32_t>(lo);
+}
+
+// lanes below this one among the bits of a 64-bit word
+__device__ __forceinline__ uint32_t bits_below_lane(uint32_t lo, uint32_t hi) {
+    return __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+}
+
+// Clears, in the word (lo, hi) of candidate lanes, those whose digit differs from this lane's: per bit of the digit
+// the lanes that voted as this lane did stay.  a & ~(b ^ c) is one v_bitop3 each for the low and the high half, so a
+// bit costs four instructions.
+template <int MAX_BITS>
+__device__ __forceinline__ void keep_equal_digits(uint32_t d, uint32_t bits, uint32_t& lo, uint32_t& hi) {
+#pragma unroll
+    for (uint32_t b = 0; b < MAX_BITS; ++b) {
+        if (b < bits) {
+            const int own = __builtin_amdgcn_sbfe(static_cast<int>(d), b, 1);
+            const uint64_t vote = __ballot(own < 0);
+            lo = __builtin_amdgcn_bitop3_b32(lo, static_cast<uint32_t>(vote), static_cast<uint32_t>(own), 0x90);
+            hi = __builtin_amdgcn_bitop3_b32(hi, static_cast<uint32_t>(vote >> 32), static_cast<uint32_t>(own), 0x90);
+        }
+    }
+}
+
+// ---- one workgroup ---------------------------------------------------------------------------------------------
+// Exclusive sum over the threads of a workgroup; s_wave: THREADS / 64 words.  Holds one barrier; s_wave may be reused
+// after the caller's next barrier.
+template <int THREADS>
+__device__ __forceinline__ uint32_t block_exclusive_sum(uint32_t v, uint32_t* s_wave, uint32_t* total = nullptr) {
+    const uint32_t wave = threadIdx.x / kWave;
+    const uint32_t upto = wave_inclusive_sum(v);
+    if (threadIdx.x % kWave == kWave - 1) s_wave[wave] = upto;
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < THREADS / kWave; ++w) {
+        const uint32_t s = s_wave[w];
+        if (w < wave) before += s;
+        all += s;
+    }
+    if (total != nullptr) *total = all;
+    return before + upto - v;
+}
+
+// Position inside the tile of a thread's i-th entry: wavefronts own consecutive slabs of `rounds` times 64 entries
+// and the lanes are interleaved inside a slab, so (wavefront, i, lane) order is the order of the entries.
+__device__ __forceinline__ uint32_t slab_place(uint32_t rounds, uint32_t i) {
+    return (threadIdx.x / kWave * rounds + i) * kWave + threadIdx.x % kWave;
+}
+// slab_place(rounds, i) < count, as one comparison with a scalar.
+__device__ __forceinline__ bool in_slab(uint32_t rounds, uint32_t i, uint32_t count) {
+    return static_cast<int>(slab_place(rounds, 0)) < static_cast<int>(count) - static_cast<int>(i * kWave);
+}
+
+// A value the compiler cannot trace back: what is worked out from it again costs an instruction and not a register held
+// from the first time on.
+__device__ __forceinline__ void forget(uint32_t& v) { asm volatile("" : "+v"(v)); }
+
+// Reads of a tile of an array through a buffer resource that ends with the tile: places past the end read as zero
+// without a test, and a thread's items differ by constants only (no register per item).
+struct TileReader {
+    __amdgpu_buffer_rsrc_t tile;
+    __device__ __forceinline__ TileReader(const void* first, uint32_t bytes) {
+        constexpr int kRawDwords = 0x00027000;  // no stride, untyped
+        tile = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(first), 0, static_cast<int>(bytes), kRawDwords);
+    }
+    template <typename W>
+    __device__ __forceinline__ W read(uint32_t place, int constant_places) const {
+        constexpr int kNonTemporal = 2;
+        if constexpr (sizeof(W) == 4) {
+            return __builtin_amdgcn_raw_buffer_load_b32(tile, static_cast<int>(place * 4), constant_places * 4, kNonTemporal);
+        } else {
+            typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+            return __builtin_bit_cast(W, static_cast<u32x2>(__builtin_amdgcn_raw_buffer_load_b64(
+                                             tile, static_cast<int>(place * 8), constant_places * 8, kNonTemporal)));
+        }
+    }
+};
+
+// Stable rank of every entry among the entries of its wavefront with the same digit, two 16-bit ranks to a word;
+// s_cnt[wave][digit] ends as the wavefront's count of the digit (zero on entry).  digit(i) is the digit of entry i;
+// entries from `count` on are left out.
+template <int ITEMS, int MAX_BITS, int WAVES, typename Digit>
+__device__ __forceinline__ void rank_entries(uint32_t count, uint32_t rounds, uint32_t bits, uint16_t* s_cnt,
+                                             uint32_t (&rank)[(ITEMS + 1) / 2], Digit digit) {
+    uint16_t* mine = s_cnt + (threadIdx.x / kWave << MAX_BITS);
+    const bool whole = count == static_cast<uint32_t>(WAVES) * rounds * kWave;  // the same for the workgroup
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        uint32_t r = 0;
+        if (static_cast<uint32_t>(i) < rounds) {
+            const uint32_t d = digit(i);
+            const bool live = whole || in_slab(rounds, i, count);
+            const uint64_t candidates = __ballot(live);
+            uint32_t lo = static_cast<uint32_t>(candidates), hi = static_cast<uint32_t>(candidates >> 32);
+            keep_equal_digits<MAX_BITS>(d, bits, lo, hi);
+            const uint32_t below = bits_below_lane(lo, hi);
+            if (live) {
+                // Every peer reads the counter, then the lowest one adds the round's count.  The LDS operations of a
+                // wavefront complete in program order; relaxed atomics keep the compiler from moving or merging them.
+                const uint32_t before = __hip_atomic_load(mine + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+                r = before + below;
+                if (below == 0) {
+                    __hip_atomic_store(mine + d, static_cast<uint16_t>(before + __popc(lo) + __popc(hi)), __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_WAVEFRONT);
+                }
+            }
+        }
+        if (i % 2 == 0) rank[i / 2] = r;
+        else rank[i / 2] |= r << 16;
+    }
+}
+
+// Ranks in no particular order, for callers that do not care how the entries of a digit follow each other: one LDS
+// counter per digit (zero on entry) hands them out.  A quarter of the instructions of rank_entries.  Entries sorted by
+// key (a long row) bring whole wavefronts of one digit, whose adds LDS would take one after the other: one lane adds
+// for all of them.
+template <int ITEMS, typename Digit>
+__device__ __forceinline__ void rank_entries_unordered(uint32_t count, uint32_t* s_count, uint32_t (&rank)[(ITEMS + 1) / 2],
+                                                       Digit digit) {
+    const uint32_t lane = threadIdx.x % kWave;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const uint32_t d = digit(i);
+        const bool live = in_slab(ITEMS, i, count);
+        const uint32_t lead = __builtin_amdgcn_readfirstlane(d);
+        uint32_t r = 0;
+        if (__all(live && d == lead)) {
+            if (lane == 0) r = atomicAdd(&s_count[lead], static_cast<uint32_t>(kWave));
+            r = __builtin_amdgcn_readfirstlane(r) + lane;
+        } else if (live) {
+            r = atomicAdd(&s_count[d], 1u);
+        }
+        if (i % 2 == 0) rank[i / 2] = r;
+        else rank[i / 2] |= r << 16;
+    }
+}
+
+// After rank_entries and a barrier: turns the counts of the wavefronts into the first place of each (wavefront, digit)
+// in the ordered tile.  per_digit(digit, first place, count) is called once for every digit below 2^bits.  Ends with
+// a barrier.
+template <int THREADS, int MAX_BITS, typename PerDigit>
+__device__ __forceinline__ void place_digits(uint32_t bits, uint16_t* s_cnt, uint32_t* s_wave, PerDigit per_digit) {
+    constexpr int kWaves = THREADS / kWave;
+    constexpr int kDigits = (1 << MAX_BITS) > THREADS ? (1 << MAX_BITS) / THREADS : 1;  // neighbouring digits per thread
+    const uint32_t first = threadIdx.x * kDigits;
+    uint32_t total[kDigits], sum = 0;
+#pragma unroll
+    for (int k = 0; k < kDigits; ++k) {
+        total[k] = 0;
+        if (first + k < (1u << MAX_BITS)) {
+            uint32_t c[kWaves];
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) c[w] = s_cnt[(w << MAX_BITS) + first + k];
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) {
+                s_cnt[(w << MAX_BITS) + first + k] = static_cast<uint16_t>(total[k]);
+                total[k] += c[w];
+            }
+        }
+        sum += total[k];
+    }
+    uint32_t at = block_exclusive_sum<THREADS>(sum, s_wave);
+#pragma unroll
+    for (int k = 0; k < kDigits; ++k) {
+        if (first + k < (1u << bits)) {
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) s_cnt[(w << MAX_BITS) + first + k] += static_cast<uint16_t>(at);
+            per_digit(first + k, at, total[k]);
+        }
+        at += total[k];
+    }
+    __syncthreads();
+}
+
+// ---- runs of tiles ---------------------------------------------------------------------------------------------
+// The entries of one bucket, in order, are the runs that its digit has in tiles 0, 1, ...: run t is `begins[t]` ..
+// of them (ascending; the next run's begin, or `all`, ends it) and lies at place start(table[t]) of tile t.  A table
+// word holds the run's place in the tile and its length.
+__device__ __forceinline__ uint32_t table_word(uint32_t place, uint32_t length) { return place | length << 16; }
+__device__ __forceinline__ uint32_t run_place(uint32_t word) { return word & 0xffffu; }
+__device__ __forceinline__ uint32_t run_length(uint32_t word) { return word >> 16; }
+
+// Where the entries q0 .. q0 + count - 1 of a bucket come from.  The runs they touch are listed in LDS, each as the
+// difference between an entry's place in memory and its place in the chunk, and a bit marks where a run begins; the
+// run of an entry is then a count of bits.
+template <int CHUNK>
+struct RunMap {
+    unsigned long long begins[CHUNK / kWave];
+    uint32_t before[CHUNK / kWave];  // runs that begin before each 64 entries, less one, the first entry's own included
+    uint32_t wave[16];
+    uint32_t first_run;
+};
+
+template <int THREADS, int CHUNK>
+__device__ __forceinline__ void map_runs(const uint32_t* __restrict__ run_begins, const uint32_t* __restrict__ table,
+                                         uint32_t tiles, uint32_t all, uint32_t q0, uint32_t count, uint32_t tile_size,
+                                         uint32_t source, RunMap<CHUNK>& s, uint32_t* s_delta) {
+    constexpr uint32_t kWords = CHUNK / kWave;
+    const uint32_t tid = threadIdx.x;
+    for (uint32_t w = tid; w < kWords; w += THREADS) s.begins[w] = 0;
+    if (tid < kWave) {  // whole wavefront
+        const uint32_t upto = q0 == 0 && tiles <= THREADS ? 1 : wave_count_up_to(run_begins, tiles, 0, q0);
+        if (tid == 0) s.first_run = upto != 0 ? upto - 1 : 0;
+    }
+    __syncthreads();
+    const uint32_t q1 = q0 + count;
+    uint32_t listed = 0;
+    for (uint32_t t0 = s.first_run; t0 < tiles; t0 += THREADS) {
+        const uint32_t t = t0 + tid;
+        uint32_t begin = all, end = all, word = 0;
+        if (t < tiles) {
+            begin = run_begins[t];
+            end = t + 1 < tiles ? run_begins[t + 1] : all;
+            word = table[t];
+        }
+        const uint32_t from = begin > q0 ? begin : q0;
+        const uint32_t to = end < q1 ? end : q1;
+        const bool used = from < to;
+        uint32_t fresh = 0;
+        const uint32_t at = listed + block_exclusive_sum<THREADS>(used ? 1u : 0u, s.wave, &fresh);
+        if (used) {
+            const uint32_t place = from - q0;
+            if (at < static_cast<uint32_t>(CHUNK)) s_delta[at] = source + t * tile_size + run_place(word) + (from - begin) - place;
+            atomicOr(&s.begins[place / kWave], 1ull << (place % kWave));
+        }
+        listed += fresh;
+        // past the chunk's end?  the last thread's run is the furthest
+        const bool more = __syncthreads_or(tid == THREADS - 1 && end < q1);
+        if (!more) break;  // whole workgroup
+    }
+    if (tid < kWave) {
+        uint32_t carried = 0;
+        for (uint32_t w0 = 0; w0 < kWords; w0 += kWave) {
+            const uint32_t w = w0 + tid;
+            const unsigned long long word = w < kWords ? s.begins[w] : 0;
+            const uint32_t c = __popcll(word);
+            const uint32_t upto = wave_inclusive_sum(c);
+            if (w < kWords) s.before[w] = carried + upto - c + static_cast<uint32_t>(word & 1u) - 1;
+            carried += __shfl(upto, kWave - 1, kWave);
+        }
+    }
+    __syncthreads();
+}
+
+// Place in memory of entry w * 64 + lane of the chunk.
+template <int CHUNK>
+__device__ __forceinline__ uint32_t mapped_place(const RunMap<CHUNK>& s, const uint32_t* s_delta, uint32_t w) {
+    const unsigned long long later = s.begins[w] >> 1;  // runs that begin at or before a lane, after the first lane
+    const uint32_t run = s.before[w] + bits_below_lane(static_cast<uint32_t>(later), static_cast<uint32_t>(later >> 32));
+    return s_delta[run] + w * kWave + threadIdx.x % kWave;
+}
+
+// ---- stores of an ordered tile ---------------------------------------------------------------------------------
+// Entries go to LDS in their new order and out as 16-byte pieces, `PLACES` of them (the tile and what its runs are
+// padded with).  Every one of these begins and ends with the workgroup through with the buffer.
+template <int ITEMS, int THREADS, uint32_t PLACES, typename Key>
+__device__ __forceinline__ void store_keys(uint32_t* s_buf, uint32_t count, const uint32_t (&dest)[(ITEMS + 1) / 2], Key* out,
+                                           const uint32_t (&key)[ITEMS], uint32_t mask) {
+    Key* s = reinterpret_cast<Key*>(s_buf);
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        if (in_slab(ITEMS, i, count)) s[(dest[i / 2] >> (i % 2 * 16)) & 0xffffu] = static_cast<Key>(key[i] & mask);
+    }
+    __syncthreads();
+    static_assert(PLACES * sizeof(Key) % 16 == 0, "whole pieces");
+    for (uint32_t v = threadIdx.x; v < PLACES * sizeof(Key) / 16; v += THREADS)
+        __builtin_nontemporal_store(reinterpret_cast<const u32x4*>(s_buf)[v], reinterpret_cast<u32x4*>(out) + v);
+    __syncthreads();
+}
+
+template <int ITEMS, int THREADS, uint32_t PLACES>
+__device__ __forceinline__ void store_words(uint32_t* s_buf, uint32_t count, const uint32_t (&dest)[(ITEMS + 1) / 2],
+                                            uint32_t* out, const uint32_t (&word)[ITEMS]) {
+    constexpr uint32_t kPieces = PLACES / 4;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        if (in_slab(ITEMS, i, count)) s_buf[(dest[i / 2] >> (i % 2 * 16)) & 0xffffu] = word[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < (kPieces + THREADS - 1) / THREADS; ++k) {
+        const uint32_t v = k * THREADS + threadIdx.x;
+        if (kPieces % THREADS == 0 || v < kPieces)
+            __builtin_nontemporal_store(reinterpret_cast<const u32x4*>(s_buf)[v], reinterpret_cast<u32x4*>(out) + v);
+    }
+    __syncthreads();
+}
+
+// 64-bit values go through the buffer in two halves.
+template <int ITEMS, int THREADS, uint32_t PLACES>
+__device__ __forceinline__ void store_words(uint32_t* s_buf, uint32_t count, const uint32_t (&dest)[(ITEMS + 1) / 2],
+                                            uint64_t* out, const uint64_t (&word)[ITEMS]) {
+    constexpr uint32_t kPieces = PLACES / 4;
+    constexpr uint32_t kMine = (kPieces + THREADS - 1) / THREADS;
+    u32x4 low[kMine];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            if (in_slab(ITEMS, i, count))
+                s_buf[(dest[i / 2] >> (i % 2 * 16)) & 0xffffu] = static_cast<uint32_t>(word[i] >> (32 * half));
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t k = 0; k < kMine; ++k) {
+            const uint32_t v = k * THREADS + threadIdx.x;
+            if (kPieces % THREADS != 0 && v >= kPieces) continue;
+            const u32x4 got = reinterpret_cast<const u32x4*>(s_buf)[v];
+            if (half == 0) {
+                low[k] = got;
+            } else {
+                const u32x4 a = {low[k].x, got.x, low[k].y, got.y}, b = {low[k].z, got.z, low[k].w, got.w};
+                __builtin_nontemporal_store(a, reinterpret_cast<u32x4*>(out) + 2 * v);
+                __builtin_nontemporal_store(b, reinterpret_cast<u32x4*>(out) + 2 * v + 1);
+            }
+        }
+        __syncthreads();
+    }
+}
+
+}  // namespace partition_detail
+}  // namespace mcsp
+
+#endif  // MCSPARSE_AMD_PARTITION_DEVICE_H_

@@ -1,0 +1,49 @@
+"""GPU parity of what is built on the partition of tiles by key bits (csrc/partition.hip), at the sizes where it can go
+wrong: entry counts around a tile, both tile sizes, keys concentrated in a few runs, empty rows.  The transposing
+mcsparseSpMV without a preprocess call is compared exactly (integer-valued operands make any order of summation exact)."""
+import numpy as np
+import pytest
+
+from mcsparse_amd import api
+from mcsparse_amd import workloads as wl
+
+from gpu_util import run_spmv
+
+pytestmark = pytest.mark.gpu
+
+LARGE_FROM = 512 * 8192  # entries up to which the tiles hold 2048 entries, beyond 8192
+
+
+def matrix(kind, m, n, nnz, dtype, seed):
+    """A CSR matrix with exactly nnz nonzeros: columns drawn from all of them, from a band around the diagonal, or mostly
+    from a few; a fifth of the rows empty in the first case."""
+    rng = np.random.default_rng(seed)
+    weights = rng.random(m) * (rng.random(m) > 0.2 if kind == "uniform" else 1.0)
+    cuts = np.concatenate([[0], np.round(np.cumsum(weights) / weights.sum() * nnz)]).astype(np.int64)
+    cuts[-1] = nnz
+    rows = np.repeat(np.arange(m), np.diff(cuts))
+    if kind == "uniform":
+        col = rng.integers(0, n, nnz)
+    elif kind == "band":
+        col = np.clip(rows * n // m + rng.integers(-20, 21, nnz), 0, n - 1)
+    else:
+        col = np.where(rng.random(nnz) < 0.7, rng.integers(0, 5, nnz) * (n // 7), rng.integers(0, n, nnz))
+    col = col[np.lexsort((col, rows))]
+    return wl.Csr(m, n, cuts, col, rng.integers(-3, 4, nnz).astype(dtype), 0)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("kind,m,n,nnz", [
+    ("uniform", 50, 40000, 1), ("uniform", 300, 40000, 2047), ("uniform", 300, 40000, 2048), ("uniform", 300, 40000, 2049),
+    ("uniform", 30000, 20000, 300001), ("band", 50000, 70000, 700000), ("few", 60000, 200000, 900000),
+    ("uniform", 400000, 1 << 22, LARGE_FROM), ("uniform", 400000, 300000, LARGE_FROM + 1),
+    ("band", 200000, 150000, LARGE_FROM + 8191), ("few", 150000, 4000000, LARGE_FROM + 8192 * 30),
+])
+def test_transposed_product_exact(torch_gpu, handle, dtype, kind, m, n, nnz):
+    a = matrix(kind, m, n, nnz, dtype, seed=nnz)
+    rng = np.random.default_rng(3)
+    x, y = rng.integers(-4, 5, m).astype(dtype), rng.integers(-8, 9, n).astype(dtype)
+    want = 2 * (a.to_scipy().T.astype(np.float64) @ x.astype(np.float64)) - 3 * y
+    st, got, _ = run_spmv(torch_gpu, handle, a, x, y, 2.0, -3.0, op=api.OP_T)
+    assert st == api.STATUS_SUCCESS
+    assert np.array_equal(got.astype(np.float64), want)
