@@ -1030,8 +1030,10 @@ void launch_coo2csr(hipStream_t stream, idx_t nnz, idx_t m, const idx_t* coo_row
     }
 }
 
-size_t csr2csc_workspace_bytes(idx_t /*m*/, idx_t /*n*/, idx_t nnz, size_t value_bytes) {
-    return csr2csc_layout(nnz, value_bytes).total;
+size_t csr2csc_workspace_bytes(idx_t /*m*/, idx_t n, idx_t nnz, size_t value_bytes) {
+    const size_t passes = csr2csc_layout(nnz, value_bytes).total;
+    const size_t sort = n != 0 ? partition_sort_workspace_bytes(nnz, bit_length(n - 1), value_bytes) : 0;
+    return passes > sort ? passes : sort;
 }
 
 size_t transposed_products_workspace_bytes(idx_t nnz, size_t value_bytes) {
@@ -1046,6 +1048,21 @@ void launch_csr2csc(hipStream_t stream, idx_t m, idx_t n, idx_t nnz, const void*
                     const idx_t* col, void* csc_val, idx_t* row_ind, idx_t* col_ptr, size_t value_bytes, idx_t base,
                     void* workspace) {
     if (m == 0 || n == 0 || nnz == 0) return;
+    if (partition_sort_usable(nnz, bit_length(n - 1))) {
+        PartitionSortArgs a;
+        a.keys_in = col;
+        a.csr_rows = m;
+        a.row_ptr = row_ptr;
+        a.vals_in = csr_val;
+        a.base = base;
+        a.key_bias = base;
+        a.aux_out = row_ind;
+        a.vals_out = csc_val;
+        a.key_ptr = col_ptr;
+        a.key_count = n;
+        launch_partition_sort(stream, nnz, bit_length(n - 1), a, value_bytes, workspace);
+        return;
+    }
     const Csr2CscLayout l = csr2csc_layout(nnz, value_bytes);
     char* w = static_cast<char*>(workspace);
     idx_t* sorted_keys = reinterpret_cast<idx_t*>(w + l.sorted_keys);

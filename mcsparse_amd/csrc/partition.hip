@@ -1,9 +1,22 @@
-// Partition of entries by the top bits of a key, tile by tile, for gfx950.
+// Partition of entries by bits of a key, tile by tile, and the stable sort by key made of it, for gfx950.
 //
 // partition_kernel orders the entries of a tile by a digit of their keys, inside the tile only, and writes the tile back
 // as one linear stream, with a table of where each digit's run begins.  Against a radix pass that writes every entry
 // straight to its bucket (src/mcprim/device_radix_sort.hpp:90-309 of the reference) it needs no counting pass and makes
 // no scattered store; the runs are put together by whoever reads them next.
+//
+// The sort orders (key, index, value) triples by a key of up to 24 bits: csr2csc
+// (src/kernels/conversion/mcsp_csr2csc.cpp:97-98 of the reference) and the index sorts.  A stable sort has one result,
+// so how it is reached is free.  What bounds it is the bytes its passes move; an LSD sort moves every triple whole, keys
+// included, once per 8 bits and reads the keys once more per pass.  Here the most significant bits go first:
+//   1. partition_kernel, by the top d1 bits;
+//   2. where more than 2^11 buckets are wanted, repartition_kernel: the same on the tiles of each bucket, whose entries
+//      it gathers from the runs of step 1, by the next d2 bits;
+//   3. bucket_sort_kernel gathers a bucket, which fits LDS, orders it by the last d3 <= 8 bits and writes it where it
+//      belongs, a linear stream again.  Where the keys begin (col_ptr of a CSC) falls out of its digit counts.
+// A key loses the bits that its place already tells: at most 16 of them travel to step 2 and 8 to step 3.
+// A bucket that does not fit LDS (popular keys) is cut into chunks by the oversize_* kernels, which find nothing to do
+// elsewhere.
 #include "partition_device.h"
 
 namespace mcsp {
@@ -263,6 +276,507 @@ __global__ __launch_bounds__(kRowStartsBlock) void partition_row_starts_kernel(c
     if (threadIdx.x % kWave == 0) tile_rows[t] = starts;
 }
 
+// run_begins[d * tiles + t] = entries of digit d in the tiles before t; totals[d] = all of them.  A workgroup per digit.
+constexpr int kScanBlock = 256;
+constexpr int kScanItems = 8;
+__global__ __launch_bounds__(kScanBlock) void run_begins_kernel(uint32_t tiles, const uint32_t* __restrict__ table,
+                                                                uint32_t* __restrict__ run_begins,
+                                                                uint32_t* __restrict__ totals) {
+    __shared__ uint32_t s_wave[kScanBlock / kWave];
+    const uint32_t* in = table + static_cast<uint64_t>(blockIdx.x) * tiles;
+    uint32_t* out = run_begins + static_cast<uint64_t>(blockIdx.x) * tiles;
+    uint32_t carried = 0;
+    for (uint32_t t0 = 0; t0 < tiles; t0 += kScanBlock * kScanItems) {
+        uint32_t n[kScanItems], sum = 0;
+#pragma unroll
+        for (int k = 0; k < kScanItems; ++k) {
+            const uint32_t t = t0 + threadIdx.x * kScanItems + k;
+            n[k] = in[t < tiles ? t : tiles - 1];
+        }
+#pragma unroll
+        for (int k = 0; k < kScanItems; ++k) {
+            n[k] = t0 + threadIdx.x * kScanItems + k < tiles ? run_length(n[k]) : 0;
+            sum += n[k];
+        }
+        uint32_t all = 0;
+        uint32_t at = carried + block_exclusive_sum<kScanBlock>(sum, s_wave, &all);
+#pragma unroll
+        for (int k = 0; k < kScanItems; ++k) {
+            const uint32_t t = t0 + threadIdx.x * kScanItems + k;
+            if (t < tiles) out[t] = at;
+            at += n[k];
+        }
+        carried += all;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) totals[blockIdx.x] = carried;
+}
+
+
+
+// ---- step 2 ----------------------------------------------------------------------------------------------------
+// What the kernels after step 1 read of it and of each other.  One level: the buckets of step 1 are sorted as they are.
+// Two levels: tile t of bucket b (its entries [t * kSecondTile, ...)) is tile number tile_first[b] + t.
+struct SortTables {
+    // step 1: [digit][tile]
+    const uint32_t* table1;
+    const uint32_t* begins1;
+    const uint32_t* totals1;
+    uint32_t tiles1, places1;
+    // step 2: [bucket][digit][tile of the bucket]
+    uint32_t* table2;
+    uint32_t* begins2;
+    uint32_t* bucket_first;  // entries before each bucket of step 1, 2^d1 + 1 of them
+    uint32_t* tile_first;    // tiles before each bucket of step 1, 2^d1 + 1 of them
+    uint32_t* tile_map;      // the order in which the tiles are taken: bucket << 24 | tile of the bucket
+    // both: entries before each bucket of step 3, 2^(d1 + d2) + 1 of them
+    uint32_t* sub_first;
+    // buckets of step 3 that do not fit LDS
+    unsigned long long* oversize_count;  // buckets | chunks << 32
+    uint2* oversize;                     // {bucket, chunks before}
+    uint32_t* oversize_begins;           // [chunk][digit]
+    uint32_t d1, d2, d3, count;
+};
+
+constexpr uint32_t kSecondTile = 8192;
+constexpr int kSecondThreads = 512, kSecondItems = 16;
+static_assert(kSecondThreads * kSecondItems == kSecondTile, "a tile per workgroup");
+constexpr int kBucketThreads = 512, kBucketItems = 12;
+constexpr uint32_t kBucketRoom = kBucketThreads * kBucketItems;  // entries of the largest bucket that is sorted in LDS
+constexpr uint32_t kMaxD3 = 8;
+constexpr uint32_t kOversizeChunk = kBucketRoom;
+
+__device__ __forceinline__ void note_oversize(const SortTables& t, uint32_t bucket, uint32_t entries) {
+    if (entries <= kBucketRoom) return;
+    const unsigned long long chunks = (entries + kOversizeChunk - 1) / kOversizeChunk;
+    const unsigned long long at = atomicAdd(t.oversize_count, chunks << 32 | 1u);  // both at once: chunks ascend with the place
+    t.oversize[static_cast<uint32_t>(at)] = make_uint2(bucket, static_cast<uint32_t>(at >> 32));
+}
+
+// Exclusive sums over the buckets of step 1 (at most 2^11), in one workgroup: of entries, and (two levels) of tiles.
+// One level: the buckets of step 1 are those of step 3.
+constexpr int kPlanBlock = 1024;
+__global__ __launch_bounds__(kPlanBlock) void sort_plan_kernel(SortTables t) {
+    __shared__ uint32_t s_wave[kPlanBlock / kWave];
+    if (threadIdx.x == 0) {
+        *t.oversize_count = 0;
+        __threadfence();  // before the adds of this workgroup's other threads
+    }
+    const uint32_t buckets = 1u << t.d1;
+    uint32_t* first = t.d2 != 0 ? t.bucket_first : t.sub_first;
+    uint32_t entries_before = 0, tiles_before = 0;
+    __syncthreads();
+    for (uint32_t b0 = 0; b0 < buckets; b0 += kPlanBlock) {
+        const uint32_t b = b0 + threadIdx.x;
+        const uint32_t n = b < buckets ? t.totals1[b] : 0;
+        uint32_t all = 0;
+        const uint32_t at = block_exclusive_sum<kPlanBlock>(n, s_wave, &all);
+        if (b < buckets) first[b] = entries_before + at;
+        entries_before += all;
+        __syncthreads();
+        if (t.d2 != 0) {
+            const uint32_t tiles = (n + kSecondTile - 1) / kSecondTile;
+            const uint32_t tile_at = block_exclusive_sum<kPlanBlock>(tiles, s_wave, &all);
+            if (b < buckets) t.tile_first[b] = tiles_before + tile_at;
+            tiles_before += all;
+            __syncthreads();
+        } else if (b < buckets) {
+            note_oversize(t, b, n);
+        }
+    }
+    if (threadIdx.x == 0) {
+        first[buckets] = entries_before;
+        if (t.d2 != 0) t.tile_first[buckets] = tiles_before;
+    }
+}
+
+// The order in which repartition_kernel takes its tiles: an eighth of the buckets at a time (what an XCD works on),
+// inside it the first tiles of all buckets, then the second ones, ...  Tiles of the same number of neighbouring buckets
+// read neighbouring runs of the same tiles of step 1 and meet on the lines at the ends of the runs.
+constexpr int kMapBlock = 256;
+__global__ __launch_bounds__(kMapBlock) void tile_map_kernel(SortTables t) {
+    __shared__ uint32_t s_first[257];
+    const uint32_t buckets = 1u << t.d1;  // at most 256
+    for (uint32_t b = threadIdx.x; b <= buckets; b += kMapBlock) s_first[b] = t.tile_first[b];
+    __syncthreads();
+    const uint32_t q = blockIdx.x * kMapBlock + threadIdx.x;
+    if (q >= s_first[buckets]) return;
+    uint32_t lo = 0, hi = buckets;  // the bucket whose tile q is: the last one that begins at or before it
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) / 2;
+        if (s_first[mid] <= q) lo = mid; else hi = mid;
+    }
+    const uint32_t tile = q - s_first[lo];
+    const uint32_t group = buckets >= 8 ? buckets / 8 : 1;
+    const uint32_t g0 = lo / group * group;
+    uint32_t at = s_first[g0];
+    for (uint32_t b = g0; b < g0 + group; ++b) {
+        const uint32_t tiles = s_first[b + 1] - s_first[b];
+        at += tiles < tile ? tiles : tile;
+        if (b < lo && tiles > tile) ++at;
+    }
+    t.tile_map[at] = lo << 24 | tile;
+}
+
+template <int VB>
+__global__ __launch_bounds__(kSecondThreads) void repartition_kernel(SortTables t, const uint16_t* __restrict__ keys_in,
+                                                                     const uint32_t* __restrict__ aux_in,
+                                                                     const void* __restrict__ vals_in,
+                                                                     uint8_t* __restrict__ keys_out,
+                                                                     uint32_t* __restrict__ aux_out,
+                                                                     void* __restrict__ vals_out, uint32_t max_tiles,
+                                                                     uint32_t xcds) {
+    constexpr int kWaves = kSecondThreads / kWave;
+    constexpr int kMaxBits = 8;
+    typedef typename WordOf<VB>::type word_t;
+    __shared__ __align__(16) uint32_t s_buf[kSecondTile];
+    __shared__ __align__(16) uint16_t s_cnt[kWaves << kMaxBits];
+    __shared__ uint32_t s_wave[kWaves];
+    __shared__ RunMap<kSecondTile> s_map;
+    const uint32_t at = tile_of_block(max_tiles, xcds);
+    if (at >= t.tile_first[1u << t.d1]) return;  // whole workgroup
+    const uint32_t bucket = t.tile_map[at] >> 24, tile = t.tile_map[at] & 0xffffffu;
+    const uint32_t tid = threadIdx.x, wave = tid / kWave;
+    const uint32_t all = t.totals1[bucket];
+    const uint32_t q0 = tile * kSecondTile;
+    const uint32_t count = min(all - q0, kSecondTile);
+    for (uint32_t i = tid; i < sizeof(s_cnt) / 16; i += kSecondThreads) reinterpret_cast<u32x4*>(s_cnt)[i] = u32x4(0);
+    const uint64_t row = static_cast<uint64_t>(bucket) * t.tiles1;
+    map_runs<kSecondThreads, kSecondTile>(t.begins1 + row, t.table1 + row, t.tiles1, all, q0, count, t.places1, 0, s_map, s_buf);
+    uint32_t key[kSecondItems], aux[kSecondItems];
+    word_t val[VB ? kSecondItems : 1];
+    const uint32_t last_word = (count - 1) / kWave;
+#pragma unroll
+    for (int i = 0; i < kSecondItems; ++i) {
+        // (past the last entry: some entry of the last runs, which is not used)
+        const uint32_t from = mapped_place(s_map, s_buf, min(wave * kSecondItems + i, last_word), count);
+        key[i] = keys_in[from];
+        aux[i] = aux_in[from];
+        if constexpr (VB != 0) val[i] = static_cast<const word_t*>(vals_in)[from];
+    }
+    const uint32_t mask = (1u << t.d2) - 1u;
+    auto digit = [&](int i) { return (key[i] >> t.d3) & mask; };
+    uint32_t dest[kSecondItems / 2];
+    rank_entries<kSecondItems, kMaxBits, kWaves>(count, kSecondItems, t.d2, s_cnt, dest, digit);
+    __syncthreads();
+    const uint32_t first_tile = t.tile_first[bucket], tiles = t.tile_first[bucket + 1] - first_tile;
+    uint32_t* table = t.table2 + (static_cast<uint64_t>(first_tile) << t.d2) + tile;
+    place_digits<kSecondThreads, kMaxBits>(t.d2, s_cnt, s_wave, [&](uint32_t d, uint32_t place, uint32_t n) {
+        table[static_cast<uint64_t>(d) * tiles] = table_word(place, n);
+    });
+#pragma unroll
+    for (int i = 0; i < kSecondItems; ++i)
+        dest[i / 2] += static_cast<uint32_t>(s_cnt[(wave << kMaxBits) + digit(i)]) << (i % 2 * 16);
+    const uint64_t out = static_cast<uint64_t>(first_tile + tile) * kSecondTile;
+    store_keys<kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, keys_out + out, key, (1u << t.d3) - 1u);
+    store_words<kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, aux_out + out, aux);
+    if constexpr (VB != 0)
+        store_words<kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, static_cast<word_t*>(vals_out) + out, val);
+}
+
+// begins2 and sub_first from table2; a workgroup per bucket of step 1, a wavefront per digit at a time.
+constexpr int kSubBlock = 1024;
+__global__ __launch_bounds__(kSubBlock) void sub_begins_kernel(SortTables t) {
+    __shared__ uint32_t s_total[256];
+    __shared__ uint32_t s_wave[kSubBlock / kWave];
+    const uint32_t bucket = blockIdx.x, tid = threadIdx.x, lane = tid % kWave;
+    const uint32_t digits = 1u << t.d2;  // at most 256
+    const uint32_t first_tile = t.tile_first[bucket], tiles = t.tile_first[bucket + 1] - first_tile;
+    const uint64_t row0 = static_cast<uint64_t>(first_tile) << t.d2;
+    for (uint32_t d = tid / kWave; d < digits; d += kSubBlock / kWave) {
+        const uint64_t row = row0 + static_cast<uint64_t>(d) * tiles;
+        uint32_t carried = 0;
+        for (uint32_t t0 = 0; t0 < tiles; t0 += kWave) {
+            const uint32_t n = t0 + lane < tiles ? run_length(t.table2[row + t0 + lane]) : 0;
+            const uint32_t upto = wave_inclusive_sum(n);
+            if (t0 + lane < tiles) t.begins2[row + t0 + lane] = carried + upto - n;
+            carried += __builtin_amdgcn_readlane(upto, kWave - 1);
+        }
+        if (lane == 0) s_total[d] = carried;
+    }
+    __syncthreads();
+    const uint32_t n = tid < digits ? s_total[tid] : 0;
+    const uint32_t at = t.bucket_first[bucket] + block_exclusive_sum<kSubBlock>(n, s_wave);
+    const uint32_t sub = (bucket << t.d2) + tid;
+    if (tid < digits) {
+        t.sub_first[sub] = at;
+        note_oversize(t, sub, n);
+    }
+    if (bucket == gridDim.x - 1 && tid == 0) t.sub_first[gridDim.x << t.d2] = t.count;
+}
+
+// ---- step 3 ----------------------------------------------------------------------------------------------------
+struct SortOutput {
+    uint32_t* keys;    // may be null
+    uint32_t* aux;
+    void* vals;
+    uint32_t* key_ptr; // may be null: where each of the `key_count` keys begins, + base, and the end
+    uint32_t key_count, base, key_bias;
+};
+
+// Runs of a bucket of step 3.
+struct BucketRuns {
+    const uint32_t* begins;
+    const uint32_t* table;
+    uint32_t tiles, places, source;
+};
+__device__ __forceinline__ BucketRuns runs_of_bucket(const SortTables& t, uint32_t sub) {
+    BucketRuns r;
+    if (t.d2 == 0) {
+        const uint64_t row = static_cast<uint64_t>(sub) * t.tiles1;
+        r.begins = t.begins1 + row;
+        r.table = t.table1 + row;
+        r.tiles = t.tiles1;
+        r.places = t.places1;
+        r.source = 0;
+    } else {
+        const uint32_t bucket = sub >> t.d2, digit = sub & ((1u << t.d2) - 1u);
+        const uint32_t first_tile = t.tile_first[bucket];
+        r.tiles = t.tile_first[bucket + 1] - first_tile;
+        const uint64_t row = (static_cast<uint64_t>(first_tile) << t.d2) + static_cast<uint64_t>(digit) * r.tiles;
+        r.begins = t.begins2 + row;
+        r.table = t.table2 + row;
+        r.places = kSecondTile;
+        r.source = first_tile * kSecondTile;
+    }
+    return r;
+}
+
+__device__ __forceinline__ void write_key_ptr(const SortOutput& out, uint32_t sub, uint32_t d3, uint32_t digit, uint32_t at,
+                                              uint32_t count) {
+    if (out.key_ptr == nullptr) return;
+    const uint64_t key = (static_cast<uint64_t>(sub) << d3) + digit;
+    if (key < out.key_count) out.key_ptr[key] = at + out.base;
+    if (key + 1 == out.key_count) out.key_ptr[out.key_count] = count + out.base;
+}
+
+// A workgroup per bucket.
+template <int VB>
+__global__ __launch_bounds__(kBucketThreads) void bucket_sort_kernel(SortTables t, const uint8_t* __restrict__ keys_in,
+                                                                     const uint32_t* __restrict__ aux_in,
+                                                                     const void* __restrict__ vals_in, SortOutput out,
+                                                                     uint32_t buckets, uint32_t xcds) {
+    constexpr int kWaves = kBucketThreads / kWave;
+    typedef typename WordOf<VB>::type word_t;
+    __shared__ __align__(16) uint32_t s_buf[kBucketRoom];
+    __shared__ __align__(16) uint16_t s_cnt[kWaves << kMaxD3];
+    __shared__ uint32_t s_wave[kWaves];
+    __shared__ RunMap<kBucketRoom> s_map;
+    const uint32_t sub = tile_of_block(buckets, xcds);
+    if (sub >= buckets) return;  // whole workgroup
+    const uint32_t tid = threadIdx.x, wave = tid / kWave;
+    const uint32_t first = t.sub_first[sub], count = t.sub_first[sub + 1] - first;
+    if (count > kBucketRoom) return;  // whole workgroup: the oversize kernels' work
+    if (count == 0) {
+        for (uint32_t d = tid; d < (1u << t.d3); d += kBucketThreads) write_key_ptr(out, sub, t.d3, d, first, t.count);
+        return;
+    }
+    for (uint32_t i = tid; i < sizeof(s_cnt) / 16; i += kBucketThreads) reinterpret_cast<u32x4*>(s_cnt)[i] = u32x4(0);
+    const BucketRuns runs = runs_of_bucket(t, sub);
+    map_runs<kBucketThreads, kBucketRoom>(runs.begins, runs.table, runs.tiles, count, 0, count, runs.places, runs.source,
+                                          s_map, s_buf);
+    const uint32_t rounds = (count + kBucketThreads - 1) / kBucketThreads;  // a wavefront owns `rounds` * 64 entries
+    uint32_t key[kBucketItems], aux[kBucketItems];
+    word_t val[VB ? kBucketItems : 1];
+    const uint32_t last_word = (count - 1) / kWave;
+#pragma unroll
+    for (int i = 0; i < kBucketItems; ++i) {
+        if (static_cast<uint32_t>(i) < rounds) {  // the same for the workgroup
+            const uint32_t from = mapped_place(s_map, s_buf, min(wave * rounds + i, last_word), count);
+            key[i] = keys_in[from];
+            aux[i] = aux_in[from];
+            if constexpr (VB != 0) val[i] = static_cast<const word_t*>(vals_in)[from];
+        } else {
+            key[i] = 0;
+            aux[i] = 0;
+            if constexpr (VB != 0) val[i] = 0;
+        }
+    }
+    uint32_t dest[kBucketItems / 2];
+    rank_entries<kBucketItems, kMaxD3, kWaves>(count, rounds, t.d3, s_cnt, dest, [&](int i) { return key[i]; });
+    __syncthreads();
+    place_digits<kBucketThreads, kMaxD3>(t.d3, s_cnt, s_wave, [&](uint32_t d, uint32_t at, uint32_t) {
+        write_key_ptr(out, sub, t.d3, d, first + at, t.count);
+    });
+#pragma unroll
+    for (int i = 0; i < kBucketItems; ++i)
+        dest[i / 2] += static_cast<uint32_t>(s_cnt[(wave << kMaxD3) + key[i]]) << (i % 2 * 16);
+
+    // every array: into LDS in its new order, out as a linear stream
+    auto ordered = [&](auto word_of) {
+#pragma unroll
+        for (int i = 0; i < kBucketItems; ++i) {
+            if (static_cast<uint32_t>(i) < rounds && in_slab(rounds, i, count))
+                s_buf[(dest[i / 2] >> (i % 2 * 16)) & 0xffffu] = word_of(i);
+        }
+        __syncthreads();
+    };
+    ordered([&](int i) { return aux[i]; });
+    for (uint32_t p = tid; p < count; p += kBucketThreads) out.aux[first + p] = s_buf[p];
+    __syncthreads();
+    if constexpr (VB == 4) {
+        ordered([&](int i) { return val[i]; });
+        for (uint32_t p = tid; p < count; p += kBucketThreads) static_cast<uint32_t*>(out.vals)[first + p] = s_buf[p];
+        __syncthreads();
+    } else if constexpr (VB == 8) {  // in two halves
+        uint32_t low[kBucketItems];
+        ordered([&](int i) { return static_cast<uint32_t>(val[i]); });
+#pragma unroll
+        for (int i = 0; i < kBucketItems; ++i) low[i] = s_buf[min(i * kBucketThreads + tid, kBucketRoom - 1)];
+        __syncthreads();
+        ordered([&](int i) { return static_cast<uint32_t>(val[i] >> 32); });
+#pragma unroll
+        for (int i = 0; i < kBucketItems; ++i) {
+            const uint32_t p = i * kBucketThreads + tid;
+            if (p < count)
+                static_cast<uint64_t*>(out.vals)[first + p] = static_cast<uint64_t>(s_buf[p]) << 32 | low[i];
+        }
+        __syncthreads();
+    }
+    if (out.keys != nullptr) {
+        ordered([&](int i) { return key[i]; });
+        const uint32_t high = (sub << t.d3) + out.key_bias;
+        for (uint32_t p = tid; p < count; p += kBucketThreads) out.keys[first + p] = high + s_buf[p];
+    }
+}
+
+// ---- buckets that do not fit LDS -------------------------------------------------------------------------------
+// In chunks of kOversizeChunk entries: the digits of every chunk are counted, the counts of a bucket's chunks are
+// added up digit by digit, and every chunk is written from there.
+struct OversizeChunk {
+    uint32_t bucket, chunk, all, q0, count;
+};
+__device__ __forceinline__ OversizeChunk oversize_chunk(const SortTables& t, uint32_t c, uint32_t listed) {
+    uint32_t lo = 0, hi = listed;  // the last listed bucket whose chunks begin at or before c
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) / 2;
+        if (t.oversize[mid].y <= c) lo = mid; else hi = mid;
+    }
+    OversizeChunk k;
+    k.bucket = t.oversize[lo].x;
+    k.chunk = c - t.oversize[lo].y;
+    k.all = t.sub_first[k.bucket + 1] - t.sub_first[k.bucket];
+    k.q0 = k.chunk * kOversizeChunk;
+    k.count = min(k.all - k.q0, kOversizeChunk);
+    return k;
+}
+constexpr uint32_t kOversizeGrid = 512;
+
+__global__ __launch_bounds__(kBucketThreads) void oversize_count_kernel(SortTables t, const uint8_t* __restrict__ keys_in) {
+    const unsigned long long counted = *t.oversize_count;
+    const uint32_t listed = static_cast<uint32_t>(counted), chunks = static_cast<uint32_t>(counted >> 32);
+    if (blockIdx.x >= chunks) return;  // whole workgroup
+    __shared__ __align__(16) uint32_t s_delta[kOversizeChunk];
+    __shared__ uint32_t s_count[1 << kMaxD3];
+    __shared__ RunMap<kOversizeChunk> s_map;
+    for (uint32_t c = blockIdx.x; c < chunks; c += gridDim.x) {
+        const OversizeChunk k = oversize_chunk(t, c, listed);
+        const BucketRuns runs = runs_of_bucket(t, k.bucket);
+        for (uint32_t d = threadIdx.x; d < (1u << kMaxD3); d += kBucketThreads) s_count[d] = 0;
+        map_runs<kBucketThreads, kOversizeChunk>(runs.begins, runs.table, runs.tiles, k.all, k.q0, k.count, runs.places,
+                                                 runs.source, s_map, s_delta);
+        for (uint32_t w = threadIdx.x / kWave; w * kWave < k.count; w += kBucketThreads / kWave) {
+            const uint32_t from = mapped_place(s_map, s_delta, w, k.count);
+            if (w * kWave + threadIdx.x % kWave < k.count) atomicAdd(&s_count[keys_in[from]], 1u);
+        }
+        __syncthreads();
+        for (uint32_t d = threadIdx.x; d < (1u << t.d3); d += kBucketThreads)
+            t.oversize_begins[(static_cast<uint64_t>(c) << t.d3) + d] = s_count[d];
+        __syncthreads();
+    }
+}
+
+// A workgroup per oversize bucket: per digit the counts of the chunks become places in the output.  The chunks are
+// dealt to kSubBlock / 256 shares of a digit's thread each.
+__global__ __launch_bounds__(kSubBlock) void oversize_begins_kernel(SortTables t, SortOutput out) {
+    constexpr uint32_t kDigits = 1 << kMaxD3, kShares = kSubBlock / kDigits;
+    __shared__ uint32_t s_sum[kShares][kDigits];
+    __shared__ uint32_t s_wave[kSubBlock / kWave];
+    const unsigned long long counted = *t.oversize_count;
+    const uint32_t listed = static_cast<uint32_t>(counted), all_chunks = static_cast<uint32_t>(counted >> 32);
+    const uint32_t d = threadIdx.x % kDigits, share = threadIdx.x / kDigits;
+    for (uint32_t k = blockIdx.x; k < listed; k += gridDim.x) {
+        const uint32_t bucket = t.oversize[k].x, c0 = t.oversize[k].y;
+        const uint32_t c1 = k + 1 < listed ? t.oversize[k + 1].y : all_chunks;
+        const uint32_t mine = (c1 - c0 + kShares - 1) / kShares;
+        const uint32_t from = min(c0 + share * mine, c1), to = min(from + mine, c1);
+        uint32_t* column = t.oversize_begins + d;
+        const bool exists = d < (1u << t.d3);
+        uint32_t sum = 0;
+#pragma unroll 8
+        for (uint32_t c = from; c < to; ++c) sum += exists ? column[static_cast<uint64_t>(c) << t.d3] : 0u;
+        s_sum[share][d] = sum;
+        __syncthreads();
+        uint32_t total = 0, before = 0;
+        for (uint32_t s = 0; s < kShares; ++s) {
+            if (s == share) before = total;
+            total += s_sum[s][d];
+        }
+        const uint32_t first = t.sub_first[bucket] + block_exclusive_sum<kSubBlock>(share == 0 ? total : 0u, s_wave);
+        if (share == 0) {
+            s_sum[0][d] = first;  // (its own sum has been read by all: the barrier in the scan)
+            if (exists) write_key_ptr(out, bucket, t.d3, d, first, t.count);
+        }
+        __syncthreads();
+        uint32_t at = s_sum[0][d] + before;
+        for (uint32_t c = from; c < to && exists; ++c) {
+            uint32_t* word = column + (static_cast<uint64_t>(c) << t.d3);
+            const uint32_t n = *word;
+            *word = at;
+            at += n;
+        }
+        __syncthreads();
+    }
+}
+
+template <int VB>
+__global__ __launch_bounds__(kBucketThreads) void oversize_sort_kernel(SortTables t, const uint8_t* __restrict__ keys_in,
+                                                                       const uint32_t* __restrict__ aux_in,
+                                                                       const void* __restrict__ vals_in, SortOutput out) {
+    constexpr int kWaves = kBucketThreads / kWave;
+    typedef typename WordOf<VB>::type word_t;
+    const unsigned long long counted = *t.oversize_count;
+    const uint32_t listed = static_cast<uint32_t>(counted), chunks = static_cast<uint32_t>(counted >> 32);
+    if (blockIdx.x >= chunks) return;  // whole workgroup
+    __shared__ __align__(16) uint32_t s_delta[kOversizeChunk];
+    __shared__ __align__(16) uint16_t s_cnt[kWaves << kMaxD3];
+    __shared__ uint32_t s_to[1 << kMaxD3];  // output place of a digit's first entry, less its place in the chunk
+    __shared__ uint32_t s_wave[kWaves];
+    __shared__ RunMap<kOversizeChunk> s_map;
+    const uint32_t wave = threadIdx.x / kWave;
+    for (uint32_t c = blockIdx.x; c < chunks; c += gridDim.x) {
+        const OversizeChunk k = oversize_chunk(t, c, listed);
+        const BucketRuns runs = runs_of_bucket(t, k.bucket);
+        for (uint32_t i = threadIdx.x; i < sizeof(s_cnt) / 16; i += kBucketThreads) reinterpret_cast<u32x4*>(s_cnt)[i] = u32x4(0);
+        map_runs<kBucketThreads, kOversizeChunk>(runs.begins, runs.table, runs.tiles, k.all, k.q0, k.count, runs.places,
+                                                 runs.source, s_map, s_delta);
+        const uint32_t rounds = (k.count + kBucketThreads - 1) / kBucketThreads;
+        const uint32_t last_word = (k.count - 1) / kWave;
+        uint32_t key[kBucketItems], from[kBucketItems];
+#pragma unroll
+        for (int i = 0; i < kBucketItems; ++i) {
+            from[i] = mapped_place(s_map, s_delta, min(wave * rounds + min(static_cast<uint32_t>(i), rounds - 1), last_word), k.count);
+            key[i] = keys_in[from[i]];
+        }
+        uint32_t dest[kBucketItems / 2];
+        rank_entries<kBucketItems, kMaxD3, kWaves>(k.count, rounds, t.d3, s_cnt, dest, [&](int i) { return key[i]; });
+        __syncthreads();
+        place_digits<kBucketThreads, kMaxD3>(t.d3, s_cnt, s_wave, [&](uint32_t d, uint32_t at, uint32_t) {
+            s_to[d] = t.oversize_begins[(static_cast<uint64_t>(c) << t.d3) + d] - at;
+        });
+#pragma unroll
+        for (int i = 0; i < kBucketItems; ++i) {
+            if (static_cast<uint32_t>(i) < rounds && in_slab(rounds, i, k.count)) {
+                const uint32_t to = s_to[key[i]] + s_cnt[(wave << kMaxD3) + key[i]] + ((dest[i / 2] >> (i % 2 * 16)) & 0xffffu);
+                out.aux[to] = aux_in[from[i]];
+                if constexpr (VB != 0) static_cast<word_t*>(out.vals)[to] = static_cast<const word_t*>(vals_in)[from[i]];
+                if (out.keys != nullptr) out.keys[to] = (k.bucket << t.d3) + key[i] + out.key_bias;
+            }
+        }
+        __syncthreads();
+    }
+}
+
 // Small inputs get small tiles, so that there are a few workgroups per compute unit.
 constexpr uint32_t kTileLarge = 8192, kTileSmall = 2048;
 constexpr uint32_t kSmallTileEntries = 512 * kTileLarge;
@@ -312,7 +826,171 @@ BucketedLayout bucketed_layout(idx_t nnz, size_t value_bytes) {
     return l;
 }
 
+// ---- the sort --------------------------------------------------------------------------------------------------
+// How many bits each step takes.  A bucket of step 3 should fill half of the room it has: keys are seldom spread
+// evenly, and a fuller one costs no more per entry.
+constexpr uint32_t kBucketWanted = kBucketRoom * 6 / 10;
+constexpr uint32_t kMaxOneLevelBits = 11;  // buckets one partition makes: more would leave runs of a few entries
+constexpr uint32_t kMaxTwoLevelBits = 16;
+
+struct SortShape {
+    uint32_t d1, d2, d3, tile_size, tiles1, max_tiles2;
+};
+bool sort_shape(uint32_t count, uint32_t key_bits, SortShape* s) {
+    if (count == 0 || key_bits > kMaxTwoLevelBits + kMaxD3) return false;
+    uint32_t bits = key_bits > kMaxD3 ? key_bits - kMaxD3 : 0;
+    while (bits < key_bits && bits < kMaxTwoLevelBits && (static_cast<uint64_t>(kBucketWanted) << bits) < count) ++bits;
+    s->d1 = bits <= kMaxOneLevelBits ? bits : (bits + 1) / 2;
+    s->d2 = bits - s->d1;
+    s->d3 = key_bits - bits;
+    s->tile_size = tile_size_for(count);
+    s->tiles1 = tiles_of(count, s->tile_size);
+    s->max_tiles2 = s->d2 != 0 ? count / kSecondTile + (1u << s->d1) : 0;
+    return true;
+}
+
+struct SortLayout {
+    size_t keys1, aux1, vals1, keys2, aux2, vals2, table1, begins1, totals1, tile_rows, table2, begins2, bucket_first,
+        tile_first, tile_map, sub_first, oversize_count, oversize, oversize_begins, total;
+};
+SortLayout sort_layout(uint32_t count, const SortShape& s, size_t value_bytes) {
+    const size_t places1 = static_cast<size_t>(s.tiles1) * s.tile_size;
+    const size_t places2 = static_cast<size_t>(s.max_tiles2) * kSecondTile;
+    const size_t runs1 = static_cast<size_t>(s.tiles1) << s.d1, runs2 = static_cast<size_t>(s.max_tiles2) << s.d2;
+    const size_t subs = size_t(1) << (s.d1 + s.d2);
+    const size_t chunks = 2 * (static_cast<size_t>(count) / kOversizeChunk) + 1;  // every oversize bucket has two at least
+    SortLayout l;
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        const size_t at = off;
+        off += align_up(bytes);
+        return at;
+    };
+    l.keys1 = take(places1 * (s.d2 != 0 ? sizeof(uint16_t) : sizeof(uint8_t)));
+    l.aux1 = take(places1 * sizeof(uint32_t));
+    l.vals1 = take(places1 * value_bytes);
+    l.keys2 = take(places2);
+    l.aux2 = take(places2 * sizeof(uint32_t));
+    l.vals2 = take(places2 * value_bytes);
+    l.table1 = take(runs1 * sizeof(uint32_t));
+    l.begins1 = take(runs1 * sizeof(uint32_t));
+    l.totals1 = take(sizeof(uint32_t) << s.d1);
+    l.tile_rows = take((static_cast<size_t>(s.tiles1) + 1) * sizeof(uint32_t));
+    l.table2 = take(runs2 * sizeof(uint32_t));
+    l.begins2 = take(runs2 * sizeof(uint32_t));
+    l.bucket_first = take((sizeof(uint32_t) << s.d1) + sizeof(uint32_t));
+    l.tile_first = take((sizeof(uint32_t) << s.d1) + sizeof(uint32_t));
+    l.tile_map = take(static_cast<size_t>(s.max_tiles2) * sizeof(uint32_t));
+    l.sub_first = take((subs + 1) * sizeof(uint32_t));
+    l.oversize_count = take(sizeof(unsigned long long));
+    l.oversize = take((static_cast<size_t>(count) / kBucketRoom + 1) * sizeof(uint2));
+    l.oversize_begins = take((chunks << s.d3) * sizeof(uint32_t));
+    l.total = off;
+    return l;
+}
+
+template <int VB, int KIND>
+void launch_sort(hipStream_t stream, EntrySource in, const SortShape& s, const SortOutput& out, char* w) {
+    const SortLayout l = sort_layout(in.count, s, VB);
+    auto words = [&](size_t at) { return reinterpret_cast<uint32_t*>(w + at); };
+    const uint32_t xcds = device_topology().xcds;
+    if constexpr (KIND == kCsr) {
+        launch_row_starts(stream, in, s.tile_size, words(l.tile_rows));
+        in.tile_rows = words(l.tile_rows);
+    }
+    SortTables t;
+    t.table1 = words(l.table1);
+    t.begins1 = words(l.begins1);
+    t.totals1 = words(l.totals1);
+    t.tiles1 = s.tiles1;
+    t.places1 = s.tile_size;
+    t.table2 = words(l.table2);
+    t.begins2 = words(l.begins2);
+    t.bucket_first = words(l.bucket_first);
+    t.tile_first = words(l.tile_first);
+    t.tile_map = words(l.tile_map);
+    t.sub_first = words(l.sub_first);
+    t.oversize_count = reinterpret_cast<unsigned long long*>(w + l.oversize_count);
+    t.oversize = reinterpret_cast<uint2*>(w + l.oversize);
+    t.oversize_begins = words(l.oversize_begins);
+    t.d1 = s.d1;
+    t.d2 = s.d2;
+    t.d3 = s.d3;
+    t.count = in.count;
+    const uint32_t shift = s.d2 + s.d3;
+    auto* partition = s.d2 != 0 ? launch_partition<VB, KIND, 8, uint16_t>
+                      : s.d1 <= 8 ? launch_partition<VB, KIND, 8, uint8_t> : launch_partition<VB, KIND, kMaxOneLevelBits, uint8_t>;
+    partition(stream, in, shift, s.d1, s.tile_size, w + l.keys1, words(l.aux1), w + l.vals1, words(l.table1));
+    hipLaunchKernelGGL(run_begins_kernel, dim3(1u << s.d1), dim3(kScanBlock), 0, stream, s.tiles1, t.table1,
+                       words(l.begins1), words(l.totals1));
+    hipLaunchKernelGGL(sort_plan_kernel, dim3(1), dim3(kPlanBlock), 0, stream, t);
+    const uint8_t* keys = reinterpret_cast<const uint8_t*>(w + l.keys1);
+    const uint32_t* aux = words(l.aux1);
+    const void* vals = w + l.vals1;
+    if (s.d2 != 0) {
+        hipLaunchKernelGGL(tile_map_kernel, dim3((s.max_tiles2 + kMapBlock - 1) / kMapBlock), dim3(kMapBlock), 0, stream, t);
+        hipLaunchKernelGGL((repartition_kernel<VB>), dim3((s.max_tiles2 + xcds - 1) / xcds * xcds), dim3(kSecondThreads), 0,
+                           stream, t, reinterpret_cast<const uint16_t*>(w + l.keys1), aux, vals,
+                           reinterpret_cast<uint8_t*>(w + l.keys2), words(l.aux2), w + l.vals2, s.max_tiles2, xcds);
+        hipLaunchKernelGGL(sub_begins_kernel, dim3(1u << s.d1), dim3(kSubBlock), 0, stream, t);
+        keys = reinterpret_cast<const uint8_t*>(w + l.keys2);
+        aux = words(l.aux2);
+        vals = w + l.vals2;
+    }
+    const uint32_t buckets = 1u << (s.d1 + s.d2);
+    hipLaunchKernelGGL((bucket_sort_kernel<VB>), dim3((buckets + xcds - 1) / xcds * xcds), dim3(kBucketThreads), 0, stream, t,
+                       keys, aux, vals, out, buckets, xcds);
+    if (in.count > kBucketRoom) {  // else no bucket is larger than that
+        hipLaunchKernelGGL(oversize_count_kernel, dim3(kOversizeGrid), dim3(kBucketThreads), 0, stream, t, keys);
+        hipLaunchKernelGGL(oversize_begins_kernel, dim3(kOversizeGrid / 4), dim3(kSubBlock), 0, stream, t, out);
+        hipLaunchKernelGGL((oversize_sort_kernel<VB>), dim3(kOversizeGrid), dim3(kBucketThreads), 0, stream, t, keys, aux, vals,
+                           out);
+    }
+}
+
 }  // namespace
+
+bool partition_sort_usable(idx_t count, uint32_t key_bits) {
+    SortShape s;
+    return sort_shape(count, key_bits, &s);
+}
+
+size_t partition_sort_workspace_bytes(idx_t count, uint32_t key_bits, size_t value_bytes) {
+    SortShape s;
+    return sort_shape(count, key_bits, &s) ? sort_layout(count, s, value_bytes).total : 0;
+}
+
+void launch_partition_sort(hipStream_t stream, idx_t count, uint32_t key_bits, const PartitionSortArgs& a, size_t value_bytes,
+                           void* workspace) {
+    SortShape s;
+    if (!sort_shape(count, key_bits, &s)) return;
+    EntrySource in;
+    in.keys = a.keys_in;
+    in.aux = a.csr_rows != 0 ? a.row_ptr : a.aux_in;
+    in.vals = a.vals_in;
+    in.x = nullptr;
+    in.count = count;
+    in.key_bias = a.key_bias;
+    in.m = a.csr_rows;
+    in.base = a.base;
+    in.tile_rows = nullptr;
+    SortOutput out;
+    out.keys = a.keys_out;
+    out.aux = a.aux_out;
+    out.vals = a.vals_out;
+    out.key_ptr = a.key_ptr;
+    out.key_count = a.key_count;
+    out.base = a.base;
+    out.key_bias = a.key_bias;
+    char* w = static_cast<char*>(workspace);
+    if (a.csr_rows != 0) {
+        auto* launch = value_bytes == 0 ? launch_sort<0, kCsr> : value_bytes == 4 ? launch_sort<4, kCsr> : launch_sort<8, kCsr>;
+        launch(stream, in, s, out, w);
+    } else {
+        auto* launch = value_bytes == 0 ? launch_sort<0, kPlain> : launch_sort<4, kPlain>;
+        launch(stream, in, s, out, w);
+    }
+}
 
 bool bucketed_products_shape(idx_t n, uint32_t* shift) {
     const uint32_t bits = bit_length(n - 1);  // of the columns without their index base

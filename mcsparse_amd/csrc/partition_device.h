@@ -289,12 +289,13 @@ __device__ __forceinline__ void map_runs(const uint32_t* __restrict__ run_begins
     __syncthreads();
 }
 
-// Place in memory of entry w * 64 + lane of the chunk.
+// Place in memory of entry w * 64 + lane of a chunk of `count` entries (of the last one, for lanes past it).
 template <int CHUNK>
-__device__ __forceinline__ uint32_t mapped_place(const RunMap<CHUNK>& s, const uint32_t* s_delta, uint32_t w) {
+__device__ __forceinline__ uint32_t mapped_place(const RunMap<CHUNK>& s, const uint32_t* s_delta, uint32_t w, uint32_t count) {
     const unsigned long long later = s.begins[w] >> 1;  // runs that begin at or before a lane, after the first lane
     const uint32_t run = s.before[w] + bits_below_lane(static_cast<uint32_t>(later), static_cast<uint32_t>(later >> 32));
-    return s_delta[run] + w * kWave + threadIdx.x % kWave;
+    // (no run begins behind the last entry: lanes past it have found that entry's run)
+    return s_delta[run] + min(w * kWave + threadIdx.x % kWave, count - 1);
 }
 
 // ---- stores of an ordered tile ---------------------------------------------------------------------------------

@@ -1,13 +1,14 @@
 """GPU parity of what is built on the partition of tiles by key bits (csrc/partition.hip), at the sizes where it can go
 wrong: entry counts around a tile, both tile sizes, keys concentrated in a few runs, empty rows.  The transposing
-mcsparseSpMV without a preprocess call is compared exactly (integer-valued operands make any order of summation exact)."""
+mcsparseSpMV without a preprocess call is compared exactly (integer-valued operands make any order of summation exact),
+csr2csc bit for bit against the oracle."""
 import numpy as np
 import pytest
 
 from mcsparse_amd import api
 from mcsparse_amd import workloads as wl
 
-from gpu_util import run_spmv
+from gpu_util import dev, run_spmv
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +48,38 @@ def test_transposed_product_exact(torch_gpu, handle, dtype, kind, m, n, nnz):
     st, got, _ = run_spmv(torch_gpu, handle, a, x, y, 2.0, -3.0, op=api.OP_T)
     assert st == api.STATUS_SUCCESS
     assert np.array_equal(got.astype(np.float64), want)
+
+
+ONE_LEVEL_UPTO = 3686 << 11  # entries up to which one partition makes the buckets that are sorted in LDS
+
+
+@pytest.mark.parametrize("dtype,action", [(np.float32, api.ACTION_NUMERIC), (np.float64, api.ACTION_NUMERIC),
+                                          (np.float32, api.ACTION_SYMBOLIC)])
+@pytest.mark.parametrize("kind,m,n,nnz,base", [
+    ("uniform", 5, 1, 40, 0), ("uniform", 50, 200, 1, 1), ("uniform", 400, 256, 2049, 0), ("uniform", 300, 257, 20000, 1),
+    ("uniform", 3000, 70000, 6145, 0), ("few", 50, 3, 30000, 0), ("few", 3000, 1 << 16, 400000, 1),
+    ("band", 100000, 90000, 1000001, 0), ("uniform", 100000, 5000, LARGE_FROM, 0), ("few", 100000, 300000, LARGE_FROM + 1, 1),
+    ("uniform", 300000, 1 << 20, ONE_LEVEL_UPTO, 0), ("uniform", 300000, (1 << 20) + 1, ONE_LEVEL_UPTO + 1, 1),
+    ("few", 300000, 1 << 22, ONE_LEVEL_UPTO + 777, 0), ("band", 300000, 3000000, 2 * ONE_LEVEL_UPTO, 0),
+    ("uniform", 20000, (1 << 24) + 1, 500000, 0),
+])
+def test_csr2csc_bit_exact(torch_gpu, handle, oracle, dtype, action, kind, m, n, nnz, base):
+    torch = torch_gpu
+    a = matrix(kind, m, n, nnz, dtype, seed=nnz).with_base(base)
+    d_ptr, d_col, d_val = dev(torch, a.ptr), dev(torch, a.col), dev(torch, a.val)
+    o_val = torch.full((nnz,), -9.0, dtype=d_val.dtype, device="cuda")
+    o_ptr, o_row = (torch.full((k,), -9, dtype=torch.int32, device="cuda") for k in (n + 1, nnz))
+    args = (handle, m, n, nnz, d_val, d_ptr, d_col, o_val, o_ptr, o_row, api.maca_type(np.dtype(dtype)), action, base)
+    st, size = api.csr2csc_buffer_size(*args)
+    assert st == api.STATUS_SUCCESS
+    buf = torch.empty(size, dtype=torch.uint8, device="cuda")
+    want_ptr, want_row, want_val = oracle.csr2csc(m, n, base, a.ptr, a.col, a.val, method="counting")
+    for _ in range(2):
+        assert api.csr2csc(*args, buf) == api.STATUS_SUCCESS
+    torch.cuda.synchronize()
+    assert np.array_equal(o_ptr.cpu().numpy().view(np.uint32), want_ptr)
+    assert np.array_equal(o_row.cpu().numpy().view(np.uint32), want_row)
+    if action == api.ACTION_NUMERIC:
+        assert np.array_equal(o_val.cpu().numpy(), want_val)
+    else:
+        assert (o_val == -9.0).all()
