@@ -114,7 +114,8 @@ __device__ __forceinline__ void count_rows(TileRows<TILE>& s) {
 //
 // Bounds at 118 M entries (the products of a transposing SpMV, fp32): 0.98 GB read and 0.79 GB written in 340 us, nine
 // tenths of the rate of a copy; tiles of 4096 or 16 wavefronts per workgroup are no faster (342 and 420 us).  The pass
-// it replaces took 486 us, with a pass over the keys (111 us) in front of it to count them.
+// it replaces took 486 us, with a pass over the keys (111 us) in front of it to count them.  The first step of csr2csc
+// (18 bytes per entry, the ranks by ballots): 2.16 GB in 380 us.
 template <int VB, int KIND, int MAX_BITS, typename Key, int THREADS, int ITEMS>
 __global__ __launch_bounds__(THREADS) void partition_kernel(EntrySource in, uint32_t shift, uint32_t bits, uint32_t tiles,
                                                                Key* __restrict__ keys_out, uint32_t* __restrict__ aux_out,
@@ -173,7 +174,7 @@ __global__ __launch_bounds__(THREADS) void partition_kernel(EntrySource in, uint
     uint32_t dest[(ITEMS + 1) / 2];
     uint32_t pad_from = 0, pad_to = 0;  // what this thread's digit leaves open behind its run
     uint32_t* const s_count = reinterpret_cast<uint32_t*>(s_cnt);
-    if constexpr (kOrdered) rank_entries<ITEMS, MAX_BITS, kWaves>(count, ITEMS, bits, s_cnt, dest, digit);
+    if constexpr (kOrdered) rank_entries<ITEMS, MAX_BITS>(count, bits, s_cnt, dest, digit);
     else rank_entries_unordered<ITEMS>(count, s_count, dest, digit);
     if constexpr (KIND != kPlain) {
         if (staged) mark_rows<ITEMS, THREADS>(s_rows, s_buf, inside, static_cast<uint32_t>(first) + in.base, aux);
@@ -277,11 +278,17 @@ __global__ __launch_bounds__(kRowStartsBlock) void partition_row_starts_kernel(c
 }
 
 // run_begins[d * tiles + t] = entries of digit d in the tiles before t; totals[d] = all of them.  A workgroup per digit.
+// first_runs (may be null), [d][tiles + 1]: for the entries q * kSecondTile of the digit the run they lie in.
 constexpr int kScanBlock = 256;
 constexpr int kScanItems = 8;
+// Tiles of step 2.  With 16 entries per thread there is room for two workgroups per compute unit only, and what a
+// workgroup waits for shows: 118 M entries in 600 us, with 12 in 535.
+constexpr int kSecondThreads = 512, kSecondItems = 12;
+constexpr uint32_t kSecondTile = kSecondThreads * kSecondItems;
 __global__ __launch_bounds__(kScanBlock) void run_begins_kernel(uint32_t tiles, const uint32_t* __restrict__ table,
                                                                 uint32_t* __restrict__ run_begins,
-                                                                uint32_t* __restrict__ totals) {
+                                                                uint32_t* __restrict__ totals,
+                                                                uint32_t* __restrict__ first_runs) {
     __shared__ uint32_t s_wave[kScanBlock / kWave];
     const uint32_t* in = table + static_cast<uint64_t>(blockIdx.x) * tiles;
     uint32_t* out = run_begins + static_cast<uint64_t>(blockIdx.x) * tiles;
@@ -304,6 +311,11 @@ __global__ __launch_bounds__(kScanBlock) void run_begins_kernel(uint32_t tiles, 
         for (int k = 0; k < kScanItems; ++k) {
             const uint32_t t = t0 + threadIdx.x * kScanItems + k;
             if (t < tiles) out[t] = at;
+            if (first_runs != nullptr && n[k] != 0) {  // (a run is no longer than a tile)
+                const uint32_t q = (at + kSecondTile - 1) / kSecondTile;
+                for (uint32_t k2 = q; k2 * kSecondTile < at + n[k]; ++k2)
+                    first_runs[static_cast<uint64_t>(blockIdx.x) * (tiles + 1) + k2] = t;
+            }
             at += n[k];
         }
         carried += all;
@@ -328,7 +340,8 @@ struct SortTables {
     uint32_t* begins2;
     uint32_t* bucket_first;  // entries before each bucket of step 1, 2^d1 + 1 of them
     uint32_t* tile_first;    // tiles before each bucket of step 1, 2^d1 + 1 of them
-    uint32_t* tile_map;      // the order in which the tiles are taken: bucket << 24 | tile of the bucket
+    const uint32_t* first_runs;  // [bucket][tiles1 + 1]: the run of step 1 in which each of its tiles begins
+    uint2* tile_map;         // the order in which the tiles are taken: {bucket << 24 | tile of the bucket, its first run}
     // both: entries before each bucket of step 3, 2^(d1 + d2) + 1 of them
     uint32_t* sub_first;
     // buckets of step 3 that do not fit LDS
@@ -338,9 +351,6 @@ struct SortTables {
     uint32_t d1, d2, d3, count;
 };
 
-constexpr uint32_t kSecondTile = 8192;
-constexpr int kSecondThreads = 512, kSecondItems = 16;
-static_assert(kSecondThreads * kSecondItems == kSecondTile, "a tile per workgroup");
 constexpr int kBucketThreads = 512, kBucketItems = 12;
 constexpr uint32_t kBucketRoom = kBucketThreads * kBucketItems;  // entries of the largest bucket that is sorted in LDS
 constexpr uint32_t kMaxD3 = 8;
@@ -415,9 +425,10 @@ __global__ __launch_bounds__(kMapBlock) void tile_map_kernel(SortTables t) {
         at += tiles < tile ? tiles : tile;
         if (b < lo && tiles > tile) ++at;
     }
-    t.tile_map[at] = lo << 24 | tile;
+    t.tile_map[at] = make_uint2(lo << 24 | tile, t.first_runs[static_cast<uint64_t>(lo) * (t.tiles1 + 1) + tile]);
 }
 
+// 118 M entries (19 bytes each): 1.33 GB read, 1.14 GB written in 500 us.
 template <int VB>
 __global__ __launch_bounds__(kSecondThreads) void repartition_kernel(SortTables t, const uint16_t* __restrict__ keys_in,
                                                                      const uint32_t* __restrict__ aux_in,
@@ -434,15 +445,17 @@ __global__ __launch_bounds__(kSecondThreads) void repartition_kernel(SortTables 
     __shared__ uint32_t s_wave[kWaves];
     __shared__ RunMap<kSecondTile> s_map;
     const uint32_t at = tile_of_block(max_tiles, xcds);
+    const uint2 mine = t.tile_map[min(at, max_tiles - 1)];
     if (at >= t.tile_first[1u << t.d1]) return;  // whole workgroup
-    const uint32_t bucket = t.tile_map[at] >> 24, tile = t.tile_map[at] & 0xffffffu;
+    const uint32_t bucket = mine.x >> 24, tile = mine.x & 0xffffffu;
     const uint32_t tid = threadIdx.x, wave = tid / kWave;
     const uint32_t all = t.totals1[bucket];
     const uint32_t q0 = tile * kSecondTile;
     const uint32_t count = min(all - q0, kSecondTile);
     for (uint32_t i = tid; i < sizeof(s_cnt) / 16; i += kSecondThreads) reinterpret_cast<u32x4*>(s_cnt)[i] = u32x4(0);
     const uint64_t row = static_cast<uint64_t>(bucket) * t.tiles1;
-    map_runs<kSecondThreads, kSecondTile>(t.begins1 + row, t.table1 + row, t.tiles1, all, q0, count, t.places1, 0, s_map, s_buf);
+    map_runs<kSecondThreads, kSecondTile>(t.begins1 + row, t.table1 + row, t.tiles1, all, q0, count, mine.y, t.places1, 0, s_map,
+                                          s_buf);
     uint32_t key[kSecondItems], aux[kSecondItems];
     word_t val[VB ? kSecondItems : 1];
     const uint32_t last_word = (count - 1) / kWave;
@@ -450,14 +463,14 @@ __global__ __launch_bounds__(kSecondThreads) void repartition_kernel(SortTables 
     for (int i = 0; i < kSecondItems; ++i) {
         // (past the last entry: some entry of the last runs, which is not used)
         const uint32_t from = mapped_place(s_map, s_buf, min(wave * kSecondItems + i, last_word), count);
-        key[i] = keys_in[from];
-        aux[i] = aux_in[from];
-        if constexpr (VB != 0) val[i] = static_cast<const word_t*>(vals_in)[from];
+        key[i] = load_at<uint16_t>(keys_in, from);
+        aux[i] = load_at<uint32_t>(aux_in, from);
+        if constexpr (VB != 0) val[i] = load_at<word_t>(vals_in, from);
     }
     const uint32_t mask = (1u << t.d2) - 1u;
     auto digit = [&](int i) { return (key[i] >> t.d3) & mask; };
     uint32_t dest[kSecondItems / 2];
-    rank_entries<kSecondItems, kMaxBits, kWaves>(count, kSecondItems, t.d2, s_cnt, dest, digit);
+    rank_entries<kSecondItems, kMaxBits>(count, t.d2, s_cnt, dest, digit);
     __syncthreads();
     const uint32_t first_tile = t.tile_first[bucket], tiles = t.tile_first[bucket + 1] - first_tile;
     uint32_t* table = t.table2 + (static_cast<uint64_t>(first_tile) << t.d2) + tile;
@@ -550,94 +563,104 @@ __device__ __forceinline__ void write_key_ptr(const SortOutput& out, uint32_t su
     if (key + 1 == out.key_count) out.key_ptr[out.key_count] = count + out.base;
 }
 
-// A workgroup per bucket.
+struct BucketLds {
+    __align__(16) uint32_t buf[kBucketRoom];
+    __align__(16) uint16_t cnt[kBucketThreads / kWave << kMaxD3];
+    uint32_t wave[kBucketThreads / kWave];
+    RunMap<kBucketRoom> map;
+};
+
+// Sorts a bucket of at most ITEMS * kBucketThreads entries, the runs of which are mapped in LDS.
+template <int VB, int ITEMS>
+__device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, uint32_t first, uint32_t count,
+                                            const uint8_t* keys_in, const uint32_t* aux_in, const void* vals_in,
+                                            const SortOutput& out, BucketLds& s) {
+    typedef typename WordOf<VB>::type word_t;
+    const uint32_t tid = threadIdx.x, wave = tid / kWave;
+    uint32_t key[ITEMS], aux[ITEMS];
+    word_t val[VB ? ITEMS : 1];
+    const uint32_t last_word = (count - 1) / kWave;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const uint32_t from = mapped_place(s.map, s.buf, min(wave * ITEMS + i, last_word), count);
+        key[i] = load_at<uint8_t>(keys_in, from);
+        aux[i] = load_at<uint32_t>(aux_in, from);
+        if constexpr (VB != 0) val[i] = load_at<word_t>(vals_in, from);
+    }
+    uint32_t dest[(ITEMS + 1) / 2];
+    rank_entries<ITEMS, kMaxD3>(count, t.d3, s.cnt, dest, [&](int i) { return key[i]; });
+    __syncthreads();
+    place_digits<kBucketThreads, kMaxD3>(t.d3, s.cnt, s.wave, [&](uint32_t d, uint32_t at, uint32_t) {
+        write_key_ptr(out, sub, t.d3, d, first + at, t.count);
+    });
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i)
+        dest[i / 2] += static_cast<uint32_t>(s.cnt[(wave << kMaxD3) + key[i]]) << (i % 2 * 16);
+
+    // every array: into LDS in its new order, out as a linear stream
+    auto ordered = [&](auto word_of) {
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            if (in_slab(ITEMS, i, count)) s.buf[(dest[i / 2] >> (i % 2 * 16)) & 0xffffu] = word_of(i);
+        }
+        __syncthreads();
+    };
+    auto stream_out = [&](auto store) {
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            const uint32_t p = i * kBucketThreads + tid;
+            if (p < count) store(i, p, s.buf[p]);
+        }
+        __syncthreads();
+    };
+    ordered([&](int i) { return aux[i]; });
+    stream_out([&](int, uint32_t p, uint32_t w) { out.aux[first + p] = w; });
+    if constexpr (VB == 4) {
+        ordered([&](int i) { return val[i]; });
+        stream_out([&](int, uint32_t p, uint32_t w) { static_cast<uint32_t*>(out.vals)[first + p] = w; });
+    } else if constexpr (VB == 8) {  // in two halves
+        uint32_t low[ITEMS];
+        ordered([&](int i) { return static_cast<uint32_t>(val[i]); });
+        stream_out([&](int i, uint32_t, uint32_t w) { low[i] = w; });
+        ordered([&](int i) { return static_cast<uint32_t>(val[i] >> 32); });
+        stream_out([&](int i, uint32_t p, uint32_t w) {
+            static_cast<uint64_t*>(out.vals)[first + p] = static_cast<uint64_t>(w) << 32 | low[i];
+        });
+    }
+    if (out.keys != nullptr) {
+        const uint32_t high = (sub << t.d3) + out.key_bias;
+        ordered([&](int i) { return key[i]; });
+        stream_out([&](int, uint32_t p, uint32_t w) { out.keys[first + p] = high + w; });
+    }
+}
+
+// A workgroup per bucket.  118 M entries (17 bytes each) in buckets of 3600: 445 us, bound by vector instructions as much
+// as by memory (86 % of the cycles, 4.6 TB/s); so most buckets, below two thirds of the room, run a version without the
+// last third of the items (458 -> 445 us).
 template <int VB>
-__global__ __launch_bounds__(kBucketThreads) void bucket_sort_kernel(SortTables t, const uint8_t* __restrict__ keys_in,
+__global__ __launch_bounds__(kBucketThreads, VB == 8 ? 6 : 8) void bucket_sort_kernel(SortTables t, const uint8_t* __restrict__ keys_in,
                                                                      const uint32_t* __restrict__ aux_in,
                                                                      const void* __restrict__ vals_in, SortOutput out,
                                                                      uint32_t buckets, uint32_t xcds) {
-    constexpr int kWaves = kBucketThreads / kWave;
-    typedef typename WordOf<VB>::type word_t;
-    __shared__ __align__(16) uint32_t s_buf[kBucketRoom];
-    __shared__ __align__(16) uint16_t s_cnt[kWaves << kMaxD3];
-    __shared__ uint32_t s_wave[kWaves];
-    __shared__ RunMap<kBucketRoom> s_map;
+    constexpr int kUsualItems = kBucketItems * 2 / 3;
+    __shared__ BucketLds s;
     const uint32_t sub = tile_of_block(buckets, xcds);
     if (sub >= buckets) return;  // whole workgroup
-    const uint32_t tid = threadIdx.x, wave = tid / kWave;
+    const uint32_t tid = threadIdx.x;
     const uint32_t first = t.sub_first[sub], count = t.sub_first[sub + 1] - first;
     if (count > kBucketRoom) return;  // whole workgroup: the oversize kernels' work
     if (count == 0) {
         for (uint32_t d = tid; d < (1u << t.d3); d += kBucketThreads) write_key_ptr(out, sub, t.d3, d, first, t.count);
         return;
     }
-    for (uint32_t i = tid; i < sizeof(s_cnt) / 16; i += kBucketThreads) reinterpret_cast<u32x4*>(s_cnt)[i] = u32x4(0);
+    for (uint32_t i = tid; i < sizeof(s.cnt) / 16; i += kBucketThreads) reinterpret_cast<u32x4*>(s.cnt)[i] = u32x4(0);
     const BucketRuns runs = runs_of_bucket(t, sub);
-    map_runs<kBucketThreads, kBucketRoom>(runs.begins, runs.table, runs.tiles, count, 0, count, runs.places, runs.source,
-                                          s_map, s_buf);
-    const uint32_t rounds = (count + kBucketThreads - 1) / kBucketThreads;  // a wavefront owns `rounds` * 64 entries
-    uint32_t key[kBucketItems], aux[kBucketItems];
-    word_t val[VB ? kBucketItems : 1];
-    const uint32_t last_word = (count - 1) / kWave;
-#pragma unroll
-    for (int i = 0; i < kBucketItems; ++i) {
-        if (static_cast<uint32_t>(i) < rounds) {  // the same for the workgroup
-            const uint32_t from = mapped_place(s_map, s_buf, min(wave * rounds + i, last_word), count);
-            key[i] = keys_in[from];
-            aux[i] = aux_in[from];
-            if constexpr (VB != 0) val[i] = static_cast<const word_t*>(vals_in)[from];
-        } else {
-            key[i] = 0;
-            aux[i] = 0;
-            if constexpr (VB != 0) val[i] = 0;
-        }
-    }
-    uint32_t dest[kBucketItems / 2];
-    rank_entries<kBucketItems, kMaxD3, kWaves>(count, rounds, t.d3, s_cnt, dest, [&](int i) { return key[i]; });
-    __syncthreads();
-    place_digits<kBucketThreads, kMaxD3>(t.d3, s_cnt, s_wave, [&](uint32_t d, uint32_t at, uint32_t) {
-        write_key_ptr(out, sub, t.d3, d, first + at, t.count);
-    });
-#pragma unroll
-    for (int i = 0; i < kBucketItems; ++i)
-        dest[i / 2] += static_cast<uint32_t>(s_cnt[(wave << kMaxD3) + key[i]]) << (i % 2 * 16);
-
-    // every array: into LDS in its new order, out as a linear stream
-    auto ordered = [&](auto word_of) {
-#pragma unroll
-        for (int i = 0; i < kBucketItems; ++i) {
-            if (static_cast<uint32_t>(i) < rounds && in_slab(rounds, i, count))
-                s_buf[(dest[i / 2] >> (i % 2 * 16)) & 0xffffu] = word_of(i);
-        }
-        __syncthreads();
-    };
-    ordered([&](int i) { return aux[i]; });
-    for (uint32_t p = tid; p < count; p += kBucketThreads) out.aux[first + p] = s_buf[p];
-    __syncthreads();
-    if constexpr (VB == 4) {
-        ordered([&](int i) { return val[i]; });
-        for (uint32_t p = tid; p < count; p += kBucketThreads) static_cast<uint32_t*>(out.vals)[first + p] = s_buf[p];
-        __syncthreads();
-    } else if constexpr (VB == 8) {  // in two halves
-        uint32_t low[kBucketItems];
-        ordered([&](int i) { return static_cast<uint32_t>(val[i]); });
-#pragma unroll
-        for (int i = 0; i < kBucketItems; ++i) low[i] = s_buf[min(i * kBucketThreads + tid, kBucketRoom - 1)];
-        __syncthreads();
-        ordered([&](int i) { return static_cast<uint32_t>(val[i] >> 32); });
-#pragma unroll
-        for (int i = 0; i < kBucketItems; ++i) {
-            const uint32_t p = i * kBucketThreads + tid;
-            if (p < count)
-                static_cast<uint64_t*>(out.vals)[first + p] = static_cast<uint64_t>(s_buf[p]) << 32 | low[i];
-        }
-        __syncthreads();
-    }
-    if (out.keys != nullptr) {
-        ordered([&](int i) { return key[i]; });
-        const uint32_t high = (sub << t.d3) + out.key_bias;
-        for (uint32_t p = tid; p < count; p += kBucketThreads) out.keys[first + p] = high + s_buf[p];
-    }
+    map_runs<kBucketThreads, kBucketRoom>(runs.begins, runs.table, runs.tiles, count, 0, count, 0, runs.places, runs.source,
+                                          s.map, s.buf);
+    if (count <= static_cast<uint32_t>(kUsualItems * kBucketThreads))
+        sort_bucket<VB, kUsualItems>(t, sub, first, count, keys_in, aux_in, vals_in, out, s);
+    else
+        sort_bucket<VB, kBucketItems>(t, sub, first, count, keys_in, aux_in, vals_in, out, s);
 }
 
 // ---- buckets that do not fit LDS -------------------------------------------------------------------------------
@@ -673,8 +696,9 @@ __global__ __launch_bounds__(kBucketThreads) void oversize_count_kernel(SortTabl
         const OversizeChunk k = oversize_chunk(t, c, listed);
         const BucketRuns runs = runs_of_bucket(t, k.bucket);
         for (uint32_t d = threadIdx.x; d < (1u << kMaxD3); d += kBucketThreads) s_count[d] = 0;
-        map_runs<kBucketThreads, kOversizeChunk>(runs.begins, runs.table, runs.tiles, k.all, k.q0, k.count, runs.places,
-                                                 runs.source, s_map, s_delta);
+        map_runs<kBucketThreads, kOversizeChunk>(runs.begins, runs.table, runs.tiles, k.all, k.q0, k.count,
+                                                 find_first_run(runs.begins, runs.tiles, k.q0), runs.places, runs.source, s_map,
+                                                 s_delta);
         for (uint32_t w = threadIdx.x / kWave; w * kWave < k.count; w += kBucketThreads / kWave) {
             const uint32_t from = mapped_place(s_map, s_delta, w, k.count);
             if (w * kWave + threadIdx.x % kWave < k.count) atomicAdd(&s_count[keys_in[from]], 1u);
@@ -748,28 +772,28 @@ __global__ __launch_bounds__(kBucketThreads) void oversize_sort_kernel(SortTable
         const OversizeChunk k = oversize_chunk(t, c, listed);
         const BucketRuns runs = runs_of_bucket(t, k.bucket);
         for (uint32_t i = threadIdx.x; i < sizeof(s_cnt) / 16; i += kBucketThreads) reinterpret_cast<u32x4*>(s_cnt)[i] = u32x4(0);
-        map_runs<kBucketThreads, kOversizeChunk>(runs.begins, runs.table, runs.tiles, k.all, k.q0, k.count, runs.places,
-                                                 runs.source, s_map, s_delta);
-        const uint32_t rounds = (k.count + kBucketThreads - 1) / kBucketThreads;
+        map_runs<kBucketThreads, kOversizeChunk>(runs.begins, runs.table, runs.tiles, k.all, k.q0, k.count,
+                                                 find_first_run(runs.begins, runs.tiles, k.q0), runs.places, runs.source, s_map,
+                                                 s_delta);
         const uint32_t last_word = (k.count - 1) / kWave;
         uint32_t key[kBucketItems], from[kBucketItems];
 #pragma unroll
         for (int i = 0; i < kBucketItems; ++i) {
-            from[i] = mapped_place(s_map, s_delta, min(wave * rounds + min(static_cast<uint32_t>(i), rounds - 1), last_word), k.count);
+            from[i] = mapped_place(s_map, s_delta, min(wave * kBucketItems + i, last_word), k.count);
             key[i] = keys_in[from[i]];
         }
         uint32_t dest[kBucketItems / 2];
-        rank_entries<kBucketItems, kMaxD3, kWaves>(k.count, rounds, t.d3, s_cnt, dest, [&](int i) { return key[i]; });
+        rank_entries<kBucketItems, kMaxD3>(k.count, t.d3, s_cnt, dest, [&](int i) { return key[i]; });
         __syncthreads();
         place_digits<kBucketThreads, kMaxD3>(t.d3, s_cnt, s_wave, [&](uint32_t d, uint32_t at, uint32_t) {
             s_to[d] = t.oversize_begins[(static_cast<uint64_t>(c) << t.d3) + d] - at;
         });
 #pragma unroll
         for (int i = 0; i < kBucketItems; ++i) {
-            if (static_cast<uint32_t>(i) < rounds && in_slab(rounds, i, k.count)) {
+            if (in_slab(kBucketItems, i, k.count)) {
                 const uint32_t to = s_to[key[i]] + s_cnt[(wave << kMaxD3) + key[i]] + ((dest[i / 2] >> (i % 2 * 16)) & 0xffffu);
-                out.aux[to] = aux_in[from[i]];
-                if constexpr (VB != 0) static_cast<word_t*>(out.vals)[to] = static_cast<const word_t*>(vals_in)[from[i]];
+                out.aux[to] = load_at<uint32_t>(aux_in, from[i]);
+                if constexpr (VB != 0) static_cast<word_t*>(out.vals)[to] = load_at<word_t>(vals_in, from[i]);
                 if (out.keys != nullptr) out.keys[to] = (k.bucket << t.d3) + key[i] + out.key_bias;
             }
         }
@@ -832,12 +856,14 @@ BucketedLayout bucketed_layout(idx_t nnz, size_t value_bytes) {
 constexpr uint32_t kBucketWanted = kBucketRoom * 6 / 10;
 constexpr uint32_t kMaxOneLevelBits = 11;  // buckets one partition makes: more would leave runs of a few entries
 constexpr uint32_t kMaxTwoLevelBits = 16;
+constexpr uint32_t kMostEntries = kBucketRoom * 3 / 4 << kMaxTwoLevelBits;  // more entries: the buckets stop fitting LDS
 
 struct SortShape {
     uint32_t d1, d2, d3, tile_size, tiles1, max_tiles2;
 };
 bool sort_shape(uint32_t count, uint32_t key_bits, SortShape* s) {
-    if (count == 0 || key_bits > kMaxTwoLevelBits + kMaxD3) return false;
+    // (and every array of the sort stays below 4 GiB)
+    if (count == 0 || count > kMostEntries || key_bits > kMaxTwoLevelBits + kMaxD3) return false;
     uint32_t bits = key_bits > kMaxD3 ? key_bits - kMaxD3 : 0;
     while (bits < key_bits && bits < kMaxTwoLevelBits && (static_cast<uint64_t>(kBucketWanted) << bits) < count) ++bits;
     s->d1 = bits <= kMaxOneLevelBits ? bits : (bits + 1) / 2;
@@ -851,7 +877,7 @@ bool sort_shape(uint32_t count, uint32_t key_bits, SortShape* s) {
 
 struct SortLayout {
     size_t keys1, aux1, vals1, keys2, aux2, vals2, table1, begins1, totals1, tile_rows, table2, begins2, bucket_first,
-        tile_first, tile_map, sub_first, oversize_count, oversize, oversize_begins, total;
+        tile_first, first_runs, tile_map, sub_first, oversize_count, oversize, oversize_begins, total;
 };
 SortLayout sort_layout(uint32_t count, const SortShape& s, size_t value_bytes) {
     const size_t places1 = static_cast<size_t>(s.tiles1) * s.tile_size;
@@ -880,7 +906,8 @@ SortLayout sort_layout(uint32_t count, const SortShape& s, size_t value_bytes) {
     l.begins2 = take(runs2 * sizeof(uint32_t));
     l.bucket_first = take((sizeof(uint32_t) << s.d1) + sizeof(uint32_t));
     l.tile_first = take((sizeof(uint32_t) << s.d1) + sizeof(uint32_t));
-    l.tile_map = take(static_cast<size_t>(s.max_tiles2) * sizeof(uint32_t));
+    l.first_runs = take(s.d2 != 0 ? (runs1 + (size_t(1) << s.d1)) * sizeof(uint32_t) : 0);
+    l.tile_map = take(static_cast<size_t>(s.max_tiles2) * sizeof(uint2));
     l.sub_first = take((subs + 1) * sizeof(uint32_t));
     l.oversize_count = take(sizeof(unsigned long long));
     l.oversize = take((static_cast<size_t>(count) / kBucketRoom + 1) * sizeof(uint2));
@@ -908,7 +935,8 @@ void launch_sort(hipStream_t stream, EntrySource in, const SortShape& s, const S
     t.begins2 = words(l.begins2);
     t.bucket_first = words(l.bucket_first);
     t.tile_first = words(l.tile_first);
-    t.tile_map = words(l.tile_map);
+    t.first_runs = words(l.first_runs);
+    t.tile_map = reinterpret_cast<uint2*>(w + l.tile_map);
     t.sub_first = words(l.sub_first);
     t.oversize_count = reinterpret_cast<unsigned long long*>(w + l.oversize_count);
     t.oversize = reinterpret_cast<uint2*>(w + l.oversize);
@@ -922,7 +950,7 @@ void launch_sort(hipStream_t stream, EntrySource in, const SortShape& s, const S
                       : s.d1 <= 8 ? launch_partition<VB, KIND, 8, uint8_t> : launch_partition<VB, KIND, kMaxOneLevelBits, uint8_t>;
     partition(stream, in, shift, s.d1, s.tile_size, w + l.keys1, words(l.aux1), w + l.vals1, words(l.table1));
     hipLaunchKernelGGL(run_begins_kernel, dim3(1u << s.d1), dim3(kScanBlock), 0, stream, s.tiles1, t.table1,
-                       words(l.begins1), words(l.totals1));
+                       words(l.begins1), words(l.totals1), s.d2 != 0 ? words(l.first_runs) : nullptr);
     hipLaunchKernelGGL(sort_plan_kernel, dim3(1), dim3(kPlanBlock), 0, stream, t);
     const uint8_t* keys = reinterpret_cast<const uint8_t*>(w + l.keys1);
     const uint32_t* aux = words(l.aux1);

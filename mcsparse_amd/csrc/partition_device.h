@@ -88,19 +88,25 @@ __device__ __forceinline__ uint32_t block_exclusive_sum(uint32_t v, uint32_t* s_
     return before + upto - v;
 }
 
-// Position inside the tile of a thread's i-th entry: wavefronts own consecutive slabs of `rounds` times 64 entries
+// Position inside the tile of a thread's i-th entry: wavefronts own consecutive slabs of `items` times 64 entries
 // and the lanes are interleaved inside a slab, so (wavefront, i, lane) order is the order of the entries.
-__device__ __forceinline__ uint32_t slab_place(uint32_t rounds, uint32_t i) {
-    return (threadIdx.x / kWave * rounds + i) * kWave + threadIdx.x % kWave;
+__device__ __forceinline__ uint32_t slab_place(uint32_t items, uint32_t i) {
+    return (threadIdx.x / kWave * items + i) * kWave + threadIdx.x % kWave;
 }
-// slab_place(rounds, i) < count, as one comparison with a scalar.
-__device__ __forceinline__ bool in_slab(uint32_t rounds, uint32_t i, uint32_t count) {
-    return static_cast<int>(slab_place(rounds, 0)) < static_cast<int>(count) - static_cast<int>(i * kWave);
+// slab_place(items, i) < count, as one comparison with a scalar.
+__device__ __forceinline__ bool in_slab(uint32_t items, uint32_t i, uint32_t count) {
+    return static_cast<int>(slab_place(items, 0)) < static_cast<int>(count) - static_cast<int>(i * kWave);
 }
 
 // A value the compiler cannot trace back: what is worked out from it again costs an instruction and not a register held
 // from the first time on.
 __device__ __forceinline__ void forget(uint32_t& v) { asm volatile("" : "+v"(v)); }
+
+// array[index] for arrays of less than 4 GiB: a scalar base and a 32-bit offset.
+template <typename W>
+__device__ __forceinline__ W load_at(const void* array, uint32_t index) {
+    return *reinterpret_cast<const W*>(static_cast<const char*>(array) + index * static_cast<uint32_t>(sizeof(W)));
+}
 
 // Reads of a tile of an array through a buffer resource that ends with the tile: places past the end read as zero
 // without a test, and a thread's items differ by constants only (no register per item).
@@ -126,30 +132,27 @@ struct TileReader {
 // Stable rank of every entry among the entries of its wavefront with the same digit, two 16-bit ranks to a word;
 // s_cnt[wave][digit] ends as the wavefront's count of the digit (zero on entry).  digit(i) is the digit of entry i;
 // entries from `count` on are left out.
-template <int ITEMS, int MAX_BITS, int WAVES, typename Digit>
-__device__ __forceinline__ void rank_entries(uint32_t count, uint32_t rounds, uint32_t bits, uint16_t* s_cnt,
+template <int ITEMS, int MAX_BITS, typename Digit>
+__device__ __forceinline__ void rank_entries(uint32_t count, uint32_t bits, uint16_t* s_cnt,
                                              uint32_t (&rank)[(ITEMS + 1) / 2], Digit digit) {
     uint16_t* mine = s_cnt + (threadIdx.x / kWave << MAX_BITS);
-    const bool whole = count == static_cast<uint32_t>(WAVES) * rounds * kWave;  // the same for the workgroup
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
         uint32_t r = 0;
-        if (static_cast<uint32_t>(i) < rounds) {
-            const uint32_t d = digit(i);
-            const bool live = whole || in_slab(rounds, i, count);
-            const uint64_t candidates = __ballot(live);
-            uint32_t lo = static_cast<uint32_t>(candidates), hi = static_cast<uint32_t>(candidates >> 32);
-            keep_equal_digits<MAX_BITS>(d, bits, lo, hi);
-            const uint32_t below = bits_below_lane(lo, hi);
-            if (live) {
-                // Every peer reads the counter, then the lowest one adds the round's count.  The LDS operations of a
-                // wavefront complete in program order; relaxed atomics keep the compiler from moving or merging them.
-                const uint32_t before = __hip_atomic_load(mine + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-                r = before + below;
-                if (below == 0) {
-                    __hip_atomic_store(mine + d, static_cast<uint16_t>(before + __popc(lo) + __popc(hi)), __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_WAVEFRONT);
-                }
+        const uint32_t d = digit(i);
+        const bool live = in_slab(ITEMS, i, count);
+        const uint64_t candidates = __ballot(live);
+        uint32_t lo = static_cast<uint32_t>(candidates), hi = static_cast<uint32_t>(candidates >> 32);
+        keep_equal_digits<MAX_BITS>(d, bits, lo, hi);
+        const uint32_t below = bits_below_lane(lo, hi);
+        if (live) {
+            // Every peer reads the counter, then the lowest one adds the round's count.  The LDS operations of a
+            // wavefront complete in program order; relaxed atomics keep the compiler from moving or merging them.
+            const uint32_t before = __hip_atomic_load(mine + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+            r = before + below;
+            if (below == 0) {
+                __hip_atomic_store(mine + d, static_cast<uint16_t>(before + __popc(lo) + __popc(hi)), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WAVEFRONT);
             }
         }
         if (i % 2 == 0) rank[i / 2] = r;
@@ -235,24 +238,25 @@ struct RunMap {
     unsigned long long begins[CHUNK / kWave];
     uint32_t before[CHUNK / kWave];  // runs that begin before each 64 entries, less one, the first entry's own included
     uint32_t wave[16];
-    uint32_t first_run;
 };
+// The last run of a bucket that begins at or before entry q0, found by search; for whole wavefronts.
+__device__ __forceinline__ uint32_t find_first_run(const uint32_t* __restrict__ run_begins, uint32_t tiles, uint32_t q0) {
+    const uint32_t upto = wave_count_up_to(run_begins, tiles, 0, q0);
+    return upto != 0 ? upto - 1 : 0;
+}
 
+// first_run: the last run that begins at or before q0 (earlier ones will do).
 template <int THREADS, int CHUNK>
 __device__ __forceinline__ void map_runs(const uint32_t* __restrict__ run_begins, const uint32_t* __restrict__ table,
-                                         uint32_t tiles, uint32_t all, uint32_t q0, uint32_t count, uint32_t tile_size,
-                                         uint32_t source, RunMap<CHUNK>& s, uint32_t* s_delta) {
+                                         uint32_t tiles, uint32_t all, uint32_t q0, uint32_t count, uint32_t first_run,
+                                         uint32_t tile_stride, uint32_t source, RunMap<CHUNK>& s, uint32_t* s_delta) {
     constexpr uint32_t kWords = CHUNK / kWave;
     const uint32_t tid = threadIdx.x;
     for (uint32_t w = tid; w < kWords; w += THREADS) s.begins[w] = 0;
-    if (tid < kWave) {  // whole wavefront
-        const uint32_t upto = q0 == 0 && tiles <= THREADS ? 1 : wave_count_up_to(run_begins, tiles, 0, q0);
-        if (tid == 0) s.first_run = upto != 0 ? upto - 1 : 0;
-    }
     __syncthreads();
     const uint32_t q1 = q0 + count;
     uint32_t listed = 0;
-    for (uint32_t t0 = s.first_run; t0 < tiles; t0 += THREADS) {
+    for (uint32_t t0 = first_run; t0 < tiles; t0 += THREADS) {
         const uint32_t t = t0 + tid;
         uint32_t begin = all, end = all, word = 0;
         if (t < tiles) {
@@ -267,14 +271,15 @@ __device__ __forceinline__ void map_runs(const uint32_t* __restrict__ run_begins
         const uint32_t at = listed + block_exclusive_sum<THREADS>(used ? 1u : 0u, s.wave, &fresh);
         if (used) {
             const uint32_t place = from - q0;
-            if (at < static_cast<uint32_t>(CHUNK)) s_delta[at] = source + t * tile_size + run_place(word) + (from - begin) - place;
+            if (at < static_cast<uint32_t>(CHUNK)) s_delta[at] = source + t * tile_stride + run_place(word) + (from - begin) - place;
             atomicOr(&s.begins[place / kWave], 1ull << (place % kWave));
         }
         listed += fresh;
+        if (t0 + THREADS >= tiles) break;  // whole workgroup
         // past the chunk's end?  the last thread's run is the furthest
-        const bool more = __syncthreads_or(tid == THREADS - 1 && end < q1);
-        if (!more) break;  // whole workgroup
+        if (!__syncthreads_or(tid == THREADS - 1 && end < q1)) break;  // whole workgroup
     }
+    __syncthreads();
     if (tid < kWave) {
         uint32_t carried = 0;
         for (uint32_t w0 = 0; w0 < kWords; w0 += kWave) {
