@@ -1204,12 +1204,24 @@ void launch_sort_triples(hipStream_t stream, idx_t nnz, uint32_t key_bits, const
     radix_sort_triples(stream, nnz, key_bits, keys_in, aux_in, vals_in, keys_out, aux_out, vals_out, value_bytes, t);
 }
 
-size_t index_sort_workspace_bytes(idx_t nnz) { return index_sort_layout(nnz).total; }
+size_t index_sort_workspace_bytes(idx_t nnz, uint32_t major_bits, uint32_t minor_bits) {
+    const size_t passes = index_sort_layout(nnz).total;
+    // either index may be the major one of the call, and a CSR sort has its rows worked out behind the sort's workspace
+    const size_t by_row = partition_sort_pairs_workspace_bytes(nnz, major_bits, minor_bits);
+    const size_t by_column = partition_sort_pairs_workspace_bytes(nnz, minor_bits, major_bits);
+    const size_t sort = (by_row > by_column ? by_row : by_column) + align_up(static_cast<size_t>(nnz) * sizeof(idx_t));
+    return passes > sort ? passes : sort;
+}
 
 void launch_coosort(hipStream_t stream, idx_t major_extent, idx_t minor_extent, idx_t nnz, idx_t* major, idx_t* minor,
                     idx_t* perm, void* workspace) {
     if (nnz == 0) return;
     // indices may be zero- or one-based: keys reach the extent itself in the second case
+    if (partition_sort_pairs_usable(nnz, bit_length(major_extent), bit_length(minor_extent))) {
+        launch_partition_sort_pairs(stream, nnz, bit_length(major_extent), bit_length(minor_extent), major, minor, perm,
+                                    workspace);
+        return;
+    }
     sort_by_two_keys(stream, nnz, bit_length(major_extent), bit_length(minor_extent), major, minor, perm, major, minor,
                      perm, static_cast<char*>(workspace), index_sort_layout(nnz));
 }
@@ -1217,8 +1229,16 @@ void launch_coosort(hipStream_t stream, idx_t major_extent, idx_t minor_extent, 
 void launch_csrsort(hipStream_t stream, idx_t m, idx_t n, idx_t nnz, idx_t base, const idx_t* row_ptr, idx_t* col,
                     idx_t* perm, void* workspace) {
     if (m == 0 || n == 0 || nnz == 0) return;
-    const IndexSortLayout l = index_sort_layout(nnz);
     char* w = static_cast<char*>(workspace);
+    // (the bits of the extents themselves, as the workspace is sized for)
+    if (partition_sort_pairs_usable(nnz, bit_length(m), bit_length(n))) {
+        idx_t* rows = reinterpret_cast<idx_t*>(w);
+        launch_csr2coo(stream, m, nnz, row_ptr, base, rows);
+        launch_partition_sort_pairs(stream, nnz, bit_length(m), bit_length(n), rows, col, perm,
+                                    w + align_up(static_cast<size_t>(nnz) * sizeof(idx_t)));
+        return;
+    }
+    const IndexSortLayout l = index_sort_layout(nnz);
     idx_t* rows = reinterpret_cast<idx_t*>(w + l.spare);  // row of every entry, then the sorted rows
     launch_csr2coo(stream, m, nnz, row_ptr, base, rows);
     sort_by_two_keys(stream, nnz, bit_length(m - 1 + base), bit_length(n - 1 + base), rows, col, perm, rows, col, perm,

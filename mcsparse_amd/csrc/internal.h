@@ -477,27 +477,30 @@ void launch_transposed_products(hipStream_t stream, idx_t m, idx_t n, idx_t nnz,
                                 const idx_t* col, const void* x, void* products, idx_t* col_ptr, size_t value_bytes,
                                 idx_t base, void* workspace);
 
-// Stable sort of (key, aux, value) triples by key (partition.hip), for keys of up to 24 bits (index base taken off).
+// Stable sort of the nonzeros of a CSR matrix where they lie, as (key, row + base, value) triples, by key (partition.hip):
+// key = column index, of up to 24 bits once key_bias is taken off.
 struct PartitionSortArgs {
     const idx_t* keys_in = nullptr;
-    const idx_t* aux_in = nullptr;
-    // csr_rows != 0: the triples are the nonzeros of a CSR matrix of that many rows, and the aux of each is its row + base
     idx_t csr_rows = 0;
     const idx_t* row_ptr = nullptr;
     const void* vals_in = nullptr;
     idx_t base = 0;      // index base of row_ptr and key_ptr
     idx_t key_bias = 0;  // subtracted from the keys before their bits are taken
-    idx_t* keys_out = nullptr;  // may be null
-    idx_t* aux_out = nullptr;
+    idx_t* aux_out = nullptr;   // the rows
     void* vals_out = nullptr;
-    idx_t* key_ptr = nullptr;   // may be null: first place of each of key_count keys and the end, + base
+    idx_t* key_ptr = nullptr;   // first place of each of key_count keys and the end, + base
     idx_t key_count = 0;
 };
 bool partition_sort_usable(idx_t count, uint32_t key_bits);
 size_t partition_sort_workspace_bytes(idx_t count, uint32_t key_bits, size_t value_bytes);
-// The outputs may be the inputs themselves.  value_bytes: 0 or 4, with csr_rows also 8.
+// value_bytes: 0, 4 or 8.
 void launch_partition_sort(hipStream_t stream, idx_t count, uint32_t key_bits, const PartitionSortArgs& a, size_t value_bytes,
                            void* workspace);
+// Stable sort of (major, minor, perm) in place by (major, minor); perm may be null.
+bool partition_sort_pairs_usable(idx_t count, uint32_t major_bits, uint32_t minor_bits);
+size_t partition_sort_pairs_workspace_bytes(idx_t count, uint32_t major_bits, uint32_t minor_bits);
+void launch_partition_sort_pairs(hipStream_t stream, idx_t count, uint32_t major_bits, uint32_t minor_bits, idx_t* major,
+                                 idx_t* minor, idx_t* perm, void* workspace);
 
 // The products of a transposing SpMV ordered by bucket of 2^shift neighbouring columns (index base taken off: bucket b holds columns
 // [b << shift, (b + 1) << shift), at most 256 of them), but only inside tiles of the CSR order: table[b * tiles + t] says
@@ -561,7 +564,8 @@ void launch_sort_triples(hipStream_t stream, idx_t nnz, uint32_t key_bits, const
                          void* workspace);
 
 // ---- index sorts (convert.hip) --------------------------------------------------------------
-size_t index_sort_workspace_bytes(idx_t nnz);
+// major_bits, minor_bits: of the largest indices, base included
+size_t index_sort_workspace_bytes(idx_t nnz, uint32_t major_bits, uint32_t minor_bits);
 // In-place stable sort of COO entries by (major, minor); perm (may be null) moves with them.
 // The extents bound the index values (inclusive, so one-based indices are covered).
 void launch_coosort(hipStream_t stream, idx_t major_extent, idx_t minor_extent, idx_t nnz, idx_t* major, idx_t* minor,

@@ -12,11 +12,12 @@
 //   1. partition_kernel, by the top d1 bits;
 //   2. where more than 2^11 buckets are wanted, repartition_kernel: the same on the tiles of each bucket, whose entries
 //      it gathers from the runs of step 1, by the next d2 bits;
-//   3. bucket_sort_kernel gathers a bucket, which fits LDS, orders it by the last d3 <= 8 bits and writes it where it
-//      belongs, a linear stream again.  Where the keys begin (col_ptr of a CSC) falls out of its digit counts.
-// A key loses the bits that its place already tells: at most 16 of them travel to step 2 and 8 to step 3.
-// A bucket that does not fit LDS (popular keys) is cut into chunks by the oversize_* kernels, which find nothing to do
-// elsewhere.
+//   3. bucket_sort_kernel gathers a bucket, which fits LDS, orders it by the last d3 bits and writes it where it belongs,
+//      a linear stream again.  Where the keys begin (col_ptr of a CSC) falls out of its digit counts.
+// A key loses the bits that its place already tells: at most 16 of them travel to step 2, 8 or 16 to step 3.
+// A sort by two keys (the index sorts) partitions by the major key alone: step 3 orders a bucket by the minor key first,
+// then by what is left of the major one, in passes of up to eight bits that stay in LDS.
+// Buckets that do not fit LDS (popular keys) are sorted in chunks by oversize_kernel, which finds nothing to do elsewhere.
 #include "partition_device.h"
 
 namespace mcsp {
@@ -346,21 +347,52 @@ struct SortTables {
     uint32_t* sub_first;
     // buckets of step 3 that do not fit LDS
     unsigned long long* oversize_count;  // buckets | chunks << 32
-    uint2* oversize;                     // {bucket, chunks before}
+    struct OversizeBucket* oversize;
     uint32_t* oversize_begins;           // [chunk][digit]
+    uint32_t* oversize_aux[2];           // where the passes over such a bucket leave its entries in between
+    void* oversize_vals[2];
+    uint16_t* oversize_keys[2];
     uint32_t d1, d2, d3, count;
+    // step 3: `minor_passes` passes of minor_width bits (the last one: what is left) over the minor_bits of aux, then
+    // passes of key_width bits over the d3 bits of the keys
+    uint32_t minor_bits, minor_passes, minor_width, key_width, passes;
 };
+struct SortPass {
+    bool on_aux;
+    uint32_t shift, bits;
+};
+__device__ __forceinline__ SortPass sort_pass(const SortTables& t, uint32_t p) {
+    SortPass s;
+    s.on_aux = p < t.minor_passes;
+    s.shift = s.on_aux ? p * t.minor_width : (p - t.minor_passes) * t.key_width;
+    s.bits = s.on_aux ? min(t.minor_width, t.minor_bits - s.shift) : min(t.key_width, t.d3 - s.shift);
+    return s;
+}
 
 constexpr int kBucketThreads = 512, kBucketItems = 12;
 constexpr uint32_t kBucketRoom = kBucketThreads * kBucketItems;  // entries of the largest bucket that is sorted in LDS
-constexpr uint32_t kMaxD3 = 8;
+constexpr uint32_t kPassBits = 8;  // the most a pass of step 3 takes
+constexpr uint32_t kMaxPasses = 6;   // 24 bits of the minor key and 16 of the major one at most
 constexpr uint32_t kOversizeChunk = kBucketRoom;
 
+// A bucket that does not fit LDS goes through two phases per pass: the digits of its chunks are counted, then the chunks
+// are written where they belong.
+struct OversizeBucket {
+    uint32_t bucket, chunks_before, chunks;
+    uint32_t phase;                     // 2 * passes: sorted
+    uint32_t taken[2 * kMaxPasses];     // chunks of a phase that somebody works on or has done
+    uint32_t done[2 * kMaxPasses];
+};
 __device__ __forceinline__ void note_oversize(const SortTables& t, uint32_t bucket, uint32_t entries) {
     if (entries <= kBucketRoom) return;
-    const unsigned long long chunks = (entries + kOversizeChunk - 1) / kOversizeChunk;
-    const unsigned long long at = atomicAdd(t.oversize_count, chunks << 32 | 1u);  // both at once: chunks ascend with the place
-    t.oversize[static_cast<uint32_t>(at)] = make_uint2(bucket, static_cast<uint32_t>(at >> 32));
+    const uint32_t chunks = (entries + kOversizeChunk - 1) / kOversizeChunk;
+    const unsigned long long at = atomicAdd(t.oversize_count, static_cast<unsigned long long>(chunks) << 32 | 1u);
+    OversizeBucket& o = t.oversize[static_cast<uint32_t>(at)];
+    o.bucket = bucket;
+    o.chunks_before = static_cast<uint32_t>(at >> 32);
+    o.chunks = chunks;
+    o.phase = 0;
+    for (uint32_t p = 0; p < 2 * kMaxPasses; ++p) o.taken[p] = o.done[p] = 0;
 }
 
 // Exclusive sums over the buckets of step 1 (at most 2^11), in one workgroup: of entries, and (two levels) of tiles.
@@ -429,11 +461,11 @@ __global__ __launch_bounds__(kMapBlock) void tile_map_kernel(SortTables t) {
 }
 
 // 118 M entries (19 bytes each): 1.33 GB read, 1.14 GB written in 500 us.
-template <int VB>
+template <int VB, typename Key>
 __global__ __launch_bounds__(kSecondThreads) void repartition_kernel(SortTables t, const uint16_t* __restrict__ keys_in,
                                                                      const uint32_t* __restrict__ aux_in,
                                                                      const void* __restrict__ vals_in,
-                                                                     uint8_t* __restrict__ keys_out,
+                                                                     Key* __restrict__ keys_out,
                                                                      uint32_t* __restrict__ aux_out,
                                                                      void* __restrict__ vals_out, uint32_t max_tiles,
                                                                      uint32_t xcds) {
@@ -565,17 +597,21 @@ __device__ __forceinline__ void write_key_ptr(const SortOutput& out, uint32_t su
 
 struct BucketLds {
     __align__(16) uint32_t buf[kBucketRoom];
-    __align__(16) uint16_t cnt[kBucketThreads / kWave << kMaxD3];
+    __align__(16) uint16_t cnt[kBucketThreads / kWave << kPassBits];
     uint32_t wave[kBucketThreads / kWave];
     RunMap<kBucketRoom> map;
+    __device__ __forceinline__ void clear_counts() {
+        for (uint32_t i = threadIdx.x; i < sizeof(cnt) / 16; i += kBucketThreads) reinterpret_cast<u32x4*>(cnt)[i] = u32x4(0);
+    }
 };
 
-// Sorts a bucket of at most ITEMS * kBucketThreads entries, the runs of which are mapped in LDS.
-template <int VB, int ITEMS>
+// Sorts a bucket of at most ITEMS * kBucketThreads entries, the runs of which are mapped in LDS.  MANY: in several passes.
+template <int VB, typename Key, bool MANY, int ITEMS>
 __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, uint32_t first, uint32_t count,
-                                            const uint8_t* keys_in, const uint32_t* aux_in, const void* vals_in,
+                                            const Key* keys_in, const uint32_t* aux_in, const void* vals_in,
                                             const SortOutput& out, BucketLds& s) {
     typedef typename WordOf<VB>::type word_t;
+    static_assert(!MANY || VB != 8, "64-bit values are sorted in one pass");
     const uint32_t tid = threadIdx.x, wave = tid / kWave;
     uint32_t key[ITEMS], aux[ITEMS];
     word_t val[VB ? ITEMS : 1];
@@ -583,21 +619,12 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
         const uint32_t from = mapped_place(s.map, s.buf, min(wave * ITEMS + i, last_word), count);
-        key[i] = load_at<uint8_t>(keys_in, from);
+        key[i] = load_at<Key>(keys_in, from);
         aux[i] = load_at<uint32_t>(aux_in, from);
         if constexpr (VB != 0) val[i] = load_at<word_t>(vals_in, from);
     }
     uint32_t dest[(ITEMS + 1) / 2];
-    rank_entries<ITEMS, kMaxD3>(count, t.d3, s.cnt, dest, [&](int i) { return key[i]; });
-    __syncthreads();
-    place_digits<kBucketThreads, kMaxD3>(t.d3, s.cnt, s.wave, [&](uint32_t d, uint32_t at, uint32_t) {
-        write_key_ptr(out, sub, t.d3, d, first + at, t.count);
-    });
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i)
-        dest[i / 2] += static_cast<uint32_t>(s.cnt[(wave << kMaxD3) + key[i]]) << (i % 2 * 16);
-
-    // every array: into LDS in its new order, out as a linear stream
+    // into LDS in the new order
     auto ordered = [&](auto word_of) {
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
@@ -605,6 +632,37 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
         }
         __syncthreads();
     };
+    for (uint32_t p = 0;; ++p) {
+        const SortPass pass = MANY ? sort_pass(t, p) : SortPass{false, 0u, t.d3};
+        const uint32_t mask = (1u << pass.bits) - 1u;
+        auto digit = [&](int i) {
+            const uint32_t of_aux = aux[i], of_key = key[i];  // (the values, so that neither array needs an address)
+            return MANY ? ((pass.on_aux ? of_aux : of_key) >> pass.shift) & mask : of_key;
+        };
+        rank_entries<ITEMS, kPassBits>(count, pass.bits, s.cnt, dest, digit);
+        __syncthreads();
+        place_digits<kBucketThreads, kPassBits>(pass.bits, s.cnt, s.wave, [&](uint32_t d, uint32_t at, uint32_t) {
+            if (!MANY) write_key_ptr(out, sub, t.d3, d, first + at, t.count);
+        });
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i)
+            dest[i / 2] += static_cast<uint32_t>(s.cnt[(wave << kPassBits) + digit(i)]) << (i % 2 * 16);
+        if (!MANY || p + 1 == t.passes) break;
+        auto back = [&](uint32_t (&word)[ITEMS]) {
+            ordered([&](int i) { return word[i]; });
+#pragma unroll
+            for (int i = 0; i < ITEMS; ++i) word[i] = s.buf[slab_place(ITEMS, i)];
+            __syncthreads();
+        };
+        if constexpr (MANY) {
+            back(aux);
+            back(key);
+            if constexpr (VB == 4) back(val);
+            s.clear_counts();
+            __syncthreads();
+        }
+    }
+    // every array out as a linear stream
     auto stream_out = [&](auto store) {
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
@@ -637,165 +695,204 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
 // A workgroup per bucket.  118 M entries (17 bytes each) in buckets of 3600: 445 us, bound by vector instructions as much
 // as by memory (86 % of the cycles, 4.6 TB/s); so most buckets, below two thirds of the room, run a version without the
 // last third of the items (458 -> 445 us).
-template <int VB>
-__global__ __launch_bounds__(kBucketThreads, VB == 8 ? 6 : 8) void bucket_sort_kernel(SortTables t, const uint8_t* __restrict__ keys_in,
-                                                                     const uint32_t* __restrict__ aux_in,
-                                                                     const void* __restrict__ vals_in, SortOutput out,
-                                                                     uint32_t buckets, uint32_t xcds) {
+template <int VB, typename Key, bool MANY>
+__global__ __launch_bounds__(kBucketThreads, VB == 8 ? 6 : 8) void bucket_sort_kernel(SortTables t, const Key* __restrict__ keys_in,
+                                                                                      const uint32_t* __restrict__ aux_in,
+                                                                                      const void* __restrict__ vals_in,
+                                                                                      SortOutput out, uint32_t buckets,
+                                                                                      uint32_t xcds) {
     constexpr int kUsualItems = kBucketItems * 2 / 3;
     __shared__ BucketLds s;
     const uint32_t sub = tile_of_block(buckets, xcds);
     if (sub >= buckets) return;  // whole workgroup
     const uint32_t tid = threadIdx.x;
     const uint32_t first = t.sub_first[sub], count = t.sub_first[sub + 1] - first;
-    if (count > kBucketRoom) return;  // whole workgroup: the oversize kernels' work
+    if (count > kBucketRoom) return;  // whole workgroup: oversize_kernel's work
     if (count == 0) {
-        for (uint32_t d = tid; d < (1u << t.d3); d += kBucketThreads) write_key_ptr(out, sub, t.d3, d, first, t.count);
+        for (uint32_t d = tid; d < (1u << t.d3) && !MANY; d += kBucketThreads) write_key_ptr(out, sub, t.d3, d, first, t.count);
         return;
     }
-    for (uint32_t i = tid; i < sizeof(s.cnt) / 16; i += kBucketThreads) reinterpret_cast<u32x4*>(s.cnt)[i] = u32x4(0);
+    s.clear_counts();
     const BucketRuns runs = runs_of_bucket(t, sub);
     map_runs<kBucketThreads, kBucketRoom>(runs.begins, runs.table, runs.tiles, count, 0, count, 0, runs.places, runs.source,
                                           s.map, s.buf);
     if (count <= static_cast<uint32_t>(kUsualItems * kBucketThreads))
-        sort_bucket<VB, kUsualItems>(t, sub, first, count, keys_in, aux_in, vals_in, out, s);
+        sort_bucket<VB, Key, MANY, kUsualItems>(t, sub, first, count, keys_in, aux_in, vals_in, out, s);
     else
-        sort_bucket<VB, kBucketItems>(t, sub, first, count, keys_in, aux_in, vals_in, out, s);
+        sort_bucket<VB, Key, MANY, kBucketItems>(t, sub, first, count, keys_in, aux_in, vals_in, out, s);
 }
 
 // ---- buckets that do not fit LDS -------------------------------------------------------------------------------
-// In chunks of kOversizeChunk entries: the digits of every chunk are counted, the counts of a bucket's chunks are
-// added up digit by digit, and every chunk is written from there.
-struct OversizeChunk {
-    uint32_t bucket, chunk, all, q0, count;
-};
-__device__ __forceinline__ OversizeChunk oversize_chunk(const SortTables& t, uint32_t c, uint32_t listed) {
-    uint32_t lo = 0, hi = listed;  // the last listed bucket whose chunks begin at or before c
-    while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) / 2;
-        if (t.oversize[mid].y <= c) lo = mid; else hi = mid;
-    }
-    OversizeChunk k;
-    k.bucket = t.oversize[lo].x;
-    k.chunk = c - t.oversize[lo].y;
-    k.all = t.sub_first[k.bucket + 1] - t.sub_first[k.bucket];
-    k.q0 = k.chunk * kOversizeChunk;
-    k.count = min(k.all - k.q0, kOversizeChunk);
-    return k;
-}
+// One launch works on all of them.  A workgroup takes the next chunk of any listed bucket's current phase; whoever
+// finishes a phase's last chunk turns the counts into places (counting phases) and opens the next phase.  A workgroup that
+// finds no chunk to take looks again until every bucket is sorted: it only ever waits for chunks that running workgroups
+// have taken, so the wait ends whether or not the other workgroups of the grid are resident.
 constexpr uint32_t kOversizeGrid = 512;
 
-__global__ __launch_bounds__(kBucketThreads) void oversize_count_kernel(SortTables t, const uint8_t* __restrict__ keys_in) {
-    const unsigned long long counted = *t.oversize_count;
-    const uint32_t listed = static_cast<uint32_t>(counted), chunks = static_cast<uint32_t>(counted >> 32);
-    if (blockIdx.x >= chunks) return;  // whole workgroup
-    __shared__ __align__(16) uint32_t s_delta[kOversizeChunk];
-    __shared__ uint32_t s_count[1 << kMaxD3];
-    __shared__ RunMap<kOversizeChunk> s_map;
-    for (uint32_t c = blockIdx.x; c < chunks; c += gridDim.x) {
-        const OversizeChunk k = oversize_chunk(t, c, listed);
-        const BucketRuns runs = runs_of_bucket(t, k.bucket);
-        for (uint32_t d = threadIdx.x; d < (1u << kMaxD3); d += kBucketThreads) s_count[d] = 0;
-        map_runs<kBucketThreads, kOversizeChunk>(runs.begins, runs.table, runs.tiles, k.all, k.q0, k.count,
-                                                 find_first_run(runs.begins, runs.tiles, k.q0), runs.places, runs.source, s_map,
-                                                 s_delta);
-        for (uint32_t w = threadIdx.x / kWave; w * kWave < k.count; w += kBucketThreads / kWave) {
-            const uint32_t from = mapped_place(s_map, s_delta, w, k.count);
-            if (w * kWave + threadIdx.x % kWave < k.count) atomicAdd(&s_count[keys_in[from]], 1u);
+struct OversizeWork {
+    uint32_t listed_at, phase, chunk, found;
+};
+__device__ __forceinline__ OversizeWork find_oversize_work(const SortTables& t, uint32_t listed, uint32_t start) {
+    OversizeWork w = {0, 0, 0, 0};
+    bool all_sorted = false;
+    while (!all_sorted) {
+        all_sorted = true;
+        for (uint32_t i = 0; i < listed; ++i) {
+            const uint32_t k = (start + i) % listed;
+            OversizeBucket& o = t.oversize[k];
+            const uint32_t phase = __hip_atomic_load(&o.phase, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (phase >= 2 * t.passes) continue;
+            all_sorted = false;
+            if (__hip_atomic_load(&o.taken[phase], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= o.chunks) continue;
+            const uint32_t c = __hip_atomic_fetch_add(&o.taken[phase], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (c < o.chunks) {
+                w.listed_at = k;
+                w.phase = phase;
+                w.chunk = c;
+                w.found = 1;
+                return w;
+            }
         }
-        __syncthreads();
-        for (uint32_t d = threadIdx.x; d < (1u << t.d3); d += kBucketThreads)
-            t.oversize_begins[(static_cast<uint64_t>(c) << t.d3) + d] = s_count[d];
-        __syncthreads();
+        __builtin_amdgcn_s_sleep(32);
     }
+    return w;
 }
 
-// A workgroup per oversize bucket: per digit the counts of the chunks become places in the output.  The chunks are
-// dealt to kSubBlock / 256 shares of a digit's thread each.
-__global__ __launch_bounds__(kSubBlock) void oversize_begins_kernel(SortTables t, SortOutput out) {
-    constexpr uint32_t kDigits = 1 << kMaxD3, kShares = kSubBlock / kDigits;
-    __shared__ uint32_t s_sum[kShares][kDigits];
-    __shared__ uint32_t s_wave[kSubBlock / kWave];
-    const unsigned long long counted = *t.oversize_count;
-    const uint32_t listed = static_cast<uint32_t>(counted), all_chunks = static_cast<uint32_t>(counted >> 32);
+// The counts of a bucket's chunks, digit by digit, become places in its stretch of the output.
+__device__ __forceinline__ void place_chunks(const SortTables& t, const OversizeBucket& o, const SortOutput& out, bool write_ptr,
+                                             uint32_t bits, uint32_t (&s_sum)[kBucketThreads], uint32_t* s_wave) {
+    constexpr uint32_t kDigits = 1 << kPassBits, kShares = kBucketThreads / kDigits;  // threads per digit
     const uint32_t d = threadIdx.x % kDigits, share = threadIdx.x / kDigits;
-    for (uint32_t k = blockIdx.x; k < listed; k += gridDim.x) {
-        const uint32_t bucket = t.oversize[k].x, c0 = t.oversize[k].y;
-        const uint32_t c1 = k + 1 < listed ? t.oversize[k + 1].y : all_chunks;
-        const uint32_t mine = (c1 - c0 + kShares - 1) / kShares;
-        const uint32_t from = min(c0 + share * mine, c1), to = min(from + mine, c1);
-        uint32_t* column = t.oversize_begins + d;
-        const bool exists = d < (1u << t.d3);
-        uint32_t sum = 0;
+    const uint32_t mine = (o.chunks + kShares - 1) / kShares;
+    const uint32_t from = min(share * mine, o.chunks), to = min(from + mine, o.chunks);
+    uint32_t* column = t.oversize_begins + (static_cast<uint64_t>(o.chunks_before) << kPassBits) + d;
+    uint32_t sum = 0;
 #pragma unroll 8
-        for (uint32_t c = from; c < to; ++c) sum += exists ? column[static_cast<uint64_t>(c) << t.d3] : 0u;
-        s_sum[share][d] = sum;
-        __syncthreads();
-        uint32_t total = 0, before = 0;
-        for (uint32_t s = 0; s < kShares; ++s) {
-            if (s == share) before = total;
-            total += s_sum[s][d];
-        }
-        const uint32_t first = t.sub_first[bucket] + block_exclusive_sum<kSubBlock>(share == 0 ? total : 0u, s_wave);
-        if (share == 0) {
-            s_sum[0][d] = first;  // (its own sum has been read by all: the barrier in the scan)
-            if (exists) write_key_ptr(out, bucket, t.d3, d, first, t.count);
-        }
-        __syncthreads();
-        uint32_t at = s_sum[0][d] + before;
-        for (uint32_t c = from; c < to && exists; ++c) {
-            uint32_t* word = column + (static_cast<uint64_t>(c) << t.d3);
-            const uint32_t n = *word;
-            *word = at;
-            at += n;
-        }
-        __syncthreads();
+    for (uint32_t c = from; c < to; ++c) sum += column[static_cast<uint64_t>(c) << kPassBits];
+    s_sum[threadIdx.x] = sum;
+    __syncthreads();
+    uint32_t total = 0, before = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kShares; ++k) {
+        if (k == share) before = total;
+        total += s_sum[k * kDigits + d];
+    }
+    const uint32_t first = t.sub_first[o.bucket] + block_exclusive_sum<kBucketThreads>(share == 0 ? total : 0u, s_wave);
+    if (share == 0) {
+        s_sum[d] = first;  // (every thread has read the sums: the barrier in the scan)
+        if (write_ptr && d < (1u << bits)) write_key_ptr(out, o.bucket, t.d3, d, first, t.count);
+    }
+    __syncthreads();
+    uint32_t at = s_sum[d] + before;
+    for (uint32_t c = from; c < to; ++c) {
+        uint32_t* word = column + (static_cast<uint64_t>(c) << kPassBits);
+        const uint32_t n = *word;
+        *word = at;
+        at += n;
     }
 }
 
-template <int VB>
-__global__ __launch_bounds__(kBucketThreads) void oversize_sort_kernel(SortTables t, const uint8_t* __restrict__ keys_in,
-                                                                       const uint32_t* __restrict__ aux_in,
-                                                                       const void* __restrict__ vals_in, SortOutput out) {
-    constexpr int kWaves = kBucketThreads / kWave;
+template <int VB, typename Key>
+__global__ __launch_bounds__(kBucketThreads) void oversize_kernel(SortTables t, const Key* __restrict__ keys_in,
+                                                                  const uint32_t* __restrict__ aux_in,
+                                                                  const void* __restrict__ vals_in, SortOutput out) {
     typedef typename WordOf<VB>::type word_t;
     const unsigned long long counted = *t.oversize_count;
-    const uint32_t listed = static_cast<uint32_t>(counted), chunks = static_cast<uint32_t>(counted >> 32);
-    if (blockIdx.x >= chunks) return;  // whole workgroup
-    __shared__ __align__(16) uint32_t s_delta[kOversizeChunk];
-    __shared__ __align__(16) uint16_t s_cnt[kWaves << kMaxD3];
-    __shared__ uint32_t s_to[1 << kMaxD3];  // output place of a digit's first entry, less its place in the chunk
-    __shared__ uint32_t s_wave[kWaves];
-    __shared__ RunMap<kOversizeChunk> s_map;
-    const uint32_t wave = threadIdx.x / kWave;
-    for (uint32_t c = blockIdx.x; c < chunks; c += gridDim.x) {
-        const OversizeChunk k = oversize_chunk(t, c, listed);
-        const BucketRuns runs = runs_of_bucket(t, k.bucket);
-        for (uint32_t i = threadIdx.x; i < sizeof(s_cnt) / 16; i += kBucketThreads) reinterpret_cast<u32x4*>(s_cnt)[i] = u32x4(0);
-        map_runs<kBucketThreads, kOversizeChunk>(runs.begins, runs.table, runs.tiles, k.all, k.q0, k.count,
-                                                 find_first_run(runs.begins, runs.tiles, k.q0), runs.places, runs.source, s_map,
-                                                 s_delta);
-        const uint32_t last_word = (k.count - 1) / kWave;
-        uint32_t key[kBucketItems], from[kBucketItems];
-#pragma unroll
-        for (int i = 0; i < kBucketItems; ++i) {
-            from[i] = mapped_place(s_map, s_delta, min(wave * kBucketItems + i, last_word), k.count);
-            key[i] = keys_in[from[i]];
-        }
-        uint32_t dest[kBucketItems / 2];
-        rank_entries<kBucketItems, kMaxD3>(k.count, t.d3, s_cnt, dest, [&](int i) { return key[i]; });
+    const uint32_t listed = static_cast<uint32_t>(counted);
+    if (blockIdx.x >= static_cast<uint32_t>(counted >> 32)) return;  // whole workgroup: more workgroups than chunks
+    __shared__ BucketLds s;
+    __shared__ uint32_t s_count[1 << kPassBits];
+    __shared__ uint32_t s_sum[kBucketThreads];
+    __shared__ OversizeWork s_work;
+    __shared__ uint32_t s_last;
+    const uint32_t tid = threadIdx.x, wave = tid / kWave;
+    while (true) {
+        if (tid == 0) s_work = find_oversize_work(t, listed, blockIdx.x);
         __syncthreads();
-        place_digits<kBucketThreads, kMaxD3>(t.d3, s_cnt, s_wave, [&](uint32_t d, uint32_t at, uint32_t) {
-            s_to[d] = t.oversize_begins[(static_cast<uint64_t>(c) << t.d3) + d] - at;
-        });
+        const OversizeWork work = s_work;
+        if (work.found == 0) return;  // whole workgroup
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // what the phase before has written
+        OversizeBucket& o = t.oversize[work.listed_at];
+        const uint32_t p = work.phase / 2;
+        const bool counting = work.phase % 2 == 0;
+        const SortPass pass = sort_pass(t, p);
+        const uint32_t mask = (1u << pass.bits) - 1u;
+        const uint32_t first = t.sub_first[o.bucket], all = t.sub_first[o.bucket + 1] - first;
+        const uint32_t q0 = work.chunk * kOversizeChunk, count = min(all - q0, kOversizeChunk);
+        uint32_t* begins = t.oversize_begins + (static_cast<uint64_t>(o.chunks_before + work.chunk) << kPassBits);
+        s.clear_counts();
+        for (uint32_t d = tid; d < (1u << kPassBits); d += kBucketThreads) s_count[d] = 0;
+        // the first pass reads the runs, the others what the one before has left in the bucket's stretch
+        const BucketRuns runs = runs_of_bucket(t, o.bucket);
+        if (p == 0)
+            map_runs<kBucketThreads, kBucketRoom>(runs.begins, runs.table, runs.tiles, all, q0, count,
+                                                  find_first_run(runs.begins, runs.tiles, q0), runs.places, runs.source, s.map,
+                                                  s.buf);
+        else
+            __syncthreads();
+        uint32_t key[kBucketItems], aux[kBucketItems];
+        word_t val[VB ? kBucketItems : 1];
+        const uint32_t last_word = (count - 1) / kWave;
 #pragma unroll
         for (int i = 0; i < kBucketItems; ++i) {
-            if (in_slab(kBucketItems, i, k.count)) {
-                const uint32_t to = s_to[key[i]] + s_cnt[(wave << kMaxD3) + key[i]] + ((dest[i / 2] >> (i % 2 * 16)) & 0xffffu);
-                out.aux[to] = load_at<uint32_t>(aux_in, from[i]);
-                if constexpr (VB != 0) static_cast<word_t*>(out.vals)[to] = load_at<word_t>(vals_in, from[i]);
-                if (out.keys != nullptr) out.keys[to] = (k.bucket << t.d3) + key[i] + out.key_bias;
+            if (p == 0) {
+                const uint32_t from = mapped_place(s.map, s.buf, min(wave * kBucketItems + i, last_word), count);
+                key[i] = load_at<Key>(keys_in, from);
+                aux[i] = load_at<uint32_t>(aux_in, from);
+                if constexpr (VB != 0) val[i] = load_at<word_t>(vals_in, from);
+            } else {
+                const uint32_t from = first + q0 + min(slab_place(kBucketItems, i), count - 1);
+                key[i] = load_at<uint16_t>(t.oversize_keys[(p - 1) % 2], from);
+                aux[i] = load_at<uint32_t>(t.oversize_aux[(p - 1) % 2], from);
+                if constexpr (VB != 0) val[i] = load_at<word_t>(t.oversize_vals[(p - 1) % 2], from);
             }
+        }
+        auto digit = [&](int i) {
+            const uint32_t of_aux = aux[i], of_key = key[i];
+            return ((pass.on_aux ? of_aux : of_key) >> pass.shift) & mask;
+        };
+        if (counting) {
+#pragma unroll
+            for (int i = 0; i < kBucketItems; ++i) {
+                if (in_slab(kBucketItems, i, count)) atomicAdd(&s_count[digit(i)], 1u);
+            }
+            __syncthreads();
+            for (uint32_t d = tid; d < (1u << kPassBits); d += kBucketThreads) begins[d] = s_count[d];
+        } else {
+            const bool to_output = p + 1 == t.passes;
+            uint32_t* aux_to = to_output ? out.aux : t.oversize_aux[p % 2];
+            word_t* vals_to = static_cast<word_t*>(to_output ? out.vals : t.oversize_vals[p % 2]);
+            uint32_t dest[kBucketItems / 2];
+            rank_entries<kBucketItems, kPassBits>(count, pass.bits, s.cnt, dest, digit);
+            __syncthreads();
+            // (s_count: where the digit's first entry of the chunk goes, less its place in the chunk)
+            place_digits<kBucketThreads, kPassBits>(pass.bits, s.cnt, s.wave,
+                                                    [&](uint32_t d, uint32_t at, uint32_t) { s_count[d] = begins[d] - at; });
+#pragma unroll
+            for (int i = 0; i < kBucketItems; ++i) {
+                if (in_slab(kBucketItems, i, count)) {
+                    const uint32_t d = digit(i);
+                    const uint32_t to = s_count[d] + s.cnt[(wave << kPassBits) + d] + ((dest[i / 2] >> (i % 2 * 16)) & 0xffffu);
+                    aux_to[to] = aux[i];
+                    if constexpr (VB != 0) vals_to[to] = val[i];
+                    if (!to_output) t.oversize_keys[p % 2][to] = static_cast<uint16_t>(key[i]);
+                    else if (out.keys != nullptr) out.keys[to] = (o.bucket << t.d3) + key[i] + out.key_bias;
+                }
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        __syncthreads();
+        if (tid == 0)
+            s_last = __hip_atomic_fetch_add(&o.done[work.phase], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == o.chunks;
+        __syncthreads();
+        if (s_last != 0) {  // whole workgroup
+            if (counting) {
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+                place_chunks(t, o, out, t.passes == 1, pass.bits, s_sum, s.wave);
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+                __syncthreads();
+            }
+            if (tid == 0) __hip_atomic_store(&o.phase, work.phase + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         __syncthreads();
     }
@@ -860,24 +957,54 @@ constexpr uint32_t kMostEntries = kBucketRoom * 3 / 4 << kMaxTwoLevelBits;  // m
 
 struct SortShape {
     uint32_t d1, d2, d3, tile_size, tiles1, max_tiles2;
+    uint32_t minor_bits;  // kNoMinorKey: a sort by one key
 };
-bool sort_shape(uint32_t count, uint32_t key_bits, SortShape* s) {
+constexpr uint32_t kNoMinorKey = ~0u;
+constexpr uint32_t kMaxKeyRest = 16;  // bits of a key behind those of step 1: it travels in 16
+bool sort_shape(uint32_t count, uint32_t key_bits, uint32_t minor_bits, SortShape* s) {
     // (and every array of the sort stays below 4 GiB)
-    if (count == 0 || count > kMostEntries || key_bits > kMaxTwoLevelBits + kMaxD3) return false;
-    uint32_t bits = key_bits > kMaxD3 ? key_bits - kMaxD3 : 0;
+    if (count == 0 || count > kMostEntries) return false;
+    uint32_t bits = 0;
     while (bits < key_bits && bits < kMaxTwoLevelBits && (static_cast<uint64_t>(kBucketWanted) << bits) < count) ++bits;
-    s->d1 = bits <= kMaxOneLevelBits ? bits : (bits + 1) / 2;
+    auto first_level = [&]() { return bits <= kMaxOneLevelBits ? bits : (bits + 1) / 2; };
+    if (minor_bits == kNoMinorKey) {
+        // one pass over a bucket, so that its digit counts say where every key begins
+        if (key_bits > kMaxTwoLevelBits + kPassBits) return false;
+        const uint32_t least = key_bits > kPassBits ? key_bits - kPassBits : 0;
+        // many more keys than entries: buckets of a few entries each, a workgroup for every one of them (2^22 columns,
+        // 1 M entries: 210 us; the passes of the LSD sort take 170)
+        if (least > kMaxOneLevelBits && (static_cast<uint64_t>(count) << 4) < static_cast<uint64_t>(kBucketWanted) << least) return false;
+        bits = bits > least ? bits : least;
+    } else {
+        if (minor_bits > 24) return false;
+        while (first_level() + kMaxKeyRest < key_bits && bits < kMaxTwoLevelBits) ++bits;
+        if (first_level() + kMaxKeyRest < key_bits) return false;
+    }
+    s->d1 = first_level();
     s->d2 = bits - s->d1;
     s->d3 = key_bits - bits;
+    s->minor_bits = minor_bits;
     s->tile_size = tile_size_for(count);
     s->tiles1 = tiles_of(count, s->tile_size);
     s->max_tiles2 = s->d2 != 0 ? count / kSecondTile + (1u << s->d1) : 0;
     return true;
 }
+void sort_passes(const SortShape& s, SortTables* t) {
+    const uint32_t minor = s.minor_bits == kNoMinorKey ? 0 : s.minor_bits;
+    auto passes_for = [](uint32_t bits) { return (bits + kPassBits - 1) / kPassBits; };
+    auto width_for = [&](uint32_t bits) { return bits == 0 ? 0 : (bits + passes_for(bits) - 1) / passes_for(bits); };
+    t->minor_bits = minor;
+    t->minor_passes = passes_for(minor);
+    t->minor_width = width_for(minor);
+    t->key_width = width_for(s.d3);
+    t->passes = t->minor_passes + passes_for(s.d3);
+    if (t->passes == 0) t->passes = 1;  // everything in order already: one pass over no bits
+}
 
 struct SortLayout {
     size_t keys1, aux1, vals1, keys2, aux2, vals2, table1, begins1, totals1, tile_rows, table2, begins2, bucket_first,
-        tile_first, first_runs, tile_map, sub_first, oversize_count, oversize, oversize_begins, total;
+        tile_first, first_runs, tile_map, sub_first, oversize_count, oversize, oversize_begins, oversize_keys[2], oversize_aux[2],
+        oversize_vals[2], total;
 };
 SortLayout sort_layout(uint32_t count, const SortShape& s, size_t value_bytes) {
     const size_t places1 = static_cast<size_t>(s.tiles1) * s.tile_size;
@@ -892,10 +1019,10 @@ SortLayout sort_layout(uint32_t count, const SortShape& s, size_t value_bytes) {
         off += align_up(bytes);
         return at;
     };
-    l.keys1 = take(places1 * (s.d2 != 0 ? sizeof(uint16_t) : sizeof(uint8_t)));
+    l.keys1 = take(places1 * (s.d2 + s.d3 > 8 ? sizeof(uint16_t) : sizeof(uint8_t)));
     l.aux1 = take(places1 * sizeof(uint32_t));
     l.vals1 = take(places1 * value_bytes);
-    l.keys2 = take(places2);
+    l.keys2 = take(places2 * (s.d3 > 8 ? sizeof(uint16_t) : sizeof(uint8_t)));
     l.aux2 = take(places2 * sizeof(uint32_t));
     l.vals2 = take(places2 * value_bytes);
     l.table1 = take(runs1 * sizeof(uint32_t));
@@ -910,8 +1037,16 @@ SortLayout sort_layout(uint32_t count, const SortShape& s, size_t value_bytes) {
     l.tile_map = take(static_cast<size_t>(s.max_tiles2) * sizeof(uint2));
     l.sub_first = take((subs + 1) * sizeof(uint32_t));
     l.oversize_count = take(sizeof(unsigned long long));
-    l.oversize = take((static_cast<size_t>(count) / kBucketRoom + 1) * sizeof(uint2));
-    l.oversize_begins = take((chunks << s.d3) * sizeof(uint32_t));
+    l.oversize = take((static_cast<size_t>(count) / kBucketRoom + 1) * sizeof(OversizeBucket));
+    l.oversize_begins = take((chunks << kPassBits) * sizeof(uint32_t));
+    SortTables passes;
+    sort_passes(s, &passes);
+    for (uint32_t k = 0; k < 2; ++k) {
+        const size_t between = count > kBucketRoom && passes.passes > k + 1 ? count : 0;
+        l.oversize_keys[k] = take(between * sizeof(uint16_t));
+        l.oversize_aux[k] = take(between * sizeof(uint32_t));
+        l.oversize_vals[k] = take(between * value_bytes);
+    }
     l.total = off;
     return l;
 }
@@ -939,62 +1074,86 @@ void launch_sort(hipStream_t stream, EntrySource in, const SortShape& s, const S
     t.tile_map = reinterpret_cast<uint2*>(w + l.tile_map);
     t.sub_first = words(l.sub_first);
     t.oversize_count = reinterpret_cast<unsigned long long*>(w + l.oversize_count);
-    t.oversize = reinterpret_cast<uint2*>(w + l.oversize);
+    t.oversize = reinterpret_cast<OversizeBucket*>(w + l.oversize);
+    for (uint32_t k = 0; k < 2; ++k) {
+        t.oversize_keys[k] = reinterpret_cast<uint16_t*>(w + l.oversize_keys[k]);
+        t.oversize_aux[k] = words(l.oversize_aux[k]);
+        t.oversize_vals[k] = w + l.oversize_vals[k];
+    }
+    sort_passes(s, &t);
     t.oversize_begins = words(l.oversize_begins);
     t.d1 = s.d1;
     t.d2 = s.d2;
     t.d3 = s.d3;
     t.count = in.count;
     const uint32_t shift = s.d2 + s.d3;
-    auto* partition = s.d2 != 0 ? launch_partition<VB, KIND, 8, uint16_t>
-                      : s.d1 <= 8 ? launch_partition<VB, KIND, 8, uint8_t> : launch_partition<VB, KIND, kMaxOneLevelBits, uint8_t>;
+    constexpr bool kMany = KIND == kPlain;  // the sorts by two keys
+    const bool short_keys1 = shift <= 8, short_keys2 = s.d3 <= 8;
+    auto* partition = s.d1 <= 8 ? (short_keys1 ? launch_partition<VB, KIND, 8, uint8_t> : launch_partition<VB, KIND, 8, uint16_t>)
+                                : (short_keys1 ? launch_partition<VB, KIND, kMaxOneLevelBits, uint8_t>
+                                               : launch_partition<VB, KIND, kMaxOneLevelBits, uint16_t>);
     partition(stream, in, shift, s.d1, s.tile_size, w + l.keys1, words(l.aux1), w + l.vals1, words(l.table1));
     hipLaunchKernelGGL(run_begins_kernel, dim3(1u << s.d1), dim3(kScanBlock), 0, stream, s.tiles1, t.table1,
                        words(l.begins1), words(l.totals1), s.d2 != 0 ? words(l.first_runs) : nullptr);
     hipLaunchKernelGGL(sort_plan_kernel, dim3(1), dim3(kPlanBlock), 0, stream, t);
-    const uint8_t* keys = reinterpret_cast<const uint8_t*>(w + l.keys1);
+    const void* keys = w + l.keys1;
     const uint32_t* aux = words(l.aux1);
     const void* vals = w + l.vals1;
     if (s.d2 != 0) {
         hipLaunchKernelGGL(tile_map_kernel, dim3((s.max_tiles2 + kMapBlock - 1) / kMapBlock), dim3(kMapBlock), 0, stream, t);
-        hipLaunchKernelGGL((repartition_kernel<VB>), dim3((s.max_tiles2 + xcds - 1) / xcds * xcds), dim3(kSecondThreads), 0,
-                           stream, t, reinterpret_cast<const uint16_t*>(w + l.keys1), aux, vals,
-                           reinterpret_cast<uint8_t*>(w + l.keys2), words(l.aux2), w + l.vals2, s.max_tiles2, xcds);
+        const dim3 grid((s.max_tiles2 + xcds - 1) / xcds * xcds);
+        const uint16_t* keys1 = reinterpret_cast<const uint16_t*>(keys);
+        if (short_keys2)
+            hipLaunchKernelGGL((repartition_kernel<VB, uint8_t>), grid, dim3(kSecondThreads), 0, stream, t, keys1, aux, vals,
+                               reinterpret_cast<uint8_t*>(w + l.keys2), words(l.aux2), w + l.vals2, s.max_tiles2, xcds);
+        else if constexpr (kMany)
+            hipLaunchKernelGGL((repartition_kernel<VB, uint16_t>), grid, dim3(kSecondThreads), 0, stream, t, keys1, aux, vals,
+                               reinterpret_cast<uint16_t*>(w + l.keys2), words(l.aux2), w + l.vals2, s.max_tiles2, xcds);
         hipLaunchKernelGGL(sub_begins_kernel, dim3(1u << s.d1), dim3(kSubBlock), 0, stream, t);
-        keys = reinterpret_cast<const uint8_t*>(w + l.keys2);
+        keys = w + l.keys2;
         aux = words(l.aux2);
         vals = w + l.vals2;
     }
     const uint32_t buckets = 1u << (s.d1 + s.d2);
-    hipLaunchKernelGGL((bucket_sort_kernel<VB>), dim3((buckets + xcds - 1) / xcds * xcds), dim3(kBucketThreads), 0, stream, t,
-                       keys, aux, vals, out, buckets, xcds);
-    if (in.count > kBucketRoom) {  // else no bucket is larger than that
-        hipLaunchKernelGGL(oversize_count_kernel, dim3(kOversizeGrid), dim3(kBucketThreads), 0, stream, t, keys);
-        hipLaunchKernelGGL(oversize_begins_kernel, dim3(kOversizeGrid / 4), dim3(kSubBlock), 0, stream, t, out);
-        hipLaunchKernelGGL((oversize_sort_kernel<VB>), dim3(kOversizeGrid), dim3(kBucketThreads), 0, stream, t, keys, aux, vals,
-                           out);
-    }
+    const dim3 grid((buckets + xcds - 1) / xcds * xcds);
+    auto sort = [&](auto key) {
+        typedef decltype(key) Key;
+        hipLaunchKernelGGL((bucket_sort_kernel<VB, Key, kMany>), grid, dim3(kBucketThreads), 0, stream, t,
+                           static_cast<const Key*>(keys), aux, vals, out, buckets, xcds);
+        if (in.count > kBucketRoom)  // else no bucket is larger than that
+            hipLaunchKernelGGL((oversize_kernel<VB, Key>), dim3(kOversizeGrid), dim3(kBucketThreads), 0, stream, t,
+                               static_cast<const Key*>(keys), aux, vals, out);
+    };
+    if (short_keys2) sort(uint8_t());
+    else if constexpr (kMany) sort(uint16_t());
 }
 
 }  // namespace
 
 bool partition_sort_usable(idx_t count, uint32_t key_bits) {
     SortShape s;
-    return sort_shape(count, key_bits, &s);
+    return sort_shape(count, key_bits, kNoMinorKey, &s);
 }
-
 size_t partition_sort_workspace_bytes(idx_t count, uint32_t key_bits, size_t value_bytes) {
     SortShape s;
-    return sort_shape(count, key_bits, &s) ? sort_layout(count, s, value_bytes).total : 0;
+    return sort_shape(count, key_bits, kNoMinorKey, &s) ? sort_layout(count, s, value_bytes).total : 0;
+}
+bool partition_sort_pairs_usable(idx_t count, uint32_t major_bits, uint32_t minor_bits) {
+    SortShape s;
+    return sort_shape(count, major_bits, minor_bits, &s);
+}
+size_t partition_sort_pairs_workspace_bytes(idx_t count, uint32_t major_bits, uint32_t minor_bits) {
+    SortShape s;
+    return sort_shape(count, major_bits, minor_bits, &s) ? sort_layout(count, s, sizeof(idx_t)).total : 0;
 }
 
 void launch_partition_sort(hipStream_t stream, idx_t count, uint32_t key_bits, const PartitionSortArgs& a, size_t value_bytes,
                            void* workspace) {
     SortShape s;
-    if (!sort_shape(count, key_bits, &s)) return;
+    if (!sort_shape(count, key_bits, kNoMinorKey, &s)) return;
     EntrySource in;
     in.keys = a.keys_in;
-    in.aux = a.csr_rows != 0 ? a.row_ptr : a.aux_in;
+    in.aux = a.row_ptr;
     in.vals = a.vals_in;
     in.x = nullptr;
     in.count = count;
@@ -1003,21 +1162,32 @@ void launch_partition_sort(hipStream_t stream, idx_t count, uint32_t key_bits, c
     in.base = a.base;
     in.tile_rows = nullptr;
     SortOutput out;
-    out.keys = a.keys_out;
+    out.keys = nullptr;
     out.aux = a.aux_out;
     out.vals = a.vals_out;
     out.key_ptr = a.key_ptr;
     out.key_count = a.key_count;
     out.base = a.base;
     out.key_bias = a.key_bias;
-    char* w = static_cast<char*>(workspace);
-    if (a.csr_rows != 0) {
-        auto* launch = value_bytes == 0 ? launch_sort<0, kCsr> : value_bytes == 4 ? launch_sort<4, kCsr> : launch_sort<8, kCsr>;
-        launch(stream, in, s, out, w);
-    } else {
-        auto* launch = value_bytes == 0 ? launch_sort<0, kPlain> : launch_sort<4, kPlain>;
-        launch(stream, in, s, out, w);
-    }
+    auto* launch = value_bytes == 0 ? launch_sort<0, kCsr> : value_bytes == 4 ? launch_sort<4, kCsr> : launch_sort<8, kCsr>;
+    launch(stream, in, s, out, static_cast<char*>(workspace));
+}
+
+void launch_partition_sort_pairs(hipStream_t stream, idx_t count, uint32_t major_bits, uint32_t minor_bits, idx_t* major,
+                                 idx_t* minor, idx_t* perm, void* workspace) {
+    SortShape s;
+    if (!sort_shape(count, major_bits, minor_bits, &s)) return;
+    EntrySource in = {};
+    in.keys = major;
+    in.aux = minor;
+    in.vals = perm;
+    in.count = count;
+    SortOutput out = {};
+    out.keys = major;
+    out.aux = minor;
+    out.vals = perm;
+    auto* launch = perm == nullptr ? launch_sort<0, kPlain> : launch_sort<4, kPlain>;
+    launch(stream, in, s, out, static_cast<char*>(workspace));
 }
 
 bool bucketed_products_shape(idx_t n, uint32_t* shift) {

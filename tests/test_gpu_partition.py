@@ -1,7 +1,7 @@
 """GPU parity of what is built on the partition of tiles by key bits (csrc/partition.hip), at the sizes where it can go
 wrong: entry counts around a tile, both tile sizes, keys concentrated in a few runs, empty rows.  The transposing
 mcsparseSpMV without a preprocess call is compared exactly (integer-valued operands make any order of summation exact),
-csr2csc bit for bit against the oracle."""
+csr2csc and the index sorts bit for bit against the oracle."""
 import numpy as np
 import pytest
 
@@ -83,3 +83,34 @@ def test_csr2csc_bit_exact(torch_gpu, handle, oracle, dtype, action, kind, m, n,
         assert np.array_equal(o_val.cpu().numpy(), want_val)
     else:
         assert (o_val == -9.0).all()
+
+
+@pytest.mark.parametrize("by", ["row", "column"])
+@pytest.mark.parametrize("with_perm", [True, False])
+@pytest.mark.parametrize("kind,m,n,nnz", [
+    ("uniform", 3, 2, 1), ("uniform", 90, 3000000, 6144), ("uniform", 3000000, 90, 6145), ("few", 40, 50, 70000),
+    ("few", 4000, 70000, 300000), ("band", 300000, 40000, 1000000), ("uniform", 1 << 23, 1 << 22, 100000),
+    ("few", 100000, 1 << 22, ONE_LEVEL_UPTO), ("uniform", 1 << 22, 1 << 20, ONE_LEVEL_UPTO + 1),
+    ("uniform", 1 << 24, 300, 50000),
+])
+def test_coosort_bit_exact(torch_gpu, handle, oracle, by, with_perm, kind, m, n, nnz):
+    torch = torch_gpu
+    a = matrix(kind, m, n, nnz, np.float32, seed=nnz)
+    rng = np.random.default_rng(nnz)
+    order = rng.permutation(nnz)
+    rows = np.repeat(np.arange(m, dtype=np.int32), a.row_lengths())[order]
+    cols, perm = a.col[order], rng.permutation(nnz).astype(np.int32)
+    if kind == "few":  # and one row with a third of all entries
+        rows[rng.random(nnz) < 0.33] = m // 2
+    d_r, d_c, d_p = dev(torch, rows), dev(torch, cols), dev(torch, perm) if with_perm else None
+    st, size = api.sort_buffer_size(handle, "coo", m, n, nnz, d_r, d_c)
+    assert st == api.STATUS_SUCCESS
+    buf = torch.empty(size, dtype=torch.uint8, device="cuda")
+    sort = api.xcoosort_by_row if by == "row" else api.xcoosort_by_column
+    assert sort(handle, m, n, nnz, d_r, d_c, d_p, buf) == api.STATUS_SUCCESS
+    torch.cuda.synchronize()
+    want = np.lexsort((cols, rows) if by == "row" else (rows, cols))  # stable
+    assert np.array_equal(d_r.cpu().numpy(), rows[want])
+    assert np.array_equal(d_c.cpu().numpy(), cols[want])
+    if with_perm:
+        assert np.array_equal(d_p.cpu().numpy(), perm[want])
