@@ -25,9 +25,7 @@ mcspStatus_t sort_buffer_size(mcsparseHandle_t handle, int m, int n, int nnz, co
         *buffer_size = kMinBuffer;
         return MCSP_STATUS_SUCCESS;
     }
-    // (indices may be one-based: the largest is the extent itself)
-    *buffer_size = mcsp::index_sort_workspace_bytes(static_cast<idx_t>(nnz), bit_length(static_cast<uint32_t>(m)),
-                                                    bit_length(static_cast<uint32_t>(n)));
+    *buffer_size = mcsp::index_sort_workspace_bytes(static_cast<idx_t>(nnz), static_cast<idx_t>(m), static_cast<idx_t>(n));
     return MCSP_STATUS_SUCCESS;
 }
 

@@ -1032,7 +1032,7 @@ void launch_coo2csr(hipStream_t stream, idx_t nnz, idx_t m, const idx_t* coo_row
 
 size_t csr2csc_workspace_bytes(idx_t /*m*/, idx_t n, idx_t nnz, size_t value_bytes) {
     const size_t passes = csr2csc_layout(nnz, value_bytes).total;
-    const size_t sort = n != 0 ? partition_sort_workspace_bytes(nnz, bit_length(n - 1), value_bytes) : 0;
+    const size_t sort = n != 0 ? partition_sort_workspace_bytes(nnz, n, value_bytes) : 0;
     return passes > sort ? passes : sort;
 }
 
@@ -1048,7 +1048,7 @@ void launch_csr2csc(hipStream_t stream, idx_t m, idx_t n, idx_t nnz, const void*
                     const idx_t* col, void* csc_val, idx_t* row_ind, idx_t* col_ptr, size_t value_bytes, idx_t base,
                     void* workspace) {
     if (m == 0 || n == 0 || nnz == 0) return;
-    if (partition_sort_usable(nnz, bit_length(n - 1))) {
+    if (partition_sort_usable(nnz, n)) {
         PartitionSortArgs a;
         a.keys_in = col;
         a.csr_rows = m;
@@ -1060,7 +1060,7 @@ void launch_csr2csc(hipStream_t stream, idx_t m, idx_t n, idx_t nnz, const void*
         a.vals_out = csc_val;
         a.key_ptr = col_ptr;
         a.key_count = n;
-        launch_partition_sort(stream, nnz, bit_length(n - 1), a, value_bytes, workspace);
+        launch_partition_sort(stream, nnz, a, value_bytes, workspace);
         return;
     }
     const Csr2CscLayout l = csr2csc_layout(nnz, value_bytes);
@@ -1204,11 +1204,11 @@ void launch_sort_triples(hipStream_t stream, idx_t nnz, uint32_t key_bits, const
     radix_sort_triples(stream, nnz, key_bits, keys_in, aux_in, vals_in, keys_out, aux_out, vals_out, value_bytes, t);
 }
 
-size_t index_sort_workspace_bytes(idx_t nnz, uint32_t major_bits, uint32_t minor_bits) {
+size_t index_sort_workspace_bytes(idx_t nnz, idx_t major_extent, idx_t minor_extent) {
     const size_t passes = index_sort_layout(nnz).total;
     // either index may be the major one of the call, and a CSR sort has its rows worked out behind the sort's workspace
-    const size_t by_row = partition_sort_pairs_workspace_bytes(nnz, major_bits, minor_bits);
-    const size_t by_column = partition_sort_pairs_workspace_bytes(nnz, minor_bits, major_bits);
+    const size_t by_row = partition_sort_pairs_workspace_bytes(nnz, major_extent + 1, minor_extent + 1);
+    const size_t by_column = partition_sort_pairs_workspace_bytes(nnz, minor_extent + 1, major_extent + 1);
     const size_t sort = (by_row > by_column ? by_row : by_column) + align_up(static_cast<size_t>(nnz) * sizeof(idx_t));
     return passes > sort ? passes : sort;
 }
@@ -1217,9 +1217,8 @@ void launch_coosort(hipStream_t stream, idx_t major_extent, idx_t minor_extent, 
                     idx_t* perm, void* workspace) {
     if (nnz == 0) return;
     // indices may be zero- or one-based: keys reach the extent itself in the second case
-    if (partition_sort_pairs_usable(nnz, bit_length(major_extent), bit_length(minor_extent))) {
-        launch_partition_sort_pairs(stream, nnz, bit_length(major_extent), bit_length(minor_extent), major, minor, perm,
-                                    workspace);
+    if (partition_sort_pairs_usable(nnz, major_extent + 1, minor_extent + 1)) {
+        launch_partition_sort_pairs(stream, nnz, major_extent + 1, minor_extent + 1, major, minor, perm, workspace);
         return;
     }
     sort_by_two_keys(stream, nnz, bit_length(major_extent), bit_length(minor_extent), major, minor, perm, major, minor,
@@ -1230,11 +1229,10 @@ void launch_csrsort(hipStream_t stream, idx_t m, idx_t n, idx_t nnz, idx_t base,
                     idx_t* perm, void* workspace) {
     if (m == 0 || n == 0 || nnz == 0) return;
     char* w = static_cast<char*>(workspace);
-    // (the bits of the extents themselves, as the workspace is sized for)
-    if (partition_sort_pairs_usable(nnz, bit_length(m), bit_length(n))) {
+    if (partition_sort_pairs_usable(nnz, m + 1, n + 1)) {
         idx_t* rows = reinterpret_cast<idx_t*>(w);
         launch_csr2coo(stream, m, nnz, row_ptr, base, rows);
-        launch_partition_sort_pairs(stream, nnz, bit_length(m), bit_length(n), rows, col, perm,
+        launch_partition_sort_pairs(stream, nnz, m + 1, n + 1, rows, col, perm,
                                     w + align_up(static_cast<size_t>(nnz) * sizeof(idx_t)));
         return;
     }

@@ -491,15 +491,15 @@ struct PartitionSortArgs {
     idx_t* key_ptr = nullptr;   // first place of each of key_count keys and the end, + base
     idx_t key_count = 0;
 };
-bool partition_sort_usable(idx_t count, uint32_t key_bits);
-size_t partition_sort_workspace_bytes(idx_t count, uint32_t key_bits, size_t value_bytes);
+bool partition_sort_usable(idx_t count, idx_t key_count);
+size_t partition_sort_workspace_bytes(idx_t count, idx_t key_count, size_t value_bytes);
 // value_bytes: 0, 4 or 8.
-void launch_partition_sort(hipStream_t stream, idx_t count, uint32_t key_bits, const PartitionSortArgs& a, size_t value_bytes,
-                           void* workspace);
-// Stable sort of (major, minor, perm) in place by (major, minor); perm may be null.
-bool partition_sort_pairs_usable(idx_t count, uint32_t major_bits, uint32_t minor_bits);
-size_t partition_sort_pairs_workspace_bytes(idx_t count, uint32_t major_bits, uint32_t minor_bits);
-void launch_partition_sort_pairs(hipStream_t stream, idx_t count, uint32_t major_bits, uint32_t minor_bits, idx_t* major,
+void launch_partition_sort(hipStream_t stream, idx_t count, const PartitionSortArgs& a, size_t value_bytes, void* workspace);
+// Stable sort of (major, minor, perm) in place by (major, minor), which are below major_count and minor_count; perm may be
+// null.
+bool partition_sort_pairs_usable(idx_t count, idx_t major_count, idx_t minor_count);
+size_t partition_sort_pairs_workspace_bytes(idx_t count, idx_t major_count, idx_t minor_count);
+void launch_partition_sort_pairs(hipStream_t stream, idx_t count, idx_t major_count, idx_t minor_count, idx_t* major,
                                  idx_t* minor, idx_t* perm, void* workspace);
 
 // The products of a transposing SpMV ordered by bucket of 2^shift neighbouring columns (index base taken off: bucket b holds columns
@@ -511,7 +511,7 @@ void launch_partition_sort_pairs(hipStream_t stream, idx_t count, uint32_t major
 // (more than 2^14 and at most 2^22 columns: a bucket's sums must fit in LDS as doubles).
 constexpr uint32_t kBucketMinKeyBits = 15;
 constexpr uint32_t kBucketMaxShift = 14;
-constexpr uint32_t kBucketTileMin = 2048;  // nonzeros of the smallest tiles
+constexpr uint32_t kBucketTileMin = 4096;  // nonzeros of the smallest tiles
 constexpr uint32_t kBucketRunPad = 4;
 struct BucketedProducts {
     const uint16_t* keys = nullptr;
@@ -564,8 +564,7 @@ void launch_sort_triples(hipStream_t stream, idx_t nnz, uint32_t key_bits, const
                          void* workspace);
 
 // ---- index sorts (convert.hip) --------------------------------------------------------------
-// major_bits, minor_bits: of the largest indices, base included
-size_t index_sort_workspace_bytes(idx_t nnz, uint32_t major_bits, uint32_t minor_bits);
+size_t index_sort_workspace_bytes(idx_t nnz, idx_t major_extent, idx_t minor_extent);
 // In-place stable sort of COO entries by (major, minor); perm (may be null) moves with them.
 // The extents bound the index values (inclusive, so one-based indices are covered).
 void launch_coosort(hipStream_t stream, idx_t major_extent, idx_t minor_extent, idx_t nnz, idx_t* major, idx_t* minor,

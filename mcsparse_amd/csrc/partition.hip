@@ -379,9 +379,10 @@ constexpr uint32_t kOversizeChunk = kBucketRoom;
 // are written where they belong.
 struct OversizeBucket {
     uint32_t bucket, chunks_before, chunks;
-    uint32_t phase;                     // 2 * passes: sorted
-    uint32_t taken[2 * kMaxPasses];     // chunks of a phase that somebody works on or has done
-    uint32_t done[2 * kMaxPasses];
+    // on lines of their own: idle workgroups keep reading `phase`
+    alignas(128) uint32_t phase;                  // 2 * passes: sorted
+    alignas(128) uint32_t taken[2 * kMaxPasses];  // chunks of a phase that somebody works on or has done
+    alignas(128) uint32_t done[2 * kMaxPasses];
 };
 __device__ __forceinline__ void note_oversize(const SortTables& t, uint32_t bucket, uint32_t entries) {
     if (entries <= kBucketRoom) return;
@@ -696,7 +697,7 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
 // as by memory (86 % of the cycles, 4.6 TB/s); so most buckets, below two thirds of the room, run a version without the
 // last third of the items (458 -> 445 us).
 template <int VB, typename Key, bool MANY>
-__global__ __launch_bounds__(kBucketThreads, VB == 8 ? 6 : 8) void bucket_sort_kernel(SortTables t, const Key* __restrict__ keys_in,
+__global__ __launch_bounds__(kBucketThreads, VB == 8 || MANY ? 6 : 8) void bucket_sort_kernel(SortTables t, const Key* __restrict__ keys_in,
                                                                                       const uint32_t* __restrict__ aux_in,
                                                                                       const void* __restrict__ vals_in,
                                                                                       SortOutput out, uint32_t buckets,
@@ -732,30 +733,40 @@ constexpr uint32_t kOversizeGrid = 512;
 struct OversizeWork {
     uint32_t listed_at, phase, chunk, found;
 };
+// For one whole wavefront, which looks at 64 listed buckets at a time, from `start` on; every lane returns the same.
 __device__ __forceinline__ OversizeWork find_oversize_work(const SortTables& t, uint32_t listed, uint32_t start) {
+    const uint32_t lane = threadIdx.x % kWave;
     OversizeWork w = {0, 0, 0, 0};
-    bool all_sorted = false;
-    while (!all_sorted) {
-        all_sorted = true;
-        for (uint32_t i = 0; i < listed; ++i) {
-            const uint32_t k = (start + i) % listed;
+    for (uint32_t idle = 0;; ++idle) {
+        bool all_sorted = true;
+        for (uint32_t i0 = 0; i0 < listed; i0 += kWave) {
+            const uint32_t i = i0 + lane;
+            const uint32_t k = (start + (i < listed ? i : 0)) % listed;
             OversizeBucket& o = t.oversize[k];
             const uint32_t phase = __hip_atomic_load(&o.phase, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (phase >= 2 * t.passes) continue;
-            all_sorted = false;
-            if (__hip_atomic_load(&o.taken[phase], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= o.chunks) continue;
-            const uint32_t c = __hip_atomic_fetch_add(&o.taken[phase], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (c < o.chunks) {
-                w.listed_at = k;
-                w.phase = phase;
-                w.chunk = c;
-                w.found = 1;
-                return w;
+            const bool open = i < listed && phase < 2 * t.passes;
+            const bool left = open && __hip_atomic_load(&o.taken[phase], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < o.chunks;
+            if (__any(open)) all_sorted = false;
+            uint64_t candidates = __ballot(left);
+            while (candidates != 0) {
+                const int src = __ffsll(static_cast<long long>(candidates)) - 1;
+                candidates &= candidates - 1;
+                uint32_t c = 0;
+                if (lane == static_cast<uint32_t>(src))
+                    c = __hip_atomic_fetch_add(&o.taken[phase], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                w.listed_at = __shfl(k, src, kWave);
+                w.phase = __shfl(phase, src, kWave);
+                w.chunk = __shfl(c, src, kWave);
+                if (w.chunk < __shfl(o.chunks, src, kWave)) {
+                    w.found = 1;
+                    return w;
+                }
             }
         }
-        __builtin_amdgcn_s_sleep(32);
+        if (all_sorted) return w;
+        // (hundreds of workgroups may be waiting for one bucket's phase: longer and longer, up to some 15 us)
+        for (uint32_t n = 0; n < (1u << min(idle, 4u)); ++n) __builtin_amdgcn_s_sleep(32);
     }
-    return w;
 }
 
 // The counts of a bucket's chunks, digit by digit, become places in its stretch of the output.
@@ -766,9 +777,18 @@ __device__ __forceinline__ void place_chunks(const SortTables& t, const Oversize
     const uint32_t mine = (o.chunks + kShares - 1) / kShares;
     const uint32_t from = min(share * mine, o.chunks), to = min(from + mine, o.chunks);
     uint32_t* column = t.oversize_begins + (static_cast<uint64_t>(o.chunks_before) << kPassBits) + d;
-    uint32_t sum = 0;
-#pragma unroll 8
-    for (uint32_t c = from; c < to; ++c) sum += column[static_cast<uint64_t>(c) << kPassBits];
+    // (a batch of loads on their way at a time: a bucket of 3 M entries has 490 chunks)
+    constexpr uint32_t kBatch = 32;
+    auto counts_of = [&](uint32_t c0, uint32_t (&n)[kBatch]) {
+#pragma unroll
+        for (uint32_t i = 0; i < kBatch; ++i) n[i] = column[static_cast<uint64_t>(min(c0 + i, to - 1)) << kPassBits];
+    };
+    uint32_t sum = 0, n[kBatch];
+    for (uint32_t c = from; c < to; c += kBatch) {
+        counts_of(c, n);
+#pragma unroll
+        for (uint32_t i = 0; i < kBatch; ++i) sum += c + i < to ? n[i] : 0u;
+    }
     s_sum[threadIdx.x] = sum;
     __syncthreads();
     uint32_t total = 0, before = 0;
@@ -784,11 +804,13 @@ __device__ __forceinline__ void place_chunks(const SortTables& t, const Oversize
     }
     __syncthreads();
     uint32_t at = s_sum[d] + before;
-    for (uint32_t c = from; c < to; ++c) {
-        uint32_t* word = column + (static_cast<uint64_t>(c) << kPassBits);
-        const uint32_t n = *word;
-        *word = at;
-        at += n;
+    for (uint32_t c = from; c < to; c += kBatch) {
+        counts_of(c, n);
+#pragma unroll
+        for (uint32_t i = 0; i < kBatch; ++i) {
+            if (c + i < to) column[static_cast<uint64_t>(c + i) << kPassBits] = at;
+            at += n[i];
+        }
     }
 }
 
@@ -806,12 +828,19 @@ __global__ __launch_bounds__(kBucketThreads) void oversize_kernel(SortTables t, 
     __shared__ OversizeWork s_work;
     __shared__ uint32_t s_last;
     const uint32_t tid = threadIdx.x, wave = tid / kWave;
+    uint32_t start = blockIdx.x % listed;
     while (true) {
-        if (tid == 0) s_work = find_oversize_work(t, listed, blockIdx.x);
+        if (wave == 0) {
+            const OversizeWork found = find_oversize_work(t, listed, start);
+            if (tid == 0) s_work = found;
+            // what the phase before has written, for the whole workgroup (it goes on behind the barrier); device-wide fences
+            // flush an XCD's L2, so one wavefront makes them for all
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        }
         __syncthreads();
         const OversizeWork work = s_work;
         if (work.found == 0) return;  // whole workgroup
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // what the phase before has written
+        start = work.listed_at;       // its next chunk or phase is what this workgroup looks for first
         OversizeBucket& o = t.oversize[work.listed_at];
         const uint32_t p = work.phase / 2;
         const bool counting = work.phase % 2 == 0;
@@ -880,27 +909,23 @@ __global__ __launch_bounds__(kBucketThreads) void oversize_kernel(SortTables t, 
                 }
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
         __syncthreads();
         if (tid == 0)
-            s_last = __hip_atomic_fetch_add(&o.done[work.phase], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == o.chunks;
+            s_last = __hip_atomic_fetch_add(&o.done[work.phase], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1 == o.chunks;
         __syncthreads();
         if (s_last != 0) {  // whole workgroup
-            if (counting) {
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-                place_chunks(t, o, out, t.passes == 1, pass.bits, s_sum, s.wave);
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-                __syncthreads();
-            }
-            if (tid == 0) __hip_atomic_store(&o.phase, work.phase + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (counting) place_chunks(t, o, out, t.passes == 1, pass.bits, s_sum, s.wave);
+            __syncthreads();
+            if (tid == 0) __hip_atomic_store(&o.phase, work.phase + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
         }
         __syncthreads();
     }
 }
 
-// Small inputs get small tiles, so that there are a few workgroups per compute unit.
-constexpr uint32_t kTileLarge = 8192, kTileSmall = 2048;
-constexpr uint32_t kSmallTileEntries = 512 * kTileLarge;
+// Small inputs get small tiles, so that there is work for every compute unit; runs twice as long are worth more as soon as
+// there are 128 of the large ones (sorting 1.5 M pairs 112 us from small, 111 from large tiles; 3 M: 174 and 168).
+constexpr uint32_t kTileLarge = 8192, kTileSmall = 4096;
+constexpr uint32_t kSmallTileEntries = 128 * kTileLarge;
 static_assert(kTileSmall == kBucketTileMin, "what the sums over buckets make room for");
 uint32_t tile_size_for(uint32_t count) { return count <= kSmallTileEntries ? kTileSmall : kTileLarge; }
 uint32_t tiles_of(uint32_t count, uint32_t tile_size) {
@@ -917,7 +942,7 @@ void launch_partition(hipStream_t stream, const EntrySource& in, uint32_t shift,
         hipLaunchKernelGGL((partition_kernel<VB, KIND, MAX_BITS, Key, 512, 16>), grid, dim3(512), 0, stream, in, shift, bits,
                            tiles, static_cast<Key*>(keys_out), aux_out, vals_out, table, xcds);
     } else {
-        hipLaunchKernelGGL((partition_kernel<VB, KIND, MAX_BITS, Key, 256, 8>), grid, dim3(256), 0, stream, in, shift, bits,
+        hipLaunchKernelGGL((partition_kernel<VB, KIND, MAX_BITS, Key, 512, 8>), grid, dim3(512), 0, stream, in, shift, bits,
                            tiles, static_cast<Key*>(keys_out), aux_out, vals_out, table, xcds);
     }
 }
@@ -961,19 +986,24 @@ struct SortShape {
 };
 constexpr uint32_t kNoMinorKey = ~0u;
 constexpr uint32_t kMaxKeyRest = 16;  // bits of a key behind those of step 1: it travels in 16
-bool sort_shape(uint32_t count, uint32_t key_bits, uint32_t minor_bits, SortShape* s) {
+// key_count: keys are below it (for a minor key in minor_bits).
+bool sort_shape(uint32_t count, uint32_t key_count, uint32_t minor_bits, SortShape* s) {
     // (and every array of the sort stays below 4 GiB)
-    if (count == 0 || count > kMostEntries) return false;
+    if (count == 0 || key_count == 0 || count > kMostEntries) return false;
+    const uint32_t key_bits = bit_length(key_count - 1);
     uint32_t bits = 0;
-    while (bits < key_bits && bits < kMaxTwoLevelBits && (static_cast<uint64_t>(kBucketWanted) << bits) < count) ++bits;
+    // (of the 2^bits buckets only those that hold keys count)
+    while (bits < key_bits && bits < kMaxTwoLevelBits &&
+           static_cast<uint64_t>(kBucketWanted) * (((key_count - 1) >> (key_bits - bits)) + 1) < count)
+        ++bits;
     auto first_level = [&]() { return bits <= kMaxOneLevelBits ? bits : (bits + 1) / 2; };
     if (minor_bits == kNoMinorKey) {
         // one pass over a bucket, so that its digit counts say where every key begins
         if (key_bits > kMaxTwoLevelBits + kPassBits) return false;
         const uint32_t least = key_bits > kPassBits ? key_bits - kPassBits : 0;
         // many more keys than entries: buckets of a few entries each, a workgroup for every one of them (2^22 columns,
-        // 1 M entries: 210 us; the passes of the LSD sort take 170)
-        if (least > kMaxOneLevelBits && (static_cast<uint64_t>(count) << 4) < static_cast<uint64_t>(kBucketWanted) << least) return false;
+        // 5 M entries: 253 us; the passes of the LSD sort take 196)
+        if (least > kMaxOneLevelBits && (static_cast<uint64_t>(count) << 3) < static_cast<uint64_t>(kBucketWanted) << least) return false;
         bits = bits > least ? bits : least;
     } else {
         if (minor_bits > 24) return false;
@@ -1130,27 +1160,26 @@ void launch_sort(hipStream_t stream, EntrySource in, const SortShape& s, const S
 
 }  // namespace
 
-bool partition_sort_usable(idx_t count, uint32_t key_bits) {
+bool partition_sort_usable(idx_t count, idx_t key_count) {
     SortShape s;
-    return sort_shape(count, key_bits, kNoMinorKey, &s);
+    return sort_shape(count, key_count, kNoMinorKey, &s);
 }
-size_t partition_sort_workspace_bytes(idx_t count, uint32_t key_bits, size_t value_bytes) {
+size_t partition_sort_workspace_bytes(idx_t count, idx_t key_count, size_t value_bytes) {
     SortShape s;
-    return sort_shape(count, key_bits, kNoMinorKey, &s) ? sort_layout(count, s, value_bytes).total : 0;
+    return sort_shape(count, key_count, kNoMinorKey, &s) ? sort_layout(count, s, value_bytes).total : 0;
 }
-bool partition_sort_pairs_usable(idx_t count, uint32_t major_bits, uint32_t minor_bits) {
+bool partition_sort_pairs_usable(idx_t count, idx_t major_count, idx_t minor_count) {
     SortShape s;
-    return sort_shape(count, major_bits, minor_bits, &s);
+    return sort_shape(count, major_count, bit_length(minor_count - 1), &s);
 }
-size_t partition_sort_pairs_workspace_bytes(idx_t count, uint32_t major_bits, uint32_t minor_bits) {
+size_t partition_sort_pairs_workspace_bytes(idx_t count, idx_t major_count, idx_t minor_count) {
     SortShape s;
-    return sort_shape(count, major_bits, minor_bits, &s) ? sort_layout(count, s, sizeof(idx_t)).total : 0;
+    return sort_shape(count, major_count, bit_length(minor_count - 1), &s) ? sort_layout(count, s, sizeof(idx_t)).total : 0;
 }
 
-void launch_partition_sort(hipStream_t stream, idx_t count, uint32_t key_bits, const PartitionSortArgs& a, size_t value_bytes,
-                           void* workspace) {
+void launch_partition_sort(hipStream_t stream, idx_t count, const PartitionSortArgs& a, size_t value_bytes, void* workspace) {
     SortShape s;
-    if (!sort_shape(count, key_bits, kNoMinorKey, &s)) return;
+    if (!sort_shape(count, a.key_count, kNoMinorKey, &s)) return;
     EntrySource in;
     in.keys = a.keys_in;
     in.aux = a.row_ptr;
@@ -1173,10 +1202,10 @@ void launch_partition_sort(hipStream_t stream, idx_t count, uint32_t key_bits, c
     launch(stream, in, s, out, static_cast<char*>(workspace));
 }
 
-void launch_partition_sort_pairs(hipStream_t stream, idx_t count, uint32_t major_bits, uint32_t minor_bits, idx_t* major,
+void launch_partition_sort_pairs(hipStream_t stream, idx_t count, idx_t major_count, idx_t minor_count, idx_t* major,
                                  idx_t* minor, idx_t* perm, void* workspace) {
     SortShape s;
-    if (!sort_shape(count, major_bits, minor_bits, &s)) return;
+    if (!sort_shape(count, major_count, bit_length(minor_count - 1), &s)) return;
     EntrySource in = {};
     in.keys = major;
     in.aux = minor;

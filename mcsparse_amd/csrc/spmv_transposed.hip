@@ -130,9 +130,10 @@ struct WaveRuns {
 template <typename T>
 struct Piece { typedef T type __attribute__((ext_vector_type(kPiece))); };
 
-// Adds the products of the windows first, first + step, ... of group g to the sums.
+// Adds the products of the windows first, first + step, ... of group g to the sums.  Returns the number of windows of
+// the group.
 template <typename T>
-__device__ __forceinline__ void add_group(uint32_t word, uint32_t g, uint32_t tile_places, uint32_t first, uint32_t step,
+__device__ __forceinline__ uint32_t add_group(uint32_t word, uint32_t g, uint32_t tile_places, uint32_t first, uint32_t step,
                                           WaveRuns& s, const uint16_t* __restrict__ keys, const T* __restrict__ products,
                                           uint32_t key_mask, double* s_acc) {
     typedef typename Piece<T>::type piece_t;
@@ -191,6 +192,7 @@ __device__ __forceinline__ void add_group(uint32_t word, uint32_t g, uint32_t ti
             }
         }
     }
+    return (total + kWindow - 1) / kWindow;
 }
 
 template <typename T>
@@ -230,26 +232,29 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_sums_kernel(idx_t n, uint
         const uint32_t t = g * kGroupTiles + lane;
         return lane < kGroupTiles && t < tiles ? row[t] : 0u;
     };
-    const uint32_t step = kWaves * mine.parts;
-    uint32_t g = mine.part + wave * mine.parts;
-    uint32_t word = g < groups ? words_of(g) : 0u;
-    for (; g < groups; g += step) {
-        const uint32_t next = g + step < groups ? words_of(g + step) : 0u;  // on its way while this group is added
+    // light groups are dealt to the parts, heavy ones are shared by all wavefronts of all parts
+    uint32_t word = wave < groups ? words_of(wave) : 0u;
+    for (uint32_t g = wave; g < groups; g += kWaves) {
+        const uint32_t next = g + kWaves < groups ? words_of(g + kWaves) : 0u;  // on its way while this group is added
         const uint32_t total = __builtin_amdgcn_readlane(wave_inclusive_sum(run_length(word) / kPiece), kWave - 1);
         if (total > kHeavyGroup) {
             if (lane == 0) atomicOr(&s_heavy[g / 32], 1u << (g % 32));
-        } else if (total != 0) {
+        } else if (total != 0 && g % mine.parts == mine.part) {
             add_group(word, g, tile_places, 0, 1, s_runs[wave], keys, products, width - 1, s_acc);
         }
         word = next;
     }
     __syncthreads();
+    const uint32_t takers = mine.parts * kWaves;
+    uint32_t turn = mine.part * kWaves + wave;  // which of the next group's windows is this wavefront's first
     for (uint32_t w = 0; w < (groups + 31) / 32; ++w) {
         uint32_t left = s_heavy[w];
         while (left != 0) {
             const uint32_t b = __ffs(left) - 1;
             left &= left - 1;
-            add_group(words_of(w * 32 + b), w * 32 + b, tile_places, wave, kWaves, s_runs[wave], keys, products, width - 1, s_acc);
+            const uint32_t windows = add_group(words_of(w * 32 + b), w * 32 + b, tile_places, turn, takers, s_runs[wave], keys,
+                                               products, width - 1, s_acc);
+            turn = (turn + takers - windows % takers) % takers;
         }
     }
     __syncthreads();

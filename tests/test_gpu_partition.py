@@ -12,7 +12,7 @@ from gpu_util import dev, run_spmv
 
 pytestmark = pytest.mark.gpu
 
-LARGE_FROM = 512 * 8192  # entries up to which the tiles hold 2048 entries, beyond 8192
+LARGE_FROM = 128 * 8192  # entries up to which the tiles hold 4096 entries, beyond 8192
 
 
 def matrix(kind, m, n, nnz, dtype, seed):
@@ -35,7 +35,7 @@ def matrix(kind, m, n, nnz, dtype, seed):
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("kind,m,n,nnz", [
-    ("uniform", 50, 40000, 1), ("uniform", 300, 40000, 2047), ("uniform", 300, 40000, 2048), ("uniform", 300, 40000, 2049),
+    ("uniform", 50, 40000, 1), ("uniform", 300, 40000, 4095), ("uniform", 300, 40000, 4096), ("uniform", 300, 40000, 4097),
     ("uniform", 30000, 20000, 300001), ("band", 50000, 70000, 700000), ("few", 60000, 200000, 900000),
     ("uniform", 400000, 1 << 22, LARGE_FROM), ("uniform", 400000, 300000, LARGE_FROM + 1),
     ("band", 200000, 150000, LARGE_FROM + 8191), ("few", 150000, 4000000, LARGE_FROM + 8192 * 30),
@@ -56,7 +56,7 @@ ONE_LEVEL_UPTO = 3686 << 11  # entries up to which one partition makes the bucke
 @pytest.mark.parametrize("dtype,action", [(np.float32, api.ACTION_NUMERIC), (np.float64, api.ACTION_NUMERIC),
                                           (np.float32, api.ACTION_SYMBOLIC)])
 @pytest.mark.parametrize("kind,m,n,nnz,base", [
-    ("uniform", 5, 1, 40, 0), ("uniform", 50, 200, 1, 1), ("uniform", 400, 256, 2049, 0), ("uniform", 300, 257, 20000, 1),
+    ("uniform", 5, 1, 40, 0), ("uniform", 50, 200, 1, 1), ("uniform", 400, 256, 4097, 0), ("uniform", 300, 257, 20000, 1),
     ("uniform", 3000, 70000, 6145, 0), ("few", 50, 3, 30000, 0), ("few", 3000, 1 << 16, 400000, 1),
     ("band", 100000, 90000, 1000001, 0), ("uniform", 100000, 5000, LARGE_FROM, 0), ("few", 100000, 300000, LARGE_FROM + 1, 1),
     ("uniform", 300000, 1 << 20, ONE_LEVEL_UPTO, 0), ("uniform", 300000, (1 << 20) + 1, ONE_LEVEL_UPTO + 1, 1),
