@@ -50,7 +50,7 @@ def test_transposed_product_exact(torch_gpu, handle, dtype, kind, m, n, nnz):
     assert np.array_equal(got.astype(np.float64), want)
 
 
-ONE_LEVEL_UPTO = 3686 << 11  # entries up to which one partition makes the buckets that are sorted in LDS
+ONE_LEVEL_UPTO = 4300 << 11  # entries up to which one partition makes the buckets that are sorted in LDS
 
 
 @pytest.mark.parametrize("dtype,action", [(np.float32, api.ACTION_NUMERIC), (np.float64, api.ACTION_NUMERIC),
