@@ -24,11 +24,11 @@ __global__ __launch_bounds__(kBlock) void spmm_rowb_kernel(idx_t m, idx_t n, idx
                                                            const idx_t* __restrict__ col, const T* __restrict__ val,
                                                            const T* __restrict__ B, int64_t ldb, T* __restrict__ C,
                                                            int64_t ldc, bool c_row_major, T alpha, T beta,
-                                                           idx_t long_row) {
+                                                           idx_t long_row, uint32_t xcd_chunk, uint32_t xcds) {
     typedef typename ByteOffset<WIDE>::type off_t;
     constexpr int kRowsPerBlock = kBlock / LR;
     const idx_t lane = threadIdx.x % LR;
-    const uint64_t row = static_cast<uint64_t>(blockIdx.x) * kRowsPerBlock + threadIdx.x / LR;
+    const uint64_t row = xcd_position(blockIdx.x, xcd_chunk, xcds) * kRowsPerBlock + threadIdx.x / LR;
     const uint64_t c_own = (static_cast<uint64_t>(blockIdx.y) * LR + lane) * V;
     if (row >= m) return;  // whole lane groups
     // Lanes past the last column still fetch their share of the row's nonzeros for the group;
@@ -68,7 +68,8 @@ __global__ __launch_bounds__(kBlock) void spmm_narrow_kernel(idx_t m, idx_t n, i
                                                              const idx_t* __restrict__ col,
                                                              const T* __restrict__ val, const T* __restrict__ B,
                                                              int64_t ldb, T* __restrict__ Cm, int64_t ldc,
-                                                             bool c_row_major, T alpha, T beta, idx_t long_row) {
+                                                             bool c_row_major, T alpha, T beta, idx_t long_row,
+                                                             uint32_t xcd_chunk, uint32_t xcds) {
     constexpr int kLanes = 16;
     constexpr int P = kLanes / C;
     constexpr int kSteps = 4;  // measured on a 27-point stencil, n = 8: 1, 2, 4, 8 steps -> 305, 280, 260, 291 us
@@ -79,7 +80,7 @@ __global__ __launch_bounds__(kBlock) void spmm_narrow_kernel(idx_t m, idx_t n, i
     const bool in_panel = c_own < n;
     const uint64_t c0 = in_panel ? c_own : 0;
     // the groups of a workgroup take neighbouring rows in every round
-    const uint64_t first_row = static_cast<uint64_t>(blockIdx.x) * (kGroups * kNarrowRowsPerGroup) + threadIdx.x / kLanes;
+    const uint64_t first_row = xcd_position(blockIdx.x, xcd_chunk, xcds) * (kGroups * kNarrowRowsPerGroup) + threadIdx.x / kLanes;
     const uint64_t last_row = static_cast<uint64_t>(m) - 1;  // m != 0 here
 
     if (nnz == 0) {  // nothing to read, only C to scale
@@ -201,10 +202,12 @@ template <typename T, int V, int C>
 void launch_narrow(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     constexpr int kRowsPerBlock = kBlock / 16 * kNarrowRowsPerGroup;
     const uint64_t blocks = (static_cast<uint64_t>(a.m) + kRowsPerBlock - 1) / kRowsPerBlock;
-    hipLaunchKernelGGL((spmm_narrow_kernel<T, V, C>), dim3(static_cast<uint32_t>(blocks)), dim3(kBlock), 0, stream, a.m,
+    const uint32_t xcds = device_topology().xcds;
+    const uint32_t chunk = xcd_stretch(blocks, kRowsPerBlock, xcds);
+    hipLaunchKernelGGL((spmm_narrow_kernel<T, V, C>), dim3(xcd_padded_grid(blocks, chunk, xcds)), dim3(kBlock), 0, stream, a.m,
                        a.n, a.nnz, a.base, a.row_ptr, a.col, static_cast<const T*>(a.val),
                        static_cast<const T*>(a.B), a.ldb, static_cast<T*>(a.C), a.ldc, a.c_row_major, alpha, beta,
-                       a.long_row);
+                       a.long_row, chunk, xcds);
 }
 
 // op(B) column-major: element (kk, j) at j*ldb + kk.  One wavefront per row of A, lanes strided
@@ -664,16 +667,22 @@ template <typename T, int LR, int V>
 void launch_rowb(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     const uint64_t row_blocks = (static_cast<uint64_t>(a.m) + (kBlock / LR) - 1) / (kBlock / LR);
     const uint64_t panels = (static_cast<uint64_t>(a.n) + LR * V - 1) / (LR * V);
-    const dim3 grid(static_cast<uint32_t>(row_blocks), static_cast<uint32_t>(panels));
+    const uint32_t xcds = device_topology().xcds;
+    // wider operands than 16 lanes gained nothing from stretches (power-law rows of 17 columns in 32 lanes: 1365 us in
+    // plain turns, 1400 in stretches)
+    const uint32_t chunk = LR <= 16 ? xcd_stretch(row_blocks, kBlock / LR, xcds) : 1;
+    const dim3 grid(xcd_padded_grid(row_blocks, chunk, xcds), static_cast<uint32_t>(panels));
     const T* val = static_cast<const T*>(a.val);
     const T* B = static_cast<const T*>(a.B);
     T* C = static_cast<T*>(a.C);
     if (narrow_offsets(a, sizeof(T))) {
         hipLaunchKernelGGL((spmm_rowb_kernel<T, LR, V, false>), grid, dim3(kBlock), 0, stream, a.m, a.n, a.base,
-                           a.row_ptr, a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta, a.long_row);
+                           a.row_ptr, a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta, a.long_row, chunk,
+                           xcds);
     } else {
         hipLaunchKernelGGL((spmm_rowb_kernel<T, LR, V, true>), grid, dim3(kBlock), 0, stream, a.m, a.n, a.base,
-                           a.row_ptr, a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta, a.long_row);
+                           a.row_ptr, a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta, a.long_row, chunk,
+                           xcds);
     }
 }
 

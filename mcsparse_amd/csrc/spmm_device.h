@@ -76,6 +76,21 @@ inline uint32_t xcd_padded_grid(uint64_t count, uint32_t chunk, uint32_t xcds) {
     return static_cast<uint32_t>((count + per_round - 1) / per_round * per_round);
 }
 
+// Length of such a stretch for the kernels without a schedule, which know nothing of the structure: workgroups that
+// hold kXcdStretchRows rows, but no more than leave every XCD kXcdStretchRounds turns, so that stretches of different
+// weight even out.  Neighbouring rows of a stencil or a mesh read mostly the same rows of op(B); in plain turns all
+// eight L2s fetch them.  27-point stencil 101 x 97 x 89, 16 fp64 columns, microseconds per product: 189 in plain turns,
+// 179, 178, 180, 185, 186 with 1024, 2048, 4096, 8192, 16384 rows; a million power-law rows, 8 fp32 columns: 407 and
+// 385, 392, 384, 390, 396.
+constexpr uint64_t kXcdStretchRows = 2048;
+constexpr uint64_t kXcdStretchRounds = 4;
+inline uint32_t xcd_stretch(uint64_t blocks, uint64_t rows_per_block, uint32_t xcds) {
+    uint32_t chunk = 1;
+    if (xcds <= 1) return chunk;
+    while (chunk * 2 * rows_per_block <= kXcdStretchRows && chunk * 2 * xcds * kXcdStretchRounds <= blocks) chunk *= 2;
+    return chunk;
+}
+
 // acc += sum over the nonzeros [begin, end) of one row of A of value * (V columns of the row of
 // op(B) the nonzero names), for a group of LR >= 4 lanes that all pass the same range.
 // B_bytes is the operand's first element, lane_off the byte offset of this lane's columns.
