@@ -591,7 +591,7 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
         const bool direct_c = l.copy_c && scheduled_here && schedule_usable() &&
                               reinterpret_cast<uintptr_t>(c_user) % 16 == 0 &&
                               (static_cast<uint64_t>(C->ld) * sizeof(T)) % 16 == 0;
-        const bool copy_c = l.copy_c && !direct_c;
+        bool copy_c = l.copy_c && !direct_c;
         if (copy_c) {
             a.C = buf + l.ct;
             a.ldc = l.n_padded;
@@ -612,6 +612,9 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
             else
                 mcsp::launch_spmm_scheduled<T>(h->stream, a, buffer, A->schedule.entries, A->schedule.mean_span, h_alpha,
                                                beta_inner);
+        } else if (copy_c && mcsp::launch_spmm_columns<T>(h->stream, a, static_cast<idx_t>(C->col_num), c_user, C->ld,
+                                                          h_alpha, h_beta)) {
+            copy_c = false;  // written into the caller's C as it lies
         } else {
             mcsp::launch_spmm<T>(h->stream, a, h_alpha, beta_inner);
         }

@@ -363,6 +363,11 @@ struct SpmmArgs {
 };
 template <typename T>
 void launch_spmm(hipStream_t stream, const SpmmArgs& a, T alpha, T beta);
+// The same into a column-major C of c_cols columns (a.C, a.ldc and a.c_row_major are not looked at), written column by
+// column by the kernel that forms the sums.  false, and nothing launched, where that kernel has no variant: a
+// column-major op(B), one or two or more than sixteen 16-byte vectors per row of it, rows that are taken apart.
+template <typename T>
+bool launch_spmm_columns(hipStream_t stream, const SpmmArgs& a, idx_t c_cols, T* C, int64_t ldc, T alpha, T beta);
 
 // Long rows (spmm_long.hip): a lane group of the row kernels walks a row by itself, so a row of tens of thousands
 // of nonzeros outlasts the rest of the launch.  Rows above kSpmmLongRow nonzeros are cut into pieces of

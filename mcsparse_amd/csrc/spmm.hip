@@ -51,6 +51,58 @@ __global__ __launch_bounds__(kBlock) void spmm_rowb_kernel(idx_t m, idx_t n, idx
     if (stores) store_c<T, V>(C, ldc, c_row_major, row, c0, acc, alpha, beta);
 }
 
+// The same product into a column-major C, without a row-major copy of C in between.  A workgroup owns kColumnRows
+// neighbouring rows, kBlock / LR at a time, gathers their sums in LDS and writes a column's stretch of rows as it lies
+// in C (512 bytes in fp64, 256 in fp32).  For LR <= 16: wider panels of as many rows do not fit LDS several times.
+// Measured together with the narrower tiles of transpose_kernel, 27-point stencil of 872 K rows: 16 fp64 columns 297 ->
+// 235 us a call, 4 fp64 columns (narrow kernel, tiles alone) 186 -> 125, 12 fp32 columns 169 -> 133, 31 fp32 columns
+// 344 -> 339.
+// C has c_cols columns, n of op(B) (n >= c_cols) may be padded to whole vectors.
+constexpr int kColumnRows = 64;
+template <typename T, int LR, int V, bool WIDE>
+__global__ __launch_bounds__(kBlock) void spmm_rowb_columns_kernel(idx_t m, idx_t n, idx_t c_cols, idx_t base,
+                                                                   const idx_t* __restrict__ row_ptr,
+                                                                   const idx_t* __restrict__ col,
+                                                                   const T* __restrict__ val, const T* __restrict__ B,
+                                                                   int64_t ldb, T* __restrict__ C, int64_t ldc, T alpha,
+                                                                   T beta, uint32_t xcd_chunk, uint32_t xcds) {
+    typedef typename ByteOffset<WIDE>::type off_t;
+    constexpr int kRowsPerPass = kBlock / LR;
+    constexpr int kCols = LR * V;
+    static_assert(kColumnRows % kRowsPerPass == 0, "whole passes");
+    __shared__ T s_c[kCols][kColumnRows + 1];
+    const idx_t lane = threadIdx.x % LR;
+    const uint64_t row0 = xcd_position(blockIdx.x, xcd_chunk, xcds) * kColumnRows;
+    if (row0 >= m) return;  // whole workgroup
+    const uint64_t panel = static_cast<uint64_t>(blockIdx.y) * kCols;
+    const uint64_t c_own = panel + lane * V;
+    const uint64_t c0 = c_own < n ? c_own : 0;  // lanes past the last column only help fetching
+#pragma unroll 1
+    for (int r0 = 0; r0 < kColumnRows; r0 += kRowsPerPass) {
+        const int r = r0 + static_cast<int>(threadIdx.x) / LR;
+        const uint64_t row = row0 + r < m ? row0 + r : m - 1;  // rows past the end repeat the last one
+        const idx_t start = row_ptr[row] - base;
+        const idx_t end = row_ptr[row + 1] - base;
+        T acc[V];
+#pragma unroll
+        for (int i = 0; i < V; ++i) acc[i] = T(0);
+        row_times_b<T, LR, V, WIDE>(start, end, lane, base, col, val, reinterpret_cast<const char*>(B),
+                                    static_cast<off_t>(c0 * sizeof(T)), static_cast<off_t>(ldb * sizeof(T)), acc);
+#pragma unroll
+        for (int i = 0; i < V; ++i) s_c[lane * V + i][r] = acc[i];
+    }
+    __syncthreads();
+    const uint64_t row = row0 + threadIdx.x % kColumnRows;
+    if (row >= m) return;
+#pragma unroll 4
+    for (int c = threadIdx.x / kColumnRows; c < kCols; c += kBlock / kColumnRows) {
+        if (panel + c >= c_cols) break;
+        T* out = C + static_cast<int64_t>(panel + c) * ldc + static_cast<int64_t>(row);
+        const T v = alpha * s_c[c][threadIdx.x % kColumnRows];
+        *out = beta == T(0) ? v : beta * *out + v;
+    }
+}
+
 // op(B) row-major with few columns (n <= 2 vectors of V).  A row of op(B) then takes only
 // C = 1 or 2 lanes, and what a row of A costs is the chain of dependent loads (offsets,
 // nonzeros, rows of op(B)) rather than bytes.  So 16 lanes share a row of A as P = 16 / C
@@ -269,39 +321,44 @@ __global__ __launch_bounds__(kBlock) void spmm_colb_kernel(idx_t m, idx_t n, idx
 // move whole cache lines.  Columns [rows, rows_padded) of dst are filled with zeros.  ACCUMULATE:
 // dst = beta * dst + transpose(src) (beta == 0 does not read dst) and nothing is padded.
 // Stands in for mcspDenseTransposeKernel (src/common/mcsp_dense_transpose_device.hpp:8-38).
-constexpr int kTransTile = 64;
-template <typename T, bool ACCUMULATE>
+// A tile of 64 x 64 for operands of 16 columns moves three clamped rows for one that is there (872 K x 16 doubles:
+// 70 us in, 56 us out), so the tile takes the narrow side as its own: R rows by 4096 / R columns.
+constexpr int kTransTile = 4096;  // elements
+template <typename T, bool ACCUMULATE, int R>
 __global__ __launch_bounds__(kBlock) void transpose_kernel(uint32_t rows, uint32_t cols, uint32_t rows_padded,
                                                            const T* __restrict__ src, int64_t lds,
                                                            T* __restrict__ dst, int64_t ldd, T beta) {
-    __shared__ T tile[kTransTile][kTransTile + 1];
-    const uint32_t tx = threadIdx.x % kTransTile;
-    const uint32_t ty = threadIdx.x / kTransTile;  // 0..3
-    const uint32_t r0 = blockIdx.x * kTransTile;   // along rows of src
-    const uint32_t c0 = blockIdx.y * kTransTile;   // along cols of src
-    T got[kTransTile / 4];
+    constexpr uint32_t kR = R;
+    constexpr uint32_t kC = kTransTile / R;
+    constexpr int kEach = kTransTile / kBlock;
+    __shared__ T tile[kR][kC + 1];
+    const uint64_t r0 = static_cast<uint64_t>(blockIdx.x) * kR;  // along rows of src
+    const uint64_t c0 = static_cast<uint64_t>(blockIdx.y) * kC;  // along cols of src
+    T got[kEach];
 #pragma unroll
-    for (int k = 0; k < kTransTile / 4; ++k) {
-        const uint32_t r = r0 + ty + 4 * k;
-        const uint32_t c = c0 + tx;
+    for (int k = 0; k < kEach; ++k) {
+        const uint32_t e = threadIdx.x + k * kBlock;
+        const uint64_t r = r0 + e / kC;
+        const uint64_t c = c0 + e % kC;
         // clamped position, so that the sixteen loads are on their way together
-        const uint32_t rr = r < rows ? r : rows - 1;
-        const uint32_t cc = c < cols ? c : cols - 1;
-        got[k] = src[static_cast<int64_t>(rr) * lds + cc];
+        const uint64_t rr = r < rows ? r : rows - 1;
+        const uint64_t cc = c < cols ? c : cols - 1;
+        got[k] = src[static_cast<int64_t>(rr) * lds + static_cast<int64_t>(cc)];
     }
 #pragma unroll
-    for (int k = 0; k < kTransTile / 4; ++k) {
-        const uint32_t r = r0 + ty + 4 * k;
-        tile[ty + 4 * k][tx] = r < rows ? got[k] : T(0);
+    for (int k = 0; k < kEach; ++k) {
+        const uint32_t e = threadIdx.x + k * kBlock;
+        tile[e / kC][e % kC] = r0 + e / kC < rows ? got[k] : T(0);
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < kTransTile / 4; ++k) {
-        const uint32_t c = c0 + ty + 4 * k;  // row of dst
-        const uint32_t r = r0 + tx;          // column of dst
+    for (int k = 0; k < kEach; ++k) {
+        const uint32_t e = threadIdx.x + k * kBlock;
+        const uint64_t c = c0 + e / kR;  // row of dst
+        const uint64_t r = r0 + e % kR;  // column of dst
         if (c < cols && r < (ACCUMULATE ? rows : rows_padded)) {
-            T* out = dst + static_cast<int64_t>(c) * ldd + r;
-            const T v = tile[tx][ty + 4 * k];
+            T* out = dst + static_cast<int64_t>(c) * ldd + static_cast<int64_t>(r);
+            const T v = tile[e % kR][e / kR];
             if constexpr (ACCUMULATE) {
                 *out = beta == T(0) ? v : beta * *out + v;
             } else {
@@ -796,24 +853,89 @@ void launch_spmm_scheduled(hipStream_t stream, const SpmmArgs& a, const void* sc
     else launch_group<T, 64>(stream, a, group_ptr, entries, total_entries, alpha, beta, mean_span);
 }
 
+namespace {
+
+template <typename T, bool ACCUMULATE, int R>
+void launch_transpose_tile(hipStream_t stream, idx_t rows, idx_t cols, idx_t rows_padded, const T* src, int64_t lds,
+                           T* dst, int64_t ldd, T beta) {
+    constexpr uint32_t kC = kTransTile / R;
+    const dim3 grid((rows_padded + R - 1) / R, (cols + kC - 1) / kC);
+    hipLaunchKernelGGL((transpose_kernel<T, ACCUMULATE, R>), grid, dim3(kBlock), 0, stream, rows, cols, rows_padded, src,
+                       lds, dst, ldd, beta);
+}
+
+// Lanes per row of A that the row kernels use for the operands as they lie, V columns each.
+template <typename T>
+int columns_per_lane(const SpmmArgs& a) {
+    constexpr int kWide = 16 / sizeof(T);  // elements per 128-bit access
+    const bool aligned = (reinterpret_cast<uintptr_t>(a.B) % 16 == 0) && (a.ldb % kWide == 0) && (a.n % kWide == 0);
+    return aligned ? kWide : 1;
+}
+
+template <typename T, int LR, int V>
+void launch_columns(hipStream_t stream, const SpmmArgs& a, idx_t c_cols, T* C, int64_t ldc, T alpha, T beta) {
+    const uint64_t blocks = (static_cast<uint64_t>(a.m) + kColumnRows - 1) / kColumnRows;
+    const uint32_t xcds = device_topology().xcds;
+    const uint32_t chunk = xcd_stretch(blocks, kColumnRows, xcds);
+    const dim3 grid(xcd_padded_grid(blocks, chunk, xcds), (a.n + LR * V - 1) / (LR * V));
+    const T* val = static_cast<const T*>(a.val);
+    const T* B = static_cast<const T*>(a.B);
+    if (narrow_offsets(a, sizeof(T))) {
+        hipLaunchKernelGGL((spmm_rowb_columns_kernel<T, LR, V, false>), grid, dim3(kBlock), 0, stream, a.m, a.n, c_cols,
+                           a.base, a.row_ptr, a.col, val, B, a.ldb, C, ldc, alpha, beta, chunk, xcds);
+    } else {
+        hipLaunchKernelGGL((spmm_rowb_columns_kernel<T, LR, V, true>), grid, dim3(kBlock), 0, stream, a.m, a.n, c_cols,
+                           a.base, a.row_ptr, a.col, val, B, a.ldb, C, ldc, alpha, beta, chunk, xcds);
+    }
+}
+
+template <typename T, int V>
+void launch_columns_v(hipStream_t stream, const SpmmArgs& a, idx_t c_cols, T* C, int64_t ldc, T alpha, T beta) {
+    const uint64_t lanes = (static_cast<uint64_t>(a.n) + V - 1) / V;
+    if (lanes <= 4) launch_columns<T, 4, V>(stream, a, c_cols, C, ldc, alpha, beta);
+    else if (lanes <= 8) launch_columns<T, 8, V>(stream, a, c_cols, C, ldc, alpha, beta);
+    else launch_columns<T, 16, V>(stream, a, c_cols, C, ldc, alpha, beta);
+}
+
+}  // namespace
+
+template <typename T>
+bool launch_spmm_columns(hipStream_t stream, const SpmmArgs& a, idx_t c_cols, T* C, int64_t ldc, T alpha, T beta) {
+    if (!a.b_row_major || a.long_row != 0 || a.m == 0 || a.nnz == 0) return false;
+    constexpr int kWide = 16 / sizeof(T);
+    const int v = columns_per_lane<T>(a);
+    const uint64_t lanes = (static_cast<uint64_t>(a.n) + v - 1) / v;
+    if (lanes <= 2 || lanes > 16) return false;
+    if (v == kWide) launch_columns_v<T, kWide>(stream, a, c_cols, C, ldc, alpha, beta);
+    else launch_columns_v<T, 1>(stream, a, c_cols, C, ldc, alpha, beta);
+    return true;
+}
+
+// The narrow side of the operand is the rows of src on the way in ...
 template <typename T>
 void launch_transpose(hipStream_t stream, idx_t rows, idx_t cols, idx_t rows_padded, const T* src, int64_t lds, T* dst,
                       int64_t ldd) {
     if (rows == 0 || cols == 0) return;
-    const dim3 grid((rows_padded + kTransTile - 1) / kTransTile, (cols + kTransTile - 1) / kTransTile);
-    hipLaunchKernelGGL((transpose_kernel<T, false>), grid, dim3(kBlock), 0, stream, rows, cols, rows_padded, src, lds,
-                       dst, ldd, T(0));
+    if (rows_padded <= 4) launch_transpose_tile<T, false, 4>(stream, rows, cols, rows_padded, src, lds, dst, ldd, T(0));
+    else if (rows_padded <= 8) launch_transpose_tile<T, false, 8>(stream, rows, cols, rows_padded, src, lds, dst, ldd, T(0));
+    else if (rows_padded <= 16) launch_transpose_tile<T, false, 16>(stream, rows, cols, rows_padded, src, lds, dst, ldd, T(0));
+    else if (rows_padded <= 32) launch_transpose_tile<T, false, 32>(stream, rows, cols, rows_padded, src, lds, dst, ldd, T(0));
+    else launch_transpose_tile<T, false, 64>(stream, rows, cols, rows_padded, src, lds, dst, ldd, T(0));
 }
 
+// ... and its columns on the way out.
 template <typename T>
 void launch_transpose_accumulate(hipStream_t stream, idx_t rows, idx_t cols, const T* src, int64_t lds, T* dst,
                                  int64_t ldd, T beta) {
     if (rows == 0 || cols == 0) return;
-    const dim3 grid((rows + kTransTile - 1) / kTransTile, (cols + kTransTile - 1) / kTransTile);
-    hipLaunchKernelGGL((transpose_kernel<T, true>), grid, dim3(kBlock), 0, stream, rows, cols, rows, src, lds, dst, ldd,
-                       beta);
+    if (cols <= 8) launch_transpose_tile<T, true, 512>(stream, rows, cols, rows, src, lds, dst, ldd, beta);
+    else if (cols <= 16) launch_transpose_tile<T, true, 256>(stream, rows, cols, rows, src, lds, dst, ldd, beta);
+    else if (cols <= 32) launch_transpose_tile<T, true, 128>(stream, rows, cols, rows, src, lds, dst, ldd, beta);
+    else launch_transpose_tile<T, true, 64>(stream, rows, cols, rows, src, lds, dst, ldd, beta);
 }
 
+template bool launch_spmm_columns<float>(hipStream_t, const SpmmArgs&, idx_t, float*, int64_t, float, float);
+template bool launch_spmm_columns<double>(hipStream_t, const SpmmArgs&, idx_t, double*, int64_t, double, double);
 template void launch_transpose<float>(hipStream_t, idx_t, idx_t, idx_t, const float*, int64_t, float*, int64_t);
 template void launch_transpose<double>(hipStream_t, idx_t, idx_t, idx_t, const double*, int64_t, double*, int64_t);
 template void launch_transpose_accumulate<float>(hipStream_t, idx_t, idx_t, const float*, int64_t, float*, int64_t, float);
