@@ -16,8 +16,7 @@ namespace {
 using namespace spmm_detail;
 
 // op(B) row-major.  LR lanes per row of A, V adjacent columns per lane; blockIdx.y walks the
-// column panels of LR*V columns.  V > 1 requires n, ldb (and ldc when C is row-major) to be
-// multiples of V and 16-byte aligned base pointers, which the launcher checks.
+// column panels of LR*V columns.  V > 1 requires n >= V, which the launcher checks.
 template <typename T, int LR, int V, bool WIDE>
 __global__ __launch_bounds__(kBlock) void spmm_rowb_kernel(idx_t m, idx_t n, idx_t base,
                                                            const idx_t* __restrict__ row_ptr,
@@ -29,12 +28,11 @@ __global__ __launch_bounds__(kBlock) void spmm_rowb_kernel(idx_t m, idx_t n, idx
     constexpr int kRowsPerBlock = kBlock / LR;
     const idx_t lane = threadIdx.x % LR;
     const uint64_t row = xcd_position(blockIdx.x, xcd_chunk, xcds) * kRowsPerBlock + threadIdx.x / LR;
-    const uint64_t c_own = (static_cast<uint64_t>(blockIdx.y) * LR + lane) * V;
     if (row >= m) return;  // whole lane groups
     // Lanes past the last column still fetch their share of the row's nonzeros for the group;
-    // they compute on column 0 and store nothing.
-    const bool stores = c_own < n;
-    const uint64_t c0 = stores ? c_own : 0;
+    // they compute on the first columns and store nothing.
+    const LaneColumns own = lane_columns<V>((static_cast<uint64_t>(blockIdx.y) * LR + lane) * V, n);
+    const uint64_t c0 = own.first;
 
     const idx_t start = row_ptr[row] - base;
     const idx_t end = row_ptr[row + 1] - base;
@@ -48,7 +46,7 @@ __global__ __launch_bounds__(kBlock) void spmm_rowb_kernel(idx_t m, idx_t n, idx
     row_times_b<T, LR, V, WIDE>(start, end, lane, base, col, val, reinterpret_cast<const char*>(B),
                                 static_cast<off_t>(c0 * sizeof(T)), static_cast<off_t>(ldb * sizeof(T)), acc);
 
-    if (stores) store_c<T, V>(C, ldc, c_row_major, row, c0, acc, alpha, beta);
+    if (own.any) store_c<T, V>(C, ldc, c_row_major, row, c0, acc, alpha, beta, own.skip);
 }
 
 // The same product into a column-major C, without a row-major copy of C in between.  A workgroup owns kColumnRows
@@ -75,8 +73,8 @@ __global__ __launch_bounds__(kBlock) void spmm_rowb_columns_kernel(idx_t m, idx_
     const uint64_t row0 = xcd_position(blockIdx.x, xcd_chunk, xcds) * kColumnRows;
     if (row0 >= m) return;  // whole workgroup
     const uint64_t panel = static_cast<uint64_t>(blockIdx.y) * kCols;
-    const uint64_t c_own = panel + lane * V;
-    const uint64_t c0 = c_own < n ? c_own : 0;  // lanes past the last column only help fetching
+    const LaneColumns own = lane_columns<V>(panel + lane * V, n);  // lanes past the last column only help fetching
+    const uint64_t c0 = own.first;
 #pragma unroll 1
     for (int r0 = 0; r0 < kColumnRows; r0 += kRowsPerPass) {
         const int r = r0 + static_cast<int>(threadIdx.x) / LR;
@@ -89,7 +87,9 @@ __global__ __launch_bounds__(kBlock) void spmm_rowb_columns_kernel(idx_t m, idx_
         row_times_b<T, LR, V, WIDE>(start, end, lane, base, col, val, reinterpret_cast<const char*>(B),
                                     static_cast<off_t>(c0 * sizeof(T)), static_cast<off_t>(ldb * sizeof(T)), acc);
 #pragma unroll
-        for (int i = 0; i < V; ++i) s_c[lane * V + i][r] = acc[i];
+        for (int i = 0; i < V; ++i) {
+            if (i >= own.skip) s_c[lane * V + i - own.skip][r] = acc[i];
+        }
     }
     __syncthreads();
     const uint64_t row = row0 + threadIdx.x % kColumnRows;
@@ -128,9 +128,9 @@ __global__ __launch_bounds__(kBlock) void spmm_narrow_kernel(idx_t m, idx_t n, i
     constexpr int kGroups = kBlock / kLanes;
     const idx_t sub = threadIdx.x % kLanes;
     const idx_t phase = sub / C;
-    const uint64_t c_own = static_cast<uint64_t>(sub % C) * V;
-    const bool in_panel = c_own < n;
-    const uint64_t c0 = in_panel ? c_own : 0;
+    const LaneColumns own = lane_columns<V>(static_cast<uint64_t>(sub % C) * V, n);
+    const bool in_panel = own.any;
+    const uint64_t c0 = own.first;
     // the groups of a workgroup take neighbouring rows in every round
     const uint64_t first_row = xcd_position(blockIdx.x, xcd_chunk, xcds) * (kGroups * kNarrowRowsPerGroup) + threadIdx.x / kLanes;
     const uint64_t last_row = static_cast<uint64_t>(m) - 1;  // m != 0 here
@@ -141,7 +141,7 @@ __global__ __launch_bounds__(kBlock) void spmm_narrow_kernel(idx_t m, idx_t n, i
         for (int i = 0; i < V; ++i) zero[i] = T(0);
         for (int it = 0; it < kNarrowRowsPerGroup; ++it) {
             const uint64_t row = first_row + static_cast<uint64_t>(it) * kGroups;
-            if (row < m && phase == 0 && in_panel) store_c<T, V>(Cm, ldc, c_row_major, row, c0, zero, alpha, beta);
+            if (row < m && phase == 0 && in_panel) store_c<T, V>(Cm, ldc, c_row_major, row, c0, zero, alpha, beta, own.skip);
         }
         return;
     }
@@ -179,7 +179,7 @@ __global__ __launch_bounds__(kBlock) void spmm_narrow_kernel(idx_t m, idx_t n, i
         for (int i = 0; i < V; ++i) acc[i] = T(0);
         Vec<T, V> b[kSteps];
 #pragma unroll
-        for (int u = 0; u < kSteps; ++u) b[u] = load_vec<T, V>(B + static_cast<int64_t>(cc[u] - base) * ldb + c0);
+        for (int u = 0; u < kSteps; ++u) b[u] = load_row<T, V>(B + static_cast<int64_t>(cc[u] - base) * ldb + c0);
         // the next row's nonzeros and the offsets of the row after it, while those are on their way
         idx_t cc_next[kSteps];
         T aa_next[kSteps];
@@ -212,7 +212,7 @@ __global__ __launch_bounds__(kBlock) void spmm_narrow_kernel(idx_t m, idx_t n, i
             }
             Vec<T, V> b2[kSteps];
 #pragma unroll
-            for (int u = 0; u < kSteps; ++u) b2[u] = load_vec<T, V>(B + static_cast<int64_t>(c2[u] - base) * ldb + c0);
+            for (int u = 0; u < kSteps; ++u) b2[u] = load_row<T, V>(B + static_cast<int64_t>(c2[u] - base) * ldb + c0);
 #pragma unroll
             for (int u = 0; u < kSteps; ++u) {
                 if (at + u * P < end) {
@@ -235,7 +235,7 @@ __global__ __launch_bounds__(kBlock) void spmm_narrow_kernel(idx_t m, idx_t n, i
                 acc[i] += dpp_mov<kRowRor8>(acc[i]);
             }
         }
-        if (!left && phase == 0 && in_panel) store_c<T, V>(Cm, ldc, c_row_major, row, c0, acc, alpha, beta);
+        if (!left && phase == 0 && in_panel) store_c<T, V>(Cm, ldc, c_row_major, row, c0, acc, alpha, beta, own.skip);
         at = at_next;
         end = end_next;
         left = left_next;
@@ -763,10 +763,11 @@ void launch_spmm(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     if (a.m == 0 || a.n == 0) return;
     if (a.b_row_major) {
         constexpr int kWide = 16 / sizeof(T);  // elements per 128-bit access
-        const bool aligned = (reinterpret_cast<uintptr_t>(a.B) % 16 == 0) && (a.ldb % kWide == 0) &&
-                             (a.n % kWide == 0) &&
-                             (!a.c_row_major || ((reinterpret_cast<uintptr_t>(a.C) % 16 == 0) && (a.ldc % kWide == 0)));
-        if (aligned) launch_rowb_v<T, kWide>(stream, a, alpha, beta);
+        // Rows that begin at any element take the wide loads too (27-point stencil, 872 K rows, fp32: 5, 17, 50, 101
+        // columns 98, 283, 796, 1670 us with one element per lane, 64, 133, 304, 545 so; fp64, 33 columns: 1131, 538),
+        // but for the fewest fp64 columns: 7 in eight lanes of one element 143 us, in four of two 157.
+        const bool aligned = reinterpret_cast<uintptr_t>(a.B) % 16 == 0 && a.ldb % kWide == 0 && a.n % kWide == 0;
+        if (a.n >= kWide && (aligned || sizeof(T) == 4 || a.n > 8)) launch_rowb_v<T, kWide>(stream, a, alpha, beta);
         else launch_rowb_v<T, 1>(stream, a, alpha, beta);
     } else {
         constexpr int kJB = 4;
@@ -864,14 +865,6 @@ void launch_transpose_tile(hipStream_t stream, idx_t rows, idx_t cols, idx_t row
                        lds, dst, ldd, beta);
 }
 
-// Lanes per row of A that the row kernels use for the operands as they lie, V columns each.
-template <typename T>
-int columns_per_lane(const SpmmArgs& a) {
-    constexpr int kWide = 16 / sizeof(T);  // elements per 128-bit access
-    const bool aligned = (reinterpret_cast<uintptr_t>(a.B) % 16 == 0) && (a.ldb % kWide == 0) && (a.n % kWide == 0);
-    return aligned ? kWide : 1;
-}
-
 template <typename T, int LR, int V>
 void launch_columns(hipStream_t stream, const SpmmArgs& a, idx_t c_cols, T* C, int64_t ldc, T alpha, T beta) {
     const uint64_t blocks = (static_cast<uint64_t>(a.m) + kColumnRows - 1) / kColumnRows;
@@ -889,25 +882,17 @@ void launch_columns(hipStream_t stream, const SpmmArgs& a, idx_t c_cols, T* C, i
     }
 }
 
-template <typename T, int V>
-void launch_columns_v(hipStream_t stream, const SpmmArgs& a, idx_t c_cols, T* C, int64_t ldc, T alpha, T beta) {
-    const uint64_t lanes = (static_cast<uint64_t>(a.n) + V - 1) / V;
-    if (lanes <= 4) launch_columns<T, 4, V>(stream, a, c_cols, C, ldc, alpha, beta);
-    else if (lanes <= 8) launch_columns<T, 8, V>(stream, a, c_cols, C, ldc, alpha, beta);
-    else launch_columns<T, 16, V>(stream, a, c_cols, C, ldc, alpha, beta);
-}
-
 }  // namespace
 
 template <typename T>
 bool launch_spmm_columns(hipStream_t stream, const SpmmArgs& a, idx_t c_cols, T* C, int64_t ldc, T alpha, T beta) {
     if (!a.b_row_major || a.long_row != 0 || a.m == 0 || a.nnz == 0) return false;
     constexpr int kWide = 16 / sizeof(T);
-    const int v = columns_per_lane<T>(a);
-    const uint64_t lanes = (static_cast<uint64_t>(a.n) + v - 1) / v;
+    const uint64_t lanes = (static_cast<uint64_t>(a.n) + kWide - 1) / kWide;
     if (lanes <= 2 || lanes > 16) return false;
-    if (v == kWide) launch_columns_v<T, kWide>(stream, a, c_cols, C, ldc, alpha, beta);
-    else launch_columns_v<T, 1>(stream, a, c_cols, C, ldc, alpha, beta);
+    if (lanes <= 4) launch_columns<T, 4, kWide>(stream, a, c_cols, C, ldc, alpha, beta);
+    else if (lanes <= 8) launch_columns<T, 8, kWide>(stream, a, c_cols, C, ldc, alpha, beta);
+    else launch_columns<T, 16, kWide>(stream, a, c_cols, C, ldc, alpha, beta);
     return true;
 }
 

@@ -36,6 +36,38 @@ __device__ __forceinline__ Vec<T, V> load_vec(const T* p) {
     return r;
 }
 
+// A row of op(B) may begin at any element (widths and leading dimensions that are no multiple of the vector): the
+// hardware takes 128-bit accesses at any multiple of four bytes, so ragged operands keep the wide loads.
+template <typename T, int V>
+__device__ __forceinline__ Vec<T, V> load_row(const T* p) {
+    if constexpr (V == 1) {
+        return load_vec<T, V>(p);
+    } else {
+        typedef T Native __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+        Vec<T, V> r;
+        const Native n = *reinterpret_cast<const Native*>(p);
+#pragma unroll
+        for (int i = 0; i < V; ++i) r.v[i] = n[i];
+        return r;
+    }
+}
+
+// The columns of a lane of a row of n >= V columns: V from `own` on, moved back where fewer are left; the first `skip`
+// of them then belong to the lane before.  Lanes past the last column (own >= n) get the row's first columns.
+struct LaneColumns {
+    uint64_t first;
+    int skip;
+    bool any;
+};
+template <int V>
+__device__ __forceinline__ LaneColumns lane_columns(uint64_t own, uint64_t n) {
+    LaneColumns c;
+    c.any = own < n;
+    c.first = !c.any ? 0 : (own + V <= n ? own : n - V);
+    c.skip = c.any ? static_cast<int>(own - c.first) : V;
+    return c;
+}
+
 // Stores of C: written once and not read again by the call, so they are marked as streaming, which keeps the
 // rows of op(B) in cache and lets the lines leave as they fill (N = 64: 552 -> 535 us, N = 256: 1.90 -> 1.82 ms).
 template <typename T, int V>
@@ -43,7 +75,7 @@ __device__ __forceinline__ void store_vec(T* p, const Vec<T, V>& r) {
     if constexpr (V == 1) {
         __builtin_nontemporal_store(r.v[0], p);
     } else {
-        typedef T Native __attribute__((ext_vector_type(V)));
+        typedef T Native __attribute__((ext_vector_type(V), aligned(sizeof(T))));
         Native n;
 #pragma unroll
         for (int i = 0; i < V; ++i) n[i] = r.v[i];
@@ -122,7 +154,7 @@ __device__ __forceinline__ void row_times_b(idx_t begin, idx_t end, idx_t lane, 
                         constexpr int k = u0 + decltype(u)::value;
                         if (!kChecked || k < left) {  // the same for all lanes of the group
                             const off_t off = group_bcast<LR, k>(roff) + lane_off;
-                            b[decltype(u)::value] = load_vec<T, V>(reinterpret_cast<const T*>(B_bytes + off));
+                            b[decltype(u)::value] = load_row<T, V>(reinterpret_cast<const T*>(B_bytes + off));
                         }
                     });
                     static_for<kBatch>([&](auto u) {
@@ -141,19 +173,27 @@ __device__ __forceinline__ void row_times_b(idx_t begin, idx_t end, idx_t lane, 
     }
 }
 
-// Writes V adjacent columns of one row of C: beta*C + alpha*acc, C untouched by reads if beta == 0.
+// Writes V adjacent columns of one row of C but for the first `skip`: beta*C + alpha*acc, C untouched by reads if
+// beta == 0.
 template <typename T, int V>
 __device__ __forceinline__ void store_c(T* __restrict__ C, int64_t ldc, bool c_row_major, uint64_t row, uint64_t c0,
-                                        const T (&acc)[V], T alpha, T beta) {
+                                        const T (&acc)[V], T alpha, T beta, int skip = 0) {
     const bool beta0 = beta == T(0);
-    if (c_row_major) {
+    if (V > 1 && skip != 0) {
+        T* Cp = c_row_major ? C + static_cast<int64_t>(row) * ldc + c0 : C + static_cast<int64_t>(c0) * ldc + row;
+        const int64_t next = c_row_major ? 1 : ldc;
+#pragma unroll
+        for (int i = 1; i < V; ++i) {
+            if (i >= skip) Cp[i * next] = beta0 ? alpha * acc[i] : beta * Cp[i * next] + alpha * acc[i];
+        }
+    } else if (c_row_major) {
         T* Cp = C + static_cast<int64_t>(row) * ldc + c0;
         Vec<T, V> out;
         if (beta0) {
 #pragma unroll
             for (int i = 0; i < V; ++i) out.v[i] = alpha * acc[i];
         } else {
-            const Vec<T, V> old = load_vec<T, V>(Cp);
+            const Vec<T, V> old = load_row<T, V>(Cp);
 #pragma unroll
             for (int i = 0; i < V; ++i) out.v[i] = beta * old.v[i] + alpha * acc[i];
         }

@@ -119,7 +119,7 @@ __global__ __launch_bounds__(kBlock) void spmm_long_find_kernel(idx_t m, const i
 // lanes: lane groups of `lanes` threads (a power of two up to 64) hold the columns of a panel of lanes * V columns
 // (blockIdx.y walks the panels); the kBlock / lanes groups take the nonzeros of the piece in turn, kAhead rows of
 // op(B) in flight each, and their sums meet in LDS, added in the order of the groups.
-// op(B)(kk, j) lies at kk * b_rs + j * b_cs; V > 1 needs b_cs == 1 and 16-byte aligned rows (the launcher checks).
+// op(B)(kk, j) lies at kk * b_rs + j * b_cs; V > 1 needs b_cs == 1 and n >= V (the launcher checks).
 template <typename T, int V>
 __global__ __launch_bounds__(kBlock) void spmm_long_chunk_kernel(idx_t n, idx_t base, uint32_t lanes,
                                                                  const idx_t* __restrict__ row_ptr,
@@ -135,9 +135,8 @@ __global__ __launch_bounds__(kBlock) void spmm_long_chunk_kernel(idx_t n, idx_t 
     const uint32_t lane = tid % lanes;
     const uint32_t group = tid / lanes;
     const uint32_t groups = kBlock / lanes;
-    const uint64_t c_own = (static_cast<uint64_t>(blockIdx.y) * lanes + lane) * V;
-    const bool stores = c_own < n;
-    const uint64_t c0 = stores ? c_own : 0;
+    const LaneColumns own = lane_columns<V>((static_cast<uint64_t>(blockIdx.y) * lanes + lane) * V, n);
+    const uint64_t c0 = own.first;
     const uint32_t count = min(c->items, cap_items);
     const idx_t last_nonzero = nnz - 1;  // nnz != 0 where a row is long
     for (uint32_t it = blockIdx.x; it < count; it += gridDim.x) {
@@ -163,7 +162,7 @@ __global__ __launch_bounds__(kBlock) void spmm_long_chunk_kernel(idx_t n, idx_t 
             Vec<T, V> b[kAhead];
 #pragma unroll
             for (int u = 0; u < kAhead; ++u)
-                b[u] = load_vec<T, V>(B + static_cast<int64_t>(cc[u]) * b_rs + static_cast<int64_t>(c0) * b_cs);
+                b[u] = load_row<T, V>(B + static_cast<int64_t>(cc[u]) * b_rs + static_cast<int64_t>(c0) * b_cs);
 #pragma unroll
             for (int u = 0; u < kAhead; ++u) {
                 if (e + u * groups < end) {  // a lane without a nonzero stays out: 0 * inf would be NaN
@@ -183,13 +182,15 @@ __global__ __launch_bounds__(kBlock) void spmm_long_chunk_kernel(idx_t n, idx_t 
 #pragma unroll
                 for (int i = 0; i < V; ++i) sum[i] += s_sum[(g * lanes + lane) * V + i];
             }
-            if (stores) {
+            if (own.any) {
                 if (pieces == 1) {
-                    store_c<T, V>(C, ldc, c_row_major, row, c0, sum, alpha, beta);
+                    store_c<T, V>(C, ldc, c_row_major, row, c0, sum, alpha, beta, own.skip);
                 } else {
                     T* out = partials + static_cast<int64_t>(item.w + piece) * ld_partials + c0;
 #pragma unroll
-                    for (int i = 0; i < V; ++i) out[i] = sum[i];
+                    for (int i = 0; i < V; ++i) {
+                        if (i >= own.skip) out[i] = sum[i];
+                    }
                 }
             }
         }
@@ -209,7 +210,8 @@ __global__ __launch_bounds__(kBlock) void spmm_long_reduce_kernel(idx_t n, T* __
     for (uint64_t w = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; w < work;
          w += static_cast<uint64_t>(gridDim.x) * kBlock) {
         const uint4 entry = rows[w / per_row];
-        const uint64_t c0 = (w % per_row) * V;
+        const LaneColumns own = lane_columns<V>((w % per_row) * V, n);
+        const uint64_t c0 = own.first;
         if (entry.z == 0) continue;
         T sum[V];
 #pragma unroll
@@ -219,7 +221,7 @@ __global__ __launch_bounds__(kBlock) void spmm_long_reduce_kernel(idx_t n, T* __
 #pragma unroll
             for (int i = 0; i < V; ++i) sum[i] += in[i];
         }
-        store_c<T, V>(C, ldc, c_row_major, entry.x, c0, sum, alpha, beta);
+        store_c<T, V>(C, ldc, c_row_major, entry.x, c0, sum, alpha, beta, own.skip);
     }
 }
 
@@ -277,9 +279,7 @@ void launch_spmm_long_rows(hipStream_t stream, const SpmmArgs& a, T alpha, T bet
     const int64_t b_rs = a.b_row_major ? a.ldb : 1;
     const int64_t b_cs = a.b_row_major ? 1 : a.ldb;
     constexpr int kWide = 16 / sizeof(T);
-    const bool wide = a.b_row_major && (reinterpret_cast<uintptr_t>(a.B) % 16 == 0) && (a.ldb % kWide == 0) &&
-                      (a.n % kWide == 0) &&
-                      (!a.c_row_major || ((reinterpret_cast<uintptr_t>(a.C) % 16 == 0) && (a.ldc % kWide == 0)));
+    const bool wide = a.b_row_major && a.n >= kWide;
     const uint32_t v = wide ? kWide : 1;
     const uint64_t lanes_needed = (static_cast<uint64_t>(a.n) + v - 1) / v;
     uint32_t lanes = 1;

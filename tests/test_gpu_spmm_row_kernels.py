@@ -1,5 +1,5 @@
 """The SpMM kernels without a schedule at the edges of their workgroups: rows dealt to the XCDs in stretches, and
-column-major products written by the kernel that forms the sums.  Parity against the CPU oracle within
+column-major products written by the kernel that forms the sums, and widths that are no whole vectors.  Parity against the CPU oracle within
 8*u*(|alpha| * (|A||B|)_ij + |beta*C_ij|)."""
 import numpy as np
 import pytest
@@ -29,3 +29,16 @@ def test_column_major_product(torch_gpu, handle, oracle, m, n, dtype):
     for b_order in (api.ORDER_COL, api.ORDER_ROW):
         check(torch_gpu, handle, oracle, a, n, 1.5, 0.0, b_order=b_order, c_order=api.ORDER_COL, pad_b=1, pad_c=3)
         check(torch_gpu, handle, oracle, a, n, 1.5, -0.5, b_order=b_order, c_order=api.ORDER_COL)
+
+
+# widths that are no multiple of a 16-byte vector: the last lane's vector reaches back over columns of the lane before;
+# rows of op(B) and C that begin at any element
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 6, 7, 9, 15, 17, 31, 33, 63, 67, 129, 261])
+def test_ragged_widths(torch_gpu, handle, oracle, n, dtype):
+    a = wl.random_ragged(611, 530, 9, dtype=dtype, seed=n)
+    for pad_b, pad_c in ((0, 0), (3, 1), (1, 2)):
+        check(torch_gpu, handle, oracle, a, n, 1.5, 0.0, pad_b=pad_b, pad_c=pad_c)
+        check(torch_gpu, handle, oracle, a, n, 1.5, -0.5, pad_b=pad_b, pad_c=pad_c)
+        check(torch_gpu, handle, oracle, a, n, 1.5, -0.5, op_b=api.OP_T, b_order=api.ORDER_COL, c_order=api.ORDER_COL,
+              pad_b=pad_b, pad_c=pad_c)
