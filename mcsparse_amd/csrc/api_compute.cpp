@@ -559,15 +559,19 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
         // built in the buffer) takes the launches.
         if (A->nnz != 0 && a.m != 0 && a.n != 0) {
             bool may_have_long_rows = true;
+            a.long_row = mcsp::kSpmmLongRow;
             if (A->format == MCSPARSE_FORMAT_CSR && (batches == 1 || shared_structure)) {
                 const mcspStatus_t ps = ensure_plan(h, A, ia.rows, A->rows, A->row_num, A->nnz,
                                                     A->col_num * static_cast<int64_t>(sizeof(T)), buf + l.long_ws, true);
                 if (ps != MCSP_STATUS_SUCCESS) return ps;
-                if (A->plan.valid && A->plan.forced_family == kFamilyAuto)
+                if (A->plan.valid && A->plan.forced_family == kFamilyAuto) {
                     may_have_long_rows = A->plan.max_row_len > mcsp::kSpmmLongRow;
+                    a.long_row = mcsp::spmm_long_cut(a.m, a.nnz);
+                }
             }
-            if (may_have_long_rows) {
-                a.long_row = mcsp::kSpmmLongRow;
+            if (!may_have_long_rows) {
+                a.long_row = 0;
+            } else {
                 a.long_ws = buf + l.long_ws;
                 a.long_n = l.n_padded;
             }

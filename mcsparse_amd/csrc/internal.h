@@ -370,10 +370,21 @@ template <typename T>
 bool launch_spmm_columns(hipStream_t stream, const SpmmArgs& a, idx_t c_cols, T* C, int64_t ldc, T alpha, T beta);
 
 // Long rows (spmm_long.hip): a lane group of the row kernels walks a row by itself, so a row of tens of thousands
-// of nonzeros outlasts the rest of the launch.  Rows above kSpmmLongRow nonzeros are cut into pieces of
-// kSpmmLongChunk, a workgroup each.  The first 2 * kAlign bytes of the area are not used by these kernels (the
+// of nonzeros outlasts the rest of the launch.  Where a matrix has rows above kSpmmLongRow nonzeros, those above
+// spmm_long_cut are taken in pieces of kSpmmLongChunk, a workgroup each.  The first 2 * kAlign bytes of the area are not used by these kernels (the
 // row-length analysis of the call writes its counters there).
 constexpr idx_t kSpmmLongRow = 1024;
+// The cut lies below that limit, since the wavefronts of the row kernels wait for the longest of their rows: four times
+// the mean row length, between 256 (a workgroup's worth) and kSpmmLongRow.  Power-law rows, microseconds a call with a
+// cut of 128, 256, 512, 1024: a million rows and 32 fp32 columns 530, 549, 582, 650; 8 columns 403, 374, 375, 393;
+// 700 K rows and 100 columns 1078, 1051, 1038, 1032; 100 K rows and 24 columns 62, 71, 94, 141.  Where the longest row
+// is not known (COO, CSC, a capture that meets the matrix first) the cut is kSpmmLongRow: the mean row may be as long.
+constexpr idx_t kSpmmLongCutLeast = 256;
+inline idx_t spmm_long_cut(idx_t m, idx_t nnz) {
+    const uint64_t cut = 4 * (static_cast<uint64_t>(nnz) / m + 1);
+    if (cut <= kSpmmLongCutLeast) return kSpmmLongCutLeast;
+    return cut < kSpmmLongRow ? static_cast<idx_t>(cut) : kSpmmLongRow;
+}
 constexpr idx_t kSpmmLongChunk = 4096;
 size_t spmm_long_rows_bytes(idx_t nnz, int64_t n, size_t value_bytes);
 void launch_spmm_long_find(hipStream_t stream, const SpmmArgs& a, size_t value_bytes);

@@ -131,19 +131,42 @@ inline uint32_t xcd_stretch(uint64_t blocks, uint64_t rows_per_block, uint32_t x
 // all lanes of a group ask for the same word still returns a word per lane.  So the lanes fetch
 // LR nonzeros of the row at once, one each, turn them into row offsets, and pass offsets and
 // values round in registers; the loop then loads rows of op(B) and nothing else.
-template <typename T, int LR, int V, bool WIDE>
+//
+// AHEAD: the group takes every step / LR-th stretch of LR nonzeros from begin on (several groups on one long row), and
+// asks for the next one before the rows of op(B) of this one, so that a round costs one trip to memory instead of two
+// (places past the end read the last nonzero again: no load sits under a test).  Not for the short rows of a stencil,
+// which it makes slower (27 nonzeros, 16 fp64 columns: 178 -> 187 us): they have other rows to wait beside.
+template <typename T, int LR, int V, bool WIDE, bool AHEAD = false>
 __device__ __forceinline__ void row_times_b(idx_t begin, idx_t end, idx_t lane, idx_t base,
                                             const idx_t* __restrict__ col, const T* __restrict__ val,
                                             const char* __restrict__ B_bytes,
                                             typename ByteOffset<WIDE>::type lane_off,
-                                            typename ByteOffset<WIDE>::type ldb_bytes, T (&acc)[V]) {
+                                            typename ByteOffset<WIDE>::type ldb_bytes, T (&acc)[V],
+                                            idx_t step = LR) {
     typedef typename ByteOffset<WIDE>::type off_t;
     constexpr int kBatch = LR < 8 ? LR : 8;  // rows of op(B) in flight per lane
-    for (idx_t j = begin; j < end; j += LR) {
-        const bool has = j + lane < end;
-        const off_t roff = has ? static_cast<off_t>(col[j + lane] - base) * ldb_bytes : off_t(0);
-        const T aa = has ? val[j + lane] : T(0);
+    if (begin >= end) return;  // whole lane groups
+    idx_t c_next = 0;
+    T a_next = T(0);
+    if constexpr (AHEAD) {
+        c_next = col[min(begin + lane, end - 1)];
+        a_next = val[min(begin + lane, end - 1)];
+    }
+    for (idx_t j = begin; j < end; j += step) {
         const idx_t left = end - j;
+        off_t roff;
+        T aa;
+        if constexpr (AHEAD) {
+            roff = static_cast<off_t>(c_next - base) * ldb_bytes;
+            aa = a_next;
+            const idx_t next = left > step ? min(j + step + lane, end - 1) : end - 1;
+            c_next = col[next];
+            a_next = val[next];
+        } else {
+            const bool has = lane < left;
+            roff = has ? static_cast<off_t>(col[j + lane] - base) * ldb_bytes : off_t(0);
+            aa = has ? val[j + lane] : T(0);
+        }
         auto chunk = [&](auto checked) {
             constexpr bool kChecked = decltype(checked)::value;
             static_for<LR / kBatch>([&](auto g) {

@@ -2,8 +2,8 @@
 // nonzeros with a handful of loads in flight: a row of 50,000 nonzeros keeps that one group busy for
 // milliseconds after every other row is done (1 M power-law rows, N = 16: 7.3 ms, of which the longest row is 7).
 // The reference has the same shape (one wavefront per row and output column,
-// src/kernels/level3/spmm/csr_spmm_device.hpp:121-137).  Here rows longer than kSpmmLongRow are left out by the
-// row kernels and taken in pieces of kSpmmLongChunk nonzeros, a workgroup each:
+// src/kernels/level3/spmm/csr_spmm_device.hpp:121-137).  Here rows longer than the call's cut (256 to
+// 1024 nonzeros, spmm_long_cut) are left out by the row kernels and taken in pieces of kSpmmLongChunk nonzeros, a workgroup each:
 //   1. spmm_long_find_kernel lists the pieces (row, piece) and, for rows of several pieces, the rows;
 //   2. spmm_long_chunk_kernel forms the sums of a piece, all 256 threads on its nonzeros, and writes the row of C
 //      (one piece) or a row of partial sums (several);
@@ -52,7 +52,7 @@ __device__ __forceinline__ void write_long_row(uint32_t row, uint32_t pieces, ui
         items[first + j] = make_uint4(row, j, fits ? pieces : 0u, slot);
 }
 
-__global__ __launch_bounds__(kBlock) void spmm_long_find_kernel(idx_t m, const idx_t* __restrict__ row_ptr,
+__global__ __launch_bounds__(kBlock) void spmm_long_find_kernel(idx_t m, idx_t long_row, const idx_t* __restrict__ row_ptr,
                                                                 LongCounters* __restrict__ c, uint4* __restrict__ items,
                                                                 uint4* __restrict__ rows, uint32_t cap_items,
                                                                 uint32_t cap_rows, uint32_t cap_slots) {
@@ -83,7 +83,7 @@ __global__ __launch_bounds__(kBlock) void spmm_long_find_kernel(idx_t m, const i
         for (uint32_t u = 0; u < kAtOnce; ++u) {
             const uint64_t row = row0 + k0 + u * kBlock;
             const idx_t len = lens[u];
-            if (len <= kSpmmLongRow) continue;
+            if (len <= long_row) continue;
             const uint32_t pieces = (len + kSpmmLongChunk - 1) / kSpmmLongChunk;
             const uint32_t at = atomicAdd(&s_count, 1u);
             if (at < kFindList) {
@@ -198,6 +198,73 @@ __global__ __launch_bounds__(kBlock) void spmm_long_chunk_kernel(idx_t n, idx_t 
     }
 }
 
+// The same for operands of LR = 4 .. 64 lanes of whole vectors that lie within 4 GiB, where most of the work is: a
+// wavefront's groups take neighbouring stretches of LR nonzeros, one per lane, read ahead, and pass them round in
+// registers (row_times_b), so that a trip to memory brings eight rows of op(B) per lane; the kernel above makes two
+// dependent trips for four, and every lane of its groups loads the same nonzero.  What bounds it is the gather of op(B):
+// a million power-law rows, 32 fp32 columns, rows of more than 256 nonzeros: 325 us; before, with rows from 1024
+// on: 270 us beside a row kernel of 369, which now takes 200.  The sums of a wavefront's groups meet
+// in registers, those of the four wavefronts in LDS, in a fixed order.
+template <typename T, int LR, int V>
+__global__ __launch_bounds__(kBlock) void spmm_long_stretch_kernel(idx_t n, idx_t base, const idx_t* __restrict__ row_ptr,
+                                                                   const idx_t* __restrict__ col,
+                                                                   const T* __restrict__ val, const T* __restrict__ B,
+                                                                   int64_t ldb, T* __restrict__ C, int64_t ldc,
+                                                                   bool c_row_major, T alpha, T beta,
+                                                                   const LongCounters* __restrict__ c,
+                                                                   const uint4* __restrict__ items, uint32_t cap_items,
+                                                                   T* __restrict__ partials, int64_t ld_partials, idx_t nnz) {
+    constexpr int kWaves = kBlock / kWave;
+    __shared__ T s_sum[kWaves][LR * V];
+    const uint32_t lane = threadIdx.x % LR;
+    const uint32_t group = threadIdx.x / LR;
+    const uint32_t wave = threadIdx.x / kWave;
+    const LaneColumns own = lane_columns<V>((static_cast<uint64_t>(blockIdx.y) * LR + lane) * V, n);
+    const uint32_t count = min(c->items, cap_items);
+    for (uint32_t it = blockIdx.x; it < count; it += gridDim.x) {
+        const uint4 item = items[it];
+        const uint32_t row = item.x, piece = item.y, pieces = item.z;
+        if (pieces == 0) continue;  // whole workgroup: a row that found no room
+        const idx_t row_start = row_ptr[row] - base;
+        const idx_t row_end = min(row_ptr[row + 1] - base, nnz);
+        const idx_t start = row_start + piece * kSpmmLongChunk;
+        const idx_t end = min(start + static_cast<idx_t>(kSpmmLongChunk), row_end);
+        T acc[V];
+#pragma unroll
+        for (int i = 0; i < V; ++i) acc[i] = T(0);
+        row_times_b<T, LR, V, false, true>(start + group * LR, end, lane, base, col, val, reinterpret_cast<const char*>(B),
+                                           static_cast<uint32_t>(own.first * sizeof(T)),
+                                           static_cast<uint32_t>(ldb * sizeof(T)), acc, kBlock);
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+#pragma unroll
+            for (int off = LR; off < kWave; off <<= 1) acc[i] += __shfl_xor(acc[i], off, kWave);
+        }
+        if (threadIdx.x % kWave < LR) {
+#pragma unroll
+            for (int i = 0; i < V; ++i) s_sum[wave][lane * V + i] = acc[i];
+        }
+        __syncthreads();
+        if (group == 0 && own.any) {
+#pragma unroll
+            for (int w = 1; w < kWaves; ++w) {
+#pragma unroll
+                for (int i = 0; i < V; ++i) acc[i] += s_sum[w][lane * V + i];
+            }
+            if (pieces == 1) {
+                store_c<T, V>(C, ldc, c_row_major, row, own.first, acc, alpha, beta, own.skip);
+            } else {
+                T* out = partials + static_cast<int64_t>(item.w + piece) * ld_partials + own.first;
+#pragma unroll
+                for (int i = 0; i < V; ++i) {
+                    if (i >= own.skip) out[i] = acc[i];
+                }
+            }
+        }
+        __syncthreads();  // the sums are read before the next piece writes them
+    }
+}
+
 // One thread per (row of several pieces, V columns): the partial sums of the pieces in their order.
 template <typename T, int V>
 __global__ __launch_bounds__(kBlock) void spmm_long_reduce_kernel(idx_t n, T* __restrict__ C, int64_t ldc,
@@ -232,13 +299,14 @@ struct LongLayout {
 };
 
 // A row of several pieces is longer than a piece, so there are at most nnz / piece such rows, with at most
-// 2 * nnz / piece pieces (ceil(len / piece) <= 2 * len / piece); rows of one piece number at most nnz / kSpmmLongRow.
+// 2 * nnz / piece pieces (ceil(len / piece) <= 2 * len / piece); rows of one piece number at most
+// nnz / kSpmmLongCutLeast.
 LongLayout long_layout(idx_t nnz, int64_t n, size_t value_bytes) {
     LongLayout l;
     const uint64_t per_piece = static_cast<uint64_t>(nnz) / kSpmmLongChunk;
     l.cap_rows = static_cast<uint32_t>(per_piece + 1);
     l.cap_slots = static_cast<uint32_t>(2 * per_piece + 2);
-    l.cap_items = static_cast<uint32_t>(static_cast<uint64_t>(nnz) / kSpmmLongRow + 2 * per_piece + 2);
+    l.cap_items = static_cast<uint32_t>(static_cast<uint64_t>(nnz) / kSpmmLongCutLeast + 2 * per_piece + 2);
     l.ld_partials = (n + 3) / 4 * 4;
     size_t off = 0;
     // the first kAlign bytes are left to the row-length analysis of the call (34 counters)
@@ -260,7 +328,7 @@ void launch_spmm_long_find(hipStream_t stream, const SpmmArgs& a, size_t value_b
     char* w = static_cast<char*>(a.long_ws);
     LongCounters* c = reinterpret_cast<LongCounters*>(w + l.counters);
     hipLaunchKernelGGL(spmm_long_zero_kernel, dim3(1), dim3(1), 0, stream, c);
-    hipLaunchKernelGGL(spmm_long_find_kernel, dim3((a.m + kFindRows - 1) / kFindRows), dim3(kBlock), 0, stream, a.m, a.row_ptr,
+    hipLaunchKernelGGL(spmm_long_find_kernel, dim3((a.m + kFindRows - 1) / kFindRows), dim3(kBlock), 0, stream, a.m, a.long_row, a.row_ptr,
                        c, reinterpret_cast<uint4*>(w + l.items), reinterpret_cast<uint4*>(w + l.rows), l.cap_items,
                        l.cap_rows, l.cap_slots);
 }
@@ -288,16 +356,31 @@ void launch_spmm_long_rows(hipStream_t stream, const SpmmArgs& a, T alpha, T bet
     // pieces are few (a 2048th of the nonzeros at most): a grid that lets every compute unit hold several
     const dim3 grid(2048, panels);
     const uint32_t reduce_blocks = 1024;
-    if (wide) {
+    auto stretches = [&](auto lr) {
+        constexpr int LR = decltype(lr)::value;
+        hipLaunchKernelGGL((spmm_long_stretch_kernel<T, LR, kWide>), grid, dim3(kBlock), 0, stream, a.n, a.base, a.row_ptr,
+                           a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta, c, items, l.cap_items, partials,
+                           l.ld_partials, a.nnz);
+    };
+    if (wide && lanes >= 4 && narrow_offsets(a, sizeof(T))) {
+        if (lanes == 4) stretches(std::integral_constant<int, 4>{});
+        else if (lanes == 8) stretches(std::integral_constant<int, 8>{});
+        else if (lanes == 16) stretches(std::integral_constant<int, 16>{});
+        else if (lanes == 32) stretches(std::integral_constant<int, 32>{});
+        else stretches(std::integral_constant<int, 64>{});
+    } else if (wide) {
         hipLaunchKernelGGL((spmm_long_chunk_kernel<T, kWide>), grid, dim3(kBlock), 0, stream, a.n, a.base, lanes,
                            a.row_ptr, a.col, val, B, b_rs, b_cs, C, a.ldc, a.c_row_major, alpha, beta, c, items,
                            l.cap_items, partials, l.ld_partials, a.nnz);
-        hipLaunchKernelGGL((spmm_long_reduce_kernel<T, kWide>), dim3(reduce_blocks), dim3(kBlock), 0, stream, a.n, C,
-                           a.ldc, a.c_row_major, alpha, beta, c, rows, l.cap_rows, partials, l.ld_partials);
     } else {
         hipLaunchKernelGGL((spmm_long_chunk_kernel<T, 1>), grid, dim3(kBlock), 0, stream, a.n, a.base, lanes, a.row_ptr,
                            a.col, val, B, b_rs, b_cs, C, a.ldc, a.c_row_major, alpha, beta, c, items, l.cap_items,
                            partials, l.ld_partials, a.nnz);
+    }
+    if (wide) {
+        hipLaunchKernelGGL((spmm_long_reduce_kernel<T, kWide>), dim3(reduce_blocks), dim3(kBlock), 0, stream, a.n, C,
+                           a.ldc, a.c_row_major, alpha, beta, c, rows, l.cap_rows, partials, l.ld_partials);
+    } else {
         hipLaunchKernelGGL((spmm_long_reduce_kernel<T, 1>), dim3(reduce_blocks), dim3(kBlock), 0, stream, a.n, C, a.ldc,
                            a.c_row_major, alpha, beta, c, rows, l.cap_rows, partials, l.ld_partials);
     }

@@ -1,5 +1,5 @@
-"""mcsparseSpMM on matrices with rows far longer than the rest: rows above 1024 nonzeros are cut into pieces of
-4096 that a workgroup each takes (one piece: the row of C written directly; several: partial sums added in the order
+"""mcsparseSpMM on matrices with rows far longer than the rest: rows above 256 to 1024 nonzeros (four times the mean)
+are cut into pieces of 4096 that a workgroup each takes (one piece: the row of C written directly; several: partial sums added in the order
 of the pieces).  Parity against the CPU oracle within 8*u*(|alpha| * (|A||B|)_ij + |beta*C_ij|), bits that repeat
 from run to run, and the time of a call."""
 import numpy as np
@@ -126,3 +126,18 @@ def test_a_row_of_fifty_thousand_does_not_hold_the_call_up(torch_gpu, handle):
     torch.cuda.synchronize()
     ms = e0.elapsed_time(e1) / 10
     assert ms < 2.0, ms
+
+
+# rows around the cut of a matrix that has longer ones (256, or four times the mean), widths of every lane count
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [2, 4, 9, 13, 17, 31, 50, 67, 130])
+@pytest.mark.parametrize("short", [2, 100])
+def test_rows_around_the_cut(torch_gpu, handle, oracle, n, dtype, short):
+    cut = 256
+    for _ in range(8):  # the cut is four times the mean row length, and its rows are part of the mean
+        lengths = ([short] * 97 + [255, 256, 257, cut - 1, cut, cut + 1, 0, 1100]) * 2
+        cut = max(256, 4 * (sum(lengths) // len(lengths) + 1))
+    assert cut + 1 in lengths and cut < 1024
+    a = rows_of_lengths(lengths, 5003, dtype, seed=n)
+    check(torch_gpu, handle, oracle, a, n, 1.25, 0.0, pad_b=1)
+    check(torch_gpu, handle, oracle, a, n, 1.25, -0.5, seed=1, c_order=api.ORDER_COL)
