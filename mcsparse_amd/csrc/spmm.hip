@@ -51,12 +51,14 @@ __global__ __launch_bounds__(kBlock) void spmm_rowb_kernel(idx_t m, idx_t n, idx
 
 // The same product into a column-major C, without a row-major copy of C in between.  A workgroup owns kColumnRows
 // neighbouring rows, kBlock / LR at a time, gathers their sums in LDS and writes a column's stretch of rows as it lies
-// in C (512 bytes in fp64, 256 in fp32).  For LR <= 16: wider panels of as many rows do not fit LDS several times.
+// in C (256 bytes in fp64, 128 in fp32, and more for LR = 4; 64 rows in two passes: 236 us a call against 226 for 16
+// fp64 columns).  For LR <= 16: wider panels of as many rows do not fit LDS several times.
 // Measured together with the narrower tiles of transpose_kernel, 27-point stencil of 872 K rows: 16 fp64 columns 297 ->
-// 235 us a call, 4 fp64 columns (narrow kernel, tiles alone) 186 -> 125, 12 fp32 columns 169 -> 133, 31 fp32 columns
+// 226 us a call, 4 fp64 columns (narrow kernel, tiles alone) 186 -> 125, 12 fp32 columns 169 -> 133, 31 fp32 columns
 // 344 -> 339.
 // C has c_cols columns, n of op(B) (n >= c_cols) may be padded to whole vectors.
-constexpr int kColumnRows = 64;
+template <int LR>
+constexpr int kColumnRows = kBlock / LR > 32 ? kBlock / LR : 32;
 template <typename T, int LR, int V, bool WIDE>
 __global__ __launch_bounds__(kBlock) void spmm_rowb_columns_kernel(idx_t m, idx_t n, idx_t c_cols, idx_t base,
                                                                    const idx_t* __restrict__ row_ptr,
@@ -67,16 +69,16 @@ __global__ __launch_bounds__(kBlock) void spmm_rowb_columns_kernel(idx_t m, idx_
     typedef typename ByteOffset<WIDE>::type off_t;
     constexpr int kRowsPerPass = kBlock / LR;
     constexpr int kCols = LR * V;
-    static_assert(kColumnRows % kRowsPerPass == 0, "whole passes");
-    __shared__ T s_c[kCols][kColumnRows + 1];
+    static_assert(kColumnRows<LR> % kRowsPerPass == 0, "whole passes");
+    __shared__ T s_c[kCols][kColumnRows<LR> + 1];
     const idx_t lane = threadIdx.x % LR;
-    const uint64_t row0 = xcd_position(blockIdx.x, xcd_chunk, xcds) * kColumnRows;
+    const uint64_t row0 = xcd_position(blockIdx.x, xcd_chunk, xcds) * kColumnRows<LR>;
     if (row0 >= m) return;  // whole workgroup
     const uint64_t panel = static_cast<uint64_t>(blockIdx.y) * kCols;
     const LaneColumns own = lane_columns<V>(panel + lane * V, n);  // lanes past the last column only help fetching
     const uint64_t c0 = own.first;
 #pragma unroll 1
-    for (int r0 = 0; r0 < kColumnRows; r0 += kRowsPerPass) {
+    for (int r0 = 0; r0 < kColumnRows<LR>; r0 += kRowsPerPass) {
         const int r = r0 + static_cast<int>(threadIdx.x) / LR;
         const uint64_t row = row0 + r < m ? row0 + r : m - 1;  // rows past the end repeat the last one
         const idx_t start = row_ptr[row] - base;
@@ -92,13 +94,13 @@ __global__ __launch_bounds__(kBlock) void spmm_rowb_columns_kernel(idx_t m, idx_
         }
     }
     __syncthreads();
-    const uint64_t row = row0 + threadIdx.x % kColumnRows;
+    const uint64_t row = row0 + threadIdx.x % kColumnRows<LR>;
     if (row >= m) return;
 #pragma unroll 4
-    for (int c = threadIdx.x / kColumnRows; c < kCols; c += kBlock / kColumnRows) {
+    for (int c = threadIdx.x / kColumnRows<LR>; c < kCols; c += kBlock / kColumnRows<LR>) {
         if (panel + c >= c_cols) break;
         T* out = C + static_cast<int64_t>(panel + c) * ldc + static_cast<int64_t>(row);
-        const T v = alpha * s_c[c][threadIdx.x % kColumnRows];
+        const T v = alpha * s_c[c][threadIdx.x % kColumnRows<LR>];
         *out = beta == T(0) ? v : beta * *out + v;
     }
 }
@@ -867,9 +869,9 @@ void launch_transpose_tile(hipStream_t stream, idx_t rows, idx_t cols, idx_t row
 
 template <typename T, int LR, int V>
 void launch_columns(hipStream_t stream, const SpmmArgs& a, idx_t c_cols, T* C, int64_t ldc, T alpha, T beta) {
-    const uint64_t blocks = (static_cast<uint64_t>(a.m) + kColumnRows - 1) / kColumnRows;
+    const uint64_t blocks = (static_cast<uint64_t>(a.m) + kColumnRows<LR> - 1) / kColumnRows<LR>;
     const uint32_t xcds = device_topology().xcds;
-    const uint32_t chunk = xcd_stretch(blocks, kColumnRows, xcds);
+    const uint32_t chunk = xcd_stretch(blocks, kColumnRows<LR>, xcds);
     const dim3 grid(xcd_padded_grid(blocks, chunk, xcds), (a.n + LR * V - 1) / (LR * V));
     const T* val = static_cast<const T*>(a.val);
     const T* B = static_cast<const T*>(a.B);
