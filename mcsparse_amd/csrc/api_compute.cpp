@@ -566,7 +566,7 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
                 if (ps != MCSP_STATUS_SUCCESS) return ps;
                 if (A->plan.valid && A->plan.forced_family == kFamilyAuto) {
                     may_have_long_rows = A->plan.max_row_len > mcsp::kSpmmLongRow;
-                    a.long_row = mcsp::spmm_long_cut(a.m, a.nnz);
+                    a.long_row = mcsp::spmm_long_cut(a.m, a.nnz, static_cast<size_t>(a.n) * sizeof(T) <= 16);
                 }
             }
             if (!may_have_long_rows) {

@@ -380,7 +380,9 @@ constexpr idx_t kSpmmLongRow = 1024;
 // 700 K rows and 100 columns 1078, 1051, 1038, 1032; 100 K rows and 24 columns 62, 71, 94, 141.  Where the longest row
 // is not known (COO, CSC, a capture that meets the matrix first) the cut is kSpmmLongRow: the mean row may be as long.
 constexpr idx_t kSpmmLongCutLeast = 256;
-inline idx_t spmm_long_cut(idx_t m, idx_t nnz) {
+// Nor where a row of op(B) is one lane: the sums of 256 groups are then added by one thread, a long way for 256 nonzeros.
+inline idx_t spmm_long_cut(idx_t m, idx_t nnz, bool one_lane) {
+    if (one_lane) return kSpmmLongRow;
     const uint64_t cut = 4 * (static_cast<uint64_t>(nnz) / m + 1);
     if (cut <= kSpmmLongCutLeast) return kSpmmLongCutLeast;
     return cut < kSpmmLongRow ? static_cast<idx_t>(cut) : kSpmmLongRow;

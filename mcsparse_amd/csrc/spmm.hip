@@ -16,9 +16,12 @@ namespace {
 using namespace spmm_detail;
 
 // op(B) row-major.  LR lanes per row of A, V adjacent columns per lane; blockIdx.y walks the
-// column panels of LR*V columns.  V > 1 requires n >= V, which the launcher checks.
-template <typename T, int LR, int V, bool WIDE>
-__global__ __launch_bounds__(kBlock) void spmm_rowb_kernel(idx_t m, idx_t n, idx_t base,
+// column panels of LR*V columns.  V > 1 requires n >= V, which the launcher checks; RAGGED: n need not be a multiple of
+// V.  Eight wavefronts per SIMD are asked for outright: left alone, the scheduler draws the batches of sixteen lanes
+// together into 102 registers instead of 59, four wavefronts (27-point stencil 128^3, 64 fp32 columns: 636 -> 707 us).
+// Not in fp64, where five or six wavefronts do better (16 columns 420 us, 439 with eight; 32 columns 657 and 677).
+template <typename T, int LR, int V, bool WIDE, bool RAGGED>
+__global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 8 : 1) void spmm_rowb_kernel(idx_t m, idx_t n, idx_t base,
                                                            const idx_t* __restrict__ row_ptr,
                                                            const idx_t* __restrict__ col, const T* __restrict__ val,
                                                            const T* __restrict__ B, int64_t ldb, T* __restrict__ C,
@@ -31,7 +34,7 @@ __global__ __launch_bounds__(kBlock) void spmm_rowb_kernel(idx_t m, idx_t n, idx
     if (row >= m) return;  // whole lane groups
     // Lanes past the last column still fetch their share of the row's nonzeros for the group;
     // they compute on the first columns and store nothing.
-    const LaneColumns own = lane_columns<V>((static_cast<uint64_t>(blockIdx.y) * LR + lane) * V, n);
+    const LaneColumns own = lane_columns<V, RAGGED>((static_cast<uint64_t>(blockIdx.y) * LR + lane) * V, n);
     const uint64_t c0 = own.first;
 
     const idx_t start = row_ptr[row] - base;
@@ -727,22 +730,29 @@ void launch_rowb(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     const uint64_t row_blocks = (static_cast<uint64_t>(a.m) + (kBlock / LR) - 1) / (kBlock / LR);
     const uint64_t panels = (static_cast<uint64_t>(a.n) + LR * V - 1) / (LR * V);
     const uint32_t xcds = device_topology().xcds;
-    // wider operands than 16 lanes gained nothing from stretches (power-law rows of 17 columns in 32 lanes: 1365 us in
-    // plain turns, 1400 in stretches)
-    const uint32_t chunk = LR <= 16 ? xcd_stretch(row_blocks, kBlock / LR, xcds) : 1;
+    // from sixteen lanes on a workgroup holds few rows, and stretches cost more than they give (27-point stencil 128^3
+    // in fp32: 16 columns 315 us in plain turns, 299 in stretches; 32 columns 377 and 379; 64 columns 636 and 674)
+    const uint32_t chunk = LR <= 8 ? xcd_stretch(row_blocks, kBlock / LR, xcds) : 1;
     const dim3 grid(xcd_padded_grid(row_blocks, chunk, xcds), static_cast<uint32_t>(panels));
     const T* val = static_cast<const T*>(a.val);
     const T* B = static_cast<const T*>(a.B);
     T* C = static_cast<T*>(a.C);
-    if (narrow_offsets(a, sizeof(T))) {
-        hipLaunchKernelGGL((spmm_rowb_kernel<T, LR, V, false>), grid, dim3(kBlock), 0, stream, a.m, a.n, a.base,
-                           a.row_ptr, a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta, a.long_row, chunk,
-                           xcds);
-    } else {
-        hipLaunchKernelGGL((spmm_rowb_kernel<T, LR, V, true>), grid, dim3(kBlock), 0, stream, a.m, a.n, a.base,
-                           a.row_ptr, a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta, a.long_row, chunk,
-                           xcds);
+    auto launch = [&](auto wide, auto ragged) {
+        hipLaunchKernelGGL((spmm_rowb_kernel<T, LR, V, decltype(wide)::value, decltype(ragged)::value>), grid, dim3(kBlock), 0,
+                           stream, a.m, a.n, a.base, a.row_ptr, a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta,
+                           a.long_row, chunk, xcds);
+    };
+    auto launch_offsets = [&](auto ragged) {
+        if (narrow_offsets(a, sizeof(T))) launch(std::false_type{}, ragged);
+        else launch(std::true_type{}, ragged);
+    };
+    if constexpr (V > 1) {
+        if (a.n % V != 0) {
+            launch_offsets(std::true_type{});
+            return;
+        }
     }
+    launch_offsets(std::false_type{});
 }
 
 template <typename T, int V>

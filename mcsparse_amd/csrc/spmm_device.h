@@ -59,12 +59,17 @@ struct LaneColumns {
     int skip;
     bool any;
 };
-template <int V>
+template <int V, bool RAGGED = true>
 __device__ __forceinline__ LaneColumns lane_columns(uint64_t own, uint64_t n) {
     LaneColumns c;
     c.any = own < n;
-    c.first = !c.any ? 0 : (own + V <= n ? own : n - V);
-    c.skip = c.any ? static_cast<int>(own - c.first) : V;
+    if constexpr (RAGGED) {
+        c.first = !c.any ? 0 : (own + V <= n ? own : n - V);
+        c.skip = c.any ? static_cast<int>(own - c.first) : V;
+    } else {  // n is a multiple of V
+        c.first = c.any ? own : 0;
+        c.skip = 0;
+    }
     return c;
 }
 
