@@ -109,7 +109,10 @@ __device__ __forceinline__ W load_at(const void* array, uint32_t index) {
 }
 
 // Reads of a tile of an array through a buffer resource that ends with the tile: places past the end read as zero
-// without a test, and a thread's items differ by constants only (no register per item).
+// without a test, and a thread's items differ by constants only.  A place, its constant part included, goes into the
+// offset operand, which the hardware compares with the resource's length (constants below 4096 bytes travel in the
+// instruction, larger ones cost an addition for every 4096 bytes); the scalar offset operand is no part of that
+// comparison and stays zero.
 struct TileReader {
     __amdgpu_buffer_rsrc_t tile;
     __device__ __forceinline__ TileReader(const void* first, uint32_t bytes) {
@@ -117,14 +120,14 @@ struct TileReader {
         tile = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(first), 0, static_cast<int>(bytes), kRawDwords);
     }
     template <typename W>
-    __device__ __forceinline__ W read(uint32_t place, int constant_places) const {
+    __device__ __forceinline__ W read(uint32_t place, uint32_t constant_places) const {
         constexpr int kNonTemporal = 2;
+        const int offset = static_cast<int>((place + constant_places) * sizeof(W));
         if constexpr (sizeof(W) == 4) {
-            return __builtin_amdgcn_raw_buffer_load_b32(tile, static_cast<int>(place * 4), constant_places * 4, kNonTemporal);
+            return __builtin_amdgcn_raw_buffer_load_b32(tile, offset, 0, kNonTemporal);
         } else {
             typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-            return __builtin_bit_cast(W, static_cast<u32x2>(__builtin_amdgcn_raw_buffer_load_b64(
-                                             tile, static_cast<int>(place * 8), constant_places * 8, kNonTemporal)));
+            return __builtin_bit_cast(W, static_cast<u32x2>(__builtin_amdgcn_raw_buffer_load_b64(tile, offset, 0, kNonTemporal)));
         }
     }
 };
