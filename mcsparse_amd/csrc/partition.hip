@@ -1067,6 +1067,9 @@ bool sort_shape(uint32_t count, uint32_t key_count, uint32_t minor_bits, SortSha
     s->max_tiles2 = s->d2 != 0 ? count / kSecondTile + (1u << s->d1) : 0;
     return true;
 }
+// Bytes a key travels in behind step 1 (step 2 reads 16 bits) and behind step 2.
+size_t first_key_bytes(const SortShape& s) { return s.d2 == 0 && s.d3 <= 8 ? sizeof(uint8_t) : sizeof(uint16_t); }
+size_t second_key_bytes(const SortShape& s) { return s.d3 <= 8 ? sizeof(uint8_t) : sizeof(uint16_t); }
 void sort_passes(const SortShape& s, SortTables* t) {
     const uint32_t minor = s.minor_bits == kNoMinorKey ? 0 : s.minor_bits;
     auto passes_for = [](uint32_t bits) { return (bits + kPassBits - 1) / kPassBits; };
@@ -1097,10 +1100,10 @@ SortLayout sort_layout(uint32_t count, const SortShape& s, size_t value_bytes) {
         off += align_up(bytes);
         return at;
     };
-    l.keys1 = take(places1 * (s.d2 + s.d3 > 8 ? sizeof(uint16_t) : sizeof(uint8_t)));
+    l.keys1 = take(places1 * first_key_bytes(s));
     l.aux1 = take(places1 * sizeof(uint32_t));
     l.vals1 = take(places1 * value_bytes);
-    l.keys2 = take(places2 * (s.d3 > 8 ? sizeof(uint16_t) : sizeof(uint8_t)));
+    l.keys2 = take(places2 * second_key_bytes(s));
     l.aux2 = take(places2 * sizeof(uint32_t));
     l.vals2 = take(places2 * value_bytes);
     l.table1 = take(runs1 * sizeof(uint32_t));
@@ -1166,7 +1169,7 @@ void launch_sort(hipStream_t stream, EntrySource in, const SortShape& s, const S
     t.count = in.count;
     const uint32_t shift = s.d2 + s.d3;
     constexpr bool kMany = KIND == kPlain;  // the sorts by two keys
-    const bool short_keys1 = shift <= 8, short_keys2 = s.d3 <= 8;
+    const bool short_keys1 = first_key_bytes(s) == 1, short_keys2 = second_key_bytes(s) == 1;
     auto* partition = s.d1 <= 8 ? (short_keys1 ? launch_partition<VB, KIND, 8, uint8_t> : launch_partition<VB, KIND, 8, uint16_t>)
                                 : (short_keys1 ? launch_partition<VB, KIND, kMaxOneLevelBits, uint8_t>
                                                : launch_partition<VB, KIND, kMaxOneLevelBits, uint16_t>);

@@ -62,6 +62,8 @@ ONE_LEVEL_UPTO = 4300 << 11  # entries up to which one partition makes the bucke
     ("uniform", 300000, 1 << 20, ONE_LEVEL_UPTO, 0), ("uniform", 300000, (1 << 20) + 1, ONE_LEVEL_UPTO + 1, 1),
     ("few", 300000, 1 << 22, ONE_LEVEL_UPTO + 777, 0), ("band", 300000, 3000000, 2 * ONE_LEVEL_UPTO, 0),
     ("uniform", 20000, (1 << 24) + 1, 500000, 0),
+    # two levels with keys short enough for 8 bits behind the first one
+    ("uniform", 300000, 4000, ONE_LEVEL_UPTO + 1, 0), ("few", 300000, 1 << 14, ONE_LEVEL_UPTO + 777, 1),
 ])
 def test_csr2csc_bit_exact(torch_gpu, handle, oracle, dtype, action, kind, m, n, nnz, base):
     torch = torch_gpu
@@ -91,7 +93,7 @@ def test_csr2csc_bit_exact(torch_gpu, handle, oracle, dtype, action, kind, m, n,
     ("uniform", 3, 2, 1), ("uniform", 90, 3000000, 6144), ("uniform", 3000000, 90, 6145), ("few", 40, 50, 70000),
     ("few", 4000, 70000, 300000), ("band", 300000, 40000, 1000000), ("uniform", 1 << 23, 1 << 22, 100000),
     ("few", 100000, 1 << 22, ONE_LEVEL_UPTO), ("uniform", 1 << 22, 1 << 20, ONE_LEVEL_UPTO + 1),
-    ("uniform", 1 << 24, 300, 50000),
+    ("uniform", 1 << 24, 300, 50000), ("uniform", 5000, 100000, ONE_LEVEL_UPTO + 1),
 ])
 def test_coosort_bit_exact(torch_gpu, handle, oracle, by, with_perm, kind, m, n, nnz):
     torch = torch_gpu
