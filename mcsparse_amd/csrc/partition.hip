@@ -953,12 +953,14 @@ __global__ __launch_bounds__(kBucketThreads) void oversize_kernel(SortTables t, 
                 }
             }
         }
+        wait_for_stores();
         __syncthreads();
         if (tid == 0)
             s_last = __hip_atomic_fetch_add(&o.done[work.phase], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1 == o.chunks;
         __syncthreads();
         if (s_last != 0) {  // whole workgroup
             if (counting) place_chunks(t, o, out, t.passes == 1, pass.bits, s_sum, s.wave);
+            wait_for_stores();
             __syncthreads();
             if (tid == 0) __hip_atomic_store(&o.phase, work.phase + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
         }

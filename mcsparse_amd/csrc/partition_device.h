@@ -68,6 +68,11 @@ __device__ __forceinline__ void keep_equal_digits(uint32_t d, uint32_t bits, uin
     }
 }
 
+// Waits until this wavefront's stores have reached the L2.  A barrier does not (the L1 keeps a workgroup's accesses in
+// order, so the compiler asks for no wait there): what all wavefronts have written can be released to other workgroups by
+// one of them only if each has waited so before the barrier.
+__device__ __forceinline__ void wait_for_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // ---- one workgroup ---------------------------------------------------------------------------------------------
 // Exclusive sum over the threads of a workgroup; s_wave: THREADS / 64 words.  Holds one barrier; s_wave may be reused
 // after the caller's next barrier.

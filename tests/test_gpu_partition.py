@@ -116,3 +116,25 @@ def test_coosort_bit_exact(torch_gpu, handle, oracle, by, with_perm, kind, m, n,
     assert np.array_equal(d_c.cpu().numpy(), cols[want])
     if with_perm:
         assert np.array_equal(d_p.cpu().numpy(), perm[want])
+
+
+@pytest.mark.parametrize("share", [0.3])
+def test_a_row_with_most_of_ten_million_entries(torch_gpu, handle, share):
+    """Many more pieces of one bucket than workgroups that work on it, in every pass: what one workgroup writes is read
+    by others of the same launch, on other XCDs."""
+    torch = torch_gpu
+    m, n, nnz = 1 << 22, 1 << 20, 10000000
+    rng = np.random.default_rng(int(10 * share))
+    rows = np.where(rng.random(nnz) < share, m // 3, rng.integers(0, m, nnz)).astype(np.int32)
+    cols, perm = rng.integers(0, n, nnz).astype(np.int32), np.arange(nnz, dtype=np.int32)
+    want = np.argsort(rows.astype(np.int64) * n + cols, kind="stable")
+    st, size = api.sort_buffer_size(handle, "coo", m, n, nnz, dev(torch, rows), dev(torch, cols))
+    assert st == api.STATUS_SUCCESS
+    buf = torch.empty(size, dtype=torch.uint8, device="cuda")
+    for _ in range(3):
+        d_r, d_c, d_p = dev(torch, rows), dev(torch, cols), dev(torch, perm)
+        assert api.xcoosort_by_row(handle, m, n, nnz, d_r, d_c, d_p, buf) == api.STATUS_SUCCESS
+        torch.cuda.synchronize()
+        assert np.array_equal(d_p.cpu().numpy(), perm[want])
+        assert np.array_equal(d_r.cpu().numpy(), rows[want])
+        assert np.array_equal(d_c.cpu().numpy(), cols[want])
