@@ -281,7 +281,7 @@ __global__ __launch_bounds__(kRowStartsBlock) void partition_row_starts_kernel(c
 }
 
 // run_begins[d * tiles + t] = entries of digit d in the tiles before t; totals[d] = all of them.  A workgroup per digit.
-// first_runs (may be null), [d][tiles + 1]: for the entries q * kSecondTile of the digit the run they lie in.
+// first_runs (may be null), [d][first_stride]: for the entries q * kSecondTile of the digit the run they lie in.
 constexpr int kScanBlock = 256;
 constexpr int kScanItems = 8;
 // Tiles of step 2.  With 16 entries per thread there is room for two workgroups per compute unit only, and what a
@@ -291,7 +291,8 @@ constexpr uint32_t kSecondTile = kSecondThreads * kSecondItems;
 __global__ __launch_bounds__(kScanBlock) void run_begins_kernel(uint32_t tiles, const uint32_t* __restrict__ table,
                                                                 uint32_t* __restrict__ run_begins,
                                                                 uint32_t* __restrict__ totals,
-                                                                uint32_t* __restrict__ first_runs) {
+                                                                uint32_t* __restrict__ first_runs,
+                                                                uint32_t first_stride) {
     __shared__ uint32_t s_wave[kScanBlock / kWave];
     const uint32_t* in = table + static_cast<uint64_t>(blockIdx.x) * tiles;
     uint32_t* out = run_begins + static_cast<uint64_t>(blockIdx.x) * tiles;
@@ -317,7 +318,7 @@ __global__ __launch_bounds__(kScanBlock) void run_begins_kernel(uint32_t tiles, 
             if (first_runs != nullptr && n[k] != 0) {  // (a run is no longer than a tile)
                 const uint32_t q = (at + kSecondTile - 1) / kSecondTile;
                 for (uint32_t k2 = q; k2 * kSecondTile < at + n[k]; ++k2)
-                    first_runs[static_cast<uint64_t>(blockIdx.x) * (tiles + 1) + k2] = t;
+                    first_runs[static_cast<uint64_t>(blockIdx.x) * first_stride + k2] = t;
             }
             at += n[k];
         }
@@ -343,7 +344,8 @@ struct SortTables {
     uint32_t* begins2;
     uint32_t* bucket_first;  // entries before each bucket of step 1, 2^d1 + 1 of them
     uint32_t* tile_first;    // tiles before each bucket of step 1, 2^d1 + 1 of them
-    const uint32_t* first_runs;  // [bucket][tiles1 + 1]: the run of step 1 in which each of its tiles begins
+    const uint32_t* first_runs;  // [bucket][first_stride]: the run of step 1 in which each of its tiles begins
+    uint32_t first_stride;       // tiles of step 2 that one bucket can have
     uint2* tile_map;         // the order in which the tiles are taken: {bucket << 24 | tile of the bucket, its first run}
     // both: entries before each bucket of step 3, 2^(d1 + d2) + 1 of them
     uint32_t* sub_first;
@@ -460,7 +462,7 @@ __global__ __launch_bounds__(kMapBlock) void tile_map_kernel(SortTables t) {
         at += tiles < tile ? tiles : tile;
         if (b < lo && tiles > tile) ++at;
     }
-    t.tile_map[at] = make_uint2(lo << 24 | tile, t.first_runs[static_cast<uint64_t>(lo) * (t.tiles1 + 1) + tile]);
+    t.tile_map[at] = make_uint2(lo << 24 | tile, t.first_runs[static_cast<uint64_t>(lo) * t.first_stride + tile]);
 }
 
 // 118 M entries (19 bytes each): 1.33 GB read, 1.14 GB written in 500 us.
@@ -1084,6 +1086,10 @@ void sort_passes(const SortShape& s, SortTables* t) {
     if (t->passes == 0) t->passes = 1;  // everything in order already: one pass over no bits
 }
 
+// Tiles of step 2 that one bucket of step 1 can have: all entries may lie in one (tiles of step 1 hold more entries, so
+// their number is no bound).
+uint32_t second_tiles_most(uint32_t count) { return (count - 1) / kSecondTile + 1; }
+
 struct SortLayout {
     size_t keys1, aux1, vals1, keys2, aux2, vals2, table1, begins1, totals1, tile_rows, table2, begins2, bucket_first,
         tile_first, first_runs, tile_map, sub_first, oversize_count, oversize, oversize_begins, oversize_keys[2], oversize_aux[2],
@@ -1116,7 +1122,7 @@ SortLayout sort_layout(uint32_t count, const SortShape& s, size_t value_bytes) {
     l.begins2 = take(runs2 * sizeof(uint32_t));
     l.bucket_first = take((sizeof(uint32_t) << s.d1) + sizeof(uint32_t));
     l.tile_first = take((sizeof(uint32_t) << s.d1) + sizeof(uint32_t));
-    l.first_runs = take(s.d2 != 0 ? (runs1 + (size_t(1) << s.d1)) * sizeof(uint32_t) : 0);
+    l.first_runs = take(s.d2 != 0 ? (static_cast<size_t>(second_tiles_most(count)) << s.d1) * sizeof(uint32_t) : 0);
     l.tile_map = take(static_cast<size_t>(s.max_tiles2) * sizeof(uint2));
     l.sub_first = take((subs + 1) * sizeof(uint32_t));
     l.oversize_count = take(sizeof(unsigned long long));
@@ -1154,6 +1160,7 @@ void launch_sort(hipStream_t stream, EntrySource in, const SortShape& s, const S
     t.bucket_first = words(l.bucket_first);
     t.tile_first = words(l.tile_first);
     t.first_runs = words(l.first_runs);
+    t.first_stride = second_tiles_most(in.count);
     t.tile_map = reinterpret_cast<uint2*>(w + l.tile_map);
     t.sub_first = words(l.sub_first);
     t.oversize_count = reinterpret_cast<unsigned long long*>(w + l.oversize_count);
@@ -1177,7 +1184,7 @@ void launch_sort(hipStream_t stream, EntrySource in, const SortShape& s, const S
                                                : launch_partition<VB, KIND, kMaxOneLevelBits, uint16_t>);
     partition(stream, in, shift, s.d1, s.tile_size, w + l.keys1, words(l.aux1), w + l.vals1, words(l.table1));
     hipLaunchKernelGGL(run_begins_kernel, dim3(1u << s.d1), dim3(kScanBlock), 0, stream, s.tiles1, t.table1,
-                       words(l.begins1), words(l.totals1), s.d2 != 0 ? words(l.first_runs) : nullptr);
+                       words(l.begins1), words(l.totals1), s.d2 != 0 ? words(l.first_runs) : nullptr, t.first_stride);
     hipLaunchKernelGGL(sort_plan_kernel, dim3(1), dim3(kPlanBlock), 0, stream, t);
     const void* keys = w + l.keys1;
     const uint32_t* aux = words(l.aux1);

@@ -118,7 +118,7 @@ def test_coosort_bit_exact(torch_gpu, handle, oracle, by, with_perm, kind, m, n,
         assert np.array_equal(d_p.cpu().numpy(), perm[want])
 
 
-@pytest.mark.parametrize("share", [0.3])
+@pytest.mark.parametrize("share", [0.3, 0.9])  # 0.9: one bucket with more tiles of the second step than the first has
 def test_a_row_with_most_of_ten_million_entries(torch_gpu, handle, share):
     """Many more pieces of one bucket than workgroups that work on it, in every pass: what one workgroup writes is read
     by others of the same launch, on other XCDs."""
