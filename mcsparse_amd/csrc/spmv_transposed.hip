@@ -4,6 +4,7 @@
 //
 // The reference builds the transpose in the scratch buffer on every call and runs its row kernel on it
 // (src/kernels/level2/spmv/mcsp_spmv_gpu.cpp:797-845).
+#include "bucket_deal.h"
 #include "partition_device.h"
 
 namespace mcsp {
@@ -232,14 +233,14 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_sums_kernel(idx_t n, uint
         const uint32_t t = g * kGroupTiles + lane;
         return lane < kGroupTiles && t < tiles ? row[t] : 0u;
     };
-    // light groups are dealt to the parts, heavy ones are shared by all wavefronts of all parts
+    // light groups are dealt to the parts (bucket_deal.h), heavy ones are shared by all wavefronts of all parts
     uint32_t word = wave < groups ? words_of(wave) : 0u;
     for (uint32_t g = wave; g < groups; g += kWaves) {
         const uint32_t next = g + kWaves < groups ? words_of(g + kWaves) : 0u;  // on its way while this group is added
         const uint32_t total = __builtin_amdgcn_readlane(wave_inclusive_sum(run_length(word) / kPiece), kWave - 1);
         if (total > kHeavyGroup) {
             if (lane == 0) atomicOr(&s_heavy[g / 32], 1u << (g % 32));
-        } else if (total != 0 && g % mine.parts == mine.part) {
+        } else if (total != 0 && part_of_group(g, kWaves, mine.parts) == mine.part) {
             add_group(word, g, tile_places, 0, 1, s_runs[wave], keys, products, width - 1, s_acc);
         }
         word = next;
