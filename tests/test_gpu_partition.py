@@ -138,3 +138,72 @@ def test_a_row_with_most_of_ten_million_entries(torch_gpu, handle, share):
         assert np.array_equal(d_p.cpu().numpy(), perm[want])
         assert np.array_equal(d_r.cpu().numpy(), rows[want])
         assert np.array_equal(d_c.cpu().numpy(), cols[want])
+
+
+def best_us(torch, call, repeats=5):
+    """Shortest time of a few calls after one that is not looked at."""
+    call()
+    torch.cuda.synchronize()
+    best = float("inf")
+    for _ in range(repeats):
+        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        e0.record()
+        call()
+        e1.record()
+        e1.synchronize()
+        best = min(best, e0.elapsed_time(e1) * 1e3)
+    return best
+
+
+def csr2csc_us(torch, handle, m, per_row, n, col):
+    """Time of csr2csc on m rows of per_row nonzeros with these columns (device tensor), which is checked first."""
+    nnz = m * per_row
+    ptr = torch.arange(m + 1, dtype=torch.int32, device="cuda") * per_row
+    val = torch.rand(nnz, dtype=torch.float32, device="cuda")
+    o_ptr = torch.zeros(n + 1, dtype=torch.int32, device="cuda")
+    o_row, o_val = torch.zeros(nnz, dtype=torch.int32, device="cuda"), torch.zeros_like(val)
+    args = (handle, m, n, nnz, val, ptr, col, o_val, o_ptr, o_row, api.R_32F, api.ACTION_NUMERIC, api.BASE_ZERO)
+    st, size = api.csr2csc_buffer_size(*args)
+    assert st == api.STATUS_SUCCESS
+    buf = torch.empty(size, dtype=torch.uint8, device="cuda")
+    assert api.csr2csc(*args, buf) == api.STATUS_SUCCESS
+    order = torch.sort(col, stable=True).indices
+    assert torch.equal(o_val, val[order]) and torch.equal(o_row, (order // per_row).to(torch.int32))
+    del order
+    return best_us(torch, lambda: api.csr2csc(*args, buf))
+
+
+def coosort_us(torch, handle, m, n, rows, cols):
+    nnz = rows.numel()
+    d_r, d_c, d_p = (torch.empty_like(rows) for _ in range(3))
+    st, size = api.sort_buffer_size(handle, "coo", m, n, nnz, d_r, d_c)
+    assert st == api.STATUS_SUCCESS
+    buf = torch.empty(size, dtype=torch.uint8, device="cuda")
+
+    def call():
+        d_r.copy_(rows)
+        d_c.copy_(cols)
+        assert api.create_identity_permutation(handle, nnz, d_p) == api.STATUS_SUCCESS
+        assert api.xcoosort_by_row(handle, m, n, nnz, d_r, d_c, d_p, buf) == api.STATUS_SUCCESS
+
+    call()
+    order = torch.sort(rows.long() * n + cols, stable=True).indices
+    assert torch.equal(d_p, order.to(torch.int32)) and torch.equal(d_r, rows[order]) and torch.equal(d_c, cols[order])
+    del order
+    return best_us(torch, call)
+
+
+@pytest.mark.parametrize("few", [16, 1000])
+def test_few_keys_take_no_longer_than_many(torch_gpu, handle, few):
+    """16.8 M entries with 16 or 1000 keys against as many with a million: keys that fill more than a bucket each go to
+    the LSD passes (two to six times the time of many keys when they were sorted in buckets)."""
+    torch = torch_gpu
+    m, per_row, many = 1 << 20, 16, 1 << 20
+
+    def drawn(k):
+        gen = torch.Generator(device="cuda").manual_seed(k)
+        return torch.randint(0, k, (m * per_row,), generator=gen, dtype=torch.int32, device="cuda")
+
+    assert csr2csc_us(torch, handle, m, per_row, few, drawn(few)) < 1.4 * csr2csc_us(torch, handle, m, per_row, many, drawn(many))
+    other = drawn(many - 1)
+    assert coosort_us(torch, handle, few, many, drawn(few), other) < 2 * coosort_us(torch, handle, many, many, drawn(many), other)
