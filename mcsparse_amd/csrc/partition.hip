@@ -17,7 +17,8 @@
 // A key loses the bits that its place already tells: at most 16 of them travel to step 2, 8 or 16 to step 3.
 // A sort by two keys (the index sorts) partitions by the major key alone: step 3 orders a bucket by the minor key first,
 // then by what is left of the major one, in passes of up to eight bits that stay in LDS.
-// Buckets that do not fit LDS (popular keys) are sorted in chunks by oversize_kernel, which finds nothing to do elsewhere.
+// Buckets that do not fit LDS (popular keys) are sorted in chunks by oversize_kernel, which finds nothing to do elsewhere;
+// inputs that would make such buckets only (few keys) are left to the LSD passes.
 #include "partition_device.h"
 
 #include <algorithm>
@@ -330,6 +331,28 @@ __global__ __launch_bounds__(kScanBlock) void run_begins_kernel(uint32_t tiles, 
 
 
 
+// ---- between workgroups of one launch --------------------------------------------------------------------------
+// An XCD's L2 does not see what another XCD writes: what workgroups of a launch hand to each other goes past the caches on
+// both sides.  (An L2 written back by each of its workgroups at the end of a phase: 70 us a phase.)
+template <typename W>
+__device__ __forceinline__ W load_shared(const W* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename W>
+__device__ __forceinline__ void store_shared(W* p, W v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// One more of `all` has come: was it the last?  For the whole workgroup; whoever comes last may load_shared what the others
+// have written with store_shared.
+__device__ __forceinline__ bool last_to_arrive(uint32_t* counter, uint32_t all, uint32_t* s_last) {
+    wait_for_stores();
+    __syncthreads();
+    if (threadIdx.x == 0)
+        *s_last = (__hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1) % all == 0;
+    __syncthreads();
+    return *s_last != 0;
+}
+
 // ---- step 2 ----------------------------------------------------------------------------------------------------
 // What the kernels after step 1 read of it and of each other.  One level: the buckets of step 1 are sorted as they are.
 // Two levels: tile t of bucket b (its entries [t * kSecondTile, ...)) is tile number tile_first[b] + t.
@@ -349,13 +372,19 @@ struct SortTables {
     uint2* tile_map;         // the order in which the tiles are taken: {bucket << 24 | tile of the bucket, its first run}
     // both: entries before each bucket of step 3, 2^(d1 + d2) + 1 of them
     uint32_t* sub_first;
-    // buckets of step 3 that do not fit LDS
-    unsigned long long* oversize_count;  // buckets | chunks << 32
-    struct OversizeBucket* oversize;
-    uint32_t* oversize_begins;           // [chunk][digit]
-    uint32_t* oversize_aux[2];           // where the passes over such a bucket leave its entries in between
+    uint32_t* sub_arrived;  // workgroups that are through with a bucket of step 1
+    // buckets of step 3 that do not fit LDS, in the order in which they were listed
+    struct OversizeState* oversize;
+    uint32_t* oversize_bucket;
+    uint32_t* oversize_first;     // chunks of the buckets before
+    uint32_t* oversize_counted;   // groups of chunks that have been counted, over all passes
+    uint32_t* oversize_arrived;   // [group]: chunks of it that have been counted, over all passes
+    uint32_t* oversize_counts;    // [chunk][digit]
+    uint32_t* oversize_begins;    // [group][digit]
+    uint32_t* oversize_aux[2];    // where the passes over such a bucket leave its entries in between
     void* oversize_vals[2];
     uint16_t* oversize_keys[2];
+    uint32_t oversize_passes, oversize_width;  // passes of so many bits over the minor and the major key together
     uint32_t d1, d2, d3, count;
     // step 3: `minor_passes` passes of minor_width bits (the last one: what is left) over the minor_bits of aux, then
     // passes of key_width bits over the d3 bits of the keys
@@ -376,28 +405,31 @@ __device__ __forceinline__ SortPass sort_pass(const SortTables& t, uint32_t p) {
 constexpr int kBucketThreads = 512, kBucketItems = 12;
 constexpr uint32_t kBucketRoom = kBucketThreads * kBucketItems;  // entries of the largest bucket that is sorted in LDS
 constexpr uint32_t kPassBits = 8;  // the most a pass of step 3 takes
-constexpr uint32_t kMaxPasses = 6;   // 24 bits of the minor key and 16 of the major one at most
-constexpr uint32_t kOversizeChunk = kBucketRoom;
 
-// A bucket that does not fit LDS goes through two phases per pass: the digits of its chunks are counted, then the chunks
-// are written where they belong.
-struct OversizeBucket {
-    uint32_t bucket, chunks_before, chunks;
-    // on lines of their own: idle workgroups keep reading `phase`
-    alignas(128) uint32_t phase;                  // 2 * passes: sorted
-    alignas(128) uint32_t taken[2 * kMaxPasses];  // chunks of a phase that somebody works on or has done
-    alignas(128) uint32_t done[2 * kMaxPasses];
+// A bucket that does not fit LDS is sorted in chunks, by passes of up to kPassBits over the bits that are left of its
+// keys.  A pass has two phases: the digits of the chunks are counted, then the chunks are written where they belong.
+constexpr uint32_t kOversizeChunk = kBucketRoom;
+constexpr uint32_t kOversizeGroup = 16;  // chunks whose counts are added up together
+constexpr uint32_t kMaxOversizePhases = 10;  // of 24 bits of the minor key and 16 of the major one
+struct OversizeState {
+    unsigned long long listed;  // buckets | chunks << 32
+    // chunks of a phase that somebody works on or has done, and that are done; on lines of their own, since idle
+    // workgroups keep reading `done`
+    alignas(128) uint32_t taken[kMaxOversizePhases];
+    alignas(128) uint32_t done[kMaxOversizePhases];
 };
+// The groups of a listed bucket are numbered from here on (a bucket has at most chunks / kOversizeGroup + 1 of them).
+__device__ __forceinline__ uint32_t oversize_slot(uint32_t first, uint32_t listed_at) { return first / kOversizeGroup + listed_at; }
 __device__ __forceinline__ void note_oversize(const SortTables& t, uint32_t bucket, uint32_t entries) {
     if (entries <= kBucketRoom) return;
     const uint32_t chunks = (entries + kOversizeChunk - 1) / kOversizeChunk;
-    const unsigned long long at = atomicAdd(t.oversize_count, static_cast<unsigned long long>(chunks) << 32 | 1u);
-    OversizeBucket& o = t.oversize[static_cast<uint32_t>(at)];
-    o.bucket = bucket;
-    o.chunks_before = static_cast<uint32_t>(at >> 32);
-    o.chunks = chunks;
-    o.phase = 0;
-    for (uint32_t p = 0; p < 2 * kMaxPasses; ++p) o.taken[p] = o.done[p] = 0;
+    const unsigned long long at = atomicAdd(&t.oversize->listed, static_cast<unsigned long long>(chunks) << 32 | 1u);
+    const uint32_t k = static_cast<uint32_t>(at), first = static_cast<uint32_t>(at >> 32);
+    t.oversize_bucket[k] = bucket;
+    t.oversize_first[k] = first;
+    t.oversize_counted[k] = 0;
+    const uint32_t groups = (chunks + kOversizeGroup - 1) / kOversizeGroup;
+    for (uint32_t g = 0; g < groups; ++g) t.oversize_arrived[oversize_slot(first, k) + g] = 0;
 }
 
 // Exclusive sums over the buckets of step 1 (at most 2^11), in one workgroup: of entries, and (two levels) of tiles.
@@ -406,7 +438,8 @@ constexpr int kPlanBlock = 1024;
 __global__ __launch_bounds__(kPlanBlock) void sort_plan_kernel(SortTables t) {
     __shared__ uint32_t s_wave[kPlanBlock / kWave];
     if (threadIdx.x == 0) {
-        *t.oversize_count = 0;
+        t.oversize->listed = 0;
+        for (uint32_t p = 0; p < kMaxOversizePhases; ++p) t.oversize->taken[p] = t.oversize->done[p] = 0;
         __threadfence();  // before the adds of this workgroup's other threads
     }
     const uint32_t buckets = 1u << t.d1;
@@ -424,7 +457,10 @@ __global__ __launch_bounds__(kPlanBlock) void sort_plan_kernel(SortTables t) {
         if (t.d2 != 0) {
             const uint32_t tiles = (n + kSecondTile - 1) / kSecondTile;
             const uint32_t tile_at = block_exclusive_sum<kPlanBlock>(tiles, s_wave, &all);
-            if (b < buckets) t.tile_first[b] = tiles_before + tile_at;
+            if (b < buckets) {
+                t.tile_first[b] = tiles_before + tile_at;
+                t.sub_arrived[b] = 0;
+            }
             tiles_before += all;
             __syncthreads();
         } else if (b < buckets) {
@@ -524,35 +560,47 @@ __global__ __launch_bounds__(kSecondThreads) void repartition_kernel(SortTables 
         store_words<kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, static_cast<word_t*>(vals_out) + out, val);
 }
 
-// begins2 and sub_first from table2; a workgroup per bucket of step 1, a wavefront per digit at a time.
-constexpr int kSubBlock = 1024;
+// begins2 and sub_first from table2; kSubParts workgroups per bucket of step 1, a wavefront per digit at a time, and
+// whoever comes last says where the bucket's digits begin.  One workgroup per bucket and one round of 64 tiles in flight
+// took 514 us where a bucket holds two thirds of 67 M entries (some 7000 tiles), now 96.
+constexpr int kSubBlock = 256;
+constexpr uint32_t kSubParts = 8;
 __global__ __launch_bounds__(kSubBlock) void sub_begins_kernel(SortTables t) {
-    __shared__ uint32_t s_total[256];
     __shared__ uint32_t s_wave[kSubBlock / kWave];
-    const uint32_t bucket = blockIdx.x, tid = threadIdx.x, lane = tid % kWave;
+    __shared__ uint32_t s_last;
+    constexpr uint32_t kAhead = 8;
+    const uint32_t bucket = blockIdx.x / kSubParts, part = blockIdx.x % kSubParts, tid = threadIdx.x, lane = tid % kWave;
     const uint32_t digits = 1u << t.d2;  // at most 256
     const uint32_t first_tile = t.tile_first[bucket], tiles = t.tile_first[bucket + 1] - first_tile;
     const uint64_t row0 = static_cast<uint64_t>(first_tile) << t.d2;
-    for (uint32_t d = tid / kWave; d < digits; d += kSubBlock / kWave) {
+    uint32_t* first = t.sub_first + (bucket << t.d2);
+    for (uint32_t d = part * (kSubBlock / kWave) + tid / kWave; d < digits; d += kSubParts * (kSubBlock / kWave)) {
         const uint64_t row = row0 + static_cast<uint64_t>(d) * tiles;
         uint32_t carried = 0;
-        for (uint32_t t0 = 0; t0 < tiles; t0 += kWave) {
-            const uint32_t n = t0 + lane < tiles ? run_length(t.table2[row + t0 + lane]) : 0;
-            const uint32_t upto = wave_inclusive_sum(n);
-            if (t0 + lane < tiles) t.begins2[row + t0 + lane] = carried + upto - n;
-            carried += __builtin_amdgcn_readlane(upto, kWave - 1);
+        for (uint32_t t0 = 0; t0 < tiles; t0 += kWave * kAhead) {
+            uint32_t n[kAhead];
+#pragma unroll
+            for (uint32_t k = 0; k < kAhead; ++k) n[k] = t.table2[row + min(t0 + k * kWave + lane, tiles - 1)];
+#pragma unroll
+            for (uint32_t k = 0; k < kAhead; ++k) {
+                const uint32_t at = t0 + k * kWave + lane;
+                n[k] = at < tiles ? run_length(n[k]) : 0;
+                const uint32_t upto = wave_inclusive_sum(n[k]);
+                if (at < tiles) t.begins2[row + at] = carried + upto - n[k];
+                carried += __builtin_amdgcn_readlane(upto, kWave - 1);
+            }
         }
-        if (lane == 0) s_total[d] = carried;
+        if (lane == 0) store_shared(first + d, carried);
     }
-    __syncthreads();
-    const uint32_t n = tid < digits ? s_total[tid] : 0;
+    if (!last_to_arrive(t.sub_arrived + bucket, kSubParts, &s_last)) return;  // whole workgroup
+    static_assert(kSubBlock == 256, "a thread per digit");
+    const uint32_t n = tid < digits ? load_shared(first + tid) : 0;
     const uint32_t at = t.bucket_first[bucket] + block_exclusive_sum<kSubBlock>(n, s_wave);
-    const uint32_t sub = (bucket << t.d2) + tid;
     if (tid < digits) {
-        t.sub_first[sub] = at;
-        note_oversize(t, sub, n);
+        first[tid] = at;
+        note_oversize(t, (bucket << t.d2) + tid, n);
     }
-    if (bucket == gridDim.x - 1 && tid == 0) t.sub_first[gridDim.x << t.d2] = t.count;
+    if (bucket == (1u << t.d1) - 1 && tid == 0) t.sub_first[1u << (t.d1 + t.d2)] = t.count;
 }
 
 // ---- step 3 ----------------------------------------------------------------------------------------------------
@@ -770,70 +818,65 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 || MANY ? 6 : 8) void bucke
 }
 
 // ---- buckets that do not fit LDS -------------------------------------------------------------------------------
-// One launch works on all of them.  A workgroup takes the next chunk of any listed bucket's current phase; whoever
-// finishes a phase's last chunk turns the counts into places (counting phases) and opens the next phase.  A workgroup that
-// finds no chunk to take looks again until every bucket is sorted: it only ever waits for chunks that running workgroups
-// have taken, so the wait ends whether or not the other workgroups of the grid are resident.
+// One launch works on all of them, phase by phase: a workgroup takes the next chunk of the phase off a counter until none
+// is left, adds what it has done to the phase's other counter, and waits there for the rest.  It only ever waits for chunks
+// that running workgroups have taken, so every wait ends whether or not the other workgroups of the grid are resident.
+// Entries and counts that are read in a later phase go past the caches.  The counts of a chunk become places in two steps:
+// whoever counts the last chunk of a group adds the group up, whoever adds up the last group of a bucket says where every
+// group's entries begin, and the second phase adds the chunks of the group in front of its own.
+//
+// Before, a workgroup looked for work among all buckets with two device-wide fences a chunk, one workgroup placed all
+// chunks of a bucket, the counting phase read whole entries, and entries were written from where they lay in registers:
+// csr2csc of 67 M nonzeros with columns by Zipf's law (53 M of them in such buckets) 3690 us, now 1475 (LSD passes: 1484);
+// an index sort of 10 M triples with rows by that law 1870 us, now 960.
+// Index sorts by a skewed major key stay slower than the LSD passes: 503 us for those, 936 against 1550 for 21.8 M triples
+// in a million power-law rows of up to 50,000 (38 % of them in such buckets).  A pass over such a bucket costs two phases
+// of 45 us at least, and there are four or five of them.  How the keys are spread is not known on the host, where the
+// choice is made, and evenly spread ones gain as much (10 M: 481 and 330 us); so does csr2csc under any spread.
 constexpr uint32_t kOversizeGrid = 512;
 
-struct OversizeWork {
-    uint32_t listed_at, phase, chunk, found;
+struct OversizeChunk {
+    uint32_t listed_at, bucket, first, entries;  // first: place of the bucket's first entry in the output
+    uint32_t chunk, chunks, slot;                // slot: the bucket's first group
 };
-// For one whole wavefront, which looks at 64 listed buckets at a time, from `start` on; every lane returns the same.
-__device__ __forceinline__ OversizeWork find_oversize_work(const SortTables& t, uint32_t listed, uint32_t start) {
-    const uint32_t lane = threadIdx.x % kWave;
-    OversizeWork w = {0, 0, 0, 0};
-    for (uint32_t idle = 0;; ++idle) {
-        bool all_sorted = true;
-        for (uint32_t i0 = 0; i0 < listed; i0 += kWave) {
-            const uint32_t i = i0 + lane;
-            const uint32_t k = (start + (i < listed ? i : 0)) % listed;
-            OversizeBucket& o = t.oversize[k];
-            const uint32_t phase = __hip_atomic_load(&o.phase, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const bool open = i < listed && phase < 2 * t.passes;
-            const bool left = open && __hip_atomic_load(&o.taken[phase], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < o.chunks;
-            if (__any(open)) all_sorted = false;
-            uint64_t candidates = __ballot(left);
-            while (candidates != 0) {
-                const int src = __ffsll(static_cast<long long>(candidates)) - 1;
-                candidates &= candidates - 1;
-                uint32_t c = 0;
-                if (lane == static_cast<uint32_t>(src))
-                    c = __hip_atomic_fetch_add(&o.taken[phase], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                w.listed_at = __shfl(k, src, kWave);
-                w.phase = __shfl(phase, src, kWave);
-                w.chunk = __shfl(c, src, kWave);
-                if (w.chunk < __shfl(o.chunks, src, kWave)) {
-                    w.found = 1;
-                    return w;
-                }
-            }
-        }
-        if (all_sorted) return w;
-        // (hundreds of workgroups may be waiting for one bucket's phase: longer and longer, up to some 15 us)
-        for (uint32_t n = 0; n < (1u << min(idle, 4u)); ++n) __builtin_amdgcn_s_sleep(32);
-    }
+// For whole wavefronts; every lane returns the same.
+__device__ __forceinline__ OversizeChunk oversize_chunk(const SortTables& t, uint32_t listed, uint32_t number) {
+    OversizeChunk c;
+    c.listed_at = wave_count_up_to(t.oversize_first, listed, 0, number) - 1;
+    const uint32_t before = t.oversize_first[c.listed_at];
+    c.bucket = t.oversize_bucket[c.listed_at];
+    c.first = t.sub_first[c.bucket];
+    c.entries = t.sub_first[c.bucket + 1] - c.first;
+    c.chunk = number - before;
+    c.chunks = (c.entries + kOversizeChunk - 1) / kOversizeChunk;
+    c.slot = oversize_slot(before, c.listed_at);
+    return c;
 }
 
-// The counts of a bucket's chunks, digit by digit, become places in its stretch of the output.
-__device__ __forceinline__ void place_chunks(const SortTables& t, const OversizeBucket& o, const SortOutput& out, bool write_ptr,
+// The next chunk of a phase that nobody has taken.
+__device__ __forceinline__ uint32_t take_chunk(const SortTables& t, uint32_t phase) {
+    return __hip_atomic_fetch_add(&t.oversize->taken[phase], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The counts of a bucket's groups, digit by digit, become places in the output.
+__device__ __forceinline__ void place_groups(const SortTables& t, const OversizeChunk& c, const SortOutput& out, bool write_ptr,
                                              uint32_t bits, uint32_t (&s_sum)[kBucketThreads], uint32_t* s_wave) {
     constexpr uint32_t kDigits = 1 << kPassBits, kShares = kBucketThreads / kDigits;  // threads per digit
     const uint32_t d = threadIdx.x % kDigits, share = threadIdx.x / kDigits;
-    const uint32_t mine = (o.chunks + kShares - 1) / kShares;
-    const uint32_t from = min(share * mine, o.chunks), to = min(from + mine, o.chunks);
-    uint32_t* column = t.oversize_begins + (static_cast<uint64_t>(o.chunks_before) << kPassBits) + d;
-    // (a batch of loads on their way at a time: a bucket of 3 M entries has 490 chunks)
-    constexpr uint32_t kBatch = 32;
-    auto counts_of = [&](uint32_t c0, uint32_t (&n)[kBatch]) {
+    const uint32_t groups = (c.chunks + kOversizeGroup - 1) / kOversizeGroup;
+    const uint32_t mine = (groups + kShares - 1) / kShares;
+    const uint32_t from = min(share * mine, groups), to = min(from + mine, groups);
+    uint32_t* column = t.oversize_begins + (static_cast<uint64_t>(c.slot) << kPassBits) + d;
+    constexpr uint32_t kBatch = 16;  // loads on their way at a time
+    auto counts_of = [&](uint32_t g0, uint32_t (&n)[kBatch]) {
 #pragma unroll
-        for (uint32_t i = 0; i < kBatch; ++i) n[i] = column[static_cast<uint64_t>(min(c0 + i, to - 1)) << kPassBits];
+        for (uint32_t i = 0; i < kBatch; ++i) n[i] = load_shared(column + (static_cast<uint64_t>(min(g0 + i, to - 1)) << kPassBits));
     };
     uint32_t sum = 0, n[kBatch];
-    for (uint32_t c = from; c < to; c += kBatch) {
-        counts_of(c, n);
+    for (uint32_t g = from; g < to; g += kBatch) {
+        counts_of(g, n);
 #pragma unroll
-        for (uint32_t i = 0; i < kBatch; ++i) sum += c + i < to ? n[i] : 0u;
+        for (uint32_t i = 0; i < kBatch; ++i) sum += g + i < to ? n[i] : 0u;
     }
     s_sum[threadIdx.x] = sum;
     __syncthreads();
@@ -843,130 +886,217 @@ __device__ __forceinline__ void place_chunks(const SortTables& t, const Oversize
         if (k == share) before = total;
         total += s_sum[k * kDigits + d];
     }
-    const uint32_t first = t.sub_first[o.bucket] + block_exclusive_sum<kBucketThreads>(share == 0 ? total : 0u, s_wave);
+    const uint32_t first = c.first + block_exclusive_sum<kBucketThreads>(share == 0 ? total : 0u, s_wave);
     if (share == 0) {
         s_sum[d] = first;  // (every thread has read the sums: the barrier in the scan)
-        if (write_ptr && d < (1u << bits)) write_key_ptr(out, o.bucket, t.d3, d, first, t.count);
+        if (write_ptr && d < (1u << bits)) write_key_ptr(out, c.bucket, t.d3, d, first, t.count);
     }
     __syncthreads();
     uint32_t at = s_sum[d] + before;
-    for (uint32_t c = from; c < to; c += kBatch) {
-        counts_of(c, n);
+    for (uint32_t g = from; g < to; g += kBatch) {
+        counts_of(g, n);
 #pragma unroll
         for (uint32_t i = 0; i < kBatch; ++i) {
-            if (c + i < to) column[static_cast<uint64_t>(c + i) << kPassBits] = at;
+            if (g + i < to) store_shared(column + (static_cast<uint64_t>(g + i) << kPassBits), at);
             at += n[i];
         }
     }
 }
 
-template <int VB, typename Key>
-__global__ __launch_bounds__(kBucketThreads) void oversize_kernel(SortTables t, const Key* __restrict__ keys_in,
+template <int VB, typename Key, bool MANY>
+__global__ __launch_bounds__(kBucketThreads, 4) void oversize_kernel(SortTables t, const Key* __restrict__ keys_in,
                                                                   const uint32_t* __restrict__ aux_in,
                                                                   const void* __restrict__ vals_in, SortOutput out) {
     typedef typename WordOf<VB>::type word_t;
-    const unsigned long long counted = *t.oversize_count;
-    const uint32_t listed = static_cast<uint32_t>(counted);
-    if (blockIdx.x >= static_cast<uint32_t>(counted >> 32)) return;  // whole workgroup: more workgroups than chunks
+    constexpr uint32_t kDigits = 1 << kPassBits;
+    static_assert(kDigits <= kBucketThreads, "a thread per digit");
+    const unsigned long long counted = t.oversize->listed;
+    const uint32_t listed = static_cast<uint32_t>(counted), all_chunks = static_cast<uint32_t>(counted >> 32);
+    if (blockIdx.x >= all_chunks) return;  // whole workgroup: more workgroups than chunks
     __shared__ BucketLds s;
-    __shared__ uint32_t s_count[1 << kPassBits];
+    __shared__ uint32_t s_count[kDigits];
     __shared__ uint32_t s_sum[kBucketThreads];
-    __shared__ OversizeWork s_work;
-    __shared__ uint32_t s_last;
+    __shared__ uint32_t s_ticket, s_last;
     const uint32_t tid = threadIdx.x, wave = tid / kWave;
-    uint32_t start = blockIdx.x % listed;
-    while (true) {
-        if (wave == 0) {
-            const OversizeWork found = find_oversize_work(t, listed, start);
-            if (tid == 0) s_work = found;
-            // what the phase before has written, for the whole workgroup (it goes on behind the barrier); device-wide fences
-            // flush an XCD's L2, so one wavefront makes them for all
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    const uint32_t phases = 2 * t.oversize_passes;
+    for (uint32_t phase = 0; phase < phases; ++phase) {
+        const uint32_t p = phase / 2;
+        const uint32_t shift = p * t.oversize_width, bits = min(t.oversize_width, t.minor_bits + t.d3 - shift);
+        const uint32_t mask = (1u << bits) - 1u;
+        // which of the two keys the pass looks at
+        const bool by_aux = MANY && shift < t.minor_bits, by_key = !MANY || shift + bits > t.minor_bits;
+        auto digit_of = [&](uint32_t of_key, uint32_t of_aux) {
+            if (!MANY) return of_key >> shift & mask;
+            return static_cast<uint32_t>((static_cast<uint64_t>(of_key) << t.minor_bits | of_aux) >> shift) & mask;
+        };
+        // the first pass reads the runs, the others what the one before has left in the bucket's stretch
+        const uint16_t* between_keys = t.oversize_keys[(p + 1) % 2];
+        const uint32_t* between_aux = t.oversize_aux[(p + 1) % 2];
+        const word_t* between_vals = static_cast<const word_t*>(t.oversize_vals[(p + 1) % 2]);
+        if (tid == 0) {
+            for (uint32_t idle = 0; phase != 0 && load_shared(&t.oversize->done[phase - 1]) < all_chunks; ++idle) {
+                // (hundreds of workgroups may be waiting: longer and longer, up to some 4 us)
+                for (uint32_t n = 0; n < (1u << min(idle, 2u)); ++n) __builtin_amdgcn_s_sleep(32);
+            }
+            s_ticket = take_chunk(t, phase);
         }
         __syncthreads();
-        const OversizeWork work = s_work;
-        if (work.found == 0) return;  // whole workgroup
-        start = work.listed_at;       // its next chunk or phase is what this workgroup looks for first
-        OversizeBucket& o = t.oversize[work.listed_at];
-        const uint32_t p = work.phase / 2;
-        const bool counting = work.phase % 2 == 0;
-        const SortPass pass = sort_pass(t, p);
-        const uint32_t mask = (1u << pass.bits) - 1u;
-        const uint32_t first = t.sub_first[o.bucket], all = t.sub_first[o.bucket + 1] - first;
-        const uint32_t q0 = work.chunk * kOversizeChunk, count = min(all - q0, kOversizeChunk);
-        uint32_t* begins = t.oversize_begins + (static_cast<uint64_t>(o.chunks_before + work.chunk) << kPassBits);
-        s.clear_counts();
-        for (uint32_t d = tid; d < (1u << kPassBits); d += kBucketThreads) s_count[d] = 0;
-        // the first pass reads the runs, the others what the one before has left in the bucket's stretch
-        const BucketRuns runs = runs_of_bucket(t, o.bucket);
-        if (p == 0)
-            map_runs<kBucketThreads, kBucketRoom>(runs.begins, runs.table, runs.tiles, all, q0, count,
-                                                  find_first_run(runs.begins, runs.tiles, q0), runs.places, runs.source, s.map,
-                                                  s.buf);
-        else
-            __syncthreads();
-        uint32_t key[kBucketItems], aux[kBucketItems];
-        word_t val[VB ? kBucketItems : 1];
-        const uint32_t last_word = (count - 1) / kWave;
-#pragma unroll
-        for (int i = 0; i < kBucketItems; ++i) {
+        uint32_t finished = 0, number = s_ticket;
+        while (number < all_chunks) {
+            ++finished;
+            // The next ticket: on its way while this chunk is worked on, unless that would take the last chunks away from
+            // workgroups that have none yet.
+            const bool ahead = all_chunks - number > gridDim.x;
+            uint32_t next = 0;
+            if (tid == 0 && ahead) next = take_chunk(t, phase);
+            const OversizeChunk c = oversize_chunk(t, listed, number);
+            const uint32_t q0 = c.chunk * kOversizeChunk, count = min(c.entries - q0, kOversizeChunk);
+            const uint32_t group = c.chunk / kOversizeGroup, in_group = c.chunk % kOversizeGroup;
+            uint32_t* counts = t.oversize_counts + (static_cast<uint64_t>(number) << kPassBits);
+            uint32_t* begins = t.oversize_begins + (static_cast<uint64_t>(c.slot + group) << kPassBits);
             if (p == 0) {
-                const uint32_t from = mapped_place(s.map, s.buf, min(wave * kBucketItems + i, last_word), count);
-                key[i] = load_at<Key>(keys_in, from);
-                aux[i] = load_at<uint32_t>(aux_in, from);
-                if constexpr (VB != 0) val[i] = load_at<word_t>(vals_in, from);
+                const BucketRuns runs = runs_of_bucket(t, c.bucket);
+                map_runs<kBucketThreads, kBucketRoom>(runs.begins, runs.table, runs.tiles, c.entries, q0, count,
+                                                      find_first_run(runs.begins, runs.tiles, q0), runs.places, runs.source,
+                                                      s.map, s.buf);
+            }
+            const uint32_t last_word = (count - 1) / kWave;
+            auto place_of = [&](int i) {
+                return p == 0 ? mapped_place(s.map, s.buf, min(wave * kBucketItems + i, last_word), count)
+                              : c.first + q0 + min(slab_place(kBucketItems, i), count - 1);
+            };
+            if (phase % 2 == 0) {
+                if (tid < kDigits) s_count[tid] = 0;
+                uint32_t key[kBucketItems], aux[MANY ? kBucketItems : 1];
+#pragma unroll
+                for (int i = 0; i < kBucketItems; ++i) {
+                    const uint32_t from = place_of(i);
+                    key[i] = 0;
+                    if (by_key) key[i] = p == 0 ? load_at<Key>(keys_in, from) : load_shared(between_keys + from);
+                    if constexpr (MANY) {
+                        aux[i] = 0;
+                        if (by_aux) aux[i] = p == 0 ? load_at<uint32_t>(aux_in, from) : load_shared(between_aux + from);
+                    }
+                }
+                __syncthreads();
+#pragma unroll
+                for (int i = 0; i < kBucketItems; ++i) {
+                    if (in_slab(kBucketItems, i, count)) atomicAdd(&s_count[digit_of(key[i], MANY ? aux[MANY ? i : 0] : 0u)], 1u);
+                }
+                __syncthreads();
+                if (tid < kDigits) store_shared(counts + tid, s_count[tid]);
+                const uint32_t chunks_here = min(c.chunks - group * kOversizeGroup, kOversizeGroup);
+                if (last_to_arrive(t.oversize_arrived + c.slot + group, chunks_here, &s_last)) {  // whole workgroup
+                    if (tid < kDigits) {
+                        const uint32_t* column = counts - (static_cast<uint64_t>(in_group) << kPassBits) + tid;
+                        uint32_t n[kOversizeGroup], sum = 0;
+#pragma unroll
+                        for (uint32_t k = 0; k < kOversizeGroup; ++k) n[k] = load_shared(column + (min(k, chunks_here - 1) << kPassBits));
+#pragma unroll
+                        for (uint32_t k = 0; k < kOversizeGroup; ++k) sum += k < chunks_here ? n[k] : 0u;
+                        store_shared(begins + tid, sum);
+                    }
+                    const uint32_t groups = (c.chunks + kOversizeGroup - 1) / kOversizeGroup;
+                    if (last_to_arrive(t.oversize_counted + c.listed_at, groups, &s_last))
+                        place_groups(t, c, out, !MANY, bits, s_sum, s.wave);
+                }
             } else {
-                const uint32_t from = first + q0 + min(slab_place(kBucketItems, i), count - 1);
-                key[i] = load_at<uint16_t>(t.oversize_keys[(p - 1) % 2], from);
-                aux[i] = load_at<uint32_t>(t.oversize_aux[(p - 1) % 2], from);
-                if constexpr (VB != 0) val[i] = load_at<word_t>(t.oversize_vals[(p - 1) % 2], from);
-            }
-        }
-        auto digit = [&](int i) {
-            const uint32_t of_aux = aux[i], of_key = key[i];
-            return ((pass.on_aux ? of_aux : of_key) >> pass.shift) & mask;
-        };
-        if (counting) {
+                s.clear_counts();
+                if (tid < kDigits) {  // where the chunk's entries of each digit begin
+                    const uint32_t* column = counts - (static_cast<uint64_t>(in_group) << kPassBits) + tid;
+                    uint32_t n[kOversizeGroup], sum = load_shared(begins + tid);
 #pragma unroll
-            for (int i = 0; i < kBucketItems; ++i) {
-                if (in_slab(kBucketItems, i, count)) atomicAdd(&s_count[digit(i)], 1u);
-            }
-            __syncthreads();
-            for (uint32_t d = tid; d < (1u << kPassBits); d += kBucketThreads) begins[d] = s_count[d];
-        } else {
-            const bool to_output = p + 1 == t.passes;
-            uint32_t* aux_to = to_output ? out.aux : t.oversize_aux[p % 2];
-            word_t* vals_to = static_cast<word_t*>(to_output ? out.vals : t.oversize_vals[p % 2]);
-            uint32_t dest[kBucketItems / 2];
-            rank_entries<kBucketItems, kPassBits>(count, pass.bits, s.cnt, dest, digit);
-            __syncthreads();
-            // (s_count: where the digit's first entry of the chunk goes, less its place in the chunk)
-            place_digits<kBucketThreads, kPassBits>(pass.bits, s.cnt, s.wave,
-                                                    [&](uint32_t d, uint32_t at, uint32_t) { s_count[d] = begins[d] - at; });
+                    for (uint32_t k = 0; k < kOversizeGroup; ++k) n[k] = load_shared(column + (min(k, in_group) << kPassBits));
 #pragma unroll
-            for (int i = 0; i < kBucketItems; ++i) {
-                if (in_slab(kBucketItems, i, count)) {
+                    for (uint32_t k = 0; k < kOversizeGroup; ++k) sum += k < in_group ? n[k] : 0u;
+                    s_sum[tid] = sum;
+                }
+                uint32_t key[kBucketItems], aux[kBucketItems];
+                word_t val[VB ? kBucketItems : 1];
+#pragma unroll
+                for (int i = 0; i < kBucketItems; ++i) {
+                    const uint32_t from = place_of(i);
+                    if (!MANY || p == 0) {
+                        key[i] = load_at<Key>(keys_in, from);
+                        aux[i] = load_at<uint32_t>(aux_in, from);
+                        if constexpr (VB != 0) val[i] = load_at<word_t>(vals_in, from);
+                    } else {
+                        key[i] = load_shared(between_keys + from);
+                        aux[i] = load_shared(between_aux + from);
+                        if constexpr (VB != 0) val[i] = load_shared(between_vals + from);
+                    }
+                }
+                __syncthreads();
+                auto digit = [&](int i) { return digit_of(key[i], aux[i]); };
+                uint32_t dest[kBucketItems / 2];
+                rank_entries<kBucketItems, kPassBits>(count, bits, s.cnt, dest, digit);
+                __syncthreads();
+                // (s_count: where the digit's first entry of the chunk goes, less its place in the chunk)
+                place_digits<kBucketThreads, kPassBits>(bits, s.cnt, s.wave,
+                                                        [&](uint32_t d, uint32_t at, uint32_t) { s_count[d] = s_sum[d] - at; });
+                uint32_t to[kBucketItems];
+#pragma unroll
+                for (int i = 0; i < kBucketItems; ++i) {
                     const uint32_t d = digit(i);
-                    const uint32_t to = s_count[d] + s.cnt[(wave << kPassBits) + d] + ((dest[i / 2] >> (i % 2 * 16)) & 0xffffu);
-                    aux_to[to] = aux[i];
-                    if constexpr (VB != 0) vals_to[to] = val[i];
-                    if (!to_output) t.oversize_keys[p % 2][to] = static_cast<uint16_t>(key[i]);
-                    else if (out.keys != nullptr) out.keys[to] = (o.bucket << t.d3) + key[i] + out.key_bias;
+                    to[i] = s_count[d];
+                    dest[i / 2] += static_cast<uint32_t>(s.cnt[(wave << kPassBits) + d]) << (i % 2 * 16);
+                }
+                // into LDS in the new order, and out of it with neighbouring lanes on neighbouring entries
+                auto in_order = [&](auto word_of, auto use) {
+#pragma unroll
+                    for (int i = 0; i < kBucketItems; ++i) {
+                        if (in_slab(kBucketItems, i, count)) s.buf[(dest[i / 2] >> (i % 2 * 16)) & 0xffffu] = word_of(i);
+                    }
+                    __syncthreads();
+#pragma unroll
+                    for (int i = 0; i < kBucketItems; ++i) {
+                        const uint32_t at = i * kBucketThreads + tid;
+                        if (at < count) use(i, at, s.buf[at]);
+                    }
+                    __syncthreads();
+                };
+                uint32_t put[kBucketItems];
+                in_order([&](int i) { return to[i]; }, [&](int i, uint32_t at, uint32_t w) { put[i] = w + at; });
+                // (what the last pass writes nobody reads in this launch)
+                const bool to_output = !MANY || p + 1 == t.oversize_passes;
+                auto move = [&](auto word_of, auto* between, auto* output, auto finish) {
+                    if (to_output)
+                        in_order(word_of, [&](int i, uint32_t, uint32_t w) { output[put[i]] = finish(i, w); });
+                    else
+                        in_order(word_of, [&](int i, uint32_t, uint32_t w) { store_shared(between + put[i], finish(i, w)); });
+                };
+                auto as_it_is = [](int, uint32_t w) { return w; };
+                move([&](int i) { return aux[i]; }, t.oversize_aux[p % 2], out.aux, as_it_is);
+                if constexpr (VB == 4) {
+                    move([&](int i) { return val[i]; }, static_cast<uint32_t*>(t.oversize_vals[p % 2]),
+                         static_cast<uint32_t*>(out.vals), as_it_is);
+                } else if constexpr (VB == 8) {  // in two halves
+                    in_order([&](int i) { return static_cast<uint32_t>(val[i]); }, [&](int i, uint32_t, uint32_t w) { to[i] = w; });
+                    move([&](int i) { return static_cast<uint32_t>(val[i] >> 32); }, static_cast<uint64_t*>(t.oversize_vals[p % 2]),
+                         static_cast<uint64_t*>(out.vals), [&](int i, uint32_t w) { return static_cast<uint64_t>(w) << 32 | to[i]; });
+                }
+                if constexpr (MANY) {
+                    if (!to_output) {
+                        uint16_t* keys_to = t.oversize_keys[p % 2];
+                        in_order([&](int i) { return key[i]; },
+                                 [&](int i, uint32_t, uint32_t w) { store_shared(keys_to + put[i], static_cast<uint16_t>(w)); });
+                    } else {
+                        const uint32_t high = (c.bucket << t.d3) + out.key_bias;
+                        in_order([&](int i) { return key[i]; }, [&](int i, uint32_t, uint32_t w) { out.keys[put[i]] = high + w; });
+                    }
                 }
             }
+            // (both barriers here: with the second one at the head of the loop the compiler, ROCm 7.2, leaves out the wait
+            // for the store of the ticket in front of it, and some wavefronts go on with the old one)
+            __syncthreads();
+            if (tid == 0) s_ticket = ahead ? next : take_chunk(t, phase);
+            __syncthreads();
+            number = s_ticket;
         }
         wait_for_stores();
         __syncthreads();
-        if (tid == 0)
-            s_last = __hip_atomic_fetch_add(&o.done[work.phase], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1 == o.chunks;
-        __syncthreads();
-        if (s_last != 0) {  // whole workgroup
-            if (counting) place_chunks(t, o, out, t.passes == 1, pass.bits, s_sum, s.wave);
-            wait_for_stores();
-            __syncthreads();
-            if (tid == 0) __hip_atomic_store(&o.phase, work.phase + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        __syncthreads();
+        if (tid == 0 && finished != 0)
+            __hip_atomic_fetch_add(&t.oversize->done[phase], finished, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -1092,6 +1222,8 @@ void sort_passes(const SortShape& s, SortTables* t) {
     t->key_width = width_for(s.d3);
     t->passes = t->minor_passes + passes_for(s.d3);
     if (t->passes == 0) t->passes = 1;  // everything in order already: one pass over no bits
+    t->oversize_passes = std::max(passes_for(minor + s.d3), 1u);
+    t->oversize_width = (minor + s.d3 + t->oversize_passes - 1) / t->oversize_passes;
 }
 
 // Tiles of step 2 that one bucket of step 1 can have: all entries may lie in one (tiles of step 1 hold more entries, so
@@ -1100,15 +1232,17 @@ uint32_t second_tiles_most(uint32_t count) { return (count - 1) / kSecondTile + 
 
 struct SortLayout {
     size_t keys1, aux1, vals1, keys2, aux2, vals2, table1, begins1, totals1, tile_rows, table2, begins2, bucket_first,
-        tile_first, first_runs, tile_map, sub_first, oversize_count, oversize, oversize_begins, oversize_keys[2], oversize_aux[2],
-        oversize_vals[2], total;
+        tile_first, first_runs, tile_map, sub_first, sub_arrived, oversize, oversize_bucket, oversize_first, oversize_counted, oversize_arrived,
+        oversize_counts, oversize_begins, oversize_keys[2], oversize_aux[2], oversize_vals[2], total;
 };
 SortLayout sort_layout(uint32_t count, const SortShape& s, size_t value_bytes) {
     const size_t places1 = static_cast<size_t>(s.tiles1) * s.tile_size;
     const size_t places2 = static_cast<size_t>(s.max_tiles2) * kSecondTile;
     const size_t runs1 = static_cast<size_t>(s.tiles1) << s.d1, runs2 = static_cast<size_t>(s.max_tiles2) << s.d2;
     const size_t subs = size_t(1) << (s.d1 + s.d2);
+    const size_t oversize = static_cast<size_t>(count) / kBucketRoom + 1;
     const size_t chunks = 2 * (static_cast<size_t>(count) / kOversizeChunk) + 1;  // every oversize bucket has two at least
+    const size_t groups = chunks / kOversizeGroup + oversize + 1;
     SortLayout l;
     size_t off = 0;
     auto take = [&](size_t bytes) {
@@ -1133,13 +1267,18 @@ SortLayout sort_layout(uint32_t count, const SortShape& s, size_t value_bytes) {
     l.first_runs = take(s.d2 != 0 ? (static_cast<size_t>(second_tiles_most(count)) << s.d1) * sizeof(uint32_t) : 0);
     l.tile_map = take(static_cast<size_t>(s.max_tiles2) * sizeof(uint2));
     l.sub_first = take((subs + 1) * sizeof(uint32_t));
-    l.oversize_count = take(sizeof(unsigned long long));
-    l.oversize = take((static_cast<size_t>(count) / kBucketRoom + 1) * sizeof(OversizeBucket));
-    l.oversize_begins = take((chunks << kPassBits) * sizeof(uint32_t));
+    l.sub_arrived = take(sizeof(uint32_t) << s.d1);
+    l.oversize = take(sizeof(OversizeState));
+    l.oversize_bucket = take(oversize * sizeof(uint32_t));
+    l.oversize_first = take(oversize * sizeof(uint32_t));
+    l.oversize_counted = take(oversize * sizeof(uint32_t));
+    l.oversize_arrived = take(groups * sizeof(uint32_t));
+    l.oversize_counts = take((chunks << kPassBits) * sizeof(uint32_t));
+    l.oversize_begins = take((groups << kPassBits) * sizeof(uint32_t));
     SortTables passes;
     sort_passes(s, &passes);
     for (uint32_t k = 0; k < 2; ++k) {
-        const size_t between = count > kBucketRoom && passes.passes > k + 1 ? count : 0;
+        const size_t between = count > kBucketRoom && passes.oversize_passes > k + 1 ? count : 0;
         l.oversize_keys[k] = take(between * sizeof(uint16_t));
         l.oversize_aux[k] = take(between * sizeof(uint32_t));
         l.oversize_vals[k] = take(between * value_bytes);
@@ -1171,15 +1310,20 @@ void launch_sort(hipStream_t stream, EntrySource in, const SortShape& s, const S
     t.first_stride = second_tiles_most(in.count);
     t.tile_map = reinterpret_cast<uint2*>(w + l.tile_map);
     t.sub_first = words(l.sub_first);
-    t.oversize_count = reinterpret_cast<unsigned long long*>(w + l.oversize_count);
-    t.oversize = reinterpret_cast<OversizeBucket*>(w + l.oversize);
+    t.sub_arrived = words(l.sub_arrived);
+    t.oversize = reinterpret_cast<OversizeState*>(w + l.oversize);
+    t.oversize_bucket = words(l.oversize_bucket);
+    t.oversize_first = words(l.oversize_first);
+    t.oversize_counted = words(l.oversize_counted);
+    t.oversize_arrived = words(l.oversize_arrived);
+    t.oversize_counts = words(l.oversize_counts);
+    t.oversize_begins = words(l.oversize_begins);
     for (uint32_t k = 0; k < 2; ++k) {
         t.oversize_keys[k] = reinterpret_cast<uint16_t*>(w + l.oversize_keys[k]);
         t.oversize_aux[k] = words(l.oversize_aux[k]);
         t.oversize_vals[k] = w + l.oversize_vals[k];
     }
     sort_passes(s, &t);
-    t.oversize_begins = words(l.oversize_begins);
     t.d1 = s.d1;
     t.d2 = s.d2;
     t.d3 = s.d3;
@@ -1207,7 +1351,7 @@ void launch_sort(hipStream_t stream, EntrySource in, const SortShape& s, const S
         else if constexpr (kMany)
             hipLaunchKernelGGL((repartition_kernel<VB, uint16_t>), grid, dim3(kSecondThreads), 0, stream, t, keys1, aux, vals,
                                reinterpret_cast<uint16_t*>(w + l.keys2), words(l.aux2), w + l.vals2, s.max_tiles2, xcds);
-        hipLaunchKernelGGL(sub_begins_kernel, dim3(1u << s.d1), dim3(kSubBlock), 0, stream, t);
+        hipLaunchKernelGGL(sub_begins_kernel, dim3(kSubParts << s.d1), dim3(kSubBlock), 0, stream, t);
         keys = w + l.keys2;
         aux = words(l.aux2);
         vals = w + l.vals2;
@@ -1219,7 +1363,7 @@ void launch_sort(hipStream_t stream, EntrySource in, const SortShape& s, const S
         hipLaunchKernelGGL((bucket_sort_kernel<VB, Key, kMany>), grid, dim3(kBucketThreads), 0, stream, t,
                            static_cast<const Key*>(keys), aux, vals, out, buckets, xcds);
         if (in.count > kBucketRoom)  // else no bucket is larger than that
-            hipLaunchKernelGGL((oversize_kernel<VB, Key>), dim3(kOversizeGrid), dim3(kBucketThreads), 0, stream, t,
+            hipLaunchKernelGGL((oversize_kernel<VB, Key, kMany>), dim3(kOversizeGrid), dim3(kBucketThreads), 0, stream, t,
                                static_cast<const Key*>(keys), aux, vals, out);
     };
     if (short_keys2) sort(uint8_t());
