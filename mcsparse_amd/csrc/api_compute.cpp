@@ -556,18 +556,16 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
         // where the matrix has such rows.  Whether it has is part of the row-length analysis that SpMV keeps on the
         // descriptor (one kernel and a 136-byte read-back the first time a structure is seen); a call that cannot
         // use it (a stream under capture, batches with offsets of their own, COO and CSC inputs, whose offsets are
-        // built in the buffer) takes the launches.
+        // built in the buffer) takes the launches, which find out on the device and come to the same sums.
         if (A->nnz != 0 && a.m != 0 && a.n != 0) {
             bool may_have_long_rows = true;
-            a.long_row = mcsp::kSpmmLongRow;
+            a.long_row = mcsp::spmm_long_cut(a.m, a.nnz, static_cast<size_t>(a.n) * sizeof(T) <= 16);
             if (A->format == MCSPARSE_FORMAT_CSR && (batches == 1 || shared_structure)) {
                 const mcspStatus_t ps = ensure_plan(h, A, ia.rows, A->rows, A->row_num, A->nnz,
                                                     A->col_num * static_cast<int64_t>(sizeof(T)), buf + l.long_ws, true);
                 if (ps != MCSP_STATUS_SUCCESS) return ps;
-                if (A->plan.valid && A->plan.forced_family == kFamilyAuto) {
+                if (A->plan.valid && A->plan.forced_family == kFamilyAuto)
                     may_have_long_rows = A->plan.max_row_len > mcsp::kSpmmLongRow;
-                    a.long_row = mcsp::spmm_long_cut(a.m, a.nnz, static_cast<size_t>(a.n) * sizeof(T) <= 16);
-                }
             }
             if (!may_have_long_rows) {
                 a.long_row = 0;

@@ -354,10 +354,12 @@ struct SpmmArgs {
     void* C;
     int64_t ldc;
     bool c_row_major;
-    // Rows of more than long_row nonzeros (0: none are treated apart) are left out by the row kernels and taken in
-    // pieces by the kernels of spmm_long.hip, which need spmm_long_rows_bytes(nnz, long_n, value size) bytes at
-    // long_ws; long_n is the width the area was sized for (at least n).
+    // Rows of more than long_row nonzeros (0: none are treated apart), in a matrix that has rows of more than
+    // kSpmmLongRow, are left out by the row kernels and taken in pieces by the kernels of spmm_long.hip, which need
+    // spmm_long_rows_bytes(nnz, long_n, value size) bytes at long_ws; long_n is the width the area was sized for (at
+    // least n).  long_apart (device memory, set on the way): not zero where the matrix has such rows.
     idx_t long_row = 0;
+    const uint32_t* long_apart = nullptr;
     void* long_ws = nullptr;
     int64_t long_n = 0;
 };
@@ -377,8 +379,8 @@ constexpr idx_t kSpmmLongRow = 1024;
 // The cut lies below that limit, since the wavefronts of the row kernels wait for the longest of their rows: four times
 // the mean row length, between 256 (a workgroup's worth) and kSpmmLongRow.  Power-law rows, microseconds a call with a
 // cut of 128, 256, 512, 1024: a million rows and 32 fp32 columns 530, 549, 582, 650; 8 columns 403, 374, 375, 393;
-// 700 K rows and 100 columns 1078, 1051, 1038, 1032; 100 K rows and 24 columns 62, 71, 94, 141.  Where the longest row
-// is not known (COO, CSC, a capture that meets the matrix first) the cut is kSpmmLongRow: the mean row may be as long.
+// 700 K rows and 100 columns 1078, 1051, 1038, 1032; 100 K rows and 24 columns 62, 71, 94, 141.  It holds however the call
+// comes to know of the longest row, so that a row is summed in the same order by every way to the same product.
 constexpr idx_t kSpmmLongCutLeast = 256;
 // Nor where a row of op(B) is one lane: the sums of 256 groups are then added by one thread, a long way for 256 nonzeros.
 inline idx_t spmm_long_cut(idx_t m, idx_t nnz, bool one_lane) {
@@ -389,7 +391,8 @@ inline idx_t spmm_long_cut(idx_t m, idx_t nnz, bool one_lane) {
 }
 constexpr idx_t kSpmmLongChunk = 4096;
 size_t spmm_long_rows_bytes(idx_t nnz, int64_t n, size_t value_bytes);
-void launch_spmm_long_find(hipStream_t stream, const SpmmArgs& a, size_t value_bytes);
+// Lists the rows above a.long_row and their pieces; returns where it notes whether there is one above kSpmmLongRow.
+const uint32_t* launch_spmm_long_find(hipStream_t stream, const SpmmArgs& a, size_t value_bytes);
 template <typename T>
 void launch_spmm_long_rows(hipStream_t stream, const SpmmArgs& a, T alpha, T beta);
 

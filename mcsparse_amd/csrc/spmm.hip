@@ -26,7 +26,8 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 8 : 1) void sp
                                                            const idx_t* __restrict__ col, const T* __restrict__ val,
                                                            const T* __restrict__ B, int64_t ldb, T* __restrict__ C,
                                                            int64_t ldc, bool c_row_major, T alpha, T beta,
-                                                           idx_t long_row, uint32_t xcd_chunk, uint32_t xcds) {
+                                                           idx_t long_row, const uint32_t* __restrict__ apart,
+                                                           uint32_t xcd_chunk, uint32_t xcds) {
     typedef typename ByteOffset<WIDE>::type off_t;
     constexpr int kRowsPerBlock = kBlock / LR;
     const idx_t lane = threadIdx.x % LR;
@@ -39,8 +40,8 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 8 : 1) void sp
 
     const idx_t start = row_ptr[row] - base;
     const idx_t end = row_ptr[row + 1] - base;
-    // long_row != 0: rows with more nonzeros are the work of the kernels in spmm_long.hip, C included
-    if (long_row != 0 && end - start > long_row) return;  // whole lane groups
+    // long_row != 0 and *apart != 0: rows with more nonzeros are the work of the kernels in spmm_long.hip, C included
+    if (long_row != 0 && end - start > long_row && *apart != 0) return;  // whole lane groups
     T acc[V];
 #pragma unroll
     for (int i = 0; i < V; ++i) acc[i] = T(0);
@@ -126,7 +127,8 @@ __global__ __launch_bounds__(kBlock) void spmm_narrow_kernel(idx_t m, idx_t n, i
                                                              const T* __restrict__ val, const T* __restrict__ B,
                                                              int64_t ldb, T* __restrict__ Cm, int64_t ldc,
                                                              bool c_row_major, T alpha, T beta, idx_t long_row,
-                                                             uint32_t xcd_chunk, uint32_t xcds) {
+                                                             const uint32_t* __restrict__ apart, uint32_t xcd_chunk,
+                                                             uint32_t xcds) {
     constexpr int kLanes = 16;
     constexpr int P = kLanes / C;
     constexpr int kSteps = 4;  // measured on a 27-point stencil, n = 8: 1, 2, 4, 8 steps -> 305, 280, 260, 291 us
@@ -154,13 +156,13 @@ __global__ __launch_bounds__(kBlock) void spmm_narrow_kernel(idx_t m, idx_t n, i
     // row clamped to the last one and nonzeros from an index clamped to the last nonzero, and whether
     // a row or a nonzero is really there is only asked where its product would be added.
     const idx_t last_nonzero = nnz - 1;
-    // left: the row is not this kernel's to write (past the end, or longer than long_row != 0: such rows are the
-    // work of the kernels in spmm_long.hip, C included)
+    // left: the row is not this kernel's to write (past the end, or longer than long_row != 0 where *apart != 0: such
+    // rows are the work of the kernels in spmm_long.hip, C included)
     auto range_of = [&](uint64_t row, idx_t& at, idx_t& end, bool& left) {
         const uint64_t r = row < last_row ? row : last_row;
         const idx_t b = row_ptr[r] - base;
         const idx_t e = row_ptr[r + 1] - base;
-        left = row >= m || (long_row != 0 && e - b > long_row);
+        left = row >= m || (long_row != 0 && e - b > long_row && *apart != 0);
         at = b + phase;
         end = left ? b : e;  // and counts as empty
     };
@@ -264,7 +266,7 @@ void launch_narrow(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     hipLaunchKernelGGL((spmm_narrow_kernel<T, V, C>), dim3(xcd_padded_grid(blocks, chunk, xcds)), dim3(kBlock), 0, stream, a.m,
                        a.n, a.nnz, a.base, a.row_ptr, a.col, static_cast<const T*>(a.val),
                        static_cast<const T*>(a.B), a.ldb, static_cast<T*>(a.C), a.ldc, a.c_row_major, alpha, beta,
-                       a.long_row, chunk, xcds);
+                       a.long_row, a.long_apart, chunk, xcds);
 }
 
 // op(B) column-major: element (kk, j) at j*ldb + kk.  One wavefront per row of A, lanes strided
@@ -276,12 +278,13 @@ __global__ __launch_bounds__(kBlock) void spmm_colb_kernel(idx_t m, idx_t n, idx
                                                            const idx_t* __restrict__ col, const T* __restrict__ val,
                                                            const T* __restrict__ B, int64_t ldb, T* __restrict__ C,
                                                            int64_t c_row_stride, int64_t c_col_stride, T alpha,
-                                                           T beta, idx_t long_row) {
+                                                           T beta, idx_t long_row,
+                                                           const uint32_t* __restrict__ apart) {
     const unsigned lane = threadIdx.x % kWave;
     const uint64_t row = static_cast<uint64_t>(blockIdx.x) * (kBlock / kWave) + threadIdx.x / kWave;
     bool live = row < m;  // dead waves still run the reductions with zero work
-    // long_row != 0: rows with more nonzeros are the work of the kernels in spmm_long.hip, C included
-    if (live && long_row != 0 && row_ptr[row + 1] - row_ptr[row] > long_row) live = false;
+    // long_row != 0 and *apart != 0: rows with more nonzeros are the work of the kernels in spmm_long.hip, C included
+    if (live && long_row != 0 && row_ptr[row + 1] - row_ptr[row] > long_row && *apart != 0) live = false;
     const idx_t start = live ? row_ptr[row] - base : 0;
     const idx_t end = live ? row_ptr[row + 1] - base : 0;
 
@@ -740,7 +743,7 @@ void launch_rowb(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     auto launch = [&](auto wide, auto ragged) {
         hipLaunchKernelGGL((spmm_rowb_kernel<T, LR, V, decltype(wide)::value, decltype(ragged)::value>), grid, dim3(kBlock), 0,
                            stream, a.m, a.n, a.base, a.row_ptr, a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta,
-                           a.long_row, chunk, xcds);
+                           a.long_row, a.long_apart, chunk, xcds);
     };
     auto launch_offsets = [&](auto ragged) {
         if (narrow_offsets(a, sizeof(T))) launch(std::false_type{}, ragged);
@@ -771,8 +774,10 @@ void launch_rowb_v(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
 }  // namespace
 
 template <typename T>
-void launch_spmm(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
-    if (a.m == 0 || a.n == 0) return;
+void launch_spmm(hipStream_t stream, const SpmmArgs& args, T alpha, T beta) {
+    if (args.m == 0 || args.n == 0) return;
+    SpmmArgs a = args;
+    if (a.long_row != 0) a.long_apart = launch_spmm_long_find(stream, a, sizeof(T));
     if (a.b_row_major) {
         constexpr int kWide = 16 / sizeof(T);  // elements per 128-bit access
         // Rows that begin at any element take the wide loads too (27-point stencil, 872 K rows, fp32: 5, 17, 50, 101
@@ -792,17 +797,14 @@ void launch_spmm(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
         if (beta == T(0)) {
             hipLaunchKernelGGL((spmm_colb_kernel<T, kJB, true>), dim3(static_cast<uint32_t>(blocks)), dim3(kBlock), 0,
                                stream, a.m, a.n, a.base, a.row_ptr, a.col, val, B, a.ldb, C, rs, cs, alpha, beta,
-                               a.long_row);
+                               a.long_row, a.long_apart);
         } else {
             hipLaunchKernelGGL((spmm_colb_kernel<T, kJB, false>), dim3(static_cast<uint32_t>(blocks)), dim3(kBlock), 0,
                                stream, a.m, a.n, a.base, a.row_ptr, a.col, val, B, a.ldb, C, rs, cs, alpha, beta,
-                               a.long_row);
+                               a.long_row, a.long_apart);
         }
     }
-    if (a.long_row != 0) {
-        launch_spmm_long_find(stream, a, sizeof(T));
-        launch_spmm_long_rows<T>(stream, a, alpha, beta);
-    }
+    if (a.long_row != 0) launch_spmm_long_rows<T>(stream, a, alpha, beta);
 }
 
 SpmmScheduleLayout spmm_schedule_layout(idx_t m, idx_t nnz) {

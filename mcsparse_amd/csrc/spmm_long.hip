@@ -4,7 +4,9 @@
 // The reference has the same shape (one wavefront per row and output column,
 // src/kernels/level3/spmm/csr_spmm_device.hpp:121-137).  Here rows longer than the call's cut (256 to
 // 1024 nonzeros, spmm_long_cut) are left out by the row kernels and taken in pieces of kSpmmLongChunk nonzeros, a workgroup each:
-//   1. spmm_long_find_kernel lists the pieces (row, piece) and, for rows of several pieces, the rows;
+//   1. spmm_long_find_kernel lists the pieces (row, piece) and, for rows of several pieces, the rows, and notes whether any
+//      row has more than kSpmmLongRow nonzeros: if none has, the row kernels take them all.  So it runs in front of the
+//      row kernels, and what becomes of a row depends on the matrix alone, not on what the call knows of it;
 //   2. spmm_long_chunk_kernel forms the sums of a piece, all 256 threads on its nonzeros, and writes the row of C
 //      (one piece) or a row of partial sums (several);
 //   3. spmm_long_reduce_kernel adds the partial sums of a row in the order of the pieces and writes the row of C.
@@ -19,14 +21,15 @@ namespace {
 using namespace spmm_detail;
 
 struct LongCounters {
-    uint32_t items, rows, slots, pad;
+    uint32_t items, rows, slots;
+    uint32_t apart;  // not zero: there is a row of more than kSpmmLongRow nonzeros
 };
 
 __global__ void spmm_long_zero_kernel(LongCounters* c) {
     c->items = 0;
     c->rows = 0;
     c->slots = 0;
-    c->pad = 0;
+    c->apart = 0;
 }
 
 // item: {row, piece, pieces of the row, first row of partial sums of the row (unused for one piece)}
@@ -59,7 +62,7 @@ __global__ __launch_bounds__(kBlock) void spmm_long_find_kernel(idx_t m, idx_t l
                                                                 uint32_t cap_rows, uint32_t cap_slots) {
     __shared__ uint4 s_list[kFindList];      // {row, pieces, first item, first slot}, relative to the workgroup
     __shared__ uint32_t s_list_row[kFindList];  // place in the list of rows of several pieces
-    __shared__ uint32_t s_count, s_items, s_slots, s_rows;
+    __shared__ uint32_t s_count, s_items, s_slots, s_rows, s_apart;
     __shared__ uint32_t s_base[3];
     const uint32_t tid = threadIdx.x;
     if (tid == 0) {
@@ -67,6 +70,7 @@ __global__ __launch_bounds__(kBlock) void spmm_long_find_kernel(idx_t m, idx_t l
         s_items = 0;
         s_slots = 0;
         s_rows = 0;
+        s_apart = 0;
     }
     __syncthreads();
     const uint64_t row0 = static_cast<uint64_t>(blockIdx.x) * kFindRows;
@@ -85,6 +89,7 @@ __global__ __launch_bounds__(kBlock) void spmm_long_find_kernel(idx_t m, idx_t l
             const uint64_t row = row0 + k0 + u * kBlock;
             const idx_t len = lens[u];
             if (len <= long_row) continue;
+            if (len > kSpmmLongRow) s_apart = 1;
             const uint32_t pieces = (len + kSpmmLongChunk - 1) / kSpmmLongChunk;
             const uint32_t at = atomicAdd(&s_count, 1u);
             if (at < kFindList) {
@@ -105,6 +110,7 @@ __global__ __launch_bounds__(kBlock) void spmm_long_find_kernel(idx_t m, idx_t l
     const uint32_t listed = min(s_count, kFindList);
     if (listed == 0) return;  // whole workgroup
     if (tid == 0) {
+        if (s_apart != 0) c->apart = 1;
         s_base[0] = atomicAdd(&c->items, s_items);
         s_base[1] = s_slots != 0 ? atomicAdd(&c->slots, s_slots) : 0u;
         s_base[2] = s_rows != 0 ? atomicAdd(&c->rows, s_rows) : 0u;
@@ -138,7 +144,7 @@ __global__ __launch_bounds__(kBlock) void spmm_long_chunk_kernel(idx_t n, idx_t 
     const uint32_t groups = kBlock / lanes;
     const LaneColumns own = lane_columns<V>((static_cast<uint64_t>(blockIdx.y) * lanes + lane) * V, n);
     const uint64_t c0 = own.first;
-    const uint32_t count = min(c->items, cap_items);
+    const uint32_t count = c->apart != 0 ? min(c->items, cap_items) : 0u;
     const idx_t last_nonzero = nnz - 1;  // nnz != 0 where a row is long
     for (uint32_t it = blockIdx.x; it < count; it += gridDim.x) {
         const uint4 item = items[it];
@@ -221,7 +227,7 @@ __global__ __launch_bounds__(kBlock) void spmm_long_stretch_kernel(idx_t n, idx_
     const uint32_t group = threadIdx.x / LR;
     const uint32_t wave = threadIdx.x / kWave;
     const LaneColumns own = lane_columns<V>((static_cast<uint64_t>(blockIdx.y) * LR + lane) * V, n);
-    const uint32_t count = min(c->items, cap_items);
+    const uint32_t count = c->apart != 0 ? min(c->items, cap_items) : 0u;
     for (uint32_t it = blockIdx.x; it < count; it += gridDim.x) {
         const uint4 item = items[it];
         const uint32_t row = item.x, piece = item.y, pieces = item.z;
@@ -274,7 +280,7 @@ __global__ __launch_bounds__(kBlock) void spmm_long_reduce_kernel(idx_t n, T* __
                                                                   const uint4* __restrict__ rows, uint32_t cap_rows,
                                                                   const T* __restrict__ partials, int64_t ld_partials) {
     const uint64_t per_row = (static_cast<uint64_t>(n) + V - 1) / V;
-    const uint64_t work = static_cast<uint64_t>(min(c->rows, cap_rows)) * per_row;
+    const uint64_t work = c->apart != 0 ? static_cast<uint64_t>(min(c->rows, cap_rows)) * per_row : 0;
     for (uint64_t w = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; w < work;
          w += static_cast<uint64_t>(gridDim.x) * kBlock) {
         const uint4 entry = rows[w / per_row];
@@ -324,7 +330,7 @@ LongLayout long_layout(idx_t nnz, int64_t n, size_t value_bytes) {
 
 size_t spmm_long_rows_bytes(idx_t nnz, int64_t n, size_t value_bytes) { return long_layout(nnz, n, value_bytes).total; }
 
-void launch_spmm_long_find(hipStream_t stream, const SpmmArgs& a, size_t value_bytes) {
+const uint32_t* launch_spmm_long_find(hipStream_t stream, const SpmmArgs& a, size_t value_bytes) {
     const LongLayout l = long_layout(a.nnz, a.long_n, value_bytes);
     char* w = static_cast<char*>(a.long_ws);
     LongCounters* c = reinterpret_cast<LongCounters*>(w + l.counters);
@@ -332,6 +338,7 @@ void launch_spmm_long_find(hipStream_t stream, const SpmmArgs& a, size_t value_b
     hipLaunchKernelGGL(spmm_long_find_kernel, dim3((a.m + kFindRows - 1) / kFindRows), dim3(kBlock), 0, stream, a.m, a.long_row, a.row_ptr,
                        c, reinterpret_cast<uint4*>(w + l.items), reinterpret_cast<uint4*>(w + l.rows), l.cap_items,
                        l.cap_rows, l.cap_slots);
+    return &c->apart;
 }
 
 template <typename T>

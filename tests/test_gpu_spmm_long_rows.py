@@ -141,3 +141,61 @@ def test_rows_around_the_cut(torch_gpu, handle, oracle, n, dtype, short):
     a = rows_of_lengths(lengths, 5003, dtype, seed=n)
     check(torch_gpu, handle, oracle, a, n, 1.25, 0.0, pad_b=1)
     check(torch_gpu, handle, oracle, a, n, 1.25, -0.5, seed=1, c_order=api.ORDER_COL)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("c_order", [api.ORDER_ROW, api.ORDER_COL])
+@pytest.mark.parametrize("n", [3, 8, 24, 40])
+@pytest.mark.parametrize("longest", [700, 1024, 1025, 5000])
+def test_every_way_to_a_product_gives_the_same_bits(torch_gpu, oracle, dtype, c_order, n, longest):
+    """Rows between the cut (256 here) and 1024 are taken apart where there is a longer one, whether the call knows that
+    from its analysis or finds out on the device: a capture that meets the matrix first, COO and CSC inputs, a plan that
+    was set by the caller."""
+    torch = torch_gpu
+    side = torch.cuda.Stream()
+    handle = api.Handle(stream=side.cuda_stream)
+    a = rows_of_lengths([4] * 200 + [255, 256, 257, 600, 0, longest, 300] * 2, 7001, dtype, seed=n)
+    rng = np.random.default_rng(5)
+    B = dev(torch, rng.uniform(-1, 1, (a.n, n)).astype(dtype))
+    start = dev(torch, rng.uniform(-1, 1, (a.m, n) if c_order == api.ORDER_ROW else (n, a.m)).astype(dtype))
+    ct = api.maca_type(np.dtype(dtype))
+    ptr, col, val = dev(torch, a.ptr), dev(torch, a.col), dev(torch, a.val)
+    rows = dev(torch, np.repeat(np.arange(a.m, dtype=np.int32), np.diff(a.ptr)))
+    t_ptr, t_row, t_val = oracle.csr2csc(a.m, a.n, 0, a.ptr, a.col, a.val, method="counting")
+    t_ptr, t_row, t_val = dev(torch, t_ptr.astype(np.int32)), dev(torch, t_row.astype(np.int32)), dev(torch, t_val)
+    torch.cuda.synchronize()
+
+    def product(kind):
+        if kind == "coo":
+            mat = api.SpMat(a.m, a.n, a.nnz, rows, col, val, fmt=api.FORMAT_COO)
+        elif kind == "csc":
+            mat = api.SpMat(a.m, a.n, a.nnz, t_ptr, t_row, t_val, fmt=api.FORMAT_CSC)
+        else:
+            mat = api.SpMat(a.m, a.n, a.nnz, ptr, col, val)
+        if kind == "forced":
+            mat.set_plan(api.FAMILY_VECTOR)
+        C = start.clone()
+        mB, mC = api.DnMat(a.n, n, n, B), api.DnMat(a.m, n, n if c_order == api.ORDER_ROW else a.m, C, order=c_order)
+        call = (handle, api.OP_N, api.OP_N, 1.25, mat, mB, -0.5, mC, ct)
+        st, size = api.spmm_buffer_size(*call)
+        assert st == 0
+        buf = torch.empty(size, dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        if kind == "captured":
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=side):
+                assert api.spmm(*call, buf) == 0
+            for _ in range(3):
+                C.copy_(start)
+                torch.cuda.synchronize()
+                graph.replay()
+                torch.cuda.synchronize()
+        else:
+            assert api.spmm(*call, buf) == 0
+            torch.cuda.synchronize()
+        return C.cpu().numpy()
+
+    want = product("csr")
+    for kind in ("captured", "coo", "csc", "forced"):
+        assert np.array_equal(product(kind), want), kind
+    handle.destroy()
