@@ -564,8 +564,10 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
                 const mcspStatus_t ps = ensure_plan(h, A, ia.rows, A->rows, A->row_num, A->nnz,
                                                     A->col_num * static_cast<int64_t>(sizeof(T)), buf + l.long_ws, true);
                 if (ps != MCSP_STATUS_SUCCESS) return ps;
-                if (A->plan.valid && A->plan.forced_family == kFamilyAuto)
+                if (A->plan.valid && A->plan.forced_family == kFamilyAuto) {
                     may_have_long_rows = A->plan.max_row_len > mcsp::kSpmmLongRow;
+                    a.long_known = true;
+                }
             }
             if (!may_have_long_rows) {
                 a.long_row = 0;

@@ -357,8 +357,10 @@ struct SpmmArgs {
     // Rows of more than long_row nonzeros (0: none are treated apart), in a matrix that has rows of more than
     // kSpmmLongRow, are left out by the row kernels and taken in pieces by the kernels of spmm_long.hip, which need
     // spmm_long_rows_bytes(nnz, long_n, value size) bytes at long_ws; long_n is the width the area was sized for (at
-    // least n).  long_apart (device memory, set on the way): not zero where the matrix has such rows.
+    // least n).  long_known: the call knows that the matrix has such rows; else long_apart (device memory, set on the
+    // way) says so.
     idx_t long_row = 0;
+    bool long_known = false;
     const uint32_t* long_apart = nullptr;
     void* long_ws = nullptr;
     int64_t long_n = 0;

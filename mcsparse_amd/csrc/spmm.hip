@@ -40,8 +40,9 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 8 : 1) void sp
 
     const idx_t start = row_ptr[row] - base;
     const idx_t end = row_ptr[row + 1] - base;
-    // long_row != 0 and *apart != 0: rows with more nonzeros are the work of the kernels in spmm_long.hip, C included
-    if (long_row != 0 && end - start > long_row && *apart != 0) return;  // whole lane groups
+    // long_row != 0: rows with more nonzeros are the work of the kernels in spmm_long.hip, C included, unless *apart is
+    // zero (null: known not to be)
+    if (long_row != 0 && end - start > long_row && (apart == nullptr || *apart != 0)) return;  // whole lane groups
     T acc[V];
 #pragma unroll
     for (int i = 0; i < V; ++i) acc[i] = T(0);
@@ -156,13 +157,13 @@ __global__ __launch_bounds__(kBlock) void spmm_narrow_kernel(idx_t m, idx_t n, i
     // row clamped to the last one and nonzeros from an index clamped to the last nonzero, and whether
     // a row or a nonzero is really there is only asked where its product would be added.
     const idx_t last_nonzero = nnz - 1;
-    // left: the row is not this kernel's to write (past the end, or longer than long_row != 0 where *apart != 0: such
-    // rows are the work of the kernels in spmm_long.hip, C included)
+    // left: the row is not this kernel's to write (past the end, or longer than long_row != 0: such rows are the work of
+    // the kernels in spmm_long.hip, C included, unless *apart is zero)
     auto range_of = [&](uint64_t row, idx_t& at, idx_t& end, bool& left) {
         const uint64_t r = row < last_row ? row : last_row;
         const idx_t b = row_ptr[r] - base;
         const idx_t e = row_ptr[r + 1] - base;
-        left = row >= m || (long_row != 0 && e - b > long_row && *apart != 0);
+        left = row >= m || (long_row != 0 && e - b > long_row && (apart == nullptr || *apart != 0));
         at = b + phase;
         end = left ? b : e;  // and counts as empty
     };
@@ -283,8 +284,8 @@ __global__ __launch_bounds__(kBlock) void spmm_colb_kernel(idx_t m, idx_t n, idx
     const unsigned lane = threadIdx.x % kWave;
     const uint64_t row = static_cast<uint64_t>(blockIdx.x) * (kBlock / kWave) + threadIdx.x / kWave;
     bool live = row < m;  // dead waves still run the reductions with zero work
-    // long_row != 0 and *apart != 0: rows with more nonzeros are the work of the kernels in spmm_long.hip, C included
-    if (live && long_row != 0 && row_ptr[row + 1] - row_ptr[row] > long_row && *apart != 0) live = false;
+    // long_row != 0: rows with more nonzeros are the work of the kernels in spmm_long.hip, C included, unless *apart is zero
+    if (live && long_row != 0 && row_ptr[row + 1] - row_ptr[row] > long_row && (apart == nullptr || *apart != 0)) live = false;
     const idx_t start = live ? row_ptr[row] - base : 0;
     const idx_t end = live ? row_ptr[row + 1] - base : 0;
 
@@ -777,7 +778,8 @@ template <typename T>
 void launch_spmm(hipStream_t stream, const SpmmArgs& args, T alpha, T beta) {
     if (args.m == 0 || args.n == 0) return;
     SpmmArgs a = args;
-    if (a.long_row != 0) a.long_apart = launch_spmm_long_find(stream, a, sizeof(T));
+    // (behind the row kernel the offsets are in cache: 1 to 2 us less where the call knows that there are long rows)
+    if (a.long_row != 0 && !a.long_known) a.long_apart = launch_spmm_long_find(stream, a, sizeof(T));
     if (a.b_row_major) {
         constexpr int kWide = 16 / sizeof(T);  // elements per 128-bit access
         // Rows that begin at any element take the wide loads too (27-point stencil, 872 K rows, fp32: 5, 17, 50, 101
@@ -804,6 +806,7 @@ void launch_spmm(hipStream_t stream, const SpmmArgs& args, T alpha, T beta) {
                                a.long_row, a.long_apart);
         }
     }
+    if (a.long_row != 0 && a.long_known) launch_spmm_long_find(stream, a, sizeof(T));
     if (a.long_row != 0) launch_spmm_long_rows<T>(stream, a, alpha, beta);
 }
 

@@ -5,8 +5,8 @@
 // src/kernels/level3/spmm/csr_spmm_device.hpp:121-137).  Here rows longer than the call's cut (256 to
 // 1024 nonzeros, spmm_long_cut) are left out by the row kernels and taken in pieces of kSpmmLongChunk nonzeros, a workgroup each:
 //   1. spmm_long_find_kernel lists the pieces (row, piece) and, for rows of several pieces, the rows, and notes whether any
-//      row has more than kSpmmLongRow nonzeros: if none has, the row kernels take them all.  So it runs in front of the
-//      row kernels, and what becomes of a row depends on the matrix alone, not on what the call knows of it;
+//      row has more than kSpmmLongRow nonzeros: if none has, the row kernels take them all.  A call that does not know
+//      that beforehand runs it in front of the row kernels, so what becomes of a row depends on the matrix alone;
 //   2. spmm_long_chunk_kernel forms the sums of a piece, all 256 threads on its nonzeros, and writes the row of C
 //      (one piece) or a row of partial sums (several);
 //   3. spmm_long_reduce_kernel adds the partial sums of a row in the order of the pieces and writes the row of C.
@@ -22,17 +22,17 @@ using namespace spmm_detail;
 
 struct LongCounters {
     uint32_t items, rows, slots;
-    // not zero: there is a row of more than kSpmmLongRow nonzeros (on a line of its own: a store among the adds to the
+    // not zero: the listed rows are taken apart, since there is one of more than kSpmmLongRow nonzeros (on a line of its own: a store among the adds to the
     // counters makes the find kernel wait, 16.5 -> 27.5 us on a million rows)
     alignas(128) uint32_t apart;
 };
 static_assert(sizeof(LongCounters) <= 2 * kAlign, "what the layout has room for");
 
-__global__ void spmm_long_zero_kernel(LongCounters* c) {
+__global__ void spmm_long_zero_kernel(LongCounters* c, bool known) {
     c->items = 0;
     c->rows = 0;
     c->slots = 0;
-    c->apart = 0;
+    c->apart = known ? 1 : 0;
 }
 
 // item: {row, piece, pieces of the row, first row of partial sums of the row (unused for one piece)}
@@ -339,7 +339,7 @@ const uint32_t* launch_spmm_long_find(hipStream_t stream, const SpmmArgs& a, siz
     const LongLayout l = long_layout(a.nnz, a.long_n, value_bytes);
     char* w = static_cast<char*>(a.long_ws);
     LongCounters* c = reinterpret_cast<LongCounters*>(w + l.counters);
-    hipLaunchKernelGGL(spmm_long_zero_kernel, dim3(1), dim3(1), 0, stream, c);
+    hipLaunchKernelGGL(spmm_long_zero_kernel, dim3(1), dim3(1), 0, stream, c, a.long_known);
     hipLaunchKernelGGL(spmm_long_find_kernel, dim3((a.m + kFindRows - 1) / kFindRows), dim3(kBlock), 0, stream, a.m, a.long_row, a.row_ptr,
                        c, reinterpret_cast<uint4*>(w + l.items), reinterpret_cast<uint4*>(w + l.rows), l.cap_items,
                        l.cap_rows, l.cap_slots);
