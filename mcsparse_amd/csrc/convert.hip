@@ -44,20 +44,6 @@ __device__ __forceinline__ idx_t wave_count_row_starts(const idx_t* __restrict__
     return static_cast<idx_t>(lo);
 }
 
-// Inclusive sum over the 64 lanes of a wavefront: four shifted adds inside each row of 16 lanes,
-// then the last lane of rows 0 and 2 is added to rows 1 and 3, then lane 31 to rows 2 and 3.
-__device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t v) {
-    constexpr int kRowShr = 0x110, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
-    int x = static_cast<int>(v);
-    x += __builtin_amdgcn_update_dpp(0, x, kRowShr + 1, 0xF, 0xF, false);
-    x += __builtin_amdgcn_update_dpp(0, x, kRowShr + 2, 0xF, 0xF, false);
-    x += __builtin_amdgcn_update_dpp(0, x, kRowShr + 4, 0xF, 0xF, false);
-    x += __builtin_amdgcn_update_dpp(0, x, kRowShr + 8, 0xF, 0xF, false);
-    x += __builtin_amdgcn_update_dpp(0, x, kRowBcast15, 0xA, 0xF, false);
-    x += __builtin_amdgcn_update_dpp(0, x, kRowBcast31, 0xC, 0xF, false);
-    return static_cast<uint32_t>(x);
-}
-
 // coo_rows[j] = row of nonzero j (+ base) = the number of rows that begin at or before j, minus one.
 // A tile is 4096 nonzeros.  The rows that begin inside it are read from row_ptr (the first of them is
 // known from the tile before; only where a workgroup's first tile begins is searched for, a chain of
@@ -563,19 +549,9 @@ __device__ __forceinline__ uint32_t digit_exclusive_scan(uint32_t v, uint32_t* s
 // position of the first key of each (digit, tile).  FROM_CSR: the triples are the nonzeros of a
 // CSR matrix in place -- rows_in is its row_ptr array (m + 1 offsets, index base `base`) and the
 // row of every nonzero (+ base) is worked out here instead of being read.
-template <int VB>
-struct ValueOf { typedef uint32_t type; };
-template <>
-struct ValueOf<8> { typedef uint64_t type; };
-
 // AUX = false: (key, value) pairs, rows_out is not written.  TIMES_X (with FROM_CSR, without AUX): the
 // value that travels is value * x[row of the nonzero], in the floating-point type of VB bytes.
 // bias is subtracted from a key wherever a digit is taken from it (the index base, where that saves a bit).
-template <int VB>
-struct RealOf { typedef float type; };
-template <>
-struct RealOf<8> { typedef double type; };
-
 template <int VB, bool FROM_CSR, bool AUX, bool TIMES_X>
 __global__ __launch_bounds__(kSortBlock) void radix_scatter_kernel(
     const idx_t* __restrict__ keys_in, const idx_t* __restrict__ rows_in, const void* __restrict__ vals_in_v,
@@ -585,7 +561,7 @@ __global__ __launch_bounds__(kSortBlock) void radix_scatter_kernel(
     uint32_t xcds) {
     static_assert(AUX || VB != 0, "pairs carry a value");
     static_assert(!TIMES_X || (FROM_CSR && !AUX), "products are formed where the rows are worked out");
-    typedef typename ValueOf<VB>::type val_t;
+    typedef typename WordOf<VB>::type val_t;
     const val_t* vals_in = static_cast<const val_t*>(vals_in_v);
     val_t* vals_out = static_cast<val_t*>(vals_out_v);
 

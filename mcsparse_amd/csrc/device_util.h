@@ -102,6 +102,30 @@ __device__ __forceinline__ void static_for(F&& f) {
     static_for_impl(static_cast<F&&>(f), std::make_integer_sequence<int, N>{});
 }
 
+// Inclusive sum over the 64 lanes: four shifted adds inside each row of 16 lanes, then the last lane of rows 0 and 2
+// is added to rows 1 and 3, then lane 31 to rows 2 and 3.
+__device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t v) {
+    constexpr int kRowShr = 0x110, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+    int x = static_cast<int>(v);
+    x += __builtin_amdgcn_update_dpp(0, x, kRowShr + 1, 0xF, 0xF, false);
+    x += __builtin_amdgcn_update_dpp(0, x, kRowShr + 2, 0xF, 0xF, false);
+    x += __builtin_amdgcn_update_dpp(0, x, kRowShr + 4, 0xF, 0xF, false);
+    x += __builtin_amdgcn_update_dpp(0, x, kRowShr + 8, 0xF, 0xF, false);
+    x += __builtin_amdgcn_update_dpp(0, x, kRowBcast15, 0xA, 0xF, false);
+    x += __builtin_amdgcn_update_dpp(0, x, kRowBcast31, 0xC, 0xF, false);
+    return static_cast<uint32_t>(x);
+}
+
+// A value of VB bytes (0: no values) as a word to move and as a number.
+template <int VB>
+struct WordOf { typedef uint32_t type; };
+template <>
+struct WordOf<8> { typedef uint64_t type; };
+template <int VB>
+struct RealOf { typedef float type; };
+template <>
+struct RealOf<8> { typedef double type; };
+
 __device__ __forceinline__ unsigned lane_id() { return __lane_id(); }
 
 // Streaming loads: data read once, kept from displacing the gathered operand in cache.

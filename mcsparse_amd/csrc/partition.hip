@@ -29,15 +29,6 @@ namespace {
 
 using namespace partition_detail;
 
-template <int VB>
-struct WordOf { typedef uint32_t type; };
-template <>
-struct WordOf<8> { typedef uint64_t type; };
-template <int VB>
-struct RealOf { typedef float type; };
-template <>
-struct RealOf<8> { typedef double type; };
-
 // ---- step 1 ----------------------------------------------------------------------------------------------------
 // What the entries of a sort are.  CSR: `aux` holds the m + 1 row offsets (index base `base`) of a matrix whose
 // nonzeros are the entries, and an entry's index is its row + base.

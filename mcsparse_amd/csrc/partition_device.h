@@ -12,20 +12,6 @@ namespace partition_detail {
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // ---- one wavefront ---------------------------------------------------------------------------------------------
-// Inclusive sum over the 64 lanes: four shifted adds inside each row of 16 lanes, then the last lane of rows 0 and 2
-// is added to rows 1 and 3, then lane 31 to rows 2 and 3.
-__device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t v) {
-    constexpr int kRowShr = 0x110, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
-    int x = static_cast<int>(v);
-    x += __builtin_amdgcn_update_dpp(0, x, kRowShr + 1, 0xF, 0xF, false);
-    x += __builtin_amdgcn_update_dpp(0, x, kRowShr + 2, 0xF, 0xF, false);
-    x += __builtin_amdgcn_update_dpp(0, x, kRowShr + 4, 0xF, 0xF, false);
-    x += __builtin_amdgcn_update_dpp(0, x, kRowShr + 8, 0xF, 0xF, false);
-    x += __builtin_amdgcn_update_dpp(0, x, kRowBcast15, 0xA, 0xF, false);
-    x += __builtin_amdgcn_update_dpp(0, x, kRowBcast31, 0xC, 0xF, false);
-    return static_cast<uint32_t>(x);
-}
-
 // How many of the ascending values a[0 .. n) are <= g, with 64 probes per round.  Every lane of the wavefront must
 // call this; all lanes return the same value.
 __device__ __forceinline__ uint32_t wave_count_up_to(const uint32_t* __restrict__ a, uint32_t n, uint32_t base, uint32_t g) {

@@ -22,8 +22,8 @@ using namespace spmm_detail;
 
 struct LongCounters {
     uint32_t items, rows, slots;
-    // not zero: the listed rows are taken apart, since there is one of more than kSpmmLongRow nonzeros (on a line of its own: a store among the adds to the
-    // counters makes the find kernel wait, 16.5 -> 27.5 us on a million rows)
+    // not zero: the listed rows are taken apart, since there is one of more than kSpmmLongRow nonzeros (on a line of its
+    // own: a store among the adds to the counters makes the find kernel wait, 16.5 -> 27.5 us on a million rows)
     alignas(128) uint32_t apart;
 };
 static_assert(sizeof(LongCounters) <= 2 * kAlign, "what the layout has room for");
