@@ -333,6 +333,19 @@ template <typename W>
 __device__ __forceinline__ void store_shared(W* p, W v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// The same at array[index], for arrays of less than 4 GiB: a scalar base and a 32-bit offset.
+template <typename W>
+__device__ __forceinline__ W load_shared_at(const void* array, uint32_t index) {
+    return load_shared(reinterpret_cast<const W*>(static_cast<const char*>(array) + index * static_cast<uint32_t>(sizeof(W))));
+}
+template <typename W>
+__device__ __forceinline__ void store_at(void* array, uint32_t index, W v) {
+    *reinterpret_cast<W*>(static_cast<char*>(array) + index * static_cast<uint32_t>(sizeof(W))) = v;
+}
+template <typename W>
+__device__ __forceinline__ void store_shared_at(void* array, uint32_t index, W v) {
+    store_shared(reinterpret_cast<W*>(static_cast<char*>(array) + index * static_cast<uint32_t>(sizeof(W))), v);
+}
 // One more of `all` has come: was it the last?  For the whole workgroup; whoever comes last may load_shared what the others
 // have written with store_shared.
 __device__ __forceinline__ bool last_to_arrive(uint32_t* counter, uint32_t all, uint32_t* s_last) {
@@ -818,10 +831,10 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 || MANY ? 6 : 8) void bucke
 //
 // Before, a workgroup looked for work among all buckets with two device-wide fences a chunk, one workgroup placed all
 // chunks of a bucket, the counting phase read whole entries, and entries were written from where they lay in registers:
-// csr2csc of 67 M nonzeros with columns by Zipf's law (53 M of them in such buckets) 3690 us, now 1475 (LSD passes: 1484);
-// an index sort of 10 M triples with rows by that law 1870 us, now 960.
-// Index sorts by a skewed major key stay slower than the LSD passes: 503 us for those, 936 against 1550 for 21.8 M triples
-// in a million power-law rows of up to 50,000 (38 % of them in such buckets).  A pass over such a bucket costs two phases
+// csr2csc of 67 M nonzeros with columns by Zipf's law (53 M of them in such buckets) 3690 us, now 1458 (LSD passes: 1484);
+// an index sort of 10 M triples with rows by that law 1870 us, now 953.
+// Index sorts by a skewed major key stay slower than the LSD passes: 503 us for those, 936 against 1609 for 21.8 M triples
+// in a million power-law rows of up to 50,000 (38 % of them in such buckets), 156 against 188 in a hundred thousand rows.  A pass over such a bucket costs two phases
 // of 45 us at least, and there are four or five of them.  How the keys are spread is not known on the host, where the
 // choice is made, and evenly spread ones gain as much (10 M: 481 and 330 us); so does csr2csc under any spread.
 constexpr uint32_t kOversizeGrid = 512;
@@ -895,7 +908,7 @@ __device__ __forceinline__ void place_groups(const SortTables& t, const Oversize
 }
 
 template <int VB, typename Key, bool MANY>
-__global__ __launch_bounds__(kBucketThreads, 4) void oversize_kernel(SortTables t, const Key* __restrict__ keys_in,
+__global__ __launch_bounds__(kBucketThreads, VB == 8 ? 2 : 4) void oversize_kernel(SortTables t, const Key* __restrict__ keys_in,
                                                                   const uint32_t* __restrict__ aux_in,
                                                                   const void* __restrict__ vals_in, SortOutput out) {
     typedef typename WordOf<VB>::type word_t;
@@ -952,9 +965,15 @@ __global__ __launch_bounds__(kBucketThreads, 4) void oversize_kernel(SortTables 
                                                       s.map, s.buf);
             }
             const uint32_t last_word = (count - 1) / kWave;
+            // (worked out for every chunk again: as what it is, the same for all chunks, each item's share of it is held in
+            // a register from the start on, and the kernel needs scratch memory)
+            uint32_t own_wave = wave, own_slab = slab_place(kBucketItems, 0), own_thread = tid;
+            forget(own_wave);
+            forget(own_slab);
+            forget(own_thread);
             auto place_of = [&](int i) {
-                return p == 0 ? mapped_place(s.map, s.buf, min(wave * kBucketItems + i, last_word), count)
-                              : c.first + q0 + min(slab_place(kBucketItems, i), count - 1);
+                return p == 0 ? mapped_place(s.map, s.buf, min(own_wave * kBucketItems + i, last_word), count)
+                              : c.first + q0 + min(own_slab + i * kWave, count - 1);
             };
             if (phase % 2 == 0) {
                 if (tid < kDigits) s_count[tid] = 0;
@@ -963,10 +982,10 @@ __global__ __launch_bounds__(kBucketThreads, 4) void oversize_kernel(SortTables 
                 for (int i = 0; i < kBucketItems; ++i) {
                     const uint32_t from = place_of(i);
                     key[i] = 0;
-                    if (by_key) key[i] = p == 0 ? load_at<Key>(keys_in, from) : load_shared(between_keys + from);
+                    if (by_key) key[i] = p == 0 ? load_at<Key>(keys_in, from) : load_shared_at<uint16_t>(between_keys, from);
                     if constexpr (MANY) {
                         aux[i] = 0;
-                        if (by_aux) aux[i] = p == 0 ? load_at<uint32_t>(aux_in, from) : load_shared(between_aux + from);
+                        if (by_aux) aux[i] = p == 0 ? load_at<uint32_t>(aux_in, from) : load_shared_at<uint32_t>(between_aux, from);
                     }
                 }
                 __syncthreads();
@@ -1012,9 +1031,9 @@ __global__ __launch_bounds__(kBucketThreads, 4) void oversize_kernel(SortTables 
                         aux[i] = load_at<uint32_t>(aux_in, from);
                         if constexpr (VB != 0) val[i] = load_at<word_t>(vals_in, from);
                     } else {
-                        key[i] = load_shared(between_keys + from);
-                        aux[i] = load_shared(between_aux + from);
-                        if constexpr (VB != 0) val[i] = load_shared(between_vals + from);
+                        key[i] = load_shared_at<uint16_t>(between_keys, from);
+                        aux[i] = load_shared_at<uint32_t>(between_aux, from);
+                        if constexpr (VB != 0) val[i] = load_shared_at<word_t>(between_vals, from);
                     }
                 }
                 __syncthreads();
@@ -1025,13 +1044,9 @@ __global__ __launch_bounds__(kBucketThreads, 4) void oversize_kernel(SortTables 
                 // (s_count: where the digit's first entry of the chunk goes, less its place in the chunk)
                 place_digits<kBucketThreads, kPassBits>(bits, s.cnt, s.wave,
                                                         [&](uint32_t d, uint32_t at, uint32_t) { s_count[d] = s_sum[d] - at; });
-                uint32_t to[kBucketItems];
 #pragma unroll
-                for (int i = 0; i < kBucketItems; ++i) {
-                    const uint32_t d = digit(i);
-                    to[i] = s_count[d];
-                    dest[i / 2] += static_cast<uint32_t>(s.cnt[(wave << kPassBits) + d]) << (i % 2 * 16);
-                }
+                for (int i = 0; i < kBucketItems; ++i)
+                    dest[i / 2] += static_cast<uint32_t>(s.cnt[(wave << kPassBits) + digit(i)]) << (i % 2 * 16);
                 // into LDS in the new order, and out of it with neighbouring lanes on neighbouring entries
                 auto in_order = [&](auto word_of, auto use) {
 #pragma unroll
@@ -1041,20 +1056,20 @@ __global__ __launch_bounds__(kBucketThreads, 4) void oversize_kernel(SortTables 
                     __syncthreads();
 #pragma unroll
                     for (int i = 0; i < kBucketItems; ++i) {
-                        const uint32_t at = i * kBucketThreads + tid;
+                        const uint32_t at = i * kBucketThreads + own_thread;
                         if (at < count) use(i, at, s.buf[at]);
                     }
                     __syncthreads();
                 };
                 uint32_t put[kBucketItems];
-                in_order([&](int i) { return to[i]; }, [&](int i, uint32_t at, uint32_t w) { put[i] = w + at; });
+                in_order([&](int i) { return s_count[digit(i)]; }, [&](int i, uint32_t at, uint32_t w) { put[i] = w + at; });
                 // (what the last pass writes nobody reads in this launch)
                 const bool to_output = !MANY || p + 1 == t.oversize_passes;
                 auto move = [&](auto word_of, auto* between, auto* output, auto finish) {
                     if (to_output)
-                        in_order(word_of, [&](int i, uint32_t, uint32_t w) { output[put[i]] = finish(i, w); });
+                        in_order(word_of, [&](int i, uint32_t, uint32_t w) { store_at(output, put[i], finish(i, w)); });
                     else
-                        in_order(word_of, [&](int i, uint32_t, uint32_t w) { store_shared(between + put[i], finish(i, w)); });
+                        in_order(word_of, [&](int i, uint32_t, uint32_t w) { store_shared_at(between, put[i], finish(i, w)); });
                 };
                 auto as_it_is = [](int, uint32_t w) { return w; };
                 move([&](int i) { return aux[i]; }, t.oversize_aux[p % 2], out.aux, as_it_is);
@@ -1062,18 +1077,19 @@ __global__ __launch_bounds__(kBucketThreads, 4) void oversize_kernel(SortTables 
                     move([&](int i) { return val[i]; }, static_cast<uint32_t*>(t.oversize_vals[p % 2]),
                          static_cast<uint32_t*>(out.vals), as_it_is);
                 } else if constexpr (VB == 8) {  // in two halves
-                    in_order([&](int i) { return static_cast<uint32_t>(val[i]); }, [&](int i, uint32_t, uint32_t w) { to[i] = w; });
+                    uint32_t low[kBucketItems];
+                    in_order([&](int i) { return static_cast<uint32_t>(val[i]); }, [&](int i, uint32_t, uint32_t w) { low[i] = w; });
                     move([&](int i) { return static_cast<uint32_t>(val[i] >> 32); }, static_cast<uint64_t*>(t.oversize_vals[p % 2]),
-                         static_cast<uint64_t*>(out.vals), [&](int i, uint32_t w) { return static_cast<uint64_t>(w) << 32 | to[i]; });
+                         static_cast<uint64_t*>(out.vals), [&](int i, uint32_t w) { return static_cast<uint64_t>(w) << 32 | low[i]; });
                 }
                 if constexpr (MANY) {
                     if (!to_output) {
                         uint16_t* keys_to = t.oversize_keys[p % 2];
                         in_order([&](int i) { return key[i]; },
-                                 [&](int i, uint32_t, uint32_t w) { store_shared(keys_to + put[i], static_cast<uint16_t>(w)); });
+                                 [&](int i, uint32_t, uint32_t w) { store_shared_at(keys_to, put[i], static_cast<uint16_t>(w)); });
                     } else {
                         const uint32_t high = (c.bucket << t.d3) + out.key_bias;
-                        in_order([&](int i) { return key[i]; }, [&](int i, uint32_t, uint32_t w) { out.keys[put[i]] = high + w; });
+                        in_order([&](int i) { return key[i]; }, [&](int i, uint32_t, uint32_t w) { store_at(out.keys, put[i], high + w); });
                     }
                 }
             }
