@@ -766,8 +766,8 @@ mcspStatus_t spmv_call(mcsparseHandle_t handle, mcsparseOperation_t opA, const v
 // banded matrix reads x line by line as it is; an x that fits an L2 next to rows long enough to fill the lanes
 // leaves the copy's extra partial sums as pure cost), so both are run here, on the handle's stream, with the
 // caller's x and a y inside the buffer, and timed with events: once each, which settles it where one takes more
-// than twice the other's time (or, for long runs, a quarter more), else twice more.  *copy_wins says whether the copy was faster by more than a
-// twentieth.
+// than twice the other's time (or, for long runs, a quarter more), else twice more.  *copy_wins says whether the
+// copy was faster by more than a twentieth.
 mcspStatus_t spmv_trial(mcsparseHandle_t handle, mcsparseOperation_t opA, mcsparseSpMatDescr_t matA,
                         mcsparseDnVecDescr_t vecX, void* trial_y, macaDataType computeType, void* buffer,
                         mcsparseSpMVAlg_t alg, bool* copy_wins) {
@@ -783,7 +783,9 @@ mcspStatus_t spmv_trial(mcsparseHandle_t handle, mcsparseOperation_t opA, mcspar
     const mcsparsePointerMode_t callers_mode = handle->ptr_mode;
     handle->ptr_mode = MCSPARSE_POINTER_MODE_HOST;
     hipEvent_t marks[3] = {nullptr, nullptr, nullptr};  // before the row kernels, between the two, after the copy
-    mcspStatus_t st = MCSP_STATUS_SUCCESS;
+    // (in a process that has run no product yet the row kernels would be loaded between the marks, look many times as slow as
+    // they are, and lose; the copy's kernels are there, its build is among them)
+    mcspStatus_t st = load_row_kernels() ? MCSP_STATUS_SUCCESS : MCSP_STATUS_INTERNAL_ERROR;
     for (hipEvent_t& e : marks)
         if (st == MCSP_STATUS_SUCCESS && hipEventCreate(&e) != hipSuccess) st = MCSP_STATUS_INTERNAL_ERROR;
     float rows_ms = 0.0f, copy_ms = 0.0f;

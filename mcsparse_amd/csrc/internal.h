@@ -279,6 +279,9 @@ struct SpmvArgs {
     void* y;
 };
 // y = alpha*A*x + beta*y; beta == 0 never reads y.
+// The kernels of spmv.hip come to the device together, with the first launch of any of them, which takes that launch
+// milliseconds.  This call brings them there beforehand.
+bool load_row_kernels();
 template <typename T>
 void launch_spmv_vector(hipStream_t stream, const SpmvArgs& a, T alpha, T beta, int lanes);
 // workspace: spmv_merge_workspace_bytes(m, nnz, sizeof(T)) bytes of device scratch.

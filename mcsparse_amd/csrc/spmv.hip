@@ -479,6 +479,11 @@ int spmv_pick_lanes(idx_t m, idx_t nnz) {
     return lanes;
 }
 
+bool load_row_kernels() {
+    hipFuncAttributes attributes;
+    return hipFuncGetAttributes(&attributes, reinterpret_cast<const void*>(spmv_vector_kernel<float, 8, 4, 0>)) == hipSuccess;
+}
+
 template <typename T>
 void launch_spmv_vector(hipStream_t stream, const SpmvArgs& a, T alpha, T beta, int lanes) {
     if (a.m == 0) return;

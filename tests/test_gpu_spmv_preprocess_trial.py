@@ -2,6 +2,10 @@
 kernels and keeps the copy only where it is the faster one.  Checked here: a preprocessed call is never much slower
 than a call that was not prepared; the trial leaves the caller's y and the handle alone; results stay within
 8*u*(|alpha| * |A||x| + |beta*y|) whichever way the trial went."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -163,3 +167,36 @@ def test_a_band_width_set_by_the_caller_is_not_tried(torch_gpu, handle, oracle):
     torch.cuda.synchronize()
     y_ref, bound = oracle.spmv(False, a.m, a.n, a.base, a.ptr, a.col, a.val, 1.0, 0.0, x_host, np.zeros(a.m, np.float32))
     assert_within(y.cpu().numpy(), y_ref, bound, np.float32, what="copy of a caller who set the band width")
+
+
+FIRST_OF_A_PROCESS = """
+import sys
+sys.path.insert(0, sys.argv[1])
+import numpy as np
+import torch
+from mcsparse_amd import api
+from mcsparse_amd import workloads as wl
+a = wl.stencil_27pt(96, dtype=np.float64)
+handle = api.Handle(stream=torch.cuda.current_stream().cuda_stream)
+ptr, col, val = (torch.from_numpy(v.astype(t)).cuda() for v, t in ((a.ptr, np.int32), (a.col, np.int32), (a.val, np.float64)))
+x, y = torch.rand(a.n, dtype=torch.float64, device="cuda"), torch.zeros(a.m, dtype=torch.float64, device="cuda")
+mat = api.SpMat(a.m, a.n, a.nnz, ptr, col, val, base=a.base)
+vx, vy = api.DnVec(x), api.DnVec(y)
+call = (handle, api.OP_N, 1.0, mat, vx, 0.0, vy, api.R_64F)
+st, size = api.spmv_preprocess_buffer_size(*call)
+assert st == 0
+buf = torch.empty(size, dtype=torch.uint8, device="cuda")
+assert api.spmv_preprocess(*call, buf) == 0
+print("state", mat.spmv_preprocess_state()[0])
+"""
+
+
+def test_the_first_preparation_of_a_process_decides_as_later_ones_do(torch_gpu):
+    """A program that prepares its one matrix and has run no product before: the row kernels come to the device with
+    their first launch, which must not count as their time (120 us a call instead of 74 on a 27-point stencil when it
+    did)."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    run = subprocess.run([sys.executable, "-c", FIRST_OF_A_PROCESS, root], stdout=subprocess.PIPE, stderr=subprocess.PIPE,
+                         text=True, timeout=100)
+    assert run.returncode == 0, run.stderr
+    assert run.stdout.strip() == "state 1", run.stdout
