@@ -834,9 +834,10 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 || MANY ? 6 : 8) void bucke
 // csr2csc of 67 M nonzeros with columns by Zipf's law (53 M of them in such buckets) 3690 us, now 1458 (LSD passes: 1484);
 // an index sort of 10 M triples with rows by that law 1870 us, now 953.
 // Index sorts by a skewed major key stay slower than the LSD passes: 503 us for those, 936 against 1609 for 21.8 M triples
-// in a million power-law rows of up to 50,000 (38 % of them in such buckets), 156 against 188 in a hundred thousand rows.  A pass over such a bucket costs two phases
-// of 45 us at least, and there are four or five of them.  How the keys are spread is not known on the host, where the
-// choice is made, and evenly spread ones gain as much (10 M: 481 and 330 us); so does csr2csc under any spread.
+// in a million power-law rows of up to 50,000 (38 % of them in such buckets), 156 against 188 in a hundred thousand rows.
+// A pass over such a bucket costs two phases of 45 us at least, and there are four or five of them.  How the keys are
+// spread is not known on the host, where the choice is made, and evenly spread ones gain as much (10 M: 481 and 330 us);
+// so does csr2csc under any spread.
 constexpr uint32_t kOversizeGrid = 512;
 
 struct OversizeChunk {
