@@ -41,6 +41,10 @@ struct EntrySource {
     uint32_t key_bias;     // subtracted from a key before its bits are taken
     uint32_t m, base;
     const uint32_t* tile_rows;  // CSR: rows that begin at or before each tile's first nonzero
+    // CSR, packed entries: the index is counted from the tile's first row; a tile with more rows than the word has room for
+    // leaves its indices in an array of their own and sets *wide
+    bool relative;
+    uint32_t* wide;
 };
 
 // The order of tiles over the workgroups: an XCD takes a contiguous range, so the table words of neighbouring tiles,
@@ -231,6 +235,23 @@ __global__ __launch_bounds__(THREADS) void partition_kernel(EntrySource in, uint
     }
     if constexpr (VB != 0 && !kValuesEarly) load_values();
     const uint64_t out = static_cast<uint64_t>(tile) * kPlaces;
+    if constexpr (packed_entries<Key>()) {
+        static_assert(KIND == kCsr, "packed entries");
+        uint32_t origin = 0u - in.base;
+        if (in.relative) {  // (shift != 0: there is a second step)
+            origin = before - 1;
+            if (inside >> (32 - shift) != 0) {  // whole workgroup
+#pragma unroll
+                for (int i = 0; i < ITEMS; ++i) aux[i] += in.base;
+                store_words<ITEMS, THREADS, kPlaces>(s_buf, count, dest, aux_out + out, aux);
+                if (tid == 0) *in.wide = 1;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) key[i] = (key[i] & ((1u << shift) - 1u)) | (aux[i] - origin) << shift;
+        store_packed<VB, ITEMS, THREADS, kPlaces>(s_buf, count, dest, keys_out, vals_out, out, [&](int i) { return key[i]; }, val);
+        return;
+    }
     store_keys<ITEMS, THREADS, kPlaces>(s_buf, count, dest, keys_out + out, key, (1u << shift) - 1u);
     if constexpr (KIND == kProducts) {
         typedef typename RealOf<VB>::type real_t;
@@ -263,8 +284,10 @@ constexpr int kRowStartsBlock = 256;
 __global__ __launch_bounds__(kRowStartsBlock) void partition_row_starts_kernel(const uint32_t* __restrict__ row_ptr,
                                                                                uint32_t m, uint32_t base, uint32_t nnz,
                                                                                uint32_t tile_size, uint32_t tiles,
-                                                                               uint32_t* __restrict__ tile_rows) {
+                                                                               uint32_t* __restrict__ tile_rows,
+                                                                               uint32_t* __restrict__ wide) {
     const uint32_t t = blockIdx.x * (kRowStartsBlock / kWave) + threadIdx.x / kWave;
+    if (wide != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *wide = 0;
     if (t > tiles) return;  // whole wavefront
     const uint64_t first = static_cast<uint64_t>(t) * tile_size;
     // (m + 1 < 2^32: the reference's limit on extents)
@@ -373,6 +396,11 @@ struct SortTables {
     uint32_t* tile_first;    // tiles before each bucket of step 1, 2^d1 + 1 of them
     const uint32_t* first_runs;  // [bucket][first_stride]: the run of step 1 in which each of its tiles begins
     uint32_t first_stride;       // tiles of step 2 that one bucket can have
+    // step 1, packed entries: rows that begin at or before each tile's first entry, less one and the index base; whether
+    // there are tiles whose indices lie in an array of their own
+    const uint32_t* tile_rows;
+    const uint32_t* wide;
+    uint32_t tile1_shift, base;  // log2 of the places of a tile of step 1
     uint2* tile_map;         // the order in which the tiles are taken: {bucket << 24 | tile of the bucket, its first run}
     // both: entries before each bucket of step 3, 2^(d1 + d2) + 1 of them
     uint32_t* sub_first;
@@ -506,8 +534,9 @@ __global__ __launch_bounds__(kMapBlock) void tile_map_kernel(SortTables t) {
 }
 
 // 118 M entries (19 bytes each): 1.33 GB read, 1.14 GB written in 500 us.
+// Key: the type the rest of a key travels in from here on, or the packed entries' word on both sides.
 template <int VB, typename Key>
-__global__ __launch_bounds__(kSecondThreads) void repartition_kernel(SortTables t, const uint16_t* __restrict__ keys_in,
+__global__ __launch_bounds__(kSecondThreads) void repartition_kernel(SortTables t, const void* __restrict__ keys_in,
                                                                      const uint32_t* __restrict__ aux_in,
                                                                      const void* __restrict__ vals_in,
                                                                      Key* __restrict__ keys_out,
@@ -536,13 +565,38 @@ __global__ __launch_bounds__(kSecondThreads) void repartition_kernel(SortTables 
     uint32_t key[kSecondItems], aux[kSecondItems];
     word_t val[VB ? kSecondItems : 1];
     const uint32_t last_word = (count - 1) / kWave;
+    constexpr bool kPacked = packed_entries<Key>();
+    const uint32_t rest_bits = t.d2 + t.d3;
+    // (past the last entry: some entry of the last runs, which is not used)
+    auto place_of = [&](int i) { return mapped_place(s_map, s_buf, min(wave * kSecondItems + i, last_word), count); };
 #pragma unroll
     for (int i = 0; i < kSecondItems; ++i) {
-        // (past the last entry: some entry of the last runs, which is not used)
-        const uint32_t from = mapped_place(s_map, s_buf, min(wave * kSecondItems + i, last_word), count);
-        key[i] = load_at<uint16_t>(keys_in, from);
-        aux[i] = load_at<uint32_t>(aux_in, from);
-        if constexpr (VB != 0) val[i] = load_at<word_t>(vals_in, from);
+        const uint32_t from = place_of(i);
+        if constexpr (kPacked) {
+            load_packed<VB>(keys_in, vals_in, from, key[i], val[VB ? i : 0]);
+            aux[i] = load_at<uint32_t>(t.tile_rows, from >> t.tile1_shift);  // the row the word counts from, plus one
+        } else {
+            key[i] = load_at<uint16_t>(keys_in, from);
+            aux[i] = load_at<uint32_t>(aux_in, from);
+            if constexpr (VB != 0) val[i] = load_at<word_t>(vals_in, from);
+        }
+    }
+    if constexpr (kPacked) {
+        if (*t.wide != 0) {  // the same for all workgroups
+#pragma unroll 1
+            for (int i0 = 0; i0 < kSecondItems; ++i0) {
+                const uint32_t from = place_of(i0), tile1 = from >> t.tile1_shift;
+                uint32_t row = aux_in[from] - t.base + 1;
+                const bool apart = (t.tile_rows[tile1 + 1] - t.tile_rows[tile1]) >> (32 - rest_bits) != 0;
+#pragma unroll
+                for (int i = 0; i < kSecondItems; ++i) {
+                    if (i == i0 && apart) {
+                        aux[i] = row;
+                        key[i] &= (1u << rest_bits) - 1u;
+                    }
+                }
+            }
+        }
     }
     const uint32_t mask = (1u << t.d2) - 1u;
     auto digit = [&](int i) { return (key[i] >> t.d3) & mask; };
@@ -558,6 +612,15 @@ __global__ __launch_bounds__(kSecondThreads) void repartition_kernel(SortTables 
     for (int i = 0; i < kSecondItems; ++i)
         dest[i / 2] += static_cast<uint32_t>(s_cnt[(wave << kMaxBits) + digit(i)]) << (i % 2 * 16);
     const uint64_t out = static_cast<uint64_t>(first_tile + tile) * kSecondTile;
+    if constexpr (kPacked) {
+        // what is left of the key, and the row with its index base
+        auto word_of = [&](int i) {
+            const uint32_t row = aux[i] + (key[i] >> rest_bits) - 1 + t.base;
+            return (key[i] & ((1u << t.d3) - 1u)) | row << t.d3;
+        };
+        store_packed<VB, kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, keys_out, vals_out, out, word_of, val);
+        return;
+    }
     store_keys<kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, keys_out + out, key, (1u << t.d3) - 1u);
     store_words<kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, aux_out + out, aux);
     if constexpr (VB != 0)
@@ -680,15 +743,21 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
     typedef typename WordOf<VB>::type word_t;
     static_assert(!MANY || VB != 8, "64-bit values are sorted in one pass");
     const uint32_t tid = threadIdx.x, wave = tid / kWave;
-    uint32_t key[ITEMS], aux[ITEMS];
+    constexpr bool kPacked = packed_entries<Key>();  // (aux is then the whole word: the key's rest below the index)
+    static_assert(!MANY || !kPacked, "sorts by one key");
+    uint32_t key[kPacked ? 1 : ITEMS], aux[ITEMS];
     word_t val[VB ? ITEMS : 1];
     const uint32_t last_word = (count - 1) / kWave;
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
         const uint32_t from = mapped_place(s.map, s.buf, min(wave * ITEMS + i, last_word), count);
-        key[i] = load_at<Key>(keys_in, from);
-        aux[i] = load_at<uint32_t>(aux_in, from);
-        if constexpr (VB != 0) val[i] = load_at<word_t>(vals_in, from);
+        if constexpr (kPacked) {
+            load_packed<VB>(keys_in, vals_in, from, aux[i], val[VB ? i : 0]);
+        } else {
+            key[i] = load_at<Key>(keys_in, from);
+            aux[i] = load_at<uint32_t>(aux_in, from);
+            if constexpr (VB != 0) val[i] = load_at<word_t>(vals_in, from);
+        }
     }
     uint32_t dest[(ITEMS + 1) / 2];
     // into LDS in the new order
@@ -706,7 +775,9 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
         bool long_run = false;
         const uint32_t mask = (1u << pass.bits) - 1u;
         auto digit = [&](int i) {
-            const uint32_t of_aux = aux[i], of_key = key[i];  // (the values, so that neither array needs an address)
+            const uint32_t of_aux = aux[i];  // (the values, so that neither array needs an address)
+            if constexpr (kPacked) return of_aux & mask;
+            const uint32_t of_key = key[kPacked ? 0 : i];
             return MANY ? ((pass.on_aux ? of_aux : of_key) >> pass.shift) & mask : of_key;
         };
         rank_entries<ITEMS, kPassBits>(count, pass.bits, s.cnt, dest, digit);
@@ -768,7 +839,7 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
         }
         __syncthreads();
     };
-    ordered([&](int i) { return aux[i]; });
+    ordered([&](int i) { return kPacked ? aux[i] >> t.d3 : aux[i]; });
     stream_out([&](int, uint32_t p, uint32_t w) { out.aux[first + p] = w; });
     if constexpr (VB == 4) {
         ordered([&](int i) { return val[i]; });
@@ -782,7 +853,7 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
             static_cast<uint64_t*>(out.vals)[first + p] = static_cast<uint64_t>(w) << 32 | low[i];
         });
     }
-    if (out.keys != nullptr) {
+    if constexpr (MANY) {
         const uint32_t high = (sub << t.d3) + out.key_bias;
         ordered([&](int i) { return key[i]; });
         stream_out([&](int, uint32_t p, uint32_t w) { out.keys[first + p] = high + w; });
@@ -983,7 +1054,8 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 ? 2 : 4) void oversize_kern
                 for (int i = 0; i < kBucketItems; ++i) {
                     const uint32_t from = place_of(i);
                     key[i] = 0;
-                    if (by_key) key[i] = p == 0 ? load_at<Key>(keys_in, from) : load_shared_at<uint16_t>(between_keys, from);
+                    if constexpr (packed_entries<Key>()) key[i] = load_at<uint32_t>(keys_in, VB == 4 ? 2 * from : from);
+                    else if (by_key) key[i] = p == 0 ? load_at<Key>(keys_in, from) : load_shared_at<uint16_t>(between_keys, from);
                     if constexpr (MANY) {
                         aux[i] = 0;
                         if (by_aux) aux[i] = p == 0 ? load_at<uint32_t>(aux_in, from) : load_shared_at<uint32_t>(between_aux, from);
@@ -1027,7 +1099,10 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 ? 2 : 4) void oversize_kern
 #pragma unroll
                 for (int i = 0; i < kBucketItems; ++i) {
                     const uint32_t from = place_of(i);
-                    if (!MANY || p == 0) {
+                    if constexpr (packed_entries<Key>()) {
+                        load_packed<VB>(keys_in, vals_in, from, key[i], val[VB ? i : 0]);
+                        aux[i] = key[i] >> t.d3;
+                    } else if (!MANY || p == 0) {
                         key[i] = load_at<Key>(keys_in, from);
                         aux[i] = load_at<uint32_t>(aux_in, from);
                         if constexpr (VB != 0) val[i] = load_at<word_t>(vals_in, from);
@@ -1133,11 +1208,11 @@ void launch_partition(hipStream_t stream, const EntrySource& in, uint32_t shift,
     }
 }
 
-void launch_row_starts(hipStream_t stream, const EntrySource& in, uint32_t tile_size, uint32_t* tile_rows) {
+void launch_row_starts(hipStream_t stream, const EntrySource& in, uint32_t tile_size, uint32_t* tile_rows, uint32_t* wide) {
     const uint32_t tiles = tiles_of(in.count, tile_size);
     constexpr uint32_t kPerBlock = kRowStartsBlock / kWave;
     hipLaunchKernelGGL(partition_row_starts_kernel, dim3(tiles / kPerBlock + 1), dim3(kRowStartsBlock), 0, stream, in.aux,
-                       in.m, in.base, in.count, tile_size, tiles, tile_rows);
+                       in.m, in.base, in.count, tile_size, tiles, tile_rows, wide);
 }
 
 struct BucketedLayout {
@@ -1173,6 +1248,7 @@ constexpr uint32_t kMostEntries = kBucketRoom * 3 / 4 << kMaxTwoLevelBits;  // m
 struct SortShape {
     uint32_t d1, d2, d3, tile_size, tiles1, max_tiles2;
     uint32_t minor_bits;  // kNoMinorKey: a sort by one key
+    bool packed = false;  // what is left of a key and the index share a word (csr2csc)
 };
 constexpr uint32_t kNoMinorKey = ~0u;
 constexpr uint32_t kMaxKeyRest = 16;  // bits of a key behind those of step 1: it travels in 16
@@ -1217,6 +1293,11 @@ bool sort_shape(uint32_t count, uint32_t key_count, uint32_t minor_bits, SortSha
     s->max_tiles2 = s->d2 != 0 ? count / kSecondTile + (1u << s->d1) : 0;
     return true;
 }
+// csr2csc: an entry's row and what is left of its column share a word where both have room in it behind the last partition.
+// (Behind the first of two the row is counted from the tile's first, with the 16 bits or more that the key leaves it.)
+// 118 M entries, 4 M columns: 18 + 19 + 17 bytes moved per entry and step become 16 each, and a run of a bucket lies in one
+// array instead of three.
+bool sort_packs(const SortShape& s, uint32_t rows) { return s.minor_bits == kNoMinorKey && bit_length(rows) + s.d3 <= 32; }
 // Bytes a key travels in behind step 1 (step 2 reads 16 bits) and behind step 2.
 size_t first_key_bytes(const SortShape& s) { return s.d2 == 0 && s.d3 <= 8 ? sizeof(uint8_t) : sizeof(uint16_t); }
 size_t second_key_bytes(const SortShape& s) { return s.d3 <= 8 ? sizeof(uint8_t) : sizeof(uint16_t); }
@@ -1239,7 +1320,7 @@ void sort_passes(const SortShape& s, SortTables* t) {
 uint32_t second_tiles_most(uint32_t count) { return (count - 1) / kSecondTile + 1; }
 
 struct SortLayout {
-    size_t keys1, aux1, vals1, keys2, aux2, vals2, table1, begins1, totals1, tile_rows, table2, begins2, bucket_first,
+    size_t keys1, aux1, vals1, keys2, aux2, vals2, wide, table1, begins1, totals1, tile_rows, table2, begins2, bucket_first,
         tile_first, first_runs, tile_map, sub_first, sub_arrived, oversize, oversize_bucket, oversize_first, oversize_counted, oversize_arrived,
         oversize_counts, oversize_begins, oversize_keys[2], oversize_aux[2], oversize_vals[2], total;
 };
@@ -1258,12 +1339,24 @@ SortLayout sort_layout(uint32_t count, const SortShape& s, size_t value_bytes) {
         off += align_up(bytes);
         return at;
     };
-    l.keys1 = take(places1 * first_key_bytes(s));
-    l.aux1 = take(places1 * sizeof(uint32_t));
-    l.vals1 = take(places1 * value_bytes);
-    l.keys2 = take(places2 * second_key_bytes(s));
-    l.aux2 = take(places2 * sizeof(uint32_t));
-    l.vals2 = take(places2 * value_bytes);
+    if (s.packed) {  // words, or {word, value} pairs
+        const bool pairs = value_bytes == sizeof(uint32_t);
+        const size_t entry = pairs ? sizeof(uint64_t) : sizeof(uint32_t), apart = pairs ? 0 : value_bytes;
+        l.keys1 = take(places1 * entry);
+        l.aux1 = take(s.d2 != 0 ? places1 * sizeof(uint32_t) : 0);
+        l.vals1 = take(places1 * apart);
+        l.keys2 = take(places2 * entry);
+        l.aux2 = off;
+        l.vals2 = take(places2 * apart);
+    } else {
+        l.keys1 = take(places1 * first_key_bytes(s));
+        l.aux1 = take(places1 * sizeof(uint32_t));
+        l.vals1 = take(places1 * value_bytes);
+        l.keys2 = take(places2 * second_key_bytes(s));
+        l.aux2 = take(places2 * sizeof(uint32_t));
+        l.vals2 = take(places2 * value_bytes);
+    }
+    l.wide = take(sizeof(uint32_t));
     l.table1 = take(runs1 * sizeof(uint32_t));
     l.begins1 = take(runs1 * sizeof(uint32_t));
     l.totals1 = take(sizeof(uint32_t) << s.d1);
@@ -1301,10 +1394,16 @@ void launch_sort(hipStream_t stream, EntrySource in, const SortShape& s, const S
     auto words = [&](size_t at) { return reinterpret_cast<uint32_t*>(w + at); };
     const uint32_t xcds = device_topology().xcds;
     if constexpr (KIND == kCsr) {
-        launch_row_starts(stream, in, s.tile_size, words(l.tile_rows));
+        in.wide = words(l.wide);
+        in.relative = s.packed && s.d2 != 0;
+        launch_row_starts(stream, in, s.tile_size, words(l.tile_rows), in.wide);
         in.tile_rows = words(l.tile_rows);
     }
     SortTables t;
+    t.tile_rows = words(l.tile_rows);
+    t.wide = words(l.wide);
+    t.tile1_shift = bit_length(s.tile_size) - 1;
+    t.base = in.base;
     t.table1 = words(l.table1);
     t.begins1 = words(l.begins1);
     t.totals1 = words(l.totals1);
@@ -1342,23 +1441,34 @@ void launch_sort(hipStream_t stream, EntrySource in, const SortShape& s, const S
     auto* partition = s.d1 <= 8 ? (short_keys1 ? launch_partition<VB, KIND, 8, uint8_t> : launch_partition<VB, KIND, 8, uint16_t>)
                                 : (short_keys1 ? launch_partition<VB, KIND, kMaxOneLevelBits, uint8_t>
                                                : launch_partition<VB, KIND, kMaxOneLevelBits, uint16_t>);
+    if constexpr (KIND == kCsr) {
+        if (s.packed)
+            partition = s.d1 <= 8 ? launch_partition<VB, KIND, 8, uint32_t> : launch_partition<VB, KIND, kMaxOneLevelBits, uint32_t>;
+    }
     partition(stream, in, shift, s.d1, s.tile_size, w + l.keys1, words(l.aux1), w + l.vals1, words(l.table1));
     hipLaunchKernelGGL(run_begins_kernel, dim3(1u << s.d1), dim3(kScanBlock), 0, stream, s.tiles1, t.table1,
                        words(l.begins1), words(l.totals1), s.d2 != 0 ? words(l.first_runs) : nullptr, t.first_stride);
     hipLaunchKernelGGL(sort_plan_kernel, dim3(1), dim3(kPlanBlock), 0, stream, t);
+    // what a key travels in behind step 2
+    auto with_key = [&](auto launch) {
+        if constexpr (KIND == kCsr) {
+            if (s.packed) return launch(uint32_t());
+        }
+        if (short_keys2) return launch(uint8_t());
+        if constexpr (kMany) launch(uint16_t());
+    };
     const void* keys = w + l.keys1;
     const uint32_t* aux = words(l.aux1);
     const void* vals = w + l.vals1;
     if (s.d2 != 0) {
         hipLaunchKernelGGL(tile_map_kernel, dim3((s.max_tiles2 + kMapBlock - 1) / kMapBlock), dim3(kMapBlock), 0, stream, t);
         const dim3 grid((s.max_tiles2 + xcds - 1) / xcds * xcds);
-        const uint16_t* keys1 = reinterpret_cast<const uint16_t*>(keys);
-        if (short_keys2)
-            hipLaunchKernelGGL((repartition_kernel<VB, uint8_t>), grid, dim3(kSecondThreads), 0, stream, t, keys1, aux, vals,
-                               reinterpret_cast<uint8_t*>(w + l.keys2), words(l.aux2), w + l.vals2, s.max_tiles2, xcds);
-        else if constexpr (kMany)
-            hipLaunchKernelGGL((repartition_kernel<VB, uint16_t>), grid, dim3(kSecondThreads), 0, stream, t, keys1, aux, vals,
-                               reinterpret_cast<uint16_t*>(w + l.keys2), words(l.aux2), w + l.vals2, s.max_tiles2, xcds);
+        auto repartition = [&](auto key) {
+            typedef decltype(key) Key;
+            hipLaunchKernelGGL((repartition_kernel<VB, Key>), grid, dim3(kSecondThreads), 0, stream, t, keys, aux, vals,
+                               reinterpret_cast<Key*>(w + l.keys2), words(l.aux2), w + l.vals2, s.max_tiles2, xcds);
+        };
+        with_key(repartition);
         hipLaunchKernelGGL(sub_begins_kernel, dim3(kSubParts << s.d1), dim3(kSubBlock), 0, stream, t);
         keys = w + l.keys2;
         aux = words(l.aux2);
@@ -1374,8 +1484,7 @@ void launch_sort(hipStream_t stream, EntrySource in, const SortShape& s, const S
             hipLaunchKernelGGL((oversize_kernel<VB, Key, kMany>), dim3(kOversizeGrid), dim3(kBucketThreads), 0, stream, t,
                                static_cast<const Key*>(keys), aux, vals, out);
     };
-    if (short_keys2) sort(uint8_t());
-    else if constexpr (kMany) sort(uint16_t());
+    with_key(sort);
 }
 
 }  // namespace
@@ -1386,7 +1495,10 @@ bool partition_sort_usable(idx_t count, idx_t key_count) {
 }
 size_t partition_sort_workspace_bytes(idx_t count, idx_t key_count, size_t value_bytes) {
     SortShape s;
-    return sort_shape(count, key_count, kNoMinorKey, &s) ? sort_layout(count, s, value_bytes).total : 0;
+    if (!sort_shape(count, key_count, kNoMinorKey, &s)) return 0;
+    const size_t apart = sort_layout(count, s, value_bytes).total;  // (the rows are not known here)
+    s.packed = true;
+    return std::max(apart, sort_layout(count, s, value_bytes).total);
 }
 bool partition_sort_pairs_usable(idx_t count, idx_t major_count, idx_t minor_count) {
     SortShape s;
@@ -1400,6 +1512,7 @@ size_t partition_sort_pairs_workspace_bytes(idx_t count, idx_t major_count, idx_
 void launch_partition_sort(hipStream_t stream, idx_t count, const PartitionSortArgs& a, size_t value_bytes, void* workspace) {
     SortShape s;
     if (!sort_shape(count, a.key_count, kNoMinorKey, &s)) return;
+    s.packed = sort_packs(s, a.csr_rows);
     EntrySource in;
     in.keys = a.keys_in;
     in.aux = a.row_ptr;
@@ -1470,7 +1583,7 @@ void launch_bucketed_products(hipStream_t stream, idx_t m, idx_t n, idx_t nnz, c
     in.tile_rows = reinterpret_cast<uint32_t*>(w + l.tile_rows);
     const uint32_t tile_size = tile_size_for(nnz);
     uint32_t* table = reinterpret_cast<uint32_t*>(w + l.table);
-    launch_row_starts(stream, in, tile_size, reinterpret_cast<uint32_t*>(w + l.tile_rows));
+    launch_row_starts(stream, in, tile_size, reinterpret_cast<uint32_t*>(w + l.tile_rows), nullptr);
     auto* launch = value_bytes == 4 ? launch_partition<4, kProducts, 8, uint16_t> : launch_partition<8, kProducts, 8, uint16_t>;
     launch(stream, in, shift, 8, tile_size, w + l.keys, nullptr, w + l.products, table);
     out->keys = reinterpret_cast<const uint16_t*>(w + l.keys);

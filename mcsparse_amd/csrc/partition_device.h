@@ -333,10 +333,10 @@ __device__ __forceinline__ void store_words(uint32_t* s_buf, uint32_t count, con
     __syncthreads();
 }
 
-// 64-bit values go through the buffer in two halves.
-template <int ITEMS, int THREADS, uint32_t PLACES>
-__device__ __forceinline__ void store_words(uint32_t* s_buf, uint32_t count, const uint32_t (&dest)[(ITEMS + 1) / 2],
-                                            uint64_t* out, const uint64_t (&word)[ITEMS]) {
+// 64-bit words, word_of(half, i) being the lower and the upper half of entry i's, go through the buffer in two halves.
+template <int ITEMS, int THREADS, uint32_t PLACES, typename WordOfHalf>
+__device__ __forceinline__ void store_halves(uint32_t* s_buf, uint32_t count, const uint32_t (&dest)[(ITEMS + 1) / 2],
+                                             uint64_t* out, WordOfHalf word_of) {
     constexpr uint32_t kPieces = PLACES / 4;
     constexpr uint32_t kMine = (kPieces + THREADS - 1) / THREADS;
     u32x4 low[kMine];
@@ -344,8 +344,7 @@ __device__ __forceinline__ void store_words(uint32_t* s_buf, uint32_t count, con
     for (int half = 0; half < 2; ++half) {
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
-            if (in_slab(ITEMS, i, count))
-                s_buf[(dest[i / 2] >> (i % 2 * 16)) & 0xffffu] = static_cast<uint32_t>(word[i] >> (32 * half));
+            if (in_slab(ITEMS, i, count)) s_buf[(dest[i / 2] >> (i % 2 * 16)) & 0xffffu] = word_of(half, i);
         }
         __syncthreads();
 #pragma unroll
@@ -362,6 +361,44 @@ __device__ __forceinline__ void store_words(uint32_t* s_buf, uint32_t count, con
             }
         }
         __syncthreads();
+    }
+}
+template <int ITEMS, int THREADS, uint32_t PLACES>
+__device__ __forceinline__ void store_words(uint32_t* s_buf, uint32_t count, const uint32_t (&dest)[(ITEMS + 1) / 2],
+                                            uint64_t* out, const uint64_t (&word)[ITEMS]) {
+    store_halves<ITEMS, THREADS, PLACES>(s_buf, count, dest, out,
+                                         [&](int half, int i) { return static_cast<uint32_t>(word[i] >> (32 * half)); });
+}
+
+// ---- packed entries --------------------------------------------------------------------------------------------
+// Where what is left of an entry's key and its index share a word (Key = uint32_t), the entries are an array of such words
+// and one of values, or, with 32-bit values, one of {word, value} pairs.
+template <typename Key>
+constexpr bool packed_entries() { return sizeof(Key) == 4; }
+template <int VB>
+__device__ __forceinline__ void load_packed(const void* words, const void* vals, uint32_t at, uint32_t& word,
+                                            typename WordOf<VB>::type& val) {
+    if constexpr (VB == 4) {
+        const uint64_t pair = load_at<uint64_t>(words, at);
+        word = static_cast<uint32_t>(pair);
+        val = static_cast<uint32_t>(pair >> 32);
+    } else {
+        word = load_at<uint32_t>(words, at);
+        if constexpr (VB != 0) val = load_at<uint64_t>(vals, at);
+    }
+}
+template <int VB, int ITEMS, int THREADS, uint32_t PLACES, typename WordOfEntry, typename Values>
+__device__ __forceinline__ void store_packed(uint32_t* s_buf, uint32_t count, const uint32_t (&dest)[(ITEMS + 1) / 2],
+                                             void* words, void* vals, uint64_t out, WordOfEntry word_of, const Values& val) {
+    if constexpr (VB == 4) {
+        store_halves<ITEMS, THREADS, PLACES>(s_buf, count, dest, static_cast<uint64_t*>(words) + out,
+                                             [&](int half, int i) { return half == 0 ? word_of(i) : val[i]; });
+    } else {
+        uint32_t word[ITEMS];
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) word[i] = word_of(i);
+        store_words<ITEMS, THREADS, PLACES>(s_buf, count, dest, static_cast<uint32_t*>(words) + out, word);
+        if constexpr (VB != 0) store_words<ITEMS, THREADS, PLACES>(s_buf, count, dest, static_cast<uint64_t*>(vals) + out, val);
     }
 }
 

@@ -87,6 +87,42 @@ def test_csr2csc_bit_exact(torch_gpu, handle, oracle, dtype, action, kind, m, n,
         assert (o_val == -9.0).all()
 
 
+@pytest.mark.parametrize("dtype,action", [(np.float32, api.ACTION_NUMERIC), (np.float64, api.ACTION_NUMERIC),
+                                          (np.float32, api.ACTION_SYMBOLIC)])
+@pytest.mark.parametrize("m,n,gap,base", [
+    # a row every `gap` rows: with 2^22 columns the word behind the first partition has room for 2^17 rows of a tile
+    ((1 << 24) - 1, 1 << 22, 131071, 0), ((1 << 24) - 1, 1 << 22, 131072, 1), ((1 << 24) - 1, 1 << 22, 1 << 20, 1),
+    # one row more than a word holds beside eight bits of the column: rows and keys apart
+    (1 << 24, 1 << 22, 131072, 1),
+    # with 2^16 columns the room behind the first partition is 2^22 rows
+    ((1 << 24) - 1, 1 << 16, (1 << 22) - 1, 0), ((1 << 24) - 1, 1 << 16, 1 << 22, 0),
+])
+def test_csr2csc_tiles_of_many_rows(torch_gpu, handle, oracle, dtype, action, m, n, gap, base):
+    torch = torch_gpu
+    nnz = ONE_LEVEL_UPTO + 12345
+    full = np.arange(0, m, gap)
+    rng = np.random.default_rng(gap)
+    lengths = np.zeros(m, dtype=np.int64)
+    lengths[full] = nnz // full.size
+    lengths[full[-1]] += nnz - lengths.sum()
+    ptr = np.concatenate([[0], np.cumsum(lengths)])
+    a = wl.Csr(m, n, ptr, rng.integers(0, n, nnz), rng.integers(-3, 4, nnz).astype(dtype), 0).with_base(base)
+    d_ptr, d_col, d_val = dev(torch, a.ptr), dev(torch, a.col), dev(torch, a.val)
+    o_val = torch.full((nnz,), -9.0, dtype=d_val.dtype, device="cuda")
+    o_ptr, o_row = (torch.full((k,), -9, dtype=torch.int32, device="cuda") for k in (n + 1, nnz))
+    args = (handle, m, n, nnz, d_val, d_ptr, d_col, o_val, o_ptr, o_row, api.maca_type(np.dtype(dtype)), action, base)
+    st, size = api.csr2csc_buffer_size(*args)
+    assert st == api.STATUS_SUCCESS
+    buf = torch.empty(size, dtype=torch.uint8, device="cuda")
+    want_ptr, want_row, want_val = oracle.csr2csc(m, n, base, a.ptr, a.col, a.val, method="counting")
+    assert api.csr2csc(*args, buf) == api.STATUS_SUCCESS
+    torch.cuda.synchronize()
+    assert np.array_equal(o_ptr.cpu().numpy().view(np.uint32), want_ptr)
+    assert np.array_equal(o_row.cpu().numpy().view(np.uint32), want_row)
+    if action == api.ACTION_NUMERIC:
+        assert np.array_equal(o_val.cpu().numpy(), want_val)
+
+
 @pytest.mark.parametrize("by", ["row", "column"])
 @pytest.mark.parametrize("with_perm", [True, False])
 @pytest.mark.parametrize("kind,m,n,nnz", [
