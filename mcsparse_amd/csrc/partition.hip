@@ -114,7 +114,7 @@ __device__ __forceinline__ void count_rows(TileRows<TILE>& s) {
 // Bounds at 118 M entries (the products of a transposing SpMV, fp32): 0.98 GB read and 0.79 GB written in 340 us, nine
 // tenths of the rate of a copy; tiles of 4096 or 16 wavefronts per workgroup are no faster (342 and 420 us).  The pass
 // it replaces took 486 us, with a pass over the keys (111 us) in front of it to count them.  The first step of csr2csc
-// (18 bytes per entry, the ranks by ballots): 2.16 GB in 380 us.
+// (16 bytes per entry, the ranks by ballots): 1.9 GB in 350 us.
 template <int VB, int KIND, int MAX_BITS, typename Key, int THREADS, int ITEMS>
 __global__ __launch_bounds__(THREADS) void partition_kernel(EntrySource in, uint32_t shift, uint32_t bits, uint32_t tiles,
                                                                Key* __restrict__ keys_out, uint32_t* __restrict__ aux_out,
@@ -248,7 +248,10 @@ __global__ __launch_bounds__(THREADS) void partition_kernel(EntrySource in, uint
             }
         }
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) key[i] = (key[i] & ((1u << shift) - 1u)) | (aux[i] - origin) << shift;
+        for (int i = 0; i < ITEMS; ++i) {
+            key[i] = (key[i] & ((1u << shift) - 1u)) | (aux[i] - origin) << shift;
+            forget(key[i]);
+        }
         store_packed<VB, ITEMS, THREADS, kPlaces>(s_buf, count, dest, keys_out, vals_out, out, [&](int i) { return key[i]; }, val);
         return;
     }
@@ -533,7 +536,7 @@ __global__ __launch_bounds__(kMapBlock) void tile_map_kernel(SortTables t) {
     t.tile_map[at] = make_uint2(lo << 24 | tile, t.first_runs[static_cast<uint64_t>(lo) * t.first_stride + tile]);
 }
 
-// 118 M entries (19 bytes each): 1.33 GB read, 1.14 GB written in 500 us.
+// 118 M entries (16 bytes each): 0.99 GB read, 1.10 GB written in 415 us.
 // Key: the type the rest of a key travels in from here on, or the packed entries' word on both sides.
 template <int VB, typename Key>
 __global__ __launch_bounds__(kSecondThreads) void repartition_kernel(SortTables t, const void* __restrict__ keys_in,
@@ -562,44 +565,58 @@ __global__ __launch_bounds__(kSecondThreads) void repartition_kernel(SortTables 
     const uint64_t row = static_cast<uint64_t>(bucket) * t.tiles1;
     map_runs<kSecondThreads, kSecondTile>(t.begins1 + row, t.table1 + row, t.tiles1, all, q0, count, mine.y, t.places1, 0, s_map,
                                           s_buf);
-    uint32_t key[kSecondItems], aux[kSecondItems];
+    constexpr bool kPacked = packed_entries<Key>();
+    uint32_t key[kPacked ? 1 : kSecondItems], aux[kSecondItems];  // packed: aux is the word that goes on from here,
+    uint32_t digits[kPacked ? (kSecondItems + 3) / 4 : 1];        // digits the bits of it this step sorts by
     word_t val[VB ? kSecondItems : 1];
     const uint32_t last_word = (count - 1) / kWave;
-    constexpr bool kPacked = packed_entries<Key>();
-    const uint32_t rest_bits = t.d2 + t.d3;
     // (past the last entry: some entry of the last runs, which is not used)
-    auto place_of = [&](int i) { return mapped_place(s_map, s_buf, min(wave * kSecondItems + i, last_word), count); };
+    uint32_t own_wave = wave;
+    auto place_of = [&](int i) { return mapped_place(s_map, s_buf, min(own_wave * kSecondItems + i, last_word), count); };
+    const uint32_t mask = (1u << t.d2) - 1u;
+    if constexpr (kPacked) {
+        const uint32_t rest_bits = t.d2 + t.d3, low_mask = (1u << t.d3) - 1u;
+        uint32_t first_row[kSecondItems];
 #pragma unroll
-    for (int i = 0; i < kSecondItems; ++i) {
-        const uint32_t from = place_of(i);
-        if constexpr (kPacked) {
-            load_packed<VB>(keys_in, vals_in, from, key[i], val[VB ? i : 0]);
-            aux[i] = load_at<uint32_t>(t.tile_rows, from >> t.tile1_shift);  // the row the word counts from, plus one
-        } else {
+        for (int i = 0; i < kSecondItems; ++i) {
+            const uint32_t from = place_of(i);
+            load_packed<VB>(keys_in, vals_in, from, aux[i], val[VB ? i : 0]);
+            first_row[i] = load_at<uint32_t>(t.tile_rows, from >> t.tile1_shift);  // the row the word counts from, plus one
+            if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // (places of so many at a time are held in registers)
+        }
+        if (*t.wide != 0) {  // the same for all workgroups
+            forget(own_wave);  // (places found again and not held in registers)
+#pragma unroll
+            for (int i = 0; i < kSecondItems; ++i) {
+                const uint32_t from = place_of(i), tile1 = from >> t.tile1_shift;
+                if ((t.tile_rows[tile1 + 1] - t.tile_rows[tile1]) >> (32 - rest_bits) != 0) {
+                    first_row[i] = aux_in[from] - t.base + 1;
+                    aux[i] &= (1u << rest_bits) - 1u;
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < kSecondItems; ++i) {
+            const uint32_t word = aux[i], d = ((word >> t.d3) & mask) << (i % 4 * 8);
+            if (i % 4 == 0) digits[i / 4] = d;
+            else digits[i / 4] |= d;
+            aux[i] = ((word >> rest_bits) + first_row[i] - 1 + t.base) << t.d3 | (word & low_mask);
+            forget(aux[i]);
+            if (i % 4 == 3) forget(digits[i / 4]);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < kSecondItems; ++i) {
+            const uint32_t from = place_of(i);
             key[i] = load_at<uint16_t>(keys_in, from);
             aux[i] = load_at<uint32_t>(aux_in, from);
             if constexpr (VB != 0) val[i] = load_at<word_t>(vals_in, from);
         }
     }
-    if constexpr (kPacked) {
-        if (*t.wide != 0) {  // the same for all workgroups
-#pragma unroll 1
-            for (int i0 = 0; i0 < kSecondItems; ++i0) {
-                const uint32_t from = place_of(i0), tile1 = from >> t.tile1_shift;
-                uint32_t row = aux_in[from] - t.base + 1;
-                const bool apart = (t.tile_rows[tile1 + 1] - t.tile_rows[tile1]) >> (32 - rest_bits) != 0;
-#pragma unroll
-                for (int i = 0; i < kSecondItems; ++i) {
-                    if (i == i0 && apart) {
-                        aux[i] = row;
-                        key[i] &= (1u << rest_bits) - 1u;
-                    }
-                }
-            }
-        }
-    }
-    const uint32_t mask = (1u << t.d2) - 1u;
-    auto digit = [&](int i) { return (key[i] >> t.d3) & mask; };
+    auto digit = [&](int i) {
+        if constexpr (kPacked) return (digits[i / 4] >> (i % 4 * 8)) & 0xffu;
+        else return (key[kPacked ? 0 : i] >> t.d3) & mask;
+    };
     uint32_t dest[kSecondItems / 2];
     rank_entries<kSecondItems, kMaxBits>(count, t.d2, s_cnt, dest, digit);
     __syncthreads();
@@ -613,18 +630,14 @@ __global__ __launch_bounds__(kSecondThreads) void repartition_kernel(SortTables 
         dest[i / 2] += static_cast<uint32_t>(s_cnt[(wave << kMaxBits) + digit(i)]) << (i % 2 * 16);
     const uint64_t out = static_cast<uint64_t>(first_tile + tile) * kSecondTile;
     if constexpr (kPacked) {
-        // what is left of the key, and the row with its index base
-        auto word_of = [&](int i) {
-            const uint32_t row = aux[i] + (key[i] >> rest_bits) - 1 + t.base;
-            return (key[i] & ((1u << t.d3) - 1u)) | row << t.d3;
-        };
-        store_packed<VB, kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, keys_out, vals_out, out, word_of, val);
-        return;
+        store_packed<VB, kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, keys_out, vals_out, out,
+                                                                    [&](int i) { return aux[i]; }, val);
+    } else {
+        store_keys<kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, keys_out + out, key, (1u << t.d3) - 1u);
+        store_words<kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, aux_out + out, aux);
+        if constexpr (VB != 0)
+            store_words<kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, static_cast<word_t*>(vals_out) + out, val);
     }
-    store_keys<kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, keys_out + out, key, (1u << t.d3) - 1u);
-    store_words<kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, aux_out + out, aux);
-    if constexpr (VB != 0)
-        store_words<kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, static_cast<word_t*>(vals_out) + out, val);
 }
 
 // begins2 and sub_first from table2; kSubParts workgroups per bucket of step 1, a wavefront per digit at a time, and
@@ -860,9 +873,9 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
     }
 }
 
-// A workgroup per bucket.  118 M entries (17 bytes each) in buckets of 3600: 445 us, bound by vector instructions as much
-// as by memory (86 % of the cycles, 4.6 TB/s); so most buckets, below two thirds of the room, run a version without the
-// last third of the items (458 -> 445 us).
+// A workgroup per bucket.  118 M entries (16 bytes each) in buckets of 3600: 390 us, bound by vector instructions as much
+// as by memory; so most buckets, below two thirds of the room, run a version without the last third of the items (458 -> 445
+// us when an entry was 17 bytes in three arrays).
 template <int VB, typename Key, bool MANY>
 __global__ __launch_bounds__(kBucketThreads, VB == 8 || MANY ? 6 : 8) void bucket_sort_kernel(SortTables t, const Key* __restrict__ keys_in,
                                                                                       const uint32_t* __restrict__ aux_in,
@@ -1199,9 +1212,12 @@ void launch_partition(hipStream_t stream, const EntrySource& in, uint32_t shift,
     const uint32_t tiles = tiles_of(in.count, tile_size);
     const uint32_t xcds = device_topology().xcds;
     const dim3 grid((tiles + xcds - 1) / xcds * xcds);
+    // Packed entries: 16 wavefronts with half the items each need half the registers and fill a compute unit (118 M entries,
+    // csr2csc 1163 -> 1139 us); with the counters of 11 bits they would fill it with one workgroup (85.6 -> 89.6 us, 2 M).
+    constexpr int kThreads = packed_entries<Key>() && MAX_BITS <= 8 ? 1024 : 512;
     if (tile_size == kTileLarge) {
-        hipLaunchKernelGGL((partition_kernel<VB, KIND, MAX_BITS, Key, 512, 16>), grid, dim3(512), 0, stream, in, shift, bits,
-                           tiles, static_cast<Key*>(keys_out), aux_out, vals_out, table, xcds);
+        hipLaunchKernelGGL((partition_kernel<VB, KIND, MAX_BITS, Key, kThreads, kTileLarge / kThreads>), grid, dim3(kThreads), 0,
+                           stream, in, shift, bits, tiles, static_cast<Key*>(keys_out), aux_out, vals_out, table, xcds);
     } else {
         hipLaunchKernelGGL((partition_kernel<VB, KIND, MAX_BITS, Key, 512, 8>), grid, dim3(512), 0, stream, in, shift, bits,
                            tiles, static_cast<Key*>(keys_out), aux_out, vals_out, table, xcds);

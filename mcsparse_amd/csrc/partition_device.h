@@ -151,6 +151,7 @@ __device__ __forceinline__ void rank_entries(uint32_t count, uint32_t bits, uint
         }
         if (i % 2 == 0) rank[i / 2] = r;
         else rank[i / 2] |= r << 16;
+        if (i % 2 != 0) forget(rank[i / 2]);  // (else the halves stay apart, in a register each, until they are used)
     }
 }
 
@@ -333,13 +334,16 @@ __device__ __forceinline__ void store_words(uint32_t* s_buf, uint32_t count, con
     __syncthreads();
 }
 
-// 64-bit words, word_of(half, i) being the lower and the upper half of entry i's, go through the buffer in two halves.
+// 64-bit words, word_of(half, i) being the lower and the upper half of entry i's, go through the buffer in two halves.  A
+// thread has two words of a store to itself, so that a wavefront's store is one stretch (four, as two stores of 16 bytes a
+// 32-byte stride apart: twice the requests to L2).
 template <int ITEMS, int THREADS, uint32_t PLACES, typename WordOfHalf>
 __device__ __forceinline__ void store_halves(uint32_t* s_buf, uint32_t count, const uint32_t (&dest)[(ITEMS + 1) / 2],
                                              uint64_t* out, WordOfHalf word_of) {
-    constexpr uint32_t kPieces = PLACES / 4;
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    constexpr uint32_t kPieces = PLACES / 2;
     constexpr uint32_t kMine = (kPieces + THREADS - 1) / THREADS;
-    u32x4 low[kMine];
+    u32x2 low[kMine];
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
 #pragma unroll
@@ -351,13 +355,12 @@ __device__ __forceinline__ void store_halves(uint32_t* s_buf, uint32_t count, co
         for (uint32_t k = 0; k < kMine; ++k) {
             const uint32_t v = k * THREADS + threadIdx.x;
             if (kPieces % THREADS != 0 && v >= kPieces) continue;
-            const u32x4 got = reinterpret_cast<const u32x4*>(s_buf)[v];
+            const u32x2 got = reinterpret_cast<const u32x2*>(s_buf)[v];
             if (half == 0) {
                 low[k] = got;
             } else {
-                const u32x4 a = {low[k].x, got.x, low[k].y, got.y}, b = {low[k].z, got.z, low[k].w, got.w};
-                __builtin_nontemporal_store(a, reinterpret_cast<u32x4*>(out) + 2 * v);
-                __builtin_nontemporal_store(b, reinterpret_cast<u32x4*>(out) + 2 * v + 1);
+                const u32x4 piece = {low[k].x, got.x, low[k].y, got.y};
+                __builtin_nontemporal_store(piece, reinterpret_cast<u32x4*>(out) + v);
             }
         }
         __syncthreads();
