@@ -165,6 +165,13 @@ class SpMat:
                                                       ctypes.byref(rows)))
         return state.value, bands.value, rows.value
 
+    def spmv_diagonals(self):
+        """How many diagonals (counted once per 64 rows) the copy along them holds that mcsparseSpMV_preprocess left; 0 =
+        none in use."""
+        count = ctypes.c_int64()
+        check(self.lib.mcsparseSpMatGetSpMVDiagonals(self._d, ctypes.byref(count)))
+        return count.value
+
     def spmm_schedule(self):
         """(state, entries) left by mcsparseSpMM_preprocess; state 2 = merged column lists, 3 = diagonal blocks over
         groups of eight rows, 4 = diagonal blocks over groups of strips (all three in use), 1 = built and declined."""

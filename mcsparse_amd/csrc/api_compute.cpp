@@ -264,6 +264,15 @@ bool banded_candidate(const mcsparseSpMatDescr* A, mcsparseOperation_t op, mcspa
                               static_cast<idx_t>(A->idxBase), value_size(A->valueType), band_bytes, shape);
 }
 
+// What mcsparseSpMV_preprocess tries a copy along the diagonals for: a direction that does not transpose, unless the caller
+// has set the width of the bands or the kernel family, i.e. looks at one of them by itself.
+bool diagonals_candidate(const mcsparseSpMatDescr* A, mcsparseOperation_t op) {
+    if (!format_is_built(A->format) || (A->valueType != MACA_R_32F && A->valueType != MACA_R_64F)) return false;
+    const CsrView v = make_view(A, op);
+    return !v.transpose && A->banded.band_bytes == 0 && A->plan.forced_family == kFamilyAuto &&
+           mcsp::spmv_diagonals_shape(static_cast<idx_t>(v.m), static_cast<idx_t>(v.n), static_cast<idx_t>(A->nnz));
+}
+
 // Scratch of the preprocess call behind the banded copy of a transposing direction: the transpose in
 // CSR form and the workspace of the csr2csc that produces it.
 struct TransposeScratch {
@@ -289,7 +298,7 @@ bool banded_matches(const mcsparseSpMatDescr* A, const void* buffer, size_t valu
     const SpmvBanded& b = A->banded;
     // MCSPARSE_SPMV_CSR_ALG2 asks for the same bits on every run, which the copy in column order does not give
     if (b.shape.by_column && alg == MCSPARSE_SPMV_CSR_ALG2) return false;
-    return b.valid && b.useful && b.buffer == buffer && b.rows == A->rows && b.cols == A->cols && b.vals == A->vals &&
+    return b.valid && (b.useful || b.along_diagonals) && b.buffer == buffer && b.rows == A->rows && b.cols == A->cols && b.vals == A->vals &&
            b.m == A->row_num && b.n == A->col_num && b.nnz == A->nnz && b.base == static_cast<int>(A->idxBase) &&
            b.type == A->valueType && value_size(b.type) == value_bytes && b.format == A->format &&
            b.transposed == transposing;
@@ -325,6 +334,10 @@ mcspStatus_t spmv_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
         a.row_ptr = nullptr;
         a.col = nullptr;
         a.val = nullptr;
+        if (A->banded.along_diagonals)
+            return mcsp::launch_spmv_diagonals<T>(h->stream, A->banded.diagonals, a, h_alpha, h_beta, buf + A->banded.region)
+                       ? MCSP_STATUS_SUCCESS
+                       : MCSP_STATUS_INTERNAL_ERROR;
         // (a device that refuses the kernel's LDS size launches nothing: an error, not a y left unwritten)
         return mcsp::launch_spmv_banded<T>(h->stream, A->banded.shape, A->banded.grid, a, h_alpha, h_beta,
                                            buf + A->banded.region)
@@ -767,10 +780,10 @@ mcspStatus_t spmv_call(mcsparseHandle_t handle, mcsparseOperation_t opA, const v
 // leaves the copy's extra partial sums as pure cost), so both are run here, on the handle's stream, with the
 // caller's x and a y inside the buffer, and timed with events: once each, which settles it where one takes more
 // than twice the other's time (or, for long runs, a quarter more), else twice more.  *copy_wins says whether the
-// copy was faster by more than a twentieth.
+// copy was faster by more than a twentieth.  in_use: the flag of matA->banded that has calls run from the copy; set on return.
 mcspStatus_t spmv_trial(mcsparseHandle_t handle, mcsparseOperation_t opA, mcsparseSpMatDescr_t matA,
                         mcsparseDnVecDescr_t vecX, void* trial_y, macaDataType computeType, void* buffer,
-                        mcsparseSpMVAlg_t alg, bool* copy_wins) {
+                        mcsparseSpMVAlg_t alg, bool* in_use, bool* copy_wins) {
     mcsparseDnVecDescr y = {};
     const CsrView v = make_view(matA, opA);
     y.valueType = computeType;
@@ -791,7 +804,7 @@ mcspStatus_t spmv_trial(mcsparseHandle_t handle, mcsparseOperation_t opA, mcspar
     float rows_ms = 0.0f, copy_ms = 0.0f;
     for (int runs = 1; runs <= 2 && st == MCSP_STATUS_SUCCESS; ++runs) {
         for (int leg = 0; leg < 2 && st == MCSP_STATUS_SUCCESS; ++leg) {
-            matA->banded.useful = leg == 1;  // leg 0 runs the row kernels, leg 1 the copy
+            *in_use = leg == 1;  // leg 0 runs the row kernels, leg 1 the copy
             if (hipEventRecord(marks[leg], handle->stream) != hipSuccess) st = MCSP_STATUS_INTERNAL_ERROR;
             for (int run = 0; run < runs && st == MCSP_STATUS_SUCCESS; ++run)
                 st = computeType == MACA_R_32F
@@ -811,7 +824,7 @@ mcspStatus_t spmv_trial(mcsparseHandle_t handle, mcsparseOperation_t opA, mcspar
     for (hipEvent_t e : marks)
         if (e != nullptr) (void)hipEventDestroy(e);
     handle->ptr_mode = callers_mode;
-    matA->banded.useful = true;
+    *in_use = true;
     *copy_wins = copy_ms * 20.0f < rows_ms * 19.0f;
     return st;
 }
@@ -877,6 +890,14 @@ mcsparseStatus_t mcsparseSpMV_preprocess_bufferSize(mcsparseHandle_t handle, mcs
                       (v.transpose ? (shape.by_column ? 0 : transpose_scratch(v, matA->nnz, vb).total)
                                    : align_up(static_cast<size_t>(rows) * vb));
     }
+    if (diagonals_candidate(matA, opA)) {
+        const size_t vb = value_size(matA->valueType);
+        const CsrView v = make_view(matA, opA);
+        const idx_t rows = static_cast<idx_t>(v.m);
+        *bufferSize = std::max(*bufferSize, banded_region_offset(matA, opA, vb) +
+                                                mcsp::spmv_diagonals_bytes(rows, static_cast<idx_t>(matA->nnz), vb) +
+                                                align_up(static_cast<size_t>(rows) * vb));  // and the y of the trial
+    }
     return MCSPARSE_STATUS_SUCCESS;
 }
 
@@ -892,7 +913,9 @@ mcsparseStatus_t mcsparseSpMV_preprocess(mcsparseHandle_t handle, mcsparseOperat
     if (stream_is_capturing(handle->stream)) return to_public_status(MCSP_STATUS_NOT_IMPLEMENTED);  // it blocks
     if (handle->spmv_deterministic) alg = MCSPARSE_SPMV_CSR_ALG2;
     BandedShape shape;
-    if (matA->nnz == 0 || !banded_candidate(matA, opA, alg, &shape)) return MCSPARSE_STATUS_SUCCESS;  // nothing to prepare
+    const bool try_bands = matA->nnz != 0 && banded_candidate(matA, opA, alg, &shape);
+    const bool try_diagonals = matA->nnz != 0 && handle->spmv_preprocess_trial && diagonals_candidate(matA, opA);
+    if (!try_bands && !try_diagonals) return MCSPARSE_STATUS_SUCCESS;  // nothing to prepare
 
     CsrView v = make_view(matA, opA);
     const idx_t m = static_cast<idx_t>(v.transpose ? v.n : v.m);  // rows of the matrix that is banded
@@ -921,6 +944,38 @@ mcsparseStatus_t mcsparseSpMV_preprocess(mcsparseHandle_t handle, mcsparseOperat
                                             v.n * static_cast<int64_t>(vb), externalBuffer, true);
         if (ps != MCSP_STATUS_SUCCESS) return to_public_status(ps);
     }
+    SpmvBanded& b = matA->banded;
+    b.buffer = externalBuffer;
+    b.rows = matA->rows;
+    b.cols = matA->cols;
+    b.vals = matA->vals;
+    b.m = matA->row_num;
+    b.n = matA->col_num;
+    b.nnz = matA->nnz;
+    b.base = static_cast<int>(matA->idxBase);
+    b.type = matA->valueType;
+    b.format = matA->format;
+    b.transposed = v.transpose;
+    b.region = banded_region_offset(matA, opA, vb);
+    b.shape = BandedShape();
+    b.useful = b.along_diagonals = false;
+    char* region = static_cast<char*>(externalBuffer) + b.region;
+    // Rows that share their diagonals (grids): a copy along them takes half the time of the row kernels or of a banded copy,
+    // and a look at a few hundred rows tells other matrices apart.
+    if (try_diagonals) {
+        if (!mcsp::build_spmv_diagonals(handle->stream, m, nnz, base, v.ptr, v.ind, matA->vals, vb, region, &b.diagonals))
+            return to_public_status(MCSP_STATUS_INTERNAL_ERROR);
+        if (b.diagonals != 0) {
+            bool copy_wins = false;
+            b.valid = true;
+            const mcspStatus_t ts = mcsp::spmv_trial(handle, opA, matA, vecX, region + mcsp::spmv_diagonals_bytes(m, nnz, vb),
+                                                     computeType, externalBuffer, alg, &b.along_diagonals, &copy_wins);
+            b.valid = ts == MCSP_STATUS_SUCCESS && copy_wins;
+            b.along_diagonals = b.valid;
+            if (ts != MCSP_STATUS_SUCCESS || copy_wins) return to_public_status(ts);
+        }
+    }
+    if (!try_bands) return MCSPARSE_STATUS_SUCCESS;
     // Where a few lines of x take most of the gathers (long rows under a transposing direction, popular columns),
     // one band group over all of x does better than groups that fit an XCD's L2: the hot lines stay in L2 anyway
     // and the planes of partial sums go.  Measured on the matrix, unless the caller has set the width.
@@ -946,26 +1001,12 @@ mcsparseStatus_t mcsparseSpMV_preprocess(mcsparseHandle_t handle, mcsparseOperat
             }
         }
     }
-    SpmvBanded& b = matA->banded;
-    b.buffer = externalBuffer;
-    b.rows = matA->rows;
-    b.cols = matA->cols;
-    b.vals = matA->vals;
-    b.m = matA->row_num;
-    b.n = matA->col_num;
-    b.nnz = matA->nnz;
-    b.base = static_cast<int>(matA->idxBase);
-    b.type = matA->valueType;
-    b.format = matA->format;
-    b.transposed = v.transpose;
     b.shape = shape;
     // the longest row is known from the analysis above; for a transposing direction (rows = the view's columns) it
     // is not, and the plain kernel is used
     b.shape.crowded_rows = shape.by_column && !v.transpose && matA->plan.valid && shape.chunks != 0 &&
                            2 * static_cast<uint64_t>(matA->plan.max_row_len) > static_cast<uint64_t>(nnz) / shape.chunks;
-    b.region = banded_region_offset(matA, opA, vb);
     b.grid = 0;
-    char* region = static_cast<char*>(externalBuffer) + b.region;
     if (shape.by_column) {
         const mcsp::BandedLayout cl = mcsp::banded_layout(shape, m, nnz, vb);
         idx_t* src_cols = reinterpret_cast<idx_t*>(region + cl.src_cols);
@@ -1013,7 +1054,7 @@ mcsparseStatus_t mcsparseSpMV_preprocess(mcsparseHandle_t handle, mcsparseOperat
         matA->plan.forced_family == kFamilyAuto) {
         bool copy_wins = true;
         const mcspStatus_t ts = mcsp::spmv_trial(handle, opA, matA, vecX, region + align_up(l.total), computeType,
-                                                 externalBuffer, alg, &copy_wins);
+                                                 externalBuffer, alg, &b.useful, &copy_wins);
         if (ts != MCSP_STATUS_SUCCESS) {
             b.valid = false;
             return to_public_status(ts);

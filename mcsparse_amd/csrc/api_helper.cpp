@@ -410,6 +410,12 @@ mcsparseStatus_t mcsparseSpMatGetSpMVPreprocess(mcsparseSpMatDescr_t d, int* sta
     return MCSPARSE_STATUS_SUCCESS;
 }
 
+mcsparseStatus_t mcsparseSpMatGetSpMVDiagonals(mcsparseSpMatDescr_t d, int64_t* diagonals) {
+    if (d == nullptr || diagonals == nullptr) return to_public_status(MCSP_STATUS_INVALID_POINTER);
+    *diagonals = d->banded.valid && d->banded.along_diagonals ? static_cast<int64_t>(d->banded.diagonals) : 0;
+    return MCSPARSE_STATUS_SUCCESS;
+}
+
 mcsparseStatus_t mcsparseSpMatSetSpMVBandBytes(mcsparseSpMatDescr_t d, size_t band_bytes) {
     if (d == nullptr) return to_public_status(MCSP_STATUS_INVALID_POINTER);
     if (band_bytes != 0 && (band_bytes < 16 || band_bytes > (size_t(1) << 30)))

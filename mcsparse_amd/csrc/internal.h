@@ -126,7 +126,7 @@ struct BandedShape {
 struct SpmvBanded {
     bool valid = false;
     bool useful = false;     // false: preprocess built the copy, timed it against the row kernels and found it
-                             // no faster; calls run the row kernels
+                             // no faster, or built none; calls go row by row
     const void* buffer = nullptr;
     const void* rows = nullptr;
     const void* cols = nullptr;
@@ -139,6 +139,9 @@ struct SpmvBanded {
     size_t region = 0;       // offset of the banded copy inside the buffer
     BandedShape shape = {};
     uint32_t grid = 0;       // workgroups of the SpMV kernel
+    // a copy along the diagonals (spmv_diagonals.hip) lies in the region instead, and is used; of so many diagonals
+    bool along_diagonals = false;
+    uint32_t diagonals = 0;
     size_t band_bytes = 0;   // user override of the band width (mcsparseSpMatSetSpMVBandBytes); 0 = default
 };
 
@@ -339,6 +342,18 @@ uint32_t banded_grid(const uint32_t* xcd_start_host);
 template <typename T>
 bool launch_spmv_banded(hipStream_t stream, const BandedShape& s, uint32_t grid, const SpmvArgs& a, T alpha, T beta,
                         void* region);
+
+// ---- SpMV along the diagonals (spmv_diagonals.hip) ----
+// (fewer nonzeros are a launch's time whichever way they are stored)
+constexpr idx_t kDiagonalsLeastNonzeros = 1u << 18;
+bool spmv_diagonals_shape(idx_t m, idx_t n, idx_t nnz);
+size_t spmv_diagonals_bytes(idx_t m, idx_t nnz, size_t value_bytes);
+// Builds the copy in `region`, of spmv_diagonals_bytes bytes, and sets *total to its number of diagonals; 0 where the rows of
+// the matrix do not share diagonals, are not sorted by column or hold a column twice.  Blocks; false on a runtime error.
+bool build_spmv_diagonals(hipStream_t stream, idx_t m, idx_t nnz, idx_t base, const idx_t* row_ptr, const idx_t* col,
+                          const void* val, size_t value_bytes, void* region, uint32_t* total);
+template <typename T>
+bool launch_spmv_diagonals(hipStream_t stream, uint32_t total, const SpmvArgs& a, T alpha, T beta, void* region);
 
 // Streaming kernels that measure what the memory takes by itself (analysis.hip): mode 0 reads src, 1 writes dst,
 // 2 copies; bytes a multiple of 16 and below 2^44, arrays 16-byte aligned, sink = at least one uint32 for mode 0.
