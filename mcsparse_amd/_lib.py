@@ -68,6 +68,7 @@ PROTOTYPES = {
     "mcsparseSpMatSetSpMVBandBytes": (c_int, [vp, c_size]),
     "mcsparseSpMatGetSpMVPreprocess": (c_int, [vp, P(c_int), P(c_int), P(c_int)]),
     "mcsparseSpMatGetSpMVDiagonals": (c_int, [vp, P(c_i64)]),
+    "mcsparseSpMatGetSpMMDiagonals": (c_int, [vp, P(c_i64)]),
     "mcsparseSpMV_bufferSize": (c_int, [vp, c_int, vp, vp, vp, vp, vp, c_int, c_int, P(c_size)]),
     "mcsparseSpMM_bufferSize": (c_int, [vp, c_int, c_int, vp, vp, vp, vp, vp, c_int, c_int, P(c_size)]),
     "mcsparseSpMM_preprocess": (c_int, [vp, c_int, c_int, vp, vp, vp, vp, vp, c_int, c_int, vp]),

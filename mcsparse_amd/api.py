@@ -172,6 +172,12 @@ class SpMat:
         check(self.lib.mcsparseSpMatGetSpMVDiagonals(self._d, ctypes.byref(count)))
         return count.value
 
+    def spmm_diagonals(self):
+        """How many diagonals mcsparseSpMM_preprocess keeps for products with column-major operands; 0 = none."""
+        count = ctypes.c_int64()
+        check(self.lib.mcsparseSpMatGetSpMMDiagonals(self._d, ctypes.byref(count)))
+        return count.value
+
     def spmm_schedule(self):
         """(state, entries) left by mcsparseSpMM_preprocess; state 2 = merged column lists, 3 = diagonal blocks over
         groups of eight rows, 4 = diagonal blocks over groups of strips (all three in use), 1 = built and declined."""

@@ -270,7 +270,7 @@ bool diagonals_candidate(const mcsparseSpMatDescr* A, mcsparseOperation_t op) {
     if (!format_is_built(A->format) || (A->valueType != MACA_R_32F && A->valueType != MACA_R_64F)) return false;
     const CsrView v = make_view(A, op);
     return !v.transpose && A->banded.band_bytes == 0 && A->plan.forced_family == kFamilyAuto &&
-           mcsp::spmv_diagonals_shape(static_cast<idx_t>(v.m), static_cast<idx_t>(v.n), static_cast<idx_t>(A->nnz));
+           mcsp::slice_diagonals_shape(static_cast<idx_t>(v.m), static_cast<idx_t>(v.n), static_cast<idx_t>(A->nnz));
 }
 
 // Scratch of the preprocess call behind the banded copy of a transposing direction: the transpose in
@@ -437,7 +437,7 @@ mcspStatus_t spmv_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
 // CSC gets the transposed copy [row_ptr m+1 | col_ind nnz][values][csr2csc workspace]
 // (mcsp_spmm_gpu.cpp:818-849); 64-bit index arrays add their narrowed copies at the end.
 struct SpmmLayout {
-    size_t ptr, ind, vals, csr2csc_ws, bt, ct, long_ws, narrow, total;
+    size_t ptr, diagonals, ind, vals, csr2csc_ws, bt, ct, long_ws, narrow, total;
     int64_t n_padded;  // leading dimension of the row-major copies of op(B) and C
     bool copy_b, copy_c;
 };
@@ -453,11 +453,19 @@ bool schedulable(const mcsparseSpMatDescr* A) {
            A->col_num <= mcsp::kSpmmMaxScheduledColumns;
 }
 
+bool diagonals_schedulable(const mcsparseSpMatDescr* A, size_t value_bytes) {
+    return schedulable(A) && (value_bytes == 4 || value_bytes == 8) &&
+           mcsp::slice_diagonals_shape(static_cast<idx_t>(A->row_num), static_cast<idx_t>(A->col_num), static_cast<idx_t>(A->nnz));
+}
+
 // The schedule of the descriptor belongs to this call: same buffer, same arrays, same extents.
-bool schedule_matches(const mcsparseSpMatDescr* A, const void* buffer) {
+bool schedule_of_call(const mcsparseSpMatDescr* A, const void* buffer) {
     const SpmmSchedule& s = A->schedule;
-    return s.valid && s.useful && s.buffer == buffer && s.rows == A->rows && s.cols == A->cols && s.m == A->row_num &&
+    return s.valid && s.buffer == buffer && s.rows == A->rows && s.cols == A->cols && s.m == A->row_num &&
            s.nnz == A->nnz && s.base == static_cast<int>(A->idxBase);
+}
+bool schedule_matches(const mcsparseSpMatDescr* A, const void* buffer) {
+    return A->schedule.useful && schedule_of_call(A, buffer);
 }
 
 // A column-major op(B) would be gathered element by element and a column-major C written element by
@@ -470,6 +478,10 @@ SpmmLayout spmm_layout(const mcsparseSpMatDescr* A, const mcsparseDnMatDescr* B,
     size_t off = 0;
     if (A->format == MCSPARSE_FORMAT_CSR) {
         if (schedulable(A)) off += mcsp::spmm_schedule_layout(static_cast<idx_t>(A->row_num), static_cast<idx_t>(A->nnz)).total;
+        // (for every order of the operands, so that a call with others leaves it alone)
+        l.diagonals = off;
+        if (diagonals_schedulable(A, value_bytes))
+            off += mcsp::slice_diagonals_layout(static_cast<idx_t>(A->row_num), static_cast<idx_t>(A->nnz), value_bytes, false).total;
     } else if (A->format == MCSPARSE_FORMAT_COO) {
         off += align_up(static_cast<size_t>(A->row_num + 1) * sizeof(idx_t));
     } else if (A->format == MCSPARSE_FORMAT_CSC) {
@@ -588,6 +600,13 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
                 a.long_ws = buf + l.long_ws;
                 a.long_n = l.n_padded;
             }
+        }
+        // both operands column-major and rows that share diagonals: nothing is transposed
+        if (l.copy_b && l.copy_c && A->nnz != 0 && (b == 0 || shared_structure) && schedule_of_call(A, buffer) &&
+            A->schedule.diagonals != 0 && A->schedule.diagonals_value_bytes == sizeof(T) &&
+            mcsp::spmm_diagonals_usable(a.k, a.n, A->schedule.longest_slice, sizeof(T))) {
+            mcsp::launch_spmm_diagonals<T>(h->stream, a, A->schedule.diagonals, buf + l.diagonals, h_alpha, h_beta);
+            continue;
         }
         T beta_inner = h_beta;
         if (l.copy_b && A->nnz != 0) {  // without nonzeros op(B) is never read (and may be NULL)
@@ -895,7 +914,7 @@ mcsparseStatus_t mcsparseSpMV_preprocess_bufferSize(mcsparseHandle_t handle, mcs
         const CsrView v = make_view(matA, opA);
         const idx_t rows = static_cast<idx_t>(v.m);
         *bufferSize = std::max(*bufferSize, banded_region_offset(matA, opA, vb) +
-                                                mcsp::spmv_diagonals_bytes(rows, static_cast<idx_t>(matA->nnz), vb) +
+                                                mcsp::slice_diagonals_layout(rows, static_cast<idx_t>(matA->nnz), vb, true).total +
                                                 align_up(static_cast<size_t>(rows) * vb));  // and the y of the trial
     }
     return MCSPARSE_STATUS_SUCCESS;
@@ -963,13 +982,14 @@ mcsparseStatus_t mcsparseSpMV_preprocess(mcsparseHandle_t handle, mcsparseOperat
     // Rows that share their diagonals (grids): a copy along them takes half the time of the row kernels or of a banded copy,
     // and a look at a few hundred rows tells other matrices apart.
     if (try_diagonals) {
-        if (!mcsp::build_spmv_diagonals(handle->stream, m, nnz, base, v.ptr, v.ind, matA->vals, vb, region, &b.diagonals))
+        if (!mcsp::build_slice_diagonals(handle->stream, m, nnz, base, v.ptr, v.ind, matA->vals, vb, region, &b.diagonals, nullptr))
             return to_public_status(MCSP_STATUS_INTERNAL_ERROR);
         if (b.diagonals != 0) {
             bool copy_wins = false;
             b.valid = true;
-            const mcspStatus_t ts = mcsp::spmv_trial(handle, opA, matA, vecX, region + mcsp::spmv_diagonals_bytes(m, nnz, vb),
-                                                     computeType, externalBuffer, alg, &b.along_diagonals, &copy_wins);
+            char* trial_y = region + mcsp::slice_diagonals_layout(m, nnz, vb, true).total;
+            const mcspStatus_t ts = mcsp::spmv_trial(handle, opA, matA, vecX, trial_y, computeType, externalBuffer, alg,
+                                                     &b.along_diagonals, &copy_wins);
             b.valid = ts == MCSP_STATUS_SUCCESS && copy_wins;
             b.along_diagonals = b.valid;
             if (ts != MCSP_STATUS_SUCCESS || copy_wins) return to_public_status(ts);
@@ -1157,6 +1177,7 @@ mcsparseStatus_t mcsparseSpMM_preprocess(mcsparseHandle_t handle, mcsparseOperat
     s.base = static_cast<int>(matA->idxBase);
     s.blocks = false;
     s.stride = 0;
+    s.diagonals = 0;
     {
         // The kernels that work from a schedule walk every row in one piece; a matrix with rows of thousands of
         // nonzeros is left to the row kernels, which hand such rows to the kernels of spmm_long.hip.
@@ -1171,6 +1192,19 @@ mcsparseStatus_t mcsparseSpMM_preprocess(mcsparseHandle_t handle, mcsparseOperat
             s.valid = true;
             return MCSPARSE_STATUS_SUCCESS;
         }
+    }
+    if (!b_image_is_row_major(opB, matB) && matC->order != MCSPARSE_ORDER_ROW &&
+        diagonals_schedulable(matA, value_size(matA->valueType))) {
+        s.diagonals_value_bytes = value_size(matA->valueType);
+        if (!mcsp::build_slice_diagonals(handle->stream, m, nnz, static_cast<idx_t>(matA->idxBase), ia.rows, ia.cols, nullptr,
+                                         s.diagonals_value_bytes,
+                                         static_cast<char*>(externalBuffer) +
+                                             spmm_layout(matA, matB, matC, opB, s.diagonals_value_bytes).diagonals,
+                                         &s.diagonals, &s.longest_slice))
+            return to_public_status(MCSP_STATUS_INTERNAL_ERROR);
+        if (!mcsp::spmm_diagonals_usable(static_cast<idx_t>(matA->col_num), static_cast<idx_t>(matC->col_num), s.longest_slice,
+                                         s.diagonals_value_bytes))
+            s.diagonals = 0;
     }
     const char* span_slot = static_cast<const char*>(externalBuffer) + l.span_sum;
 

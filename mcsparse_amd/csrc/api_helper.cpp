@@ -410,6 +410,12 @@ mcsparseStatus_t mcsparseSpMatGetSpMVPreprocess(mcsparseSpMatDescr_t d, int* sta
     return MCSPARSE_STATUS_SUCCESS;
 }
 
+mcsparseStatus_t mcsparseSpMatGetSpMMDiagonals(mcsparseSpMatDescr_t d, int64_t* diagonals) {
+    if (d == nullptr || diagonals == nullptr) return to_public_status(MCSP_STATUS_INVALID_POINTER);
+    *diagonals = d->schedule.valid ? static_cast<int64_t>(d->schedule.diagonals) : 0;
+    return MCSPARSE_STATUS_SUCCESS;
+}
+
 mcsparseStatus_t mcsparseSpMatGetSpMVDiagonals(mcsparseSpMatDescr_t d, int64_t* diagonals) {
     if (d == nullptr || diagonals == nullptr) return to_public_status(MCSP_STATUS_INVALID_POINTER);
     *diagonals = d->banded.valid && d->banded.along_diagonals ? static_cast<int64_t>(d->banded.diagonals) : 0;

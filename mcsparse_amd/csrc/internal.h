@@ -99,6 +99,11 @@ struct SpmmSchedule {
     bool blocks = false;   // the schedule holds diagonal blocks (spmm_blocks.hip) instead of merged lists
     uint32_t longest_group = 0;  // blocks: the most nonzeros in one group of rows (strips: in one strip)
     uint32_t stride = 0;   // blocks: != 0 says the groups are strips this many rows apart (spmm_strips.hip)
+    // beside that (whether useful or not), for column-major operands: the diagonals of slices of rows (spmm_diagonals.hip),
+    // behind the region of the above; 0: none
+    uint32_t diagonals = 0;
+    uint32_t longest_slice = 0;  // most nonzeros of a slice
+    size_t diagonals_value_bytes = 0;  // the slices' length goes with it
 };
 
 // Column-banded copy of a CSR matrix built by mcsparseSpMV_preprocess inside the caller's buffer
@@ -343,15 +348,26 @@ template <typename T>
 bool launch_spmv_banded(hipStream_t stream, const BandedShape& s, uint32_t grid, const SpmvArgs& a, T alpha, T beta,
                         void* region);
 
-// ---- SpMV along the diagonals (spmv_diagonals.hip) ----
+// ---- rows that share diagonals (spmv_diagonals.hip, spmm_diagonals.hip) ----
 // (fewer nonzeros are a launch's time whichever way they are stored)
 constexpr idx_t kDiagonalsLeastNonzeros = 1u << 18;
-bool spmv_diagonals_shape(idx_t m, idx_t n, idx_t nnz);
-size_t spmv_diagonals_bytes(idx_t m, idx_t nnz, size_t value_bytes);
-// Builds the copy in `region`, of spmv_diagonals_bytes bytes, and sets *total to its number of diagonals; 0 where the rows of
-// the matrix do not share diagonals, are not sorted by column or hold a column twice.  Blocks; false on a runtime error.
-bool build_spmv_diagonals(hipStream_t stream, idx_t m, idx_t nnz, idx_t base, const idx_t* row_ptr, const idx_t* col,
-                          const void* val, size_t value_bytes, void* region, uint32_t* total);
+bool slice_diagonals_shape(idx_t m, idx_t n, idx_t nnz);
+struct SliceDiagonalsLayout {
+    size_t totals, diagonal_first, diagonals, vals, scan_ws, total;
+    uint32_t slices, most;
+};
+SliceDiagonalsLayout slice_diagonals_layout(idx_t m, idx_t nnz, size_t value_bytes, bool with_values);
+// Finds the diagonals of every slice of rows, and copies the values along them where val != nullptr, in `region` (the
+// layout's total).  *total = their number; 0 where the rows of the matrix do not share diagonals, are not sorted by column or
+// hold a column twice.  longest (may be null): the most nonzeros of a slice.  Blocks; false on a runtime error.
+bool build_slice_diagonals(hipStream_t stream, idx_t m, idx_t nnz, idx_t base, const idx_t* row_ptr, const idx_t* col,
+                           const void* val, size_t value_bytes, void* region, uint32_t* total, uint32_t* longest);
+// op(B) and C column-major (B: element (kk, j) at kk + j * ldb), the product row by row from the caller's values; region: what
+// build_slice_diagonals has left without values.
+bool spmm_diagonals_usable(idx_t k, idx_t n, uint32_t longest, size_t value_bytes);
+struct SpmmArgs;
+template <typename T>
+void launch_spmm_diagonals(hipStream_t stream, const SpmmArgs& a, uint32_t total, const void* region, T alpha, T beta);
 template <typename T>
 bool launch_spmv_diagonals(hipStream_t stream, uint32_t total, const SpmvArgs& a, T alpha, T beta, void* region);
 

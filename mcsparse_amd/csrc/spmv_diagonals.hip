@@ -13,12 +13,13 @@
 // fp32, copy in column order and this: 134 and 54; 5-point Laplacian 1900 x 1801, fp32: 49.6 and 18.
 //
 // Stands in, like spmv.hip, for the reference's row kernel (src/kernels/level2/spmv/csr_vector_device.hpp:22-79).
-#include "device_util.h"
-#include "internal.h"
+#include "diagonals_device.h"
 
 namespace mcsp {
 
 namespace {
+
+using namespace diagonals_detail;
 
 constexpr int kBlock = 256;
 constexpr uint32_t kWaves = kBlock / kWave;
@@ -32,22 +33,10 @@ constexpr uint64_t kKeptBytes = 128ull << 20;
 constexpr uint32_t kFewDiagonals = 12;
 constexpr uint32_t kMostDiagonals = 512;  // of a slice; more: not a matrix for this copy
 
-template <typename T>
-constexpr int lane_rows() { return 16 / static_cast<int>(sizeof(T)); }  // neighbouring rows of a lane
-template <typename T>
-constexpr uint32_t slice_rows() { return kWave * lane_rows<T>(); }
-uint32_t slice_rows_of(size_t value_bytes) { return value_bytes == 4 ? slice_rows<float>() : slice_rows<double>(); }
-
-// A diagonal of a slice: row r0 + R * lane + j holds column row + offset (mod 2^32) where bit `lane` of rows[j] is set.
-template <int R>
-struct SliceDiagonal {
-    uint32_t offset, unused;
-    unsigned long long rows[R];
-};
-
 struct DiagonalTotals {
     unsigned long long diagonals, nonzeros;  // of the slices looked at
     uint32_t refused;                        // != 0: a row with unsorted or repeated columns, or too many diagonals
+    uint32_t longest;                        // most nonzeros of a slice
 };
 
 // the smallest over the wavefront, in every lane
@@ -64,9 +53,10 @@ __device__ __forceinline__ int wave_min(int v) {
 
 // A wavefront per slice merges its rows by offset.  The slice's columns (and values) are brought to LDS in one piece where
 // they fit: walked where they lie, the rows of the slices in flight push each other's lines out of the caches (1000 us for
-// both passes over 23 M nonzeros).  FILL: the diagonals are written; else they are counted, into counts[slice] or, where
-// that is null, added up (`stride` slices apart).
-template <typename T, bool FILL>
+// both passes over 23 M nonzeros).  The diagonals are counted, into counts[slice] or, where that is null, added up (`stride`
+// slices apart), or written, with or without their values.
+enum SlicePass : int { kCount, kDescribe, kCopy };
+template <typename T, int PASS>
 __global__ __launch_bounds__(kWave) void slice_diagonals_kernel(idx_t m, idx_t base, uint32_t slices, uint32_t stride,
                                                                 const idx_t* __restrict__ row_ptr,
                                                                 const idx_t* __restrict__ col, const T* __restrict__ val,
@@ -77,7 +67,7 @@ __global__ __launch_bounds__(kWave) void slice_diagonals_kernel(idx_t m, idx_t b
     constexpr uint32_t kRows = slice_rows<T>(), kStaged = kRows * 28;
     typedef T vec_t __attribute__((ext_vector_type(R)));
     __shared__ idx_t s_col[kStaged];
-    __shared__ T s_val[FILL ? kStaged : 1];
+    __shared__ T s_val[PASS == kCopy ? kStaged : 1];
     const uint64_t slice = static_cast<uint64_t>(blockIdx.x) * stride;
     if (slice >= slices) return;  // whole workgroup
     const uint32_t lane = lane_id();
@@ -89,7 +79,7 @@ __global__ __launch_bounds__(kWave) void slice_diagonals_kernel(idx_t m, idx_t b
 #pragma unroll 8
         for (uint32_t p = lane; p < nonzeros; p += kWave) {
             s_col[p] = col[first + p];
-            if constexpr (FILL) s_val[p] = val[first + p];
+            if constexpr (PASS == kCopy) s_val[p] = val[first + p];
         }
         __syncthreads();
     }
@@ -110,7 +100,7 @@ __global__ __launch_bounds__(kWave) void slice_diagonals_kernel(idx_t m, idx_t b
         offset[j] = offset_at(j, at[j]);
     }
     uint32_t found = 0;
-    const uint64_t out = FILL ? counts[slice] : 0;
+    const uint64_t out = PASS != kCount ? counts[slice] : 0;
     bool refused = false;
     while (true) {
         int least = offset[0];
@@ -131,24 +121,23 @@ __global__ __launch_bounds__(kWave) void slice_diagonals_kernel(idx_t m, idx_t b
             const bool mine = offset[j] == least;
             d.rows[j] = __ballot(mine);
             if (mine) {
-                if constexpr (FILL) v[j] = staged ? s_val[at[j]] : val[first + at[j]];
+                if constexpr (PASS == kCopy) v[j] = staged ? s_val[at[j]] : val[first + at[j]];
                 offset[j] = offset_at(j, ++at[j]);
                 refused |= offset[j] <= least;
             }
         }
-        if constexpr (FILL) {
-            reinterpret_cast<vec_t*>(vals_out)[(out + found) * kWave + lane] = v;
-            if (lane == 0) diagonals[out + found] = d;
-        }
+        if constexpr (PASS == kCopy) reinterpret_cast<vec_t*>(vals_out)[(out + found) * kWave + lane] = v;
+        if (PASS != kCount && lane == 0) diagonals[out + found] = d;
         ++found;
         if (__any(refused)) break;
     }
-    if constexpr (!FILL) {
+    if constexpr (PASS == kCount) {
         if (__any(refused)) {
             found = 0;
             if (lane == 0) totals->refused = 1;
         }
         if (lane == 0) {
+            if (nonzeros > totals->longest) atomicMax(&totals->longest, nonzeros);  // (mostly not: no queue at the counter)
             if (counts != nullptr) {
                 counts[slice] = found;
             } else {
@@ -160,7 +149,7 @@ __global__ __launch_bounds__(kWave) void slice_diagonals_kernel(idx_t m, idx_t b
 }
 
 __global__ void clear_totals_kernel(DiagonalTotals* totals, uint32_t* last_count) {
-    *totals = DiagonalTotals{0, 0, 0};
+    *totals = DiagonalTotals{0, 0, 0, 0};
     *last_count = 0;  // the scan leaves the sum of all counts there
 }
 
@@ -181,8 +170,7 @@ __global__ __launch_bounds__(kBlock) void spmv_diagonals_kernel(idx_t m, idx_t n
     typedef T vec_t __attribute__((ext_vector_type(R)));
     typedef vec_t element_aligned __attribute__((aligned(sizeof(T))));  // a vector of x or y from any element on
     __shared__ double s_sum[kWaves][R][kWave];
-    const uint32_t per_xcd = gridDim.x / xcds;  // neighbouring slices read the same x: an XCD takes a stretch of them
-    const uint32_t block = (blockIdx.x % xcds) * per_xcd + blockIdx.x / xcds;
+    const uint32_t block = block_in_stretch(xcds);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const uint32_t slice = block * (kWaves / WAVES) + wave / WAVES;
     const uint32_t lane = lane_id();
@@ -273,14 +261,12 @@ __global__ __launch_bounds__(kBlock) void spmv_diagonals_kernel(idx_t m, idx_t n
     }
 }
 
-struct DiagonalsLayout {
-    size_t totals, diagonal_first, diagonals, vals, scan_ws, total;
-    uint32_t slices, most;
-};
-DiagonalsLayout diagonals_layout(idx_t m, idx_t nnz, size_t value_bytes) {
+}  // namespace
+
+SliceDiagonalsLayout slice_diagonals_layout(idx_t m, idx_t nnz, size_t value_bytes, bool with_values) {
     const uint32_t rows = slice_rows_of(value_bytes);
     const size_t diagonal = value_bytes == 4 ? sizeof(SliceDiagonal<4>) : sizeof(SliceDiagonal<2>);
-    DiagonalsLayout l;
+    SliceDiagonalsLayout l;
     l.slices = static_cast<uint32_t>((static_cast<uint64_t>(m) + rows - 1) / rows);
     // two thirds of the places filled: with fewer, fp64 values alone are as long as values and columns in rows
     l.most = static_cast<uint32_t>(static_cast<uint64_t>(nnz) * 3 / (2 * rows));
@@ -288,16 +274,22 @@ DiagonalsLayout diagonals_layout(idx_t m, idx_t nnz, size_t value_bytes) {
     l.totals = off; off += align_up(sizeof(DiagonalTotals));
     l.diagonal_first = off; off += align_up((static_cast<size_t>(l.slices) + 1) * sizeof(uint32_t));
     l.diagonals = off; off += align_up(static_cast<size_t>(l.most) * diagonal);
-    l.vals = off; off += align_up(static_cast<size_t>(l.most) * rows * value_bytes);
+    l.vals = off; off += with_values ? align_up(static_cast<size_t>(l.most) * rows * value_bytes) : 0;
     l.scan_ws = off; off += align_up(exclusive_scan_workspace_bytes(static_cast<uint64_t>(l.slices) + 1));
     l.total = off;
     return l;
 }
 
+bool slice_diagonals_shape(idx_t m, idx_t n, idx_t nnz) {
+    return m != 0 && nnz >= kDiagonalsLeastNonzeros && m < (1u << 31) && n < (1u << 31);
+}
+
+namespace {
+
 template <typename T>
 bool build_typed(hipStream_t stream, idx_t m, idx_t nnz, idx_t base, const idx_t* row_ptr, const idx_t* col, const T* val,
-                 void* region, uint32_t* total) {
-    const DiagonalsLayout l = diagonals_layout(m, nnz, sizeof(T));
+                 void* region, uint32_t* total, uint32_t* longest) {
+    const SliceDiagonalsLayout l = slice_diagonals_layout(m, nnz, sizeof(T), val != nullptr);
     char* w = static_cast<char*>(region);
     DiagonalTotals* totals = reinterpret_cast<DiagonalTotals*>(w + l.totals);
     uint32_t* counts = reinterpret_cast<uint32_t*>(w + l.diagonal_first);
@@ -307,44 +299,41 @@ bool build_typed(hipStream_t stream, idx_t m, idx_t nnz, idx_t base, const idx_t
         return hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToHost, stream) == hipSuccess &&
                hipStreamSynchronize(stream) == hipSuccess;
     };
+    auto run = [&](auto* kernel, uint32_t stride, uint32_t* per_slice) {
+        hipLaunchKernelGGL(kernel, dim3((l.slices + stride - 1) / stride), dim3(kWave), 0, stream, m, base, l.slices, stride,
+                           row_ptr, col, val, per_slice, totals, diagonals, vals);
+    };
     hipLaunchKernelGGL(clear_totals_kernel, dim3(1), dim3(1), 0, stream, totals, counts + l.slices);
     // a sample first: most matrices are turned away here
-    const uint32_t stride = l.slices / kSampledSlices + 1;
-    hipLaunchKernelGGL((slice_diagonals_kernel<T, false>), dim3((l.slices + stride - 1) / stride), dim3(kWave), 0, stream, m,
-                       base, l.slices, stride, row_ptr, col, val, nullptr, totals, diagonals, vals);
+    run(slice_diagonals_kernel<T, kCount>, l.slices / kSampledSlices + 1, nullptr);
     DiagonalTotals t;
     if (!read_back(&t, totals, sizeof(t))) return false;
     if (t.refused != 0 || t.diagonals * slice_rows<T>() * 2 > t.nonzeros * 3) return true;
-    hipLaunchKernelGGL((slice_diagonals_kernel<T, false>), dim3(l.slices), dim3(kWave), 0, stream, m, base, l.slices, 1u,
-                       row_ptr, col, val, counts, totals, diagonals, vals);
+    run(slice_diagonals_kernel<T, kCount>, 1, counts);
     launch_exclusive_scan_u32(stream, counts, static_cast<uint64_t>(l.slices) + 1, w + l.scan_ws);
     uint32_t found = 0;
     if (!read_back(&found, counts + l.slices, sizeof(found)) || !read_back(&t, totals, sizeof(t))) return false;
     if (t.refused != 0 || found > l.most) return true;
-    hipLaunchKernelGGL((slice_diagonals_kernel<T, true>), dim3(l.slices), dim3(kWave), 0, stream, m, base, l.slices, 1u,
-                       row_ptr, col, val, counts, totals, diagonals, vals);
+    if (val != nullptr) run(slice_diagonals_kernel<T, kCopy>, 1, counts);
+    else run(slice_diagonals_kernel<T, kDescribe>, 1, counts);
     *total = found;
+    if (longest != nullptr) *longest = t.longest;
     return true;
 }
 
 }  // namespace
 
-bool spmv_diagonals_shape(idx_t m, idx_t n, idx_t nnz) {
-    return m != 0 && nnz >= kDiagonalsLeastNonzeros && m < (1u << 31) && n < (1u << 31);
-}
-
-size_t spmv_diagonals_bytes(idx_t m, idx_t nnz, size_t value_bytes) { return diagonals_layout(m, nnz, value_bytes).total; }
-
-bool build_spmv_diagonals(hipStream_t stream, idx_t m, idx_t nnz, idx_t base, const idx_t* row_ptr, const idx_t* col,
-                          const void* val, size_t value_bytes, void* region, uint32_t* total) {
+bool build_slice_diagonals(hipStream_t stream, idx_t m, idx_t nnz, idx_t base, const idx_t* row_ptr, const idx_t* col,
+                           const void* val, size_t value_bytes, void* region, uint32_t* total, uint32_t* longest) {
     *total = 0;
-    return value_bytes == 4 ? build_typed(stream, m, nnz, base, row_ptr, col, static_cast<const float*>(val), region, total)
-                            : build_typed(stream, m, nnz, base, row_ptr, col, static_cast<const double*>(val), region, total);
+    return value_bytes == 4
+               ? build_typed(stream, m, nnz, base, row_ptr, col, static_cast<const float*>(val), region, total, longest)
+               : build_typed(stream, m, nnz, base, row_ptr, col, static_cast<const double*>(val), region, total, longest);
 }
 
 template <typename T>
 bool launch_spmv_diagonals(hipStream_t stream, uint32_t total, const SpmvArgs& a, T alpha, T beta, void* region) {
-    const DiagonalsLayout l = diagonals_layout(a.m, a.nnz, sizeof(T));
+    const SliceDiagonalsLayout l = slice_diagonals_layout(a.m, a.nnz, sizeof(T), true);
     char* w = static_cast<char*>(region);
     const uint32_t xcds = device_topology().xcds;
     auto launch = [&](auto waves, auto stream_values) {
