@@ -437,7 +437,7 @@ mcspStatus_t spmv_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
 // CSC gets the transposed copy [row_ptr m+1 | col_ind nnz][values][csr2csc workspace]
 // (mcsp_spmm_gpu.cpp:818-849); 64-bit index arrays add their narrowed copies at the end.
 struct SpmmLayout {
-    size_t ptr, diagonals, ind, vals, csr2csc_ws, bt, ct, long_ws, narrow, total;
+    size_t ptr, ind, vals, csr2csc_ws, bt, ct, long_ws, narrow, diagonals, total;
     int64_t n_padded;  // leading dimension of the row-major copies of op(B) and C
     bool copy_b, copy_c;
 };
@@ -478,10 +478,6 @@ SpmmLayout spmm_layout(const mcsparseSpMatDescr* A, const mcsparseDnMatDescr* B,
     size_t off = 0;
     if (A->format == MCSPARSE_FORMAT_CSR) {
         if (schedulable(A)) off += mcsp::spmm_schedule_layout(static_cast<idx_t>(A->row_num), static_cast<idx_t>(A->nnz)).total;
-        // (for every order of the operands, so that a call with others leaves it alone)
-        l.diagonals = off;
-        if (diagonals_schedulable(A, value_bytes))
-            off += mcsp::slice_diagonals_layout(static_cast<idx_t>(A->row_num), static_cast<idx_t>(A->nnz), value_bytes, false).total;
     } else if (A->format == MCSPARSE_FORMAT_COO) {
         off += align_up(static_cast<size_t>(A->row_num + 1) * sizeof(idx_t));
     } else if (A->format == MCSPARSE_FORMAT_CSC) {
@@ -507,6 +503,10 @@ SpmmLayout spmm_layout(const mcsparseSpMatDescr* A, const mcsparseDnMatDescr* B,
         off += align_up(mcsp::spmm_long_rows_bytes(static_cast<idx_t>(A->nnz), l.n_padded, value_bytes));
     l.narrow = off;
     off += narrow_bytes(A);
+    // behind what any call with operands of these extents writes, whatever their orders
+    l.diagonals = off;
+    if (l.copy_b && l.copy_c && diagonals_schedulable(A, value_bytes))
+        off += mcsp::slice_diagonals_layout(static_cast<idx_t>(A->row_num), static_cast<idx_t>(A->nnz), value_bytes, false).total;
     l.total = off < kMinBuffer ? kMinBuffer : off;
     return l;
 }
@@ -526,6 +526,8 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
     // strides; the reference runs them as blockIdx.z of one launch, here they are launches in a
     // row on the stream, sharing the scratch buffer.
     const int64_t batches = C->batchCount;
+    // a call with wider operands may write over the diagonals kept for narrower ones: they end there
+    if (A->schedule.buffer == buffer && l.diagonals > A->schedule.diagonals_at) A->schedule.diagonals = 0;
     const bool shared_structure = A->offsetsBatchStride == 0 && A->batchStride == 0;
     const size_t idx_bytes = wide_indices(A) ? sizeof(int64_t) : sizeof(idx_t);
     for (int64_t b = 0; b < batches; ++b) {
@@ -605,7 +607,7 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
         if (l.copy_b && l.copy_c && A->nnz != 0 && (b == 0 || shared_structure) && schedule_of_call(A, buffer) &&
             A->schedule.diagonals != 0 && A->schedule.diagonals_value_bytes == sizeof(T) &&
             mcsp::spmm_diagonals_usable(a.k, a.n, A->schedule.longest_slice, sizeof(T))) {
-            mcsp::launch_spmm_diagonals<T>(h->stream, a, A->schedule.diagonals, buf + l.diagonals, h_alpha, h_beta);
+            mcsp::launch_spmm_diagonals<T>(h->stream, a, A->schedule.diagonals, buf + A->schedule.diagonals_at, h_alpha, h_beta);
             continue;
         }
         T beta_inner = h_beta;
@@ -1196,11 +1198,10 @@ mcsparseStatus_t mcsparseSpMM_preprocess(mcsparseHandle_t handle, mcsparseOperat
     if (!b_image_is_row_major(opB, matB) && matC->order != MCSPARSE_ORDER_ROW &&
         diagonals_schedulable(matA, value_size(matA->valueType))) {
         s.diagonals_value_bytes = value_size(matA->valueType);
+        s.diagonals_at = spmm_layout(matA, matB, matC, opB, s.diagonals_value_bytes).diagonals;
         if (!mcsp::build_slice_diagonals(handle->stream, m, nnz, static_cast<idx_t>(matA->idxBase), ia.rows, ia.cols, nullptr,
                                          s.diagonals_value_bytes,
-                                         static_cast<char*>(externalBuffer) +
-                                             spmm_layout(matA, matB, matC, opB, s.diagonals_value_bytes).diagonals,
-                                         &s.diagonals, &s.longest_slice))
+                                         static_cast<char*>(externalBuffer) + s.diagonals_at, &s.diagonals, &s.longest_slice))
             return to_public_status(MCSP_STATUS_INTERNAL_ERROR);
         if (!mcsp::spmm_diagonals_usable(static_cast<idx_t>(matA->col_num), static_cast<idx_t>(matC->col_num), s.longest_slice,
                                          s.diagonals_value_bytes))

@@ -99,9 +99,10 @@ struct SpmmSchedule {
     bool blocks = false;   // the schedule holds diagonal blocks (spmm_blocks.hip) instead of merged lists
     uint32_t longest_group = 0;  // blocks: the most nonzeros in one group of rows (strips: in one strip)
     uint32_t stride = 0;   // blocks: != 0 says the groups are strips this many rows apart (spmm_strips.hip)
-    // beside that (whether useful or not), for column-major operands: the diagonals of slices of rows (spmm_diagonals.hip),
-    // behind the region of the above; 0: none
+    // beside that (whether useful or not), for column-major operands: the diagonals of slices of rows (spmm_diagonals.hip), at
+    // diagonals_at of the buffer; 0: none
     uint32_t diagonals = 0;
+    size_t diagonals_at = 0;
     uint32_t longest_slice = 0;  // most nonzeros of a slice
     size_t diagonals_value_bytes = 0;  // the slices' length goes with it
 };

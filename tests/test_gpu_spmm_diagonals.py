@@ -99,6 +99,22 @@ def test_row_major_call_in_between_leaves_them_alone(torch_gpu, handle, oracle):
     call.check(oracle, what="column-major again")
 
 
+def test_wider_operands_in_the_same_buffer_end_them(torch_gpu, handle, oracle):
+    torch = torch_gpu
+    a = grid((41, 37, 29), BOX, np.float32, 7)
+    call, wide = Call(torch, handle, a, 6), Call(torch, handle, a, 30, seed=3)
+    assert wide.buf.numel() > call.buf.numel()
+    call.buf = wide.buf
+    assert api.spmm_preprocess(*call.args, call.buf) == api.STATUS_SUCCESS
+    call.check(oracle)
+    args = list(wide.args)
+    args[4] = call.mat  # the same matrix, the buffer that holds its diagonals
+    wide.args = tuple(args)
+    wide.check(oracle, what="wider")
+    assert call.mat.spmm_diagonals() == 0
+    call.check(oracle, what="narrow again")
+
+
 def test_matrices_without_such_rows(torch_gpu, handle, oracle):
     a = grid((41, 37, 29), BOX, np.float64, 9)
     row = slice(int(a.ptr[20000]), int(a.ptr[20001]))
