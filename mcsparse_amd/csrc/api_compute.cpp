@@ -437,7 +437,7 @@ mcspStatus_t spmv_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
 // CSC gets the transposed copy [row_ptr m+1 | col_ind nnz][values][csr2csc workspace]
 // (mcsp_spmm_gpu.cpp:818-849); 64-bit index arrays add their narrowed copies at the end.
 struct SpmmLayout {
-    size_t ptr, ind, vals, csr2csc_ws, bt, ct, long_ws, narrow, diagonals, total;
+    size_t ptr, band_ws, ind, vals, csr2csc_ws, bt, ct, long_ws, narrow, diagonals, total;
     int64_t n_padded;  // leading dimension of the row-major copies of op(B) and C
     bool copy_b, copy_c;
 };
@@ -477,9 +477,12 @@ SpmmLayout spmm_layout(const mcsparseSpMatDescr* A, const mcsparseDnMatDescr* B,
     SpmmLayout l = {};
     size_t off = 0;
     if (A->format == MCSPARSE_FORMAT_CSR) {
+        l.band_ws = off;
         if (schedulable(A)) off += mcsp::spmm_schedule_layout(static_cast<idx_t>(A->row_num), static_cast<idx_t>(A->nnz)).total;
     } else if (A->format == MCSPARSE_FORMAT_COO) {
         off += align_up(static_cast<size_t>(A->row_num + 1) * sizeof(idx_t));
+        l.band_ws = off;
+        off += align_up(static_cast<size_t>(A->nnz) * sizeof(idx_t));
     } else if (A->format == MCSPARSE_FORMAT_CSC) {
         l.ind = static_cast<size_t>(A->row_num + 1) * sizeof(idx_t);
         off += align_up(static_cast<size_t>(A->row_num + 1 + A->nnz) * sizeof(idx_t));
@@ -601,6 +604,11 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
             } else {
                 a.long_ws = buf + l.long_ws;
                 a.long_n = l.n_padded;
+                // where a schedule would lie (there is none for such a matrix, unless the caller has set its kernels), the sort
+                // of a CSC input has ended, or a COO input has room of its own
+                if (A->format == MCSPARSE_FORMAT_CSC) a.band_ws = buf + l.csr2csc_ws;
+                else if (A->format == MCSPARSE_FORMAT_COO) a.band_ws = buf + l.band_ws;
+                else if (schedulable(A) && !schedule_matches(A, buffer)) a.band_ws = buf + l.band_ws;
             }
         }
         // both operands column-major and rows that share diagonals: nothing is transposed

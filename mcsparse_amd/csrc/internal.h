@@ -399,6 +399,7 @@ struct SpmmArgs {
     const uint32_t* long_apart = nullptr;
     void* long_ws = nullptr;
     int64_t long_n = 0;
+    void* band_ws = nullptr;  // nnz words more for them, or null
 };
 template <typename T>
 void launch_spmm(hipStream_t stream, const SpmmArgs& a, T alpha, T beta);

@@ -25,6 +25,7 @@ struct LongCounters {
     // not zero: the listed rows are taken apart, since there is one of more than kSpmmLongRow nonzeros (on a line of its
     // own: a store among the adds to the counters makes the find kernel wait, 16.5 -> 27.5 us on a million rows)
     alignas(128) uint32_t apart;
+    uint32_t unsorted;  // not zero: a piece whose columns do not ascend
 };
 static_assert(sizeof(LongCounters) <= 2 * kAlign, "what the layout has room for");
 
@@ -33,6 +34,7 @@ __global__ void spmm_long_zero_kernel(LongCounters* c, bool known) {
     c->rows = 0;
     c->slots = 0;
     c->apart = known ? 1 : 0;
+    c->unsorted = 0;
 }
 
 // item: {row, piece, pieces of the row, first row of partial sums of the row (unused for one piece)}
@@ -125,6 +127,219 @@ __global__ __launch_bounds__(kBlock) void spmm_long_find_kernel(idx_t m, idx_t l
         const uint4 e = s_list[k];
         write_long_row(e.x, e.y, s_base[0] + e.z, s_base[1] + e.w, s_base[2] + s_list_row[k], items, rows, cap_items,
                        cap_rows, cap_slots);
+    }
+}
+
+// ---- bands of op(B) --------------------------------------------------------------------------------------------
+// The long rows of a matrix name every row of op(B) many times (a million power-law rows: 20 times), but a piece walks all of
+// op(B), so each time it comes from behind the L2s.  Where op(B) is larger than they are, the pieces are taken band by band: a
+// band is a stretch of rows of op(B) that fits an L2, an XCD works on every eighth band, and a wavefront takes the
+// nonzeros that one piece has in one band, which lie side by side where columns ascend.  Their sum is a row of partial sums,
+// added up per row in the order of pieces and bands.  Whether and how is decided on the device, from the number of pieces
+// found, so that every way to a product comes to the same sums.
+// A million power-law rows, 32 fp32 columns (20 M of 28 M nonzeros in rows of more than 256), microseconds: pieces whole 327,
+// band by band 225 and 30 for the bounds, 560 -> 507 a call; 16 columns 520 -> 457; 3 M rows, 20 columns 1942 -> 1466; 400 K
+// rows, 11 fp64 columns 258 -> 227.  Half of the rows of op(B) still come from behind the L2 (its wavefronts are not all in
+// one band); bands of 2 MB bring that down to a quarter and the nonzeros of a pair to 32, half a round: 524.  Bands of 8 MB:
+// 549.  Rows of op(B) wider than a panel of kBandLanes lanes keep their pieces whole: A's long rows would be read once per
+// panel (100 fp32 columns: 1763 us whole, 2740 in panels).
+constexpr uint64_t kBandBytes = size_t(4) << 20;  // of op(B)
+constexpr uint32_t kBandStretches = 8;            // bands are dealt to so many XCDs
+constexpr idx_t kBandLeastNonzeros = 1u << 20;
+constexpr uint64_t kBandLeastBytes = size_t(16) << 20;
+constexpr int kBandLanes = 8;
+struct BandSpace {
+    void* ws;            // null: no room, or no need
+    uint64_t bytes;
+    idx_t k;             // rows of op(B)
+    uint32_t row_bytes, sum_bytes;  // of a row of op(B), and of a row of partial sums
+};
+constexpr uint32_t kBandTake = 8;  // items a wavefront takes off its XCD's counter at a time
+struct BandPlan {
+    uint32_t bands, items;  // 0 bands: pieces are taken whole
+    uint32_t* taken;        // [stretch], a line each: (band, item) pairs that have been taken
+    uint32_t* bounds;       // [item][band]: the item's first nonzero in that band or a later one; and behind the last band
+    void* sums;             // [item][band]
+    float of_column;        // band = column times this (whatever the rounding: it ascends with the column)
+};
+__device__ __forceinline__ BandPlan band_plan(const BandSpace& s, const LongCounters* __restrict__ c, uint32_t cap_items) {
+    BandPlan p = {0, 0, nullptr, nullptr, nullptr, 0.0f};
+    if (s.ws == nullptr || c->apart == 0 || c->unsorted != 0) return p;
+    p.items = min(c->items, cap_items);
+    if (p.items == 0) return p;
+    const uint64_t wanted = (static_cast<uint64_t>(s.k) * s.row_bytes + kBandBytes - 1) / kBandBytes;
+    uint64_t bands = (wanted + kBandStretches - 1) / kBandStretches * kBandStretches;
+    auto bounds_bytes = [&](uint64_t n) { return (p.items * (n + 1) * sizeof(uint32_t) + kAlign - 1) / kAlign * kAlign; };
+    constexpr uint64_t kTakenBytes = kBandStretches * kAlign;
+    while (bands != 0 && kTakenBytes + bounds_bytes(bands) + bands * p.items * s.sum_bytes > s.bytes) bands -= kBandStretches;
+    if (2 * bands < wanted) return p;  // (bands of twice the size still keep half of their rows)
+    p.bands = static_cast<uint32_t>(bands);
+    p.taken = static_cast<uint32_t*>(s.ws);
+    p.bounds = p.taken + kTakenBytes / sizeof(uint32_t);
+    p.sums = reinterpret_cast<char*>(p.bounds) + bounds_bytes(bands);
+    p.of_column = static_cast<float>(bands) / static_cast<float>(s.k);
+    return p;
+}
+
+// The bounds of every item, a workgroup at a time.
+__global__ __launch_bounds__(kBlock) void spmm_long_bounds_kernel(BandSpace space, idx_t base, idx_t nnz,
+                                                                  const idx_t* __restrict__ row_ptr,
+                                                                  const idx_t* __restrict__ col, LongCounters* c,
+                                                                  const uint4* __restrict__ items, uint32_t cap_items) {
+    const BandPlan plan = band_plan(space, c, cap_items);  // (a workgroup that sees another's `unsorted` may stop early)
+    if (plan.bands == 0) return;  // whole workgroup
+    constexpr int kAtOnce = 2, kQuad = 4;
+    typedef idx_t quad_t __attribute__((ext_vector_type(kQuad)));
+    typedef quad_t element_aligned __attribute__((aligned(sizeof(idx_t))));
+    if (blockIdx.x == 0 && threadIdx.x < kBandStretches) plan.taken[threadIdx.x * (kAlign / sizeof(uint32_t))] = 0;
+    auto band_of = [&](idx_t column) {
+        return min(static_cast<uint32_t>(static_cast<float>(column - base) * plan.of_column), plan.bands - 1);
+    };
+    for (uint32_t it = blockIdx.x; it < plan.items; it += gridDim.x) {
+        const uint4 item = items[it];
+        uint32_t* bounds = plan.bounds + static_cast<uint64_t>(it) * (plan.bands + 1);
+        const idx_t row_end = min(row_ptr[item.x + 1] - base, nnz);
+        const idx_t start = min(row_ptr[item.x] - base + item.y * kSpmmLongChunk, row_end);
+        const idx_t end = item.z != 0 ? min(start + static_cast<idx_t>(kSpmmLongChunk), row_end) : start;
+        if (start == end) {  // whole workgroup: a row that found no room
+            for (uint32_t b = threadIdx.x; b <= plan.bands; b += kBlock) bounds[b] = start;
+            continue;
+        }
+        bool unsorted = false;
+        // neighbouring nonzeros by fours to a thread: the one before its first is the thread's before
+        for (idx_t j0 = start + threadIdx.x * kQuad; j0 < end; j0 += kBlock * kQuad * kAtOnce) {
+            quad_t here[kAtOnce];
+            idx_t before[kAtOnce];
+#pragma unroll
+            for (int u = 0; u < kAtOnce; ++u) {
+                const idx_t j = j0 + u * kBlock * kQuad;
+                if (j + kQuad <= end) {
+                    here[u] = *reinterpret_cast<const element_aligned*>(col + j);
+                } else {
+#pragma unroll
+                    for (int q = 0; q < kQuad; ++q) here[u][q] = col[min(j + q, end - 1)];
+                }
+                before[u] = col[min(j, end) - (j != start ? 1 : 0)];
+            }
+#pragma unroll
+            for (int u = 0; u < kAtOnce; ++u) {
+                idx_t last = before[u];
+                uint32_t last_band = band_of(last);
+#pragma unroll
+                for (int q = 0; q < kQuad; ++q) {
+                    const idx_t j = j0 + u * kBlock * kQuad + q;
+                    if (j >= end) break;
+                    unsorted |= here[u][q] < last;
+                    const uint32_t band = band_of(here[u][q]);
+                    for (uint32_t b = j == start ? 0 : last_band + 1; b <= band; ++b) bounds[b] = j;
+                    if (j == end - 1) {
+                        for (uint32_t b = band + 1; b <= plan.bands; ++b) bounds[b] = end;
+                    }
+                    last = here[u][q];
+                    last_band = band;
+                }
+            }
+        }
+        if (unsorted) c->unsorted = 1;
+    }
+}
+
+// A wavefront's share of the bands: kBandTake pairs of band and item at a time.  A round is up to 64 nonzeros of a pair, one
+// asked for by every lane: nonzero t goes to lane group t % G, so that the groups load equally many rows of op(B).  The
+// nonzeros of the next round, often the next pair's, are asked for before the rows of this one.
+template <typename T, int LR, int V>
+__device__ __forceinline__ void take_bands(const BandPlan& plan, const LaneColumns& own, idx_t base, const idx_t* __restrict__ col,
+                                           const T* __restrict__ val, const T* __restrict__ B, int64_t ldb, int64_t ld_partials) {
+    constexpr uint32_t G = kWave / LR;
+    const uint32_t lane = threadIdx.x % kWave, group = lane / LR, place = lane % LR * G + group;
+    const uint32_t stretch = blockIdx.x % kBandStretches;
+    const uint32_t all = plan.bands / kBandStretches * plan.items;  // pairs of the stretch, band after band
+    uint32_t* taken = plan.taken + stretch * (kAlign / sizeof(uint32_t));
+    T* sums = static_cast<T*>(plan.sums);
+    const char* B_bytes = reinterpret_cast<const char*>(B);
+    const uint32_t lane_off = static_cast<uint32_t>(own.first * sizeof(T)), ldb_bytes = static_cast<uint32_t>(ldb * sizeof(T));
+    auto take = [&]() {
+        uint32_t at = 0;
+        if (lane == 0) at = atomicAdd(taken, kBandTake);
+        return at;
+    };
+    uint32_t next = take();
+    while (true) {
+        const uint32_t from = __builtin_amdgcn_readfirstlane(next);
+        if (from >= all) break;  // whole wavefront
+        next = take();  // on its way while this share is worked on
+        const uint32_t pairs = min(kBandTake, all - from);
+        // lane p keeps the bounds of pair p
+        const uint32_t mine = from + min(lane, pairs - 1), turn = mine / plan.items, it = mine - turn * plan.items;
+        const uint64_t at = static_cast<uint64_t>(it) * (plan.bands + 1) + turn * kBandStretches + stretch;
+        const uint32_t my_begin = plan.bounds[at], my_end = plan.bounds[at + 1];
+        const uint32_t my_sum = it * plan.bands + turn * kBandStretches + stretch;
+        unsigned long long left = __ballot(lane < pairs && my_begin < my_end);
+        if (left == 0) continue;  // whole wavefront
+        uint32_t p = __builtin_ctzll(left);
+        left &= left - 1;
+        uint32_t j = __builtin_amdgcn_readlane(my_begin, p), end = __builtin_amdgcn_readlane(my_end, p);
+        idx_t c_next = col[min(j + place, end - 1)];
+        T a_next = val[min(j + place, end - 1)];
+        T acc[V];
+#pragma unroll
+        for (int i = 0; i < V; ++i) acc[i] = T(0);
+        while (true) {  // a round of pair p
+            const uint32_t count = min(end - j, static_cast<uint32_t>(kWave));
+            const uint32_t roff = (c_next - base) * ldb_bytes;
+            const T aa = a_next;
+            const bool last = j + kWave >= end;
+            const uint32_t p_now = p;
+            if (last) {
+                if (left != 0) {
+                    p = __builtin_ctzll(left);
+                    left &= left - 1;
+                    j = __builtin_amdgcn_readlane(my_begin, p);
+                    end = __builtin_amdgcn_readlane(my_end, p);
+                } else {
+                    p = kWave;  // none
+                }
+            } else {
+                j += kWave;
+            }
+            c_next = col[min(j + place, end - 1)];
+            a_next = val[min(j + place, end - 1)];
+            Vec<T, V> b[LR];
+            static_for<LR>([&](auto k) {
+                constexpr int kk = decltype(k)::value;
+                if (kk * G < count)  // the same for the wavefront
+                    b[kk] = load_row<T, V>(reinterpret_cast<const T*>(B_bytes + (group_bcast<LR, kk>(roff) + lane_off)));
+            });
+            T of_round[V];  // (a sum of its own, so that a pair of thousands is no chain of hundreds)
+#pragma unroll
+            for (int i = 0; i < V; ++i) of_round[i] = T(0);
+            static_for<LR>([&](auto k) {
+                constexpr int kk = decltype(k)::value;
+                if (kk * G + group < count) {  // a lane without a nonzero stays out: 0 * inf would be NaN
+                    const T a = group_bcast<LR, kk>(aa);
+#pragma unroll
+                    for (int i = 0; i < V; ++i) of_round[i] += a * b[kk].v[i];
+                }
+            });
+#pragma unroll
+            for (int i = 0; i < V; ++i) acc[i] += of_round[i];
+            if (!last) continue;
+#pragma unroll
+            for (int i = 0; i < V; ++i) {
+#pragma unroll
+                for (int off = LR; off < kWave; off <<= 1) acc[i] += __shfl_xor(acc[i], off, kWave);
+            }
+            if (group == 0 && own.any) {
+                T* out = sums + static_cast<int64_t>(__builtin_amdgcn_readlane(my_sum, p_now)) * ld_partials + own.first;
+#pragma unroll
+                for (int i = 0; i < V; ++i) {
+                    if (i >= own.skip) out[i] = acc[i];
+                }
+            }
+            if (p == kWave) break;
+#pragma unroll
+            for (int i = 0; i < V; ++i) acc[i] = T(0);
+        }
     }
 }
 
@@ -225,13 +440,19 @@ __global__ __launch_bounds__(kBlock) void spmm_long_stretch_kernel(idx_t n, idx_
                                                                    bool c_row_major, T alpha, T beta,
                                                                    const LongCounters* __restrict__ c,
                                                                    const uint4* __restrict__ items, uint32_t cap_items,
-                                                                   T* __restrict__ partials, int64_t ld_partials, idx_t nnz) {
+                                                                   T* __restrict__ partials, int64_t ld_partials, idx_t nnz,
+                                                                   BandSpace space) {
     constexpr int kWaves = kBlock / kWave;
     __shared__ T s_sum[kWaves][LR * V];
     const uint32_t lane = threadIdx.x % LR;
     const uint32_t group = threadIdx.x / LR;
     const uint32_t wave = threadIdx.x / kWave;
     const LaneColumns own = lane_columns<V>((static_cast<uint64_t>(blockIdx.y) * LR + lane) * V, n);
+    const BandPlan plan = band_plan(space, c, cap_items);
+    if (plan.bands != 0) {  // the same for all workgroups
+        if constexpr (LR <= kBandLanes) take_bands<T, LR, V>(plan, own, base, col, val, B, ldb, ld_partials);
+        return;
+    }
     const uint32_t count = c->apart != 0 ? min(c->items, cap_items) : 0u;
     for (uint32_t it = blockIdx.x; it < count; it += gridDim.x) {
         const uint4 item = items[it];
@@ -283,8 +504,58 @@ __global__ __launch_bounds__(kBlock) void spmm_long_reduce_kernel(idx_t n, T* __
                                                                   bool c_row_major, T alpha, T beta,
                                                                   const LongCounters* __restrict__ c,
                                                                   const uint4* __restrict__ rows, uint32_t cap_rows,
-                                                                  const T* __restrict__ partials, int64_t ld_partials) {
+                                                                  const T* __restrict__ partials, int64_t ld_partials,
+                                                                  const uint4* __restrict__ items, uint32_t cap_items,
+                                                                  BandSpace space) {
     const uint64_t per_row = (static_cast<uint64_t>(n) + V - 1) / V;
+    const BandPlan plan = band_plan(space, c, cap_items);
+    if (plan.bands != 0) {  // the same for all workgroups: the partial sums of all pieces of a row, band by band
+        constexpr uint32_t kLanes = 8, kGroups = kWave / kLanes;
+        static_assert(kBandStretches % kGroups == 0, "whole rounds");
+        const T* sums = static_cast<const T*>(plan.sums);
+        const uint32_t lane = threadIdx.x % kLanes, group = threadIdx.x % kWave / kLanes;
+        const uint64_t panels = (per_row + kLanes - 1) / kLanes;
+        for (uint64_t w = static_cast<uint64_t>(blockIdx.x) * (kBlock / kWave) + threadIdx.x / kWave; w < plan.items * panels;
+             w += static_cast<uint64_t>(gridDim.x) * (kBlock / kWave)) {
+            const uint32_t it = static_cast<uint32_t>(w / panels);
+            const uint4 item = items[it];
+            if (item.y != 0 || item.z == 0) continue;  // whole wavefront: not the first piece of its row
+            const LaneColumns own = lane_columns<V>((w % panels * kLanes + lane) * V, n);
+            T sum[V];
+#pragma unroll
+            for (int i = 0; i < V; ++i) sum[i] = T(0);
+            for (uint32_t j = 0; j < item.z; ++j) {
+                const uint32_t* bounds = plan.bounds + static_cast<uint64_t>(it + j) * (plan.bands + 1);
+                const T* in = sums + static_cast<int64_t>(it + j) * plan.bands * ld_partials + own.first;
+                for (uint32_t b0 = 0; b0 < plan.bands; b0 += kWave) {
+                    // the bands that hold nonzeros of the piece (for the others nothing was written), the groups in turn
+                    const uint32_t b = min(b0 + threadIdx.x % kWave, plan.bands - 1);
+                    const bool holds = b0 + threadIdx.x % kWave < plan.bands && bounds[b] != bounds[b + 1];
+                    const unsigned long long holding = __ballot(holds);
+                    const uint32_t rank = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(holding >> 32),
+                                                                    __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(holding), 0u));
+                    // lane r learns the r-th of them (lanes without one send to the last lane, where nobody looks unless all hold)
+                    const uint32_t bands_held = __popcll(holding);
+                    const uint32_t band = __builtin_amdgcn_ds_permute(static_cast<int>((holds ? rank : kWave - 1) * 4), static_cast<int>(b));
+                    for (uint32_t r0 = 0; r0 < bands_held; r0 += kGroups) {
+                        const uint32_t r = min(r0 + group, bands_held - 1);
+                        const Vec<T, V> part = load_row<T, V>(in + static_cast<int64_t>(__shfl(band, r, kWave)) * ld_partials);
+                        if (r0 + group < bands_held) {
+#pragma unroll
+                            for (int i = 0; i < V; ++i) sum[i] += part.v[i];
+                        }
+                    }
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < V; ++i) {
+#pragma unroll
+                for (int off = kLanes; off < kWave; off <<= 1) sum[i] += __shfl_xor(sum[i], off, kWave);
+            }
+            if (group == 0 && own.any) store_c<T, V>(C, ldc, c_row_major, item.x, own.first, sum, alpha, beta, own.skip);
+        }
+        return;
+    }
     const uint64_t work = c->apart != 0 ? static_cast<uint64_t>(min(c->rows, cap_rows)) * per_row : 0;
     for (uint64_t w = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; w < work;
          w += static_cast<uint64_t>(gridDim.x) * kBlock) {
@@ -367,15 +638,28 @@ void launch_spmm_long_rows(hipStream_t stream, const SpmmArgs& a, T alpha, T bet
     while (lanes < kWave && lanes < lanes_needed) lanes *= 2;
     const uint32_t panels = static_cast<uint32_t>((lanes_needed + lanes - 1) / lanes);
     // pieces are few (a 2048th of the nonzeros at most): a grid that lets every compute unit hold several
+    static_assert(2048 % kBandStretches == 0, "workgroups of a launch");
     const dim3 grid(2048, panels);
     const uint32_t reduce_blocks = 1024;
+    // op(B) beyond the L2s, and nonzeros enough for the launch in front
+    const bool stretched = wide && lanes >= 4 && narrow_offsets(a, sizeof(T));
+    BandSpace space = {nullptr, 0, 0, 0, 0};
+    if (stretched && a.band_ws != nullptr && a.nnz >= kBandLeastNonzeros &&
+        static_cast<uint64_t>(a.k) * a.n * sizeof(T) >= kBandLeastBytes && lanes_needed <= kBandLanes) {
+        space.ws = a.band_ws;
+        space.bytes = static_cast<uint64_t>(a.nnz) * sizeof(idx_t);
+        space.k = a.k;
+        space.row_bytes = static_cast<uint32_t>(lanes_needed * 16);
+        space.sum_bytes = static_cast<uint32_t>(l.ld_partials * sizeof(T));
+        hipLaunchKernelGGL(spmm_long_bounds_kernel, dim3(8192), dim3(kBlock), 0, stream, space, a.base, a.nnz, a.row_ptr, a.col,
+                           reinterpret_cast<LongCounters*>(w + l.counters), items, l.cap_items);
+    }
     auto stretches = [&](auto lr) {
         constexpr int LR = decltype(lr)::value;
-        hipLaunchKernelGGL((spmm_long_stretch_kernel<T, LR, kWide>), grid, dim3(kBlock), 0, stream, a.n, a.base, a.row_ptr,
-                           a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta, c, items, l.cap_items, partials,
-                           l.ld_partials, a.nnz);
+        hipLaunchKernelGGL((spmm_long_stretch_kernel<T, LR, kWide>), grid, dim3(kBlock), 0, stream, a.n, a.base, a.row_ptr, a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta, c, items, l.cap_items,
+                           partials, l.ld_partials, a.nnz, space);
     };
-    if (wide && lanes >= 4 && narrow_offsets(a, sizeof(T))) {
+    if (stretched) {
         if (lanes == 4) stretches(std::integral_constant<int, 4>{});
         else if (lanes == 8) stretches(std::integral_constant<int, 8>{});
         else if (lanes == 16) stretches(std::integral_constant<int, 16>{});
@@ -392,10 +676,12 @@ void launch_spmm_long_rows(hipStream_t stream, const SpmmArgs& a, T alpha, T bet
     }
     if (wide) {
         hipLaunchKernelGGL((spmm_long_reduce_kernel<T, kWide>), dim3(reduce_blocks), dim3(kBlock), 0, stream, a.n, C,
-                           a.ldc, a.c_row_major, alpha, beta, c, rows, l.cap_rows, partials, l.ld_partials);
+                           a.ldc, a.c_row_major, alpha, beta, c, rows, l.cap_rows, partials, l.ld_partials, items, l.cap_items,
+                           space);
     } else {
         hipLaunchKernelGGL((spmm_long_reduce_kernel<T, 1>), dim3(reduce_blocks), dim3(kBlock), 0, stream, a.n, C, a.ldc,
-                           a.c_row_major, alpha, beta, c, rows, l.cap_rows, partials, l.ld_partials);
+                           a.c_row_major, alpha, beta, c, rows, l.cap_rows, partials, l.ld_partials, items, l.cap_items,
+                           space);
     }
 }
 

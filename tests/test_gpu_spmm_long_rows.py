@@ -199,3 +199,83 @@ def test_every_way_to_a_product_gives_the_same_bits(torch_gpu, oracle, dtype, c_
     for kind in ("captured", "coo", "csc", "forced"):
         assert np.array_equal(product(kind), want), kind
     handle.destroy()
+
+
+def banded_matrix(dtype, k=300000, base=0, seed=31):
+    """20,000 short rows and 1,200 of 257 to 9,000 nonzeros, over a k large enough that the long ones are taken in bands of
+    op(B) (16 MB from 54 bytes a row on)."""
+    rng = np.random.default_rng(seed)
+    lengths = np.concatenate([rng.integers(0, 8, 20000), rng.integers(257, 2200, 1150), rng.integers(4000, 9001, 50)])
+    rng.shuffle(lengths)
+    ptr = np.concatenate([[0], np.cumsum(lengths)])
+    rows = np.repeat(np.arange(lengths.size), lengths)
+    col = np.sort(rng.integers(0, k, rows.size) + rows * k) - rows * k  # ascending, now and then a column twice
+    return wl.Csr(lengths.size, k, ptr, col, rng.uniform(-1, 1, rows.size).astype(dtype), 0).with_base(base)
+
+
+@pytest.mark.parametrize("dtype,n,base", [(np.float32, 14, 0), (np.float32, 16, 1), (np.float32, 29, 0), (np.float32, 32, 0),
+                                          (np.float64, 7, 1), (np.float64, 16, 0)])
+def test_long_rows_in_bands_of_the_operand(torch_gpu, handle, oracle, dtype, n, base):
+    a = banded_matrix(dtype, base=base)
+    assert a.nnz >= 1 << 20 and a.n * n * a.val.itemsize >= 16 << 20
+    check(torch_gpu, handle, oracle, a, n, 1.25, 0.0, pad_b=n % 3)
+    check(torch_gpu, handle, oracle, a, n, 1.25, -0.5, seed=1, c_order=api.ORDER_COL)
+
+
+@pytest.mark.parametrize("how", ["one row descends", "all columns in one band", "long rows name the ends of op(B)"])
+def test_long_rows_whose_bands_are_unlike(torch_gpu, handle, oracle, how):
+    a = banded_matrix(np.float32)
+    long_rows = np.nonzero(a.row_lengths() > 256)[0]
+    for r in long_rows[:1] if how == "one row descends" else long_rows:
+        span = slice(a.ptr[r], a.ptr[r + 1])
+        if how == "one row descends":
+            a.col[span] = a.col[span][::-1]
+        elif how == "all columns in one band":
+            a.col[span] = 150000 + np.arange(span.stop - span.start) % 1000
+            a.col[span].sort()
+        else:
+            a.col[span] = np.where(np.arange(span.stop - span.start) < 100, 0, a.n - 1)
+    check(torch_gpu, handle, oracle, a, 32, -1.5, 0.5)
+
+
+def test_every_way_to_bands_gives_the_same_bits(torch_gpu, oracle):
+    torch = torch_gpu
+    side = torch.cuda.Stream()
+    handle = api.Handle(stream=side.cuda_stream)
+    a, n = banded_matrix(np.float32), 24
+    rng = np.random.default_rng(5)
+    B = dev(torch, rng.uniform(-1, 1, (a.n, n)).astype(np.float32))
+    ptr, col, val = dev(torch, a.ptr), dev(torch, a.col), dev(torch, a.val)
+    rows = dev(torch, np.repeat(np.arange(a.m, dtype=np.int32), a.row_lengths()))
+    t_ptr, t_row, t_val = oracle.csr2csc(a.m, a.n, 0, a.ptr, a.col, a.val, method="counting")
+    t_ptr, t_row, t_val = dev(torch, t_ptr.astype(np.int32)), dev(torch, t_row.astype(np.int32)), dev(torch, t_val)
+    results = {}
+    for kind in ("csr", "captured", "coo", "csc", "csr again"):
+        if kind == "coo":
+            mat = api.SpMat(a.m, a.n, a.nnz, rows, col, val, fmt=api.FORMAT_COO)
+        elif kind == "csc":
+            mat = api.SpMat(a.m, a.n, a.nnz, t_ptr, t_row, t_val, fmt=api.FORMAT_CSC)
+        else:
+            mat = api.SpMat(a.m, a.n, a.nnz, ptr, col, val)
+        C = torch.full((a.m, n), 3.0, device="cuda")
+        call = (handle, api.OP_N, api.OP_N, 1.25, mat, api.DnMat(a.n, n, n, B), 0.0, api.DnMat(a.m, n, n, C), api.R_32F)
+        st, size = api.spmm_buffer_size(*call)
+        assert st == 0
+        buf = torch.full((size,), 0xFF, dtype=torch.uint8, device="cuda")  # (NaN wherever sums are read that were not written)
+        torch.cuda.synchronize()
+        if kind == "captured":
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=side):
+                assert api.spmm(*call, buf) == 0
+            for _ in range(3):
+                C.fill_(9.0)
+                torch.cuda.synchronize()
+                graph.replay()
+                torch.cuda.synchronize()
+        else:
+            assert api.spmm(*call, buf) == 0
+            torch.cuda.synchronize()
+        results[kind] = C.cpu().numpy()
+    for kind, got in results.items():
+        assert np.array_equal(got, results["csr"]), kind
+    handle.destroy()
