@@ -16,7 +16,8 @@
 //      a linear stream again.  Where the keys begin (col_ptr of a CSC) falls out of its digit counts.
 // A key loses the bits that its place already tells: at most 16 of them travel to step 2, 8 or 16 to step 3.
 // A sort by two keys (the index sorts) partitions by the major key alone: step 3 orders a bucket by the minor key first,
-// then by what is left of the major one, in passes of up to eight bits that stay in LDS.
+// then by what is left of the major one, in passes of up to eight bits that stay in LDS.  Where the two have room in one
+// word (sort_packs) it is the words that are ordered.
 // Buckets that do not fit LDS (popular keys) are sorted in chunks by oversize_kernel, which finds nothing to do elsewhere;
 // inputs that would make such buckets only (few keys) are left to the LSD passes.
 #include "partition_device.h"
@@ -45,6 +46,7 @@ struct EntrySource {
     // leaves its indices in an array of their own and sets *wide
     bool relative;
     uint32_t* wide;
+    uint32_t minor_bits;  // plain, packed entries: bits of the index, which lies below the key's rest
 };
 
 // The order of tiles over the workgroups: an XCD takes a contiguous range, so the table words of neighbouring tiles,
@@ -236,9 +238,9 @@ __global__ __launch_bounds__(THREADS) void partition_kernel(EntrySource in, uint
     if constexpr (VB != 0 && !kValuesEarly) load_values();
     const uint64_t out = static_cast<uint64_t>(tile) * kPlaces;
     if constexpr (packed_entries<Key>()) {
-        static_assert(KIND == kCsr, "packed entries");
+        static_assert(KIND != kProducts, "no index travels with a product");
         uint32_t origin = 0u - in.base;
-        if (in.relative) {  // (shift != 0: there is a second step)
+        if (KIND == kCsr && in.relative) {  // (shift != 0: there is a second step)
             origin = before - 1;
             if (inside >> (32 - shift) != 0) {  // whole workgroup
 #pragma unroll
@@ -249,7 +251,10 @@ __global__ __launch_bounds__(THREADS) void partition_kernel(EntrySource in, uint
         }
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
-            key[i] = (key[i] & ((1u << shift) - 1u)) | (aux[i] - origin) << shift;
+            const uint32_t rest = key[i] & ((1u << shift) - 1u);
+            // (a minor key that is out of range must not reach the bits above it)
+            key[i] = KIND == kCsr ? rest | (aux[i] - origin) << shift
+                                  : rest << in.minor_bits | (aux[i] & ((1u << in.minor_bits) - 1u));
             forget(key[i]);
         }
         store_packed<VB, ITEMS, THREADS, kPlaces>(s_buf, count, dest, keys_out, vals_out, out, [&](int i) { return key[i]; }, val);
@@ -437,6 +442,12 @@ __device__ __forceinline__ SortPass sort_pass(const SortTables& t, uint32_t p) {
     return s;
 }
 
+// The same over the words of packed pairs.
+__device__ __forceinline__ SortPass word_pass(const SortTables& t, uint32_t p) {
+    const uint32_t shift = p * t.oversize_width;
+    return {false, shift, min(t.oversize_width, t.minor_bits + t.d3 - shift)};
+}
+
 constexpr int kBucketThreads = 512, kBucketItems = 12;
 constexpr uint32_t kBucketRoom = kBucketThreads * kBucketItems;  // entries of the largest bucket that is sorted in LDS
 constexpr uint32_t kPassBits = 8;  // the most a pass of step 3 takes
@@ -537,8 +548,9 @@ __global__ __launch_bounds__(kMapBlock) void tile_map_kernel(SortTables t) {
 }
 
 // 118 M entries (16 bytes each): 0.99 GB read, 1.10 GB written in 415 us.
-// Key: the type the rest of a key travels in from here on, or the packed entries' word on both sides.
-template <int VB, typename Key>
+// Key: the type the rest of a key travels in from here on, or the packed entries' word (on both sides; PAIRS, a sort by two
+// keys: only from here on).
+template <int VB, typename Key, bool PAIRS>
 __global__ __launch_bounds__(kSecondThreads) void repartition_kernel(SortTables t, const void* __restrict__ keys_in,
                                                                      const uint32_t* __restrict__ aux_in,
                                                                      const void* __restrict__ vals_in,
@@ -565,7 +577,7 @@ __global__ __launch_bounds__(kSecondThreads) void repartition_kernel(SortTables 
     const uint64_t row = static_cast<uint64_t>(bucket) * t.tiles1;
     map_runs<kSecondThreads, kSecondTile>(t.begins1 + row, t.table1 + row, t.tiles1, all, q0, count, mine.y, t.places1, 0, s_map,
                                           s_buf);
-    constexpr bool kPacked = packed_entries<Key>();
+    constexpr bool kPacked = packed_entries<Key>() && !PAIRS;
     uint32_t key[kPacked ? 1 : kSecondItems], aux[kSecondItems];  // packed: aux is the word that goes on from here,
     uint32_t digits[kPacked ? (kSecondItems + 3) / 4 : 1];        // digits the bits of it this step sorts by
     word_t val[VB ? kSecondItems : 1];
@@ -629,9 +641,12 @@ __global__ __launch_bounds__(kSecondThreads) void repartition_kernel(SortTables 
     for (int i = 0; i < kSecondItems; ++i)
         dest[i / 2] += static_cast<uint32_t>(s_cnt[(wave << kMaxBits) + digit(i)]) << (i % 2 * 16);
     const uint64_t out = static_cast<uint64_t>(first_tile + tile) * kSecondTile;
-    if constexpr (kPacked) {
-        store_packed<VB, kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, keys_out, vals_out, out,
-                                                                    [&](int i) { return aux[i]; }, val);
+    if constexpr (packed_entries<Key>()) {
+        auto word_of = [&](int i) {
+            if (kPacked) return aux[i];
+            return (key[kPacked ? 0 : i] & ((1u << t.d3) - 1u)) << t.minor_bits | (aux[i] & ((1u << t.minor_bits) - 1u));
+        };
+        store_packed<VB, kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, keys_out, vals_out, out, word_of, val);
     } else {
         store_keys<kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, keys_out + out, key, (1u << t.d3) - 1u);
         store_words<kSecondItems, kSecondThreads, kSecondTile>(s_buf, count, dest, aux_out + out, aux);
@@ -746,6 +761,10 @@ struct BucketLds {
 // same order from any order that is stable in the major key; buckets whose mean run is above kUsualRun don't try.
 // Assembly, all calls, with the radix passes alone and with this: 7.2 M triples of a mesh 219 -> 200 us; random triples,
 // 2 a row (8 M) 452 -> 423, 16 a row (8 M) 423 -> 393; tried with 30 a row (12 M) 555 -> 562, with 60 a row 549 -> 580.
+// Packed words: the first pass takes the eight upper bits of the word, also where more or fewer of them are the major key's,
+// and entries are compared as words, four at a time from where the run's stretch of 16 bytes begins: the words of the runs
+// around it compare as they should.  (Tried wherever the minor key's upper bits may cut the runs short: bands of 216 and 400
+// triples a row 212 -> 252 and 306 -> 357 us, for there they seldom do.)
 constexpr uint32_t kShortRun = 64, kUsualRun = 20;
 
 // Sorts a bucket of at most ITEMS * kBucketThreads entries, the runs of which are mapped in LDS.  MANY: in several passes.
@@ -756,8 +775,8 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
     typedef typename WordOf<VB>::type word_t;
     static_assert(!MANY || VB != 8, "64-bit values are sorted in one pass");
     const uint32_t tid = threadIdx.x, wave = tid / kWave;
-    constexpr bool kPacked = packed_entries<Key>();  // (aux is then the whole word: the key's rest below the index)
-    static_assert(!MANY || !kPacked, "sorts by one key");
+    // (aux is then the whole word: the key's rest below the index, or, MANY, above it, so that words sort as pairs do)
+    constexpr bool kPacked = packed_entries<Key>();
     uint32_t key[kPacked ? 1 : ITEMS], aux[ITEMS];
     word_t val[VB ? ITEMS : 1];
     const uint32_t last_word = (count - 1) / kWave;
@@ -781,15 +800,20 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
         }
         __syncthreads();
     };
-    // MANY: one pass by the key first (-1) where its runs are likely to be short; see kShortRun.
-    const bool key_first = MANY && t.d3 <= kPassBits && t.minor_passes > 1 && count <= kUsualRun << t.d3;
+    // MANY: one pass by the key first (-1), packed: by the upper bits of the word, where its runs are likely to be short; see
+    // kShortRun.
+    const uint32_t upper = kPacked ? min(t.minor_bits + t.d3, kPassBits) : t.d3;
+    const uint32_t below = kPacked ? t.minor_bits + t.d3 - upper : 0;
+    const bool key_first = MANY && upper <= kPassBits && (kPacked ? t.oversize_passes > 2 : t.minor_passes > 1) &&
+                           count <= kUsualRun << min(t.d3, kPassBits);
     for (int p = key_first ? -1 : 0;; ++p) {
-        const SortPass pass = MANY && p >= 0 ? sort_pass(t, static_cast<uint32_t>(p)) : SortPass{false, 0u, t.d3};
+        SortPass pass = {false, MANY ? below : 0u, MANY ? upper : t.d3};
+        if (MANY && p >= 0) pass = kPacked ? word_pass(t, static_cast<uint32_t>(p)) : sort_pass(t, static_cast<uint32_t>(p));
         bool long_run = false;
         const uint32_t mask = (1u << pass.bits) - 1u;
         auto digit = [&](int i) {
             const uint32_t of_aux = aux[i];  // (the values, so that neither array needs an address)
-            if constexpr (kPacked) return of_aux & mask;
+            if constexpr (kPacked) return (of_aux >> pass.shift) & mask;
             const uint32_t of_key = key[kPacked ? 0 : i];
             return MANY ? ((pass.on_aux ? of_aux : of_key) >> pass.shift) & mask : of_key;
         };
@@ -800,14 +824,14 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
                 write_key_ptr(out, sub, t.d3, d, first + at, t.count);
             } else if (p < 0) {
                 s.key_begin[d] = static_cast<uint16_t>(at);
-                if (d + 1 == 1u << t.d3) s.key_begin[d + 1] = static_cast<uint16_t>(count);
+                if (d + 1 == 1u << upper) s.key_begin[d + 1] = static_cast<uint16_t>(count);
                 long_run |= entries > kShortRun;
             }
         });
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i)
             dest[i / 2] += static_cast<uint32_t>(s.cnt[(wave << kPassBits) + digit(i)]) << (i % 2 * 16);
-        if (!MANY || p + 1 == static_cast<int>(t.passes)) break;
+        if (!MANY || p + 1 == static_cast<int>(kPacked ? t.oversize_passes : t.passes)) break;
         auto back = [&](uint32_t (&word)[ITEMS]) {
             ordered([&](int i) { return word[i]; });
 #pragma unroll
@@ -815,23 +839,38 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
             __syncthreads();
         };
         if constexpr (MANY) {
-            back(key);
+            if constexpr (!kPacked) back(key);
             if constexpr (VB == 4) back(val);
             back(aux);
+            if (kPacked && p < 0) {
+                // (the words behind the last one are looked at too, and must not go in front of any)
+                if (tid < 4 - count % 4 && count % 4 != 0) s.buf[count + tid] = ~0u;
+            }
             if (p < 0 && !__syncthreads_or(long_run)) {
                 // buf still holds the minor keys in this order: an entry's place is that of its run, plus the entries
                 // of the run that go before it
 #pragma unroll
                 for (int i = 0; i < ITEMS; ++i) {
                     const bool live = in_slab(ITEMS, i, count);
-                    const uint32_t here = slab_place(ITEMS, i), mine = aux[i], run = live ? key[i] & mask : 0u;
+                    const uint32_t here = slab_place(ITEMS, i), mine = aux[i];
+                    const uint32_t run = !live ? 0u : kPacked ? mine >> below : key[kPacked ? 0 : i] & mask;
                     uint32_t q = s.key_begin[run];
                     const uint32_t end = live ? s.key_begin[run + 1] : q;
                     uint32_t place = q;
+                    if constexpr (kPacked) {
+                        // (no word is all ones: see sort_packs)
+                        place = q &= ~3u;
+                        for (; q < end; q += 4) {
+                            const u32x4 others = *reinterpret_cast<const u32x4*>(&s.buf[q]);
+#pragma unroll
+                            for (uint32_t j = 0; j < 4; ++j) place += others[j] < mine + (static_cast<int>(here - q) > static_cast<int>(j));
+                        }
+                    } else {
 #pragma unroll 4
-                    for (; q < end; ++q) {
-                        const uint32_t other = s.buf[q];
-                        place += other < mine || (other == mine && q < here);
+                        for (; q < end; ++q) {
+                            const uint32_t other = s.buf[q];
+                            place += other < mine || (other == mine && q < here);
+                        }
                     }
                     if (i % 2 == 0) dest[i / 2] = place;
                     else dest[i / 2] |= place << 16;
@@ -852,7 +891,8 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
         }
         __syncthreads();
     };
-    ordered([&](int i) { return kPacked ? aux[i] >> t.d3 : aux[i]; });
+    const uint32_t minor_mask = (1u << t.minor_bits) - 1u;
+    ordered([&](int i) { return !kPacked ? aux[i] : MANY ? aux[i] & minor_mask : aux[i] >> t.d3; });
     stream_out([&](int, uint32_t p, uint32_t w) { out.aux[first + p] = w; });
     if constexpr (VB == 4) {
         ordered([&](int i) { return val[i]; });
@@ -868,14 +908,15 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
     }
     if constexpr (MANY) {
         const uint32_t high = (sub << t.d3) + out.key_bias;
-        ordered([&](int i) { return key[i]; });
+        ordered([&](int i) { return kPacked ? aux[i] >> t.minor_bits : key[kPacked ? 0 : i]; });
         stream_out([&](int, uint32_t p, uint32_t w) { out.keys[first + p] = high + w; });
     }
 }
 
 // A workgroup per bucket.  118 M entries (16 bytes each) in buckets of 3600: 390 us, bound by vector instructions as much
 // as by memory; so most buckets, below two thirds of the room, run a version without the last third of the items (458 -> 445
-// us when an entry was 17 bytes in three arrays).
+// us when an entry was 17 bytes in three arrays).  Packed pairs: another one without the last quarter, for the buckets of a
+// mean size (1.5 M rows, 6 M triples, all of the assembly: 274 -> 263 us).
 template <int VB, typename Key, bool MANY>
 __global__ __launch_bounds__(kBucketThreads, VB == 8 || MANY ? 6 : 8) void bucket_sort_kernel(SortTables t, const Key* __restrict__ keys_in,
                                                                                       const uint32_t* __restrict__ aux_in,
@@ -883,6 +924,7 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 || MANY ? 6 : 8) void bucke
                                                                                       SortOutput out, uint32_t buckets,
                                                                                       uint32_t xcds) {
     constexpr int kUsualItems = kBucketItems * 2 / 3, kFewItems = kBucketItems / 3;
+    constexpr int kMoreItems = MANY && packed_entries<Key>() ? kBucketItems * 3 / 4 : kUsualItems;
     __shared__ BucketLds s;
     const uint32_t sub = tile_of_block(buckets, xcds);
     if (sub >= buckets) return;  // whole workgroup
@@ -901,6 +943,8 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 || MANY ? 6 : 8) void bucke
         sort_bucket<VB, Key, MANY, kFewItems>(t, sub, first, count, keys_in, aux_in, vals_in, out, s);
     else if (count <= static_cast<uint32_t>(kUsualItems * kBucketThreads))
         sort_bucket<VB, Key, MANY, kUsualItems>(t, sub, first, count, keys_in, aux_in, vals_in, out, s);
+    else if (kMoreItems != kUsualItems && count <= static_cast<uint32_t>(kMoreItems * kBucketThreads))
+        sort_bucket<VB, Key, MANY, kMoreItems>(t, sub, first, count, keys_in, aux_in, vals_in, out, s);
     else
         sort_bucket<VB, Key, MANY, kBucketItems>(t, sub, first, count, keys_in, aux_in, vals_in, out, s);
 }
@@ -1067,11 +1111,15 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 ? 2 : 4) void oversize_kern
                 for (int i = 0; i < kBucketItems; ++i) {
                     const uint32_t from = place_of(i);
                     key[i] = 0;
-                    if constexpr (packed_entries<Key>()) key[i] = load_at<uint32_t>(keys_in, VB == 4 ? 2 * from : from);
+                    if constexpr (packed_entries<Key>() && !MANY) key[i] = load_at<uint32_t>(keys_in, VB == 4 ? 2 * from : from);
+                    else if (packed_entries<Key>() && p == 0) key[i] = load_at<uint32_t>(keys_in, VB == 4 ? 2 * from : from);
                     else if (by_key) key[i] = p == 0 ? load_at<Key>(keys_in, from) : load_shared_at<uint16_t>(between_keys, from);
                     if constexpr (MANY) {
                         aux[i] = 0;
-                        if (by_aux) aux[i] = p == 0 ? load_at<uint32_t>(aux_in, from) : load_shared_at<uint32_t>(between_aux, from);
+                        if (packed_entries<Key>() && p == 0) {
+                            aux[i] = key[i] & ((1u << t.minor_bits) - 1u);
+                            key[i] >>= t.minor_bits;
+                        } else if (by_aux) aux[i] = p == 0 ? load_at<uint32_t>(aux_in, from) : load_shared_at<uint32_t>(between_aux, from);
                     }
                 }
                 __syncthreads();
@@ -1112,9 +1160,10 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 ? 2 : 4) void oversize_kern
 #pragma unroll
                 for (int i = 0; i < kBucketItems; ++i) {
                     const uint32_t from = place_of(i);
-                    if constexpr (packed_entries<Key>()) {
+                    if (packed_entries<Key>() && (!MANY || p == 0)) {
                         load_packed<VB>(keys_in, vals_in, from, key[i], val[VB ? i : 0]);
-                        aux[i] = key[i] >> t.d3;
+                        aux[i] = MANY ? key[i] & ((1u << t.minor_bits) - 1u) : key[i] >> t.d3;
+                        if (MANY) key[i] >>= t.minor_bits;
                     } else if (!MANY || p == 0) {
                         key[i] = load_at<Key>(keys_in, from);
                         aux[i] = load_at<uint32_t>(aux_in, from);
@@ -1313,9 +1362,18 @@ bool sort_shape(uint32_t count, uint32_t key_count, uint32_t minor_bits, SortSha
 // (Behind the first of two the row is counted from the tile's first, with the 16 bits or more that the key leaves it.)
 // 118 M entries, 4 M columns: 18 + 19 + 17 bytes moved per entry and step become 16 each, and a run of a bucket lies in one
 // array instead of three.
-bool sort_packs(const SortShape& s, uint32_t rows) { return s.minor_bits == kNoMinorKey && bit_length(rows) + s.d3 <= 32; }
+// Index sorts: likewise the minor key and above it what is left of the major one, behind the last partition; the word then
+// sorts as the pair does, a pass in LDS moves two words instead of three, and there may be a pass less.  Assembly, all
+// calls, with what kShortRun says of words: 7.2 M triples of a mesh 198 -> 192 us, random ones, 2 M in 300 k rows 121 -> 100,
+// 6 M in 1.5 M rows 331 -> 263, 16 M in 4 M rows 787 -> 683.
+// extent: what indices or minor keys are at most, or one more; with that, no word of a pair is all ones.
+bool sort_packs(const SortShape& s, uint32_t extent) { return bit_length(extent) + s.d3 <= 32; }
+// Whether entries are packed behind the first partition already.
+bool packs_first(const SortShape& s) { return s.packed && (s.minor_bits == kNoMinorKey || s.d2 == 0); }
 // Bytes a key travels in behind step 1 (step 2 reads 16 bits) and behind step 2.
-size_t first_key_bytes(const SortShape& s) { return s.d2 == 0 && s.d3 <= 8 ? sizeof(uint8_t) : sizeof(uint16_t); }
+size_t first_key_bytes(const SortShape& s) {
+    return s.d2 == 0 && s.d3 <= 8 && s.minor_bits == kNoMinorKey ? sizeof(uint8_t) : sizeof(uint16_t);
+}
 size_t second_key_bytes(const SortShape& s) { return s.d3 <= 8 ? sizeof(uint8_t) : sizeof(uint16_t); }
 void sort_passes(const SortShape& s, SortTables* t) {
     const uint32_t minor = s.minor_bits == kNoMinorKey ? 0 : s.minor_bits;
@@ -1355,23 +1413,16 @@ SortLayout sort_layout(uint32_t count, const SortShape& s, size_t value_bytes) {
         off += align_up(bytes);
         return at;
     };
-    if (s.packed) {  // words, or {word, value} pairs
-        const bool pairs = value_bytes == sizeof(uint32_t);
-        const size_t entry = pairs ? sizeof(uint64_t) : sizeof(uint32_t), apart = pairs ? 0 : value_bytes;
-        l.keys1 = take(places1 * entry);
-        l.aux1 = take(s.d2 != 0 ? places1 * sizeof(uint32_t) : 0);
-        l.vals1 = take(places1 * apart);
-        l.keys2 = take(places2 * entry);
-        l.aux2 = off;
-        l.vals2 = take(places2 * apart);
-    } else {
-        l.keys1 = take(places1 * first_key_bytes(s));
-        l.aux1 = take(places1 * sizeof(uint32_t));
-        l.vals1 = take(places1 * value_bytes);
-        l.keys2 = take(places2 * second_key_bytes(s));
-        l.aux2 = take(places2 * sizeof(uint32_t));
-        l.vals2 = take(places2 * value_bytes);
-    }
+    // packed: words, or {word, value} pairs
+    const bool pairs = value_bytes == sizeof(uint32_t);
+    const size_t entry = pairs ? sizeof(uint64_t) : sizeof(uint32_t), apart = pairs ? 0 : value_bytes;
+    const bool rows_apart = s.minor_bits == kNoMinorKey && s.d2 != 0;  // of tiles that span many
+    l.keys1 = take(places1 * (packs_first(s) ? entry : first_key_bytes(s)));
+    l.aux1 = take(!packs_first(s) || rows_apart ? places1 * sizeof(uint32_t) : 0);
+    l.vals1 = take(places1 * (packs_first(s) ? apart : value_bytes));
+    l.keys2 = take(places2 * (s.packed ? entry : second_key_bytes(s)));
+    l.aux2 = take(s.packed ? 0 : places2 * sizeof(uint32_t));
+    l.vals2 = take(places2 * (s.packed ? apart : value_bytes));
     l.wide = take(sizeof(uint32_t));
     l.table1 = take(runs1 * sizeof(uint32_t));
     l.begins1 = take(runs1 * sizeof(uint32_t));
@@ -1453,13 +1504,15 @@ void launch_sort(hipStream_t stream, EntrySource in, const SortShape& s, const S
     t.count = in.count;
     const uint32_t shift = s.d2 + s.d3;
     constexpr bool kMany = KIND == kPlain;  // the sorts by two keys
-    const bool short_keys1 = first_key_bytes(s) == 1, short_keys2 = second_key_bytes(s) == 1;
-    auto* partition = s.d1 <= 8 ? (short_keys1 ? launch_partition<VB, KIND, 8, uint8_t> : launch_partition<VB, KIND, 8, uint16_t>)
-                                : (short_keys1 ? launch_partition<VB, KIND, kMaxOneLevelBits, uint8_t>
-                                               : launch_partition<VB, KIND, kMaxOneLevelBits, uint16_t>);
-    if constexpr (KIND == kCsr) {
-        if (s.packed)
-            partition = s.d1 <= 8 ? launch_partition<VB, KIND, 8, uint32_t> : launch_partition<VB, KIND, kMaxOneLevelBits, uint32_t>;
+    in.minor_bits = t.minor_bits;
+    auto with_digits = [&](auto key) {
+        typedef decltype(key) Key;
+        return s.d1 <= 8 ? launch_partition<VB, KIND, 8, Key> : launch_partition<VB, KIND, kMaxOneLevelBits, Key>;
+    };
+    // (a minor key of up to 24 bits leaves room for eight of the major one: eight alone are never left apart)
+    auto* partition = packs_first(s) ? with_digits(uint32_t()) : with_digits(uint16_t());
+    if constexpr (!kMany) {
+        if (!s.packed && first_key_bytes(s) == 1) partition = with_digits(uint8_t());
     }
     partition(stream, in, shift, s.d1, s.tile_size, w + l.keys1, words(l.aux1), w + l.vals1, words(l.table1));
     hipLaunchKernelGGL(run_begins_kernel, dim3(1u << s.d1), dim3(kScanBlock), 0, stream, s.tiles1, t.table1,
@@ -1467,11 +1520,9 @@ void launch_sort(hipStream_t stream, EntrySource in, const SortShape& s, const S
     hipLaunchKernelGGL(sort_plan_kernel, dim3(1), dim3(kPlanBlock), 0, stream, t);
     // what a key travels in behind step 2
     auto with_key = [&](auto launch) {
-        if constexpr (KIND == kCsr) {
-            if (s.packed) return launch(uint32_t());
-        }
-        if (short_keys2) return launch(uint8_t());
+        if (s.packed) return launch(uint32_t());
         if constexpr (kMany) launch(uint16_t());
+        else launch(uint8_t());
     };
     const void* keys = w + l.keys1;
     const uint32_t* aux = words(l.aux1);
@@ -1481,7 +1532,7 @@ void launch_sort(hipStream_t stream, EntrySource in, const SortShape& s, const S
         const dim3 grid((s.max_tiles2 + xcds - 1) / xcds * xcds);
         auto repartition = [&](auto key) {
             typedef decltype(key) Key;
-            hipLaunchKernelGGL((repartition_kernel<VB, Key>), grid, dim3(kSecondThreads), 0, stream, t, keys, aux, vals,
+            hipLaunchKernelGGL((repartition_kernel<VB, Key, kMany>), grid, dim3(kSecondThreads), 0, stream, t, keys, aux, vals,
                                reinterpret_cast<Key*>(w + l.keys2), words(l.aux2), w + l.vals2, s.max_tiles2, xcds);
         };
         with_key(repartition);
@@ -1522,7 +1573,9 @@ bool partition_sort_pairs_usable(idx_t count, idx_t major_count, idx_t minor_cou
 }
 size_t partition_sort_pairs_workspace_bytes(idx_t count, idx_t major_count, idx_t minor_count) {
     SortShape s;
-    return sort_shape(count, major_count, bit_length(minor_count - 1), &s) ? sort_layout(count, s, sizeof(idx_t)).total : 0;
+    if (!sort_shape(count, major_count, bit_length(minor_count - 1), &s)) return 0;
+    s.packed = sort_packs(s, minor_count);
+    return sort_layout(count, s, sizeof(idx_t)).total;
 }
 
 void launch_partition_sort(hipStream_t stream, idx_t count, const PartitionSortArgs& a, size_t value_bytes, void* workspace) {
@@ -1555,6 +1608,7 @@ void launch_partition_sort_pairs(hipStream_t stream, idx_t count, idx_t major_co
                                  idx_t* minor, idx_t* perm, void* workspace) {
     SortShape s;
     if (!sort_shape(count, major_count, bit_length(minor_count - 1), &s)) return;
+    s.packed = sort_packs(s, minor_count);
     EntrySource in = {};
     in.keys = major;
     in.aux = minor;

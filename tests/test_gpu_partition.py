@@ -130,6 +130,9 @@ def test_csr2csc_tiles_of_many_rows(torch_gpu, handle, oracle, dtype, action, m,
     ("few", 4000, 70000, 300000), ("band", 300000, 40000, 1000000), ("uniform", 1 << 23, 1 << 22, 100000),
     ("few", 100000, 1 << 22, ONE_LEVEL_UPTO), ("uniform", 1 << 22, 1 << 20, ONE_LEVEL_UPTO + 1),
     ("uniform", 1 << 24, 300, 50000), ("uniform", 5000, 100000, ONE_LEVEL_UPTO + 1),
+    # what is left of the major key and the minor one: more than 32 bits, so that no word holds both, and one row in pieces;
+    # 32 bits, where only the sort by column may have both in a word (the other could be all ones)
+    ("few", 1 << 22, 1 << 22, 2000000), ("uniform", 1 << 22, (1 << 21) - 1, ONE_LEVEL_UPTO + 1),
 ])
 def test_coosort_bit_exact(torch_gpu, handle, oracle, by, with_perm, kind, m, n, nnz):
     torch = torch_gpu
@@ -152,6 +155,27 @@ def test_coosort_bit_exact(torch_gpu, handle, oracle, by, with_perm, kind, m, n,
     assert np.array_equal(d_c.cpu().numpy(), cols[want])
     if with_perm:
         assert np.array_equal(d_p.cpu().numpy(), perm[want])
+
+
+@pytest.mark.parametrize("longest", [3, 64, 65, 700])  # 64: up to there a bucket's entries are counted, not sorted in passes
+@pytest.mark.parametrize("columns", [2, 70000])
+def test_coosort_runs_and_equal_pairs(torch_gpu, handle, longest, columns):
+    torch, rng, m, nnz = torch_gpu, np.random.default_rng(longest), 300000, 600001
+    rows, cols = rng.integers(0, m, nnz, dtype=np.int32), rng.integers(0, columns, nnz, dtype=np.int32)
+    rows[:longest] = m - 1  # in the last bucket, and in front of the places behind it
+    cols[:longest] = rng.integers(69998, 70000, longest)
+    order = rng.permutation(nnz)
+    rows, cols, perm = rows[order], cols[order], np.arange(nnz, dtype=np.int32)
+    d_r, d_c, d_p = dev(torch, rows), dev(torch, cols), dev(torch, perm)
+    st, size = api.sort_buffer_size(handle, "coo", m, 70000, nnz, d_r, d_c)
+    assert st == api.STATUS_SUCCESS
+    buf = torch.full((size,), 255, dtype=torch.uint8, device="cuda")
+    assert api.xcoosort_by_row(handle, m, 70000, nnz, d_r, d_c, d_p, buf) == api.STATUS_SUCCESS
+    torch.cuda.synchronize()
+    want = np.lexsort((cols, rows))  # stable
+    assert np.array_equal(d_p.cpu().numpy(), want)
+    assert np.array_equal(d_r.cpu().numpy(), rows[want])
+    assert np.array_equal(d_c.cpu().numpy(), cols[want])
 
 
 @pytest.mark.parametrize("share", [0.3, 0.9])  # 0.9: one bucket with more tiles of the second step than the first has
