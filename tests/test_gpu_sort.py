@@ -107,3 +107,14 @@ def test_identity_and_gather_with_base(torch_gpu, handle):
     assert api.gthr(handle, 777, dev(torch_gpu, y), d_x, dev(torch_gpu, ind + 1), api.BASE_ONE) == 0
     torch_gpu.cuda.synchronize()
     assert np.array_equal(d_x.cpu().numpy(), y[ind])
+
+
+@pytest.mark.parametrize("offset", [0, 1, 2, 3])  # elements: 16-byte stores need p at a multiple of four
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 1023, 1024, 1026])
+def test_identity_wherever_it_begins(torch_gpu, handle, offset, n):
+    d_p = torch_gpu.full((n + 8,), -1, dtype=torch_gpu.int32, device="cuda")
+    assert api.create_identity_permutation(handle, n, d_p[offset:offset + n]) == 0
+    torch_gpu.cuda.synchronize()
+    want = np.full(n + 8, -1, np.int32)
+    want[offset:offset + n] = np.arange(n)
+    assert np.array_equal(d_p.cpu().numpy(), want)
