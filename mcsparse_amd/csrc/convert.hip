@@ -45,150 +45,112 @@ __device__ __forceinline__ idx_t wave_count_row_starts(const idx_t* __restrict__
 }
 
 // coo_rows[j] = row of nonzero j (+ base) = the number of rows that begin at or before j, minus one.
-// A tile is 4096 nonzeros.  The rows that begin inside it are read from row_ptr (the first of them is
-// known from the tile before; only where a workgroup's first tile begins is searched for, a chain of
-// dependent loads) and set bits in a 4096-bit map in LDS; a thread then writes four neighbouring rows at a
-// time, each a count of bits, as one 16-byte store.  A tile in which two rows begin at the same nonzero
-// (an empty row) cannot be told from the map: its threads search the staged row starts instead, or
-// row_ptr itself when more rows begin in the tile than LDS holds.  A workgroup takes kExpandTiles tiles in
-// a row, and asks for the row starts of the next one before it writes this one: what bounds it is the store stream (a
-// fill of 472 MB runs at 6.8 TB/s), and a tile used to wait for its row starts first and then for 256 atomic maxima on
-// one word of LDS (now an add per wavefront).  4 M power-law rows, 118 M nonzeros: 108 -> 95 us; a million rows: 37 ->
-// 20 us; 150,000 rows: 33 -> 17 us.  Reference semantics: src/kernels/conversion/coo2csr_device.hpp:26-41.
-constexpr int kExpandTiles = 8;
-constexpr int kCooBlock = 256;
-constexpr int kCooTile = kCooBlock * 16;  // four stores of four rows per thread
-constexpr int kCooWords = kCooTile / kWave;
-constexpr int kCooLoads = 4;  // row starts per thread and round
-__global__ __launch_bounds__(kCooBlock) void csr2coo_kernel(idx_t m, idx_t nnz, idx_t base,
-                                                         const idx_t* __restrict__ row_ptr,
-                                                         idx_t* __restrict__ coo_rows) {
+// What bounds it is the store stream (a fill of 472 MB runs at 6.8 TB/s).  A wavefront has 1024 nonzeros for itself and waits
+// for no other: it searches row_ptr for the row that holds the first of them, reads the offsets from there on until one lies
+// past them, and each leaves its number in LDS at the nonzero it begins at, the last one of those that begin there (the others
+// are empty).  A running maximum over the 1024 places is what is written, 16 bytes a thread.  Where more offsets lie inside
+// than kCooRounds reads take (empty rows mostly) every nonzero searches row_ptr.  118 M nonzeros in 4 M power-law rows: 96 ->
+// 78 us (6.3 TB/s), 4 M rows of two nonzeros 31 -> 17, 120 k rows 17 -> 4.1, against workgroups that share tiles of 4096 and
+// wait for each other's LDS and stores at barriers.  More tiles in a row for a wavefront save searches but write at as many
+// places at once as there are wavefronts: 2, 3, 14 tiles 88, 93, 101 us.  512 or 2048 nonzeros: 116, 89; workgroups of 64,
+// 256, 1024 threads: 84, 81, 78.  Ordinary stores: 100 (2 tiles).
+// Reference semantics: src/kernels/conversion/coo2csr_device.hpp:26-41.
+constexpr int kCooBlock = 512;
+constexpr int kCooVecs = 4;                             // of four nonzeros, per thread and tile
+constexpr uint32_t kCooTile = kWave * 4 * kCooVecs;
+constexpr int kCooLoads = 4;                            // row starts per thread and round
+constexpr uint32_t kCooRound = kWave * kCooLoads, kCooRounds = 8;
+__device__ __forceinline__ uint32_t wave_inclusive_max(uint32_t v) {
+    constexpr int kRowShr = 0x110, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+    int x = static_cast<int>(v);
+    auto with = [&](int other) { x = static_cast<int>(max(static_cast<uint32_t>(x), static_cast<uint32_t>(other))); };
+    with(__builtin_amdgcn_update_dpp(0, x, kRowShr + 1, 0xF, 0xF, false));
+    with(__builtin_amdgcn_update_dpp(0, x, kRowShr + 2, 0xF, 0xF, false));
+    with(__builtin_amdgcn_update_dpp(0, x, kRowShr + 4, 0xF, 0xF, false));
+    with(__builtin_amdgcn_update_dpp(0, x, kRowShr + 8, 0xF, 0xF, false));
+    with(__builtin_amdgcn_update_dpp(0, x, kRowBcast15, 0xA, 0xF, false));
+    with(__builtin_amdgcn_update_dpp(0, x, kRowBcast31, 0xC, 0xF, false));
+    return static_cast<uint32_t>(x);
+}
+__global__ __launch_bounds__(kCooBlock, 8) void csr2coo_kernel(idx_t m, idx_t nnz, idx_t base,
+                                                            const idx_t* __restrict__ row_ptr,
+                                                            idx_t* __restrict__ coo_rows) {
     typedef idx_t idx4 __attribute__((ext_vector_type(4)));
-    static_assert((kCooWords % kWave == 0 || kCooWords < kWave) && kCooWords <= kCooBlock && kCooBlock % kWave == 0,
-                  "the words of the map are counted a wavefront at a time");
-    constexpr int kScanLanes = (kCooWords + kWave - 1) / kWave * kWave;
-    __shared__ idx_t s_start[kCooTile];
-    __shared__ unsigned long long s_begins[kCooWords];
-    __shared__ uint32_t s_begins_before[kCooWords];
-    __shared__ uint32_t s_wave_begins[(kCooWords + kWave - 1) / kWave];
-    __shared__ idx_t s_first;
-    __shared__ uint32_t s_empty_rows;
-    __shared__ uint32_t s_inside;
-
-    const uint32_t tid = threadIdx.x;
-    const unsigned lane = tid % kWave;
-    const uint64_t group_first = static_cast<uint64_t>(blockIdx.x) * kExpandTiles * kCooTile;
-    if (group_first >= nnz) return;  // whole workgroup
-    if (tid / kWave == 0) {
-        const idx_t c = wave_count_row_starts(row_ptr, m, base, static_cast<idx_t>(group_first));
-        if (tid == 0) s_first = c;
-    }
-    __syncthreads();
-    uint64_t before = s_first;  // rows (of the m + 1 offsets) that begin at or before the tile's first nonzero
-    const bool wide = (reinterpret_cast<uintptr_t>(coo_rows) & 15u) == 0;
-    idx_t ahead[kCooLoads];  // the first row starts of the next tile
-    auto look_ahead = [&]() {
+    __shared__ __align__(16) uint32_t s_rows[kCooBlock / kWave][kCooTile];
+    const unsigned lane = threadIdx.x % kWave;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    uint32_t* rows = s_rows[wave];
+    const uint64_t j0 = static_cast<uint64_t>(blockIdx.x * (kCooBlock / kWave) + wave) * kCooTile;
+    if (j0 >= nnz) return;  // whole wavefront; nobody waits for it
+    const uint32_t count = static_cast<uint32_t>(min(static_cast<uint64_t>(kCooTile), nnz - j0));
+    // rows (of the m + 1 offsets, the last of which lies behind j0) that begin at or before the tile's first nonzero
+    const uint32_t before = __builtin_amdgcn_readfirstlane(wave_count_row_starts(row_ptr, m, base, static_cast<idx_t>(j0)));
+    const uint32_t from = static_cast<uint32_t>(j0) + base;
+    // the offsets from `before` on, until one lies past the tile
+    uint32_t inside = 0;
+    idx_t offset[kCooLoads];
+    auto read_offsets = [&]() {
+#pragma unroll
+        for (int k = 0; k < kCooLoads; ++k) offset[k] = row_ptr[min(before + inside + k * kWave + lane, static_cast<uint32_t>(m))];
+    };
+    read_offsets();
+#pragma unroll
+    for (int k = 0; k < kCooVecs; ++k) reinterpret_cast<idx4*>(rows)[k * kWave + lane] = idx4(0);
+    bool ended = false;
+    for (uint32_t round = 0; round < kCooRounds && !ended; ++round) {
+        if (round != 0) read_offsets();
+        uint32_t here = 0;
 #pragma unroll
         for (int k = 0; k < kCooLoads; ++k) {
-            const uint64_t r = before + static_cast<uint32_t>(k) * kCooBlock + tid;
-            ahead[k] = row_ptr[r <= m ? r : m];
+            const uint32_t i = inside + k * kWave + lane;
+            const uint32_t at = i <= m - before ? offset[k] - from : ~0u;
+            if (at < kCooTile) atomicMax(&rows[at], i + 1);
+            here += __popcll(__ballot(at < kCooTile));
         }
-    };
-    look_ahead();
-    for (int t = 0; t < kExpandTiles; ++t) {
-        const uint64_t j0 = group_first + static_cast<uint64_t>(t) * kCooTile;
-        if (j0 >= nnz) break;  // whole workgroup
-        const uint32_t count = static_cast<uint32_t>(nnz - j0 < kCooTile ? nnz - j0 : kCooTile);
-        if (tid < kCooWords) s_begins[tid] = 0;
-        if (tid == 0) {
-            s_empty_rows = 0;
-            s_inside = 0;
-        }
-        __syncthreads();
-        // the offsets from `before` on, until one lies past the tile: those up to j0 + 4096 begin a row of this
-        // tile (or, at j0 + 4096 itself, are counted for the next one)
-        uint32_t inside = 0;
-        for (uint32_t loaded = 0;; loaded += kCooBlock * kCooLoads) {
-            uint64_t at[kCooLoads];
+        inside += here;
+        ended = here < kCooRound;  // the round held one past the tile, or the last one
+    }
+    if (!ended) inside = wave_count_row_starts(row_ptr, m, base, static_cast<idx_t>(j0 + count - 1)) - before;
+    const bool wide = (reinterpret_cast<uintptr_t>(coo_rows) & 15u) == 0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    idx4 row[kCooVecs];
+    uint32_t upto[kCooVecs];
 #pragma unroll
-            for (int k = 0; k < kCooLoads; ++k) {
-                const uint64_t r = before + loaded + static_cast<uint32_t>(k) * kCooBlock + tid;
-                if (loaded != 0) ahead[k] = row_ptr[r <= m ? r : m];
-                at[k] = r <= m ? static_cast<uint64_t>(ahead[k] - base) - j0 : ~0ull;  // > 0: row `before` begins after j0
-            }
-            uint32_t in_wave = 0;  // offsets of this wavefront that lie inside
+    for (int k = 0; k < kCooVecs; ++k) {
+        row[k] = reinterpret_cast<const idx4*>(rows)[k * kWave + lane];
 #pragma unroll
-            for (int k = 0; k < kCooLoads; ++k) {
-                const bool in_tile = at[k] <= static_cast<uint64_t>(kCooTile);
-                in_wave += __popcll(__ballot(in_tile));
-                if (!in_tile) continue;
-                const uint32_t i = loaded + static_cast<uint32_t>(k) * kCooBlock + tid;
-                if (i < static_cast<uint32_t>(kCooTile)) s_start[i] = static_cast<idx_t>(at[k]);
-                if (at[k] < static_cast<uint64_t>(kCooTile)) {
-                    const unsigned long long bit = 1ull << (at[k] % kWave);
-                    if ((atomicOr(&s_begins[at[k] / kWave], bit) & bit) != 0) s_empty_rows = 1;
+        for (int e = 1; e < 4; ++e) row[k][e] = max(row[k][e], row[k][e - 1]);
+        upto[k] = wave_inclusive_max(row[k][3]);
+    }
+    uint32_t carried = 0;
+#pragma unroll
+    for (int k = 0; k < kCooVecs; ++k) {
+        const uint32_t p = (k * kWave + lane) * 4;  // four neighbouring nonzeros of the tile
+        // (what the lanes before have; wave_shr:1, nothing for the first)
+        const int shifted = __builtin_amdgcn_update_dpp(0, static_cast<int>(upto[k]), 0x138, 0xF, 0xF, false);
+        const uint32_t others = max(carried, static_cast<uint32_t>(shifted));
+        carried = max(carried, static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(upto[k]), kWave - 1)));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            uint32_t begun = max(others, row[k][e]);
+            if (!ended) {
+                uint32_t lo = 0, hi = inside;  // row starts of the tile at or before nonzero p + e
+                while (lo < hi) {
+                    const uint32_t mid = (lo + hi) >> 1;
+                    if (row_ptr[before + mid] - from <= p + e) lo = mid + 1; else hi = mid;
                 }
+                begun = lo;
             }
-            if (lane == 0 && in_wave != 0) atomicAdd(&s_inside, in_wave);
-            __syncthreads();
-            inside = s_inside;
-            if (inside < loaded + kCooBlock * kCooLoads) break;  // whole workgroup: the round held one past the tile
+            row[k][e] = before + begun - 1 + base;
         }
-        const bool by_bits = s_empty_rows == 0;  // the same for the whole workgroup
-        if (by_bits) {
-            if (tid < kScanLanes) {  // whole wavefronts
-                const uint32_t c = tid < kCooWords ? __popcll(s_begins[tid]) : 0;
-                const uint32_t upto = wave_inclusive_sum(c);
-                if (tid < kCooWords) s_begins_before[tid] = upto - c;
-                if (lane == kWave - 1) s_wave_begins[tid / kWave] = upto;
-            }
-            __syncthreads();
+        idx_t* out = coo_rows + j0 + p;
+        if (wide && p + 4 <= count) {
+            __builtin_nontemporal_store(row[k], reinterpret_cast<idx4*>(out));
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (p + e < count) out[e] = row[k][e];
         }
-        const bool staged = inside <= static_cast<uint32_t>(kCooTile);
-        const uint64_t tile_before = before;
-        before += inside;
-        look_ahead();  // on their way while this tile is written
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const uint32_t p = (static_cast<uint32_t>(k) * kCooBlock + tid) * 4;  // four neighbouring nonzeros of the tile
-            if (p >= count) continue;
-            idx_t rows[4];
-            if (by_bits) {
-                const uint32_t word = p / kWave, bit = p % kWave;
-                const unsigned long long w = s_begins[word];
-                // rows that begin before nonzero p, then one more for every bit of the four at p .. p + 3
-                uint64_t upto = tile_before + s_begins_before[word];
-                for (uint32_t v = 0; v < word / kWave; ++v) upto += s_wave_begins[v];  // wavefronts of words before this one
-                idx_t row = static_cast<idx_t>(upto + __popcll(w & ((1ull << bit) - 1ull)) - 1 + base);
-                const uint32_t four = static_cast<uint32_t>(w >> bit) & 0xFu;  // bit <= 60
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    row += (four >> e) & 1u;
-                    rows[e] = row;
-                }
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    uint32_t lo = 0, hi = inside;  // row starts of the tile at or before nonzero p + e
-                    while (lo < hi) {
-                        const uint32_t mid = (lo + hi) >> 1;
-                        const uint64_t begins = staged ? s_start[mid] : static_cast<uint64_t>(row_ptr[tile_before + mid] - base) - j0;
-                        if (begins <= p + e) lo = mid + 1; else hi = mid;
-                    }
-                    rows[e] = static_cast<idx_t>(tile_before + lo - 1 + base);
-                }
-            }
-            idx_t* out = coo_rows + j0 + p;
-            if (wide && p + 4 <= count) {
-                idx4 v = {rows[0], rows[1], rows[2], rows[3]};
-                __builtin_nontemporal_store(v, reinterpret_cast<idx4*>(out));
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (p + e < count) out[e] = rows[e];
-            }
-        }
-        __syncthreads();  // the next tile clears the map
     }
 }
 
@@ -1007,9 +969,9 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(idx_t nnz, const T* __re
 
 void launch_csr2coo(hipStream_t stream, idx_t m, idx_t nnz, const idx_t* row_ptr, idx_t base, idx_t* coo_rows) {
     if (nnz == 0) return;
-    const uint64_t per_group = static_cast<uint64_t>(kExpandTiles) * kCooTile;
-    const uint32_t groups = static_cast<uint32_t>((static_cast<uint64_t>(nnz) + per_group - 1) / per_group);
-    hipLaunchKernelGGL(csr2coo_kernel, dim3(groups), dim3(kCooBlock), 0, stream, m, nnz, base, row_ptr, coo_rows);
+    const uint32_t tiles = (static_cast<uint32_t>(nnz) - 1) / kCooTile + 1;
+    hipLaunchKernelGGL(csr2coo_kernel, dim3((tiles - 1) / (kCooBlock / kWave) + 1), dim3(kCooBlock), 0, stream, m, nnz, base,
+                       row_ptr, coo_rows);
 }
 
 void launch_coo2csr(hipStream_t stream, idx_t nnz, idx_t m, const idx_t* coo_rows, idx_t base, idx_t* row_ptr) {

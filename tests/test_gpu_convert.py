@@ -232,12 +232,14 @@ def test_unaligned_input_arrays(torch_gpu, handle, oracle, shift):
     assert np.array_equal(d_out.cpu().numpy().view(np.uint32), oracle.coo2csr(300, m_big, 0, rows))
 
 
-@pytest.mark.parametrize("nnz", [4095, 4096, 4097, 8 * 4096 - 1, 8 * 4096, 8 * 4096 + 1, 3 * 8 * 4096 + 5])
-@pytest.mark.parametrize("shape", ["ones", "even", "empty_head", "empty_tail", "one_long_row", "every_other_empty"])
+@pytest.mark.parametrize("nnz", [1023, 1024, 1025, 4095, 4096, 4097, 8 * 1024 - 1, 8 * 1024 + 1, 8 * 4096 - 1, 8 * 4096,
+                                 8 * 4096 + 1, 3 * 8 * 4096 + 5])
+@pytest.mark.parametrize("shape", ["ones", "even", "empty_head", "empty_tail", "one_long_row", "every_other_empty",
+                                   "two_of_three_empty"])
 def test_csr2coo_around_the_tile_and_group_sizes(torch_gpu, handle, oracle, nnz, shape):
-    """csr2coo cuts the nonzeros into tiles of 4096 and walks 8 tiles per workgroup; the rows of a tile come from a
-    map of the 4096 places a row can begin at (rows of one nonzero fill it), from the staged offsets when a row is
-    empty, and from row_ptr itself when more than 4096 rows begin in a tile."""
+    """csr2coo cuts the nonzeros into tiles of 1024, eight to a workgroup; the rows of a tile come from a running maximum
+    over the 1024 places a row can begin at (rows of one nonzero fill them), and from a search in row_ptr when 2048 offsets
+    or more lie in a tile."""
     rng = np.random.default_rng(nnz)
     if shape == "ones":
         lens = np.ones(nnz, np.int64)
@@ -254,9 +256,10 @@ def test_csr2coo_around_the_tile_and_group_sizes(torch_gpu, handle, oracle, nnz,
     elif shape == "one_long_row":
         lens = np.zeros(nnz // 2, np.int64)
         lens[int(rng.integers(0, lens.size))] = nnz
-    else:                         # two rows begin at every nonzero: 8192 in a tile
-        lens = np.zeros(2 * nnz, np.int64)
-        lens[1::2] = 1
+    else:                         # two or three rows begin at every nonzero: 2048 or 3072 in a tile
+        each = 2 if shape == "every_other_empty" else 3
+        lens = np.zeros(each * nnz, np.int64)
+        lens[each - 1::each] = 1
     m = lens.size
     assert lens.sum() == nnz
     ptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
