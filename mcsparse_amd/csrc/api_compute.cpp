@@ -614,7 +614,8 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
         // both operands column-major and rows that share diagonals: nothing is transposed
         if (l.copy_b && l.copy_c && A->nnz != 0 && (b == 0 || shared_structure) && schedule_of_call(A, buffer) &&
             A->schedule.diagonals != 0 && A->schedule.diagonals_value_bytes == sizeof(T) &&
-            mcsp::spmm_diagonals_usable(a.k, a.n, A->schedule.longest_slice, sizeof(T))) {
+            mcsp::spmm_diagonals_usable(a.k, a.n, A->schedule.longest_slice, sizeof(T)) &&
+            !(A->schedule.blocks && schedule_matches(A, buffer) && mcsp::spmm_diagonals_alias(a.n, B->ld, C->ld, c_user, sizeof(T)))) {
             mcsp::launch_spmm_diagonals<T>(h->stream, a, A->schedule.diagonals, buf + A->schedule.diagonals_at, h_alpha, h_beta);
             continue;
         }

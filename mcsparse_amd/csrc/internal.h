@@ -366,6 +366,7 @@ bool build_slice_diagonals(hipStream_t stream, idx_t m, idx_t nnz, idx_t base, c
 // op(B) and C column-major (B: element (kk, j) at kk + j * ldb), the product row by row from the caller's values; region: what
 // build_slice_diagonals has left without values.
 bool spmm_diagonals_usable(idx_t k, idx_t n, uint32_t longest, size_t value_bytes);
+bool spmm_diagonals_alias(idx_t n, int64_t ldb, int64_t ldc, const void* C, size_t value_bytes);  // left to the blocks
 struct SpmmArgs;
 template <typename T>
 void launch_spmm_diagonals(hipStream_t stream, const SpmmArgs& a, uint32_t total, const void* region, T alpha, T beta);

@@ -12,7 +12,7 @@
 // columns: 157 us with a load for each, 106 so; the transposes and the row kernel took 224).  A, op(B) and C
 // are 408 MB, 85 us at the rate of a copy.  Other widths and sizes, microseconds before and now: fp64 37 columns 1004 and 293; fp32 6, 16, 64 and 128 columns 96, 160, 644, 1157 and
 // 47, 63, 242, 477; 40 x 38 x 55, fp32, 4 and 9 columns 17.4, 16.6 and 10.4, 15.8.  Columns a power of two apart (128^3: 8 MB)
-// fall on the same sets of the caches: 64 and 128 columns there are level with the strips and transposes (676 and 683).
+// fall on the same sets of the caches: see spmm_diagonals_alias.
 //
 // The reference copies the operands into the other order (src/kernels/level3/spmm/mcsp_spmm_gpu.cpp:119-133).
 #include "diagonals_device.h"
@@ -253,6 +253,16 @@ bool spmm_diagonals_usable(idx_t k, idx_t n, uint32_t longest, size_t value_byte
     // the values of a slice fit LDS; places in a column of op(B) fit 32 bits
     return longest <= (value_bytes == 4 ? staged_values<float>() : staged_values<double>()) &&
            static_cast<uint64_t>(k) * value_bytes < (1ull << 32);
+}
+
+// Columns of op(B) a multiple of 2 MB and more than an L2 apart fall on the same sets of it.  Fp32 operands that fill the lane
+// groups of the kernel by blocks are its then, 27-point stencils, microseconds with it and from the diagonals: 128^3, 64 and 128
+// columns (C where it can write it) 676 and 684, 1353 and 1355; 128 x 128 x 96 517 and 524, 1048 and 1036.  Else the diagonals win: 128 x 128 x 64 (4 MB)
+// 351 and 341, 128 x 128 x 120 652 and 637, 128^3 with 32 and 100 columns 374 and 347, 1480 and 1102, fp64 2495 and 1412.
+bool spmm_diagonals_alias(idx_t n, int64_t ldb, int64_t ldc, const void* C, size_t value_bytes) {
+    const uint64_t apart = static_cast<uint64_t>(ldb) * value_bytes;
+    return value_bytes == 4 && n % 64 == 0 && apart % (2u << 20) == 0 && apart > (4u << 20) &&
+           reinterpret_cast<uintptr_t>(C) % 16 == 0 && static_cast<uint64_t>(ldc) * value_bytes % 16 == 0;
 }
 
 template <typename T>

@@ -179,3 +179,12 @@ def test_replays_in_a_graph(torch_gpu, oracle):
         ref, bound = oracle.spmm(a.m, 5, 0, a.ptr, a.col, a.val, 1.0, 0.0, B.ravel(), 5, True, None, 5, True)
         assert_within(call.d_C.cpu().numpy().T, ref, bound, np.float64, what="replay %d" % replay)
     handle.destroy()
+
+
+@pytest.mark.parametrize("n", [64, 63])  # columns of op(B) 6 MB apart: 64 are left to the blocks; 63 are not
+@pytest.mark.parametrize("pad_c", [4, 1])  # 1: a C that the blocks do not write directly
+def test_columns_on_the_same_sets_of_the_caches(torch_gpu, handle, oracle, n, pad_c):
+    a = grid((64, 32, 16), BOX, np.float32, 31)
+    call = Call(torch_gpu, handle, a, n, pad_b=(3 << 19) - a.n, pad_c=pad_c)
+    assert call.mat.spmm_diagonals() > 0 and call.mat.spmm_schedule()[0] in (3, 4)
+    call.check(oracle)
