@@ -10,6 +10,7 @@
 //   2. spmm_long_chunk_kernel forms the sums of a piece, all 256 threads on its nonzeros, and writes the row of C
 //      (one piece) or a row of partial sums (several);
 //   3. spmm_long_reduce_kernel adds the partial sums of a row in the order of the pieces and writes the row of C.
+// Where op(B) is far larger than the L2s, step 2 goes band by band of op(B): see the bands below.
 // Every sum is formed in a fixed order, so results repeat bit for bit; where the pieces and partial sums of a row
 // lie in the scratch area depends on the order in which the rows were found, which nothing else depends on.
 #include "spmm_device.h"
