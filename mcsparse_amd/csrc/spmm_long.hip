@@ -22,7 +22,11 @@ namespace {
 using namespace spmm_detail;
 
 struct LongCounters {
-    uint32_t items, rows, slots;
+    // the pieces listed; rows of several pieces << 32 | the pieces of those.  (Adds to one line take their turns, 5 ns each,
+    // whichever counters they are for: three for each of 1024 workgroups were the time of the find kernel on 4 M rows, 17 us.)
+    uint32_t items;
+    unsigned long long several;
+    __device__ uint32_t rows() const { return static_cast<uint32_t>(several >> 32); }
     // not zero: the listed rows are taken apart, since there is one of more than kSpmmLongRow nonzeros (on a line of its
     // own: a store among the adds to the counters makes the find kernel wait, 16.5 -> 27.5 us on a million rows)
     alignas(128) uint32_t apart;
@@ -32,8 +36,7 @@ static_assert(sizeof(LongCounters) <= 2 * kAlign, "what the layout has room for"
 
 __global__ void spmm_long_zero_kernel(LongCounters* c, bool known) {
     c->items = 0;
-    c->rows = 0;
-    c->slots = 0;
+    c->several = 0;
     c->apart = known ? 1 : 0;
     c->unsorted = 0;
 }
@@ -69,7 +72,8 @@ __global__ __launch_bounds__(kBlock) void spmm_long_find_kernel(idx_t m, idx_t l
     __shared__ uint4 s_list[kFindList];      // {row, pieces, first item, first slot}, relative to the workgroup
     __shared__ uint32_t s_list_row[kFindList];  // place in the list of rows of several pieces
     __shared__ uint32_t s_count, s_items, s_slots, s_rows, s_apart;
-    __shared__ uint32_t s_base[3];
+    __shared__ uint32_t s_base;
+    __shared__ unsigned long long s_base_several;
     const uint32_t tid = threadIdx.x;
     if (tid == 0) {
         s_count = 0;
@@ -106,10 +110,9 @@ __global__ __launch_bounds__(kBlock) void spmm_long_find_kernel(idx_t m, idx_t l
                 s_list[at] = make_uint4(static_cast<uint32_t>(row), pieces, first, slot);
             } else {  // no room in the workgroup's list: places straight off the counters
                 const uint32_t first = atomicAdd(&c->items, pieces);
-                const uint32_t slot = pieces > 1 ? atomicAdd(&c->slots, pieces) : 0u;
-                const uint32_t place = pieces > 1 ? atomicAdd(&c->rows, 1u) : 0u;
-                write_long_row(static_cast<uint32_t>(row), pieces, first, slot, place, items, rows, cap_items, cap_rows,
-                               cap_slots);
+                const unsigned long long there = pieces > 1 ? atomicAdd(&c->several, 1ull << 32 | pieces) : 0ull;
+                write_long_row(static_cast<uint32_t>(row), pieces, first, static_cast<uint32_t>(there),
+                               static_cast<uint32_t>(there >> 32), items, rows, cap_items, cap_rows, cap_slots);
             }
         }
     }
@@ -119,15 +122,14 @@ __global__ __launch_bounds__(kBlock) void spmm_long_find_kernel(idx_t m, idx_t l
     if (listed == 0) return;  // whole workgroup
     if (tid == 0) {
         if (s_apart != 0) c->apart = 1;
-        s_base[0] = atomicAdd(&c->items, s_items);
-        s_base[1] = s_slots != 0 ? atomicAdd(&c->slots, s_slots) : 0u;
-        s_base[2] = s_rows != 0 ? atomicAdd(&c->rows, s_rows) : 0u;
+        s_base = atomicAdd(&c->items, s_items);
+        s_base_several = s_rows != 0 ? atomicAdd(&c->several, static_cast<unsigned long long>(s_rows) << 32 | s_slots) : 0ull;
     }
     __syncthreads();
     for (uint32_t k = tid; k < listed; k += kBlock) {
         const uint4 e = s_list[k];
-        write_long_row(e.x, e.y, s_base[0] + e.z, s_base[1] + e.w, s_base[2] + s_list_row[k], items, rows, cap_items,
-                       cap_rows, cap_slots);
+        write_long_row(e.x, e.y, s_base + e.z, static_cast<uint32_t>(s_base_several) + e.w,
+                       static_cast<uint32_t>(s_base_several >> 32) + s_list_row[k], items, rows, cap_items, cap_rows, cap_slots);
     }
 }
 
@@ -139,7 +141,7 @@ __global__ __launch_bounds__(kBlock) void spmm_long_find_kernel(idx_t m, idx_t l
 // added up per row in the order of pieces and bands.  Whether and how is decided on the device, from the number of pieces
 // found, so that every way to a product comes to the same sums.
 // A million power-law rows, 32 fp32 columns (20 M of 28 M nonzeros in rows of more than 256), microseconds: pieces whole 327,
-// band by band 225 and 30 for the bounds, 560 -> 507 a call; 16 columns 520 -> 457; 3 M rows, 20 columns 1942 -> 1466; 400 K
+// band by band 225 and 30 for the bounds, 560 -> 501 a call; 16 columns 520 -> 457; 3 M rows, 20 columns 1942 -> 1443; 400 K
 // rows, 11 fp64 columns 258 -> 227.  Half of the rows of op(B) still come from behind the L2 (its wavefronts are not all in
 // one band); bands of 2 MB bring that down to a quarter and the nonzeros of a pair to 32, half a round: 524.  Bands of 8 MB:
 // 549.  Rows of op(B) wider than a panel of kBandLanes lanes keep their pieces whole: A's long rows would be read once per
@@ -511,6 +513,8 @@ __global__ __launch_bounds__(kBlock) void spmm_long_reduce_kernel(idx_t n, T* __
     const uint64_t per_row = (static_cast<uint64_t>(n) + V - 1) / V;
     const BandPlan plan = band_plan(space, c, cap_items);
     if (plan.bands != 0) {  // the same for all workgroups: the partial sums of all pieces of a row, band by band
+        // (bound by the chain of the longest row: its bounds are asked for a step ahead, four sums at once: 21.6 -> 19 us where
+        // the longest row has 13 pieces)
         constexpr uint32_t kLanes = 8, kGroups = kWave / kLanes;
         static_assert(kBandStretches % kGroups == 0, "whole rounds");
         const T* sums = static_cast<const T*>(plan.sums);
@@ -525,25 +529,46 @@ __global__ __launch_bounds__(kBlock) void spmm_long_reduce_kernel(idx_t n, T* __
             T sum[V];
 #pragma unroll
             for (int i = 0; i < V; ++i) sum[i] = T(0);
-            for (uint32_t j = 0; j < item.z; ++j) {
-                const uint32_t* bounds = plan.bounds + static_cast<uint64_t>(it + j) * (plan.bands + 1);
-                const T* in = sums + static_cast<int64_t>(it + j) * plan.bands * ld_partials + own.first;
-                for (uint32_t b0 = 0; b0 < plan.bands; b0 += kWave) {
-                    // the bands that hold nonzeros of the piece (for the others nothing was written), the groups in turn
-                    const uint32_t b = min(b0 + threadIdx.x % kWave, plan.bands - 1);
-                    const bool holds = b0 + threadIdx.x % kWave < plan.bands && bounds[b] != bounds[b + 1];
-                    const unsigned long long holding = __ballot(holds);
-                    const uint32_t rank = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(holding >> 32),
-                                                                    __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(holding), 0u));
-                    // lane r learns the r-th of them (lanes without one send to the last lane, where nobody looks unless all hold)
-                    const uint32_t bands_held = __popcll(holding);
-                    const uint32_t band = __builtin_amdgcn_ds_permute(static_cast<int>((holds ? rank : kWave - 1) * 4), static_cast<int>(b));
-                    for (uint32_t r0 = 0; r0 < bands_held; r0 += kGroups) {
-                        const uint32_t r = min(r0 + group, bands_held - 1);
-                        const Vec<T, V> part = load_row<T, V>(in + static_cast<int64_t>(__shfl(band, r, kWave)) * ld_partials);
-                        if (r0 + group < bands_held) {
+            // 64 bands of a piece at a time; the bounds of the next 64 are asked for before the sums of these
+            const uint32_t rounds = (plan.bands + kWave - 1) / kWave;
+            const uint32_t* bounds = plan.bounds + static_cast<uint64_t>(it) * (plan.bands + 1);
+            const T* in = sums + static_cast<int64_t>(it) * plan.bands * ld_partials + own.first;
+            uint32_t b0 = 0, b = min(threadIdx.x % kWave, plan.bands - 1), begin = bounds[b], end = bounds[b + 1];
+            for (uint32_t steps = item.z * rounds; steps != 0; --steps) {
+                const bool holds = b0 + threadIdx.x % kWave < plan.bands && begin != end;
+                const uint32_t band_here = b;
+                const T* in_here = in;
+                b0 += kWave;
+                if (b0 >= plan.bands) {
+                    b0 = 0;
+                    if (steps != 1) {
+                        bounds += plan.bands + 1;
+                        in += static_cast<int64_t>(plan.bands) * ld_partials;
+                    }
+                }
+                b = min(b0 + threadIdx.x % kWave, plan.bands - 1);
+                begin = bounds[b];
+                end = bounds[b + 1];
+                // the bands that hold nonzeros of the piece (for the others nothing was written), the groups in turn
+                const unsigned long long holding = __ballot(holds);
+                const uint32_t rank = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(holding >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(holding), 0u));
+                // lane r learns the r-th of them (lanes without one send to the last lane, where nobody looks unless all hold)
+                const uint32_t bands_held = __popcll(holding);
+                const uint32_t band = __builtin_amdgcn_ds_permute(static_cast<int>((holds ? rank : kWave - 1) * 4), static_cast<int>(band_here));
+                constexpr uint32_t kAtOnce = 4;
+                for (uint32_t r0 = 0; r0 < bands_held; r0 += kGroups * kAtOnce) {
+                    Vec<T, V> part[kAtOnce];
 #pragma unroll
-                            for (int i = 0; i < V; ++i) sum[i] += part.v[i];
+                    for (uint32_t u = 0; u < kAtOnce; ++u) {
+                        const uint32_t r = min(r0 + u * kGroups + group, bands_held - 1);
+                        part[u] = load_row<T, V>(in_here + static_cast<int64_t>(__shfl(band, r, kWave)) * ld_partials);
+                    }
+#pragma unroll
+                    for (uint32_t u = 0; u < kAtOnce; ++u) {
+                        if (r0 + u * kGroups + group < bands_held) {
+#pragma unroll
+                            for (int i = 0; i < V; ++i) sum[i] += part[u].v[i];
                         }
                     }
                 }
@@ -557,7 +582,7 @@ __global__ __launch_bounds__(kBlock) void spmm_long_reduce_kernel(idx_t n, T* __
         }
         return;
     }
-    const uint64_t work = c->apart != 0 ? static_cast<uint64_t>(min(c->rows, cap_rows)) * per_row : 0;
+    const uint64_t work = c->apart != 0 ? static_cast<uint64_t>(min(c->rows(), cap_rows)) * per_row : 0;
     for (uint64_t w = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; w < work;
          w += static_cast<uint64_t>(gridDim.x) * kBlock) {
         const uint4 entry = rows[w / per_row];

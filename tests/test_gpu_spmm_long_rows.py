@@ -238,6 +238,11 @@ def test_long_rows_whose_bands_are_unlike(torch_gpu, handle, oracle, how):
     check(torch_gpu, handle, oracle, a, 32, -1.5, 0.5)
 
 
+def test_long_rows_in_more_than_64_bands(torch_gpu, handle, oracle):
+    a = banded_matrix(np.float32, k=4300000)
+    check(torch_gpu, handle, oracle, a, 16, 1.25, -0.5)  # op(B): 275 MB, bands of 4 MB
+
+
 def test_every_way_to_bands_gives_the_same_bits(torch_gpu, oracle):
     torch = torch_gpu
     side = torch.cuda.Stream()
