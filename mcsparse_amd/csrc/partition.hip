@@ -128,8 +128,12 @@ __global__ __launch_bounds__(THREADS) void partition_kernel(EntrySource in, uint
     constexpr int kWaves = THREADS / kWave;
     constexpr bool kOrdered = KIND != kProducts;  // products: the entries of a digit may follow each other in any order
     typedef typename WordOf<VB>::type word_t;
-    __shared__ __align__(16) uint32_t s_buf[kPlaces];
-    __shared__ __align__(16) uint16_t s_cnt[kOrdered ? kWaves << MAX_BITS : 2 << MAX_BITS];
+    // plain: the counts' place is the words' afterwards (nothing is staged before)
+    constexpr uint32_t kCounts = kOrdered ? kWaves << MAX_BITS : 2 << MAX_BITS;
+    constexpr bool kOnePlace = KIND == kPlain;
+    __shared__ __align__(16) uint32_t s_buf[kOnePlace && kCounts / 2 > kPlaces ? kCounts / 2 : kPlaces];
+    __shared__ __align__(16) uint16_t s_apart[kOnePlace ? 8 : kCounts];
+    uint16_t* const s_cnt = kOnePlace ? reinterpret_cast<uint16_t*>(s_buf) : s_apart;
     __shared__ uint32_t s_wave[kWaves];
     __shared__ TileRows<KIND != kPlain ? kTile : kWave> s_rows;
 
@@ -165,7 +169,7 @@ __global__ __launch_bounds__(THREADS) void partition_kernel(EntrySource in, uint
         for (int i = 0; i < ITEMS; ++i) val[i] = TileReader(vals_in + first, count * VB).template read<word_t>(slab, i * kWave);
     };
     if constexpr (kValuesEarly) load_values();
-    for (uint32_t i = tid; i < sizeof(s_cnt) / 16; i += THREADS) reinterpret_cast<u32x4*>(s_cnt)[i] = u32x4(0);
+    for (uint32_t i = tid; i < kCounts / 8; i += THREADS) reinterpret_cast<u32x4*>(s_cnt)[i] = u32x4(0);
     __syncthreads();
 
     const uint32_t mask = (1u << bits) - 1u;
@@ -209,6 +213,7 @@ __global__ __launch_bounds__(THREADS) void partition_kernel(EntrySource in, uint
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) forget(key[i]);
 
+    if constexpr (kOnePlace) __syncthreads();  // the counts have been read
     if constexpr (KIND == kPlain) {
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) aux[i] = TileReader(in.aux + first, count * 4).read<uint32_t>(slab, i * kWave);
@@ -1264,9 +1269,10 @@ void launch_partition(hipStream_t stream, const EntrySource& in, uint32_t shift,
     const uint32_t tiles = tiles_of(in.count, tile_size);
     const uint32_t xcds = device_topology().xcds;
     const dim3 grid((tiles + xcds - 1) / xcds * xcds);
-    // Packed entries: 16 wavefronts with half the items each need half the registers and fill a compute unit (118 M entries,
-    // csr2csc 1163 -> 1139 us); with the counters of 11 bits they would fill it with one workgroup (85.6 -> 89.6 us, 2 M).
-    constexpr int kThreads = packed_entries<Key>() && MAX_BITS <= 8 ? 1024 : 512;
+    // 16 wavefronts with half the items each need half the registers and fill a compute unit: packed entries of csr2csc (118 M,
+    // 1163 -> 1139 us; with the counters of 11 bits they would fill it with one workgroup, 2 M: 85.6 -> 89.6), and index sorts,
+    // whose counts and words share their place (7.2 M triples, partition 42.9 -> 39.5 us; all of the assembly 185 -> 181).
+    constexpr int kThreads = KIND == kPlain || (packed_entries<Key>() && MAX_BITS <= 8) ? 1024 : 512;
     if (tile_size == kTileLarge) {
         hipLaunchKernelGGL((partition_kernel<VB, KIND, MAX_BITS, Key, kThreads, kTileLarge / kThreads>), grid, dim3(kThreads), 0,
                            stream, in, shift, bits, tiles, static_cast<Key*>(keys_out), aux_out, vals_out, table, xcds);
