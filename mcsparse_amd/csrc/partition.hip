@@ -756,6 +756,7 @@ struct BucketLds {
     __align__(16) uint16_t cnt[kBucketThreads / kWave << kPassBits];
     uint32_t wave[kBucketThreads / kWave];
     uint16_t key_begin[(1 << kPassBits) + 1];  // first place of each key, for short runs of keys
+    uint16_t long_run;                         // != 0: one of the runs is not short
     RunMap<kBucketRoom> map;
     __device__ __forceinline__ void clear_counts() {
         for (uint32_t i = threadIdx.x; i < sizeof(cnt) / 16; i += kBucketThreads) reinterpret_cast<u32x4*>(cnt)[i] = u32x4(0);
@@ -817,7 +818,10 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
     for (int p = key_first ? -1 : 0;; ++p) {
         SortPass pass = {false, MANY ? below : 0u, MANY ? upper : t.d3};
         if (MANY && p >= 0) pass = kPacked ? word_pass(t, static_cast<uint32_t>(p)) : sort_pass(t, static_cast<uint32_t>(p));
-        bool long_run = false;
+        if (MANY && p < 0 && tid == 0) {
+            s.long_run = 0;
+            s.key_begin[1u << upper] = static_cast<uint16_t>(count);
+        }
         const uint32_t mask = (1u << pass.bits) - 1u;
         auto digit = [&](int i) {
             const uint32_t of_aux = aux[i];  // (the values, so that neither array needs an address)
@@ -827,18 +831,25 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
         };
         rank_entries<ITEMS, kPassBits>(count, pass.bits, s.cnt, dest, digit);
         __syncthreads();
+        if constexpr (MANY && kPacked) {
+#pragma unroll
+            for (int i = 0; i < ITEMS; ++i) forget(aux[i]);
+        }
         place_digits<kBucketThreads, kPassBits>(pass.bits, s.cnt, s.wave, [&](uint32_t d, uint32_t at, uint32_t entries) {
             if (!MANY) {
                 write_key_ptr(out, sub, t.d3, d, first + at, t.count);
             } else if (p < 0) {
                 s.key_begin[d] = static_cast<uint16_t>(at);
-                if (d + 1 == 1u << upper) s.key_begin[d + 1] = static_cast<uint16_t>(count);
-                long_run |= entries > kShortRun;
+                if (entries > kShortRun) s.long_run = 1;
             }
         });
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i)
             dest[i / 2] += static_cast<uint32_t>(s.cnt[(wave << kPassBits) + digit(i)]) << (i % 2 * 16);
+        if constexpr (MANY && kPacked) {
+#pragma unroll
+            for (int i = 0; i < ITEMS; ++i) forget(aux[i]);
+        }
         if (!MANY || p + 1 == static_cast<int>(kPacked ? t.oversize_passes : t.passes)) break;
         auto back = [&](uint32_t (&word)[ITEMS]) {
             ordered([&](int i) { return word[i]; });
@@ -853,8 +864,9 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
             if (kPacked && p < 0) {
                 // (the words behind the last one are looked at too, and must not go in front of any)
                 if (tid < 4 - count % 4 && count % 4 != 0) s.buf[count + tid] = ~0u;
+                __syncthreads();
             }
-            if (p < 0 && !__syncthreads_or(long_run)) {
+            if (p < 0 && s.long_run == 0) {  // the same for the workgroup
                 // buf still holds the minor keys in this order: an entry's place is that of its run, plus the entries
                 // of the run that go before it
 #pragma unroll
@@ -924,9 +936,12 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
 // A workgroup per bucket.  118 M entries (16 bytes each) in buckets of 3600: 390 us, bound by vector instructions as much
 // as by memory; so most buckets, below two thirds of the room, run a version without the last third of the items (458 -> 445
 // us when an entry was 17 bytes in three arrays).  Packed pairs: another one without the last quarter, for the buckets of a
-// mean size (1.5 M rows, 6 M triples, all of the assembly: 274 -> 263 us).
+// mean size (1.5 M rows, 6 M triples, all of the assembly: 274 -> 263 us), and 64 registers, so that a compute unit has four
+// workgroups and not three (7.2 M triples of a mesh 181 -> 177, 2 M random ones 97 -> 93, 7.9 M 331 -> 322; with
+// __syncthreads_or for long_run, which holds the thread's three numbers all along, six registers went to scratch memory: 180, 94,
+// 326, and 0.6 M triples 52.8 -> 53.8, where it is 53.0 so).
 template <int VB, typename Key, bool MANY>
-__global__ __launch_bounds__(kBucketThreads, VB == 8 || MANY ? 6 : 8) void bucket_sort_kernel(SortTables t, const Key* __restrict__ keys_in,
+__global__ __launch_bounds__(kBucketThreads, VB == 8 || (MANY && !packed_entries<Key>()) ? 6 : 8) void bucket_sort_kernel(SortTables t, const Key* __restrict__ keys_in,
                                                                                       const uint32_t* __restrict__ aux_in,
                                                                                       const void* __restrict__ vals_in,
                                                                                       SortOutput out, uint32_t buckets,
