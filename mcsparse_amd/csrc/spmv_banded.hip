@@ -342,10 +342,10 @@ __global__ __launch_bounds__(kBlock) void column_order_pack_kernel(idx_t nnz, id
 constexpr int kColumnBlock = 1024;
 constexpr int kColumnSet32 = 12;
 constexpr int kColumnSet64 = 13;
-// fp32: the entries of a tile lie in blocks of kColumnQuad * 64, counted from the tile's first entry at a multiple
-// of kColumnQuad (the up to three entries ahead of it are taken one by one).  A block of L entries in column order is
-// stored so that lane l < L / 4 finds its entries l, L/4 + l, 2 L/4 + l, 3 L/4 + l of the block side by side at
-// 4 l .. 4 l + 3 (the last L % 4 entries stay where they are): one 128-bit load per lane brings a wavefront four
+// fp32: the entries of a tile lie in blocks of kColumnQuad * 64, counted from the multiple of kColumnQuad at or before the
+// tile's first entry; the up to three places of the first block that belong to the tile before are left out.  A block of L
+// places in column order is stored so that lane l < L / 4 finds its entries l, L/4 + l, 2 L/4 + l, 3 L/4 + l of the block side
+// by side at 4 l .. 4 l + 3 (the last L % 4 entries stay where they are): one 128-bit load per lane brings a wavefront four
 // runs of neighbouring entries (the vector memory unit takes a load instruction in the same time whatever its
 // width: power-law matrix 384 -> 343 us, its transpose 324 -> 295 us), an element is an entry of the block exactly
 // when its place is below L, and a tile's last, partial block needs no code of its own.  With fp64 values the same
@@ -370,8 +370,9 @@ __global__ __launch_bounds__(kColumnQuadBlock) void column_order_interleave_kern
     e0 = e0 < nnz ? e0 : nnz;
     e1 = e1 < nnz ? e1 : nnz;
     e1 = e1 > e0 ? e1 : e0;
-    const idx_t a0 = (e0 + kColumnQuad - 1) / kColumnQuad * kColumnQuad;
-    if (a0 >= e1) return;  // whole workgroup
+    if (e0 == e1) return;  // whole workgroup
+    const idx_t a0 = e0 / kColumnQuad * kColumnQuad;
+    const uint32_t foreign = e0 - a0;  // places of the first block that are the tile's before: neither moved nor counted
     const uint32_t len = e1 - a0;
     const uint32_t blocks = (len + kColumnQuadBlock - 1) / kColumnQuadBlock;
     __shared__ idx_t s_w[kInterleaveBlocks][kColumnQuadBlock];
@@ -389,10 +390,15 @@ __global__ __launch_bounds__(kColumnQuadBlock) void column_order_interleave_kern
 #pragma unroll
         for (int i = 0; i < kInterleaveBlocks; ++i) {
             const uint32_t first = (b0 + i) * kColumnQuadBlock;
-            if (first + p < len) {
+            if (first + p < len && first + p >= foreign) {
                 const uint32_t in_block = len - first < kColumnQuadBlock ? len - first : kColumnQuadBlock;
                 const uint32_t q = in_block / kColumnQuad;
-                const uint32_t to = p < q * kColumnQuad ? (p % q) * kColumnQuad + p / q : p;
+                uint32_t nth = p;  // of the block's places in the order of their lanes
+                if (first == 0) {  // the p - foreign-th of those that are this tile's: lane 0 lacks its first `foreign` ones
+                    nth -= foreign;
+                    for (uint32_t j = 0; j < foreign; ++j) nth += nth >= j * q ? 1u : 0u;
+                }
+                const uint32_t to = nth < q * kColumnQuad ? (nth % q) * kColumnQuad + nth / q : nth;
                 s_w[i][to] = w[i];
                 s_v[i][to] = v[i];
             }
@@ -401,7 +407,7 @@ __global__ __launch_bounds__(kColumnQuadBlock) void column_order_interleave_kern
 #pragma unroll
         for (int i = 0; i < kInterleaveBlocks; ++i) {
             const uint32_t first = (b0 + i) * kColumnQuadBlock;
-            if (first + p < len) {
+            if (first + p < len && first + p >= foreign) {
                 entries[a0 + first + p] = s_w[i][p];
                 vals[a0 + first + p] = s_v[i][p];
             }
@@ -448,6 +454,44 @@ __global__ __launch_bounds__(kBlock) void column_order_split_kernel(idx_t nnz, u
     if (tid <= kXcds) xcd_start[tid] = s_start[s_worst[1] <= s_worst[0] ? 1 : 0][tid];
 }
 
+// unit_order: the units of every stretch, group by group as they lie and inside a group by falling number of nonzeros, so that
+// what a workgroup takes last is small (power-law rows: units of a group differ 2:1, and eight of them are a workgroup's work).
+// {unit, first of its tiles that has entries (sub: none), where those begin, where they end}: all that a workgroup needs to ask
+// for a unit's first entries, in one load.
+// A workgroup per stretch.  Longer stretches than kOrderedUnits, which are dozens of units to a workgroup, stay as they lie.
+constexpr uint32_t kOrderedUnits = 2048;
+constexpr int kOrderBlock = 1024;
+__global__ __launch_bounds__(kOrderBlock) void column_order_rank_kernel(idx_t nnz, uint32_t units, uint32_t chunks, uint32_t sub,
+                                                                        const idx_t* __restrict__ tile_ptr,
+                                                                        const uint32_t* __restrict__ xcd_start,
+                                                                        uint4* __restrict__ unit_order) {
+    auto record = [&](uint32_t unit) {
+        const idx_t* bounds = tile_ptr + static_cast<uint64_t>(unit) * sub;
+        uint32_t b = 0;
+        while (b < sub && bounds[b] == bounds[b + 1]) ++b;
+        return make_uint4(unit, b, bounds[b], bounds[min(b + 1, sub)]);
+    };
+    __shared__ unsigned long long s_key[kOrderedUnits];  // group, then the nonzeros, the largest first
+    const uint32_t first = min(xcd_start[blockIdx.x], units), end = min(xcd_start[blockIdx.x + 1], units);
+    const uint32_t count = end > first ? end - first : 0;
+    if (count > kOrderedUnits) {  // whole workgroup
+        for (uint32_t i = threadIdx.x; i < count; i += kOrderBlock) unit_order[first + i] = record(first + i);
+        return;
+    }
+    for (uint32_t i = threadIdx.x; i < count; i += kOrderBlock) {
+        const uint64_t tile = static_cast<uint64_t>(first + i) * sub;
+        const uint32_t held = tile_ptr[tile + sub] - tile_ptr[tile];
+        s_key[i] = static_cast<unsigned long long>((first + i) / chunks) << 32 | (nnz - min(held, nnz));
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < count; i += kOrderBlock) {
+        const unsigned long long mine = s_key[i];
+        uint32_t before = 0;
+        for (uint32_t j = 0; j < count; ++j) before += s_key[j] < mine || (s_key[j] == mine && j < i) ? 1u : 0u;
+        unit_order[first + before] = record(first + i);
+    }
+}
+
 // Adds product p to the sum of row r of the tile, for one entry per lane of a wavefront of which most lanes hold row
 // `lead` (a row with an entry in nearly every column of the band: LDS would take the adds to its sum one after the
 // other).  Those lanes are summed in registers and added once.  live: this lane's entry exists.
@@ -477,192 +521,260 @@ __global__ __launch_bounds__(kColumnBlock) void spmv_column_order_kernel(idx_t m
                                                                         uint32_t chunks, uint32_t units, uint32_t sub,
                                                                         const XcdStarts stretches,
                                                                         uint32_t* __restrict__ next_unit,
+                                                                        const uint4* __restrict__ unit_order,
                                                                         const idx_t* __restrict__ tile_ptr,
                                                                         const idx_t* __restrict__ entries,
                                                                         const T* __restrict__ vals,
                                                                         const T* __restrict__ x,
                                                                         T* __restrict__ partials, T* __restrict__ y,
                                                                         T alpha, T beta) {
-    const uint32_t* xcd_start = stretches.first;
     extern __shared__ __align__(16) unsigned char s_raw[];
-    __shared__ uint32_t s_unit;
+    __shared__ uint32_t s_next;
     double* s_acc = reinterpret_cast<double*>(s_raw);
     const uint32_t tid = threadIdx.x;
     const uint32_t xcd = blockIdx.x % kXcds;
-    const uint32_t stretch_end = min(xcd_start[xcd + 1], units);
+    const uint32_t stretch_first = stretches.first[xcd], stretch_end = min(stretches.first[xcd + 1], units);
     const idx_t band_mask = (1u << band_shift) - 1u;
-    for (uint32_t r = tid; r < rows_per_tile; r += kColumnBlock) s_acc[r] = 0.0;
-    __syncthreads();
-    // The units of an XCD's stretch differ in size (power-law rows): a workgroup starts with the unit of
-    // its own number and takes the next off a counter whenever it gets free.  The counter starts at the
-    // number of workgroups per XCD: the reduce kernel of the call before, or the build, has left it so.
-    // Every workgroup ends when the counter has passed the stretch.
-    bool first = true;
-    while (true) {
-        if (tid == 0)
-            s_unit = xcd_start[xcd] + (first ? blockIdx.x / kXcds : atomicAdd(&next_unit[xcd], 1u));
-        first = false;
-        __syncthreads();
-        const uint32_t unit = s_unit;
-        __syncthreads();  // read by all before it is written again
-        if (unit >= stretch_end) break;  // whole workgroup; also where an overwritten counter ends up
-        const uint32_t group = unit / chunks;
-        const uint32_t chunk = unit - group * chunks;
-        const uint64_t row0 = static_cast<uint64_t>(chunk) * rows_per_tile;
-        if (row0 >= m) continue;  // whole workgroup
-        const uint32_t tile_rows = static_cast<uint32_t>(m - row0 < rows_per_tile ? m - row0 : rows_per_tile);
-        for (uint32_t b = 0; b < sub; ++b) {
-            const uint64_t tile = static_cast<uint64_t>(unit) * sub + b;
-            idx_t e0 = tile_ptr[tile];
-            idx_t e1 = tile_ptr[tile + 1];
-            e0 = e0 < nnz ? e0 : nnz;
-            e1 = e1 < nnz ? e1 : nnz;
-            e1 = e1 > e0 ? e1 : e0;
-            const idx_t band_key = (group * sub + b) << band_shift;
-            // Two sets of kSet entries per thread take turns.  A set is gathered for and added while the loads of
-            // the other are on their way: the gathers of a set are issued first, then the loads of the next set,
-            // and only then are the gathers waited for (loads return in the order they were issued, so a wait for
-            // gathers that had been issued after the next set's loads would wait for those as well; in that order
-            // 1 M rows x 16 in fp64 took 78.3 us and the power-law matrix in fp32 395 us, in this one 70.3 and 384).
-            constexpr int kSet = sizeof(T) == 4 ? kColumnSet32 : kColumnSet64;
-            constexpr idx_t kPart = kColumnBlock * kSet;  // entries the workgroup takes per set
-            idx_t packed[2][kSet];
-            T v[2][kSet];
-            // Element i of a thread's set lies at place(i) of the set.  In blocks: block i / 4 of the wavefront, at
-            // 4 * lane + i % 4; else entry by entry across the workgroup.
-            constexpr bool kQuads = column_order_quads<T>();
-            const uint32_t lane_first = (tid / kWave) * kColumnQuadBlock + (tid % kWave) * kColumnQuad;
-            auto place = [&](int i) {
-                if constexpr (kQuads) {
-                    return static_cast<uint32_t>(i / kColumnQuad) * (kColumnBlock * kColumnQuad) + lane_first +
-                           static_cast<uint32_t>(i % kColumnQuad);
-                } else {
-                    return static_cast<uint32_t>(i) * kColumnBlock + tid;
-                }
-            };
-            auto ask = [&](int h, idx_t start) {  // start < e1 (and a multiple of kColumnQuad where that matters)
-                const uint32_t cnt = e1 - start < kPart ? e1 - start : kPart;
-                if constexpr (kQuads) {
-                    typedef idx_t quad_t __attribute__((ext_vector_type(4)));
-                    const uint32_t last_quad = (cnt - 1) / kColumnQuad * kColumnQuad;
-#pragma unroll
-                    for (int j = 0; j < kSet / kColumnQuad; ++j) {
-                        // (array + start) + place: a uniform base and a small offset per lane, one register
-                        const uint32_t at = min(place(j * kColumnQuad), last_quad);
-                        const quad_t q = __builtin_nontemporal_load(reinterpret_cast<const quad_t*>((entries + start) + at));
-                        const quad_t f = __builtin_nontemporal_load(reinterpret_cast<const quad_t*>((vals + start) + at));
-                        packed[h][j * 4 + 0] = q.x;
-                        packed[h][j * 4 + 1] = q.y;
-                        packed[h][j * 4 + 2] = q.z;
-                        packed[h][j * 4 + 3] = q.w;
-                        v[h][j * 4 + 0] = __uint_as_float(f.x);
-                        v[h][j * 4 + 1] = __uint_as_float(f.y);
-                        v[h][j * 4 + 2] = __uint_as_float(f.z);
-                        v[h][j * 4 + 3] = __uint_as_float(f.w);
-                    }
-                } else {
-#pragma unroll
-                    for (int i = 0; i < kSet; ++i) {
-                        const uint32_t k = min(place(i), cnt - 1);
-                        packed[h][i] = load_stream(entries + start + k);
-                        v[h][i] = load_stream(vals + start + k);
-                    }
-                }
-            };
-            auto gather = [&](int h, T (&xv)[kSet]) {
-#pragma unroll
-                for (int i = 0; i < kSet; ++i) {
-                    idx_t key = band_key | (packed[h][i] & band_mask);  // column + base
-                    key = key > base ? key : base;
-                    xv[i] = x[min(key - base, n - 1)];
-                }
-            };
-            auto add = [&](int h, idx_t start, const T (&xv)[kSet], bool whole_set) {
-                const uint32_t cnt = e1 - start < kPart ? e1 - start : kPart;
-                // a row past the end of the tile (an overwritten layout) still lies inside the sums
-                if constexpr (CROWD) {
-                    const uint32_t r_first = min(packed[h][0] >> band_shift, rows_per_tile - 1);
-                    const uint32_t lead = __builtin_amdgcn_readfirstlane(r_first);
-                    if (__popcll(__ballot(r_first == lead)) >= kCrowdedLanes) {  // whole wavefront
-#pragma unroll
-                        for (int i = 0; i < kSet; ++i) {
-                            const uint32_t k = place(i);
-                            const uint32_t r = min(packed[h][i] >> band_shift, rows_per_tile - 1);
-                            add_to_crowded_row(s_acc, r, static_cast<double>(v[h][i] * xv[i]), whole_set || k < cnt, lead);
-                        }
-                        return;
-                    }
-                }
-#pragma unroll
-                for (int i = 0; i < kSet; ++i) {
-                    const uint32_t k = place(i);
-                    const uint32_t r = min(packed[h][i] >> band_shift, rows_per_tile - 1);
-                    if (whole_set || k < cnt) unsafeAtomicAdd(&s_acc[r], static_cast<double>(v[h][i] * xv[i]));
-                }
-            };
-            // A set with a successor: gathers, then the successor's loads, then the adds.  The loads are not
-            // made conditional inside it: the compiler then counts the loads in flight for the path without them
-            // and waits for all of them before the first add.  The last set of a tile runs without.
-            auto step = [&](int h, idx_t start) {
-                T xv[kSet];
-                gather(h, xv);
-                __builtin_amdgcn_sched_barrier(0);
-                ask(h ^ 1, start + kPart);
-                __builtin_amdgcn_sched_barrier(0);
-                add(h, start, xv, true);
-            };
-            auto last = [&](int h, idx_t start) {
-                T xv[kSet];
-                gather(h, xv);
-                add(h, start, xv, false);
-            };
-            if constexpr (kQuads) {  // the entries ahead of the first multiple of kColumnQuad, a lane each
-                const idx_t a0 = (e0 + kColumnQuad - 1) / kColumnQuad * kColumnQuad;
-                const idx_t head_end = a0 < e1 ? a0 : e1;
-                if (tid < head_end - e0) {
-                    const idx_t w = entries[e0 + tid];
-                    idx_t key = band_key | (w & band_mask);
-                    key = key > base ? key : base;
-                    const uint32_t r = min(w >> band_shift, rows_per_tile - 1);
-                    unsafeAtomicAdd(&s_acc[r], static_cast<double>(vals[e0 + tid] * x[min(key - base, n - 1)]));
-                }
-                e0 = head_end;
-            }
-            if (e0 < e1) {
-                ask(0, e0);
-                idx_t start = e0;
-                int h = 0;  // the set that holds the entries from `start` (the same for the workgroup)
-                while (e1 - start > kPart) {
-                    step(0, start);
-                    start += kPart;
-                    h = 1;
-                    if (e1 - start <= kPart) break;
-                    step(1, start);
-                    start += kPart;
-                    h = 0;
-                }
-                if (h == 0) last(0, start);
-                else last(1, start);
-            }
+    // What the build has left and no kernel of this call writes, at places that are the same for the workgroup: scalar loads,
+    // which the entries on their way need not be waited for.
+    typedef const __attribute__((address_space(4))) uint32_t* scalar_words;
+    const scalar_words bounds = reinterpret_cast<scalar_words>(reinterpret_cast<uintptr_t>(tile_ptr));
+    const scalar_words order = reinterpret_cast<scalar_words>(reinterpret_cast<uintptr_t>(unit_order));
+
+    // Two sets of kSet entries per thread take turns.  A set is gathered for and added while the loads of
+    // the other are on their way: the gathers of a set are issued first, then the loads of the next set,
+    // and only then are the gathers waited for (loads return in the order they were issued, so a wait for
+    // gathers that had been issued after the next set's loads would wait for those as well; in that order
+    // 1 M rows x 16 in fp64 took 78.3 us and the power-law matrix in fp32 395 us, in this one 70.3 and 384).
+    constexpr int kSet = sizeof(T) == 4 ? kColumnSet32 : CROWD ? kColumnSet64 - 2 : kColumnSet64;
+    constexpr idx_t kPart = kColumnBlock * kSet;  // entries the workgroup takes per set
+    constexpr bool kQuads = column_order_quads<T>();
+    idx_t packed[2][kSet];
+    T v[2][kSet];
+
+    // The set a workgroup is at: the places [start, start + kPart) of the entries, of which those from `skip` on and below
+    // `count` belong to the tile; `end` is the tile's.  start is a multiple of kColumnQuad where entries lie in blocks.
+    struct Part {
+        idx_t start, end;
+        uint32_t skip, count;
+        idx_t band_key;
+    };
+    auto first_part = [&](idx_t e0, idx_t e1, uint32_t band) {
+        Part p;
+        p.start = kQuads ? e0 / kColumnQuad * kColumnQuad : e0;
+        p.end = e1;
+        p.skip = e0 - p.start;
+        p.count = min(e1 - p.start, kPart);
+        p.band_key = band << band_shift;
+        return p;
+    };
+    // the first set of the first tile from `tile` on that has entries; none: tile = tile_end and an empty set
+    auto seek = [&](uint64_t& tile, uint64_t tile_end, uint32_t band) {
+        Part p = {0, 0, 0, 0, 0};
+        for (; tile < tile_end; ++tile, ++band) {
+            const idx_t e0 = min(bounds[tile], nnz), e1 = min(bounds[tile + 1], nnz);
+            if (e0 >= e1) continue;
+            p = first_part(e0, e1, band);
+            break;
         }
-        __syncthreads();
-        if constexpr (DIRECT) {
-            T* out = y + row0;
-            for (uint32_t r = tid; r < rows_per_tile; r += kColumnBlock) {
-                if (r < tile_rows) {
-                    const T sum = alpha * static_cast<T>(s_acc[r]);
-                    out[r] = beta == T(0) ? sum : sum + beta * out[r];
-                }
-                s_acc[r] = 0.0;
+        return p;
+    };
+    // Element i of a thread's set lies at place(i) of the set.  In blocks: block i / 4 of the wavefront, at
+    // 4 * lane + i % 4; else entry by entry across the workgroup.
+    const uint32_t lane_first = (tid / kWave) * kColumnQuadBlock + (tid % kWave) * kColumnQuad;
+    auto place = [&](int i) {
+        if constexpr (kQuads) {
+            return static_cast<uint32_t>(i / kColumnQuad) * (kColumnBlock * kColumnQuad) + lane_first +
+                   static_cast<uint32_t>(i % kColumnQuad);
+        } else {
+            return static_cast<uint32_t>(i) * kColumnBlock + tid;
+        }
+    };
+    auto ask = [&](int h, const Part& p) {
+        const uint32_t last_place = p.count != 0 ? p.count - 1 : 0;  // (an empty set reads the arrays' first elements)
+        if constexpr (kQuads) {
+            typedef idx_t quad_t __attribute__((ext_vector_type(4)));
+            const uint32_t last_quad = last_place / kColumnQuad * kColumnQuad;
+#pragma unroll
+            for (int j = 0; j < kSet / kColumnQuad; ++j) {
+                // (array + start) + place: a uniform base and a small offset per lane, one register
+                const uint32_t at = min(place(j * kColumnQuad), last_quad);
+                const quad_t q = __builtin_nontemporal_load(reinterpret_cast<const quad_t*>((entries + p.start) + at));
+                const quad_t f = __builtin_nontemporal_load(reinterpret_cast<const quad_t*>((vals + p.start) + at));
+                packed[h][j * 4 + 0] = q.x;
+                packed[h][j * 4 + 1] = q.y;
+                packed[h][j * 4 + 2] = q.z;
+                packed[h][j * 4 + 3] = q.w;
+                v[h][j * 4 + 0] = __uint_as_float(f.x);
+                v[h][j * 4 + 1] = __uint_as_float(f.y);
+                v[h][j * 4 + 2] = __uint_as_float(f.z);
+                v[h][j * 4 + 3] = __uint_as_float(f.w);
             }
         } else {
-            T* out = partials + static_cast<uint64_t>(group) * m + row0;
-            for (uint32_t r = tid; r < rows_per_tile; r += kColumnBlock) {
-                if (r < tile_rows) out[r] = static_cast<T>(s_acc[r]);
-                s_acc[r] = 0.0;
+#pragma unroll
+            for (int i = 0; i < kSet; ++i) {
+                const uint32_t k = min(place(i), last_place);
+                packed[h][i] = load_stream((entries + p.start) + k);
+                v[h][i] = load_stream((vals + p.start) + k);
             }
         }
+    };
+    auto gather = [&](int h, idx_t band_key, T (&xv)[kSet]) {
+#pragma unroll
+        for (int i = 0; i < kSet; ++i) {
+            idx_t key = band_key | (packed[h][i] & band_mask);  // column + base
+            key = key > base ? key : base;
+            xv[i] = x[min(key - base, n - 1)];
+        }
+    };
+    auto add = [&](int h, const Part& p, const T (&xv)[kSet]) {
+        auto live = [&](int i) { return place(i) - p.skip < p.count - p.skip; };
+        // a row past the end of the tile (an overwritten layout) still lies inside the sums
+        if constexpr (CROWD) {
+            const uint32_t r_first = min(packed[h][0] >> band_shift, rows_per_tile - 1);
+            const uint32_t lead = __builtin_amdgcn_readfirstlane(r_first);
+            if (__popcll(__ballot(r_first == lead)) >= kCrowdedLanes) {  // whole wavefront
+#pragma unroll
+                for (int i = 0; i < kSet; ++i) {
+                    const uint32_t r = min(packed[h][i] >> band_shift, rows_per_tile - 1);
+                    add_to_crowded_row(s_acc, r, static_cast<double>(v[h][i] * xv[i]), live(i), lead);
+                }
+                return;
+            }
+        }
+        auto each = [&](auto whole) {
+#pragma unroll
+            for (int i = 0; i < kSet; ++i) {
+                const uint32_t r = min(packed[h][i] >> band_shift, rows_per_tile - 1);
+                if (decltype(whole)::value || live(i)) unsafeAtomicAdd(&s_acc[r], static_cast<double>(v[h][i] * xv[i]));
+            }
+        };
+        // (fp64: without a test per entry 1 M rows x 16 take 68.4 us instead of 69.7; fp32: a second copy of the adds costs 308 ->
+        // 315 us on the power-law matrix)
+        if (sizeof(T) == 8 && p.count == kPart) each(std::true_type{});  // whole workgroup
+        else each(std::false_type{});
+    };
+
+    // The units of an XCD's stretch differ in size (power-law rows): a workgroup starts with the unit at
+    // its own place and takes the next place off a counter when it has two sets left.  The counter starts at the
+    // number of workgroups per XCD: the reduce kernel of the call before, or the build, has left it so.
+    // Every workgroup ends when the counter has passed the stretch.
+    uint32_t at = stretch_first + blockIdx.x / kXcds;
+    uint32_t unit = 0;
+    uint64_t tile = 0, tile_end = 0;
+    idx_t unit_end = 0;
+    auto begin_unit = [&]() {  // and its first set
+        const uint32_t record[4] = {order[4 * static_cast<uint64_t>(at)], order[4 * static_cast<uint64_t>(at) + 1],
+                                    order[4 * static_cast<uint64_t>(at) + 2], order[4 * static_cast<uint64_t>(at) + 3]};
+        unit = min(record[0], units - 1);
+        const uint32_t band = min(record[1], sub);
+        tile = static_cast<uint64_t>(unit) * sub + band;
+        tile_end = static_cast<uint64_t>(unit) * sub + sub;
+        unit_end = bounds[tile_end];
+        const idx_t e0 = min(record[2], nnz), e1 = min(record[3], nnz);
+        const Part empty = {0, 0, 0, 0, 0};
+        return e0 < e1 ? first_part(e0, e1, unit / chunks * sub + band) : empty;
+    };
+    Part now = {0, 0, 0, 0, 0};
+    const bool any = at < stretch_end;  // the same for the workgroup
+    const bool one_each = stretch_end - stretch_first <= kColumnGroupsPerXcd;  // no unit is left for a second turn
+    if (any) {
+        now = begin_unit();
+        ask(0, now);
+    }
+    for (uint32_t r = tid; r < rows_per_tile; r += kColumnBlock) s_acc[r] = 0.0;
+    __syncthreads();
+    bool taken = false;    // s_next holds the place of the next unit, counted from the stretch's first, or will
+    uint32_t next_at = 0;
+    auto take = [&]() {
+        // (at an address the compiler takes for a lane's own: of a scalar one it makes an add for the wavefront, and waits for
+        // it and all loads on the spot)
+        uint32_t counter = xcd;
+        asm volatile("" : "+v"(counter));
+        return atomicAdd(&next_unit[counter], 1u);
+    };
+    auto write_sums = [&](uint32_t of_unit, bool more) {
         __syncthreads();
+        const uint32_t group = of_unit / chunks;
+        const uint64_t row0 = static_cast<uint64_t>(of_unit - group * chunks) * rows_per_tile;
+        const uint32_t tile_rows = row0 >= m ? 0 : static_cast<uint32_t>(m - row0 < rows_per_tile ? m - row0 : rows_per_tile);
+        T* out = DIRECT ? y + row0 : partials + static_cast<uint64_t>(group) * m + row0;
+        // (no loop: in front of one the compiler would wait for the loads on their way; and rows it cannot work out ahead
+        // and hold in registers)
+        uint32_t row = tid;
+        asm volatile("" : "+v"(row));
+#pragma unroll
+        for (uint32_t r0 = 0; r0 < kColumnOrderRows; r0 += kColumnBlock) {
+            const uint32_t r = r0 + row;
+            if (r < tile_rows) {
+                if constexpr (DIRECT) {
+                    const T sum = alpha * static_cast<T>(s_acc[r]);
+                    out[r] = beta == T(0) ? sum : sum + beta * out[r];
+                } else {
+                    out[r] = static_cast<T>(s_acc[r]);
+                }
+            }
+            if (more && r < rows_per_tile) s_acc[r] = 0.0;
+        }
+        if (more) __syncthreads();
+    };
+    // One set: its gathers, then the loads of the set that follows, the next unit's first one behind a unit's last, then the
+    // adds.  So the stream of entries does not pause between tiles and units: before, a tile's last set ran without a
+    // successor, and a unit's sums were written before the next unit was looked for (power-law matrix, 4 M rows, fp32, eight
+    // units of two tiles to a workgroup: 342 -> 324 us a call, and 309 with the units in the order of unit_order).
+    // The loads sit under no test: the compiler then counts the loads in flight for the path without them and waits
+    // for all of them before the first add.  (fp64, where a unit is often all that a workgroup has: the set behind which
+    // nothing follows has code of its own; fp32: 310 us instead of 313 without.)  False: that was the last one.
+    auto step = [&](int h) {
+        T xv[kSet];
+        gather(h, now.band_key, xv);
+        __builtin_amdgcn_sched_barrier(0);
+        Part next = now;
+        next.skip = 0;
+        bool unit_done = false, more = true;
+        const uint32_t unit_now = unit;
+        if (now.end - now.start > kPart) {
+            next.start = now.start + kPart;
+            next.count = min(now.end - next.start, kPart);
+        } else {
+            if (tile < tile_end) ++tile;
+            next = seek(tile, tile_end, unit / chunks * sub + static_cast<uint32_t>(tile + sub - tile_end));
+            if (tile >= tile_end) {
+                unit_done = true;
+                more = !one_each;
+                if (more) {
+                    if (!taken && tid == 0) s_next = take();
+                    __syncthreads();
+                    at = __builtin_amdgcn_readfirstlane(s_next);
+                    more = at < stretch_end - stretch_first;  // (also where an overwritten counter ends up)
+                    at += stretch_first;
+                    taken = false;
+                }
+                if (more) next = begin_unit();
+            }
+        }
+        if (sizeof(T) == 8 && !more) {
+            add(h, now, xv);
+            write_sums(unit_now, false);
+            return false;
+        }
+        const bool take_now = !unit_done && !taken && !one_each && unit_end - now.start <= 2 * kPart;
+        if (take_now) {
+            taken = true;
+            if (tid == 0) next_at = take();
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        ask(h ^ 1, next);
+        __builtin_amdgcn_sched_barrier(0);
+        add(h, now, xv);
+        if (take_now && tid == 0) s_next = next_at;  // (has come with the gathers)
+        now = next;
+        if (unit_done) write_sums(unit_now, true);
+        return more;
+    };
+    if (any) {
+        while (step(0) && step(1)) {
+        }
     }
     if constexpr (DIRECT) {
         // every workgroup comes here once, after its last look at a work counter
@@ -840,6 +952,7 @@ BandedLayout banded_layout(const BandedShape& s, idx_t m, idx_t nnz, size_t valu
     l.tile_ptr = off; off += align_up((static_cast<size_t>(s.tiles) + 1) * sizeof(idx_t));
     l.xcd_start = off; off += align_up((kXcds + 1) * sizeof(uint32_t));
     l.next_unit = off; off += align_up((kXcds + 1) * sizeof(uint32_t));  // the counters and the count of finished workgroups
+    l.unit_order = off; off += align_up(s.by_column ? s.tiles / s.sub * sizeof(uint4) : 0);
     l.entries = off; off += idx_bytes;
     l.vals = off; off += align_up(static_cast<size_t>(nnz) * value_bytes);
     l.partials = off; off += align_up(static_cast<size_t>(s.bands) * m * value_bytes);
@@ -886,6 +999,9 @@ void launch_column_order_build(hipStream_t stream, const BandedShape& s, idx_t m
     hipLaunchKernelGGL(column_order_split_kernel, dim3(1), dim3(kBlock), 0, stream, nnz, s.tiles / s.sub, s.sub,
                        reinterpret_cast<const idx_t*>(w + l.tile_ptr), reinterpret_cast<uint32_t*>(w + l.xcd_start),
                        reinterpret_cast<uint32_t*>(w + l.next_unit));
+    hipLaunchKernelGGL(column_order_rank_kernel, dim3(kXcds), dim3(kOrderBlock), 0, stream, nnz, s.tiles / s.sub, s.chunks, s.sub,
+                       reinterpret_cast<const idx_t*>(w + l.tile_ptr), reinterpret_cast<const uint32_t*>(w + l.xcd_start),
+                       reinterpret_cast<uint4*>(w + l.unit_order));
 }
 
 void launch_banded_build(hipStream_t stream, const BandedShape& s, idx_t m, idx_t nnz, idx_t base, const idx_t* row_ptr,
@@ -935,7 +1051,7 @@ bool launch_spmv_banded(hipStream_t stream, const BandedShape& s, uint32_t grid,
         hipLaunchKernelGGL(kernel, dim3(kColumnGroupsPerXcd * kXcds), dim3(kColumnBlock), lds, stream, a.m, a.n, a.nnz,
                            a.base, s.band_shift, s.rows_per_tile, s.chunks, s.tiles / s.sub, s.sub,
                            stretches, reinterpret_cast<uint32_t*>(w + l.next_unit),
-                           reinterpret_cast<const idx_t*>(w + l.tile_ptr), reinterpret_cast<const idx_t*>(w + l.entries),
+                           reinterpret_cast<const uint4*>(w + l.unit_order), reinterpret_cast<const idx_t*>(w + l.tile_ptr), reinterpret_cast<const idx_t*>(w + l.entries),
                            reinterpret_cast<const T*>(w + l.vals), static_cast<const T*>(a.x), partials,
                            static_cast<T*>(a.y), alpha, beta);
         if (direct) return launches_taken();

@@ -439,3 +439,22 @@ def test_a_call_in_the_other_direction_on_the_same_buffer_ends_the_copy(torch_gp
     assert api.spmv(handle, api.OP_N, 1.5, mat, vxn, 0.5, vyn, ct, buf, alg=alg) == api.STATUS_SUCCESS
     torch.cuda.synchronize()
     assert_within(d_yn.cpu().numpy(), ref_n, bound_n, np.float64, what="A x after the copy was written over")
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("m,n,nnz,band_bytes", [
+    (110000, 2200000, 2500, 0),         # fp32: two tiles to a unit; most tiles hold a few entries, many none
+    (140003, 30011, 3000, 1 << 12),     # 30 or 59 planes: several units to a workgroup
+    (140003, 30011, 400000, 1 << 12),
+    (1 << 22, 1 << 14, 20000, 1 << 10), # fp32: more units to an XCD than are put in order of size
+])
+def test_tiles_and_units_of_a_few_entries_or_none(torch_gpu, handle, oracle, dtype, m, n, nnz, band_bytes):
+    """Where one tile or unit ends the next one's entries are on their way already: tiles that begin anywhere in a block of
+    four entries, that are shorter than one, and units without entries, whose sums are zero all the same."""
+    if dtype == np.float64 and m == 1 << 22:
+        band_bytes = 1 << 11
+    rng = np.random.default_rng(91)
+    rows = np.sort(rng.integers(0, m, nnz))
+    ptr = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=m))])
+    a = wl.Csr(m, n, ptr, rng.integers(0, n, nnz), rng.integers(-8, 9, nnz).astype(dtype))
+    run(torch_gpu, handle, oracle, a, 2.0, -1.0, band_bytes=band_bytes)
