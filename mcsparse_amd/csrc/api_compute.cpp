@@ -258,7 +258,8 @@ bool banded_candidate(const mcsparseSpMatDescr* A, mcsparseOperation_t op, mcspa
     // column order with sums formed in LDS as the products arrive, where the shape allows it.
     if (alg != MCSPARSE_SPMV_CSR_ALG2 &&
         mcsp::column_order_shape(static_cast<idx_t>(rows), static_cast<idx_t>(cols), static_cast<idx_t>(A->nnz),
-                                 static_cast<idx_t>(A->idxBase), value_size(A->valueType), band_bytes, shape))
+                                 static_cast<idx_t>(A->idxBase), value_size(A->valueType), band_bytes,
+                                 A->banded.band_bytes == 0, shape))
         return true;
     return mcsp::banded_shape(static_cast<idx_t>(rows), static_cast<idx_t>(cols), static_cast<idx_t>(A->nnz),
                               static_cast<idx_t>(A->idxBase), value_size(A->valueType), band_bytes, shape);
@@ -1057,8 +1058,8 @@ mcsparseStatus_t mcsparseSpMV_preprocess(mcsparseHandle_t handle, mcsparseOperat
                 size_t all_of_x = mcsp::kBandedBandBytes;
                 while (all_of_x < (static_cast<size_t>(gathered) + base) * vb) all_of_x *= 2;
                 BandedShape wide;
-                if (mcsp::column_order_shape(m, gathered, nnz, base, vb, all_of_x, &wide) &&
-                    wide.rows_per_tile == shape.rows_per_tile &&
+                if (mcsp::column_order_shape(m, gathered, nnz, base, vb, all_of_x, true, &wide) &&
+                    mcsp::column_order_halved_rows(m, 1) == mcsp::column_order_halved_rows(m, shape.bands) &&
                     align_up(mcsp::banded_layout(wide, m, nnz, vb).total) <= room)
                     shape = wide;
             }
@@ -1078,7 +1079,7 @@ mcsparseStatus_t mcsparseSpMV_preprocess(mcsparseHandle_t handle, mcsparseOperat
             // the nonzeros of the transpose sorted by its columns are the arrays as they lie: its
             // columns are the rows of the view, its rows the column indices
             mcsp::launch_csr2coo(handle->stream, static_cast<idx_t>(v.m), nnz, v.ptr, base, src_rows);
-            mcsp::launch_column_order_build(handle->stream, shape, m, nnz, base, v.ind, src_rows, matA->vals, vb, region);
+            mcsp::launch_column_order_build(handle->stream, shape, m, nnz, base, nullptr, v.ind, src_rows, matA->vals, vb, region);
         } else {
             // what the kernel gains from is lanes that share a 128-byte line of x: the order of the columns
             // inside a line does not matter, so the sort leaves the bits that tell them apart alone
@@ -1086,8 +1087,8 @@ mcsparseStatus_t mcsparseSpMV_preprocess(mcsparseHandle_t handle, mcsparseOperat
             mcsp::launch_sort_by_column(handle->stream, static_cast<idx_t>(v.m), static_cast<idx_t>(v.n), nnz, base, v.ptr,
                                         v.ind, matA->vals, vb, line_bits, src_cols, src_rows, region + cl.src_vals,
                                         region + cl.sort_ws);
-            mcsp::launch_column_order_build(handle->stream, shape, m, nnz, base, src_rows, src_cols, region + cl.src_vals,
-                                            vb, region);
+            mcsp::launch_column_order_build(handle->stream, shape, m, nnz, base, matA->banded.band_bytes == 0 ? v.ptr : nullptr,
+                                            src_rows, src_cols, region + cl.src_vals, vb, region);
         }
     } else if (v.transpose) {
         // the transpose in CSR form, behind the banded copy it is only the source of

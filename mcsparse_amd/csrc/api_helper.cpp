@@ -406,7 +406,13 @@ mcsparseStatus_t mcsparseSpMatGetSpMVPreprocess(mcsparseSpMatDescr_t d, int* sta
         return to_public_status(MCSP_STATUS_INVALID_POINTER);
     *state = !d->banded.valid ? 0 : (!d->banded.useful ? 1 : (d->banded.shape.by_column ? 3 : 2));
     *bands = d->banded.valid && d->banded.useful ? static_cast<int>(d->banded.shape.bands) : 0;
-    *rows_per_tile = d->banded.valid && d->banded.useful ? static_cast<int>(d->banded.shape.rows_per_tile) : 0;
+    *rows_per_tile = 0;
+    if (d->banded.valid && d->banded.useful) {
+        uint32_t rows = d->banded.shape.rows_per_tile;
+        // (tiles of any number of rows: the power of two at or below their mean)
+        if (d->banded.shape.by_column) rows = 1u << (mcsp::bit_length(d->banded.shape.mean_rows) - 1);
+        *rows_per_tile = static_cast<int>(rows);
+    }
     return MCSPARSE_STATUS_SUCCESS;
 }
 

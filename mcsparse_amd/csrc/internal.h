@@ -113,10 +113,12 @@ struct SpmmSchedule {
 // values: SpMV uses it only while the buffer, the three CSR arrays and the extents of the call are the
 // ones it was built from.
 struct BandedShape {
-    uint32_t band_shift;     // a band holds 2^band_shift keys (column index + index base)
+    uint32_t band_shift;     // a band holds 2^band_shift keys (column index + index base); by_column: band_keys of them, no more
+    uint32_t band_keys;
     uint32_t band_bits;      // bits needed to number the bands
     uint32_t bands;
-    uint32_t rows_per_tile;
+    uint32_t rows_per_tile;  // by_column: at most; mean_rows on average
+    uint32_t mean_rows;
     uint32_t chunks;         // row chunks = tiles per band
     uint32_t tiles;
     // false: entries of a tile in CSR order, row sums formed in a fixed order (bit-reproducible);
@@ -310,14 +312,19 @@ struct BandedLayout {
     size_t src_cols, src_rows, src_vals, tile_ids;
     size_t next_unit;  // by_column: one work counter per XCD
     size_t unit_order;  // by_column: the order in which the units of every stretch are taken
+    size_t chunk_first;  // by_column: first row of every chunk
 };
-// The same decision for the copy whose tiles are in column order (BandedShape::by_column): tiles of
-// kColumnOrderMinRows .. kColumnOrderRows rows, at most 64 planes of partial sums and 65536 tiles, and at
-// least one unit of work per compute unit.
+// The same decision for the copy whose tiles are in column order (BandedShape::by_column): tiles of up to kColumnOrderRows
+// rows, at most 64 planes of partial sums and 65536 tiles, and at least one unit of work per compute unit.
+// even: the tiles are cut as tall as give every compute unit the same number of units, all of a matrix's rows to be had in so
+// many turns.  Else kColumnOrderRows is halved until there is a unit for each, down to kColumnOrderMinRows, and the
+// compute units may be left with a turn in which most have no unit.
 constexpr uint32_t kColumnOrderRows = 16384;
 constexpr uint32_t kColumnOrderMinRows = 2048;
-bool column_order_shape(idx_t m, idx_t n, idx_t nnz, idx_t base, size_t value_bytes, size_t band_bytes,
+constexpr uint32_t kColumnOrderMinEvenRows = 512;
+bool column_order_shape(idx_t m, idx_t n, idx_t nnz, idx_t base, size_t value_bytes, size_t band_bytes, bool even,
                         BandedShape* out);
+uint32_t column_order_halved_rows(idx_t m, uint64_t groups);
 // How the gathers of an SpMV are spread over the 128-byte lines of x: launch_line_gathers fills, at the head of
 // `workspace` (line_gathers_workspace_bytes), kLineGatherBins pairs (lines, gathers) binned by the highest bit of a
 // line's count: of_rows from the row lengths (the gathered element is the row: a transposing direction), else from
@@ -331,7 +338,8 @@ bool gathers_favour_wide_groups(const unsigned long long* bins);
 // r_keys / c_keys: row + base and column + base of every nonzero of the matrix to copy, in an order
 // sorted by the 128-byte line of x the column lies in (any order inside a line); vals in the same
 // order.  Neither is written.
-void launch_column_order_build(hipStream_t stream, const BandedShape& s, idx_t m, idx_t nnz, idx_t base,
+// row_ptr: that matrix's row offsets, if there are any (else null).
+void launch_column_order_build(hipStream_t stream, const BandedShape& s, idx_t m, idx_t nnz, idx_t base, const idx_t* row_ptr,
                                const idx_t* r_keys, const idx_t* c_keys, const void* vals, size_t value_bytes,
                                void* region);
 // False when the banded copy cannot help or cannot be built: x fits one band, more than 256 bands.

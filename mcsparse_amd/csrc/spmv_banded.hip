@@ -23,6 +23,8 @@
 #include "device_util.h"
 #include "internal.h"
 
+#include <algorithm>
+
 namespace mcsp {
 
 namespace {
@@ -313,23 +315,65 @@ __global__ __launch_bounds__(kBlock) void banded_reduce_wide_kernel(idx_t m, uin
 // are neighbours in the tile list (tile = (group * chunks + chunk) * sub + band inside the group) and a
 // workgroup takes them in one go, keeping the row sums in LDS across them.
 //
+// chunk_first: the first row of every chunk, and m.  A chunk has at most rows_per_tile rows, on average mean_rows.  Where that
+// leaves room and there are row offsets (row_ptr), the chunks hold equally many nonzeros, else mean_rows rows each.
+constexpr uint32_t kCutChunks = 4096;
+constexpr int kCutBlock = 1024;
+__global__ __launch_bounds__(kCutBlock) void column_order_cut_kernel(idx_t m, idx_t nnz, idx_t base, const idx_t* __restrict__ row_ptr,
+                                                                     uint32_t chunks, uint32_t mean_rows, uint32_t rows_per_tile,
+                                                                     uint32_t* __restrict__ chunk_first) {
+    __shared__ long long s_cut[2][kCutChunks + 1];
+    const uint32_t tid = threadIdx.x;
+    if (row_ptr == nullptr || chunks > kCutChunks || mean_rows == rows_per_tile) {  // whole workgroup
+        for (uint32_t i = tid; i <= chunks; i += kCutBlock)
+            chunk_first[i] = static_cast<uint32_t>(min(static_cast<uint64_t>(i) * mean_rows, static_cast<uint64_t>(m)));
+        return;
+    }
+    // where chunk i should begin: t[i].  It may begin rows_per_tile rows behind the chunk before at most, so at
+    // min over j <= i of (t[j] + (i - j) * rows_per_tile); and not so early that the chunks left cannot hold the rows left.
+    for (uint32_t i = tid; i <= chunks; i += kCutBlock) {
+        const uint64_t target = static_cast<uint64_t>(nnz) * i / chunks;
+        uint64_t lo = 0, hi = m;  // first row with `target` or more nonzeros in front of it
+        while (lo < hi) {
+            const uint64_t mid = (lo + hi) / 2;
+            if (row_ptr[mid] - base < target) lo = mid + 1; else hi = mid;
+        }
+        s_cut[0][i] = static_cast<long long>(i == chunks ? m : lo) - static_cast<long long>(i) * rows_per_tile;
+    }
+    __syncthreads();
+    uint32_t from = 0;
+    for (uint32_t step = 1; step <= chunks; step *= 2, from ^= 1) {  // running minimum
+        for (uint32_t i = tid; i <= chunks; i += kCutBlock)
+            s_cut[from ^ 1][i] = i >= step ? min(s_cut[from][i], s_cut[from][i - step]) : s_cut[from][i];
+        __syncthreads();
+    }
+    for (uint32_t i = tid; i <= chunks; i += kCutBlock) {
+        const long long least = static_cast<long long>(m) - static_cast<long long>(chunks - i) * rows_per_tile;
+        const long long at = max(s_cut[from][i] + static_cast<long long>(i) * rows_per_tile, least);
+        chunk_first[i] = static_cast<uint32_t>(min(max(at, 0ll), static_cast<long long>(m)));
+    }
+}
+
 // Nonzero k (row key r, column key c, both with the index base in) gets its tile number and the same
 // packed word as above.  ids_out / packed_out may be the input arrays themselves (element k is read
 // before it is written).
-__global__ __launch_bounds__(kBlock) void column_order_pack_kernel(idx_t nnz, idx_t base, uint32_t band_shift,
-                                                                   uint32_t rows_per_tile, uint32_t chunks, uint32_t sub,
+__global__ __launch_bounds__(kBlock) void column_order_pack_kernel(idx_t nnz, idx_t base, uint32_t band_shift, uint32_t band_keys,
+                                                                   idx_t m, uint32_t mean_rows, uint32_t chunks, uint32_t sub,
+                                                                   const uint32_t* __restrict__ chunk_first,
                                                                    const idx_t* r_keys, const idx_t* c_keys,
                                                                    idx_t* ids_out, idx_t* packed_out) {
     const uint64_t k = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x;
     if (k >= nnz) return;
-    const idx_t band_mask = (1u << band_shift) - 1u;
     const idx_t key = c_keys[k];
-    const idx_t row = r_keys[k] - base;
-    const uint32_t chunk = row / rows_per_tile;
-    const uint32_t band = key >> band_shift;
+    const idx_t row = min(r_keys[k] - base, m - 1);
+    uint32_t chunk = min(row / mean_rows, chunks - 1);  // or one near it
+    uint32_t chunk_row = chunk_first[chunk];
+    while (chunk != 0 && row < chunk_row) chunk_row = chunk_first[--chunk];
+    for (uint32_t next; chunk + 1 < chunks && row >= (next = chunk_first[chunk + 1]); ++chunk) chunk_row = next;
+    const uint32_t band = key / band_keys;
     const uint32_t group = band / sub;
     ids_out[k] = (group * chunks + chunk) * sub + (band - group * sub);
-    packed_out[k] = ((row - chunk * rows_per_tile) << band_shift) | (key & band_mask);
+    packed_out[k] = ((row - chunk_row) << band_shift) | (key - band * band_keys);
 }
 
 // One workgroup per compute unit: workgroup i belongs to XCD i % 8 and takes every 32nd unit (the tiles
@@ -456,20 +500,31 @@ __global__ __launch_bounds__(kBlock) void column_order_split_kernel(idx_t nnz, u
 
 // unit_order: the units of every stretch, group by group as they lie and inside a group by falling number of nonzeros, so that
 // what a workgroup takes last is small (power-law rows: units of a group differ 2:1, and eight of them are a workgroup's work).
-// {unit, first of its tiles that has entries (sub: none), where those begin, where they end}: all that a workgroup needs to ask
-// for a unit's first entries, in one load.
+// A record says all that a workgroup needs to begin a unit and to write its sums, in one load.
+struct UnitRecord {
+    uint32_t unit;
+    uint32_t band;        // the first of its tiles that has entries; sub: none
+    uint32_t begin, end;  // that tile's entries
+    uint32_t unit_end;    // where the unit's entries end
+    uint32_t row, rows;   // rows of the matrix that it sums
+    uint32_t unused;
+};
+static_assert(sizeof(UnitRecord) == 32, "eight words");
 // A workgroup per stretch.  Longer stretches than kOrderedUnits, which are dozens of units to a workgroup, stay as they lie.
 constexpr uint32_t kOrderedUnits = 2048;
 constexpr int kOrderBlock = 1024;
 __global__ __launch_bounds__(kOrderBlock) void column_order_rank_kernel(idx_t nnz, uint32_t units, uint32_t chunks, uint32_t sub,
                                                                         const idx_t* __restrict__ tile_ptr,
                                                                         const uint32_t* __restrict__ xcd_start,
-                                                                        uint4* __restrict__ unit_order) {
+                                                                        const uint32_t* __restrict__ chunk_first,
+                                                                        UnitRecord* __restrict__ unit_order) {
     auto record = [&](uint32_t unit) {
         const idx_t* bounds = tile_ptr + static_cast<uint64_t>(unit) * sub;
+        const uint32_t chunk = unit % chunks;
         uint32_t b = 0;
         while (b < sub && bounds[b] == bounds[b + 1]) ++b;
-        return make_uint4(unit, b, bounds[b], bounds[min(b + 1, sub)]);
+        return UnitRecord{unit, b, bounds[b], bounds[min(b + 1, sub)], bounds[sub], chunk_first[chunk],
+                          chunk_first[chunk + 1] - chunk_first[chunk], 0};
     };
     __shared__ unsigned long long s_key[kOrderedUnits];  // group, then the nonzeros, the largest first
     const uint32_t first = min(xcd_start[blockIdx.x], units), end = min(xcd_start[blockIdx.x + 1], units);
@@ -512,16 +567,18 @@ struct XcdStarts {
 // wavefront meet on one row in the first entries of a slab, the slab's products for that row are summed in registers
 // (a matrix with dense rows: 0.78 -> 0.36 ms with one such row among 4 M, 0.99 -> 0.55 ms with four).  The test and
 // the second copy of the loop cost the kernel 2 to 10 % on matrices without such rows, which is why it is a variant.
+// ONE: no workgroup has a second unit, and none looks for one.
 // DIRECT: one band group spans all of x, so a unit's sums are the rows of y themselves: the kernel writes
 // y = alpha * sums + beta * y and no reduce kernel follows (11.7 us of 254 on the power-law matrix under op T).
 // The work counters are then put back by the workgroup that is through last: next_unit[kXcds] counts them.
-template <typename T, bool CROWD, bool DIRECT>
+template <typename T, bool CROWD, bool DIRECT, bool ONE>
 __global__ __launch_bounds__(kColumnBlock) void spmv_column_order_kernel(idx_t m, idx_t n, idx_t nnz, idx_t base,
-                                                                        uint32_t band_shift, uint32_t rows_per_tile,
+                                                                        uint32_t band_shift, uint32_t band_keys,
+                                                                        uint32_t rows_per_tile,
                                                                         uint32_t chunks, uint32_t units, uint32_t sub,
                                                                         const XcdStarts stretches,
                                                                         uint32_t* __restrict__ next_unit,
-                                                                        const uint4* __restrict__ unit_order,
+                                                                        const UnitRecord* __restrict__ unit_order,
                                                                         const idx_t* __restrict__ tile_ptr,
                                                                         const idx_t* __restrict__ entries,
                                                                         const T* __restrict__ vals,
@@ -565,7 +622,7 @@ __global__ __launch_bounds__(kColumnBlock) void spmv_column_order_kernel(idx_t m
         p.end = e1;
         p.skip = e0 - p.start;
         p.count = min(e1 - p.start, kPart);
-        p.band_key = band << band_shift;
+        p.band_key = band * band_keys;
         return p;
     };
     // the first set of the first tile from `tile` on that has entries; none: tile = tile_end and an empty set
@@ -622,12 +679,12 @@ __global__ __launch_bounds__(kColumnBlock) void spmv_column_order_kernel(idx_t m
     auto gather = [&](int h, idx_t band_key, T (&xv)[kSet]) {
 #pragma unroll
         for (int i = 0; i < kSet; ++i) {
-            idx_t key = band_key | (packed[h][i] & band_mask);  // column + base
+            idx_t key = band_key + (packed[h][i] & band_mask);  // column + base
             key = key > base ? key : base;
             xv[i] = x[min(key - base, n - 1)];
         }
     };
-    auto add = [&](int h, const Part& p, const T (&xv)[kSet]) {
+    auto add = [&](int h, const Part& p, const T (&xv)[kSet], bool whole_set = false) {
         auto live = [&](int i) { return place(i) - p.skip < p.count - p.skip; };
         // a row past the end of the tile (an overwritten layout) still lies inside the sums
         if constexpr (CROWD) {
@@ -642,17 +699,27 @@ __global__ __launch_bounds__(kColumnBlock) void spmv_column_order_kernel(idx_t m
                 return;
             }
         }
-        auto each = [&](auto whole) {
+        if constexpr (sizeof(T) == 4) {
+            // Lanes without an entry add to a sum that nobody reads, one of 64 behind the tile's.  (Under a branch the compiler
+            // sees a way past the adds, on which loads are still on their way to registers that the next set's gathers use
+            // again, and waits for those in front of them: power-law matrix 307 -> 310 us.  In fp64 the registers are too few.)
 #pragma unroll
             for (int i = 0; i < kSet; ++i) {
                 const uint32_t r = min(packed[h][i] >> band_shift, rows_per_tile - 1);
-                if (decltype(whole)::value || live(i)) unsafeAtomicAdd(&s_acc[r], static_cast<double>(v[h][i] * xv[i]));
+                unsafeAtomicAdd(&s_acc[live(i) ? r : rows_per_tile + tid % kWave], static_cast<double>(v[h][i] * xv[i]));
             }
-        };
-        // (fp64: without a test per entry 1 M rows x 16 take 68.4 us instead of 69.7; fp32: a second copy of the adds costs 308 ->
-        // 315 us on the power-law matrix)
-        if (sizeof(T) == 8 && p.count == kPart) each(std::true_type{});  // whole workgroup
-        else each(std::false_type{});
+        } else {
+            auto each = [&](auto whole) {
+#pragma unroll
+                for (int i = 0; i < kSet; ++i) {
+                    const uint32_t r = min(packed[h][i] >> band_shift, rows_per_tile - 1);
+                    if (decltype(whole)::value || live(i)) unsafeAtomicAdd(&s_acc[r], static_cast<double>(v[h][i] * xv[i]));
+                }
+            };
+            // (without a test per entry 1 M rows x 16 take 68.4 us instead of 69.7)
+            if (whole_set || p.count == kPart) each(std::true_type{});  // whole workgroup
+            else each(std::false_type{});
+        }
     };
 
     // The units of an XCD's stretch differ in size (power-law rows): a workgroup starts with the unit at
@@ -660,24 +727,30 @@ __global__ __launch_bounds__(kColumnBlock) void spmv_column_order_kernel(idx_t m
     // number of workgroups per XCD: the reduce kernel of the call before, or the build, has left it so.
     // Every workgroup ends when the counter has passed the stretch.
     uint32_t at = stretch_first + blockIdx.x / kXcds;
-    uint32_t unit = 0;
+    struct Unit {
+        uint32_t number;
+        idx_t end;            // of its entries
+        idx_t row;
+        uint32_t rows;
+    };
+    Unit unit = {0, 0, 0, 0};
     uint64_t tile = 0, tile_end = 0;
-    idx_t unit_end = 0;
     auto begin_unit = [&]() {  // and its first set
-        const uint32_t record[4] = {order[4 * static_cast<uint64_t>(at)], order[4 * static_cast<uint64_t>(at) + 1],
-                                    order[4 * static_cast<uint64_t>(at) + 2], order[4 * static_cast<uint64_t>(at) + 3]};
-        unit = min(record[0], units - 1);
-        const uint32_t band = min(record[1], sub);
-        tile = static_cast<uint64_t>(unit) * sub + band;
-        tile_end = static_cast<uint64_t>(unit) * sub + sub;
-        unit_end = bounds[tile_end];
-        const idx_t e0 = min(record[2], nnz), e1 = min(record[3], nnz);
+        const scalar_words r = order + static_cast<uint64_t>(at) * (sizeof(UnitRecord) / sizeof(uint32_t));
+        const UnitRecord record = {r[0], r[1], r[2], r[3], r[4], r[5], r[6], r[7]};
+        unit.number = min(record.unit, units - 1);
+        unit.end = record.unit_end;
+        unit.row = min(record.row, m);
+        unit.rows = min(min(record.rows, m - unit.row), rows_per_tile);
+        const uint32_t band = min(record.band, sub);
+        tile = static_cast<uint64_t>(unit.number) * sub + band;
+        tile_end = static_cast<uint64_t>(unit.number) * sub + sub;
+        const idx_t e0 = min(record.begin, nnz), e1 = min(record.end, nnz);
         const Part empty = {0, 0, 0, 0, 0};
-        return e0 < e1 ? first_part(e0, e1, unit / chunks * sub + band) : empty;
+        return e0 < e1 ? first_part(e0, e1, unit.number / chunks * sub + band) : empty;
     };
     Part now = {0, 0, 0, 0, 0};
     const bool any = at < stretch_end;  // the same for the workgroup
-    const bool one_each = stretch_end - stretch_first <= kColumnGroupsPerXcd;  // no unit is left for a second turn
     if (any) {
         now = begin_unit();
         ask(0, now);
@@ -693,38 +766,40 @@ __global__ __launch_bounds__(kColumnBlock) void spmv_column_order_kernel(idx_t m
         asm volatile("" : "+v"(counter));
         return atomicAdd(&next_unit[counter], 1u);
     };
-    auto write_sums = [&](uint32_t of_unit, bool more) {
+    auto write_sums = [&](const Unit& done, auto more) {
         __syncthreads();
-        const uint32_t group = of_unit / chunks;
-        const uint64_t row0 = static_cast<uint64_t>(of_unit - group * chunks) * rows_per_tile;
-        const uint32_t tile_rows = row0 >= m ? 0 : static_cast<uint32_t>(m - row0 < rows_per_tile ? m - row0 : rows_per_tile);
-        T* out = DIRECT ? y + row0 : partials + static_cast<uint64_t>(group) * m + row0;
-        // (no loop: in front of one the compiler would wait for the loads on their way; and rows it cannot work out ahead
-        // and hold in registers)
-        uint32_t row = tid;
-        asm volatile("" : "+v"(row));
-#pragma unroll
-        for (uint32_t r0 = 0; r0 < kColumnOrderRows; r0 += kColumnBlock) {
-            const uint32_t r = r0 + row;
-            if (r < tile_rows) {
-                if constexpr (DIRECT) {
-                    const T sum = alpha * static_cast<T>(s_acc[r]);
-                    out[r] = beta == T(0) ? sum : sum + beta * out[r];
-                } else {
-                    out[r] = static_cast<T>(s_acc[r]);
-                }
+        T* out = DIRECT ? y + done.row : partials + (static_cast<uint64_t>(done.number / chunks) * m + done.row);
+        auto write = [&](uint32_t r) {
+            if constexpr (DIRECT) {
+                const T sum = alpha * static_cast<T>(s_acc[r]);
+                out[r] = beta == T(0) ? sum : sum + beta * out[r];
+            } else {
+                out[r] = static_cast<T>(s_acc[r]);
             }
-            if (more && r < rows_per_tile) s_acc[r] = 0.0;
+        };
+        if constexpr (ONE) {
+            for (uint32_t r = tid; r < done.rows; r += kColumnBlock) write(r);
+        } else {
+            // (no loop: in front of one the compiler would wait for the loads on their way; and rows it cannot work out ahead
+            // and hold in registers)
+            uint32_t row = tid;
+            asm volatile("" : "+v"(row));
+#pragma unroll
+            for (uint32_t r0 = 0; r0 < kColumnOrderRows; r0 += kColumnBlock) {
+                const uint32_t r = r0 + row;
+                if (r < done.rows) write(r);
+                if (decltype(more)::value && r < rows_per_tile) s_acc[r] = 0.0;
+            }
+            if constexpr (decltype(more)::value) __syncthreads();
         }
-        if (more) __syncthreads();
     };
     // One set: its gathers, then the loads of the set that follows, the next unit's first one behind a unit's last, then the
     // adds.  So the stream of entries does not pause between tiles and units: before, a tile's last set ran without a
     // successor, and a unit's sums were written before the next unit was looked for (power-law matrix, 4 M rows, fp32, eight
     // units of two tiles to a workgroup: 342 -> 324 us a call, and 309 with the units in the order of unit_order).
     // The loads sit under no test: the compiler then counts the loads in flight for the path without them and waits
-    // for all of them before the first add.  (fp64, where a unit is often all that a workgroup has: the set behind which
-    // nothing follows has code of its own; fp32: 310 us instead of 313 without.)  False: that was the last one.
+    // for all of them before the first add.  (The set behind which nothing follows has code of its own, but for fp32 units that
+    // others follow: 313 us instead of 310.)  False: that was the last one.
     auto step = [&](int h) {
         T xv[kSet];
         gather(h, now.band_key, xv);
@@ -732,17 +807,17 @@ __global__ __launch_bounds__(kColumnBlock) void spmv_column_order_kernel(idx_t m
         Part next = now;
         next.skip = 0;
         bool unit_done = false, more = true;
-        const uint32_t unit_now = unit;
+        const Unit unit_now = unit;
         if (now.end - now.start > kPart) {
             next.start = now.start + kPart;
             next.count = min(now.end - next.start, kPart);
         } else {
             if (tile < tile_end) ++tile;
-            next = seek(tile, tile_end, unit / chunks * sub + static_cast<uint32_t>(tile + sub - tile_end));
+            next = seek(tile, tile_end, unit.number / chunks * sub + static_cast<uint32_t>(tile + sub - tile_end));
             if (tile >= tile_end) {
                 unit_done = true;
-                more = !one_each;
-                if (more) {
+                more = !ONE;
+                if constexpr (!ONE) {
                     if (!taken && tid == 0) s_next = take();
                     __syncthreads();
                     at = __builtin_amdgcn_readfirstlane(s_next);
@@ -753,12 +828,12 @@ __global__ __launch_bounds__(kColumnBlock) void spmv_column_order_kernel(idx_t m
                 if (more) next = begin_unit();
             }
         }
-        if (sizeof(T) == 8 && !more) {
+        if ((ONE || sizeof(T) == 8) && !more) {
             add(h, now, xv);
-            write_sums(unit_now, false);
+            write_sums(unit_now, std::false_type{});
             return false;
         }
-        const bool take_now = !unit_done && !taken && !one_each && unit_end - now.start <= 2 * kPart;
+        const bool take_now = !ONE && !unit_done && !taken && unit.end - now.start <= 2 * kPart;
         if (take_now) {
             taken = true;
             if (tid == 0) next_at = take();
@@ -769,14 +844,52 @@ __global__ __launch_bounds__(kColumnBlock) void spmv_column_order_kernel(idx_t m
         add(h, now, xv);
         if (take_now && tid == 0) s_next = next_at;  // (has come with the gathers)
         now = next;
-        if (unit_done) write_sums(unit_now, true);
+        if (!ONE && unit_done) write_sums(unit_now, std::true_type{});
         return more;
     };
-    if (any) {
+    if constexpr (ONE && sizeof(T) == 8) {
+        // A single tile, as a rule: less to hold in registers than in the steps below, which fp64 has none to spare for
+        // (1 M rows x 16 in those steps: 70.1 us a call instead of 68.8).
+        while (any) {
+            auto whole_step = [&](int h) {
+                T xv[kSet];
+                gather(h, now.band_key, xv);
+                __builtin_amdgcn_sched_barrier(0);
+                Part next = now;
+                next.skip = 0;
+                next.start = now.start + kPart;
+                next.count = min(now.end - next.start, kPart);
+                ask(h ^ 1, next);
+                __builtin_amdgcn_sched_barrier(0);
+                add(h, now, xv, true);
+                now = next;
+            };
+            auto last = [&](int h) {
+                T xv[kSet];
+                gather(h, now.band_key, xv);
+                add(h, now, xv);
+            };
+            int h = 0;
+            while (now.end - now.start > kPart) {
+                whole_step(0);
+                h = 1;
+                if (now.end - now.start <= kPart) break;
+                whole_step(1);
+                h = 0;
+            }
+            if (h == 0) last(0);
+            else last(1);
+            if (tile < tile_end) ++tile;
+            now = seek(tile, tile_end, unit.number / chunks * sub + static_cast<uint32_t>(tile + sub - tile_end));
+            if (tile >= tile_end) break;
+            ask(0, now);
+        }
+        if (any) write_sums(unit, std::false_type{});
+    } else if (any) {
         while (step(0) && step(1)) {
         }
     }
-    if constexpr (DIRECT) {
+    if constexpr (DIRECT && !ONE) {
         // every workgroup comes here once, after its last look at a work counter
         if (tid == 0 && atomicAdd(&next_unit[kXcds], 1u) == gridDim.x - 1) {
             for (uint32_t i = 0; i < kXcds; ++i) atomicExch(&next_unit[i], static_cast<uint32_t>(kColumnGroupsPerXcd));
@@ -911,33 +1024,86 @@ bool gathers_favour_wide_groups(const unsigned long long* bins) {
     return 2.0 * gathers > static_cast<double>(all);
 }
 
-bool column_order_shape(idx_t m, idx_t n, idx_t nnz, idx_t base, size_t value_bytes, size_t band_bytes,
+namespace {
+constexpr uint64_t kUnitsWanted = kXcds * kColumnGroupsPerXcd;
+}  // namespace
+
+uint32_t column_order_halved_rows(idx_t m, uint64_t groups) {
+    uint32_t rows = kColumnOrderRows;
+    while (rows > kColumnOrderMinRows && groups * ((static_cast<uint64_t>(m) + rows - 1) / rows) < kUnitsWanted) rows /= 2;
+    return rows;
+}
+
+namespace {
+constexpr idx_t kShortTilesLeastNonzeros = 1u << 21;
+struct EvenTiles {
+    uint64_t groups, turns;
+    uint32_t rows;
+};
+// The tiles whose units every compute unit gets equally many of (`turns`), for the number of band groups with which that is
+// estimated to take the shortest.  A unit takes what its nonzeros take, and as much as a quarter more where its tile is half
+// as tall.  Against tiles halved from 16384 rows until there is a unit for each, in bands of 2 MB and a last one of what is
+// left, microseconds a call, the trial's way before that where it refused: uniform rows, fp64 604 K x 17 69 -> 48, 788 K x 38
+// 134 -> 92, 2.6 M x 33 368 -> 337, 1.4 M x 22 133 -> 135; fp32 903 K x 7 43 -> 31; power-law rows, fp32 271 K 33 -> 15, 553 K
+// 41 -> 27, 637 K 41 -> 29, fp64 451 K 53 -> 40, 843 K 92 -> 64, 1.4 M 127 -> 115 (of 843 K rows' 92, 80 with tiles of equally
+// many rows, 74 cut by nonzeros, 65 with groups of one width).
+EvenTiles even_tiles(idx_t m, uint64_t groups, uint64_t least_groups) {
+    EvenTiles best = {0, 0, 0};
+    double best_time = 0;
+    for (uint64_t g = groups; g >= least_groups && g != 0; --g) {
+        uint64_t turns = 1;
+        while (turns * kUnitsWanted / g * kColumnOrderRows < m) ++turns;
+        const uint64_t chunks = turns * kUnitsWanted / g;
+        const uint32_t rows = static_cast<uint32_t>((static_cast<uint64_t>(m) + chunks - 1) / chunks);
+        const double time = static_cast<double>(turns) * rows / static_cast<double>(g) * (0.75 + 0.25 * kColumnOrderRows / rows);
+        if (best.rows == 0 || time < 0.98 * best_time) {
+            best = {g, turns, rows};
+            best_time = time;
+        }
+    }
+    return best;
+}
+}  // namespace
+
+bool column_order_shape(idx_t m, idx_t n, idx_t nnz, idx_t base, size_t value_bytes, size_t band_bytes, bool even,
                         BandedShape* out) {
     if (m == 0 || n == 0 || nnz == 0 || (value_bytes != 4 && value_bytes != 8)) return false;
     uint32_t wanted = 0;  // log2 of the keys in band_bytes of x
     while ((static_cast<size_t>(value_bytes) << (wanted + 1)) <= band_bytes) ++wanted;
     const uint64_t max_key = static_cast<uint64_t>(n) - 1 + base;
-    const uint64_t groups = (max_key >> wanted) + 1;  // planes of partial sums: every one costs a sum per row
+    uint64_t groups = (max_key >> wanted) + 1;  // planes of partial sums: every one costs a sum per row
     if (groups > 64) return false;
-    // The taller a tile, the more of its entries share a line of x; but the kernel runs one workgroup per
-    // compute unit, so there must be a unit of work for each: the tiles are halved until there is, and a
-    // matrix too small for that is left to the other kernels.
-    constexpr uint64_t kUnitsWanted = kXcds * kColumnGroupsPerXcd;
-    uint32_t rows_per_tile = kColumnOrderRows;
-    while (rows_per_tile > kColumnOrderMinRows &&
-           groups * ((static_cast<uint64_t>(m) + rows_per_tile - 1) / rows_per_tile) < kUnitsWanted)
-        rows_per_tile /= 2;
-    const uint64_t chunks = (static_cast<uint64_t>(m) + rows_per_tile - 1) / rows_per_tile;
-    if (groups * chunks < kUnitsWanted) return false;
+    // The taller a tile, the more of its entries share a line of x; but the kernel runs one workgroup per compute unit, so
+    // there must be a unit of work for each, and a matrix too small for that is left to the other kernels.
+    uint32_t rows_per_tile = column_order_halved_rows(m, groups), mean_rows = rows_per_tile;
+    if (even) {
+        const uint64_t least_groups = groups >= 3 ? (4 * (max_key + 1) + (5ull << wanted) - 1) / (5ull << wanted) : groups;
+        const EvenTiles best = even_tiles(m, groups, std::min(least_groups, groups));
+        // Tiles of few rows: worth building for matrices with nonzeros enough.  Microseconds a call before (row kernels, merge
+        // path for the power law) and with 256 units, and what the copy costs: 250 K rows of 16 fp32 23.6, 16.5 and 480; of 40
+        // 65, 22 and 550; 131 K rows of 16 13.8, 11.3 and 375; 131 K power-law rows 21.3, 12.1 and 390; rows of 4 level.
+        const bool short_tiles = groups * ((static_cast<uint64_t>(m) + kColumnOrderMinRows - 1) / kColumnOrderMinRows) < kUnitsWanted;
+        if (best.rows < kColumnOrderMinEvenRows || (short_tiles && (nnz < kShortTilesLeastNonzeros || nnz / 8 < m))) return false;
+        groups = best.groups;
+        mean_rows = best.rows;
+        rows_per_tile = best.turns == 1 ? std::min(2 * mean_rows, kColumnOrderRows) : mean_rows;
+    }
+    const uint64_t chunks = (static_cast<uint64_t>(m) + mean_rows - 1) / mean_rows;
+    if (!even && groups * chunks < kUnitsWanted) return false;
+    // groups of the same width, in bands of the same width (with bands of a power of two the last group had what was left:
+    // 788 K fp64 columns in groups of 2, 2, 2 and 0.3 MB)
+    const uint64_t group_keys = (max_key + groups) / groups;
     const uint32_t row_bits = bit_length(rows_per_tile - 1);
-    const uint32_t shift = wanted > 32 - row_bits ? 32 - row_bits : wanted;
-    const uint32_t sub = 1u << (wanted - shift);  // bands that share a plane of partial sums
+    const uint32_t sub = static_cast<uint32_t>(((group_keys - 1) >> (32 - row_bits)) + 1);  // bands that share a plane of sums
+    const uint32_t band_keys = static_cast<uint32_t>((group_keys + sub - 1) / sub);
     // the tile numbers are sorted in at most two passes of eight bits
     if (sub > 64 || groups * chunks * sub > 65536) return false;
-    out->band_shift = shift;
+    out->band_shift = 32 - row_bits;
+    out->band_keys = band_keys;
     out->band_bits = bit_length(static_cast<uint32_t>(groups * sub - 1));
     out->bands = static_cast<uint32_t>(groups);
     out->rows_per_tile = rows_per_tile;
+    out->mean_rows = mean_rows;
     out->chunks = static_cast<uint32_t>(chunks);
     out->tiles = static_cast<uint32_t>(groups * chunks * sub);
     out->sub = sub;
@@ -952,10 +1118,11 @@ BandedLayout banded_layout(const BandedShape& s, idx_t m, idx_t nnz, size_t valu
     l.tile_ptr = off; off += align_up((static_cast<size_t>(s.tiles) + 1) * sizeof(idx_t));
     l.xcd_start = off; off += align_up((kXcds + 1) * sizeof(uint32_t));
     l.next_unit = off; off += align_up((kXcds + 1) * sizeof(uint32_t));  // the counters and the count of finished workgroups
-    l.unit_order = off; off += align_up(s.by_column ? s.tiles / s.sub * sizeof(uint4) : 0);
     l.entries = off; off += idx_bytes;
     l.vals = off; off += align_up(static_cast<size_t>(nnz) * value_bytes);
     l.partials = off; off += align_up(static_cast<size_t>(s.bands) * m * value_bytes);
+    l.unit_order = off; off += align_up(s.by_column ? s.tiles / s.sub * sizeof(UnitRecord) : 0);
+    l.chunk_first = off; off += align_up(s.by_column ? (s.chunks + 1) * sizeof(uint32_t) : 0);
     l.keep = off;
     l.src_cols = l.src_rows = l.src_vals = l.tile_ids = 0;
     if (s.by_column) {
@@ -975,7 +1142,7 @@ BandedLayout banded_layout(const BandedShape& s, idx_t m, idx_t nnz, size_t valu
     return l;
 }
 
-void launch_column_order_build(hipStream_t stream, const BandedShape& s, idx_t m, idx_t nnz, idx_t base,
+void launch_column_order_build(hipStream_t stream, const BandedShape& s, idx_t m, idx_t nnz, idx_t base, const idx_t* row_ptr,
                                const idx_t* r_keys, const idx_t* c_keys, const void* vals, size_t value_bytes,
                                void* region) {
     const BandedLayout l = banded_layout(s, m, nnz, value_bytes);
@@ -984,8 +1151,11 @@ void launch_column_order_build(hipStream_t stream, const BandedShape& s, idx_t m
     // own arrays (the transposing directions hand them in) are copied from, never written
     idx_t* ids = reinterpret_cast<idx_t*>(w + l.src_cols);
     idx_t* packed = reinterpret_cast<idx_t*>(w + l.src_rows);
+    uint32_t* chunk_first = reinterpret_cast<uint32_t*>(w + l.chunk_first);
+    hipLaunchKernelGGL(column_order_cut_kernel, dim3(1), dim3(kCutBlock), 0, stream, m, nnz, base, row_ptr, s.chunks, s.mean_rows,
+                       s.rows_per_tile, chunk_first);
     hipLaunchKernelGGL(column_order_pack_kernel, dim3((nnz + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, nnz, base,
-                       s.band_shift, s.rows_per_tile, s.chunks, s.sub, r_keys, c_keys, ids, packed);
+                       s.band_shift, s.band_keys, m, s.mean_rows, s.chunks, s.sub, chunk_first, r_keys, c_keys, ids, packed);
     idx_t* sorted_ids = reinterpret_cast<idx_t*>(w + l.tile_ids);
     launch_sort_triples(stream, nnz, bit_length(s.tiles - 1), ids, packed, vals, sorted_ids,
                         reinterpret_cast<idx_t*>(w + l.entries), w + l.vals, value_bytes, w + l.sort_ws);
@@ -1001,7 +1171,7 @@ void launch_column_order_build(hipStream_t stream, const BandedShape& s, idx_t m
                        reinterpret_cast<uint32_t*>(w + l.next_unit));
     hipLaunchKernelGGL(column_order_rank_kernel, dim3(kXcds), dim3(kOrderBlock), 0, stream, nnz, s.tiles / s.sub, s.chunks, s.sub,
                        reinterpret_cast<const idx_t*>(w + l.tile_ptr), reinterpret_cast<const uint32_t*>(w + l.xcd_start),
-                       reinterpret_cast<uint4*>(w + l.unit_order));
+                       chunk_first, reinterpret_cast<UnitRecord*>(w + l.unit_order));
 }
 
 void launch_banded_build(hipStream_t stream, const BandedShape& s, idx_t m, idx_t nnz, idx_t base, const idx_t* row_ptr,
@@ -1031,6 +1201,16 @@ uint32_t banded_grid(const uint32_t* xcd_start_host) {
 }
 
 template <typename T>
+static auto column_order_kernel(bool crowd, bool direct, bool one) {
+    if (one) {
+        if (direct) return crowd ? spmv_column_order_kernel<T, true, true, true> : spmv_column_order_kernel<T, false, true, true>;
+        return crowd ? spmv_column_order_kernel<T, true, false, true> : spmv_column_order_kernel<T, false, false, true>;
+    }
+    if (direct) return crowd ? spmv_column_order_kernel<T, true, true, false> : spmv_column_order_kernel<T, false, true, false>;
+    return crowd ? spmv_column_order_kernel<T, true, false, false> : spmv_column_order_kernel<T, false, false, false>;
+}
+
+template <typename T>
 bool launch_spmv_banded(hipStream_t stream, const BandedShape& s, uint32_t grid, const SpmvArgs& a, T alpha, T beta,
                         void* region) {
     if (a.m == 0) return true;
@@ -1038,20 +1218,20 @@ bool launch_spmv_banded(hipStream_t stream, const BandedShape& s, uint32_t grid,
     char* w = static_cast<char*>(region);
     T* partials = reinterpret_cast<T*>(w + l.partials);
     if (s.by_column) {
-        const int lds = static_cast<int>(s.rows_per_tile * sizeof(double));
+        const int lds = static_cast<int>((s.rows_per_tile + kWave) * sizeof(double));  // (and those of lanes without an entry)
         XcdStarts stretches;
         for (uint32_t i = 0; i <= kXcds; ++i) stretches.first[i] = s.xcd_start[i];
         // one band group: the kernel writes y itself, and no reduce follows
         const bool direct = s.bands == 1;
-        auto* kernel = direct ? (s.crowded_rows ? spmv_column_order_kernel<T, true, true>
-                                                : spmv_column_order_kernel<T, false, true>)
-                              : (s.crowded_rows ? spmv_column_order_kernel<T, true, false>
-                                                : spmv_column_order_kernel<T, false, false>);
+        bool one = true;  // unit a workgroup at most
+        for (uint32_t i = 0; i < kXcds; ++i) one = one && s.xcd_start[i + 1] - s.xcd_start[i] <= kColumnGroupsPerXcd;
+        auto* kernel = column_order_kernel<T>(s.crowded_rows, direct, one);
         if (!allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds)) return false;
         hipLaunchKernelGGL(kernel, dim3(kColumnGroupsPerXcd * kXcds), dim3(kColumnBlock), lds, stream, a.m, a.n, a.nnz,
-                           a.base, s.band_shift, s.rows_per_tile, s.chunks, s.tiles / s.sub, s.sub,
+                           a.base, s.band_shift, s.band_keys, s.rows_per_tile, s.chunks, s.tiles / s.sub, s.sub,
                            stretches, reinterpret_cast<uint32_t*>(w + l.next_unit),
-                           reinterpret_cast<const uint4*>(w + l.unit_order), reinterpret_cast<const idx_t*>(w + l.tile_ptr), reinterpret_cast<const idx_t*>(w + l.entries),
+                           reinterpret_cast<const UnitRecord*>(w + l.unit_order),
+                           reinterpret_cast<const idx_t*>(w + l.tile_ptr), reinterpret_cast<const idx_t*>(w + l.entries),
                            reinterpret_cast<const T*>(w + l.vals), static_cast<const T*>(a.x), partials,
                            static_cast<T*>(a.y), alpha, beta);
         if (direct) return launches_taken();

@@ -458,3 +458,23 @@ def test_tiles_and_units_of_a_few_entries_or_none(torch_gpu, handle, oracle, dty
     ptr = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=m))])
     a = wl.Csr(m, n, ptr, rng.integers(0, n, nnz), rng.integers(-8, 9, nnz).astype(dtype))
     run(torch_gpu, handle, oracle, a, 2.0, -1.0, band_bytes=band_bytes)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("op", [api.OP_N, api.OP_T])
+@pytest.mark.parametrize("m,n,nnz,heavy", [
+    (300001, 290003, 3300000, 0),     # one unit a compute unit, a thousand rows each
+    (300001, 290003, 3300000, 9),     # the first and the last rows hold most nonzeros: the tiles between them are as tall as may be
+    (700001, 1600003, 200000, 0),     # several band groups, two or three turns of units of nearly full height
+])
+def test_tiles_cut_evenly(torch_gpu, handle, oracle, dtype, op, m, n, nnz, heavy):
+    """Without a band width of the caller's the tiles are cut so that all compute units get as many units, of equally many
+    nonzeros where there is room for that, and the band groups are of one width."""
+    rng = np.random.default_rng(92)
+    rows = rng.integers(0, m, nnz)
+    if heavy:
+        rows[nnz // 8:] = np.concatenate([np.arange(heavy), m - 1 - np.arange(heavy)])[rng.integers(0, 2 * heavy, nnz - nnz // 8)]
+    rows.sort()
+    ptr = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=m))])
+    a = wl.Csr(m, n, ptr, rng.integers(0, n, nnz), rng.integers(-8, 9, nnz).astype(dtype))
+    run(torch_gpu, handle, oracle, a, 2.0, -1.0, op=op)
