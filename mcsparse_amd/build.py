@@ -19,7 +19,7 @@ EXPORTS = os.path.join(CSRC, "exports.map")
 SOURCES = ["api_helper.cpp", "api_compute.cpp", "api_legacy.cpp", "api_sort.cpp", "topology.cpp", "analysis.hip", "spmv.hip",
            "spmv_banded.hip", "spmv_diagonals.hip", "spmm.hip", "spmm_blocks.hip", "spmm_strips.hip", "spmm_long.hip", "spmm_diagonals.hip", "convert.hip", "partition.hip",
            "spmv_transposed.hip", "static_scratch.hip"]
-HEADERS = ["internal.h", "device_util.h", "spmm_device.h", "partition_device.h", "bucket_deal.h", "diagonals_device.h",
+HEADERS = ["internal.h", "device_util.h", "spmm_device.h", "spmm_long_device.h", "partition_device.h", "bucket_deal.h", "diagonals_device.h",
            "sort_shape.h"]
 
 COMPILE_FLAGS = [

@@ -405,6 +405,7 @@ struct SpmmArgs {
     idx_t long_row = 0;
     bool long_known = false;
     const uint32_t* long_apart = nullptr;
+    bool long_cut = false;  // the row kernel has cut the pieces (spmm_long_bounds)
     void* long_ws = nullptr;
     int64_t long_n = 0;
     void* band_ws = nullptr;  // nnz words more for them, or null

@@ -7,7 +7,7 @@
 // columns of C, so every nonzero pulls one contiguous stretch of a row of B with wide loads and
 // A is read once per column panel.  A column-major op(B) is handled by a gather kernel with the
 // lanes spread over the nonzeros of the row.  With beta == 0, C is never read.
-#include "spmm_device.h"
+#include "spmm_long_device.h"
 
 namespace mcsp {
 
@@ -52,6 +52,115 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 8 : 1) void sp
                                 static_cast<off_t>(c0 * sizeof(T)), static_cast<off_t>(ldb * sizeof(T)), acc);
 
     if (own.any) store_c<T, V>(C, ldc, c_row_major, row, c0, acc, alpha, beta, own.skip);
+}
+
+// The same sums where rows differ much in length (the call knows of rows above kSpmmLongRow, which are not this kernel's).
+// With a row to a lane group, and groups that walk their row and end, the groups of a wavefront wait for the longest of their
+// rows, and most rows, of one or two nonzeros, are three dependent trips to memory by themselves.  Here a wavefront has
+// kTurnRows neighbouring rows: a group that is through with one takes the next, the long ones first, and the nonzeros of what a group
+// is at next, the next LR of its row or the first of another, are asked for behind the rows of op(B) of the present ones.
+constexpr int kTurnRows = kWave;
+template <typename T, int LR, int V, bool RAGGED>
+__global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 7 : 1) void spmm_rowb_turns_kernel(idx_t m, idx_t n, idx_t nnz, idx_t base,
+                                                                 const idx_t* __restrict__ row_ptr,
+                                                                 const idx_t* __restrict__ col, const T* __restrict__ val,
+                                                                 const T* __restrict__ B, int64_t ldb, T* __restrict__ C,
+                                                                 int64_t ldc, bool c_row_major, T alpha, T beta,
+                                                                 idx_t long_row, const BoundsWork cut) {
+    if (blockIdx.x < cut.blocks) {  // whole workgroup
+        cut_pieces(cut, base, nnz, row_ptr, col);
+        return;
+    }
+    constexpr int kBatch = LR < 8 ? LR : 8;  // rows of op(B) in flight per lane
+    const uint32_t wave_lane = threadIdx.x % kWave, lane = wave_lane % LR, group = wave_lane / LR;
+    const uint64_t row0 = (static_cast<uint64_t>(blockIdx.x - cut.blocks) * (kBlock / kWave) + threadIdx.x / kWave) * kTurnRows;
+    if (row0 >= m) return;  // whole wavefront
+    const LaneColumns own = lane_columns<V, RAGGED>((static_cast<uint64_t>(blockIdx.y) * LR + lane) * V, n);
+    const uint32_t lane_off = static_cast<uint32_t>(own.first * sizeof(T)), ldb_bytes = static_cast<uint32_t>(ldb * sizeof(T));
+    const char* B_bytes = reinterpret_cast<const char*>(B);
+    // the rows in the order in which they are taken: lane i keeps the i-th
+    const uint32_t my_row = static_cast<uint32_t>(min(row0 + wave_lane, static_cast<uint64_t>(m) - 1));
+    const idx_t my_start = row_ptr[my_row] - base, my_end = row_ptr[my_row + 1] - base;
+    const uint32_t length = my_end - my_start;
+    const bool live = row0 + wave_lane < m && length <= long_row;
+    const unsigned long long first = __ballot(live && length > 4 * LR), second = __ballot(live && length <= 4 * LR);
+    auto below = [&](unsigned long long mask) {
+        return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u));
+    };
+    const uint32_t rows = __popcll(first) + __popcll(second);
+    if (rows == 0) return;  // whole wavefront
+    // (rows that are not taken send to the last lane, where nobody looks unless all are)
+    const int to = static_cast<int>(!live ? kWave - 1 : (length > 4 * LR ? below(first) : __popcll(first) + below(second))) * 4;
+    const uint32_t list_row = __builtin_amdgcn_ds_permute(to, static_cast<int>(wave_lane));
+    const uint32_t list_start = __builtin_amdgcn_ds_permute(to, static_cast<int>(my_start));
+    const uint32_t list_end = __builtin_amdgcn_ds_permute(to, static_cast<int>(my_end));
+
+    uint32_t turn = group, next_turn = kWave / LR;
+    bool active = turn < rows;
+    uint32_t row = __shfl(list_row, turn), j = __shfl(list_start, turn), end = __shfl(list_end, turn);
+    if (!active) j = end = 0;
+    const uint32_t last_nonzero = nnz - 1;  // nnz != 0: there is a long row
+    idx_t c_now = col[min(j + lane, last_nonzero)];
+    T a_now = val[min(j + lane, last_nonzero)];
+    T acc[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) acc[i] = T(0);
+    while (true) {
+        const uint32_t left = end - j;
+        const uint32_t roff = (c_now - base) * ldb_bytes;
+        const T aa = a_now;
+        const bool done = left <= LR;  // whole lane groups
+        uint32_t row_next = row, j_next = j + LR, end_next = end;
+        bool active_next = active;
+        auto ask_next = [&]() {
+            const unsigned long long through = __ballot(done && active && lane == 0);
+            if (through != 0) {
+                const uint32_t taken = next_turn + below(through & ~(1ull << (group * LR)) & ((1ull << (group * LR)) - 1));
+                next_turn += __popcll(through);
+                const uint32_t at = done ? taken : turn;
+                turn = at;
+                const uint32_t r = __shfl(list_row, at % kWave), s = __shfl(list_start, at % kWave), e = __shfl(list_end, at % kWave);
+                if (done) {
+                    active_next = active && at < rows;
+                    row_next = r;
+                    j_next = active_next ? s : 0;
+                    end_next = active_next ? e : 0;
+                }
+            }
+            c_now = col[min(j_next + lane, last_nonzero)];
+            a_now = val[min(j_next + lane, last_nonzero)];
+        };
+        static_for<LR / kBatch>([&](auto g) {
+            constexpr int u0 = decltype(g)::value * kBatch;
+            Vec<T, V> b[kBatch];
+            static_for<kBatch>([&](auto u) {
+                constexpr int k = u0 + decltype(u)::value;
+                if (k < left) {  // the same for all lanes of the group
+                    const uint32_t off = group_bcast<LR, k>(roff) + lane_off;
+                    b[decltype(u)::value] = load_row<T, V>(reinterpret_cast<const T*>(B_bytes + off));
+                }
+            });
+            if constexpr (u0 + kBatch == LR) ask_next();
+            static_for<kBatch>([&](auto u) {
+                constexpr int k = u0 + decltype(u)::value;
+                if (k < left) {
+                    const T a = group_bcast<LR, k>(aa);
+#pragma unroll
+                    for (int i = 0; i < V; ++i) acc[i] += a * b[decltype(u)::value].v[i];
+                }
+            });
+        });
+        if (done) {  // whole lane groups
+            if (active && own.any) store_c<T, V>(C, ldc, c_row_major, row0 + row, own.first, acc, alpha, beta, own.skip);
+#pragma unroll
+            for (int i = 0; i < V; ++i) acc[i] = T(0);
+        }
+        row = row_next;
+        j = j_next;
+        end = end_next;
+        active = active_next;
+        if (!__any(active)) break;  // whole wavefront
+    }
 }
 
 // The same product into a column-major C, without a row-major copy of C in between.  A workgroup owns kColumnRows
@@ -729,6 +838,16 @@ void launch_group(hipStream_t stream, const SpmmArgs& a, const uint32_t* group_p
     }
 }
 
+// Whether a call's rows are taken in turns: where it knows of long rows, for the widths with several rows to a wavefront.
+// Microseconds a call with power-law rows, a row to a group and in turns: a million rows, 32 fp32 columns 498, 454 (the row kernel
+// 195, 163); fp64, 275 K rows and 7 columns 146, 134, 440 K and 19 294, 268, 254 K and 15 154, 147; 30 columns level; with 32
+// lanes to a row 88 fp32 columns 636, 677, 35 fp64 columns 1529, 1444, 66 columns 325, 369.  Where a row fits a lane or two
+// spmm_narrow_kernel reads ahead by itself.
+template <typename T, int LR>
+bool takes_rows_in_turns(const SpmmArgs& a) {
+    return LR <= 16 && a.long_row != 0 && a.long_known && narrow_offsets(a, sizeof(T));
+}
+
 template <typename T, int LR, int V>
 void launch_rowb(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     const uint64_t row_blocks = (static_cast<uint64_t>(a.m) + (kBlock / LR) - 1) / (kBlock / LR);
@@ -750,6 +869,21 @@ void launch_rowb(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
         if (narrow_offsets(a, sizeof(T))) launch(std::false_type{}, ragged);
         else launch(std::true_type{}, ragged);
     };
+    if constexpr (LR <= 16) {
+        if (takes_rows_in_turns<T, LR>(a)) {
+            constexpr uint32_t kRowsPerBlock = kBlock / kWave * kTurnRows;
+            const BoundsWork cut = spmm_long_bounds(a, sizeof(T));
+            const dim3 turns_grid(cut.blocks + (a.m + kRowsPerBlock - 1) / kRowsPerBlock, static_cast<uint32_t>(panels));
+            auto turns = [&](auto ragged) {
+                hipLaunchKernelGGL((spmm_rowb_turns_kernel<T, LR, V, decltype(ragged)::value>), turns_grid, dim3(kBlock), 0, stream,
+                                   a.m, a.n, a.nnz, a.base, a.row_ptr, a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta,
+                                   a.long_row, cut);
+            };
+            if (a.n % V != 0) turns(std::true_type{});
+            else turns(std::false_type{});
+            return;
+        }
+    }
     if constexpr (V > 1) {
         if (a.n % V != 0) {
             launch_offsets(std::true_type{});
@@ -778,8 +912,14 @@ template <typename T>
 void launch_spmm(hipStream_t stream, const SpmmArgs& args, T alpha, T beta) {
     if (args.m == 0 || args.n == 0) return;
     SpmmArgs a = args;
-    // (behind the row kernel the offsets are in cache: 1 to 2 us less where the call knows that there are long rows)
-    if (a.long_row != 0 && !a.long_known) a.long_apart = launch_spmm_long_find(stream, a, sizeof(T));
+    // A row kernel that cuts the pieces needs the list of them; else it is made behind the row kernel, when the offsets are in
+    // cache, where the call knows that there are long rows (1 to 2 us less).
+    const bool cut = a.long_row != 0 && a.long_known && spmm_long_bounds(a, sizeof(T)).blocks != 0;
+    if (a.long_row != 0 && (cut || !a.long_known)) {
+        const uint32_t* apart = launch_spmm_long_find(stream, a, sizeof(T));
+        if (!a.long_known) a.long_apart = apart;
+    }
+    a.long_cut = cut;  // (those widths are all taken in turns)
     if (a.b_row_major) {
         constexpr int kWide = 16 / sizeof(T);  // elements per 128-bit access
         // Rows that begin at any element take the wide loads too (27-point stencil, 872 K rows, fp32: 5, 17, 50, 101
@@ -806,7 +946,7 @@ void launch_spmm(hipStream_t stream, const SpmmArgs& args, T alpha, T beta) {
                                a.long_row, a.long_apart);
         }
     }
-    if (a.long_row != 0 && a.long_known) launch_spmm_long_find(stream, a, sizeof(T));
+    if (a.long_row != 0 && a.long_known && !cut) launch_spmm_long_find(stream, a, sizeof(T));
     if (a.long_row != 0) launch_spmm_long_rows<T>(stream, a, alpha, beta);
 }
 

@@ -201,6 +201,17 @@ __device__ __forceinline__ void row_times_b(idx_t begin, idx_t end, idx_t lane, 
     }
 }
 
+// beta*old + alpha*acc, rounded the same way in every kernel (left to the compiler it is the one or the other product that
+// goes into the fused operation unrounded).
+template <typename T>
+__device__ __forceinline__ T scaled_sum(T alpha, T acc, T beta, T old) {
+    return __builtin_fma(beta, old, alpha * acc);
+}
+template <>
+__device__ __forceinline__ float scaled_sum<float>(float alpha, float acc, float beta, float old) {
+    return __builtin_fmaf(beta, old, alpha * acc);
+}
+
 // Writes V adjacent columns of one row of C but for the first `skip`: beta*C + alpha*acc, C untouched by reads if
 // beta == 0.
 template <typename T, int V>
@@ -212,7 +223,7 @@ __device__ __forceinline__ void store_c(T* __restrict__ C, int64_t ldc, bool c_r
         const int64_t next = c_row_major ? 1 : ldc;
 #pragma unroll
         for (int i = 1; i < V; ++i) {
-            if (i >= skip) Cp[i * next] = beta0 ? alpha * acc[i] : beta * Cp[i * next] + alpha * acc[i];
+            if (i >= skip) Cp[i * next] = beta0 ? alpha * acc[i] : scaled_sum(alpha, acc[i], beta, Cp[i * next]);
         }
     } else if (c_row_major) {
         T* Cp = C + static_cast<int64_t>(row) * ldc + c0;
@@ -223,14 +234,14 @@ __device__ __forceinline__ void store_c(T* __restrict__ C, int64_t ldc, bool c_r
         } else {
             const Vec<T, V> old = load_row<T, V>(Cp);
 #pragma unroll
-            for (int i = 0; i < V; ++i) out.v[i] = beta * old.v[i] + alpha * acc[i];
+            for (int i = 0; i < V; ++i) out.v[i] = scaled_sum(alpha, acc[i], beta, old.v[i]);
         }
         store_vec<T, V>(Cp, out);
     } else {
 #pragma unroll
         for (int i = 0; i < V; ++i) {
             T* Cp = C + static_cast<int64_t>(c0 + i) * ldc + row;
-            *Cp = beta0 ? alpha * acc[i] : beta * *Cp + alpha * acc[i];
+            *Cp = beta0 ? alpha * acc[i] : scaled_sum(alpha, acc[i], beta, *Cp);
         }
     }
 }

@@ -13,26 +13,13 @@
 // Where op(B) is far larger than the L2s, step 2 goes band by band of op(B): see the bands below.
 // Every sum is formed in a fixed order, so results repeat bit for bit; where the pieces and partial sums of a row
 // lie in the scratch area depends on the order in which the rows were found, which nothing else depends on.
-#include "spmm_device.h"
+#include "spmm_long_device.h"
 
 namespace mcsp {
 
 namespace {
 
 using namespace spmm_detail;
-
-struct LongCounters {
-    // the pieces listed; rows of several pieces << 32 | the pieces of those.  (Adds to one line take their turns, 5 ns each,
-    // whichever counters they are for: three for each of 1024 workgroups were the time of the find kernel on 4 M rows, 17 us.)
-    uint32_t items;
-    unsigned long long several;
-    __device__ uint32_t rows() const { return static_cast<uint32_t>(several >> 32); }
-    // not zero: the listed rows are taken apart, since there is one of more than kSpmmLongRow nonzeros (on a line of its
-    // own: a store among the adds to the counters makes the find kernel wait, 16.5 -> 27.5 us on a million rows)
-    alignas(128) uint32_t apart;
-    uint32_t unsorted;  // not zero: a piece whose columns do not ascend
-};
-static_assert(sizeof(LongCounters) <= 2 * kAlign, "what the layout has room for");
 
 __global__ void spmm_long_zero_kernel(LongCounters* c, bool known) {
     c->items = 0;
@@ -59,7 +46,7 @@ __device__ __forceinline__ void write_long_row(uint32_t row, uint32_t pieces, ui
     bool fits = first + pieces <= cap_items && first + pieces >= first;
     if (pieces > 1) {
         fits = fits && slot + pieces <= cap_slots && slot + pieces >= slot && at < cap_rows;
-        if (at < cap_rows) rows[at] = fits ? make_uint4(row, slot, pieces, 0u) : make_uint4(row, 0u, 0u, 0u);
+        if (at < cap_rows) rows[at] = fits ? make_uint4(row, slot, pieces, first) : make_uint4(row, 0u, 0u, 0u);
     }
     for (uint32_t j = 0; j < pieces && first + j < cap_items; ++j)
         items[first + j] = make_uint4(row, j, fits ? pieces : 0u, slot);
@@ -133,118 +120,10 @@ __global__ __launch_bounds__(kBlock) void spmm_long_find_kernel(idx_t m, idx_t l
     }
 }
 
-// ---- bands of op(B) --------------------------------------------------------------------------------------------
-// The long rows of a matrix name every row of op(B) many times (a million power-law rows: 20 times), but a piece walks all of
-// op(B), so each time it comes from behind the L2s.  Where op(B) is larger than they are, the pieces are taken band by band: a
-// band is a stretch of rows of op(B) that fits an L2, an XCD works on every eighth band, and a wavefront takes the
-// nonzeros that one piece has in one band, which lie side by side where columns ascend.  Their sum is a row of partial sums,
-// added up per row in the order of pieces and bands.  Whether and how is decided on the device, from the number of pieces
-// found, so that every way to a product comes to the same sums.
-// A million power-law rows, 32 fp32 columns (20 M of 28 M nonzeros in rows of more than 256), microseconds: pieces whole 327,
-// band by band 225 and 30 for the bounds, 560 -> 501 a call; 16 columns 520 -> 457; 3 M rows, 20 columns 1942 -> 1443; 400 K
-// rows, 11 fp64 columns 258 -> 227.  Half of the rows of op(B) still come from behind the L2 (its wavefronts are not all in
-// one band); bands of 2 MB bring that down to a quarter and the nonzeros of a pair to 32, half a round: 524.  Bands of 8 MB:
-// 549.  Rows of op(B) wider than a panel of kBandLanes lanes keep their pieces whole: A's long rows would be read once per
-// panel (100 fp32 columns: 1763 us whole, 2740 in panels).
-constexpr uint64_t kBandBytes = size_t(4) << 20;  // of op(B)
-constexpr uint32_t kBandStretches = 8;            // bands are dealt to so many XCDs
-constexpr idx_t kBandLeastNonzeros = 1u << 20;
-constexpr uint64_t kBandLeastBytes = size_t(16) << 20;
-constexpr int kBandLanes = 8;
-struct BandSpace {
-    void* ws;            // null: no room, or no need
-    uint64_t bytes;
-    idx_t k;             // rows of op(B)
-    uint32_t row_bytes, sum_bytes;  // of a row of op(B), and of a row of partial sums
-};
-constexpr uint32_t kBandTake = 8;  // items a wavefront takes off its XCD's counter at a time
-struct BandPlan {
-    uint32_t bands, items;  // 0 bands: pieces are taken whole
-    uint32_t* taken;        // [stretch], a line each: (band, item) pairs that have been taken
-    uint32_t* bounds;       // [item][band]: the item's first nonzero in that band or a later one; and behind the last band
-    void* sums;             // [item][band]
-    float of_column;        // band = column times this (whatever the rounding: it ascends with the column)
-};
-__device__ __forceinline__ BandPlan band_plan(const BandSpace& s, const LongCounters* __restrict__ c, uint32_t cap_items) {
-    BandPlan p = {0, 0, nullptr, nullptr, nullptr, 0.0f};
-    if (s.ws == nullptr || c->apart == 0 || c->unsorted != 0) return p;
-    p.items = min(c->items, cap_items);
-    if (p.items == 0) return p;
-    const uint64_t wanted = (static_cast<uint64_t>(s.k) * s.row_bytes + kBandBytes - 1) / kBandBytes;
-    uint64_t bands = (wanted + kBandStretches - 1) / kBandStretches * kBandStretches;
-    auto bounds_bytes = [&](uint64_t n) { return (p.items * (n + 1) * sizeof(uint32_t) + kAlign - 1) / kAlign * kAlign; };
-    constexpr uint64_t kTakenBytes = kBandStretches * kAlign;
-    while (bands != 0 && kTakenBytes + bounds_bytes(bands) + bands * p.items * s.sum_bytes > s.bytes) bands -= kBandStretches;
-    if (2 * bands < wanted) return p;  // (bands of twice the size still keep half of their rows)
-    p.bands = static_cast<uint32_t>(bands);
-    p.taken = static_cast<uint32_t*>(s.ws);
-    p.bounds = p.taken + kTakenBytes / sizeof(uint32_t);
-    p.sums = reinterpret_cast<char*>(p.bounds) + bounds_bytes(bands);
-    p.of_column = static_cast<float>(bands) / static_cast<float>(s.k);
-    return p;
-}
-
-// The bounds of every item, a workgroup at a time.
-__global__ __launch_bounds__(kBlock) void spmm_long_bounds_kernel(BandSpace space, idx_t base, idx_t nnz,
+__global__ __launch_bounds__(kBlock) void spmm_long_bounds_kernel(BoundsWork work, idx_t base, idx_t nnz,
                                                                   const idx_t* __restrict__ row_ptr,
-                                                                  const idx_t* __restrict__ col, LongCounters* c,
-                                                                  const uint4* __restrict__ items, uint32_t cap_items) {
-    const BandPlan plan = band_plan(space, c, cap_items);  // (a workgroup that sees another's `unsorted` may stop early)
-    if (plan.bands == 0) return;  // whole workgroup
-    constexpr int kAtOnce = 2, kQuad = 4;
-    typedef idx_t quad_t __attribute__((ext_vector_type(kQuad)));
-    typedef quad_t element_aligned __attribute__((aligned(sizeof(idx_t))));
-    if (blockIdx.x == 0 && threadIdx.x < kBandStretches) plan.taken[threadIdx.x * (kAlign / sizeof(uint32_t))] = 0;
-    auto band_of = [&](idx_t column) {
-        return min(static_cast<uint32_t>(static_cast<float>(column - base) * plan.of_column), plan.bands - 1);
-    };
-    for (uint32_t it = blockIdx.x; it < plan.items; it += gridDim.x) {
-        const uint4 item = items[it];
-        uint32_t* bounds = plan.bounds + static_cast<uint64_t>(it) * (plan.bands + 1);
-        const idx_t row_end = min(row_ptr[item.x + 1] - base, nnz);
-        const idx_t start = min(row_ptr[item.x] - base + item.y * kSpmmLongChunk, row_end);
-        const idx_t end = item.z != 0 ? min(start + static_cast<idx_t>(kSpmmLongChunk), row_end) : start;
-        if (start == end) {  // whole workgroup: a row that found no room
-            for (uint32_t b = threadIdx.x; b <= plan.bands; b += kBlock) bounds[b] = start;
-            continue;
-        }
-        bool unsorted = false;
-        // neighbouring nonzeros by fours to a thread: the one before its first is the thread's before
-        for (idx_t j0 = start + threadIdx.x * kQuad; j0 < end; j0 += kBlock * kQuad * kAtOnce) {
-            quad_t here[kAtOnce];
-            idx_t before[kAtOnce];
-#pragma unroll
-            for (int u = 0; u < kAtOnce; ++u) {
-                const idx_t j = j0 + u * kBlock * kQuad;
-                if (j + kQuad <= end) {
-                    here[u] = *reinterpret_cast<const element_aligned*>(col + j);
-                } else {
-#pragma unroll
-                    for (int q = 0; q < kQuad; ++q) here[u][q] = col[min(j + q, end - 1)];
-                }
-                before[u] = col[min(j, end) - (j != start ? 1 : 0)];
-            }
-#pragma unroll
-            for (int u = 0; u < kAtOnce; ++u) {
-                idx_t last = before[u];
-                uint32_t last_band = band_of(last);
-#pragma unroll
-                for (int q = 0; q < kQuad; ++q) {
-                    const idx_t j = j0 + u * kBlock * kQuad + q;
-                    if (j >= end) break;
-                    unsorted |= here[u][q] < last;
-                    const uint32_t band = band_of(here[u][q]);
-                    for (uint32_t b = j == start ? 0 : last_band + 1; b <= band; ++b) bounds[b] = j;
-                    if (j == end - 1) {
-                        for (uint32_t b = band + 1; b <= plan.bands; ++b) bounds[b] = end;
-                    }
-                    last = here[u][q];
-                    last_band = band;
-                }
-            }
-        }
-        if (unsorted) c->unsorted = 1;
-    }
+                                                                  const idx_t* __restrict__ col) {
+    cut_pieces(work, base, nnz, row_ptr, col);
 }
 
 // A wavefront's share of the bands: kBandTake pairs of band and item at a time.  A round is up to 64 nonzeros of a pair, one
@@ -513,40 +392,32 @@ __global__ __launch_bounds__(kBlock) void spmm_long_reduce_kernel(idx_t n, T* __
     const uint64_t per_row = (static_cast<uint64_t>(n) + V - 1) / V;
     const BandPlan plan = band_plan(space, c, cap_items);
     if (plan.bands != 0) {  // the same for all workgroups: the partial sums of all pieces of a row, band by band
-        // (bound by the chain of the longest row: its bounds are asked for a step ahead, four sums at once: 21.6 -> 19 us where
-        // the longest row has 13 pieces)
-        constexpr uint32_t kLanes = 8, kGroups = kWave / kLanes;
+        constexpr uint32_t kLanes = 8, kGroups = kWave / kLanes, kWaves = kBlock / kWave;
         static_assert(kBandStretches % kGroups == 0, "whole rounds");
-        const T* sums = static_cast<const T*>(plan.sums);
-        const uint32_t lane = threadIdx.x % kLanes, group = threadIdx.x % kWave / kLanes;
+        __shared__ T s_sum[kWaves][kLanes * V];
+        const uint32_t wave_lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, lane = threadIdx.x % kLanes, group = wave_lane / kLanes;
         const uint64_t panels = (per_row + kLanes - 1) / kLanes;
-        for (uint64_t w = static_cast<uint64_t>(blockIdx.x) * (kBlock / kWave) + threadIdx.x / kWave; w < plan.items * panels;
-             w += static_cast<uint64_t>(gridDim.x) * (kBlock / kWave)) {
-            const uint32_t it = static_cast<uint32_t>(w / panels);
-            const uint4 item = items[it];
-            if (item.y != 0 || item.z == 0) continue;  // whole wavefront: not the first piece of its row
-            const LaneColumns own = lane_columns<V>((w % panels * kLanes + lane) * V, n);
-            T sum[V];
-#pragma unroll
-            for (int i = 0; i < V; ++i) sum[i] = T(0);
+        // sum += the sums of every `step`-th of `pieces` pieces of a row, the first of which is item `it`
+        auto add_pieces = [&](uint32_t it, uint32_t pieces, uint32_t step, const LaneColumns& own, T (&sum)[V]) {
             // 64 bands of a piece at a time; the bounds of the next 64 are asked for before the sums of these
             const uint32_t rounds = (plan.bands + kWave - 1) / kWave;
+            const uint64_t next_bounds = static_cast<uint64_t>(step) * (plan.bands + 1);
             const uint32_t* bounds = plan.bounds + static_cast<uint64_t>(it) * (plan.bands + 1);
-            const T* in = sums + static_cast<int64_t>(it) * plan.bands * ld_partials + own.first;
-            uint32_t b0 = 0, b = min(threadIdx.x % kWave, plan.bands - 1), begin = bounds[b], end = bounds[b + 1];
-            for (uint32_t steps = item.z * rounds; steps != 0; --steps) {
-                const bool holds = b0 + threadIdx.x % kWave < plan.bands && begin != end;
+            const T* in = static_cast<const T*>(plan.sums) + static_cast<int64_t>(it) * plan.bands * ld_partials + own.first;
+            uint32_t b0 = 0, b = min(wave_lane, plan.bands - 1), begin = bounds[b], end = bounds[b + 1];
+            for (uint32_t steps = (pieces + step - 1) / step * rounds; steps != 0; --steps) {
+                const bool holds = b0 + wave_lane < plan.bands && begin != end;
                 const uint32_t band_here = b;
                 const T* in_here = in;
                 b0 += kWave;
                 if (b0 >= plan.bands) {
                     b0 = 0;
                     if (steps != 1) {
-                        bounds += plan.bands + 1;
-                        in += static_cast<int64_t>(plan.bands) * ld_partials;
+                        bounds += next_bounds;
+                        in += static_cast<int64_t>(step) * plan.bands * ld_partials;
                     }
                 }
-                b = min(b0 + threadIdx.x % kWave, plan.bands - 1);
+                b = min(b0 + wave_lane, plan.bands - 1);
                 begin = bounds[b];
                 end = bounds[b + 1];
                 // the bands that hold nonzeros of the piece (for the others nothing was written), the groups in turn
@@ -578,6 +449,43 @@ __global__ __launch_bounds__(kBlock) void spmm_long_reduce_kernel(idx_t n, T* __
 #pragma unroll
                 for (int off = kLanes; off < kWave; off <<= 1) sum[i] += __shfl_xor(sum[i], off, kWave);
             }
+        };
+        // A row of several pieces is a workgroup's, a wavefront every fourth piece (a wavefront for all 13 of the longest row
+        // took as long as all other rows: 18.0 -> 15.0 us).
+        const uint64_t several = static_cast<uint64_t>(min(c->rows(), cap_rows)) * panels;
+        for (uint64_t w = blockIdx.x; w < several; w += gridDim.x) {
+            const uint4 row = rows[w / panels];
+            if (row.z == 0) continue;  // whole workgroup: a row that found no room
+            const LaneColumns own = lane_columns<V>((w % panels * kLanes + lane) * V, n);
+            T sum[V];
+#pragma unroll
+            for (int i = 0; i < V; ++i) sum[i] = T(0);
+            if (wave < row.z) add_pieces(row.w + wave, row.z - wave, kWaves, own, sum);
+            if (group == 0) {
+#pragma unroll
+                for (int i = 0; i < V; ++i) s_sum[wave][lane * V + i] = sum[i];
+            }
+            __syncthreads();
+            if (wave == 0 && group == 0 && own.any) {
+#pragma unroll
+                for (uint32_t k = 1; k < kWaves; ++k) {
+#pragma unroll
+                    for (int i = 0; i < V; ++i) sum[i] += s_sum[k][lane * V + i];
+                }
+                store_c<T, V>(C, ldc, c_row_major, row.x, own.first, sum, alpha, beta, own.skip);
+            }
+            __syncthreads();  // the sums are read before the next row's are written
+        }
+        for (uint64_t w = static_cast<uint64_t>(blockIdx.x) * kWaves + wave; w < plan.items * panels;
+             w += static_cast<uint64_t>(gridDim.x) * kWaves) {
+            const uint32_t it = static_cast<uint32_t>(w / panels);
+            const uint4 item = items[it];
+            if (item.z != 1) continue;  // whole wavefront: of several pieces, or a row that found no room
+            const LaneColumns own = lane_columns<V>((w % panels * kLanes + lane) * V, n);
+            T sum[V];
+#pragma unroll
+            for (int i = 0; i < V; ++i) sum[i] = T(0);
+            add_pieces(it, 1, 1, own, sum);
             if (group == 0 && own.any) store_c<T, V>(C, ldc, c_row_major, item.x, own.first, sum, alpha, beta, own.skip);
         }
         return;
@@ -643,6 +551,27 @@ const uint32_t* launch_spmm_long_find(hipStream_t stream, const SpmmArgs& a, siz
     return &c->apart;
 }
 
+spmm_detail::BoundsWork spmm_long_bounds(const SpmmArgs& a, size_t value_bytes) {
+    BoundsWork w = {0, {nullptr, 0, 0, 0, 0}, nullptr, nullptr, 0};
+    const int64_t per_vector = static_cast<int64_t>(16 / value_bytes), vectors = (a.n + per_vector - 1) / per_vector;
+    // op(B) beyond the L2s, four to kBandLanes lanes a row of it, and nonzeros enough to be worth cutting
+    if (!a.b_row_major || a.n < per_vector || vectors <= 2 || vectors > kBandLanes || !narrow_offsets(a, value_bytes) ||
+        a.band_ws == nullptr || a.nnz < kBandLeastNonzeros || static_cast<uint64_t>(a.k) * a.n * value_bytes < kBandLeastBytes)
+        return w;
+    const LongLayout l = long_layout(a.nnz, a.long_n, value_bytes);
+    char* ws = static_cast<char*>(a.long_ws);
+    w.blocks = 512;  // (see spmm_rowb_turns_kernel)
+    w.space.ws = a.band_ws;
+    w.space.bytes = static_cast<uint64_t>(a.nnz) * sizeof(idx_t);
+    w.space.k = a.k;
+    w.space.row_bytes = static_cast<uint32_t>(vectors * 16);
+    w.space.sum_bytes = static_cast<uint32_t>(l.ld_partials * value_bytes);
+    w.counters = reinterpret_cast<LongCounters*>(ws + l.counters);
+    w.items = reinterpret_cast<const uint4*>(ws + l.items);
+    w.cap_items = l.cap_items;
+    return w;
+}
+
 template <typename T>
 void launch_spmm_long_rows(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     const LongLayout l = long_layout(a.nnz, a.long_n, sizeof(T));
@@ -667,18 +596,14 @@ void launch_spmm_long_rows(hipStream_t stream, const SpmmArgs& a, T alpha, T bet
     static_assert(2048 % kBandStretches == 0, "workgroups of a launch");
     const dim3 grid(2048, panels);
     const uint32_t reduce_blocks = 1024;
-    // op(B) beyond the L2s, and nonzeros enough for the launch in front
     const bool stretched = wide && lanes >= 4 && narrow_offsets(a, sizeof(T));
-    BandSpace space = {nullptr, 0, 0, 0, 0};
-    if (stretched && a.band_ws != nullptr && a.nnz >= kBandLeastNonzeros &&
-        static_cast<uint64_t>(a.k) * a.n * sizeof(T) >= kBandLeastBytes && lanes_needed <= kBandLanes) {
-        space.ws = a.band_ws;
-        space.bytes = static_cast<uint64_t>(a.nnz) * sizeof(idx_t);
-        space.k = a.k;
-        space.row_bytes = static_cast<uint32_t>(lanes_needed * 16);
-        space.sum_bytes = static_cast<uint32_t>(l.ld_partials * sizeof(T));
-        hipLaunchKernelGGL(spmm_long_bounds_kernel, dim3(8192), dim3(kBlock), 0, stream, space, a.base, a.nnz, a.row_ptr, a.col,
-                           reinterpret_cast<LongCounters*>(w + l.counters), items, l.cap_items);
+    const BoundsWork work = spmm_long_bounds(a, sizeof(T));
+    const BandSpace space = work.space;
+    if (work.blocks != 0 && !a.long_cut) {
+        BoundsWork whole_launch = work;
+        whole_launch.blocks = 8192;
+        hipLaunchKernelGGL(spmm_long_bounds_kernel, dim3(whole_launch.blocks), dim3(kBlock), 0, stream, whole_launch, a.base, a.nnz,
+                           a.row_ptr, a.col);
     }
     auto stretches = [&](auto lr) {
         constexpr int LR = decltype(lr)::value;

@@ -284,3 +284,32 @@ def test_every_way_to_bands_gives_the_same_bits(torch_gpu, oracle):
     for kind, got in results.items():
         assert np.array_equal(got, results["csr"]), kind
     handle.destroy()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [5, 12, 16, 19, 32, 37, 64])  # four, eight and sixteen lanes to a row, whole vectors and ragged
+@pytest.mark.parametrize("m", [64, 65, 200, 449])
+def test_short_rows_are_taken_in_turns(torch_gpu, handle, oracle, n, dtype, m):
+    """A wavefront's 64 rows where all are long, none, the last ones missing; lengths around what a group asks for at a time
+    and around what it counts as long among them, empty rows, and one that keeps a group while the others take the rest."""
+    edge = [0, 1, 2, 3, 4, 5, 7, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 65, 128, 255, 256]
+    rng = np.random.default_rng(m + n)
+    lengths = list(rng.choice(edge, m))
+    lengths[0] = 256
+    if m > 200:
+        lengths[128:192] = [1100] * 64  # a wavefront without rows of its own
+        lengths[192:256] = [1] * 64     # more rows than groups, all of one turn
+    a = rows_of_lengths(lengths + [1100], 1501, dtype, seed=n, base=1)
+    check(torch_gpu, handle, oracle, a, n, 1.25, 0.0, pad_b=2)
+    check(torch_gpu, handle, oracle, a, n, 0.5, -1.5, seed=1, c_order=api.ORDER_COL)
+
+
+@pytest.mark.parametrize("dtype,n", [(np.float32, 16), (np.float32, 30), (np.float64, 7), (np.float64, 16)])
+def test_pieces_cut_beside_the_row_kernel(torch_gpu, handle, oracle, dtype, n):
+    """op(B) beyond the L2s: rows of one piece, of as many as a workgroup has wavefronts, of one more and of many."""
+    lengths = [3] * 3000
+    for at, length in zip(range(5, 3000, 30), [300, 4096, 4097, 8193, 16384, 16385, 20481, 90001] * 8):
+        lengths[at] = length
+    a = rows_of_lengths(lengths, 400009, dtype, seed=2)
+    assert a.nnz >= 1 << 20 and a.n * n * np.dtype(dtype).itemsize >= 16 << 20
+    check(torch_gpu, handle, oracle, a, n, 1.25, -0.5)
