@@ -912,21 +912,22 @@ template <typename T>
 void launch_spmm(hipStream_t stream, const SpmmArgs& args, T alpha, T beta) {
     if (args.m == 0 || args.n == 0) return;
     SpmmArgs a = args;
-    // A row kernel that cuts the pieces needs the list of them; else it is made behind the row kernel, when the offsets are in
-    // cache, where the call knows that there are long rows (1 to 2 us less).
-    const bool cut = a.long_row != 0 && a.long_known && spmm_long_bounds(a, sizeof(T)).blocks != 0;
-    if (a.long_row != 0 && (cut || !a.long_known)) {
+    constexpr int kWide = 16 / sizeof(T);  // elements per 128-bit access
+    // Rows that begin at any element take the wide loads too (27-point stencil, 872 K rows, fp32: 5, 17, 50, 101
+    // columns 98, 283, 796, 1670 us with one element per lane, 64, 133, 304, 545 so; fp64, 33 columns: 1131, 538),
+    // but for the fewest fp64 columns: 7 in eight lanes of one element 143 us, in four of two 157.
+    const bool aligned = reinterpret_cast<uintptr_t>(a.B) % 16 == 0 && a.ldb % kWide == 0 && a.n % kWide == 0;
+    const bool wide = a.n >= kWide && (aligned || sizeof(T) == 4 || a.n > 8);
+    // A row kernel that cuts the pieces (of more than two lanes to a row, which all are taken in turns) needs the list of them;
+    // else it is made behind the row kernel, when the offsets are in cache, where the call knows that there are long rows (1 to 2
+    // us less).
+    a.long_cut = a.long_row != 0 && a.long_known && a.n > (wide ? 2 * kWide : 2) && spmm_long_bounds(a, sizeof(T)).blocks != 0;
+    if (a.long_row != 0 && (a.long_cut || !a.long_known)) {
         const uint32_t* apart = launch_spmm_long_find(stream, a, sizeof(T));
         if (!a.long_known) a.long_apart = apart;
     }
-    a.long_cut = cut;  // (those widths are all taken in turns)
     if (a.b_row_major) {
-        constexpr int kWide = 16 / sizeof(T);  // elements per 128-bit access
-        // Rows that begin at any element take the wide loads too (27-point stencil, 872 K rows, fp32: 5, 17, 50, 101
-        // columns 98, 283, 796, 1670 us with one element per lane, 64, 133, 304, 545 so; fp64, 33 columns: 1131, 538),
-        // but for the fewest fp64 columns: 7 in eight lanes of one element 143 us, in four of two 157.
-        const bool aligned = reinterpret_cast<uintptr_t>(a.B) % 16 == 0 && a.ldb % kWide == 0 && a.n % kWide == 0;
-        if (a.n >= kWide && (aligned || sizeof(T) == 4 || a.n > 8)) launch_rowb_v<T, kWide>(stream, a, alpha, beta);
+        if (wide) launch_rowb_v<T, kWide>(stream, a, alpha, beta);
         else launch_rowb_v<T, 1>(stream, a, alpha, beta);
     } else {
         constexpr int kJB = 4;
@@ -946,7 +947,7 @@ void launch_spmm(hipStream_t stream, const SpmmArgs& args, T alpha, T beta) {
                                a.long_row, a.long_apart);
         }
     }
-    if (a.long_row != 0 && a.long_known && !cut) launch_spmm_long_find(stream, a, sizeof(T));
+    if (a.long_row != 0 && a.long_known && !a.long_cut) launch_spmm_long_find(stream, a, sizeof(T));
     if (a.long_row != 0) launch_spmm_long_rows<T>(stream, a, alpha, beta);
 }
 

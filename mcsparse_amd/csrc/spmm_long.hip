@@ -126,7 +126,7 @@ __global__ __launch_bounds__(kBlock) void spmm_long_bounds_kernel(BoundsWork wor
     cut_pieces(work, base, nnz, row_ptr, col);
 }
 
-// A wavefront's share of the bands: kBandTake pairs of band and item at a time.  A round is up to 64 nonzeros of a pair, one
+// A wavefront's share of the bands: kBandTake pairs of band and item at a time, off one of its XCD's counters.  A round is up to 64 nonzeros of a pair, one
 // asked for by every lane: nonzero t goes to lane group t % G, so that the groups load equally many rows of op(B).  The
 // nonzeros of the next round, often the next pair's, are asked for before the rows of this one.
 template <typename T, int LR, int V>
@@ -136,18 +136,19 @@ __device__ __forceinline__ void take_bands(const BandPlan& plan, const LaneColum
     const uint32_t lane = threadIdx.x % kWave, group = lane / LR, place = lane % LR * G + group;
     const uint32_t stretch = blockIdx.x % kBandStretches;
     const uint32_t all = plan.bands / kBandStretches * plan.items;  // pairs of the stretch, band after band
-    uint32_t* taken = plan.taken + stretch * (kAlign / sizeof(uint32_t));
+    const uint32_t queue = (blockIdx.x / kBandStretches * (kBlock / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave)) % kBandQueues;
+    uint32_t* taken = plan.taken + (stretch * kBandQueues + queue) * (kAlign / sizeof(uint32_t));
     T* sums = static_cast<T*>(plan.sums);
     const char* B_bytes = reinterpret_cast<const char*>(B);
     const uint32_t lane_off = static_cast<uint32_t>(own.first * sizeof(T)), ldb_bytes = static_cast<uint32_t>(ldb * sizeof(T));
     auto take = [&]() {
         uint32_t at = 0;
-        if (lane == 0) at = atomicAdd(taken, kBandTake);
+        if (lane == 0) at = atomicAdd(taken, 1u);
         return at;
     };
     uint32_t next = take();
     while (true) {
-        const uint32_t from = __builtin_amdgcn_readfirstlane(next);
+        const uint32_t from = (__builtin_amdgcn_readfirstlane(next) * kBandQueues + queue) * kBandTake;
         if (from >= all) break;  // whole wavefront
         next = take();  // on its way while this share is worked on
         const uint32_t pairs = min(kBandTake, all - from);
@@ -554,8 +555,8 @@ const uint32_t* launch_spmm_long_find(hipStream_t stream, const SpmmArgs& a, siz
 spmm_detail::BoundsWork spmm_long_bounds(const SpmmArgs& a, size_t value_bytes) {
     BoundsWork w = {0, {nullptr, 0, 0, 0, 0}, nullptr, nullptr, 0};
     const int64_t per_vector = static_cast<int64_t>(16 / value_bytes), vectors = (a.n + per_vector - 1) / per_vector;
-    // op(B) beyond the L2s, four to kBandLanes lanes a row of it, and nonzeros enough to be worth cutting
-    if (!a.b_row_major || a.n < per_vector || vectors <= 2 || vectors > kBandLanes || !narrow_offsets(a, value_bytes) ||
+    // op(B) beyond the L2s, two to kBandLanes lanes a row of it, and nonzeros enough to be worth cutting
+    if (!a.b_row_major || a.n < per_vector || vectors < 2 || vectors > kBandLanes || !narrow_offsets(a, value_bytes) ||
         a.band_ws == nullptr || a.nnz < kBandLeastNonzeros || static_cast<uint64_t>(a.k) * a.n * value_bytes < kBandLeastBytes)
         return w;
     const LongLayout l = long_layout(a.nnz, a.long_n, value_bytes);
@@ -596,9 +597,12 @@ void launch_spmm_long_rows(hipStream_t stream, const SpmmArgs& a, T alpha, T bet
     static_assert(2048 % kBandStretches == 0, "workgroups of a launch");
     const dim3 grid(2048, panels);
     const uint32_t reduce_blocks = 1024;
-    const bool stretched = wide && lanes >= 4 && narrow_offsets(a, sizeof(T));
     const BoundsWork work = spmm_long_bounds(a, sizeof(T));
     const BandSpace space = work.space;
+    // (Two lanes to a row: in groups of four, half of them idle, where that way leads band by band; its gathers count, not its
+    // lanes.  Power-law rows, pieces whole and in bands: 1.1 M, 6 fp32 columns 425 -> 315 us a call, 3.3 M, 4 fp64 columns 1478 -> 1087.)
+    if (work.blocks != 0 && lanes < 4) lanes = 4;
+    const bool stretched = wide && lanes >= 4 && narrow_offsets(a, sizeof(T));
     if (work.blocks != 0 && !a.long_cut) {
         BoundsWork whole_launch = work;
         whole_launch.blocks = 8192;

@@ -37,7 +37,9 @@ static_assert(sizeof(LongCounters) <= 2 * kAlign, "what the layout has room for"
 constexpr uint64_t kBandBytes = size_t(4) << 20;  // of op(B)
 constexpr uint32_t kBandStretches = 8;            // bands are dealt to so many XCDs
 constexpr idx_t kBandLeastNonzeros = 1u << 20;
-constexpr uint64_t kBandLeastBytes = size_t(16) << 20;
+// (of 10 to 16 MB: 416 K rows and 5 fp64 columns 157 -> 140 us, 176 K and 17 fp32 columns 106 -> 100; of 6 to 10 MB 2 to 5 % slower
+// as often as faster)
+constexpr uint64_t kBandLeastBytes = size_t(10) << 20;
 constexpr int kBandLanes = 8;
 struct BandSpace {
     void* ws;            // null: no room, or no need
@@ -45,10 +47,15 @@ struct BandSpace {
     idx_t k;             // rows of op(B)
     uint32_t row_bytes, sum_bytes;  // of a row of op(B), and of a row of partial sums
 };
-constexpr uint32_t kBandTake = 8;  // items a wavefront takes off its XCD's counter at a time
+// The pairs of a stretch are taken off kBandQueues counters, kBandTake at a time, every queue each kBandQueues-th take: adds to one
+// address take their turns, some 14 ns each with all wavefronts of an XCD at it.  One counter, takes of 2, 4, 8 and 16 pairs: 622,
+// 487, 457 and 475 us a call (a million rows, 32 fp32 columns, when the rest of it took 27 us more); 4 counters, takes of 2, 4, 8: 402,
+// 401, 410 against 433; 8 counters 398, 398; 16 counters 397, 397.  3 M rows, 22 columns: 1464; 16 counters, takes of 2 and 4: 1458, 1417.
+constexpr uint32_t kBandTake = 4;
+constexpr uint32_t kBandQueues = 16;
 struct BandPlan {
     uint32_t bands, items;  // 0 bands: pieces are taken whole
-    uint32_t* taken;        // [stretch], a line each: (band, item) pairs that have been taken
+    uint32_t* taken;        // [stretch][queue], a line each: takes of kBandTake (band, item) pairs so far
     uint32_t* bounds;       // [item][band]: the item's first nonzero in that band or a later one; and behind the last band
     void* sums;             // [item][band]
     float of_column;        // band = column times this (whatever the rounding: it ascends with the column)
@@ -61,7 +68,7 @@ __device__ __forceinline__ BandPlan band_plan(const BandSpace& s, const LongCoun
     const uint64_t wanted = (static_cast<uint64_t>(s.k) * s.row_bytes + kBandBytes - 1) / kBandBytes;
     uint64_t bands = (wanted + kBandStretches - 1) / kBandStretches * kBandStretches;
     auto bounds_bytes = [&](uint64_t n) { return (p.items * (n + 1) * sizeof(uint32_t) + kAlign - 1) / kAlign * kAlign; };
-    constexpr uint64_t kTakenBytes = kBandStretches * kAlign;
+    constexpr uint64_t kTakenBytes = kBandStretches * kBandQueues * kAlign;
     while (bands != 0 && kTakenBytes + bounds_bytes(bands) + bands * p.items * s.sum_bytes > s.bytes) bands -= kBandStretches;
     if (2 * bands < wanted) return p;  // (bands of twice the size still keep half of their rows)
     p.bands = static_cast<uint32_t>(bands);
@@ -87,7 +94,8 @@ __device__ __forceinline__ void cut_pieces(const BoundsWork& w, idx_t base, idx_
     constexpr int kAtOnce = 2, kQuad = 4;
     typedef idx_t quad_t __attribute__((ext_vector_type(kQuad)));
     typedef quad_t element_aligned __attribute__((aligned(sizeof(idx_t))));
-    if (blockIdx.x == 0 && threadIdx.x < kBandStretches) plan.taken[threadIdx.x * (kAlign / sizeof(uint32_t))] = 0;
+    static_assert(kBandStretches * kBandQueues <= kBlock, "a thread per counter");
+    if (blockIdx.x == 0 && threadIdx.x < kBandStretches * kBandQueues) plan.taken[threadIdx.x * (kAlign / sizeof(uint32_t))] = 0;
     auto band_of = [&](idx_t column) {
         return min(static_cast<uint32_t>(static_cast<float>(column - base) * plan.of_column), plan.bands - 1);
     };

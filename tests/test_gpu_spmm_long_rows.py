@@ -304,12 +304,12 @@ def test_short_rows_are_taken_in_turns(torch_gpu, handle, oracle, n, dtype, m):
     check(torch_gpu, handle, oracle, a, n, 0.5, -1.5, seed=1, c_order=api.ORDER_COL)
 
 
-@pytest.mark.parametrize("dtype,n", [(np.float32, 16), (np.float32, 30), (np.float64, 7), (np.float64, 16)])
+@pytest.mark.parametrize("dtype,n", [(np.float32, 7), (np.float32, 16), (np.float32, 30), (np.float64, 4), (np.float64, 7), (np.float64, 16)])
 def test_pieces_cut_beside_the_row_kernel(torch_gpu, handle, oracle, dtype, n):
     """op(B) beyond the L2s: rows of one piece, of as many as a workgroup has wavefronts, of one more and of many."""
     lengths = [3] * 3000
     for at, length in zip(range(5, 3000, 30), [300, 4096, 4097, 8193, 16384, 16385, 20481, 90001] * 8):
         lengths[at] = length
     a = rows_of_lengths(lengths, 400009, dtype, seed=2)
-    assert a.nnz >= 1 << 20 and a.n * n * np.dtype(dtype).itemsize >= 16 << 20
+    assert a.nnz >= 1 << 20 and a.n * n * np.dtype(dtype).itemsize >= 10 << 20
     check(torch_gpu, handle, oracle, a, n, 1.25, -0.5)
