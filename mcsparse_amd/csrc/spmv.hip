@@ -3,7 +3,8 @@
 // Two kernel families, picked from the row-length analysis of the structure:
 //  * vector : L consecutive lanes of a wavefront own one row (L = 1..64, chosen from the mean
 //             row length); U rows per lane group are kept in flight at once so that a wave has
-//             enough bytes outstanding to cover HBM latency.  Best for regular matrices.
+//             enough bytes outstanding to cover HBM latency.  Best for regular matrices.  Where the rows are too short
+//             for L lanes to have a nonzero each, a wavefront reads its rows' nonzeros as one stretch instead.
 //  * merge  : the rows' end offsets and the nonzero indices are merged into one path of m+nnz
 //             items that is cut into equal tiles, one per workgroup, so a 200k-nonzero row and
 //             a million 1-nonzero rows cost the same per item.  Rows that straddle tiles leave a
@@ -15,6 +16,7 @@
 // (src/kernels/level2/spmv/csr_vector_device.hpp:22-79), which runs one wavefront per row.
 #include "device_util.h"
 #include "internal.h"
+#include <type_traits>
 
 namespace mcsp {
 
@@ -106,6 +108,129 @@ __global__ __launch_bounds__(kBlock) void spmv_vector_kernel(idx_t m, idx_t base
             }
         }
     }
+}
+
+// Rows of a few nonzeros: a wavefront has R neighbouring rows, whose nonzeros lie in one stretch.  The stretch is read as
+// such, U * 64 nonzeros at a time, and the products go through LDS, where each row's lane adds up its own.
+//
+// What bounds the kernel above on such rows is the number of its memory instructions, not their bytes: five nonzeros in
+// eight lanes leave three lanes of every load and every gather without work, and a matrix in row order with x in the
+// caches has nothing else to wait for.  Here every lane of every instruction has a nonzero and a row costs one more load
+// than its pointer; that leaves the latency of a chain of three loads and one passage through LDS.  Before and after, in
+// us: five-point Laplacian of 512 x 512, fp32 5.5 and 4.8, of 1700 x 1700 42 and 30 (fp64 58 and 43); nine-point of 1000 x
+// 1000 34 and 19 (fp64 39 and 25), which is 97 MB at 5.0 TB/s and 133 MB at 5.3.
+template <typename T, int R, int U, int UPDATE>
+__global__ __launch_bounds__(kBlock) void spmv_short_rows_kernel(idx_t m, idx_t base, const idx_t* __restrict__ row_ptr,
+                                                                 const idx_t* __restrict__ col, const T* __restrict__ val,
+                                                                 const T* __restrict__ x, T* __restrict__ y, T alpha, T beta) {
+    constexpr uint32_t kWindow = U * kWave;
+    // (a place is skipped behind every 32: rows of 4, 8 or 16 nonzeros would begin on the same banks)
+    auto place = [](uint32_t k) { return k + k / 32; };
+    constexpr uint32_t kPlaces = kWindow + kWindow / 32;
+    __shared__ T s_products[kBlock / kWave][kPlaces];
+    T* products = s_products[threadIdx.x / kWave];
+    const uint32_t lane = threadIdx.x % kWave;
+    const uint64_t row0 = (static_cast<uint64_t>(blockIdx.x) * (kBlock / kWave) + threadIdx.x / kWave) * R;
+    if (row0 >= m) return;  // whole wavefront
+    const uint64_t row = min(row0 + min(lane, static_cast<uint32_t>(R)), static_cast<uint64_t>(m));  // lanes past the last row have an empty one
+    const idx_t start = row_ptr[row] - base, behind = __shfl_down(start, 1, kWave);
+    idx_t end = behind;
+    if constexpr (R == kWave) {
+        if (lane == kWave - 1) end = row_ptr[min(row + 1, static_cast<uint64_t>(m))] - base;
+    } else {
+        if (lane >= R) end = start;
+    }
+    const idx_t first = __builtin_amdgcn_readfirstlane(start), last = __builtin_amdgcn_readlane(end, R - 1);
+    // fp32 products are added up as doubles, in two sums.  fp64 ones go to about as many sums as the row had lanes, and
+    // those are added up in pairs, so that no row takes a longer chain of roundings than before (rms error in units of the
+    // last place of sum |a||x|, rows of 8 to 10: 0.416 spread over lanes, 0.410 here; 40 to 500 among rows of 9: 0.134 and
+    // 0.124, where 8 sums give 0.134 to 0.140).
+    constexpr bool kWide = sizeof(T) == 4;
+    constexpr int kAtOnce = U * kWave / R < 4 ? 4 : U * kWave / R, kSums = kWide ? 2 : kAtOnce > 8 ? 16 : 8;
+    typedef typename std::conditional<kWide, double, T>::type Sum;
+    Sum sum[kSums] = {}, total = 0;
+    auto fold = [&] {
+#pragma unroll
+        for (int half = kSums / 2; half > 0; half /= 2) {
+#pragma unroll
+            for (int u = 0; u < half; ++u) sum[u] += sum[u + half];
+        }
+        total += sum[0];
+#pragma unroll
+        for (int u = 0; u < kSums; ++u) sum[u] = 0;
+    };
+    for (idx_t w0 = first; w0 < last; w0 += kWindow) {  // the same for the wavefront; once, as a rule
+        const uint32_t left = last - w0;
+        idx_t c[U];
+        T v[U], xv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t k = min(u * kWave + lane, left - 1);
+            c[u] = load_stream((col + w0) + k);
+            v[u] = load_stream((val + w0) + k);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) xv[u] = x[c[u] - base];
+#pragma unroll
+        for (int u = 0; u < U; ++u) asm volatile("" : "+v"(xv[u]));
+#pragma unroll
+        for (int u = 0; u < U; ++u) products[place(u * kWave + lane)] = v[u] * xv[u];
+        const uint32_t from = start > w0 ? start - w0 : 0u, to = min(end > w0 ? end - w0 : 0u, kWindow);
+        auto add = [&](uint32_t j) {
+            T p[kAtOnce];
+#pragma unroll
+            for (int u = 0; u < kAtOnce; ++u) p[u] = products[place(min(j + u, to - 1))];
+#pragma unroll
+            for (int u = 0; u < kAtOnce; ++u) {
+                if (j + u < to) sum[u % kSums] += p[u];
+            }
+        };
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if constexpr (kWide) {
+            for (uint32_t j = from; j < to; j += kAtOnce) add(j);
+        } else {
+            if (from < to) add(from);
+            // a longer row than most: pairs of products to four sums, and the next ones to the next four
+#pragma unroll 1
+            for (uint32_t j = from + kAtOnce; j < to; j += 8) {
+                T p[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) p[u] = products[place(min(j + u, to - 1))];
+                Sum next[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) next[u] = sum[u] + ((j + u < to ? p[u] : T(0)) + (j + u + 4 < to ? p[u + 4] : T(0))) ;
+#pragma unroll
+                for (int u = 0; u + 4 < kSums; ++u) sum[u] = sum[u + 4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) sum[kSums - 4 + u] = next[u];
+            }
+            fold();
+        }
+        // the next window's products wait for these reads
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    if constexpr (kWide) fold();
+    const T s = static_cast<T>(total);
+    if (lane < R && row < m) {
+        if constexpr (UPDATE == kYSet) {
+            y[row] = alpha * s;
+        } else {
+            y[row] = beta * y[row] + alpha * s;
+        }
+    }
+}
+
+template <typename T, int R, int U>
+void launch_short_rows(hipStream_t stream, const SpmvArgs& a, T alpha, T beta) {
+    constexpr uint32_t kRows = kBlock / kWave * R;
+    const dim3 grid(static_cast<uint32_t>((static_cast<uint64_t>(a.m) + kRows - 1) / kRows));
+    auto* kernel = beta == T(0) ? spmv_short_rows_kernel<T, R, U, kYSet> : spmv_short_rows_kernel<T, R, U, kYScale>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, stream, a.m, a.base, a.row_ptr, a.col, static_cast<const T*>(a.val),
+                       static_cast<const T*>(a.x), static_cast<T*>(a.y), alpha, beta);
 }
 
 template <typename T, int L, int U>
@@ -487,6 +612,36 @@ bool load_row_kernels() {
 template <typename T>
 void launch_spmv_vector(hipStream_t stream, const SpmvArgs& a, T alpha, T beta, int lanes) {
     if (a.m == 0) return;
+    // Rows of 3, 5 to 7 or 9 to 15 nonzeros are read as one stretch.  (4 and 8 fill the lanes of the kernel below: random
+    // columns, 200,000 rows of 8, fp64, 14.4 us below and 14.9 here.)  A row takes a whole lane here, so it needs more rows
+    // than the kernel below before the chip is full of loads: random columns, 160,000 rows of 5, fp64, 8.7 us below and
+    // 9.9 here; 300,000 rows of 5 15.6 and 15.4 (fp32 13.1 and 12.5), 160,000 rows of 9 14.4 and 12.9.  64 rows to a
+    // wavefront read a stencil with the fewest instructions (7 points of 140^3, fp32: 36 us, with 32 rows 41, below 44);
+    // 32 rows give more wavefronts and fewer of x's lines to each (500,000 random rows of 6: 20.0 us, 22.2 with 64 rows,
+    // 22.5 below).
+    const uint64_t mean = (static_cast<uint64_t>(a.nnz) + a.m - 1) / a.m;
+    if (lanes == spmv_pick_lanes(a.m, a.nnz) && mean < static_cast<uint64_t>(lanes) && lanes <= 16 && a.m >= 150000 && a.nnz >= 1200000) {
+        const bool many = a.m >= 500000;
+        switch (mean) {
+            case 3: launch_short_rows<T, 64, 3>(stream, a, alpha, beta); return;
+            case 5: launch_short_rows<T, 64, 5>(stream, a, alpha, beta); return;
+            case 6:
+                if (many) launch_short_rows<T, 64, 6>(stream, a, alpha, beta);
+                else launch_short_rows<T, 32, 3>(stream, a, alpha, beta);
+                return;
+            case 7:
+                if (many) launch_short_rows<T, 64, 7>(stream, a, alpha, beta);
+                else launch_short_rows<T, 32, 4>(stream, a, alpha, beta);
+                return;
+            case 9:
+            case 10: launch_short_rows<T, 32, 5>(stream, a, alpha, beta); return;
+            case 11:
+            case 12: launch_short_rows<T, 32, 6>(stream, a, alpha, beta); return;
+            case 13:
+            case 14: launch_short_rows<T, 32, 7>(stream, a, alpha, beta); return;
+            default: launch_short_rows<T, 32, 8>(stream, a, alpha, beta); return;
+        }
+    }
     switch (lanes) {
         case 1: launch_vector_lu<T, 1, 2>(stream, a, alpha, beta); break;
         case 2: launch_vector_lu<T, 2, 4>(stream, a, alpha, beta); break;

@@ -213,3 +213,42 @@ def test_a_few_long_rows_among_many_short_ones(torch_gpu, handle, oracle):
     st, got, _ = run_spmv(torch_gpu, handle, a, x, y, 1.0, 0.0, family=api.FAMILY_VECTOR)
     assert st == api.STATUS_SUCCESS
     assert_within(got, y_ref, bound, np.float32, what="mixed rows, vector family")
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("mean, m", [(3, 400_063), (5, 240_001), (6, 200_031), (6, 500_001), (7, 200_033), (7, 500_065),
+                                     (9, 150_001), (12, 150_015), (14, 150_031), (15, 150_047)])
+def test_short_rows_are_read_as_one_stretch(torch_gpu, handle, oracle, dtype, mean, m):
+    """Rows of a few nonzeros, as many to a wavefront as it reads in one go: each mean length and number of rows that has
+    a kernel of its own, with a last wavefront that is not full, long empty runs (also at both ends), rows that span
+    windows and a stretch of longer ones.  A row's sum takes at most len / 8 additions, five more for its sums and one for
+    each window of at least 192 products; the product, the scaling by alpha and the addition of beta * y round once each."""
+    rng = np.random.default_rng(mean)
+    lens = rng.integers(max(mean - 3, 0), mean + 4, m)
+    lens[:200] = 0
+    lens[m - 131:m - 1] = 0
+    lens[m // 3:m // 3 + 400] = 0
+    lens[[200, 1000, 1063, 1064, m // 2, m - 1]] = [2000, 700, 449, 512, 65, 321]
+    lens[2000:2200] = rng.integers(20, 90, 200)
+    short = np.nonzero(lens == mean)[0]
+    lens[short[:lens.sum() - mean * m]] -= 1  # the mean is not more than asked for
+    n, base = 70_001, mean % 2
+    ptr = np.concatenate([[0], np.cumsum(lens)])
+    assert ptr[-1] >= 1_200_000 and mean - 1 < ptr[-1] / m <= mean
+    a = wl.Csr(m, n, (ptr + base).astype(np.int32), (rng.integers(1, n, ptr[-1]) + base).astype(np.int32),
+               rng.uniform(-1, 1, ptr[-1]).astype(dtype), base=base)
+    x, y = rng.uniform(-1, 1, n).astype(dtype), rng.uniform(-1, 1, m).astype(dtype)
+    x[0] = np.inf  # column 0 holds nothing
+    x_ref = x.copy()
+    x_ref[0] = 0
+    for alpha, beta in ((1.0, 0.0), (1.5, -0.5)):
+        want, bound = oracle.spmv(False, m, n, base, a.ptr, a.col, a.val, alpha, beta, x_ref, y)
+        st, got, plan = run_spmv(torch_gpu, handle, a, x, y, alpha, beta, family=api.FAMILY_VECTOR)
+        assert st == api.STATUS_SUCCESS and plan[0] == api.FAMILY_VECTOR and plan[1] > mean
+        assert_within(got, want, bound * (lens // 8 + 5 + lens // 192 + 4), dtype, factor=1.0, what="mean %d" % mean)
+    # an infinite element of x reaches the rows that use it and no other
+    x[0], x[n // 2] = 0, np.inf
+    hit = np.zeros(m, bool)
+    hit[np.repeat(np.arange(m), lens)[a.col == n // 2 + base]] = True
+    _, got, _ = run_spmv(torch_gpu, handle, a, x, y, 1.0, 0.0, family=api.FAMILY_VECTOR)
+    assert hit.any() and np.array_equal(~np.isfinite(got), hit)
