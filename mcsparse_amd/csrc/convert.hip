@@ -166,86 +166,10 @@ __global__ __launch_bounds__(kCooBlock, 8) void csr2coo_kernel(idx_t m, idx_t nn
     }
 }
 
-// Offsets from sorted row indices: boundary t (between entry t-1 and entry t, 0 <= t <= nnz) fills
-// the offsets of the rows that lie in between, so empty rows are covered.  A thread takes kCooVectors
-// times four consecutive entries (one 128-bit load each when the array allows it, all asked for before the
-// first is used; 1, 2, 4, 8 vectors: 127, 121, 120, 158 us on 117 M entries) and the boundaries in front of
-// them; the entry before a thread's four comes from the neighbouring lane.
-// Reference semantics: src/kernels/conversion/coo2csr_device.hpp:8-24.
 constexpr int kCooPerThread = 4;
 constexpr int kCooVectors = 2;
-constexpr uint32_t kCooFillRows = 4096;        // offsets a workgroup of the fill kernel looks after
+constexpr uint32_t kCooFillRows = 4096;        // offsets a workgroup that fills long stretches looks after
 constexpr uint64_t kCooDeferredFill = 8192;    // stretches of more offsets than this are its work (>= kCooFillRows)
-template <bool VEC>
-__global__ __launch_bounds__(kBlock) void coo2csr_kernel(idx_t nnz, idx_t m, idx_t base,
-                                                         const idx_t* __restrict__ coo_rows,
-                                                         idx_t* __restrict__ row_ptr) {
-    typedef idx_t idx4 __attribute__((ext_vector_type(4)));
-    const unsigned lane = threadIdx.x % kWave;
-    // entries t0 .. t0+3 of every vector; past the end they read as row m, which makes boundary nnz close
-    // the offsets up to m and the boundaries after it empty
-    uint64_t first[kCooVectors];
-    idx_t r[kCooVectors][kCooPerThread];
-    idx_t lead[kCooVectors];  // entry t0-1 for the first lane of a wavefront
-#pragma unroll
-    for (int j = 0; j < kCooVectors; ++j) {
-        const uint64_t t0 = ((static_cast<uint64_t>(blockIdx.x) * kCooVectors + j) * kBlock + threadIdx.x) * kCooPerThread;
-        first[j] = t0;
-        if (VEC && t0 + kCooPerThread <= nnz) {
-            const idx4 v = __builtin_nontemporal_load(reinterpret_cast<const idx4*>(coo_rows + t0));
-#pragma unroll
-            for (int e = 0; e < kCooPerThread; ++e) r[j][e] = v[e] - base;
-        } else {
-#pragma unroll
-            for (int e = 0; e < kCooPerThread; ++e) r[j][e] = t0 + e < nnz ? load_stream(coo_rows + t0 + e) - base : m;
-        }
-        lead[j] = lane == 0 && t0 != 0 && t0 <= nnz ? coo_rows[t0 - 1] - base : 0;
-    }
-#pragma unroll
-    for (int j = 0; j < kCooVectors; ++j) {
-        const uint64_t t0 = first[j];
-        // entry t0-1: the last entry of the lane below, a load of its own for the first lane of a wavefront
-        idx_t before = __shfl_up(r[j][kCooPerThread - 1], 1, kWave);
-        if (lane == 0) before = lead[j];
-        // rows [prev, cur) get offset t: prev = row of entry t-1 plus one (0 in front of the first entry).
-        // A thread fills short stretches itself; a longer stretch of empty rows is left to the whole
-        // wavefront below, lane by lane 64 offsets at a time; one of more than kCooDeferredFill offsets (up to
-        // all m of them after the last entry) to the kernel after this one.
-        constexpr uint64_t kSerialFill = 16;
-        uint64_t prev = t0 == 0 ? 0 : static_cast<uint64_t>(before) + 1;
-        uint64_t long_from = 0, long_to = 0;  // at most one long stretch is kept per thread; more are filled serially
-        idx_t long_value = 0;
-        if (t0 <= nnz) {
-#pragma unroll
-            for (int e = 0; e < kCooPerThread; ++e) {
-                const uint64_t t = t0 + e;
-                if (t > nnz) break;
-                const uint64_t cur = static_cast<uint64_t>(r[j][e]) + 1;  // t == nnz: m + 1
-                if (cur > prev + kCooDeferredFill) {
-                    // left to coo2csr_fill_kernel: the rows of a matrix with few entries, or all those after the
-                    // last entry, would keep one wavefront busy for as long as the rest of the launch takes
-                } else if (cur > prev + kSerialFill && long_to == long_from) {
-                    long_from = prev;
-                    long_to = cur;
-                    long_value = static_cast<idx_t>(t) + base;
-                } else {
-                    for (uint64_t i = prev; i < cur; ++i) row_ptr[i] = static_cast<idx_t>(t) + base;
-                }
-                prev = cur;
-            }
-        }
-        // every lane of the wavefront gets here: the stretches are handed round and filled cooperatively
-        uint64_t pending = __ballot(long_to > long_from);
-        while (pending != 0) {
-            const int src = __ffsll(static_cast<long long>(pending)) - 1;
-            pending &= pending - 1;
-            const uint64_t from = __shfl(long_from, src, kWave);
-            const uint64_t to = __shfl(long_to, src, kWave);
-            const idx_t value = __shfl(long_value, src, kWave);
-            for (uint64_t i = from + lane; i < to; i += kWave) row_ptr[i] = value;
-        }
-    }
-}
 
 // Number of entries whose row (index base taken off) is below p, in sorted rows, found with 64 probes per
 // round.  Every lane of the wave must call this; all lanes return the same value.
@@ -270,17 +194,16 @@ __device__ __forceinline__ idx_t wave_count_rows_below(const idx_t* __restrict__
     return static_cast<idx_t>(lo);
 }
 
-// The stretches of more than kCooDeferredFill equal offsets that coo2csr_kernel leaves out: a workgroup looks
-// after kCooFillRows offsets.  Such a stretch is longer than that, so if it touches the workgroup's offsets it holds
+// The stretches of more than kCooDeferredFill equal offsets that the other workgroups leave out: this one looks after
+// kCooFillRows offsets.  Such a stretch is longer than that, so if it touches the workgroup's offsets it holds
 // the first or the last of them: for both, the number t of entries in rows below says which stretch they lie in
 // (from the row of entry t-1, exclusive, to the row of entry t, inclusive) and what it holds (t + base).
-__global__ __launch_bounds__(kBlock) void coo2csr_fill_kernel(idx_t nnz, idx_t m, idx_t base,
-                                                              const idx_t* __restrict__ coo_rows,
-                                                              idx_t* __restrict__ row_ptr) {
+__device__ __forceinline__ void fill_long_stretches(uint32_t block, idx_t nnz, idx_t m, idx_t base,
+                                                    const idx_t* __restrict__ coo_rows, idx_t* __restrict__ row_ptr) {
     __shared__ uint64_t s_from[2], s_to[2];
     __shared__ idx_t s_value[2];
     const uint32_t tid = threadIdx.x;
-    const uint64_t i0 = static_cast<uint64_t>(blockIdx.x) * kCooFillRows;
+    const uint64_t i0 = static_cast<uint64_t>(block) * kCooFillRows;
     const uint64_t total = static_cast<uint64_t>(m) + 1;  // offsets 0 .. m
     if (i0 >= total) return;  // whole workgroup
     const uint64_t i1 = i0 + kCooFillRows < total ? i0 + kCooFillRows : total;
@@ -303,6 +226,90 @@ __global__ __launch_bounds__(kBlock) void coo2csr_fill_kernel(idx_t nnz, idx_t m
     for (int k = 0; k < stretches; ++k) {
         const idx_t value = s_value[k];
         for (uint64_t i = s_from[k] + tid; i < s_to[k]; i += kBlock) row_ptr[i] = value;
+    }
+}
+
+// Offsets from sorted row indices: boundary t (between entry t-1 and entry t, 0 <= t <= nnz) fills
+// the offsets of the rows that lie in between, so empty rows are covered.  A thread takes kCooVectors
+// times four consecutive entries (one 128-bit load each when the array allows it, all asked for before the
+// first is used; 1, 2, 4, 8 vectors: 127, 121, 120, 158 us on 117 M entries) and the boundaries in front of
+// them; the entry before a thread's four comes from the neighbouring lane.
+// The grid's first fill_blocks workgroups fill the long stretches of empty rows: neither part reads what the other writes
+// (a kernel of its own took 3 us of the 176 of an assembly of 7.2 M triples).
+// Reference semantics: src/kernels/conversion/coo2csr_device.hpp:8-24.
+template <bool VEC>
+__global__ __launch_bounds__(kBlock) void coo2csr_kernel(idx_t nnz, idx_t m, idx_t base,
+                                                         const idx_t* __restrict__ coo_rows,
+                                                         idx_t* __restrict__ row_ptr, uint32_t fill_blocks) {
+    if (blockIdx.x < fill_blocks) {  // whole workgroup
+        fill_long_stretches(blockIdx.x, nnz, m, base, coo_rows, row_ptr);
+        return;
+    }
+    const uint32_t block = blockIdx.x - fill_blocks;
+    typedef idx_t idx4 __attribute__((ext_vector_type(4)));
+    const unsigned lane = threadIdx.x % kWave;
+    // entries t0 .. t0+3 of every vector; past the end they read as row m, which makes boundary nnz close
+    // the offsets up to m and the boundaries after it empty
+    uint64_t first[kCooVectors];
+    idx_t r[kCooVectors][kCooPerThread];
+    idx_t lead[kCooVectors];  // entry t0-1 for the first lane of a wavefront
+#pragma unroll
+    for (int j = 0; j < kCooVectors; ++j) {
+        const uint64_t t0 = ((static_cast<uint64_t>(block) * kCooVectors + j) * kBlock + threadIdx.x) * kCooPerThread;
+        first[j] = t0;
+        if (VEC && t0 + kCooPerThread <= nnz) {
+            const idx4 v = __builtin_nontemporal_load(reinterpret_cast<const idx4*>(coo_rows + t0));
+#pragma unroll
+            for (int e = 0; e < kCooPerThread; ++e) r[j][e] = v[e] - base;
+        } else {
+#pragma unroll
+            for (int e = 0; e < kCooPerThread; ++e) r[j][e] = t0 + e < nnz ? load_stream(coo_rows + t0 + e) - base : m;
+        }
+        lead[j] = lane == 0 && t0 != 0 && t0 <= nnz ? coo_rows[t0 - 1] - base : 0;
+    }
+#pragma unroll
+    for (int j = 0; j < kCooVectors; ++j) {
+        const uint64_t t0 = first[j];
+        // entry t0-1: the last entry of the lane below, a load of its own for the first lane of a wavefront
+        idx_t before = __shfl_up(r[j][kCooPerThread - 1], 1, kWave);
+        if (lane == 0) before = lead[j];
+        // rows [prev, cur) get offset t: prev = row of entry t-1 plus one (0 in front of the first entry).
+        // A thread fills short stretches itself; a longer stretch of empty rows is left to the whole
+        // wavefront below, lane by lane 64 offsets at a time; one of more than kCooDeferredFill offsets (up to
+        // all m of them after the last entry) to the workgroups for those.
+        constexpr uint64_t kSerialFill = 16;
+        uint64_t prev = t0 == 0 ? 0 : static_cast<uint64_t>(before) + 1;
+        uint64_t long_from = 0, long_to = 0;  // at most one long stretch is kept per thread; more are filled serially
+        idx_t long_value = 0;
+        if (t0 <= nnz) {
+#pragma unroll
+            for (int e = 0; e < kCooPerThread; ++e) {
+                const uint64_t t = t0 + e;
+                if (t > nnz) break;
+                const uint64_t cur = static_cast<uint64_t>(r[j][e]) + 1;  // t == nnz: m + 1
+                if (cur > prev + kCooDeferredFill) {
+                    // left to fill_long_stretches: the rows of a matrix with few entries, or all those after the
+                    // last entry, would keep one wavefront busy for as long as the rest of the launch takes
+                } else if (cur > prev + kSerialFill && long_to == long_from) {
+                    long_from = prev;
+                    long_to = cur;
+                    long_value = static_cast<idx_t>(t) + base;
+                } else {
+                    for (uint64_t i = prev; i < cur; ++i) row_ptr[i] = static_cast<idx_t>(t) + base;
+                }
+                prev = cur;
+            }
+        }
+        // every lane of the wavefront gets here: the stretches are handed round and filled cooperatively
+        uint64_t pending = __ballot(long_to > long_from);
+        while (pending != 0) {
+            const int src = __ffsll(static_cast<long long>(pending)) - 1;
+            pending &= pending - 1;
+            const uint64_t from = __shfl(long_from, src, kWave);
+            const uint64_t to = __shfl(long_to, src, kWave);
+            const idx_t value = __shfl(long_value, src, kWave);
+            for (uint64_t i = from + lane; i < to; i += kWave) row_ptr[i] = value;
+        }
     }
 }
 
@@ -989,17 +996,13 @@ void launch_csr2coo(hipStream_t stream, idx_t m, idx_t nnz, const idx_t* row_ptr
 void launch_coo2csr(hipStream_t stream, idx_t nnz, idx_t m, const idx_t* coo_rows, idx_t base, idx_t* row_ptr) {
     const uint64_t threads = (static_cast<uint64_t>(nnz) + kCooPerThread) / kCooPerThread;  // boundaries 0 .. nnz
     const uint64_t per_block = static_cast<uint64_t>(kBlock) * kCooVectors;
-    const dim3 grid(static_cast<uint32_t>((threads + per_block - 1) / per_block));
-    if (reinterpret_cast<uintptr_t>(coo_rows) % 16 == 0) {
-        hipLaunchKernelGGL(coo2csr_kernel<true>, grid, dim3(kBlock), 0, stream, nnz, m, base, coo_rows, row_ptr);
-    } else {
-        hipLaunchKernelGGL(coo2csr_kernel<false>, grid, dim3(kBlock), 0, stream, nnz, m, base, coo_rows, row_ptr);
-    }
-    if (static_cast<uint64_t>(m) + 1 > kCooDeferredFill) {  // else no stretch is long enough to have been left out
-        const uint64_t blocks = (static_cast<uint64_t>(m) + 1 + kCooFillRows - 1) / kCooFillRows;
-        hipLaunchKernelGGL(coo2csr_fill_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kBlock), 0, stream, nnz, m, base,
-                           coo_rows, row_ptr);
-    }
+    // (without more offsets than that no stretch is long enough to be left out)
+    const uint64_t offsets = static_cast<uint64_t>(m) + 1;
+    const uint32_t fill_blocks =
+        offsets > kCooDeferredFill ? static_cast<uint32_t>((offsets + kCooFillRows - 1) / kCooFillRows) : 0;
+    const dim3 grid(fill_blocks + static_cast<uint32_t>((threads + per_block - 1) / per_block));
+    auto* kernel = reinterpret_cast<uintptr_t>(coo_rows) % 16 == 0 ? coo2csr_kernel<true> : coo2csr_kernel<false>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, stream, nnz, m, base, coo_rows, row_ptr, fill_blocks);
 }
 
 size_t csr2csc_workspace_bytes(idx_t /*m*/, idx_t n, idx_t nnz, size_t value_bytes) {
