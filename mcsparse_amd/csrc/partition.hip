@@ -766,9 +766,39 @@ struct BucketLds {
 // 2 a row (8 M) 452 -> 423, 16 a row (8 M) 423 -> 393; tried with 30 a row (12 M) 555 -> 562, with 60 a row 549 -> 580.
 // Packed words: the first pass takes the eight upper bits of the word, also where more or fewer of them are the major key's,
 // and entries are compared as words, four at a time from where the run's stretch of 16 bytes begins: the words of the runs
-// around it compare as they should.  (Tried wherever the minor key's upper bits may cut the runs short: bands of 216 and 400
-// triples a row 212 -> 252 and 306 -> 357 us, for there they seldom do.)
+// around it compare as they should.  One bound serves four of them: words in front of an entry's own four go before it also
+// if they are equal, those of its four are its neighbours' and are looked at there.  (With a bound for every word, 21
+// instructions for four words and not 13, the assembly of the 7.2 M triples took 174 us, where it takes 168.)  (Tried
+// wherever the minor key's upper bits may cut the runs short: bands of 216 and 400 triples a row 212 -> 252 and 306 -> 357
+// us, for there they seldom do.)
 constexpr uint32_t kShortRun = 64, kUsualRun = 20;
+
+// place + how many of the four words are below the bound.  (The compiler waits for every comparison by itself and sends half
+// of them through a register.)
+__device__ __forceinline__ uint32_t add_smaller(uint32_t place, u32x4 words, uint32_t bound) {
+    uint64_t a, b, c, d;
+    asm("v_cmp_lt_u32_e64 %1, %5, %9\n\t"
+        "v_cmp_lt_u32_e64 %2, %6, %9\n\t"
+        "v_cmp_lt_u32_e64 %3, %7, %9\n\t"
+        "v_cmp_lt_u32_e64 %4, %8, %9\n\t"
+        "v_addc_co_u32_e64 %0, %1, 0, %0, %1\n\t"
+        "v_addc_co_u32_e64 %0, %2, 0, %0, %2\n\t"
+        "v_addc_co_u32_e64 %0, %3, 0, %0, %3\n\t"
+        "v_addc_co_u32_e64 %0, %4, 0, %0, %4"
+        : "+v"(place), "=&s"(a), "=&s"(b), "=&s"(c), "=&s"(d)
+        : "v"(words.x), "v"(words.y), "v"(words.z), "v"(words.w), "v"(bound));
+    return place;
+}
+
+// How many of the lanes below this one in its four hold the same word.
+__device__ __forceinline__ uint32_t equal_below_in_quad(uint32_t word) {
+    const uint32_t lane = threadIdx.x % 4;
+    const int w = static_cast<int>(word);
+    const bool first = __builtin_amdgcn_update_dpp(0, w, 0x00, 0xF, 0xF, false) == w;
+    const bool second = __builtin_amdgcn_update_dpp(0, w, 0x55, 0xF, 0xF, false) == w;
+    const bool third = __builtin_amdgcn_update_dpp(0, w, 0xAA, 0xF, 0xF, false) == w;
+    return (first && lane > 0 ? 1u : 0u) + (second && lane > 1 ? 1u : 0u) + (third && lane > 2 ? 1u : 0u);
+}
 
 // Sorts a bucket of at most ITEMS * kBucketThreads entries, the runs of which are mapped in LDS.  MANY: in several passes.
 template <int VB, typename Key, bool MANY, int ITEMS>
@@ -873,12 +903,14 @@ __device__ __forceinline__ void sort_bucket(const SortTables& t, uint32_t sub, u
                     uint32_t place = q;
                     if constexpr (kPacked) {
                         // (no word is all ones: see sort_packs)
-                        place = q &= ~3u;
-                        for (; q < end; q += 4) {
-                            const u32x4 others = *reinterpret_cast<const u32x4*>(&s.buf[q]);
-#pragma unroll
-                            for (uint32_t j = 0; j < 4; ++j) place += others[j] < mine + (static_cast<int>(here - q) > static_cast<int>(j));
-                        }
+                        // (of equal words those in front count: in front of this four by the bound, in it by the lanes below)
+                        q &= ~3u;
+                        uint32_t own = mine;
+                        forget(own);  // (not all items' at the start, a register each)
+                        place = q + equal_below_in_quad(own);
+                        const uint32_t four = here & ~3u;
+                        const u32x4* others = reinterpret_cast<const u32x4*>(&s.buf[q]);
+                        for (; q < end; q += 4, ++others) place = add_smaller(place, *others, mine + (q < four ? 1u : 0u));
                     } else {
 #pragma unroll 4
                         for (; q < end; ++q) {

@@ -44,6 +44,29 @@ def test_coosort(torch_gpu, handle, oracle, by, with_perm, m, n, nnz, base):
         assert np.array_equal(d_p.cpu().numpy(), p.view(np.int32))
 
 
+@pytest.mark.parametrize("with_perm", [True, False])
+@pytest.mark.parametrize("distinct", [1, 2, 5, 70000])
+def test_coosort_of_short_rows_with_equal_pairs(torch_gpu, handle, oracle, distinct, with_perm):
+    """Rows of 1 to 40 triples, which begin and end anywhere among the groups of four that they are compared in, with every
+    pair many times over (distinct columns in a row: 1, 2, 5) or once: equal pairs stay in the order they came in."""
+    m, n = 20011, 70000
+    rng = np.random.default_rng(distinct)
+    lens = rng.permutation(np.resize(np.arange(1, 41), m))
+    rows = np.repeat(np.arange(m), lens).astype(np.int32)
+    cols = ((rows.astype(np.int64) * 7919 + rng.integers(0, distinct, rows.size) * 31) % n).astype(np.int32)
+    order = rng.permutation(rows.size)
+    rows, cols = rows[order], cols[order]
+    d_r, d_c = dev(torch_gpu, rows), dev(torch_gpu, cols)
+    d_p = dev(torch_gpu, np.arange(rows.size, dtype=np.int32)) if with_perm else None
+    buf = _buffer(torch_gpu, handle, "coo", m, n, rows.size, d_r, d_c)
+    assert api.xcoosort_by_row(handle, m, n, rows.size, d_r, d_c, d_p, buf) == 0
+    torch_gpu.cuda.synchronize()
+    r, c, p = oracle.coosort(m, n, rows, cols, np.arange(rows.size, dtype=np.int32) if with_perm else None)
+    assert np.array_equal(d_r.cpu().numpy(), r.view(np.int32)) and np.array_equal(d_c.cpu().numpy(), c.view(np.int32))
+    if with_perm:
+        assert np.array_equal(d_p.cpu().numpy(), p.view(np.int32))
+
+
 def _shuffle_rows(a, rng):
     col, val = a.col.copy(), a.val.copy()
     for r in np.flatnonzero(a.row_lengths() > 1):
