@@ -132,7 +132,8 @@ __global__ __launch_bounds__(kBlock) void spmv_short_rows_kernel(idx_t m, idx_t 
     const uint32_t lane = threadIdx.x % kWave;
     const uint64_t row0 = (static_cast<uint64_t>(blockIdx.x) * (kBlock / kWave) + threadIdx.x / kWave) * R;
     if (row0 >= m) return;  // whole wavefront
-    const uint64_t row = min(row0 + min(lane, static_cast<uint32_t>(R)), static_cast<uint64_t>(m));  // lanes past the last row have an empty one
+    // (lanes past the last row have an empty one)
+    const uint64_t row = min(row0 + min(lane, static_cast<uint32_t>(R)), static_cast<uint64_t>(m));
     const idx_t start = row_ptr[row] - base, behind = __shfl_down(start, 1, kWave);
     idx_t end = behind;
     if constexpr (R == kWave) {
@@ -620,7 +621,8 @@ void launch_spmv_vector(hipStream_t stream, const SpmvArgs& a, T alpha, T beta, 
     // 32 rows give more wavefronts and fewer of x's lines to each (500,000 random rows of 6: 20.0 us, 22.2 with 64 rows,
     // 22.5 below).
     const uint64_t mean = (static_cast<uint64_t>(a.nnz) + a.m - 1) / a.m;
-    if (lanes == spmv_pick_lanes(a.m, a.nnz) && mean < static_cast<uint64_t>(lanes) && lanes <= 16 && a.m >= 150000 && a.nnz >= 1200000) {
+    if (lanes == spmv_pick_lanes(a.m, a.nnz) && mean < static_cast<uint64_t>(lanes) && lanes <= 16 && a.m >= 150000 &&
+        a.nnz >= 1200000) {
         const bool many = a.m >= 500000;
         switch (mean) {
             case 3: launch_short_rows<T, 64, 3>(stream, a, alpha, beta); return;
