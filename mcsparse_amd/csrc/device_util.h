@@ -134,6 +134,17 @@ __device__ __forceinline__ T load_stream(const T* p) {
     return __builtin_nontemporal_load(p);
 }
 
+// beta*old + alpha*sum of an SpMM, rounded the same way in every kernel that writes C (left to the compiler it is the one or
+// the other product that goes into the fused operation unrounded).
+template <typename T>
+__device__ __forceinline__ T scaled_sum(T alpha, T sum, T beta, T old) {
+    return __builtin_fma(beta, old, alpha * sum);
+}
+template <>
+__device__ __forceinline__ float scaled_sum<float>(float alpha, float sum, float beta, float old) {
+    return __builtin_fmaf(beta, old, alpha * sum);
+}
+
 }  // namespace mcsp
 
 #endif  // MCSPARSE_AMD_DEVICE_UTIL_H_

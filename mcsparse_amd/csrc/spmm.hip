@@ -214,8 +214,8 @@ __global__ __launch_bounds__(kBlock) void spmm_rowb_columns_kernel(idx_t m, idx_
     for (int c = threadIdx.x / kColumnRows<LR>; c < kCols; c += kBlock / kColumnRows<LR>) {
         if (panel + c >= c_cols) break;
         T* out = C + static_cast<int64_t>(panel + c) * ldc + static_cast<int64_t>(row);
-        const T v = alpha * s_c[c][threadIdx.x % kColumnRows<LR>];
-        *out = beta == T(0) ? v : beta * *out + v;
+        const T sum = s_c[c][threadIdx.x % kColumnRows<LR>];
+        *out = beta == T(0) ? alpha * sum : scaled_sum(alpha, sum, beta, *out);
     }
 }
 
@@ -425,7 +425,7 @@ __global__ __launch_bounds__(kBlock) void spmm_colb_kernel(idx_t m, idx_t n, idx
                     if constexpr (BETA0) {
                         *Cp = alpha * s[jj];
                     } else {
-                        *Cp = beta * *Cp + alpha * s[jj];
+                        *Cp = scaled_sum(alpha, s[jj], beta, *Cp);
                     }
                 }
             }

@@ -201,17 +201,6 @@ __device__ __forceinline__ void row_times_b(idx_t begin, idx_t end, idx_t lane, 
     }
 }
 
-// beta*old + alpha*acc, rounded the same way in every kernel (left to the compiler it is the one or the other product that
-// goes into the fused operation unrounded).
-template <typename T>
-__device__ __forceinline__ T scaled_sum(T alpha, T acc, T beta, T old) {
-    return __builtin_fma(beta, old, alpha * acc);
-}
-template <>
-__device__ __forceinline__ float scaled_sum<float>(float alpha, float acc, float beta, float old) {
-    return __builtin_fmaf(beta, old, alpha * acc);
-}
-
 // Writes V adjacent columns of one row of C but for the first `skip`: beta*C + alpha*acc, C untouched by reads if
 // beta == 0.
 template <typename T, int V>
@@ -262,7 +251,7 @@ __device__ __forceinline__ void store_c_four_rows(T* __restrict__ Cp, T a0, T a1
         } else {
             const Vec<T, W> old = load_vec<T, W>(Cp + h * W);
 #pragma unroll
-            for (int i = 0; i < W; ++i) out.v[i] = beta * old.v[i] + alpha * acc[h * W + i];
+            for (int i = 0; i < W; ++i) out.v[i] = scaled_sum(alpha, acc[h * W + i], beta, old.v[i]);
         }
         store_vec<T, W>(Cp + h * W, out);
     }

@@ -202,13 +202,13 @@ __global__ __launch_bounds__(kPanelWaves * kWave, 4) void spmm_diagonals_kernel(
             if constexpr (!BETA0) {
                 const vec_t old = *reinterpret_cast<const element_aligned*>(out);
 #pragma unroll
-                for (int j = 0; j < R; ++j) s[j] = beta * old[j] + alpha * sum[c][j];
+                for (int j = 0; j < R; ++j) s[j] = scaled_sum(alpha, sum[c][j], beta, old[j]);
             }
             __builtin_nontemporal_store(s, reinterpret_cast<element_aligned*>(out));
         } else {
 #pragma unroll
             for (int j = 0; j < R; ++j) {
-                if (row + j < m) out[j] = BETA0 ? alpha * sum[c][j] : beta * out[j] + alpha * sum[c][j];
+                if (row + j < m) out[j] = BETA0 ? alpha * sum[c][j] : scaled_sum(alpha, sum[c][j], beta, out[j]);
             }
         }
     }
