@@ -478,3 +478,25 @@ def test_tiles_cut_evenly(torch_gpu, handle, oracle, dtype, op, m, n, nnz, heavy
     ptr = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=m))])
     a = wl.Csr(m, n, ptr, rng.integers(0, n, nnz), rng.integers(-8, 9, nnz).astype(dtype))
     run(torch_gpu, handle, oracle, a, 2.0, -1.0, op=op)
+
+
+def test_bands_have_the_width_the_caller_sets(torch_gpu, handle, oracle):
+    """Bands of 1024 columns, the last one of 100.  The partial sum of a band is rounded to fp32, which tells where a band ends:
+    2^24 + 1 in one band is 2^24, 1 + 1 in the next is 2."""
+    torch = torch_gpu
+    m, n = 70001, 29 * 1024 + 100
+    cols = np.tile(np.array([5, 1000, 1500], np.int32), m)
+    a = wl.Csr(m, n, np.arange(m + 1) * 3, cols, np.tile(np.array([2.0 ** 24, 1, 1], np.float32), m))
+    mat = api.SpMat(m, n, a.nnz, dev(torch, a.ptr.astype(np.int32)), dev(torch, a.col), dev(torch, a.val))
+    mat.set_band_bytes(4096)
+    d_y = torch.zeros(m, dtype=torch.float32, device="cuda")
+    vx, vy = api.DnVec(torch.ones(n, dtype=torch.float32, device="cuda")), api.DnVec(d_y)
+    args = (handle, api.OP_N, 1.0, mat, vx, 0.0, vy, api.R_32F)
+    st, size = api.spmv_preprocess_buffer_size(*args)
+    assert st == api.STATUS_SUCCESS
+    buf = torch.empty(size, dtype=torch.uint8, device="cuda")
+    assert api.spmv_preprocess(*args, buf) == api.STATUS_SUCCESS
+    assert mat.spmv_preprocess_state()[:2] == (3, 30)
+    assert api.spmv(*args, buf) == api.STATUS_SUCCESS
+    torch.cuda.synchronize()
+    assert (d_y.cpu().numpy() == 2.0 ** 24).all()
