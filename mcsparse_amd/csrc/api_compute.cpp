@@ -397,7 +397,7 @@ mcspStatus_t spmv_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
         if (A->plan.family == kFamilyMerge) {
             mcsp::launch_spmv_merge<T>(h->stream, a, h_alpha, h_beta, buf + l.merge_ws, A->plan.lanes != 0);
         } else {
-            mcsp::launch_spmv_vector<T>(h->stream, a, h_alpha, h_beta, A->plan.lanes);
+            mcsp::launch_spmv_vector<T>(h->stream, a, h_alpha, h_beta, A->plan.lanes, true);
         }
         return MCSP_STATUS_SUCCESS;
     }

@@ -51,8 +51,8 @@ mcspStatus_t csrmv_impl(mcsparseHandle_t handle, int m, int n, int nnz, const T*
     a.x = x;
     a.y = y;
     // the typed entry points have no buffer whose size is known (csrmv has none, CsrmvEx's is the
-    // reference's constant 128 bytes and is never touched there, :905-944): row-per-lane-group kernel
-    mcsp::launch_spmv_vector<T>(handle->stream, a, h_alpha, h_beta, mcsp::spmv_pick_lanes(a.m, a.nnz));
+    // reference's constant 128 bytes and is never touched there, :905-944): row-per-lane-group kernel, for rows of any length
+    mcsp::launch_spmv_vector<T>(handle->stream, a, h_alpha, h_beta, mcsp::spmv_pick_lanes(a.m, a.nnz), false);
     return MCSP_STATUS_SUCCESS;
 }
 

@@ -285,12 +285,12 @@ struct SpmvArgs {
     const void* x;
     void* y;
 };
-// y = alpha*A*x + beta*y; beta == 0 never reads y.
+// y = alpha*A*x + beta*y; beta == 0 never reads y.  stretches: rows of a few nonzeros may be read as one stretch.
 // The kernels of spmv.hip come to the device together, with the first launch of any of them, which takes that launch
 // milliseconds.  This call brings them there beforehand.
 bool load_row_kernels();
 template <typename T>
-void launch_spmv_vector(hipStream_t stream, const SpmvArgs& a, T alpha, T beta, int lanes);
+void launch_spmv_vector(hipStream_t stream, const SpmvArgs& a, T alpha, T beta, int lanes, bool stretches);
 // workspace: spmv_merge_workspace_bytes(m, nnz, sizeof(T)) bytes of device scratch.
 size_t spmv_merge_workspace_bytes(idx_t m, idx_t nnz, size_t value_bytes);
 // order_tiles: the tiles run in the order of their first column.

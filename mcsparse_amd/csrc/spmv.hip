@@ -611,7 +611,7 @@ bool load_row_kernels() {
 }
 
 template <typename T>
-void launch_spmv_vector(hipStream_t stream, const SpmvArgs& a, T alpha, T beta, int lanes) {
+void launch_spmv_vector(hipStream_t stream, const SpmvArgs& a, T alpha, T beta, int lanes, bool stretches) {
     if (a.m == 0) return;
     // Rows of 3, 5 to 7 or 9 to 15 nonzeros are read as one stretch.  (4 and 8 fill the lanes of the kernel below: random
     // columns, 200,000 rows of 8, fp64, 14.4 us below and 14.9 here.)  A row takes a whole lane here, so it needs more rows
@@ -619,9 +619,11 @@ void launch_spmv_vector(hipStream_t stream, const SpmvArgs& a, T alpha, T beta, 
     // 9.9 here; 300,000 rows of 5 15.6 and 15.4 (fp32 13.1 and 12.5), 160,000 rows of 9 14.4 and 12.9.  64 rows to a
     // wavefront read a stencil with the fewest instructions (7 points of 140^3, fp32: 36 us, with 32 rows 41, below 44);
     // 32 rows give more wavefronts and fewer of x's lines to each (500,000 random rows of 6: 20.0 us, 22.2 with 64 rows,
-    // 22.5 below).
+    // 22.5 below).  Rows of very different length keep most of these lanes waiting for the longest one's: a call that knows
+    // nothing of its rows takes the kernel below (a million power-law rows, at most 1000 long, mean 6, through csrmv: fp32 125 us
+    // below, 173 here; fp64 160 and 211; 200,000 rows of 12 and a hundred of 3000, fp64, 148 and 187).
     const uint64_t mean = (static_cast<uint64_t>(a.nnz) + a.m - 1) / a.m;
-    if (lanes == spmv_pick_lanes(a.m, a.nnz) && mean < static_cast<uint64_t>(lanes) && lanes <= 16 && a.m >= 150000 &&
+    if (stretches && lanes == spmv_pick_lanes(a.m, a.nnz) && mean < static_cast<uint64_t>(lanes) && lanes <= 16 && a.m >= 150000 &&
         a.nnz >= 1200000) {
         const bool many = a.m >= 500000;
         switch (mean) {
@@ -824,8 +826,8 @@ template bool launch_skinny_transpose<double>(hipStream_t, idx_t, idx_t, idx_t, 
 
 template void launch_row_sums_merge<float>(hipStream_t, const SpmvArgs&, float, float, void*);
 template void launch_row_sums_merge<double>(hipStream_t, const SpmvArgs&, double, double, void*);
-template void launch_spmv_vector<float>(hipStream_t, const SpmvArgs&, float, float, int);
-template void launch_spmv_vector<double>(hipStream_t, const SpmvArgs&, double, double, int);
+template void launch_spmv_vector<float>(hipStream_t, const SpmvArgs&, float, float, int, bool);
+template void launch_spmv_vector<double>(hipStream_t, const SpmvArgs&, double, double, int, bool);
 template void launch_spmv_merge<float>(hipStream_t, const SpmvArgs&, float, float, void*, bool);
 template void launch_spmv_merge<double>(hipStream_t, const SpmvArgs&, double, double, void*, bool);
 

@@ -53,6 +53,41 @@ def test_csrmv(torch_gpu, handle, oracle, lib, dtype, base, entry):
     lib.mcsparseDestroyMatDescr(d)
 
 
+def rows_of(lens, n, dtype, seed):
+    rng = np.random.default_rng(seed)
+    ptr = np.concatenate([[0], np.cumsum(lens)])
+    return wl.Csr(len(lens), n, ptr.astype(np.int32), rng.integers(0, n, ptr[-1]).astype(np.int32),
+                  rng.uniform(-1, 1, ptr[-1]).astype(dtype))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("mean,m,longest", [(5, 280_001, 3000), (7, 500_003, 5000), (12, 160_001, 3000)])
+def test_csrmv_knows_nothing_of_its_rows(torch_gpu, handle, oracle, lib, dtype, mean, m, longest):
+    """Many short rows with a few long ones among them, and the bits of its first rows by themselves: no row-length analysis
+    is there to say that rows may share lanes, so it is a lane group to a row, however many rows there are."""
+    rng = np.random.default_rng(mean)
+    lens = rng.integers(mean - 2, mean + 2, m)
+    lens[100::m // 20] = longest
+    a = rows_of(lens, 50_021, dtype, 3)
+    x = rng.uniform(-1, 1, a.n).astype(dtype)
+    sc = ctypes.c_float if dtype == np.float32 else ctypes.c_double
+    pa, pb = sc(1.25), sc(0.0)
+    d = mat_descr(lib, 0)
+    d_ptr, d_col, d_val, d_x = (dev(torch_gpu, v) for v in (a.ptr, a.col, a.val, x))
+    fn = lib.mcsparseScsrmv if dtype == np.float32 else lib.mcsparseDcsrmv
+    out = []
+    for rows in (m, 100_000):
+        d_y = dev(torch_gpu, np.full(rows, 7, dtype))
+        assert fn(handle.ptr, api.OP_N, rows, a.n, int(a.ptr[rows]), ctypes.addressof(pa), d, d_val.data_ptr(), d_ptr.data_ptr(),
+                  d_col.data_ptr(), d_x.data_ptr(), ctypes.addressof(pb), d_y.data_ptr()) == 0
+        torch_gpu.cuda.synchronize()
+        out.append(d_y.cpu().numpy())
+    y_ref, bound = oracle.spmv(False, m, a.n, 0, a.ptr, a.col, a.val, 1.25, 0.0, x, np.zeros(m, dtype))
+    assert_within(out[0], y_ref, bound, dtype, what="csrmv")
+    assert np.array_equal(out[0][:100_000], out[1])
+    lib.mcsparseDestroyMatDescr(d)
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("trans_b", [api.OP_N, api.OP_T])
 @pytest.mark.parametrize("n", [1, 8, 33])
