@@ -216,6 +216,7 @@ mcspStatus_t ensure_plan(mcsparseHandle_t h, mcsparseSpMatDescr* A, const idx_t*
         p.family = p.forced_family;
         // merge family: lanes != 0 asks for the tiles to run in the order of their first column
         p.lanes = p.family == kFamilyVector ? (p.forced_lanes ? p.forced_lanes : mean_lanes) : (p.forced_lanes ? 1 : 0);
+        p.stretches = p.forced_lanes == 0;
         p.max_row_len = 0;
         p.valid = true;
         return MCSP_STATUS_SUCCESS;
@@ -230,6 +231,7 @@ mcspStatus_t ensure_plan(mcsparseHandle_t h, mcsparseSpMatDescr* A, const idx_t*
     p.max_row_len = host_hist[MCSPARSE_ROW_BIN_COUNT];
     mcsp::spmv_plan_from_bins(host_hist, m, nnz, x_bytes, &p.family, &p.lanes);
     if (p.family == kFamilyVector && p.forced_lanes) p.lanes = p.forced_lanes;
+    p.stretches = p.forced_lanes == 0;
     p.valid = true;
     return MCSP_STATUS_SUCCESS;
 }
@@ -397,7 +399,7 @@ mcspStatus_t spmv_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
         if (A->plan.family == kFamilyMerge) {
             mcsp::launch_spmv_merge<T>(h->stream, a, h_alpha, h_beta, buf + l.merge_ws, A->plan.lanes != 0);
         } else {
-            mcsp::launch_spmv_vector<T>(h->stream, a, h_alpha, h_beta, A->plan.lanes, true);
+            mcsp::launch_spmv_vector<T>(h->stream, a, h_alpha, h_beta, A->plan.lanes, A->plan.stretches);
         }
         return MCSP_STATUS_SUCCESS;
     }

@@ -76,6 +76,7 @@ struct SpmvPlan {
     // outcome
     int family = kFamilyAuto;
     int lanes = 0;
+    bool stretches = false;  // vector family: rows of a few nonzeros may be read as one stretch (launch_spmv_vector)
     uint32_t max_row_len = 0;
     uint32_t hist[MCSPARSE_ROW_BIN_COUNT] = {0};
     // user override (mcsparseSpMatSetSpMVPlan); kFamilyAuto = none

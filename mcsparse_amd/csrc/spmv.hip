@@ -623,7 +623,7 @@ void launch_spmv_vector(hipStream_t stream, const SpmvArgs& a, T alpha, T beta, 
     // nothing of its rows takes the kernel below (a million power-law rows, at most 1000 long, mean 6, through csrmv: fp32 125 us
     // below, 173 here; fp64 160 and 211; 200,000 rows of 12 and a hundred of 3000, fp64, 148 and 187).
     const uint64_t mean = (static_cast<uint64_t>(a.nnz) + a.m - 1) / a.m;
-    if (stretches && lanes == spmv_pick_lanes(a.m, a.nnz) && mean < static_cast<uint64_t>(lanes) && lanes <= 16 && a.m >= 150000 &&
+    if (stretches && mean < static_cast<uint64_t>(lanes) && lanes <= 16 && a.m >= 150000 &&
         a.nnz >= 1200000) {
         const bool many = a.m >= 500000;
         switch (mean) {

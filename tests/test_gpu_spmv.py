@@ -252,3 +252,28 @@ def test_short_rows_are_read_as_one_stretch(torch_gpu, handle, oracle, dtype, me
     hit[np.repeat(np.arange(m), lens)[a.col == n // 2 + base]] = True
     _, got, _ = run_spmv(torch_gpu, handle, a, x, y, 1.0, 0.0, family=api.FAMILY_VECTOR)
     assert hit.any() and np.array_equal(~np.isfinite(got), hit)
+
+
+def first_rows(a, rows):
+    last = a.ptr[rows] - a.base
+    return wl.Csr(rows, a.n, a.ptr[:rows + 1], a.col[:last], a.val[:last], base=a.base)
+
+
+def rows_like_the_first_ones_alone(torch, handle, a, family, lanes, plan, rows=100_000):
+    """Whether the first rows of A x have the bits of a product of these rows alone, too few to be read as one stretch."""
+    x = np.random.default_rng(2).uniform(-1, 1, a.n).astype(a.val.dtype)
+    out = []
+    for b in (a, first_rows(a, rows)):
+        st, y, chosen = run_spmv(torch, handle, b, x, np.zeros(b.m, a.val.dtype), 1.0, 0.0, family=family, lanes=lanes)
+        assert st == api.STATUS_SUCCESS and chosen == plan
+        out.append(y[:rows])
+    return np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("family", [api.FAMILY_VECTOR, api.FAMILY_AUTO])
+@pytest.mark.parametrize("per_row,lanes,m", [(3, 4, 400_063), (6, 8, 300_001), (12, 16, 150_031)])
+def test_lanes_that_are_asked_for_are_used(torch_gpu, handle, dtype, family, per_row, lanes, m):
+    """Also where they are as many as the library would choose."""
+    a = wl.uniform_rows(m=m, n=60_000, per_row=per_row, dtype=dtype)
+    assert rows_like_the_first_ones_alone(torch_gpu, handle, a, family, lanes, (api.FAMILY_VECTOR, lanes))
