@@ -110,7 +110,8 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 7 : 1) void sp
         const uint32_t roff = (c_now - base) * ldb_bytes;
         const T aa = a_now;
         const bool done = left <= LR;  // whole lane groups
-        uint32_t row_next = row, j_next = j + LR, end_next = end;
+        // (a group that has run out of rows stays at an empty one: else it would gather for nonzeros that are none of its own)
+        uint32_t row_next = row, j_next = active ? j + LR : end, end_next = end;
         bool active_next = active;
         auto ask_next = [&]() {
             const unsigned long long through = __ballot(done && active && lane == 0);
