@@ -366,10 +366,17 @@ __global__ __launch_bounds__(kBlock) void column_order_pack_kernel(idx_t nnz, id
     if (k >= nnz) return;
     const idx_t key = c_keys[k];
     const idx_t row = min(r_keys[k] - base, m - 1);
-    uint32_t chunk = min(row / mean_rows, chunks - 1);  // or one near it
+    uint32_t chunk = min(row / mean_rows, chunks - 1);  // unless the chunks are cut by nonzeros
     uint32_t chunk_row = chunk_first[chunk];
-    while (chunk != 0 && row < chunk_row) chunk_row = chunk_first[--chunk];
-    for (uint32_t next; chunk + 1 < chunks && row >= (next = chunk_first[chunk + 1]); ++chunk) chunk_row = next;
+    if (row < chunk_row || (chunk + 1 < chunks && row >= chunk_first[chunk + 1])) {
+        uint32_t end = chunks;  // the last chunk that begins at or before the row
+        chunk = 0;
+        while (end - chunk > 1) {
+            const uint32_t mid = (chunk + end) / 2;
+            if (chunk_first[mid] <= row) chunk = mid; else end = mid;
+        }
+        chunk_row = chunk_first[chunk];
+    }
     const uint32_t band = key / band_keys;
     const uint32_t group = band / sub;
     ids_out[k] = (group * chunks + chunk) * sub + (band - group * sub);

@@ -465,6 +465,7 @@ def test_tiles_and_units_of_a_few_entries_or_none(torch_gpu, handle, oracle, dty
 @pytest.mark.parametrize("m,n,nnz,heavy", [
     (300001, 290003, 3300000, 0),     # one unit a compute unit, a thousand rows each
     (300001, 290003, 3300000, 9),     # the first and the last rows hold most nonzeros: the tiles between them are as tall as may be
+    (300001, 290003, 3300000, 150),   # so many that most tiles are a row or two: no tile is where its rows would be in even ones
     (700001, 1600003, 200000, 0),     # several band groups, two or three turns of units of nearly full height
 ])
 def test_tiles_cut_evenly(torch_gpu, handle, oracle, dtype, op, m, n, nnz, heavy):
