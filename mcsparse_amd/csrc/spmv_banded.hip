@@ -317,14 +317,15 @@ __global__ __launch_bounds__(kBlock) void banded_reduce_wide_kernel(idx_t m, uin
 //
 // chunk_first: the first row of every chunk, and m.  A chunk has at most rows_per_tile rows, on average mean_rows.  Where that
 // leaves room and there are row offsets (row_ptr), the chunks hold equally many nonzeros, else mean_rows rows each.
-constexpr uint32_t kCutChunks = 4096;
+// (Only where every compute unit has one unit (column_order_shape), so there are at most as many chunks.)
+constexpr uint32_t kCutChunks = kXcds * kColumnGroupsPerXcd;
 constexpr int kCutBlock = 1024;
 __global__ __launch_bounds__(kCutBlock) void column_order_cut_kernel(idx_t m, idx_t nnz, idx_t base, const idx_t* __restrict__ row_ptr,
                                                                      uint32_t chunks, uint32_t mean_rows, uint32_t rows_per_tile,
                                                                      uint32_t* __restrict__ chunk_first) {
     __shared__ long long s_cut[2][kCutChunks + 1];
     const uint32_t tid = threadIdx.x;
-    if (row_ptr == nullptr || chunks > kCutChunks || mean_rows == rows_per_tile) {  // whole workgroup
+    if (row_ptr == nullptr || mean_rows == rows_per_tile) {  // whole workgroup
         for (uint32_t i = tid; i <= chunks; i += kCutBlock)
             chunk_first[i] = static_cast<uint32_t>(min(static_cast<uint64_t>(i) * mean_rows, static_cast<uint64_t>(m)));
         return;
