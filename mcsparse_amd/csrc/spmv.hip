@@ -119,18 +119,18 @@ __global__ __launch_bounds__(kBlock) void spmv_vector_kernel(idx_t m, idx_t base
 // than its pointer; that leaves the latency of a chain of three loads and one passage through LDS.  Before and after, in
 // us: five-point Laplacian of 512 x 512, fp32 5.5 and 4.8, of 1700 x 1700 42 and 30 (fp64 58 and 43); nine-point of 1000 x
 // 1000 34 and 19 (fp64 39 and 25), which is 97 MB at 5.0 TB/s and 133 MB at 5.3.
-template <typename T, int R, int U, int UPDATE>
-__global__ __launch_bounds__(kBlock) void spmv_short_rows_kernel(idx_t m, idx_t base, const idx_t* __restrict__ row_ptr,
+template <typename T, int R, int U, int THREADS, int UPDATE>
+__global__ __launch_bounds__(THREADS) void spmv_short_rows_kernel(idx_t m, idx_t base, const idx_t* __restrict__ row_ptr,
                                                                  const idx_t* __restrict__ col, const T* __restrict__ val,
                                                                  const T* __restrict__ x, T* __restrict__ y, T alpha, T beta) {
     constexpr uint32_t kWindow = U * kWave;
     // (a place is skipped behind every 32: rows of 4, 8 or 16 nonzeros would begin on the same banks)
     auto place = [](uint32_t k) { return k + k / 32; };
     constexpr uint32_t kPlaces = kWindow + kWindow / 32;
-    __shared__ T s_products[kBlock / kWave][kPlaces];
+    __shared__ T s_products[THREADS / kWave][kPlaces];
     T* products = s_products[threadIdx.x / kWave];
     const uint32_t lane = threadIdx.x % kWave;
-    const uint64_t row0 = (static_cast<uint64_t>(blockIdx.x) * (kBlock / kWave) + threadIdx.x / kWave) * R;
+    const uint64_t row0 = (static_cast<uint64_t>(blockIdx.x) * (THREADS / kWave) + threadIdx.x / kWave) * R;
     if (row0 >= m) return;  // whole wavefront
     // (lanes past the last row have an empty one)
     const uint64_t row = min(row0 + min(lane, static_cast<uint32_t>(R)), static_cast<uint64_t>(m));
@@ -225,12 +225,12 @@ __global__ __launch_bounds__(kBlock) void spmv_short_rows_kernel(idx_t m, idx_t 
     }
 }
 
-template <typename T, int R, int U>
+template <typename T, int R, int U, int THREADS>
 void launch_short_rows(hipStream_t stream, const SpmvArgs& a, T alpha, T beta) {
-    constexpr uint32_t kRows = kBlock / kWave * R;
+    constexpr uint32_t kRows = THREADS / kWave * R;
     const dim3 grid(static_cast<uint32_t>((static_cast<uint64_t>(a.m) + kRows - 1) / kRows));
-    auto* kernel = beta == T(0) ? spmv_short_rows_kernel<T, R, U, kYSet> : spmv_short_rows_kernel<T, R, U, kYScale>;
-    hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, stream, a.m, a.base, a.row_ptr, a.col, static_cast<const T*>(a.val),
+    auto* kernel = beta == T(0) ? spmv_short_rows_kernel<T, R, U, THREADS, kYSet> : spmv_short_rows_kernel<T, R, U, THREADS, kYScale>;
+    hipLaunchKernelGGL(kernel, grid, dim3(THREADS), 0, stream, a.m, a.base, a.row_ptr, a.col, static_cast<const T*>(a.val),
                        static_cast<const T*>(a.x), static_cast<T*>(a.y), alpha, beta);
 }
 
@@ -622,28 +622,40 @@ void launch_spmv_vector(hipStream_t stream, const SpmvArgs& a, T alpha, T beta, 
     // 22.5 below).  Rows of very different length keep most of these lanes waiting for the longest one's: a call that knows
     // nothing of its rows takes the kernel below (a million power-law rows, at most 1000 long, mean 6, through csrmv: fp32 125 us
     // below, 173 here; fp64 160 and 211; 200,000 rows of 12 and a hundred of 3000, fp64, 148 and 187).
+    // Workgroups of two wavefronts for the shortest rows, below a million of them: with four, a few hundred thousand rows are
+    // four to six workgroups to a compute unit, and where some have one more than the others the call waits for those (random
+    // columns, fp64, four and two: 270,000 rows of 5 14.8 and 14.0 us, below 14.2; 350,000 17.8 and 16.8, below 17.4; 171,500
+    // rows of 7 12.3 and 12.0, below 11.9; five-point stencil of 1900 x 1900 55.5 and 57.0).  With 64 rows of 7 to a wavefront
+    // four stay (stencil of 110^3, fp64, 26.8 and 27.6), but in fp64 that is from 700,000 rows on: 500,000 random rows of 7
+    // 31.7 us, with 32 rows 29.7, below 30.9.
     const uint64_t mean = (static_cast<uint64_t>(a.nnz) + a.m - 1) / a.m;
     if (stretches && mean < static_cast<uint64_t>(lanes) && lanes <= 16 && a.m >= 150000 &&
         a.nnz >= 1200000) {
-        const bool many = a.m >= 500000;
+        const bool many = a.m >= 1000000;
         switch (mean) {
-            case 3: launch_short_rows<T, 64, 3>(stream, a, alpha, beta); return;
-            case 5: launch_short_rows<T, 64, 5>(stream, a, alpha, beta); return;
+            case 3:
+                if (many) launch_short_rows<T, 64, 3, 256>(stream, a, alpha, beta);
+                else launch_short_rows<T, 64, 3, 128>(stream, a, alpha, beta);
+                return;
+            case 5:
+                if (many) launch_short_rows<T, 64, 5, 256>(stream, a, alpha, beta);
+                else launch_short_rows<T, 64, 5, 128>(stream, a, alpha, beta);
+                return;
             case 6:
-                if (many) launch_short_rows<T, 64, 6>(stream, a, alpha, beta);
-                else launch_short_rows<T, 32, 3>(stream, a, alpha, beta);
+                if (a.m >= 500000) launch_short_rows<T, 64, 6, 256>(stream, a, alpha, beta);
+                else launch_short_rows<T, 32, 3, 128>(stream, a, alpha, beta);
                 return;
             case 7:
-                if (many) launch_short_rows<T, 64, 7>(stream, a, alpha, beta);
-                else launch_short_rows<T, 32, 4>(stream, a, alpha, beta);
+                if (a.m >= (sizeof(T) == 8 ? 700000 : 500000)) launch_short_rows<T, 64, 7, 256>(stream, a, alpha, beta);
+                else launch_short_rows<T, 32, 4, 128>(stream, a, alpha, beta);
                 return;
             case 9:
-            case 10: launch_short_rows<T, 32, 5>(stream, a, alpha, beta); return;
+            case 10: launch_short_rows<T, 32, 5, 256>(stream, a, alpha, beta); return;
             case 11:
-            case 12: launch_short_rows<T, 32, 6>(stream, a, alpha, beta); return;
+            case 12: launch_short_rows<T, 32, 6, 256>(stream, a, alpha, beta); return;
             case 13:
-            case 14: launch_short_rows<T, 32, 7>(stream, a, alpha, beta); return;
-            default: launch_short_rows<T, 32, 8>(stream, a, alpha, beta); return;
+            case 14: launch_short_rows<T, 32, 7, 256>(stream, a, alpha, beta); return;
+            default: launch_short_rows<T, 32, 8, 256>(stream, a, alpha, beta); return;
         }
     }
     switch (lanes) {
