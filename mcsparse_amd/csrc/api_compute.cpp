@@ -15,6 +15,9 @@ namespace {
 constexpr size_t kAnalysisBytes = align_up((MCSPARSE_ROW_BIN_COUNT + 1) * sizeof(uint32_t));
 
 bool fits_32(int64_t v) { return (v >> 32) == 0; }
+// The kernels step through the nonzeros with 32-bit places, some ten thousand at a time: a step from near 2^32 must not come
+// round to the first ones, where it would never end.
+bool nonzeros_fit(int64_t nnz) { return nnz <= (int64_t(1) << 32) - (int64_t(1) << 16); }
 
 // A stream that is being captured into a HIP graph cannot be synchronised: trying to would fail and
 // invalidate the caller's capture.
@@ -123,7 +126,7 @@ mcspStatus_t check_spmv_args(mcsparseHandle_t handle, mcsparseOperation_t opA, c
     if (handle == nullptr) return MCSP_STATUS_INVALID_HANDLE;
     if (alpha == nullptr || beta == nullptr || A == nullptr || x == nullptr || y == nullptr || !other_pointers_ok)
         return MCSP_STATUS_INVALID_POINTER;
-    if (!fits_32(A->row_num) || !fits_32(A->col_num) || !fits_32(A->nnz) || !fits_32(x->size) || !fits_32(y->size))
+    if (!fits_32(A->row_num) || !fits_32(A->col_num) || !nonzeros_fit(A->nnz) || !fits_32(x->size) || !fits_32(y->size))
         return MCSP_STATUS_NOT_IMPLEMENTED;
     if (need_buffer && buffer == nullptr) return MCSP_STATUS_INVALID_POINTER;
     if (!(A->format == MCSPARSE_FORMAT_CSR || A->format == MCSPARSE_FORMAT_COO ||
@@ -708,7 +711,7 @@ mcspStatus_t check_spmm_args(mcsparseHandle_t handle, const void* alpha, const m
     if (handle == nullptr) return MCSP_STATUS_INVALID_HANDLE;
     if (A == nullptr || B == nullptr || C == nullptr || alpha == nullptr || beta == nullptr)
         return MCSP_STATUS_INVALID_POINTER;
-    if (!fits_32(A->row_num) || !fits_32(A->col_num) || !fits_32(A->nnz) || !fits_32(B->row_num) ||
+    if (!fits_32(A->row_num) || !fits_32(A->col_num) || !nonzeros_fit(A->nnz) || !fits_32(B->row_num) ||
         !fits_32(B->col_num) || !fits_32(B->ld) || !fits_32(C->row_num) || !fits_32(C->col_num) || !fits_32(C->ld))
         return MCSP_STATUS_NOT_IMPLEMENTED;
     if (A->format != MCSPARSE_FORMAT_CSR && A->format != MCSPARSE_FORMAT_COO &&

@@ -227,6 +227,22 @@ def test_spmv_argument_checks(lib):
     assert cplx.spmv(ct=api.C_32F) == api.STATUS_NOT_SUPPORTED
 
 
+def test_nonzeros_stay_a_step_below_32_bits(lib):
+    """Kernels step through the nonzeros with 32-bit places, up to 2^16 at a time: a matrix whose last ones are nearer to 2^32
+    is refused as one beyond it is, for its last step would come round to the first nonzeros."""
+    most = (1 << 32) - (1 << 16)
+    assert Objs(lib, nnz=most).spmv_size()[0] == api.STATUS_SUCCESS
+    for nnz in (most + 1, (1 << 32) - 1, 1 << 32):
+        o = Objs(lib, nnz=nnz)
+        assert o.spmv_size()[0] == o.spmv() == api.STATUS_NOT_SUPPORTED
+        B, C = ctypes.c_void_p(), ctypes.c_void_p()
+        assert lib.mcsparseCreateDnMat(ctypes.byref(B), 6, 4, 4, FAKE, api.R_32F, api.ORDER_ROW) == 0
+        assert lib.mcsparseCreateDnMat(ctypes.byref(C), 8, 4, 4, FAKE, api.R_32F, api.ORDER_ROW) == 0
+        assert lib.mcsparseSpMM(o.h, api.OP_N, api.OP_N, o.pa, o.A, B, o.pa, C, api.R_32F, 0, FAKE) == api.STATUS_NOT_SUPPORTED
+        lib.mcsparseDestroyDnMat(B)
+        lib.mcsparseDestroyDnMat(C)
+
+
 def test_spmv_early_outs_touch_nothing(lib):
     # mcsp_spmv_gpu.cpp:235-237: nnz == 0, or alpha == beta == 0, returns before any launch.
     # The pointers here are fake, so reaching a kernel would fault rather than pass.
