@@ -325,7 +325,7 @@ __global__ __launch_bounds__(kCutBlock) void column_order_cut_kernel(idx_t m, id
                                                                      uint32_t* __restrict__ chunk_first) {
     __shared__ long long s_cut[2][kCutChunks + 1];
     const uint32_t tid = threadIdx.x;
-    if (row_ptr == nullptr || mean_rows == rows_per_tile) {  // whole workgroup
+    if (row_ptr == nullptr) {  // whole workgroup
         for (uint32_t i = tid; i <= chunks; i += kCutBlock)
             chunk_first[i] = static_cast<uint32_t>(min(static_cast<uint64_t>(i) * mean_rows, static_cast<uint64_t>(m)));
         return;
@@ -358,30 +358,52 @@ __global__ __launch_bounds__(kCutBlock) void column_order_cut_kernel(idx_t m, id
 // Nonzero k (row key r, column key c, both with the index base in) gets its tile number and the same
 // packed word as above.  ids_out / packed_out may be the input arrays themselves (element k is read
 // before it is written).
+// CUT: the chunks are cut by nonzeros (else mean_rows rows each), so a row's is searched for, from LDS: the rows of neighbouring
+// nonzeros are anywhere, and a lane that reads a line of its own from the L1 waits for the 63 others.
+constexpr int kPackAhead = 4;
+template <bool CUT>
 __global__ __launch_bounds__(kBlock) void column_order_pack_kernel(idx_t nnz, idx_t base, uint32_t band_shift, uint32_t band_keys,
                                                                    idx_t m, uint32_t mean_rows, uint32_t chunks, uint32_t sub,
                                                                    const uint32_t* __restrict__ chunk_first,
                                                                    const idx_t* r_keys, const idx_t* c_keys,
                                                                    idx_t* ids_out, idx_t* packed_out) {
-    const uint64_t k = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x;
-    if (k >= nnz) return;
-    const idx_t key = c_keys[k];
-    const idx_t row = min(r_keys[k] - base, m - 1);
-    uint32_t chunk = min(row / mean_rows, chunks - 1);  // unless the chunks are cut by nonzeros
-    uint32_t chunk_row = chunk_first[chunk];
-    if (row < chunk_row || (chunk + 1 < chunks && row >= chunk_first[chunk + 1])) {
-        uint32_t end = chunks;  // the last chunk that begins at or before the row
-        chunk = 0;
-        while (end - chunk > 1) {
-            const uint32_t mid = (chunk + end) / 2;
-            if (chunk_first[mid] <= row) chunk = mid; else end = mid;
-        }
-        chunk_row = chunk_first[chunk];
+    __shared__ uint32_t s_first[CUT ? kCutChunks : 1];
+    if constexpr (CUT) {
+        for (uint32_t i = threadIdx.x; i < chunks; i += kBlock) s_first[i] = chunk_first[i];
+        __syncthreads();
     }
-    const uint32_t band = key / band_keys;
-    const uint32_t group = band / sub;
-    ids_out[k] = (group * chunks + chunk) * sub + (band - group * sub);
-    packed_out[k] = ((row - chunk_row) << band_shift) | (key - band * band_keys);
+    const uint64_t k0 = static_cast<uint64_t>(blockIdx.x) * (kBlock * kPackAhead) + threadIdx.x;
+    idx_t keys[kPackAhead], rows[kPackAhead];
+#pragma unroll
+    for (int u = 0; u < kPackAhead; ++u) {
+        const uint64_t k = min(k0 + u * kBlock, static_cast<uint64_t>(nnz) - 1);  // nnz != 0 here
+        keys[u] = c_keys[k];
+        rows[u] = r_keys[k];
+    }
+#pragma unroll
+    for (int u = 0; u < kPackAhead; ++u) {
+        const uint64_t k = k0 + u * kBlock;
+        if (k >= nnz) return;
+        const idx_t key = keys[u];
+        const idx_t row = min(rows[u] - base, m - 1);
+        uint32_t chunk, chunk_row;
+        if constexpr (CUT) {
+            uint32_t end = chunks;  // the last chunk that begins at or before the row
+            chunk = 0;
+            while (end - chunk > 1) {
+                const uint32_t mid = (chunk + end) / 2;
+                if (s_first[mid] <= row) chunk = mid; else end = mid;
+            }
+            chunk_row = s_first[chunk];
+        } else {
+            chunk = min(row / mean_rows, chunks - 1);
+            chunk_row = chunk * mean_rows;
+        }
+        const uint32_t band = key / band_keys;
+        const uint32_t group = band / sub;
+        ids_out[k] = (group * chunks + chunk) * sub + (band - group * sub);
+        packed_out[k] = ((row - chunk_row) << band_shift) | (key - band * band_keys);
+    }
 }
 
 // One workgroup per compute unit: workgroup i belongs to XCD i % 8 and takes every 32nd unit (the tiles
@@ -1162,9 +1184,12 @@ void launch_column_order_build(hipStream_t stream, const BandedShape& s, idx_t m
     idx_t* ids = reinterpret_cast<idx_t*>(w + l.src_cols);
     idx_t* packed = reinterpret_cast<idx_t*>(w + l.src_rows);
     uint32_t* chunk_first = reinterpret_cast<uint32_t*>(w + l.chunk_first);
-    hipLaunchKernelGGL(column_order_cut_kernel, dim3(1), dim3(kCutBlock), 0, stream, m, nnz, base, row_ptr, s.chunks, s.mean_rows,
-                       s.rows_per_tile, chunk_first);
-    hipLaunchKernelGGL(column_order_pack_kernel, dim3((nnz + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, nnz, base,
+    const bool cut = row_ptr != nullptr && s.mean_rows != s.rows_per_tile;  // by nonzeros
+    hipLaunchKernelGGL(column_order_cut_kernel, dim3(1), dim3(kCutBlock), 0, stream, m, nnz, base, cut ? row_ptr : nullptr, s.chunks,
+                       s.mean_rows, s.rows_per_tile, chunk_first);
+    constexpr uint64_t kPacked = static_cast<uint64_t>(kBlock) * kPackAhead;
+    auto* pack = cut ? column_order_pack_kernel<true> : column_order_pack_kernel<false>;
+    hipLaunchKernelGGL(pack, dim3(static_cast<uint32_t>((nnz + kPacked - 1) / kPacked)), dim3(kBlock), 0, stream, nnz, base,
                        s.band_shift, s.band_keys, m, s.mean_rows, s.chunks, s.sub, chunk_first, r_keys, c_keys, ids, packed);
     idx_t* sorted_ids = reinterpret_cast<idx_t*>(w + l.tile_ids);
     launch_sort_triples(stream, nnz, bit_length(s.tiles - 1), ids, packed, vals, sorted_ids,
