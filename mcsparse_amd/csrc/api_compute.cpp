@@ -1064,7 +1064,7 @@ mcsparseStatus_t mcsparseSpMV_preprocess(mcsparseHandle_t handle, mcsparseOperat
                 while (all_of_x < (static_cast<size_t>(gathered) + base) * vb) all_of_x *= 2;
                 BandedShape wide;
                 if (mcsp::column_order_shape(m, gathered, nnz, base, vb, all_of_x, true, &wide) &&
-                    mcsp::column_order_halved_rows(m, 1) == mcsp::column_order_halved_rows(m, shape.bands) &&
+                    mcsp::wide_group_wins(wide, shape, vb) &&
                     align_up(mcsp::banded_layout(wide, m, nnz, vb).total) <= room)
                     shape = wide;
             }

@@ -120,6 +120,7 @@ struct BandedShape {
     uint32_t bands;
     uint32_t rows_per_tile;  // by_column: at most; mean_rows on average
     uint32_t mean_rows;
+    float even_time;         // by_column: what its tiles are estimated to take (even_tiles); 0: not cut evenly
     uint32_t chunks;         // row chunks = tiles per band
     uint32_t tiles;
     // false: entries of a tile in CSR order, row sums formed in a fixed order (bit-reproducible);
@@ -325,7 +326,6 @@ constexpr uint32_t kColumnOrderMinRows = 2048;
 constexpr uint32_t kColumnOrderMinEvenRows = 512;
 bool column_order_shape(idx_t m, idx_t n, idx_t nnz, idx_t base, size_t value_bytes, size_t band_bytes, bool even,
                         BandedShape* out);
-uint32_t column_order_halved_rows(idx_t m, uint64_t groups);
 // How the gathers of an SpMV are spread over the 128-byte lines of x: launch_line_gathers fills, at the head of
 // `workspace` (line_gathers_workspace_bytes), kLineGatherBins pairs (lines, gathers) binned by the highest bit of a
 // line's count: of_rows from the row lengths (the gathered element is the row: a transposing direction), else from
@@ -336,6 +336,8 @@ size_t line_gathers_workspace_bytes(idx_t gathered, size_t value_bytes);
 void launch_line_gathers(hipStream_t stream, bool of_rows, idx_t gathered, idx_t nnz, idx_t base, const idx_t* ptr,
                          const idx_t* ind, size_t value_bytes, void* workspace);
 bool gathers_favour_wide_groups(const unsigned long long* bins);
+// Whether it does on this matrix: from the copies that would be built, with one group (wide) and with several.
+bool wide_group_wins(const BandedShape& wide, const BandedShape& several, size_t value_bytes);
 // r_keys / c_keys: row + base and column + base of every nonzero of the matrix to copy, in an order
 // sorted by the 128-byte line of x the column lies in (any order inside a line); vals in the same
 // order.  Neither is written.

@@ -1055,9 +1055,20 @@ bool gathers_favour_wide_groups(const unsigned long long* bins) {
     return 2.0 * gathers > static_cast<double>(all);
 }
 
+// The tiles of one group are the shorter ones, so it has to save more than they cost: a plane of sums less for every group of
+// several, of twice the bytes in fp64, and the gathers of hot lines that every group repeats.  wide / several by the estimate of
+// even_tiles, and us a call with several and with one, transposing power-law products: fp32 1.35 (6 M rows, 1.5 M columns) 285 and
+// 300, 1.36 (4 M, 1.4 M) 197 and 207, 1.26 (2 M square) 120 and 117, 1.20 (1.4 M) 90 and 82, 1.16 (2.5 M) 157 and 146, 1.0 (0.7 M
+// rows, 3 M columns) 55 and 41; 1.55 (1.2 M) 60 and 65; fp64 1.78 (1 M) level, 1.47 (1.2 M) 107 and 101, 1.42 (1.4 M) 144 and 130,
+// 1.26 (2 M) 209 and 190, 1.0 (4.1 M) 545 and 390.  Where the tiles are short either way the estimate says little: 300 K to 500 K
+// square, fp64, 1.6 to 1.7: 27.5 and 25.5, 42 and 40.
+bool wide_group_wins(const BandedShape& wide, const BandedShape& several, size_t value_bytes) {
+    constexpr uint32_t kShortRows = 4096;
+    return several.mean_rows < kShortRows || wide.even_time < (value_bytes == 8 ? 1.45f : 1.3f) * several.even_time;
+}
+
 namespace {
 constexpr uint64_t kUnitsWanted = kXcds * kColumnGroupsPerXcd;
-}  // namespace
 
 uint32_t column_order_halved_rows(idx_t m, uint64_t groups) {
     uint32_t rows = kColumnOrderRows;
@@ -1065,11 +1076,11 @@ uint32_t column_order_halved_rows(idx_t m, uint64_t groups) {
     return rows;
 }
 
-namespace {
 constexpr idx_t kShortTilesLeastNonzeros = 1u << 21;
 struct EvenTiles {
     uint64_t groups, turns;
     uint32_t rows;
+    double time;
 };
 // The tiles whose units every compute unit gets equally many of (`turns`), for the number of band groups with which that is
 // estimated to take the shortest.  A unit takes what its nonzeros take, and as much as a quarter more where its tile is half
@@ -1079,18 +1090,14 @@ struct EvenTiles {
 // 41 -> 27, 637 K 41 -> 29, fp64 451 K 53 -> 40, 843 K 92 -> 64, 1.4 M 127 -> 115 (of 843 K rows' 92, 80 with tiles of equally
 // many rows, 74 cut by nonzeros, 65 with groups of one width).
 EvenTiles even_tiles(idx_t m, uint64_t groups, uint64_t least_groups) {
-    EvenTiles best = {0, 0, 0};
-    double best_time = 0;
+    EvenTiles best = {0, 0, 0, 0};
     for (uint64_t g = groups; g >= least_groups && g != 0; --g) {
         uint64_t turns = 1;
         while (turns * kUnitsWanted / g * kColumnOrderRows < m) ++turns;
         const uint64_t chunks = turns * kUnitsWanted / g;
         const uint32_t rows = static_cast<uint32_t>((static_cast<uint64_t>(m) + chunks - 1) / chunks);
         const double time = static_cast<double>(turns) * rows / static_cast<double>(g) * (0.75 + 0.25 * kColumnOrderRows / rows);
-        if (best.rows == 0 || time < 0.98 * best_time) {
-            best = {g, turns, rows};
-            best_time = time;
-        }
+        if (best.rows == 0 || time < 0.98 * best.time) best = {g, turns, rows, time};
     }
     return best;
 }
@@ -1107,6 +1114,7 @@ bool column_order_shape(idx_t m, idx_t n, idx_t nnz, idx_t base, size_t value_by
     // The taller a tile, the more of its entries share a line of x; but the kernel runs one workgroup per compute unit, so
     // there must be a unit of work for each, and a matrix too small for that is left to the other kernels.
     uint32_t rows_per_tile = column_order_halved_rows(m, groups), mean_rows = rows_per_tile;
+    out->even_time = 0;
     if (even) {
         const uint64_t least_groups = groups >= 3 ? (4 * (max_key + 1) + (5ull << wanted) - 1) / (5ull << wanted) : groups;
         const EvenTiles best = even_tiles(m, groups, std::min(least_groups, groups));
@@ -1117,6 +1125,7 @@ bool column_order_shape(idx_t m, idx_t n, idx_t nnz, idx_t base, size_t value_by
         if (best.rows < kColumnOrderMinEvenRows || (short_tiles && (nnz < kShortTilesLeastNonzeros || nnz / 8 < m))) return false;
         groups = best.groups;
         mean_rows = best.rows;
+        out->even_time = static_cast<float>(best.time);
         rows_per_tile = best.turns == 1 ? std::min(2 * mean_rows, kColumnOrderRows) : mean_rows;
     }
     const uint64_t chunks = (static_cast<uint64_t>(m) + mean_rows - 1) / mean_rows;

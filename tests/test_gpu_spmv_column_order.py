@@ -501,3 +501,22 @@ def test_bands_have_the_width_the_caller_sets(torch_gpu, handle, oracle):
     assert api.spmv(*args, buf) == api.STATUS_SUCCESS
     torch.cuda.synchronize()
     assert (d_y.cpu().numpy() == 2.0 ** 24).all()
+
+
+@pytest.mark.parametrize("dtype,m,n,groups", [
+    (np.float32, 1_500_001, 1_500_001, 1),
+    (np.float32, 1_200_001, 1_200_001, 3),   # the tiles of one group would be too short for what it saves
+    (np.float64, 1_400_003, 1_400_003, 1),
+    (np.float64, 1_000_003, 1_000_003, 4),
+    (np.float64, 400_001, 1_500_003, 1),     # tall either way, and a plane of sums for each of several groups
+])
+def test_one_group_where_it_saves_more_than_its_tiles_cost(torch_gpu, handle, oracle, dtype, m, n, groups):
+    """Transposing products whose gathers go to a few rows' lines of x for the most part."""
+    rng = np.random.default_rng(3)
+    lens = np.zeros(m, np.int64)
+    lens[rng.choice(m, 60, replace=False)] = 20000
+    lens[1::4] += 1
+    a = wl.Csr(m, n, np.concatenate([[0], np.cumsum(lens)]), rng.integers(0, n, lens.sum()),
+               rng.integers(-8, 9, lens.sum()).astype(dtype))
+    state, bands, *_ = run(torch_gpu, handle, oracle, a, 2.0, -1.0, op=api.OP_T)
+    assert (state, bands) == (3, groups)
