@@ -317,10 +317,11 @@ struct BandedLayout {
     size_t chunk_first;  // by_column: first row of every chunk
 };
 // The same decision for the copy whose tiles are in column order (BandedShape::by_column): tiles of up to kColumnOrderRows
-// rows, at most 64 planes of partial sums and 65536 tiles, and at least one unit of work per compute unit.
-// even: the tiles are cut as tall as give every compute unit the same number of units, all of a matrix's rows to be had in so
-// many turns.  Else kColumnOrderRows is halved until there is a unit for each, down to kColumnOrderMinRows, and the
-// compute units may be left with a turn in which most have no unit.
+// rows, at most 64 planes of partial sums and 65536 tiles.
+// even: the tiles are cut as tall as give the compute units equally many units, all of a matrix's rows to be had in so many
+// turns (where the groups do not divide the units, a few compute units have one less).  Else kColumnOrderRows is halved until
+// there is a unit for each, down to kColumnOrderMinRows, a matrix too small for that has no such copy, and the compute units may
+// be left with a turn in which most have no unit.
 constexpr uint32_t kColumnOrderRows = 16384;
 constexpr uint32_t kColumnOrderMinRows = 2048;
 constexpr uint32_t kColumnOrderMinEvenRows = 512;

@@ -774,7 +774,9 @@ struct BucketLds {
 constexpr uint32_t kShortRun = 64, kUsualRun = 20;
 
 // place + how many of the four words are below the bound.  (The compiler waits for every comparison by itself and sends half
-// of them through a register.)
+// of them through a register.)  An SGPR that a vector instruction has written may be read by another one, as its carry, two
+// instructions later at the earliest: nobody else looks after that inside the block, so three stand between a comparison and its
+// add, and no fewer than two may.
 __device__ __forceinline__ uint32_t add_smaller(uint32_t place, u32x4 words, uint32_t bound) {
     uint64_t a, b, c, d;
     asm("v_cmp_lt_u32_e64 %1, %5, %9\n\t"

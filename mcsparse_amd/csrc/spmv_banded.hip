@@ -406,8 +406,8 @@ __global__ __launch_bounds__(kBlock) void column_order_pack_kernel(idx_t nnz, id
     }
 }
 
-// One workgroup per compute unit: workgroup i belongs to XCD i % 8 and takes every 32nd unit (the tiles
-// of one row chunk in one band group) of that XCD's stretch.  The row sums of a unit live in LDS as
+// One workgroup per compute unit: workgroup i belongs to XCD i % 8 and takes units (the tiles of one row chunk in one band
+// group) of that XCD's stretch, its first by its own number and the next ones off a counter.  The row sums of a unit live in LDS as
 // doubles (fp32 products are widened: ds_add_f32 runs at a quarter of the rate of ds_add_f64 on this
 // chip).  A thread keeps two sets of entries in registers, kColumnSet32 or kColumnSet64 each: what fits the 128
 // registers a thread of a 1024-thread workgroup can have (fp64, one entry per load, 8 / 10 / 12 / 13: 75.0 / 73.7 /
@@ -1086,7 +1086,7 @@ struct EvenTiles {
 // estimated to take the shortest.  A unit takes what its nonzeros take, and as much as a quarter more where its tile is half
 // as tall.  Against tiles halved from 16384 rows until there is a unit for each, in bands of 2 MB and a last one of what is
 // left, microseconds a call, the trial's way before that where it refused: uniform rows, fp64 604 K x 17 69 -> 48, 788 K x 38
-// 134 -> 92, 2.6 M x 33 368 -> 337, 1.4 M x 22 133 -> 135; fp32 903 K x 7 43 -> 31; power-law rows, fp32 271 K 33 -> 15, 553 K
+// 134 -> 92, 2.6 M x 33 368 -> 334, 1.43 M x 22 128 -> 132 (x 10 97 -> 92); fp32 903 K x 7 43 -> 31; power-law rows, fp32 271 K 33 -> 15, 553 K
 // 41 -> 27, 637 K 41 -> 29, fp64 451 K 53 -> 40, 843 K 92 -> 64, 1.4 M 127 -> 115 (of 843 K rows' 92, 80 with tiles of equally
 // many rows, 74 cut by nonzeros, 65 with groups of one width).
 EvenTiles even_tiles(idx_t m, uint64_t groups, uint64_t least_groups) {
