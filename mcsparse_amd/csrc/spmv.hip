@@ -622,31 +622,36 @@ void launch_spmv_vector(hipStream_t stream, const SpmvArgs& a, T alpha, T beta, 
     // 22.5 below).  Rows of very different length keep most of these lanes waiting for the longest one's: a call that knows
     // nothing of its rows takes the kernel below (a million power-law rows, at most 1000 long, mean 6, through csrmv: fp32 125 us
     // below, 173 here; fp64 160 and 211; 200,000 rows of 12 and a hundred of 3000, fp64, 148 and 187).
-    // Workgroups of two wavefronts for the shortest rows, below a million of them: with four, a few hundred thousand rows are
+    // Workgroups of two wavefronts for the shortest fp64 rows, below a million of them: with four, a few hundred thousand rows are
     // four to six workgroups to a compute unit, and where some have one more than the others the call waits for those (random
-    // columns, fp64, four and two: 270,000 rows of 5 14.8 and 14.0 us, below 14.2; 350,000 17.8 and 16.8, below 17.4; 171,500
-    // rows of 7 12.3 and 12.0, below 11.9; five-point stencil of 1900 x 1900 55.5 and 57.0).  With 64 rows of 7 to a wavefront
-    // four stay (stencil of 110^3, fp64, 26.8 and 27.6), but in fp64 that is from 700,000 rows on: 500,000 random rows of 7
-    // 31.7 us, with 32 rows 29.7, below 30.9.
+    // columns, four and two: 240,000 rows of 5 10.6 and 10.0 us, 280,000 12.7 and 11.8, 320,000 13.4 and 13.5, below 10.9, 12.8 and
+    // 14.5; 200,000 rows of 6 9.8 and 9.6; five-point stencil of 1900 x 1900 55.5 and 57.0).  fp32 has lost nothing to the kernel
+    // below and loses with two (320,000 rows of 5 9.6 and 10.2, 440,000 of 3 8.4 and 8.9, 480,000 of 6 16.2 and 16.9).  Rows of
+    // 7: two below 250,000 (200,000 11.2 and 10.8, fp32 9.4 and 9.2; 300,000 16.6 and 17.0, fp32 13.5 and 13.7).  With 64 of them to
+    // a wavefront four stay (stencil of 110^3, fp64, 26.8 and 27.6), but in fp64 that is from 700,000 rows on: 520,000 random rows
+    // 30.7 us, with 32 rows 29.3, below 30.5.
     const uint64_t mean = (static_cast<uint64_t>(a.nnz) + a.m - 1) / a.m;
     if (stretches && mean < static_cast<uint64_t>(lanes) && lanes <= 16 && a.m >= 150000 &&
         a.nnz >= 1200000) {
+        constexpr bool kDouble = sizeof(T) == 8;
+        constexpr int kFewRows = kDouble ? 128 : 256;  // threads of a workgroup below a million rows
         const bool many = a.m >= 1000000;
         switch (mean) {
             case 3:
                 if (many) launch_short_rows<T, 64, 3, 256>(stream, a, alpha, beta);
-                else launch_short_rows<T, 64, 3, 128>(stream, a, alpha, beta);
+                else launch_short_rows<T, 64, 3, kFewRows>(stream, a, alpha, beta);
                 return;
             case 5:
                 if (many) launch_short_rows<T, 64, 5, 256>(stream, a, alpha, beta);
-                else launch_short_rows<T, 64, 5, 128>(stream, a, alpha, beta);
+                else launch_short_rows<T, 64, 5, kFewRows>(stream, a, alpha, beta);
                 return;
             case 6:
                 if (a.m >= 500000) launch_short_rows<T, 64, 6, 256>(stream, a, alpha, beta);
-                else launch_short_rows<T, 32, 3, 128>(stream, a, alpha, beta);
+                else launch_short_rows<T, 32, 3, kFewRows>(stream, a, alpha, beta);
                 return;
             case 7:
-                if (a.m >= (sizeof(T) == 8 ? 700000 : 500000)) launch_short_rows<T, 64, 7, 256>(stream, a, alpha, beta);
+                if (a.m >= (kDouble ? 700000 : 500000)) launch_short_rows<T, 64, 7, 256>(stream, a, alpha, beta);
+                else if (a.m >= 250000) launch_short_rows<T, 32, 4, 256>(stream, a, alpha, beta);
                 else launch_short_rows<T, 32, 4, 128>(stream, a, alpha, beta);
                 return;
             case 9:

@@ -218,7 +218,7 @@ def test_a_few_long_rows_among_many_short_ones(torch_gpu, handle, oracle):
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("mean, m", [(3, 400_063), (5, 240_001), (6, 200_031), (6, 500_001), (7, 200_033), (7, 500_065),
                                      (9, 150_001), (12, 150_015), (14, 150_031), (15, 150_047),
-                                     (3, 1_000_033), (5, 1_000_001), (7, 700_001)])
+                                     (3, 1_000_033), (5, 1_000_001), (7, 700_001), (7, 250_033)])
 def test_short_rows_are_read_as_one_stretch(torch_gpu, handle, oracle, dtype, mean, m):
     """Rows of a few nonzeros, as many to a wavefront as it reads in one go: each mean length and number of rows that has
     a kernel of its own, with a last wavefront that is not full, long empty runs (also at both ends), rows that span
