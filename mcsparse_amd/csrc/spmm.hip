@@ -59,14 +59,31 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 8 : 1) void sp
 // rows, and most rows, of one or two nonzeros, are three dependent trips to memory by themselves.  Here a wavefront has
 // kTurnRows neighbouring rows: a group that is through with one takes the next, the long ones first, and the nonzeros of what a group
 // is at next, the next LR of its row or the first of another, are asked for behind the rows of op(B) of the present ones.
+//
+// A row of more than kTogether nonzeros is the whole wavefront's, its groups on neighbouring stretches of it: walked by one group,
+// four or eight rows of op(B) at a time, the longest of them outlast the launch.  Power-law rows, microseconds a call before and
+// so: 16 fp32 columns, 100 K rows 69 and 49, 400 K 142 and 123, a million 313 and 293, 2.5 M 863 and 839; 12 fp64 columns, 100 K
+// 65 and 57, a million 427 and 415 (150 K rows, 16 fp32 columns, with limits of 4, 8 and 16 times LR 55, 53 and 54).  Eight lanes
+// of fp32 get there faster, and the code beside the loop costs them more than it gives (32 columns, 100 K rows 69 and 67, 200 K
+// 91 and 92, a million 348 and 351, 2.5 M 1006 and 1019); with sixteen lanes the limit is the least length of a row taken apart.
 constexpr int kTurnRows = kWave;
-template <typename T, int LR, int V, bool RAGGED>
+template <int LR>
+constexpr idx_t kTogether = 16 * LR;
+template <typename T, int LR>
+constexpr bool kTakenTogether = LR == 4 || (LR == 8 && sizeof(T) == 8);
+static_assert(kTogether<8> < kSpmmLongCutLeast, "rows that are not taken apart");
+// BESIDE: another kernel has taken the rows of up to kTogether<LR>, and all of them unless *apart says that there are long rows.
+template <typename T, int LR, int V, bool RAGGED, bool BESIDE>
 __global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 7 : 1) void spmm_rowb_turns_kernel(idx_t m, idx_t n, idx_t nnz, idx_t base,
                                                                  const idx_t* __restrict__ row_ptr,
                                                                  const idx_t* __restrict__ col, const T* __restrict__ val,
                                                                  const T* __restrict__ B, int64_t ldb, T* __restrict__ C,
                                                                  int64_t ldc, bool c_row_major, T alpha, T beta,
-                                                                 idx_t long_row, const BoundsWork cut) {
+                                                                 idx_t long_row, const uint32_t* __restrict__ apart,
+                                                                 const BoundsWork cut) {
+    if constexpr (BESIDE) {
+        if (*apart == 0) return;  // all workgroups
+    }
     if (blockIdx.x < cut.blocks) {  // whole workgroup
         cut_pieces(cut, base, nnz, row_ptr, col);
         return;
@@ -82,7 +99,24 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 7 : 1) void sp
     const uint32_t my_row = static_cast<uint32_t>(min(row0 + wave_lane, static_cast<uint64_t>(m) - 1));
     const idx_t my_start = row_ptr[my_row] - base, my_end = row_ptr[my_row + 1] - base;
     const uint32_t length = my_end - my_start;
-    const bool live = row0 + wave_lane < m && length <= long_row;
+    const bool mine = row0 + wave_lane < m && length <= long_row, live = mine && (!kTakenTogether<T, LR> || length <= kTogether<LR>);
+    if constexpr (kTakenTogether<T, LR>) {
+        for (unsigned long long together = __ballot(mine && length > kTogether<LR>); together != 0; together &= together - 1) {  // whole wavefront
+            const uint32_t r = __builtin_ctzll(together);
+            const idx_t begin = __builtin_amdgcn_readlane(my_start, r), end = __builtin_amdgcn_readlane(my_end, r);
+            T acc[V];
+#pragma unroll
+            for (int i = 0; i < V; ++i) acc[i] = T(0);
+            row_times_b<T, LR, V, false, true>(begin + group * LR, end, lane, base, col, val, B_bytes, lane_off, ldb_bytes, acc, kWave);
+#pragma unroll
+            for (int i = 0; i < V; ++i) {
+#pragma unroll
+                for (int off = LR; off < kWave; off <<= 1) acc[i] += __shfl_xor(acc[i], off, kWave);
+            }
+            if (group == 0 && own.any) store_c<T, V>(C, ldc, c_row_major, row0 + r, own.first, acc, alpha, beta, own.skip);
+        }
+        if constexpr (BESIDE) return;
+    }
     const unsigned long long first = __ballot(live && length > 4 * LR), second = __ballot(live && length <= 4 * LR);
     auto below = [&](unsigned long long mask) {
         return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u));
@@ -845,8 +879,8 @@ void launch_group(hipStream_t stream, const SpmmArgs& a, const uint32_t* group_p
 // lanes to a row 88 fp32 columns 636, 677, 35 fp64 columns 1529, 1444, 66 columns 325, 369.  Where a row fits a lane or two
 // spmm_narrow_kernel reads ahead by itself.
 template <typename T, int LR>
-bool takes_rows_in_turns(const SpmmArgs& a) {
-    return LR <= 16 && a.long_row != 0 && a.long_known && narrow_offsets(a, sizeof(T));
+bool takes_rows_in_turns(const SpmmArgs& a, bool known) {
+    return LR <= 16 && a.long_row != 0 && a.long_known == known && narrow_offsets(a, sizeof(T));
 }
 
 template <typename T, int LR, int V>
@@ -861,28 +895,36 @@ void launch_rowb(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     const T* val = static_cast<const T*>(a.val);
     const T* B = static_cast<const T*>(a.B);
     T* C = static_cast<T*>(a.C);
+    // A call that does not know whether there are long rows leaves those that the kernel for turns gives to whole wavefronts to it,
+    // so that a row's sum is the same by every way to the product.
+    const bool in_turns = takes_rows_in_turns<T, LR>(a, true), beside = kTakenTogether<T, LR> && takes_rows_in_turns<T, LR>(a, false);
     auto launch = [&](auto wide, auto ragged) {
         hipLaunchKernelGGL((spmm_rowb_kernel<T, LR, V, decltype(wide)::value, decltype(ragged)::value>), grid, dim3(kBlock), 0,
                            stream, a.m, a.n, a.base, a.row_ptr, a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta,
-                           a.long_row, a.long_apart, chunk, xcds);
+                           beside ? kTogether<LR> : a.long_row, a.long_apart, chunk, xcds);
     };
     auto launch_offsets = [&](auto ragged) {
         if (narrow_offsets(a, sizeof(T))) launch(std::false_type{}, ragged);
         else launch(std::true_type{}, ragged);
     };
     if constexpr (LR <= 16) {
-        if (takes_rows_in_turns<T, LR>(a)) {
+        if (in_turns || beside) {
             constexpr uint32_t kRowsPerBlock = kBlock / kWave * kTurnRows;
-            const BoundsWork cut = spmm_long_bounds(a, sizeof(T));
+            const BoundsWork none = {0, {nullptr, 0, 0, 0, 0}, nullptr, nullptr, 0};
+            const BoundsWork cut = in_turns ? spmm_long_bounds(a, sizeof(T)) : none;
             const dim3 turns_grid(cut.blocks + (a.m + kRowsPerBlock - 1) / kRowsPerBlock, static_cast<uint32_t>(panels));
-            auto turns = [&](auto ragged) {
-                hipLaunchKernelGGL((spmm_rowb_turns_kernel<T, LR, V, decltype(ragged)::value>), turns_grid, dim3(kBlock), 0, stream,
-                                   a.m, a.n, a.nnz, a.base, a.row_ptr, a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta,
-                                   a.long_row, cut);
+            auto turns = [&](auto ragged, auto other) {
+                hipLaunchKernelGGL((spmm_rowb_turns_kernel<T, LR, V, decltype(ragged)::value, decltype(other)::value>), turns_grid,
+                                   dim3(kBlock), 0, stream, a.m, a.n, a.nnz, a.base, a.row_ptr, a.col, val, B, a.ldb, C, a.ldc,
+                                   a.c_row_major, alpha, beta, a.long_row, a.long_apart, cut);
             };
-            if (a.n % V != 0) turns(std::true_type{});
-            else turns(std::false_type{});
-            return;
+            auto turns_of = [&](auto other) {
+                if (a.n % V != 0) turns(std::true_type{}, other);
+                else turns(std::false_type{}, other);
+            };
+            if (in_turns) turns_of(std::false_type{});
+            else if constexpr (kTakenTogether<T, LR>) turns_of(std::true_type{});
+            if (in_turns) return;
         }
     }
     if constexpr (V > 1) {

@@ -313,3 +313,29 @@ def test_pieces_cut_beside_the_row_kernel(torch_gpu, handle, oracle, dtype, n):
     a = rows_of_lengths(lengths, 400009, dtype, seed=2)
     assert a.nnz >= 1 << 20 and a.n * n * np.dtype(dtype).itemsize >= 10 << 20
     check(torch_gpu, handle, oracle, a, n, 1.25, -0.5)
+
+
+@pytest.mark.parametrize("dtype,n", [(np.float32, 9), (np.float32, 16), (np.float64, 8), (np.float64, 9), (np.float64, 15), (np.float64, 16)])
+def test_rows_taken_by_a_whole_wavefront(torch_gpu, handle, oracle, dtype, n):
+    """Lengths around the limit above which a row that is not taken apart is a wavefront's (64 with four lanes to a row, 128 with
+    eight): alone among short rows, all 64 of a wavefront, the last row; by a call that knows of the long row and by one that
+    does not (COO), to the same bits."""
+    edge = [63, 64, 65, 127, 128, 129, 191, 255, 256]
+    lengths = [1] * 70 + edge + [0, 2] * 40 + edge * 8 + [3] * 5 + [1025, 129]
+    a = rows_of_lengths(lengths, 3001, dtype, seed=n)
+    check(torch_gpu, handle, oracle, a, n, 1.25, 0.0, pad_b=1)
+    check(torch_gpu, handle, oracle, a, n, 0.5, -1.5, seed=1, c_order=api.ORDER_COL)
+    torch = torch_gpu
+    B = dev(torch, np.random.default_rng(2).uniform(-1, 1, (a.n, n)).astype(dtype))
+    ptr, col, val = dev(torch, a.ptr), dev(torch, a.col), dev(torch, a.val)
+    rows = dev(torch, np.repeat(np.arange(a.m, dtype=np.int32), np.diff(a.ptr)))
+    products = []
+    for mat in (api.SpMat(a.m, a.n, a.nnz, ptr, col, val), api.SpMat(a.m, a.n, a.nnz, rows, col, val, fmt=api.FORMAT_COO)):
+        C = torch.zeros((a.m, n), dtype=B.dtype, device="cuda")
+        call = (handle, api.OP_N, api.OP_N, 1.0, mat, api.DnMat(a.n, n, n, B), 0.0, api.DnMat(a.m, n, n, C), api.maca_type(np.dtype(dtype)))
+        st, size = api.spmm_buffer_size(*call)
+        assert st == 0
+        assert api.spmm(*call, torch.empty(size, dtype=torch.uint8, device="cuda")) == 0
+        torch.cuda.synchronize()
+        products.append(C.cpu().numpy())
+    assert np.array_equal(products[0], products[1])
