@@ -1011,7 +1011,9 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 || (MANY && !packed_entries
 // Before, a workgroup looked for work among all buckets with two device-wide fences a chunk, one workgroup placed all
 // chunks of a bucket, the counting phase read whole entries, and entries were written from where they lay in registers:
 // csr2csc of 67 M nonzeros with columns by Zipf's law (53 M of them in such buckets) 3690 us, now 1458 (LSD passes: 1484);
-// an index sort of 10 M triples with rows by that law 1870 us, now 953.
+// an index sort of 10 M triples with rows by that law 1870 us, then 953.  Since then: a workgroup looks a chunk's bucket up only
+// where it is another one than before, waits for the end of a phase with fewer looks at the counter (848 -> 833 us; 512 of them
+// looking hold the workgroups up that add to it), and pairs of keys that share a word stay one to the last pass (833 -> 748).
 // Index sorts by a skewed major key stay slower than the LSD passes: 503 us for those, 936 against 1609 for 21.8 M triples
 // in a million power-law rows of up to 50,000 (38 % of them in such buckets), 156 against 188 in a hundred thousand rows.
 // A pass over such a bucket costs two phases of 45 us at least, and there are four or five of them.  How the keys are
@@ -1022,18 +1024,19 @@ constexpr uint32_t kOversizeGrid = 512;
 struct OversizeChunk {
     uint32_t listed_at, bucket, first, entries;  // first: place of the bucket's first entry in the output
     uint32_t chunk, chunks, slot;                // slot: the bucket's first group
+    uint32_t before;                             // chunks of the buckets listed before
 };
 // For whole wavefronts; every lane returns the same.
 __device__ __forceinline__ OversizeChunk oversize_chunk(const SortTables& t, uint32_t listed, uint32_t number) {
     OversizeChunk c;
     c.listed_at = wave_count_up_to(t.oversize_first, listed, 0, number) - 1;
-    const uint32_t before = t.oversize_first[c.listed_at];
+    c.before = t.oversize_first[c.listed_at];
     c.bucket = t.oversize_bucket[c.listed_at];
     c.first = t.sub_first[c.bucket];
     c.entries = t.sub_first[c.bucket + 1] - c.first;
-    c.chunk = number - before;
+    c.chunk = number - c.before;
     c.chunks = (c.entries + kOversizeChunk - 1) / kOversizeChunk;
-    c.slot = oversize_slot(before, c.listed_at);
+    c.slot = oversize_slot(c.before, c.listed_at);
     return c;
 }
 
@@ -1094,6 +1097,7 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 ? 2 : 4) void oversize_kern
     typedef typename WordOf<VB>::type word_t;
     constexpr uint32_t kDigits = 1 << kPassBits;
     static_assert(kDigits <= kBucketThreads, "a thread per digit");
+    constexpr bool kWords = MANY && packed_entries<Key>();  // both keys in a word, as which they travel to the last pass
     const unsigned long long counted = t.oversize->listed;
     const uint32_t listed = static_cast<uint32_t>(counted), all_chunks = static_cast<uint32_t>(counted >> 32);
     if (blockIdx.x >= all_chunks) return;  // whole workgroup: more workgroups than chunks
@@ -1103,6 +1107,7 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 ? 2 : 4) void oversize_kern
     __shared__ uint32_t s_ticket, s_last;
     const uint32_t tid = threadIdx.x, wave = tid / kWave;
     const uint32_t phases = 2 * t.oversize_passes;
+    OversizeChunk c = {};
     for (uint32_t phase = 0; phase < phases; ++phase) {
         const uint32_t p = phase / 2;
         const uint32_t shift = p * t.oversize_width, bits = min(t.oversize_width, t.minor_bits + t.d3 - shift);
@@ -1110,7 +1115,7 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 ? 2 : 4) void oversize_kern
         // which of the two keys the pass looks at
         const bool by_aux = MANY && shift < t.minor_bits, by_key = !MANY || shift + bits > t.minor_bits;
         auto digit_of = [&](uint32_t of_key, uint32_t of_aux) {
-            if (!MANY) return of_key >> shift & mask;
+            if (!MANY || kWords) return of_key >> shift & mask;
             return static_cast<uint32_t>((static_cast<uint64_t>(of_key) << t.minor_bits | of_aux) >> shift) & mask;
         };
         // the first pass reads the runs, the others what the one before has left in the bucket's stretch
@@ -1119,8 +1124,8 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 ? 2 : 4) void oversize_kern
         const word_t* between_vals = static_cast<const word_t*>(t.oversize_vals[(p + 1) % 2]);
         if (tid == 0) {
             for (uint32_t idle = 0; phase != 0 && load_shared(&t.oversize->done[phase - 1]) < all_chunks; ++idle) {
-                // (hundreds of workgroups may be waiting: longer and longer, up to some 4 us)
-                for (uint32_t n = 0; n < (1u << min(idle, 2u)); ++n) __builtin_amdgcn_s_sleep(32);
+                // (hundreds of workgroups may be waiting: some 3 us, then 6)
+                for (uint32_t n = 0; n < (1u << min(idle, 1u)); ++n) __builtin_amdgcn_s_sleep(100);
             }
             s_ticket = take_chunk(t, phase);
         }
@@ -1133,7 +1138,9 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 ? 2 : 4) void oversize_kern
             const bool ahead = all_chunks - number > gridDim.x;
             uint32_t next = 0;
             if (tid == 0 && ahead) next = take_chunk(t, phase);
-            const OversizeChunk c = oversize_chunk(t, listed, number);
+            // (a chunk of the same bucket as the one before, as a rule where there are many: no search, five trips to memory)
+            if (number - c.before < c.chunks) c.chunk = number - c.before;
+            else c = oversize_chunk(t, listed, number);
             const uint32_t q0 = c.chunk * kOversizeChunk, count = min(c.entries - q0, kOversizeChunk);
             const uint32_t group = c.chunk / kOversizeGroup, in_group = c.chunk % kOversizeGroup;
             uint32_t* counts = t.oversize_counts + (static_cast<uint64_t>(number) << kPassBits);
@@ -1157,26 +1164,26 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 ? 2 : 4) void oversize_kern
             };
             if (phase % 2 == 0) {
                 if (tid < kDigits) s_count[tid] = 0;
-                uint32_t key[kBucketItems], aux[MANY ? kBucketItems : 1];
+                uint32_t key[kBucketItems], aux[MANY && !kWords ? kBucketItems : 1];
 #pragma unroll
                 for (int i = 0; i < kBucketItems; ++i) {
                     const uint32_t from = place_of(i);
                     key[i] = 0;
-                    if constexpr (packed_entries<Key>() && !MANY) key[i] = load_at<uint32_t>(keys_in, VB == 4 ? 2 * from : from);
-                    else if (packed_entries<Key>() && p == 0) key[i] = load_at<uint32_t>(keys_in, VB == 4 ? 2 * from : from);
-                    else if (by_key) key[i] = p == 0 ? load_at<Key>(keys_in, from) : load_shared_at<uint16_t>(between_keys, from);
-                    if constexpr (MANY) {
-                        aux[i] = 0;
-                        if (packed_entries<Key>() && p == 0) {
-                            aux[i] = key[i] & ((1u << t.minor_bits) - 1u);
-                            key[i] >>= t.minor_bits;
-                        } else if (by_aux) aux[i] = p == 0 ? load_at<uint32_t>(aux_in, from) : load_shared_at<uint32_t>(between_aux, from);
+                    if constexpr (packed_entries<Key>()) {
+                        key[i] = !MANY || p == 0 ? load_at<uint32_t>(keys_in, VB == 4 ? 2 * from : from)
+                                                 : load_shared_at<uint32_t>(between_aux, from);
+                    } else {
+                        if (by_key) key[i] = p == 0 ? load_at<Key>(keys_in, from) : load_shared_at<uint16_t>(between_keys, from);
+                        if constexpr (MANY) {
+                            aux[i] = 0;
+                            if (by_aux) aux[i] = p == 0 ? load_at<uint32_t>(aux_in, from) : load_shared_at<uint32_t>(between_aux, from);
+                        }
                     }
                 }
                 __syncthreads();
 #pragma unroll
                 for (int i = 0; i < kBucketItems; ++i) {
-                    if (in_slab(kBucketItems, i, count)) atomicAdd(&s_count[digit_of(key[i], MANY ? aux[MANY ? i : 0] : 0u)], 1u);
+                    if (in_slab(kBucketItems, i, count)) atomicAdd(&s_count[digit_of(key[i], MANY && !kWords ? aux[MANY && !kWords ? i : 0] : 0u)], 1u);
                 }
                 __syncthreads();
                 if (tid < kDigits) store_shared(counts + tid, s_count[tid]);
@@ -1206,27 +1213,33 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 ? 2 : 4) void oversize_kern
                     for (uint32_t k = 0; k < kOversizeGroup; ++k) sum += k < in_group ? n[k] : 0u;
                     s_sum[tid] = sum;
                 }
-                uint32_t key[kBucketItems], aux[kBucketItems];
+                uint32_t key[kBucketItems], aux[kWords ? 1 : kBucketItems];  // words: in key
                 word_t val[VB ? kBucketItems : 1];
 #pragma unroll
                 for (int i = 0; i < kBucketItems; ++i) {
                     const uint32_t from = place_of(i);
-                    if (packed_entries<Key>() && (!MANY || p == 0)) {
+                    if constexpr (kWords) {
+                        if (p == 0) {
+                            load_packed<VB>(keys_in, vals_in, from, key[i], val[VB ? i : 0]);
+                        } else {
+                            key[i] = load_shared_at<uint32_t>(between_aux, from);
+                            if constexpr (VB != 0) val[i] = load_shared_at<word_t>(between_vals, from);
+                        }
+                    } else if (packed_entries<Key>()) {
                         load_packed<VB>(keys_in, vals_in, from, key[i], val[VB ? i : 0]);
-                        aux[i] = MANY ? key[i] & ((1u << t.minor_bits) - 1u) : key[i] >> t.d3;
-                        if (MANY) key[i] >>= t.minor_bits;
+                        aux[kWords ? 0 : i] = key[i] >> t.d3;
                     } else if (!MANY || p == 0) {
                         key[i] = load_at<Key>(keys_in, from);
-                        aux[i] = load_at<uint32_t>(aux_in, from);
+                        aux[kWords ? 0 : i] = load_at<uint32_t>(aux_in, from);
                         if constexpr (VB != 0) val[i] = load_at<word_t>(vals_in, from);
                     } else {
                         key[i] = load_shared_at<uint16_t>(between_keys, from);
-                        aux[i] = load_shared_at<uint32_t>(between_aux, from);
+                        aux[kWords ? 0 : i] = load_shared_at<uint32_t>(between_aux, from);
                         if constexpr (VB != 0) val[i] = load_shared_at<word_t>(between_vals, from);
                     }
                 }
                 __syncthreads();
-                auto digit = [&](int i) { return digit_of(key[i], aux[i]); };
+                auto digit = [&](int i) { return digit_of(key[i], aux[kWords ? 0 : i]); };
                 uint32_t dest[kBucketItems / 2];
                 rank_entries<kBucketItems, kPassBits>(count, bits, s.cnt, dest, digit);
                 __syncthreads();
@@ -1261,7 +1274,12 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 ? 2 : 4) void oversize_kern
                         in_order(word_of, [&](int i, uint32_t, uint32_t w) { store_shared_at(between, put[i], finish(i, w)); });
                 };
                 auto as_it_is = [](int, uint32_t w) { return w; };
-                move([&](int i) { return aux[i]; }, t.oversize_aux[p % 2], out.aux, as_it_is);
+                if constexpr (kWords) {
+                    const uint32_t minor_mask = to_output ? (1u << t.minor_bits) - 1u : ~0u;
+                    move([&](int i) { return key[i]; }, t.oversize_aux[p % 2], out.aux, [&](int, uint32_t w) { return w & minor_mask; });
+                } else {
+                    move([&](int i) { return aux[i]; }, t.oversize_aux[p % 2], out.aux, as_it_is);
+                }
                 if constexpr (VB == 4) {
                     move([&](int i) { return val[i]; }, static_cast<uint32_t*>(t.oversize_vals[p % 2]),
                          static_cast<uint32_t*>(out.vals), as_it_is);
@@ -1271,7 +1289,13 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 ? 2 : 4) void oversize_kern
                     move([&](int i) { return static_cast<uint32_t>(val[i] >> 32); }, static_cast<uint64_t*>(t.oversize_vals[p % 2]),
                          static_cast<uint64_t*>(out.vals), [&](int i, uint32_t w) { return static_cast<uint64_t>(w) << 32 | low[i]; });
                 }
-                if constexpr (MANY) {
+                if constexpr (kWords) {
+                    if (to_output) {
+                        const uint32_t high = (c.bucket << t.d3) + out.key_bias;
+                        in_order([&](int i) { return key[i] >> t.minor_bits; },
+                                 [&](int i, uint32_t, uint32_t w) { store_at(out.keys, put[i], high + w); });
+                    }
+                } else if constexpr (MANY) {
                     if (!to_output) {
                         uint16_t* keys_to = t.oversize_keys[p % 2];
                         in_order([&](int i) { return key[i]; },

@@ -217,6 +217,31 @@ def test_coosort_runs_and_equal_pairs(torch_gpu, handle, longest, columns):
     assert np.array_equal(d_c.cpu().numpy(), cols[want])
 
 
+# buckets beyond what LDS holds: one chunk and an entry more, several of a bucket and of buckets in turn; the two keys in a word
+# (of 9 to 32 bits, in one to four passes) and apart
+@pytest.mark.parametrize("with_perm", [True, False])
+@pytest.mark.parametrize("columns", [1, 200, 70000, (1 << 22) - 2, 1 << 24])
+@pytest.mark.parametrize("popular", [[6145], [6144, 6145, 12289], [30000, 1, 100000]])
+def test_coosort_of_popular_rows(torch_gpu, handle, popular, columns, with_perm):
+    torch = torch_gpu
+    m, rest = 3001, 40000
+    gen = torch.Generator(device="cuda").manual_seed(columns)
+    rows = torch.randint(0, m, (rest,), generator=gen, dtype=torch.int32, device="cuda")
+    rows = torch.cat([rows] + [torch.full((c,), 17 + 900 * i, dtype=torch.int32, device="cuda") for i, c in enumerate(popular)])
+    rows = rows[torch.randperm(rows.numel(), generator=gen, device="cuda")]
+    cols = torch.randint(0, columns, (rows.numel(),), generator=gen, dtype=torch.int32, device="cuda")
+    order = torch.sort(rows.long() * columns + cols, stable=True).indices
+    perm = torch.arange(rows.numel(), dtype=torch.int32, device="cuda") if with_perm else None
+    got_rows, got_cols = rows.clone(), cols.clone()
+    st, size = api.sort_buffer_size(handle, "coo", m, columns, rows.numel(), rows, cols)
+    assert st == 0
+    buffer = torch.empty(size, dtype=torch.uint8, device="cuda")
+    assert api.xcoosort_by_row(handle, m, columns, rows.numel(), got_rows, got_cols, perm, buffer) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(got_rows, rows[order]) and torch.equal(got_cols, cols[order])
+    assert perm is None or torch.equal(perm.long(), order)
+
+
 @pytest.mark.parametrize("share", [0.3, 0.9])  # 0.9: one bucket with more tiles of the second step than the first has
 def test_a_row_with_most_of_ten_million_entries(torch_gpu, handle, share):
     """Many more pieces of one bucket than workgroups that work on it, in every pass: what one workgroup writes is read
