@@ -936,6 +936,27 @@ void launch_rowb(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     launch_offsets(std::false_type{});
 }
 
+// Rows of op(B) of more than 512 bytes, panel after panel: all rows for the first 512 bytes, ..., for what is left.  (A whole row to
+// 64 lanes: its columns are read once, but a wavefront has one row in flight instead of two, lanes past the last column idle, and
+// neighbouring rows of A find less of what they share in L2.  Fp64, 66, 96 and 128 columns: 48^3 159, 157, 159 us and 93, 94, 122
+// in panels; 97 x 61 x 97 954, 964, 991 and 533, 569, 748.)
+template <typename T, int V>
+void launch_panels(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
+    SpmmArgs panels = a, rest = a;
+    panels.n = a.n / (32 * V) * (32 * V);
+    launch_rowb<T, 32, V>(stream, panels, alpha, beta);
+    rest.n = a.n - panels.n;
+    if (rest.n == 0) return;
+    rest.B = static_cast<const T*>(a.B) + panels.n;
+    rest.C = static_cast<T*>(a.C) + static_cast<int64_t>(panels.n) * (a.c_row_major ? 1 : a.ldc);
+    // (not spmm_narrow_kernel, which adds a row up in another order)
+    if (rest.n < V) launch_rowb<T, 4, 1>(stream, rest, alpha, beta);
+    else if (rest.n <= 4 * V) launch_rowb<T, 4, V>(stream, rest, alpha, beta);
+    else if (rest.n <= 8 * V) launch_rowb<T, 8, V>(stream, rest, alpha, beta);
+    else if (rest.n <= 16 * V) launch_rowb<T, 16, V>(stream, rest, alpha, beta);
+    else launch_rowb<T, 32, V>(stream, rest, alpha, beta);
+}
+
 template <typename T, int V>
 void launch_rowb_v(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     const uint64_t lanes_needed = (static_cast<uint64_t>(a.n) + V - 1) / V;
@@ -945,7 +966,8 @@ void launch_rowb_v(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     else if (lanes_needed <= 8) launch_rowb<T, 8, V>(stream, a, alpha, beta);
     else if (lanes_needed <= 16) launch_rowb<T, 16, V>(stream, a, alpha, beta);
     else if (lanes_needed <= 32) launch_rowb<T, 32, V>(stream, a, alpha, beta);
-    else launch_rowb<T, 64, V>(stream, a, alpha, beta);
+    else if (V == 1 || a.long_row != 0) launch_rowb<T, 64, V>(stream, a, alpha, beta);
+    else launch_panels<T, V>(stream, a, alpha, beta);
 }
 
 

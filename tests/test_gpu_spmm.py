@@ -480,6 +480,17 @@ def test_strips_grid_with_broken_rows(torch_gpu, handle, oracle, dtype, n):
           prepare_for_row_major_c=True)
 
 
+@pytest.mark.parametrize("dtype,n", [(np.float32, 129), (np.float32, 133), (np.float32, 150), (np.float32, 190), (np.float32, 253),
+                                     (np.float32, 384), (np.float64, 65), (np.float64, 67), (np.float64, 75), (np.float64, 90),
+                                     (np.float64, 127), (np.float64, 192)])
+def test_rows_of_more_than_512_bytes_in_panels(torch_gpu, handle, oracle, dtype, n):
+    """No preprocess call: panels of 512 bytes, and what is left in every width a panel can have."""
+    a = wl.stencil_27pt(9, dtype=dtype)
+    for c_order in (api.ORDER_ROW, api.ORDER_COL):
+        check(torch_gpu, handle, oracle, a, n, 1.0, 0.0, c_order=c_order)
+        check(torch_gpu, handle, oracle, a.with_base(1), n, -0.5, 1.5, c_order=c_order, pad_b=1, pad_c=3)
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_strips_and_the_size_of_their_copy_in_lds(torch_gpu, handle, oracle, dtype):
     """A strip's values are copied into LDS when they are at most 128: a 27-point stencil in fp64 (4 rows x 27 values)
