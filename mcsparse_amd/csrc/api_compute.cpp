@@ -546,6 +546,37 @@ SpmmLayout spmm_layout(const mcsparseSpMatDescr* A, const mcsparseDnMatDescr* B,
     return l;
 }
 
+// Whether a product with a row-major op(B) and C takes less time from its diagonal blocks than from the kernel without a schedule,
+// which has more wavefronts in flight for the same rows.  Where lines are a whole number of strips, and operands of more than 128
+// bytes a row begin at whole vectors, it is left at the strips.  Microseconds with a schedule and without, 27-point stencils:
+bool schedule_pays(const SpmmSchedule& s, const mcsp::SpmmArgs& a, size_t value_bytes) {
+    if (!s.blocks) return true;
+    constexpr uint64_t kNarrow = 128;  // bytes of a row: half of a strip's lanes
+    const uint64_t row_bytes = static_cast<uint64_t>(a.n) * value_bytes, window = s.mean_span * row_bytes;
+    if (s.stride == 0) {
+        // groups of eight rows: not where they take in line ends (45 x 47 x 49 points, too few for strips of such lines; 24, 32, 48
+        // fp32 columns 56 and 17, 56 and 18, 60 and 30), nor narrow ones of few rows (27 diagonals, 24 fp32 columns, 30, 60 and 100 K
+        // rows: 14 and 8, 15 and 11, 17 and 16; 125 and 500 K: 19 and 20, 54 and 63)
+        constexpr idx_t kNarrowRows = 100000;
+        return !s.lines_cut && (row_bytes > kNarrow || a.m >= kNarrowRows);
+    }
+    const uint64_t wavefronts = mcsp::spmm_strip_wavefronts(a, s.stride, value_bytes);
+    // three to a SIMD are resident at a time
+    constexpr uint64_t kTwiceFull = 6144, kThriceFull = 9216;
+    // Narrow ones have the rows of op(B) that a row reads in L2 for longer: 81 x 83 x 90, 20 and 32 fp32 columns, 1.1 and 1.7 MB, 93
+    // and 74, 94 and 81; 101 x 101 x 90, 1.6 and 2.6 MB, 128 and 122, 129 and 157; 149 x 149 x 60, 5.7 MB, 185 and 244; but 150 x 150 x
+    // 12, 4400 wavefronts, 53 and 38.
+    constexpr uint64_t kNarrowWindow = 2000000;
+    if (row_bytes <= kNarrow) return wavefronts >= kThriceFull && window >= kNarrowWindow;
+    // 61 x 55 x 59, fp32, 64 and 128 columns, 3100 and 6200 wavefronts, 65 and 62, 104 and 107; 150 x 150 x 12, 64 columns, 4400
+    // wavefronts, 11 MB: 65 and 102.  Rows that begin at any element cost the strips a third line to a load: fp64, 61 x 55 x 59 and
+    // 64 x 64 x 64, 57 columns, 6200 and 8200 wavefronts, 139 and 113, 169 and 146; 97 x 61 x 97, 18500 wavefronts, 340 and 374.
+    constexpr uint64_t kL2 = 4 << 20;
+    const bool whole_vectors = row_bytes % 16 == 0;
+    if (whole_vectors && s.stride % mcsp::kSpmmStripRows == 0) return true;
+    return wavefronts >= (whole_vectors ? kTwiceFull : kThriceFull) || window > kL2;
+}
+
 template <typename T>
 mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOperation_t opB, const void* alpha,
                         const void* beta, const mcsparseDnMatDescr* B, mcsparseDnMatDescr* C, void* buffer) {
@@ -662,7 +693,10 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
         // into a column-major C as they lie there, 16 bytes per column: no row-major copy of C then.
         const bool scheduled_here = (b == 0 || shared_structure) && schedule_matches(A, buffer);
         const bool by_blocks = A->schedule.blocks;
+        const bool by_strips = by_blocks && A->schedule.stride != 0;
         auto schedule_usable = [&]() {
+            if (!l.copy_c && !schedule_pays(A->schedule, a, sizeof(T))) return false;
+            if (by_strips) return mcsp::spmm_strips_usable(a, sizeof(T));
             return by_blocks ? mcsp::spmm_blocks_usable(a, sizeof(T)) : mcsp::spmm_schedule_usable(a, sizeof(T));
         };
         const bool direct_c = l.copy_c && scheduled_here && schedule_usable() &&
@@ -679,7 +713,7 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
         }
         // the schedule was built from batch 0's structure
         if (scheduled_here && schedule_usable()) {
-            if (by_blocks && A->schedule.stride != 0)
+            if (by_strips)
                 mcsp::launch_spmm_strips<T>(h->stream, a, buffer, A->schedule.stride, A->schedule.entries,
                                             A->schedule.longest_group, A->schedule.mean_span, h_alpha, beta_inner);
             else if (by_blocks)
@@ -1228,8 +1262,16 @@ mcsparseStatus_t build_spmm_schedule(mcsparseHandle_t handle, mcsparseSpMatDescr
             // distance is read off a row in the middle, the gain is measured by covering the matrix that way, and the
             // strips are kept when they load a fifth fewer rows.
             // (Their kernel gives sixteen lanes of 16 bytes to a group and writes a column-major C in pieces of four
-            // rows: for operands of up to 128 bytes per row, and for a column-major C, the groups of eight rows stay.)
-            const bool strips_suit = row_bytes > 128 && matC->order == MCSPARSE_ORDER_ROW;
+            // rows: for operands of up to 128 bytes per row, and for a column-major C, the groups of eight rows stay.
+            // But where grid lines end inside groups of eight rows, which a block, with one range of rows for each of its
+            // diagonals, cannot say: such a group has five times the blocks, its wavefront takes as much longer, and strips are
+            // faster at 17 fp32 columns already: 20, 24, 32 columns of a 27-point stencil, 127 x 127 x 60, 255, 255, 257 us
+            // from groups of eight rows and 129, 129, 129 from strips; with lines of 120 points 93, 94, 101 and 124, 124, 125.
+            // With fewer rows, see schedule_pays, they would not be used.)
+            constexpr idx_t kNarrowStripRows = 1 << 19;
+            s.lines_cut = static_cast<uint64_t>(counters[2] >> 32) * block_groups >= 2 * static_cast<uint64_t>(blocks) &&
+                          static_cast<uint64_t>(blocks) * 23 > nz;
+            const bool strips_suit = (row_bytes > 128 || (s.lines_cut && m >= kNarrowStripRows)) && matC->order == MCSPARSE_ORDER_ROW;
             const uint32_t stride = !strips_suit ? 0u
                                                  : strip_stride_of_middle_row(handle->stream, m, static_cast<idx_t>(matA->idxBase),
                                                                               ia.rows, ia.cols);
@@ -1328,6 +1370,7 @@ mcsparseStatus_t mcsparseSpMM_preprocess(mcsparseHandle_t handle, mcsparseOperat
     s.base = static_cast<int>(matA->idxBase);
     s.blocks = false;
     s.stride = 0;
+    s.lines_cut = false;
     s.diagonals = 0;
     {
         // The kernels that work from a schedule walk every row in one piece; a matrix with rows of thousands of

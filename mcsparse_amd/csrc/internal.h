@@ -101,6 +101,7 @@ struct SpmmSchedule {
     bool blocks = false;   // the schedule holds diagonal blocks (spmm_blocks.hip) instead of merged lists
     uint32_t longest_group = 0;  // blocks: the most nonzeros in one group of rows (strips: in one strip)
     uint32_t stride = 0;   // blocks: != 0 says the groups are strips this many rows apart (spmm_strips.hip)
+    bool lines_cut = false;  // blocks: groups of eight rows take in the ends of grid lines, and need several times the blocks there
     // beside that (whether useful or not), for column-major operands: the diagonals of slices of rows (spmm_diagonals.hip), at
     // diagonals_at of the buffer; 0: none
     uint32_t diagonals = 0;
@@ -488,7 +489,7 @@ void launch_spmm_block_count(hipStream_t stream, idx_t m, idx_t nnz, idx_t base,
                              void* schedule);
 // Strip schedule of a CSR structure (spmm_strips.hip), the third kind: a group is kSpmmStrips strips of
 // kSpmmStripRows consecutive rows, strip q beginning `stride` rows behind strip q - 1; the rows are cut into stretches
-// of kSpmmStrips * stride rows, each holding stride / kSpmmStripRows groups.  Blocks are 16 bytes (see the file), the
+// of kSpmmStrips * stride rows, each holding stride / kSpmmStripRows groups (rounded up: the last has shorter strips).  Blocks are 16 bytes (see the file), the
 // region is used like the one of the block schedule, and the counters' place also holds the stride.
 constexpr int kSpmmStripRows = 4;
 constexpr int kSpmmStrips = 4;
@@ -496,7 +497,7 @@ constexpr int kSpmmStrips = 4;
 constexpr uint32_t kSpmmStripStagedValues = 128;
 constexpr uint64_t spmm_strip_groups(idx_t m, uint32_t stride) {
     return (static_cast<uint64_t>(m) + static_cast<uint64_t>(kSpmmStrips) * stride - 1) /
-           (static_cast<uint64_t>(kSpmmStrips) * stride) * (stride / kSpmmStripRows);
+           (static_cast<uint64_t>(kSpmmStrips) * stride) * ((stride + kSpmmStripRows - 1) / kSpmmStripRows);
 }
 // stride is one the schedule can be built with for a matrix of m rows
 bool spmm_strip_stride_usable(idx_t m, uint32_t stride);
@@ -505,7 +506,10 @@ void launch_spmm_strip_count(hipStream_t stream, idx_t m, idx_t nnz, idx_t base,
 void launch_spmm_strip_fill(hipStream_t stream, idx_t m, idx_t nnz, idx_t base, uint32_t stride, const idx_t* row_ptr,
                             const idx_t* col, void* schedule);
 bool spmm_strip_schedule_fits(idx_t m, idx_t nnz, uint32_t stride, uint32_t blocks);
-// Same conditions on the operands as the block schedule (spmm_blocks_usable).
+// Any row-major op(B) of at least five 128-bit vectors a row, wherever its rows and those of C begin.
+bool spmm_strips_usable(const SpmmArgs& a, size_t value_bytes);
+// How many wavefronts such a product is.
+uint64_t spmm_strip_wavefronts(const SpmmArgs& a, uint32_t stride, size_t value_bytes);
 template <typename T>
 void launch_spmm_strips(hipStream_t stream, const SpmmArgs& a, const void* schedule, uint32_t stride, uint32_t total_blocks,
                         uint32_t longest_strip, uint64_t mean_span, T alpha, T beta);

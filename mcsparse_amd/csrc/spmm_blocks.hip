@@ -30,12 +30,14 @@ struct BlockCounters {
     unsigned long long span_sum;  // sum over the groups of (last column - first column)
     unsigned long long loads;     // rows of op(B) all blocks load together
     unsigned int longest_group;   // most nonzeros in one group that has blocks
+    unsigned int most_blocks;     // of one group
 };
 
 __global__ void zero_block_counters_kernel(BlockCounters* c) {
     c->span_sum = 0;
     c->loads = 0;
     c->longest_group = 0;
+    c->most_blocks = 0;
 }
 
 // One thread covers the nonzeros of one group of K rows with blocks.  It merges the rows by the key
@@ -181,8 +183,10 @@ __global__ __launch_bounds__(kWave) void block_cover_kernel(idx_t m, idx_t base,
     if (!FILL) {
         if (group <= groups) block_ptr[group] = count;  // slot `groups` receives the total after the scan
         unsigned long long span = count != 0 ? last_col - first_col : 0;
+        uint32_t most = count;
 #pragma unroll
         for (int off = kWave / 2; off > 0; off >>= 1) {
+            most = max(most, static_cast<uint32_t>(__shfl_xor(static_cast<int>(most), off, kWave)));
             span += __shfl_xor(span, off, kWave);
             loads += __shfl_xor(loads, off, kWave);
             group_nnz = max(group_nnz, static_cast<uint32_t>(__shfl_xor(static_cast<int>(group_nnz), off, kWave)));
@@ -191,6 +195,7 @@ __global__ __launch_bounds__(kWave) void block_cover_kernel(idx_t m, idx_t base,
             if (span != 0) atomicAdd(&counters->span_sum, span);
             if (loads != 0) atomicAdd(&counters->loads, loads);
             if (group_nnz != 0) atomicMax(&counters->longest_group, group_nnz);
+            if (most != 0) atomicMax(&counters->most_blocks, most);
         }
     }
 }

@@ -31,6 +31,9 @@ constexpr int D = kSpmmBlockMaxDiagonals;
 constexpr int kRowsOfB = H + D - 1;
 constexpr int kLanes = 16;  // lanes per group: one per row where the values are fetched
 constexpr int kNoKey = 0x7fffffff;
+// Lines that are no whole number of strips, from so many rows on: with fewer, strips have too few wavefronts to be faster than the
+// kernel without a schedule (64 fp32 columns, 61 x 55 x 59 points 65 us and 62, 150 x 50 x 30 69 and 72, 97 x 61 x 97 137 and 161).
+constexpr idx_t kRaggedStripRows = 1 << 17;
 static_assert(R == kLanes && H == 4 && D == 3, "a lane per row; quads of lanes are strips; three bits per row");
 
 struct StripCounters {
@@ -54,10 +57,18 @@ __global__ void zero_strip_counters_kernel(StripCounters* c, uint32_t stride) {
     c->stride = stride;
 }
 
-__device__ __forceinline__ uint64_t first_row_of_group(uint64_t group, uint32_t stride) {
-    const uint64_t per_tile = stride / H;  // groups in a stretch of Q * stride rows
-    return group / per_tile * (static_cast<uint64_t>(Q) * stride) + group % per_tile * H;
-}
+// Rows of a group: strip q has the rows first + q * stride + [0, rows).  Where the stride is no multiple of H the last group of
+// a stretch has fewer than H rows in each of its strips.
+struct GroupRows {
+    uint64_t first;
+    uint32_t rows;
+    __device__ __forceinline__ GroupRows(uint64_t group, uint32_t stride) {
+        const uint64_t per_tile = (stride + H - 1) / H;  // groups in a stretch of Q * stride rows
+        const uint32_t in_tile = static_cast<uint32_t>(group % per_tile) * H;
+        first = group / per_tile * (static_cast<uint64_t>(Q) * stride) + in_tile;
+        rows = min(stride - in_tile, static_cast<uint32_t>(H));
+    }
+};
 
 // v of another lane of the same row of 16 lanes, chosen by a DPP control (quad permutes and mirrors, as in group_sum).
 template <int CTRL>
@@ -103,10 +114,12 @@ __global__ __launch_bounds__(kBlock) void strip_cover_kernel(idx_t m, idx_t nnz,
     int first_col = 0x7fffffff, last_col = -1;
     int longest_strip = 0;
     if (group < groups) {
-        const uint64_t row = first_row_of_group(group, stride) + static_cast<uint64_t>(lane / H) * stride + lane % H;
-        const bool exists = row < static_cast<uint64_t>(m);
-        idx_t i = exists ? row_ptr[row] - base : 0;
-        const idx_t e = exists ? row_ptr[row + 1] - base : 0;
+        // (a row that the strip does not have is empty and lies where the strip ends)
+        const GroupRows g(group, stride);
+        const uint64_t row = min(g.first + static_cast<uint64_t>(lane / H) * stride + min(lane % H, g.rows), static_cast<uint64_t>(m));
+        const bool exists = lane % H < g.rows && row < static_cast<uint64_t>(m);
+        idx_t i = row_ptr[row] - base;
+        const idx_t e = exists ? row_ptr[row + 1] - base : i;
         const int row_nnz = static_cast<int>(e - i);
         int strip_nnz = row_nnz + dpp_int<kDppQuadXor1>(row_nnz);
         strip_nnz += dpp_int<kDppQuadXor2>(strip_nnz);
@@ -314,10 +327,12 @@ constexpr int strip_room() { return strip_capacity<T>() + 2 * (16 / static_cast<
 // broadcasts.  STAGED: no strip holds more than strip_capacity<T>() nonzeros and the value array is 16-byte aligned;
 // the four lanes of a strip then copy its values into LDS once, in whole 16-byte pieces, and the blocks read them
 // there.
+// RAGGED: rows of op(B) and C begin at any element, and n need not be a multiple of V (27-point stencil 97 x 61 x 97, fp32, 37 and
+// 57 columns: 151 and 180 us without a schedule, 100 and 128 so; fp64, 37 and 83: 359 and 798, 261 and 492).
 // A workgroup is one wavefront (four groups): a wavefront that is through makes room for the next at once instead of
 // waiting for the others of its workgroup (256 threads: 360 us at N = 64 on the 128^3 stencil, 128 or 64: 349 us).
 constexpr int kStripBlock = kWave;
-template <typename T, bool WIDE, bool STAGED>
+template <typename T, bool WIDE, bool STAGED, bool RAGGED>
 __global__ __launch_bounds__(kStripBlock, 3) void spmm_strips_kernel(idx_t m, idx_t n, idx_t base, uint32_t stride,
                                                              const idx_t* __restrict__ row_ptr,
                                                              const idx_t* __restrict__ col, const T* __restrict__ val,
@@ -336,10 +351,11 @@ __global__ __launch_bounds__(kStripBlock, 3) void spmm_strips_kernel(idx_t m, id
     if (turn >= groups) return;  // whole lane groups
     // which group takes this turn (held to the groups that exist, whatever the buffer holds)
     const uint64_t group = min(static_cast<uint64_t>(order[turn]), groups - 1);
-    const uint64_t g0 = first_row_of_group(group, stride);
-    const uint64_t c_own = (static_cast<uint64_t>(blockIdx.y) * kLanes + lane) * V;
-    const bool stores = c_own < static_cast<uint64_t>(n);  // lanes past the last column only help fetching
-    const uint64_t c0 = stores ? c_own : 0;
+    const GroupRows rows_of(group, stride);
+    const uint64_t g0 = rows_of.first;
+    // lanes past the last column only help fetching
+    const LaneColumns own = lane_columns<V, RAGGED>((static_cast<uint64_t>(blockIdx.y) * kLanes + lane) * V, n);
+    const uint64_t c0 = own.first;
 
     T acc[R][V];
 #pragma unroll
@@ -351,11 +367,12 @@ __global__ __launch_bounds__(kStripBlock, 3) void spmm_strips_kernel(idx_t m, id
     const off_t lane_off = static_cast<off_t>(c0 * sizeof(T));
     const off_t ldb_bytes = static_cast<off_t>(ldb * sizeof(T));
 
-    // this lane's row of the group: where its nonzeros begin and end (a row past the matrix's end holds none)
-    const uint64_t my_row = g0 + static_cast<uint64_t>(lane / H) * stride + lane % H;
+    // this lane's row of the group: where its nonzeros begin and end (a row that the strip or the matrix does not have holds none)
+    const uint64_t my_row = g0 + static_cast<uint64_t>(lane / H) * stride + min(lane % H, rows_of.rows);
     const uint64_t row_at = my_row < static_cast<uint64_t>(m) ? my_row : static_cast<uint64_t>(m);
+    const bool row_exists = lane % H < rows_of.rows && my_row < static_cast<uint64_t>(m);
     const idx_t row_begin = row_ptr[row_at] - base;
-    const idx_t row_end = (my_row < static_cast<uint64_t>(m) ? row_ptr[row_at + 1] : row_ptr[row_at]) - base;
+    const idx_t row_end = (row_exists ? row_ptr[row_at + 1] : row_ptr[row_at]) - base;
     // its strip's nonzeros: from the first row's begin to the last row's end (DPP inside the quad of lanes)
     const idx_t strip_begin = static_cast<idx_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(row_begin), 0x00, 0xF, 0xF, true));
     const idx_t strip_end = static_cast<idx_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(row_end), 0xFF, 0xF, 0xF, true));
@@ -472,7 +489,9 @@ __global__ __launch_bounds__(kStripBlock, 3) void spmm_strips_kernel(idx_t m, id
             static_for<kRowsOfB>([&](auto jc) {
                 constexpr uint32_t j = decltype(jc)::value;
                 const uint32_t jj = min(max(j, sh.j_first), sh.j_last);
-                o.b[j] = load_vec<T, V>(reinterpret_cast<const T*>(B_bytes + (roff + static_cast<off_t>(jj) * ldb_bytes)));
+                const T* at = reinterpret_cast<const T*>(B_bytes + (roff + static_cast<off_t>(jj) * ldb_bytes));
+                if constexpr (RAGGED) o.b[j] = load_row<T, V>(at);
+                else o.b[j] = load_vec<T, V>(at);
             });
         };
         auto consume = [&](const Shape& sh, const Operands& o) {
@@ -560,12 +579,13 @@ __global__ __launch_bounds__(kStripBlock, 3) void spmm_strips_kernel(idx_t m, id
         });
     }
 
-    if (!stores) return;
+    if (!own.any) return;
     // A column-major C holds the rows of a strip next to each other in every column: 16 or 32 bytes.
-    const bool whole_columns = !c_row_major && ((reinterpret_cast<uintptr_t>(C) | static_cast<uintptr_t>(ldc * sizeof(T))) & 15u) == 0;
+    const bool whole_columns = !RAGGED && !c_row_major && stride % H == 0 &&
+                               ((reinterpret_cast<uintptr_t>(C) | static_cast<uintptr_t>(ldc * sizeof(T))) & 15u) == 0;
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-        const uint64_t strip_row = g0 + static_cast<uint64_t>(q) * stride;  // a multiple of H
+        const uint64_t strip_row = g0 + static_cast<uint64_t>(q) * stride;
         if (whole_columns && strip_row + H <= static_cast<uint64_t>(m)) {
 #pragma unroll
             for (int c = 0; c < V; ++c)
@@ -574,8 +594,8 @@ __global__ __launch_bounds__(kStripBlock, 3) void spmm_strips_kernel(idx_t m, id
         } else {
 #pragma unroll
             for (int h = 0; h < H; ++h) {
-                if (strip_row + h < static_cast<uint64_t>(m))
-                    store_c<T, V>(C, ldc, c_row_major, strip_row + h, c0, acc[q * H + h], alpha, beta);
+                if (static_cast<uint32_t>(h) < rows_of.rows && strip_row + h < static_cast<uint64_t>(m))
+                    store_c<T, V>(C, ldc, c_row_major, strip_row + h, c0, acc[q * H + h], alpha, beta, own.skip);
             }
         }
     }
@@ -583,6 +603,10 @@ __global__ __launch_bounds__(kStripBlock, 3) void spmm_strips_kernel(idx_t m, id
 
 // The strip schedule inside the region spmm_schedule_layout describes: the offsets where the merged lists keep
 // theirs, the blocks from the start of the entries' place, the order of the groups at its end.
+bool whole_vectors(const SpmmArgs& a, size_t value_bytes) {
+    const int64_t wide = static_cast<int64_t>(16 / value_bytes);
+    return reinterpret_cast<uintptr_t>(a.B) % 16 == 0 && a.ldb % wide == 0 && a.n % wide == 0;
+}
 struct Carved {
     uint32_t* block_ptr;
     StripCounters* counters;
@@ -602,9 +626,20 @@ Carved carve(idx_t m, idx_t nnz, uint32_t stride, void* schedule) {
 
 }  // namespace
 
+bool spmm_strips_usable(const SpmmArgs& a, size_t value_bytes) {
+    // at least five 128-bit vectors per row, as for the blocks over eight rows
+    return a.b_row_major && a.n >= 4 * static_cast<int64_t>(16 / value_bytes) + 1 && a.k <= kSpmmMaxScheduledColumns &&
+           a.m < (idx_t(1) << 31);
+}
+
+uint64_t spmm_strip_wavefronts(const SpmmArgs& a, uint32_t stride, size_t value_bytes) {
+    const uint64_t row_bytes = static_cast<uint64_t>(a.n) * value_bytes, panel = kLanes * 16;
+    return (spmm_strip_groups(a.m, stride) + kStripBlock / kLanes - 1) / (kStripBlock / kLanes) * ((row_bytes + panel - 1) / panel);
+}
+
 bool spmm_strip_stride_usable(idx_t m, uint32_t stride) {
-    // whole strips per stretch, more than one group per stretch, and no more offsets than the region has slots for
-    return stride >= 2 * H && stride % H == 0 && static_cast<uint64_t>(stride) * 8 <= static_cast<uint64_t>(m) &&
+    // more than one group per stretch, whole strips unless there are many rows, and no more offsets than the region has slots for
+    return stride >= 2 * H && (stride % H == 0 || m >= kRaggedStripRows) && static_cast<uint64_t>(stride) * 8 <= static_cast<uint64_t>(m) &&
            spmm_strip_groups(m, stride) + 1 <= spmm_groups(m) + 1;
 }
 
@@ -664,10 +699,14 @@ void launch_spmm_strips(hipStream_t stream, const SpmmArgs& a, const void* sched
     const T* B = static_cast<const T*>(a.B);
     T* C = static_cast<T*>(a.C);
     const bool staged = longest_strip <= static_cast<uint32_t>(strip_capacity<T>()) && reinterpret_cast<uintptr_t>(val) % 16 == 0;
+    auto launch_kind = [&](auto wide_c, auto staged_c, auto ragged_c) {
+        hipLaunchKernelGGL((spmm_strips_kernel<T, decltype(wide_c)::value, decltype(staged_c)::value, decltype(ragged_c)::value>), grid,
+                           dim3(kStripBlock), 0, stream, a.m, a.n, a.base, stride, a.row_ptr, a.col, val, c.block_ptr, c.blocks,
+                           c.order, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta, xcd_chunk, xcds, a.k, a.nnz, total_blocks);
+    };
     auto launch = [&](auto wide_c, auto staged_c) {
-        hipLaunchKernelGGL((spmm_strips_kernel<T, decltype(wide_c)::value, decltype(staged_c)::value>), grid, dim3(kStripBlock), 0,
-                           stream, a.m, a.n, a.base, stride, a.row_ptr, a.col, val, c.block_ptr, c.blocks, c.order, B, a.ldb, C,
-                           a.ldc, a.c_row_major, alpha, beta, xcd_chunk, xcds, a.k, a.nnz, total_blocks);
+        if (whole_vectors(a, sizeof(T))) launch_kind(wide_c, staged_c, std::false_type{});
+        else launch_kind(wide_c, staged_c, std::true_type{});
     };
     if (narrow_offsets(a, sizeof(T))) {
         if (staged) launch(std::false_type{}, std::true_type{});

@@ -480,6 +480,18 @@ def test_strips_grid_with_broken_rows(torch_gpu, handle, oracle, dtype, n):
           prepare_for_row_major_c=True)
 
 
+@pytest.mark.parametrize("line", [51, 53])
+@pytest.mark.parametrize("dtype,n", [(np.float32, 256), (np.float32, 250), (np.float64, 128), (np.float64, 125)])
+def test_strips_of_lines_that_are_no_whole_number_of_strips(torch_gpu, handle, oracle, dtype, n, line):
+    """Lines of 51 and 53 points: the last group of a stretch has three rows or one in each of its strips.  Rows of op(B) and C
+    that begin at whole vectors, and at any element."""
+    a = wl.stencil_27pt(line, dtype=dtype)
+    check(torch_gpu, handle, oracle, a, n, 1.0, 0.0, preprocess=True, expect_schedule=4)
+    check(torch_gpu, handle, oracle, a.with_base(1), n, -0.5, 1.5, preprocess=True, expect_schedule=4, pad_b=3, pad_c=5)
+    check(torch_gpu, handle, oracle, a, n, 0.5, -1.0, preprocess=True, expect_schedule=4, c_order=api.ORDER_COL,
+          prepare_for_row_major_c=True)
+
+
 @pytest.mark.parametrize("dtype,n", [(np.float32, 129), (np.float32, 133), (np.float32, 150), (np.float32, 190), (np.float32, 253),
                                      (np.float32, 384), (np.float64, 65), (np.float64, 67), (np.float64, 75), (np.float64, 90),
                                      (np.float64, 127), (np.float64, 192)])
