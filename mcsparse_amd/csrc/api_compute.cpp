@@ -107,7 +107,7 @@ SpmvLayout spmv_layout(const CsrView& v, int64_t nnz, size_t value_bytes, size_t
         l.vals = off;
         off += align_up(static_cast<size_t>(nnz) * value_bytes);
         l.csr2csc_ws = off;
-        off += align_up(mcsp::transposed_products_workspace_bytes(static_cast<idx_t>(nnz), value_bytes));
+        off += align_up(mcsp::transposed_products_workspace_bytes(static_cast<idx_t>(v.n), static_cast<idx_t>(nnz), value_bytes));
     }
     l.narrow = off;
     off += narrow;
@@ -435,9 +435,9 @@ mcspStatus_t spmv_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
                    ? MCSP_STATUS_SUCCESS
                    : MCSP_STATUS_INTERNAL_ERROR;
     }
-    uint32_t bucket_shift = 0;
+    mcsp::ColumnBuckets columns;
     if (alg != MCSPARSE_SPMV_CSR_ALG2 &&
-        mcsp::bucketed_products_shape(static_cast<idx_t>(v.n), &bucket_shift)) {
+        mcsp::bucketed_products_shape(static_cast<idx_t>(v.n), &columns)) {
         mcsp::BucketedProducts b;
         mcsp::launch_bucketed_products(h->stream, static_cast<idx_t>(v.m), static_cast<idx_t>(v.n), nnz, v.val, v.ptr,
                                        v.ind, x->values, sizeof(T), base, buf + l.csr2csc_ws, l.narrow - l.csr2csc_ws, &b);

@@ -1011,9 +1011,11 @@ size_t csr2csc_workspace_bytes(idx_t /*m*/, idx_t n, idx_t nnz, size_t value_byt
     return passes > sort ? passes : sort;
 }
 
-size_t transposed_products_workspace_bytes(idx_t nnz, size_t value_bytes) {
+size_t transposed_products_workspace_bytes(idx_t n, idx_t nnz, size_t value_bytes) {
     const size_t sort = csr2csc_layout(nnz, value_bytes, true).total;
-    const size_t buckets = bucketed_products_workspace_bytes(nnz, value_bytes);
+    ColumnBuckets columns;
+    const uint32_t bits = bucketed_products_shape(n, &columns) ? columns.bits : kBucketFewBits;
+    const size_t buckets = bucketed_products_workspace_bytes(nnz, bits, value_bytes);
     return sort > buckets ? sort : buckets;
 }
 

@@ -547,8 +547,8 @@ void launch_csr2csc(hipStream_t stream, idx_t m, idx_t n, idx_t nnz, const void*
                     idx_t base, void* workspace);
 // products[nnz] = value * x[row] of every nonzero in the order of a stable sort by column, and
 // col_ptr[n+1] (+ base): what op(A) = A^T needs of the transpose.  value_bytes is 4 (fp32 values and
-// x) or 8 (fp64); workspace of transposed_products_workspace_bytes(nnz, value_bytes) bytes.
-size_t transposed_products_workspace_bytes(idx_t nnz, size_t value_bytes);
+// x) or 8 (fp64); workspace of transposed_products_workspace_bytes(n, nnz, value_bytes) bytes.
+size_t transposed_products_workspace_bytes(idx_t n, idx_t nnz, size_t value_bytes);
 void launch_transposed_products(hipStream_t stream, idx_t m, idx_t n, idx_t nnz, const void* csr_val, const idx_t* row_ptr,
                                 const idx_t* col, const void* x, void* products, idx_t* col_ptr, size_t value_bytes,
                                 idx_t base, void* workspace);
@@ -578,28 +578,51 @@ size_t partition_sort_pairs_workspace_bytes(idx_t count, idx_t major_count, idx_
 void launch_partition_sort_pairs(hipStream_t stream, idx_t count, idx_t major_count, idx_t minor_count, idx_t* major,
                                  idx_t* minor, idx_t* perm, void* workspace);
 
-// The products of a transposing SpMV ordered by bucket of 2^shift neighbouring columns (index base taken off: bucket b holds columns
-// [b << shift, (b + 1) << shift), at most 256 of them), but only inside tiles of the CSR order: table[b * tiles + t] says
-// where in tile t, which begins at place t * tile_places, the run of bucket b lies (place | length << 16,
-// partition_device.h).  Runs begin at multiples of kBucketRunPad and are padded with products of 0 to such a length.
-// keys[] holds a column's place in its bucket (in its low `shift` bits).  One pass over the nonzeros instead of the three of a full sort, for
+// The columns of a matrix in at most 2^bits stretches ("buckets") of `width`: with a power of two of columns to each, half of the
+// compute units have no bucket where the columns are a few more than a power of two (2.2 M columns, 43 M nonzeros: a call 234 us,
+// 208 so).
+// Bucket of a column: the high word of its product with factor, 2^(32 + shift) / width rounded up, shifted.  That is too large by less
+// than column / 2^(32 + shift) of a bucket, which is below 1 / width for columns below 2^31: exact.
+struct ColumnBuckets {
+    uint32_t width = 0, factor = 0, shift = 0, bits = 0;
+};
+// n: at least two columns, and at least as many to a bucket
+constexpr ColumnBuckets column_buckets(idx_t n, uint32_t bits) {
+    ColumnBuckets b;
+    b.bits = bits;
+    b.width = static_cast<uint32_t>(((static_cast<uint64_t>(n) - 1) >> bits) + 1);
+    while ((2u << b.shift) < b.width) ++b.shift;
+    b.factor = static_cast<uint32_t>(((uint64_t(1) << (32 + b.shift)) + b.width - 1) / b.width);
+    return b;
+}
+constexpr uint32_t bucket_of(const ColumnBuckets& b, uint32_t column) {
+    return static_cast<uint32_t>(static_cast<uint64_t>(column) * b.factor >> 32) >> b.shift;
+}
+
+// The products of a transposing SpMV ordered by such buckets of columns (index base taken off), but only inside tiles of the CSR
+// order: table[b * tiles + t] says where in tile t, which begins at place t * tile_places, the run of bucket b lies (place | length
+// << 16, partition_device.h).  Runs begin at multiples of kBucketRunPad and are padded with products of 0, of any column, to such
+// a length.  keys[] holds the low half of a column.  One pass over the nonzeros instead of the three of a full sort, for
 // callers that then add the products of a column in any order.  The shape function says whether the shape allows it
-// (more than 2^14 and at most 2^22 columns: a bucket's sums must fit in LDS as doubles).
-constexpr uint32_t kBucketMinKeyBits = 15;
-constexpr uint32_t kBucketMaxShift = 14;
+// (more than 2^14 columns, and a bucket's sums must fit in LDS as doubles: 256 buckets where that does, 1024 beyond).
+constexpr idx_t kBucketMinColumns = (1 << 14) + 1;
+constexpr uint32_t kSkinnyMaxColumns = 1 << 14;
+constexpr uint32_t kBucketMaxColumns = 18432;  // of a bucket: 144 of the 160 KB of LDS
+constexpr uint32_t kBucketFewBits = 8, kBucketManyBits = 10;
 constexpr uint32_t kBucketTileMin = 4096;  // nonzeros of the smallest tiles
 constexpr uint32_t kBucketRunPad = 4;
 struct BucketedProducts {
     const uint16_t* keys = nullptr;
     const void* products = nullptr;
     const uint32_t* table = nullptr;
-    uint32_t* totals = nullptr;  // room for 256 words
-    uint32_t tiles = 0, tile_places = 0, shift = 0, buckets = 0;
+    uint32_t* totals = nullptr;  // room for a word per bucket
+    uint32_t tiles = 0, tile_places = 0;
+    ColumnBuckets columns;
     void* spare = nullptr;  // part of the workspace the pass did not use, for the sums of buckets that are split
     size_t spare_bytes = 0;
 };
-bool bucketed_products_shape(idx_t n, uint32_t* shift);
-size_t bucketed_products_workspace_bytes(idx_t nnz, size_t value_bytes);
+bool bucketed_products_shape(idx_t n, ColumnBuckets* columns);
+size_t bucketed_products_workspace_bytes(idx_t nnz, uint32_t bits, size_t value_bytes);
 void launch_bucketed_products(hipStream_t stream, idx_t m, idx_t n, idx_t nnz, const void* csr_val, const idx_t* row_ptr,
                               const idx_t* col, const void* x, size_t value_bytes, idx_t base, void* workspace,
                               size_t workspace_bytes, BucketedProducts* out);

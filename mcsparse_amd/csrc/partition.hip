@@ -49,6 +49,7 @@ struct EntrySource {
     bool relative;
     uint32_t* wide;
     uint32_t minor_bits;  // plain, packed entries: bits of the index, which lies below the key's rest
+    ColumnBuckets columns;  // products
 };
 
 // The order of tiles over the workgroups: an XCD takes a contiguous range, so the table words of neighbouring tiles,
@@ -124,7 +125,7 @@ __device__ __forceinline__ void count_rows(TileRows<TILE>& s) {
     }
 }
 
-// A workgroup per tile.  Key: the type the rest of a key travels in.
+// A workgroup per tile.  Key: the type the rest of a key travels in.  Products: the digit is the bucket of ColumnBuckets.
 //
 // Bounds at 118 M entries (the products of a transposing SpMV, fp32): 0.98 GB read and 0.79 GB written in 340 us, nine
 // tenths of the rate of a copy; tiles of 4096 or 16 wavefronts per workgroup are no faster (342 and 420 us).  The pass
@@ -187,10 +188,15 @@ __global__ __launch_bounds__(THREADS) void partition_kernel(EntrySource in, uint
 
     const uint32_t mask = (1u << bits) - 1u;
 #pragma unroll
-    for (int i = 0; i < ITEMS; ++i) key[i] -= in.key_bias;
-    auto digit = [&](int i) { return (key[i] >> shift) & mask; };
+    for (int i = 0; i < ITEMS; ++i) {
+        key[i] -= in.key_bias;
+        // the bucket above the column's low half, and no bucket but those that exist, whatever the column
+        if constexpr (!kOrdered) key[i] = min(bucket_of(in.columns, key[i]), mask) << 16 | (key[i] & 0xffffu);
+    }
+    auto digit = [&](int i) { return kOrdered ? (key[i] >> shift) & mask : key[i] >> 16; };
     uint32_t dest[(ITEMS + 1) / 2];
-    uint32_t pad_from = 0, pad_to = 0;  // what this thread's digit leaves open behind its run
+    constexpr int kDigits = (1 << MAX_BITS) > THREADS ? (1 << MAX_BITS) / THREADS : 1;  // products: neighbouring digits of a thread
+    uint32_t pad_from[kDigits], pad_to[kDigits];  // what they leave open behind their runs
     uint32_t* const s_count = reinterpret_cast<uint32_t*>(s_cnt);
     if constexpr (kOrdered) rank_entries<ITEMS, MAX_BITS>(count, bits, s_cnt, dest, digit);
     else rank_entries_unordered<ITEMS>(count, s_count, dest, digit);
@@ -206,16 +212,26 @@ __global__ __launch_bounds__(THREADS) void partition_kernel(EntrySource in, uint
             table[static_cast<uint64_t>(d) * tiles + tile] = table_word(at, n);
         });
     } else {
-        static_assert(1 << MAX_BITS <= THREADS, "a thread per digit");
-        const uint32_t n = tid < (1u << MAX_BITS) ? s_count[tid] : 0;
-        const uint32_t padded = (n + kPad - 1) / kPad * kPad;
-        const uint32_t at = block_exclusive_sum<THREADS>(padded, s_wave);
-        if (tid < (1u << MAX_BITS)) {
-            s_count[tid] = at;
-            if (tid < (1u << bits)) table[static_cast<uint64_t>(tid) * tiles + tile] = table_word(at, padded);
+        uint32_t n[kDigits], padded[kDigits], sum = 0;
+#pragma unroll
+        for (int k = 0; k < kDigits; ++k) {
+            const uint32_t d = tid * kDigits + k;
+            n[k] = d < (1u << MAX_BITS) ? s_count[d] : 0;
+            padded[k] = (n[k] + kPad - 1) / kPad * kPad;
+            sum += padded[k];
         }
-        pad_from = at + n;
-        pad_to = at + padded;
+        uint32_t at = block_exclusive_sum<THREADS>(sum, s_wave);
+#pragma unroll
+        for (int k = 0; k < kDigits; ++k) {
+            const uint32_t d = tid * kDigits + k;
+            if (d < (1u << MAX_BITS)) {
+                s_count[d] = at;
+                if (d < (1u << bits)) table[static_cast<uint64_t>(d) * tiles + tile] = table_word(at, padded[k]);
+            }
+            pad_from[k] = at + n[k];
+            at += padded[k];
+            pad_to[k] = at;
+        }
         __syncthreads();
     }
 #pragma unroll
@@ -278,7 +294,7 @@ __global__ __launch_bounds__(THREADS) void partition_kernel(EntrySource in, uint
         store_packed<VB, ITEMS, THREADS, kPlaces>(s_buf, count, dest, keys_out, vals_out, out, [&](int i) { return key[i]; }, val);
         return;
     }
-    store_keys<ITEMS, THREADS, kPlaces>(s_buf, count, dest, keys_out + out, key, (1u << shift) - 1u);
+    store_keys<ITEMS, THREADS, kPlaces>(s_buf, count, dest, keys_out + out, key, kOrdered ? (1u << shift) - 1u : 0xffffu);
     if constexpr (KIND == kProducts) {
         typedef typename RealOf<VB>::type real_t;
         const real_t* x = static_cast<const real_t*>(in.x);
@@ -294,7 +310,10 @@ __global__ __launch_bounds__(THREADS) void partition_kernel(EntrySource in, uint
             __builtin_amdgcn_sched_barrier(0);
         }
         // (a product of 0 and whatever key lies beside it: both halves of a 64-bit zero are the same word)
-        for (uint32_t p = pad_from; p < pad_to; ++p) s_buf[p] = 0;
+#pragma unroll
+        for (int k = 0; k < kDigits; ++k) {
+            for (uint32_t p = pad_from[k]; p < pad_to[k]; ++p) s_buf[p] = 0;
+        }
     } else {
         if constexpr (KIND == kCsr) {
 #pragma unroll
@@ -1362,16 +1381,16 @@ void launch_row_starts(hipStream_t stream, const EntrySource& in, uint32_t tile_
 struct BucketedLayout {
     size_t keys, products, table, totals, tile_rows, spare;
 };
-BucketedLayout bucketed_layout(idx_t nnz, size_t value_bytes) {
+BucketedLayout bucketed_layout(idx_t nnz, uint32_t bits, size_t value_bytes) {
     const uint32_t tile_size = tile_size_for(nnz);
     const size_t tiles = tiles_of(nnz, tile_size);
     BucketedLayout l;
     size_t off = 0;
-    const size_t places = tile_places(tile_size, kProducts, 8);
+    const size_t places = tile_places(tile_size, kProducts, bits);
     l.keys = off; off += align_up(tiles * places * sizeof(uint16_t));
     l.products = off; off += align_up(tiles * places * value_bytes);
-    l.table = off; off += align_up(256 * tiles * sizeof(uint32_t));
-    l.totals = off; off += align_up(256 * sizeof(uint32_t));
+    l.table = off; off += align_up((tiles << bits) * sizeof(uint32_t));
+    l.totals = off; off += align_up(sizeof(uint32_t) << bits);
     l.tile_rows = off; off += align_up((tiles + 1) * sizeof(uint32_t));
     l.spare = off;
     return l;
@@ -1630,24 +1649,28 @@ void launch_partition_sort_pairs(hipStream_t stream, idx_t count, idx_t major_co
     launch(stream, in, s, out, static_cast<char*>(workspace));
 }
 
-bool bucketed_products_shape(idx_t n, uint32_t* shift) {
-    const uint32_t bits = bit_length(n - 1);  // of the columns without their index base
-    // fewer keys than that: the full sort is two short passes; more: a bucket's sums no longer fit in LDS
-    if (bits < kBucketMinKeyBits || bits > 8 + kBucketMaxShift) return false;
-    *shift = bits - 8;
-    return true;
+bool bucketed_products_shape(idx_t n, ColumnBuckets* columns) {
+    // fewer columns than that: the full sort is two short passes; more: a bucket's sums no longer fit in LDS
+    if (n < kBucketMinColumns) return false;
+    for (const uint32_t bits : {kBucketFewBits, kBucketManyBits}) {
+        *columns = column_buckets(n, bits);
+        if (columns->width <= kBucketMaxColumns) return true;
+    }
+    return false;
 }
 
-size_t bucketed_products_workspace_bytes(idx_t nnz, size_t value_bytes) { return bucketed_layout(nnz, value_bytes).spare; }
+size_t bucketed_products_workspace_bytes(idx_t nnz, uint32_t bits, size_t value_bytes) {
+    return bucketed_layout(nnz, bits, value_bytes).spare;
+}
 
-// One partition by the top eight bits of the columns (index base taken off), the values multiplied by x[row] on the
+// One partition by the buckets of the columns (index base taken off), the values multiplied by x[row] on the
 // way.  What lies behind workspace_bytes is not touched.
 void launch_bucketed_products(hipStream_t stream, idx_t m, idx_t n, idx_t nnz, const void* csr_val, const idx_t* row_ptr,
                               const idx_t* col, const void* x, size_t value_bytes, idx_t base, void* workspace,
                               size_t workspace_bytes, BucketedProducts* out) {
-    uint32_t shift = 0;
-    if (m == 0 || nnz == 0 || !bucketed_products_shape(n, &shift)) return;
-    const BucketedLayout l = bucketed_layout(nnz, value_bytes);
+    if (m == 0 || nnz == 0 || !bucketed_products_shape(n, &out->columns)) return;
+    const uint32_t bits = out->columns.bits;
+    const BucketedLayout l = bucketed_layout(nnz, bits, value_bytes);
     char* w = static_cast<char*>(workspace);
     EntrySource in;
     in.keys = col;
@@ -1662,16 +1685,20 @@ void launch_bucketed_products(hipStream_t stream, idx_t m, idx_t n, idx_t nnz, c
     const uint32_t tile_size = tile_size_for(nnz);
     uint32_t* table = reinterpret_cast<uint32_t*>(w + l.table);
     launch_row_starts(stream, in, tile_size, reinterpret_cast<uint32_t*>(w + l.tile_rows), nullptr);
-    auto* launch = value_bytes == 4 ? launch_partition<4, kProducts, 8, uint16_t> : launch_partition<8, kProducts, 8, uint16_t>;
-    launch(stream, in, shift, 8, tile_size, w + l.keys, nullptr, w + l.products, table);
+    auto of_bits = [&](auto vb) {
+        constexpr int VB = decltype(vb)::value;
+        return bits == kBucketFewBits ? launch_partition<VB, kProducts, kBucketFewBits, uint16_t>
+                                      : launch_partition<VB, kProducts, kBucketManyBits, uint16_t>;
+    };
+    auto* launch = value_bytes == 4 ? of_bits(std::integral_constant<int, 4>{}) : of_bits(std::integral_constant<int, 8>{});
+    in.columns = out->columns;
+    launch(stream, in, 0, bits, tile_size, w + l.keys, nullptr, w + l.products, table);
     out->keys = reinterpret_cast<const uint16_t*>(w + l.keys);
     out->products = w + l.products;
     out->table = table;
     out->totals = reinterpret_cast<uint32_t*>(w + l.totals);
     out->tiles = tiles_of(nnz, tile_size);
-    out->tile_places = tile_places(tile_size, kProducts, 8);
-    out->shift = shift;
-    out->buckets = static_cast<uint32_t>((n - 1) >> shift) + 1;
+    out->tile_places = tile_places(tile_size, kProducts, bits);
     out->spare = w + l.spare;
     out->spare_bytes = workspace_bytes > l.spare ? workspace_bytes - l.spare : 0;
 }

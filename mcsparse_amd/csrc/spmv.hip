@@ -814,7 +814,7 @@ __global__ __launch_bounds__(kBlock) void skinny_reduce_kernel(idx_t n, const do
 bool skinny_transpose_shape(idx_t n, idx_t nnz) {
     // at most 2^14 columns: a copy of y fits in LDS as doubles; enough columns that the lanes of a wavefront
     // seldom meet on one sum; enough nonzeros that the planes are small beside them (and fit the scratch)
-    return n <= (1u << kBucketMaxShift) && n >= 256 &&
+    return n <= kSkinnyMaxColumns && n >= 256 &&
            static_cast<uint64_t>(nnz) >= static_cast<uint64_t>(kSkinnyMinNonzerosPerColumn) * n;
 }
 

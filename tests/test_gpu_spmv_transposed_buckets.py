@@ -64,6 +64,21 @@ def test_exact_on_integers_across_the_key_range(torch_gpu, handle, dtype, base, 
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("base", [0, 1])
+@pytest.mark.parametrize("rows,n", [(3001, 16641), (3001, 65537), (60001, 2200003), (3001, 18432 * 256), (3001, 18432 * 256 + 1),
+                                    (60001, 5000011), (60001, 18432 * 1024), (3001, 18432 * 1024 + 1)])
+def test_exact_on_integers_where_buckets_are_no_power_of_two(torch_gpu, handle, dtype, base, rows, n):
+    # 18432 columns are the most of a bucket; up to 256 of them, 1024 beyond, behind those the full sort
+    a = wl.random_ragged(rows, n, 40, dtype=dtype, seed=n % 97 + base, base=base)
+    a.col[::50] = n - 1 + base  # the last column, and the first
+    a.col[1::50] = base
+    x, y = integer_valued(a, n)
+    want = 2 * (a.to_scipy().T.astype(np.float64) @ x.astype(np.float64)) - 3 * y
+    got = run(torch_gpu, handle, a, x, y, 2.0, -3.0)
+    assert np.array_equal(got.astype(np.float64), want), "n=%d base=%d" % (n, base)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_within_the_bound_and_columns_without_entries(torch_gpu, handle, oracle, dtype):
     # 200 rows of 30 entries over 70001 columns: most columns have no entry and must still get beta * y
     a = wl.random_ragged(200, 70001, 30, dtype=dtype, seed=5, empty_fraction=0.5)
