@@ -134,6 +134,10 @@ __device__ __forceinline__ T load_stream(const T* p) {
     return __builtin_nontemporal_load(p);
 }
 
+// A value the compiler cannot trace back: what is worked out from it again costs an instruction and not a register held
+// from the first time on.
+__device__ __forceinline__ void forget(uint32_t& v) { asm volatile("" : "+v"(v)); }
+
 // beta*old + alpha*sum of an SpMM, rounded the same way in every kernel that writes C (left to the compiler it is the one or
 // the other product that goes into the fused operation unrounded).
 template <typename T>

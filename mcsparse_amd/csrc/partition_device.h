@@ -89,10 +89,6 @@ __device__ __forceinline__ bool in_slab(uint32_t items, uint32_t i, uint32_t cou
     return static_cast<int>(slab_place(items, 0)) < static_cast<int>(count) - static_cast<int>(i * kWave);
 }
 
-// A value the compiler cannot trace back: what is worked out from it again costs an instruction and not a register held
-// from the first time on.
-__device__ __forceinline__ void forget(uint32_t& v) { asm volatile("" : "+v"(v)); }
-
 // array[index] for arrays of less than 4 GiB: a scalar base and a 32-bit offset.
 template <typename W>
 __device__ __forceinline__ W load_at(const void* array, uint32_t index) {

@@ -59,14 +59,15 @@ __global__ void zero_strip_counters_kernel(StripCounters* c, uint32_t stride) {
 
 // Rows of a group: strip q has the rows first + q * stride + [0, rows).  Where the stride is no multiple of H the last group of
 // a stretch has fewer than H rows in each of its strips.
+__device__ __forceinline__ uint32_t rows_of_strip(uint32_t in_tile, uint32_t stride) { return min(stride - in_tile, static_cast<uint32_t>(H)); }
 struct GroupRows {
-    uint64_t first;
+    uint32_t first;  // (below 1.5 m)
     uint32_t rows;
-    __device__ __forceinline__ GroupRows(uint64_t group, uint32_t stride) {
-        const uint64_t per_tile = (stride + H - 1) / H;  // groups in a stretch of Q * stride rows
-        const uint32_t in_tile = static_cast<uint32_t>(group % per_tile) * H;
-        first = group / per_tile * (static_cast<uint64_t>(Q) * stride) + in_tile;
-        rows = min(stride - in_tile, static_cast<uint32_t>(H));
+    __device__ __forceinline__ GroupRows(uint32_t group, uint32_t stride) {
+        const uint32_t per_tile = (stride + H - 1) / H;  // groups in a stretch of Q * stride rows
+        const uint32_t in_tile = group % per_tile * H;
+        first = group / per_tile * (Q * stride) + in_tile;
+        rows = rows_of_strip(in_tile, stride);
     }
 };
 
@@ -115,8 +116,8 @@ __global__ __launch_bounds__(kBlock) void strip_cover_kernel(idx_t m, idx_t nnz,
     int longest_strip = 0;
     if (group < groups) {
         // (a row that the strip does not have is empty and lies where the strip ends)
-        const GroupRows g(group, stride);
-        const uint64_t row = min(g.first + static_cast<uint64_t>(lane / H) * stride + min(lane % H, g.rows), static_cast<uint64_t>(m));
+        const GroupRows g(static_cast<uint32_t>(group), stride);
+        const uint64_t row = min(static_cast<uint64_t>(g.first) + static_cast<uint64_t>(lane / H) * stride + min(lane % H, g.rows), static_cast<uint64_t>(m));
         const bool exists = lane % H < g.rows && row < static_cast<uint64_t>(m);
         idx_t i = row_ptr[row] - base;
         const idx_t e = exists ? row_ptr[row + 1] - base : i;
@@ -350,9 +351,9 @@ __global__ __launch_bounds__(kStripBlock, 3) void spmm_strips_kernel(idx_t m, id
     const uint64_t groups = spmm_strip_groups(m, stride);
     if (turn >= groups) return;  // whole lane groups
     // which group takes this turn (held to the groups that exist, whatever the buffer holds)
-    const uint64_t group = min(static_cast<uint64_t>(order[turn]), groups - 1);
+    const uint32_t group = min(order[turn], static_cast<uint32_t>(groups - 1));
     const GroupRows rows_of(group, stride);
-    const uint64_t g0 = rows_of.first;
+    uint32_t g0 = rows_of.first;
     // lanes past the last column only help fetching
     const LaneColumns own = lane_columns<V, RAGGED>((static_cast<uint64_t>(blockIdx.y) * kLanes + lane) * V, n);
     const uint64_t c0 = own.first;
@@ -368,7 +369,7 @@ __global__ __launch_bounds__(kStripBlock, 3) void spmm_strips_kernel(idx_t m, id
     const off_t ldb_bytes = static_cast<off_t>(ldb * sizeof(T));
 
     // this lane's row of the group: where its nonzeros begin and end (a row that the strip or the matrix does not have holds none)
-    const uint64_t my_row = g0 + static_cast<uint64_t>(lane / H) * stride + min(lane % H, rows_of.rows);
+    const uint64_t my_row = static_cast<uint64_t>(g0) + static_cast<uint64_t>(lane / H) * stride + min(lane % H, rows_of.rows);
     const uint64_t row_at = my_row < static_cast<uint64_t>(m) ? my_row : static_cast<uint64_t>(m);
     const bool row_exists = lane % H < rows_of.rows && my_row < static_cast<uint64_t>(m);
     const idx_t row_begin = row_ptr[row_at] - base;
@@ -384,7 +385,7 @@ __global__ __launch_bounds__(kStripBlock, 3) void spmm_strips_kernel(idx_t m, id
         // The schedule lives in the caller's buffer.  Whatever it holds, nothing is read outside the arrays: list
         // bounds are held to the list, a block whose rows of op(B) do not all exist counts as a block that holds
         // nothing, value positions are held to the copy in LDS or to the nonzeros.
-        const uint32_t s_end = min(block_ptr[group + 1], total_blocks);
+        const uint32_t s_end = min(block_ptr[group + 1ull], total_blocks);
         const uint32_t s_begin = min(block_ptr[group], s_end);
         const idx_t last_value = nnz - 1;  // nnz != 0: total_blocks != 0
         const uint32_t last_block = total_blocks - 1;
@@ -579,23 +580,30 @@ __global__ __launch_bounds__(kStripBlock, 3) void spmm_strips_kernel(idx_t m, id
         });
     }
 
-    if (!own.any) return;
+    // Where the group and the lane lie, worked out again: held through the loop it costs registers that fp64 has not got (128 x 128 x
+    // 60, 36, 64 and 128 columns 383, 378, 729 us, and 373, 365, 713 so).
+    static_assert(kStripBlock == kWave, "a thread's number is its lane's");
+    const uint32_t end_lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) % kLanes;
+    forget(g0);
+    const LaneColumns stored = lane_columns<V, RAGGED>((static_cast<uint64_t>(blockIdx.y) * kLanes + end_lane) * V, n);
+    if (!stored.any) return;
+    const uint32_t rows = stride % H == 0 ? static_cast<uint32_t>(H) : rows_of_strip(g0 % (Q * stride), stride);
     // A column-major C holds the rows of a strip next to each other in every column: 16 or 32 bytes.
     const bool whole_columns = !RAGGED && !c_row_major && stride % H == 0 &&
                                ((reinterpret_cast<uintptr_t>(C) | static_cast<uintptr_t>(ldc * sizeof(T))) & 15u) == 0;
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-        const uint64_t strip_row = g0 + static_cast<uint64_t>(q) * stride;
+        const uint64_t strip_row = static_cast<uint64_t>(g0) + static_cast<uint64_t>(q) * stride;
         if (whole_columns && strip_row + H <= static_cast<uint64_t>(m)) {
 #pragma unroll
             for (int c = 0; c < V; ++c)
-                store_c_four_rows<T>(C + static_cast<int64_t>(c0 + c) * ldc + strip_row, acc[q * H][c], acc[q * H + 1][c],
+                store_c_four_rows<T>(C + static_cast<int64_t>(stored.first + c) * ldc + strip_row, acc[q * H][c], acc[q * H + 1][c],
                                      acc[q * H + 2][c], acc[q * H + 3][c], alpha, beta);
         } else {
 #pragma unroll
             for (int h = 0; h < H; ++h) {
-                if (static_cast<uint32_t>(h) < rows_of.rows && strip_row + h < static_cast<uint64_t>(m))
-                    store_c<T, V>(C, ldc, c_row_major, strip_row + h, c0, acc[q * H + h], alpha, beta, own.skip);
+                if (static_cast<uint32_t>(h) < rows && strip_row + h < static_cast<uint64_t>(m))
+                    store_c<T, V>(C, ldc, c_row_major, strip_row + h, stored.first, acc[q * H + h], alpha, beta, stored.skip);
             }
         }
     }
