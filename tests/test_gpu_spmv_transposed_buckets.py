@@ -1,7 +1,7 @@
 """GPU parity of the transposing mcsparseSpMV without a preprocess call (CSR op T, CSC op N, COO op T).
 
-With more than 2^14 and at most 2^22 columns and any algorithm but MCSPARSE_SPMV_CSR_ALG2 the call orders the
-products value * x[row] by the top eight bits of their column only and forms the sums of each bucket of columns in
+With more than 2^14 and at most 1024 * 18432 columns and any algorithm but MCSPARSE_SPMV_CSR_ALG2 the call orders the
+products value * x[row] by the bucket of their column only and forms the sums of each bucket of columns in
 LDS, in the order the products arrive; with at most 2^14 columns and many nonzeros in each it orders nothing and
 sums into copies of y in LDS; otherwise, and under ALG2, it sorts the products completely and adds them in row
 order.  Integer-valued operands make every order of summation exact, so those cases are compared bit for
@@ -54,8 +54,8 @@ def integer_valued(a, seed):
 @pytest.mark.parametrize("base", [0, 1])
 @pytest.mark.parametrize("n", [16384, 16385, 100003, 1 << 20, 1 << 22, (1 << 22) + 1])
 def test_exact_on_integers_across_the_key_range(torch_gpu, handle, dtype, base, n):
-    # 16384 columns with few nonzeros each take the full sort, 16385 are the first bucketed shape, 2^22 the last one;
-    # the index base does not count
+    # 16384 columns with few nonzeros each take the full sort, 16385 are the first bucketed shape; 2^22 are buckets of
+    # 16384; the index base does not count
     a = wl.random_ragged(3001, n, 40, dtype=dtype, seed=n % 97 + base, base=base)
     x, y = integer_valued(a, n)
     want = 2 * (a.to_scipy().T.astype(np.float64) @ x.astype(np.float64)) - 3 * y
