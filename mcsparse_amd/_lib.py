@@ -118,6 +118,8 @@ PROTOTYPES = {
     "mcsparseSpMatGetSpMVPlan": (c_int, [vp, P(c_int), P(c_int)]),
     "mcsparseSpMatSetSpMVPlan": (c_int, [vp, c_int, c_int]),
     "mcsparseSpMatGetSpMMSchedule": (c_int, [vp, P(c_int), P(c_i64)]),
+    "mcsparseSpMatGetSpMMKernel": (c_int, [vp, P(c_int)]),
+    "mcsparseSpMatSetSpMMSchedule": (c_int, [vp, c_int]),
 }
 
 _lib = None

@@ -185,6 +185,17 @@ class SpMat:
         check(self.lib.mcsparseSpMatGetSpMMSchedule(self._d, ctypes.byref(state), ctypes.byref(entries)))
         return state.value, entries.value
 
+    def spmm_kernel(self):
+        """Which kernel the last mcsparseSpMM took: 1 = without a schedule, 2, 3, 4 = the schedule of that state, 5 = the
+        diagonals, 6 = without a schedule, in panels; 0 = no product yet."""
+        kernel = ctypes.c_int()
+        check(self.lib.mcsparseSpMatGetSpMMKernel(self._d, ctypes.byref(kernel)))
+        return kernel.value
+
+    def set_spmm_schedule(self, use):
+        """1: mcsparseSpMM takes the schedule wherever the operands allow it; 0: where it is the faster way."""
+        check(self.lib.mcsparseSpMatSetSpMMSchedule(self._d, use), "mcsparseSpMatSetSpMMSchedule")
+
     def destroy(self):
         if self._d:
             self.lib.mcsparseDestroySpMat(self._d)

@@ -594,6 +594,7 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
     const int64_t batches = C->batchCount;
     const bool shared_structure = A->offsetsBatchStride == 0 && A->batchStride == 0;
     const size_t idx_bytes = wide_indices(A) ? sizeof(int64_t) : sizeof(idx_t);
+    SpmmKernel kernel = kSpmmNone;
     for (int64_t b = 0; b < batches; ++b) {
         mcsparseSpMatDescr Ab = *A;  // this batch's view of A
         const int64_t rows_stride = A->format == MCSPARSE_FORMAT_CSR ? A->offsetsBatchStride : A->batchStride;
@@ -678,6 +679,7 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
             A->schedule.diagonals != 0 && A->schedule.diagonals_value_bytes == sizeof(T) &&
             mcsp::spmm_diagonals_usable(a.m, a.k, a.n, A->schedule.longest_slice, sizeof(T))) {
             mcsp::launch_spmm_diagonals<T>(h->stream, a, A->schedule.diagonals, buf + A->schedule.diagonals_at, h_alpha, h_beta);
+            kernel = kSpmmDiagonals;
             continue;
         }
         T beta_inner = h_beta;
@@ -695,7 +697,7 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
         const bool by_blocks = A->schedule.blocks;
         const bool by_strips = by_blocks && A->schedule.stride != 0;
         auto schedule_usable = [&]() {
-            if (!l.copy_c && !schedule_pays(A->schedule, a, sizeof(T))) return false;
+            if (!l.copy_c && !A->schedule_always && !schedule_pays(A->schedule, a, sizeof(T))) return false;
             if (by_strips) return mcsp::spmm_strips_usable(a, sizeof(T));
             return by_blocks ? mcsp::spmm_blocks_usable(a, sizeof(T)) : mcsp::spmm_schedule_usable(a, sizeof(T));
         };
@@ -713,6 +715,7 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
         }
         // the schedule was built from batch 0's structure
         if (scheduled_here && schedule_usable()) {
+            kernel = by_strips ? kSpmmStrips : by_blocks ? kSpmmBlocks : kSpmmLists;
             if (by_strips)
                 mcsp::launch_spmm_strips<T>(h->stream, a, buffer, A->schedule.stride, A->schedule.entries,
                                             A->schedule.longest_group, A->schedule.mean_span, h_alpha, beta_inner);
@@ -726,8 +729,9 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
         } else if (copy_c && mcsp::launch_spmm_columns<T>(h->stream, a, static_cast<idx_t>(C->col_num), c_user, C->ld,
                                                           h_alpha, h_beta)) {
             copy_c = false;  // written into the caller's C as it lies
+            kernel = kSpmmRows;
         } else {
-            mcsp::launch_spmm<T>(h->stream, a, h_alpha, beta_inner);
+            kernel = mcsp::launch_spmm<T>(h->stream, a, h_alpha, beta_inner);
         }
         if (copy_c) {
             mcsp::launch_transpose_accumulate<T>(h->stream, a.m, static_cast<idx_t>(C->col_num),
@@ -735,6 +739,7 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
                                                  h_beta);
         }
     }
+    A->spmm_kernel.kernel.store(kernel, std::memory_order_relaxed);
     // a launch the runtime refused (a kernel image that does not fit the device) must not pass for a product
     return launches_taken() ? MCSP_STATUS_SUCCESS : MCSP_STATUS_INTERNAL_ERROR;
 }

@@ -401,6 +401,19 @@ mcsparseStatus_t mcsparseSpMatGetSpMMSchedule(mcsparseSpMatDescr_t d, int* state
     return MCSPARSE_STATUS_SUCCESS;
 }
 
+mcsparseStatus_t mcsparseSpMatGetSpMMKernel(mcsparseSpMatDescr_t d, int* kernel) {
+    if (d == nullptr || kernel == nullptr) return to_public_status(MCSP_STATUS_INVALID_POINTER);
+    *kernel = d->spmm_kernel.kernel.load(std::memory_order_relaxed);
+    return MCSPARSE_STATUS_SUCCESS;
+}
+
+mcsparseStatus_t mcsparseSpMatSetSpMMSchedule(mcsparseSpMatDescr_t d, int use) {
+    if (d == nullptr) return to_public_status(MCSP_STATUS_INVALID_POINTER);
+    if (use != 0 && use != 1) return to_public_status(MCSP_STATUS_INVALID_VALUE);
+    d->schedule_always = use == 1;
+    return MCSPARSE_STATUS_SUCCESS;
+}
+
 mcsparseStatus_t mcsparseSpMatGetSpMVPreprocess(mcsparseSpMatDescr_t d, int* state, int* bands, int* rows_per_tile) {
     if (d == nullptr || state == nullptr || bands == nullptr || rows_per_tile == nullptr)
         return to_public_status(MCSP_STATUS_INVALID_POINTER);

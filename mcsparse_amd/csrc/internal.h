@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <atomic>
 #include <cstddef>
 #include <cstdint>
 
@@ -110,6 +111,15 @@ struct SpmmSchedule {
     size_t diagonals_value_bytes = 0;  // the slices' length goes with it
 };
 
+// Which kernel a product took (mcsparseSpMatGetSpMMKernel).
+enum SpmmKernel : int { kSpmmNone = 0, kSpmmRows = 1, kSpmmLists = 2, kSpmmBlocks = 3, kSpmmStrips = 4, kSpmmDiagonals = 5, kSpmmPanels = 6 };
+// The last one of a descriptor, which several threads may multiply by.
+struct LastSpmmKernel {
+    std::atomic<int> kernel{kSpmmNone};
+    LastSpmmKernel() = default;
+    LastSpmmKernel(const LastSpmmKernel& other) : kernel(other.kernel.load(std::memory_order_relaxed)) {}
+};
+
 // Column-banded copy of a CSR matrix built by mcsparseSpMV_preprocess inside the caller's buffer
 // (spmv_banded.hip).  Like the SpMM schedule it is part of the computation, and it holds a copy of the
 // values: SpMV uses it only while the buffer, the three CSR arrays and the extents of the call are the
@@ -187,6 +197,8 @@ struct mcsparseSpMatDescr {
     size_t fixed_length_buffer_size = 0;
     SpmvPlan plan;
     SpmmSchedule schedule;
+    bool schedule_always = false;  // mcsparseSpMatSetSpMMSchedule
+    LastSpmmKernel spmm_kernel;
     SpmvBanded banded;
 };
 
@@ -415,8 +427,9 @@ struct SpmmArgs {
     int64_t long_n = 0;
     void* band_ws = nullptr;  // nnz words more for them, or null
 };
+// Returns kSpmmRows or kSpmmPanels.
 template <typename T>
-void launch_spmm(hipStream_t stream, const SpmmArgs& a, T alpha, T beta);
+SpmmKernel launch_spmm(hipStream_t stream, const SpmmArgs& a, T alpha, T beta);
 // The same into a column-major C of c_cols columns (a.C, a.ldc and a.c_row_major are not looked at), written column by
 // column by the kernel that forms the sums.  false, and nothing launched, where that kernel has no variant: a
 // column-major op(B), one or two or more than sixteen 16-byte vectors per row of it, rows that are taken apart.

@@ -958,7 +958,7 @@ void launch_panels(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
 }
 
 template <typename T, int V>
-void launch_rowb_v(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
+SpmmKernel launch_rowb_v(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     const uint64_t lanes_needed = (static_cast<uint64_t>(a.n) + V - 1) / V;
     if (lanes_needed <= 1) launch_narrow<T, V, 1>(stream, a, alpha, beta);
     else if (lanes_needed <= 2) launch_narrow<T, V, 2>(stream, a, alpha, beta);
@@ -967,15 +967,20 @@ void launch_rowb_v(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     else if (lanes_needed <= 16) launch_rowb<T, 16, V>(stream, a, alpha, beta);
     else if (lanes_needed <= 32) launch_rowb<T, 32, V>(stream, a, alpha, beta);
     else if (V == 1 || a.long_row != 0) launch_rowb<T, 64, V>(stream, a, alpha, beta);
-    else launch_panels<T, V>(stream, a, alpha, beta);
+    else {
+        launch_panels<T, V>(stream, a, alpha, beta);
+        return kSpmmPanels;
+    }
+    return kSpmmRows;
 }
 
 
 }  // namespace
 
 template <typename T>
-void launch_spmm(hipStream_t stream, const SpmmArgs& args, T alpha, T beta) {
-    if (args.m == 0 || args.n == 0) return;
+SpmmKernel launch_spmm(hipStream_t stream, const SpmmArgs& args, T alpha, T beta) {
+    if (args.m == 0 || args.n == 0) return kSpmmNone;
+    SpmmKernel kernel = kSpmmRows;
     SpmmArgs a = args;
     constexpr int kWide = 16 / sizeof(T);  // elements per 128-bit access
     // Rows that begin at any element take the wide loads too (27-point stencil, 872 K rows, fp32: 5, 17, 50, 101
@@ -992,8 +997,8 @@ void launch_spmm(hipStream_t stream, const SpmmArgs& args, T alpha, T beta) {
         if (!a.long_known) a.long_apart = apart;
     }
     if (a.b_row_major) {
-        if (wide) launch_rowb_v<T, kWide>(stream, a, alpha, beta);
-        else launch_rowb_v<T, 1>(stream, a, alpha, beta);
+        if (wide) kernel = launch_rowb_v<T, kWide>(stream, a, alpha, beta);
+        else kernel = launch_rowb_v<T, 1>(stream, a, alpha, beta);
     } else {
         constexpr int kJB = 4;
         const uint64_t blocks = (static_cast<uint64_t>(a.m) + (kBlock / kWave) - 1) / (kBlock / kWave);
@@ -1014,6 +1019,7 @@ void launch_spmm(hipStream_t stream, const SpmmArgs& args, T alpha, T beta) {
     }
     if (a.long_row != 0 && a.long_known && !a.long_cut) launch_spmm_long_find(stream, a, sizeof(T));
     if (a.long_row != 0) launch_spmm_long_rows<T>(stream, a, alpha, beta);
+    return kernel;
 }
 
 SpmmScheduleLayout spmm_schedule_layout(idx_t m, idx_t nnz) {
@@ -1151,7 +1157,7 @@ template void launch_transpose_accumulate<double>(hipStream_t, idx_t, idx_t, con
                                                   double);
 template void launch_spmm_scheduled<float>(hipStream_t, const SpmmArgs&, const void*, uint32_t, uint64_t, float, float);
 template void launch_spmm_scheduled<double>(hipStream_t, const SpmmArgs&, const void*, uint32_t, uint64_t, double, double);
-template void launch_spmm<float>(hipStream_t, const SpmmArgs&, float, float);
-template void launch_spmm<double>(hipStream_t, const SpmmArgs&, double, double);
+template SpmmKernel launch_spmm<float>(hipStream_t, const SpmmArgs&, float, float);
+template SpmmKernel launch_spmm<double>(hipStream_t, const SpmmArgs&, double, double);
 
 }  // namespace mcsp

@@ -308,6 +308,10 @@ def test_spmm_argument_checks(lib):
     assert lib.mcsparseSpMatGetSpMMSchedule(o.A, ctypes.byref(state), ctypes.byref(entries)) == 0
     assert state.value == 0 and entries.value == 0
     assert lib.mcsparseSpMatGetSpMMSchedule(o.A, None, ctypes.byref(entries)) == 3
+    assert lib.mcsparseSpMatGetSpMMKernel(o.A, ctypes.byref(state)) == 0 and state.value == 0
+    assert lib.mcsparseSpMatGetSpMMKernel(o.A, None) == 3 and lib.mcsparseSpMatGetSpMMKernel(None, ctypes.byref(state)) == 3
+    assert [lib.mcsparseSpMatSetSpMMSchedule(o.A, use) for use in (1, 0, 2, -1)] == [0, 0] + 2 * [api.STATUS_INVALID_VALUE]
+    assert lib.mcsparseSpMatSetSpMMSchedule(None, 1) == 3
     for f, need in ((api.FORMAT_COO, 9 * 4), (api.FORMAT_CSC, (9 + 20) * 4 + 20 * 4)):
         o2 = Objs(lib, m=8, n=6, nnz=20, fmt=f)
         assert lib.mcsparseSpMM_bufferSize(o2.h, 0, 0, o2.pa, o2.A, B, o2.pa, C, api.R_32F, 0, ctypes.byref(size)) == 0

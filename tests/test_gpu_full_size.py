@@ -155,7 +155,8 @@ def test_config4_stencil_full_size(torch_gpu, handle, oracle, stencil_full, n, p
     rng = np.random.default_rng(n)
     B = rng.uniform(-1, 1, (a.n, n)).astype(np.float32)
     st, got, _ = run_spmm(torch_gpu, handle, a, B, np.zeros((a.m, n), np.float32), 1.0, 0.0, preprocess=preprocess,
-                          expect_schedule=(2 if n == 8 else 4) if preprocess else None)
+                          expect_schedule=(2 if n == 8 else 4) if preprocess else None,
+                          expect_kernel=(1 if n == 8 else 4) if preprocess else None)
     assert st == 0
     # oracle on a sample of rows: first/last planes, and random interior rows
     rows = np.unique(np.concatenate([np.arange(0, 300), np.arange(a.m - 300, a.m),
@@ -170,3 +171,18 @@ def test_config4_stencil_full_size(torch_gpu, handle, oracle, stencil_full, n, p
     for j in (0, n - 1):
         y_ref, bnd = oracle.spmv(False, a.m, a.n, 0, a.ptr, a.col, a.val, 1.0, 0.0, np.ascontiguousarray(B[:, j]), None)
         assert_within(np.ascontiguousarray(got[:, j]), y_ref, bnd, np.float32, what="C4 N=%d column %d" % (n, j))
+
+
+def test_strips_of_narrow_operands_full_size(torch_gpu, handle, oracle):
+    """Operands of 65 to 128 bytes a row get groups of strips where grid lines end inside groups of eight rows and there are
+    many rows: lines of 102 points (the last group of a stretch has two rows in each strip), 31 columns of 16 lanes' 64."""
+    a = wl.stencil_27pt(102, dtype=np.float32)
+    n = 31
+    rng = np.random.default_rng(n)
+    B = rng.uniform(-1, 1, (a.n, n)).astype(np.float32)
+    st, got, _ = run_spmm(torch_gpu, handle, a, B, np.zeros((a.m, n), np.float32), 1.0, 0.0, preprocess=True, expect_schedule=4,
+                          expect_kernel=4)
+    assert st == 0
+    for j in (0, 15, 16, n - 1):  # all rows: column j of C equals the SpMV of A with column j of B
+        y_ref, bnd = oracle.spmv(False, a.m, a.n, 0, a.ptr, a.col, a.val, 1.0, 0.0, np.ascontiguousarray(B[:, j]), None)
+        assert_within(np.ascontiguousarray(got[:, j]), y_ref, bnd, np.float32, what="102 points, column %d" % j)

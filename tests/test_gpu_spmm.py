@@ -11,11 +11,24 @@ from gpu_util import assert_within, dev
 pytestmark = pytest.mark.gpu
 
 
+def kernel_of_schedule(state, n, dt, ldb, ldc, c_order):
+    """Which kernel a product takes that is told to use a schedule of that state (row-major op(B)), 0 if this does not say."""
+    wide = 16 // np.dtype(dt).itemsize
+    whole = n % wide == 0 and ldb % wide == 0 and (c_order != api.ORDER_ROW or ldc % wide == 0)
+    vectors = {2: 9 if wide == 4 else 17, 3: 5, 4: 5}.get(state)  # least of a row of op(B)
+    if vectors is None or (state != 4 and not whole) or n <= (vectors - 1) * wide:
+        return 0
+    return state
+
+
 def run_spmm(torch, handle, a, B, C0, alpha, beta, op_b=api.OP_N, b_order=api.ORDER_ROW, c_order=api.ORDER_ROW,
-             pad_b=0, pad_c=0, preprocess=False, expect_schedule=None, prepare_for_row_major_c=False, seen=None):
+             pad_b=0, pad_c=0, preprocess=False, expect_schedule=None, prepare_for_row_major_c=False, seen=None,
+             expect_kernel=None):
     """B is the k x n operand op(B); it is stored as the call's (op_b, b_order) pair requires.
     prepare_for_row_major_c: mcsparseSpMM_preprocess is given a row-major C of the same shape, whatever the call's is
-    (a schedule belongs to the structure of A; which kind is built depends on the operands of the preprocess call)."""
+    (a schedule belongs to the structure of A; which kind is built depends on the operands of the preprocess call).
+    expect_schedule: the product takes it wherever the operands allow it.  expect_kernel: the product takes what the library
+    chooses, which is this one."""
     k, n = B.shape
     dt = a.val.dtype
     # memory image of op(B): row-major k x n  <=>  (N, ROW) or (T, COL)
@@ -57,8 +70,13 @@ def run_spmm(torch, handle, a, B, C0, alpha, beta, op_b=api.OP_N, b_order=api.OR
             assert mat.spmm_schedule()[0] in wanted, mat.spmm_schedule()
         if seen is not None:
             seen.add(mat.spmm_schedule()[0])
+        mat.set_spmm_schedule(0 if expect_kernel is not None or expect_schedule is None else 1)
     st = api.spmm(handle, api.OP_N, op_b, alpha, mat, mB, beta, mC, ct, buf)
     torch.cuda.synchronize()
+    if expect_kernel is not None:
+        assert mat.spmm_kernel() == expect_kernel, (mat.spmm_kernel(), expect_kernel)
+    elif expect_schedule is not None and b_row_image:
+        assert mat.spmm_kernel() == (kernel_of_schedule(mat.spmm_schedule()[0], n, dt, ldb, ldc, c_order) or mat.spmm_kernel())
     out = d_C.cpu().numpy()
     if c_order == api.ORDER_ROW:
         got, padding = out[:, :n], out[:, n:]
@@ -228,7 +246,7 @@ def test_schedule_is_dropped_with_other_buffer_or_pointers(torch_gpu, handle, or
     assert mat.spmm_schedule()[0] == 0
 
 
-@pytest.mark.parametrize("grid,n", [(10, 64), (40, 64), (40, 128), (41, 64), (41, 128), (10, 16)])
+@pytest.mark.parametrize("grid,n", [(10, 64), (40, 64), (40, 128), (41, 64), (41, 128), (10, 16), (51, 64), (51, 61)])
 def test_overwritten_schedule_stays_in_bounds(torch_gpu, handle, grid, n):
     """The reference's preprocess is a no-op, so a caller written against it may reuse the scratch
     buffer between preprocess and SpMM.  The schedule is then garbage: the product may be wrong, but
@@ -243,7 +261,9 @@ def test_overwritten_schedule_stays_in_bounds(torch_gpu, handle, grid, n):
     st, size = api.spmm_buffer_size(handle, api.OP_N, api.OP_N, 1.0, mat, mB, 0.0, mC, api.R_32F)
     buf = torch.empty(size, dtype=torch.uint8, device="cuda")
     assert api.spmm_preprocess(handle, api.OP_N, api.OP_N, 1.0, mat, mB, 0.0, mC, api.R_32F, buf) == 0
-    assert mat.spmm_schedule()[0] == (4 if grid == 40 else 3 if grid == 41 else 2), mat.spmm_schedule()
+    state = mat.spmm_schedule()[0]
+    assert state == {10: 2, 40: 4, 41: 3, 51: 4}[grid], mat.spmm_schedule()
+    mat.set_spmm_schedule(1)
     gen = torch.Generator(device="cuda")
     gen.manual_seed(3)
     for fill in (0xFF, None, 0x00):
@@ -253,6 +273,7 @@ def test_overwritten_schedule_stays_in_bounds(torch_gpu, handle, grid, n):
             buf.fill_(fill)
         assert api.spmm(handle, api.OP_N, api.OP_N, 1.0, mat, mB, 0.0, mC, api.R_32F, buf) == 0
         torch.cuda.synchronize()
+        assert mat.spmm_kernel() == (state if n > 32 else 1)
     # a fresh preprocess makes the same buffer good again
     assert api.spmm_preprocess(handle, api.OP_N, api.OP_N, 1.0, mat, mB, 0.0, mC, api.R_32F, buf) == 0
     assert api.spmm(handle, api.OP_N, api.OP_N, 1.0, mat, mB, 0.0, mC, api.R_32F, buf) == 0
@@ -492,6 +513,50 @@ def test_strips_of_lines_that_are_no_whole_number_of_strips(torch_gpu, handle, o
           prepare_for_row_major_c=True)
 
 
+@pytest.mark.parametrize("line", [51, 53, 54])
+@pytest.mark.parametrize("dtype,n", [(np.float32, 17), (np.float32, 18), (np.float32, 20), (np.float32, 31), (np.float32, 32),
+                                     (np.float64, 9), (np.float64, 10), (np.float64, 15), (np.float64, 16)])
+def test_strips_of_narrow_operands(torch_gpu, handle, oracle, dtype, n, line):
+    """Half and more of the sixteen lanes of a group past the last column, the last lane's vector moved back over columns of the
+    lane before; the last group of a stretch with three rows, one and two in each strip.  Prepared for 64 columns."""
+    torch = torch_gpu
+    a = wl.stencil_27pt(line, dtype=dtype)
+    rng = np.random.default_rng(n)
+    B = rng.uniform(-1, 1, (a.n, n)).astype(dtype)
+    d_ptr, d_col, d_val, d_B = dev(torch, a.ptr), dev(torch, a.col), dev(torch, a.val), dev(torch, B)
+    d_C = torch.full((a.m, n + 1), 99.0, dtype=d_B.dtype, device="cuda")
+    wide = torch.zeros((a.m, 64), dtype=d_B.dtype, device="cuda")
+    mat = api.SpMat(a.m, a.n, a.nnz, d_ptr, d_col, d_val)
+    mW, ct = api.DnMat(a.m, 64, 64, wide), api.maca_type(np.dtype(dtype))
+    mB, mC = api.DnMat(a.n, n, n, d_B), api.DnMat(a.m, n, n + 1, d_C)
+    st, size = api.spmm_buffer_size(handle, api.OP_N, api.OP_N, 1.0, mat, mW, 0.0, mW, ct)
+    assert st == 0
+    buf = torch.empty(size, dtype=torch.uint8, device="cuda")
+    assert api.spmm_preprocess(handle, api.OP_N, api.OP_N, 1.0, mat, mW, 0.0, mW, ct, buf) == 0
+    mat.set_spmm_schedule(1)
+    assert api.spmm(handle, api.OP_N, api.OP_N, 1.0, mat, mB, 0.0, mC, ct, buf) == 0
+    torch.cuda.synchronize()
+    assert mat.spmm_kernel() == 4
+    got = d_C.cpu().numpy()
+    assert (got[:, n:] == 99.0).all()
+    c_ref, bound = oracle.spmm(a.m, n, 0, a.ptr, a.col, a.val, 1.0, 0.0, B.ravel(), n, True, None, n, True)
+    assert_within(np.ascontiguousarray(got[:, :n]), c_ref, bound, dtype)
+
+
+@pytest.mark.parametrize("n", [17, 20, 24, 32])
+def test_blocks_of_narrow_operands(torch_gpu, handle, oracle, n):
+    """Rows of op(B) of 65 to 128 bytes, more than 100,000 rows and no line that ends inside a group of eight: blocks."""
+    m = 100003
+    offsets = np.array([-9, -8, -7, -1, 0, 1, 7, 8, 9])
+    col = np.arange(m)[:, None] + offsets
+    kept = (col >= 0) & (col < m)
+    ptr = np.concatenate([[0], np.cumsum(kept.sum(1))]).astype(np.int32)
+    rng = np.random.default_rng(n)
+    a = wl.Csr(m, m, ptr, col[kept].astype(np.int32), rng.uniform(-1, 1, int(ptr[-1])).astype(np.float32))
+    check(torch_gpu, handle, oracle, a, n, 1.0, 0.0, preprocess=True, expect_schedule=3, expect_kernel=3 if n % 4 == 0 else 1)
+    check(torch_gpu, handle, oracle, a.with_base(1), n, -0.5, 1.5, preprocess=True, expect_schedule=3, pad_b=4, pad_c=8)
+
+
 @pytest.mark.parametrize("dtype,n", [(np.float32, 129), (np.float32, 133), (np.float32, 150), (np.float32, 190), (np.float32, 253),
                                      (np.float32, 384), (np.float64, 65), (np.float64, 67), (np.float64, 75), (np.float64, 90),
                                      (np.float64, 127), (np.float64, 192)])
@@ -548,8 +613,10 @@ def test_blocks_with_a_value_array_that_is_not_16_byte_aligned(torch_gpu, handle
     buf = torch.empty(size, dtype=torch.uint8, device="cuda")
     assert api.spmm_preprocess(handle, api.OP_N, api.OP_N, 1.0, mat, mB, 0.0, mC, api.R_32F, buf) == 0
     assert mat.spmm_schedule()[0] == state
+    mat.set_spmm_schedule(1)
     assert api.spmm(handle, api.OP_N, api.OP_N, 1.0, mat, mB, 0.0, mC, api.R_32F, buf) == 0
     torch.cuda.synchronize()
+    assert mat.spmm_kernel() == state
     c_ref, bound = oracle.spmm(a.m, n, 0, a.ptr, a.col, a.val, 1.0, 0.0, B.ravel(), n, True, np.zeros(a.m * n, np.float32),
                                n, True)
     assert_within(d_C.cpu().numpy(), c_ref, bound, np.float32)
@@ -597,10 +664,12 @@ def test_blocks_schedule_used_with_a_wider_operand_than_it_was_built_for(torch_g
     buf = torch.empty(max(sizes.values()), dtype=torch.uint8, device="cuda")
     assert api.spmm_preprocess(handle, api.OP_N, api.OP_N, 1.0, mat, ops[64][3], 0.0, ops[64][4], api.R_32F, buf) == 0
     assert mat.spmm_schedule()[0] == state
+    mat.set_spmm_schedule(1)
     for n in (64, 256, 8):
         B, d_B, d_C, mB, mC = ops[n]
         assert api.spmm(handle, api.OP_N, api.OP_N, 1.0, mat, mB, 0.0, mC, api.R_32F, buf) == 0
         torch.cuda.synchronize()
+        assert mat.spmm_kernel() == (state if n != 8 else 1)
         c_ref, bound = oracle.spmm(a.m, n, 0, a.ptr, a.col, a.val, 1.0, 0.0, B.ravel(), n, True,
                                    np.zeros(a.m * n, np.float32), n, True)
         assert_within(d_C.cpu().numpy(), c_ref, bound, np.float32, what="n=%d" % n)
