@@ -659,6 +659,7 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
                 if (A->plan.valid && A->plan.forced_family == kFamilyAuto) {
                     may_have_long_rows = A->plan.max_row_len > mcsp::kSpmmLongRow;
                     a.long_known = true;
+                    a.longest_row = A->plan.max_row_len;
                 }
             }
             if (!may_have_long_rows) {
@@ -731,6 +732,7 @@ mcspStatus_t spmm_typed(mcsparseHandle_t h, mcsparseSpMatDescr* A, mcsparseOpera
             copy_c = false;  // written into the caller's C as it lies
             kernel = kSpmmRows;
         } else {
+            a.shared_rows = scheduled_here && by_blocks;
             kernel = mcsp::launch_spmm<T>(h->stream, a, h_alpha, beta_inner);
         }
         if (copy_c) {

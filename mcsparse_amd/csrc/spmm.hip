@@ -939,7 +939,7 @@ void launch_rowb(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
 // Rows of op(B) of more than 512 bytes, panel after panel: all rows for the first 512 bytes, ..., for what is left.  (A whole row to
 // 64 lanes: its columns are read once, but a wavefront has one row in flight instead of two, lanes past the last column idle, and
 // neighbouring rows of A find less of what they share in L2.  Fp64, 66, 96 and 128 columns: 48^3 159, 157, 159 us and 93, 94, 122
-// in panels; 97 x 61 x 97 954, 964, 991 and 533, 569, 748.)
+// in panels; 97 x 61 x 97 954, 964, 991 and 533, 569, 748.  For which matrices and widths: spmm_takes_panels.)
 template <typename T, int V>
 void launch_panels(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     SpmmArgs panels = a, rest = a;
@@ -960,13 +960,15 @@ void launch_panels(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
 template <typename T, int V>
 SpmmKernel launch_rowb_v(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     const uint64_t lanes_needed = (static_cast<uint64_t>(a.n) + V - 1) / V;
+    const bool whole_lines = (reinterpret_cast<uintptr_t>(a.B) | static_cast<uintptr_t>(a.ldb * sizeof(T))) % 128 == 0;
     if (lanes_needed <= 1) launch_narrow<T, V, 1>(stream, a, alpha, beta);
     else if (lanes_needed <= 2) launch_narrow<T, V, 2>(stream, a, alpha, beta);
     else if (lanes_needed <= 4) launch_rowb<T, 4, V>(stream, a, alpha, beta);  // measured faster than four column lanes above
     else if (lanes_needed <= 8) launch_rowb<T, 8, V>(stream, a, alpha, beta);
     else if (lanes_needed <= 16) launch_rowb<T, 16, V>(stream, a, alpha, beta);
     else if (lanes_needed <= 32) launch_rowb<T, 32, V>(stream, a, alpha, beta);
-    else if (V == 1 || a.long_row != 0) launch_rowb<T, 64, V>(stream, a, alpha, beta);
+    else if (V == 1 || a.long_row != 0 || !spmm_takes_panels(a.n * sizeof(T), a.m, a.nnz, a.longest_row, a.shared_rows, whole_lines))
+        launch_rowb<T, 64, V>(stream, a, alpha, beta);
     else {
         launch_panels<T, V>(stream, a, alpha, beta);
         return kSpmmPanels;

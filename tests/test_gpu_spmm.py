@@ -557,15 +557,51 @@ def test_blocks_of_narrow_operands(torch_gpu, handle, oracle, n):
     check(torch_gpu, handle, oracle, a.with_base(1), n, -0.5, 1.5, preprocess=True, expect_schedule=3, pad_b=4, pad_c=8)
 
 
-@pytest.mark.parametrize("dtype,n", [(np.float32, 129), (np.float32, 133), (np.float32, 150), (np.float32, 190), (np.float32, 253),
-                                     (np.float32, 384), (np.float64, 65), (np.float64, 67), (np.float64, 75), (np.float64, 90),
-                                     (np.float64, 127), (np.float64, 192)])
+@pytest.mark.parametrize("dtype,n", [(np.float32, 129), (np.float32, 133), (np.float32, 150), (np.float32, 190), (np.float32, 192),
+                                     (np.float64, 65), (np.float64, 67), (np.float64, 75), (np.float64, 90), (np.float64, 96)])
+def test_what_is_left_behind_panels_of_512_bytes(torch_gpu, handle, oracle, dtype, n):
+    """Prepared, so that the call knows that neighbouring rows share columns, but too small for the schedule to pay: panels of
+    512 bytes, and what is left in every width it can have."""
+    a = wl.stencil_27pt(27, dtype=dtype)
+    check(torch_gpu, handle, oracle, a, n, 1.0, 0.0, preprocess=True, expect_schedule=3, expect_kernel=6)
+    check(torch_gpu, handle, oracle, a.with_base(1), n, -0.5, 1.5, preprocess=True, expect_schedule=3, expect_kernel=6, pad_b=1, pad_c=3)
+
+
+@pytest.mark.parametrize("dtype,n", [(np.float32, 256), (np.float32, 320), (np.float32, 384), (np.float32, 448), (np.float64, 128),
+                                     (np.float64, 160), (np.float64, 192), (np.float64, 256)])
 def test_rows_of_more_than_512_bytes_in_panels(torch_gpu, handle, oracle, dtype, n):
-    """No preprocess call: panels of 512 bytes, and what is left in every width a panel can have."""
-    a = wl.stencil_27pt(9, dtype=dtype)
+    """No preprocess call: whole panels of 512 bytes, and half a one behind two and three; rows of op(B) that begin inside a line
+    are left whole."""
+    a = wl.stencil_27pt(27, dtype=dtype)
     for c_order in (api.ORDER_ROW, api.ORDER_COL):
-        check(torch_gpu, handle, oracle, a, n, 1.0, 0.0, c_order=c_order)
-        check(torch_gpu, handle, oracle, a.with_base(1), n, -0.5, 1.5, c_order=c_order, pad_b=1, pad_c=3)
+        check(torch_gpu, handle, oracle, a, n, 1.0, 0.0, c_order=c_order, expect_kernel=6)
+        check(torch_gpu, handle, oracle, a.with_base(1), n, -0.5, 1.5, c_order=c_order, pad_b=128, pad_c=3, expect_kernel=6)
+        check(torch_gpu, handle, oracle, a, n, -0.5, 1.5, c_order=c_order, pad_b=1, expect_kernel=1)
+
+
+@pytest.mark.parametrize("dtype,n", [(np.float32, 129), (np.float32, 150), (np.float32, 192), (np.float32, 256), (np.float64, 67),
+                                     (np.float64, 75), (np.float64, 96)])
+def test_short_rows_in_panels(torch_gpu, handle, oracle, dtype, n):
+    """Rows of up to four nonzeros: panels whatever is left behind them, up to half a one."""
+    a = wl.random_ragged(40000, 5000, 3, dtype=dtype, seed=n)
+    assert a.row_lengths().max() * 4096 <= a.nnz
+    check(torch_gpu, handle, oracle, a, n, 1.0, 0.0, expect_kernel=6)
+    check(torch_gpu, handle, oracle, a.with_base(1), n, -0.5, 1.5, pad_b=1, pad_c=3, expect_kernel=6)
+
+
+@pytest.mark.parametrize("dtype,n", [(np.float32, 129), (np.float32, 133), (np.float32, 253), (np.float32, 256), (np.float32, 390),
+                                     (np.float64, 65), (np.float64, 67), (np.float64, 127), (np.float64, 128)])
+def test_rows_of_more_than_512_bytes_whole(torch_gpu, handle, oracle, dtype, n):
+    """Where panels would cost more than they give: what is left behind one, not known to be shared; few rows; one long row."""
+    if n * np.dtype(dtype).itemsize % 512 != 0:
+        check(torch_gpu, handle, oracle, wl.stencil_27pt(27, dtype=dtype), n, 1.0, 0.5, expect_kernel=1, pad_c=1)
+    check(torch_gpu, handle, oracle, wl.stencil_27pt(9, dtype=dtype), n, 1.0, 0.5, expect_kernel=1, pad_c=1)
+    lengths = np.full(4000, 5)
+    lengths[1234] = 900
+    rng = np.random.default_rng(1)
+    col = np.concatenate([np.sort(rng.choice(5000, k, replace=False)) for k in lengths]).astype(np.int32)
+    a = wl.Csr(4000, 5000, np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32), col, rng.uniform(-1, 1, len(col)).astype(dtype))
+    check(torch_gpu, handle, oracle, a, n, 1.0, 0.5, expect_kernel=1)
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
