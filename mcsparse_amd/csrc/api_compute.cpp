@@ -554,11 +554,27 @@ bool schedule_pays(const SpmmSchedule& s, const mcsp::SpmmArgs& a, size_t value_
     constexpr uint64_t kNarrow = 128;  // bytes of a row: half of a strip's lanes
     const uint64_t row_bytes = static_cast<uint64_t>(a.n) * value_bytes, window = s.mean_span * row_bytes;
     if (s.stride == 0) {
-        // groups of eight rows: not where they take in line ends (45 x 47 x 49 points, too few for strips of such lines; 24, 32, 48
-        // fp32 columns 56 and 17, 56 and 18, 60 and 30), nor narrow ones of few rows (27 diagonals, 24 fp32 columns, 30, 60 and 100 K
-        // rows: 14 and 8, 15 and 11, 17 and 16; 125 and 500 K: 19 and 20, 54 and 63)
+        // Groups of eight rows.  The kernel without a schedule takes about this long (200 K and a million rows of five diagonals, 64 fp32
+        // columns, 27 and 136 for 22 and 127; a million of fifteen 216 for 190; 27-point stencil 120 x 60 x 60 133 for 123):
+        const uint64_t groups = mcsp::spmm_block_groups(a.m);
+        const double us = (1.5 * a.m + a.nnz / 8.0) * static_cast<double>(row_bytes) / 4e6;
+        // A group's blocks are one chain, some 0.7 us each, which outlasts a short product: 20 K rows of five diagonals, 64 columns, 5.5
+        // and 4.7, with eight nonzeros more in one row 13.9 and 4.8; 200 K rows 20.3 and 22.3, 128 columns 35 and 49.  Where such groups lie
+        // everywhere the last wavefronts have some (one group in 500: 200 K rows, 64 columns 29.5 and 22.3, a million 117 and 127).
+        const bool everywhere = static_cast<uint64_t>(s.odd_groups) * 1024 > groups;
+        if (us < s.most_blocks * (everywhere ? 4.0 : 1.5)) return false;
+        // Wavefronts with groups of different blocks run them one after the other: 27-point stencils whose lines end inside groups,
+        // which takes a fifth to a quarter of the blocks (97 x 61 x 97 and 127 x 127 x 60, 128 fp32 columns 378 and 345, 686 and 578).
+        // Of many short rows the kernel without a schedule has to write as much: a million of 5 and 15 diagonals, one group in 20, 243
+        // and 309, 337 and 427.
+        constexpr idx_t kManyRows = 1 << 19;
+        const bool short_rows = a.m >= kManyRows && a.nnz / 16 <= a.m;
+        if (static_cast<uint64_t>(s.odd_blocks) * 8 > s.entries && !short_rows) return false;
+        // narrow ones: not of few rows (27 diagonals, 24 fp32 columns, 30, 60 and 100 K rows: 14 and 8, 15 and 11, 17 and 16; 125 and
+        // 500 K: 19 and 20, 54 and 63), nor where there are more than a few such groups (a million rows of five diagonals, none, one, one in
+        // 500: 44 and 45, 44 and 49, 66 and 45)
         constexpr idx_t kNarrowRows = 100000;
-        return !s.lines_cut && (row_bytes > kNarrow || a.m >= kNarrowRows);
+        return row_bytes > kNarrow || (a.m >= kNarrowRows && static_cast<uint64_t>(s.odd_groups) * 4096 <= groups);
     }
     const uint64_t wavefronts = mcsp::spmm_strip_wavefronts(a, s.stride, value_bytes);
     // three to a SIMD are resident at a time
@@ -1256,7 +1272,8 @@ mcsparseStatus_t build_spmm_schedule(mcsparseHandle_t handle, mcsparseSpMatDescr
                                       externalBuffer);
         const uint64_t block_groups = mcsp::spmm_block_groups(m);
         uint32_t blocks = 0;
-        unsigned long long counters[3] = {0, 0, 0};  // span sum, rows of op(B) loaded, longest group (low 32 bits)
+        // span sum, rows of op(B) loaded, longest group and (high 32 bits) most blocks of a group, odd groups and their blocks
+        unsigned long long counters[4] = {0, 0, 0, 0};
         const char* total_slot = static_cast<const char*>(externalBuffer) + l.group_ptr + block_groups * sizeof(uint32_t);
         if (hipMemcpyAsync(&blocks, total_slot, sizeof(blocks), hipMemcpyDeviceToHost, handle->stream) != hipSuccess ||
             hipMemcpyAsync(counters, span_slot, sizeof(counters), hipMemcpyDeviceToHost, handle->stream) != hipSuccess ||
@@ -1272,14 +1289,16 @@ mcsparseStatus_t build_spmm_schedule(mcsparseHandle_t handle, mcsparseSpMatDescr
             // (Their kernel gives sixteen lanes of 16 bytes to a group and writes a column-major C in pieces of four
             // rows: for operands of up to 128 bytes per row, and for a column-major C, the groups of eight rows stay.
             // But where grid lines end inside groups of eight rows, which a block, with one range of rows for each of its
-            // diagonals, cannot say: such a group has five times the blocks, its wavefront takes as much longer, and strips are
-            // faster at 17 fp32 columns already: 20, 24, 32 columns of a 27-point stencil, 127 x 127 x 60, 255, 255, 257 us
+            // diagonals, cannot say: such a group has up to four times the blocks, its wavefront takes as much longer, and strips are
+            // faster at 17 fp32 columns already, where such groups have more than a sixteenth of the blocks (lines of up to 400 points): 20, 24, 32 columns of a 27-point stencil, 127 x 127 x 60, 255, 255, 257 us
             // from groups of eight rows and 129, 129, 129 from strips; with lines of 120 points 93, 94, 101 and 124, 124, 125.
             // With fewer rows, see schedule_pays, they would not be used.)
             constexpr idx_t kNarrowStripRows = 1 << 19;
-            s.lines_cut = static_cast<uint64_t>(counters[2] >> 32) * block_groups >= 2 * static_cast<uint64_t>(blocks) &&
-                          static_cast<uint64_t>(blocks) * 23 > nz;
-            const bool strips_suit = (row_bytes > 128 || (s.lines_cut && m >= kNarrowStripRows)) && matC->order == MCSPARSE_ORDER_ROW;
+            s.most_blocks = static_cast<uint32_t>(counters[2] >> 32);
+            s.odd_groups = static_cast<uint32_t>(counters[3]);
+            s.odd_blocks = static_cast<uint32_t>(counters[3] >> 32);
+            const bool lines_cut = static_cast<uint64_t>(s.odd_blocks) * 16 > blocks;
+            const bool strips_suit = (row_bytes > 128 || (lines_cut && m >= kNarrowStripRows)) && matC->order == MCSPARSE_ORDER_ROW;
             const uint32_t stride = !strips_suit ? 0u
                                                  : strip_stride_of_middle_row(handle->stream, m, static_cast<idx_t>(matA->idxBase),
                                                                               ia.rows, ia.cols);
@@ -1378,7 +1397,7 @@ mcsparseStatus_t mcsparseSpMM_preprocess(mcsparseHandle_t handle, mcsparseOperat
     s.base = static_cast<int>(matA->idxBase);
     s.blocks = false;
     s.stride = 0;
-    s.lines_cut = false;
+    s.most_blocks = s.odd_groups = s.odd_blocks = 0;
     s.diagonals = 0;
     {
         // The kernels that work from a schedule walk every row in one piece; a matrix with rows of thousands of

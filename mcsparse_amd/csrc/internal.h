@@ -102,7 +102,9 @@ struct SpmmSchedule {
     bool blocks = false;   // the schedule holds diagonal blocks (spmm_blocks.hip) instead of merged lists
     uint32_t longest_group = 0;  // blocks: the most nonzeros in one group of rows (strips: in one strip)
     uint32_t stride = 0;   // blocks: != 0 says the groups are strips this many rows apart (spmm_strips.hip)
-    bool lines_cut = false;  // blocks: groups of eight rows take in the ends of grid lines, and need several times the blocks there
+    // blocks of groups of eight rows: the most of one group, and the groups with twice the blocks of those near them or more (they take
+    // in the end of a grid line, or a row of its own kind), and their blocks
+    uint32_t most_blocks = 0, odd_groups = 0, odd_blocks = 0;
     // beside that (whether useful or not), for column-major operands: the diagonals of slices of rows (spmm_diagonals.hip), at
     // diagonals_at of the buffer; 0: none
     uint32_t diagonals = 0;

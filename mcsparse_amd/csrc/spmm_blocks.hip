@@ -31,6 +31,8 @@ struct BlockCounters {
     unsigned long long loads;     // rows of op(B) all blocks load together
     unsigned int longest_group;   // most nonzeros in one group that has blocks
     unsigned int most_blocks;     // of one group
+    unsigned int odd_groups;      // with twice the blocks of a group near them, or more
+    unsigned int odd_blocks;      // of these
 };
 
 __global__ void zero_block_counters_kernel(BlockCounters* c) {
@@ -38,6 +40,8 @@ __global__ void zero_block_counters_kernel(BlockCounters* c) {
     c->loads = 0;
     c->longest_group = 0;
     c->most_blocks = 0;
+    c->odd_groups = 0;
+    c->odd_blocks = 0;
 }
 
 // One thread covers the nonzeros of one group of K rows with blocks.  It merges the rows by the key
@@ -183,10 +187,28 @@ __global__ __launch_bounds__(kWave) void block_cover_kernel(idx_t m, idx_t base,
     if (!FILL) {
         if (group <= groups) block_ptr[group] = count;  // slot `groups` receives the total after the scan
         unsigned long long span = count != 0 ? last_col - first_col : 0;
+        // A group is odd that has twice as many blocks as the wavefront's first quarter: three quarters of the groups may hold a
+        // grid line's end before these count as the rule.
+        uint32_t rank = 0;
+#pragma unroll
+        for (int j = 0; j < kWave; ++j) {
+            const uint32_t other = __builtin_amdgcn_readlane(count, j);
+            rank += other != 0 && (other < count || (other == count && static_cast<uint32_t>(j) < threadIdx.x)) ? 1u : 0u;
+        }
+        const uint32_t with_blocks = __popcll(__ballot(count != 0));
+        const unsigned long long first_quarter = __ballot(count != 0 && rank == with_blocks / 4);
+        uint32_t odd_blocks = 0;
+        unsigned long long odd = 0;
+        if (first_quarter != 0) {
+            const uint32_t usual = __builtin_amdgcn_readlane(count, __builtin_ctzll(first_quarter));
+            odd = __ballot(count >= 2 * usual);
+            odd_blocks = count >= 2 * usual ? count : 0;
+        }
         uint32_t most = count;
 #pragma unroll
         for (int off = kWave / 2; off > 0; off >>= 1) {
             most = max(most, static_cast<uint32_t>(__shfl_xor(static_cast<int>(most), off, kWave)));
+            odd_blocks += __shfl_xor(odd_blocks, off, kWave);
             span += __shfl_xor(span, off, kWave);
             loads += __shfl_xor(loads, off, kWave);
             group_nnz = max(group_nnz, static_cast<uint32_t>(__shfl_xor(static_cast<int>(group_nnz), off, kWave)));
@@ -196,6 +218,10 @@ __global__ __launch_bounds__(kWave) void block_cover_kernel(idx_t m, idx_t base,
             if (loads != 0) atomicAdd(&counters->loads, loads);
             if (group_nnz != 0) atomicMax(&counters->longest_group, group_nnz);
             if (most != 0) atomicMax(&counters->most_blocks, most);
+            if (odd != 0) {
+                atomicAdd(&counters->odd_groups, static_cast<unsigned int>(__popcll(odd)));
+                atomicAdd(&counters->odd_blocks, odd_blocks);
+            }
         }
     }
 }

@@ -440,6 +440,35 @@ def test_blocks_banded_matrix_with_broken_rows(torch_gpu, handle, oracle, dtype,
     check(torch_gpu, handle, oracle, a.with_base(1), n, -0.5, 1.5, preprocess=True, expect_schedule=want, pad_b=4, pad_c=8)
 
 
+def banded_with_odd_rows(m, odd, dtype, further=8):
+    """Five diagonals, and `further` nonzeros more, anywhere, in the rows `odd`."""
+    rng = np.random.default_rng(7)
+    col = np.arange(m)[:, None] + np.arange(-2, 3)
+    kept = (col >= 0) & (col < m)
+    key = np.concatenate([(np.arange(m)[:, None] * m + col)[kept], (np.asarray(odd)[:, None] * m + rng.integers(0, m, (len(odd), further))).ravel()])
+    key = np.unique(key)
+    ptr = np.concatenate([[0], np.cumsum(np.bincount(key // m, minlength=m))]).astype(np.int32)
+    return wl.Csr(m, m, ptr, (key % m).astype(np.int32), rng.uniform(-1, 1, len(key)).astype(dtype))
+
+
+@pytest.mark.parametrize("m,odd_every,dtype,n,kernel",
+                         [(200000, 0, np.float32, 128, 3), (200000, 200000, np.float32, 128, 3), (200000, 200000, np.float64, 64, 3),
+                          (200000, 200000, np.float32, 64, 3), (200000, 4000, np.float32, 64, 1), (600000, 4000, np.float32, 128, 3),
+                          (600000, 160, np.float32, 128, 3), (20000, 20000, np.float32, 64, 1), (200000, 200000, np.float32, 24, 1)])
+def test_blocks_of_a_matrix_with_odd_rows(torch_gpu, handle, oracle, m, odd_every, dtype, n, kernel):
+    """A few groups with many times the blocks of the others do not keep a large product from the blocks; they do keep a small one,
+    which such a group would outlast, and one where they are everywhere."""
+    odd = np.arange(odd_every // 2, m, odd_every) // 8 * 8 + 3 if odd_every else np.zeros(0, np.int64)
+    a = banded_with_odd_rows(m, odd, dtype)
+    check(torch_gpu, handle, oracle, a, n, 1.5, 0.0, preprocess=True, expect_schedule=3, expect_kernel=kernel)
+
+
+@pytest.mark.parametrize("line,n", [(41, 48), (41, 64), (46, 128)])
+def test_blocks_that_take_in_line_ends_are_left(torch_gpu, handle, oracle, line, n):
+    a = wl.stencil_27pt(line, dtype=np.float32)
+    check(torch_gpu, handle, oracle, a, n, 1.0, 0.0, preprocess=True, expect_schedule=3, expect_kernel=1)
+
+
 def test_blocks_row_ignores_rows_of_b_only_its_neighbours_use(torch_gpu, handle):
     """A block loads rows of op(B) for all its rows of A; a row must only see the ones it names (0 * inf = NaN)."""
     m = 64
