@@ -547,8 +547,8 @@ SpmmLayout spmm_layout(const mcsparseSpMatDescr* A, const mcsparseDnMatDescr* B,
 }
 
 // Whether a product with a row-major op(B) and C takes less time from its diagonal blocks than from the kernel without a schedule,
-// which has more wavefronts in flight for the same rows.  Where lines are a whole number of strips, and operands of more than 128
-// bytes a row begin at whole vectors, it is left at the strips.  Microseconds with a schedule and without, 27-point stencils:
+// which has more wavefronts in flight for the same rows.  Where lines are a whole number of strips, and rows of op(B), of more than 128
+// bytes, are whole vectors, it is left at the strips.  Microseconds with a schedule and without, 27-point stencils:
 bool schedule_pays(const SpmmSchedule& s, const mcsp::SpmmArgs& a, size_t value_bytes) {
     if (!s.blocks) return true;
     constexpr uint64_t kNarrow = 128;  // bytes of a row: half of a strip's lanes
@@ -585,12 +585,19 @@ bool schedule_pays(const SpmmSchedule& s, const mcsp::SpmmArgs& a, size_t value_
     constexpr uint64_t kNarrowWindow = 2000000;
     if (row_bytes <= kNarrow) return wavefronts >= kThriceFull && window >= kNarrowWindow;
     // 61 x 55 x 59, fp32, 64 and 128 columns, 3100 and 6200 wavefronts, 65 and 62, 104 and 107; 150 x 150 x 12, 64 columns, 4400
-    // wavefronts, 11 MB: 65 and 102.  Rows that begin at any element cost the strips a third line to a load: fp64, 61 x 55 x 59 and
-    // 64 x 64 x 64, 57 columns, 6200 and 8200 wavefronts, 139 and 113, 169 and 146; 97 x 61 x 97, 18500 wavefronts, 340 and 374.
+    // wavefronts, 11 MB: 65 and 102.
     constexpr uint64_t kL2 = 4 << 20;
-    const bool whole_vectors = row_bytes % 16 == 0;
-    if (whole_vectors && s.stride % mcsp::kSpmmStripRows == 0) return true;
-    return wavefronts >= (whole_vectors ? kTwiceFull : kThriceFull) || window > kL2;
+    if (mcsp::spmm_strips_whole_vectors(a, value_bytes))
+        return s.stride % mcsp::kSpmmStripRows == 0 || wavefronts >= kTwiceFull || window > kL2;
+    // Rows that begin or end at any element, by the rows of A alone (a panel more is as much more work for both): 76^3, 6900 wavefronts, 64
+    // and 128 fp32 columns 103 and 150, 261 and 295; 64^3, 4100 wavefronts, 75 and 62, 175 and 128; 60 x 56 x 60, 64 fp64 columns 133 and 117.
+    // Fewer where the rows of op(B) that a group reads have left the L2s: 100 x 100 x 20, 3100 wavefronts, 5.0 MB, 64 columns 52 and 65, 10
+    // MB, 128 columns 118 and 159; 120 x 120 x 12, 2700 wavefronts, 7.4 MB, 32 fp64 columns 58 and 53, 15 MB, 64 columns 109 and 126; 72^3,
+    // 5800 wavefronts, 5.5 MB, 128 fp32 columns 221 and 203.
+    constexpr uint64_t kPanel = 256, kFew = 3072, kOnePanelWindow = 4500000, kPanelsWindow = 8000000;
+    const uint64_t of_a_panel = wavefronts / ((row_bytes + kPanel - 1) / kPanel);
+    if (of_a_panel >= kTwiceFull) return true;
+    return row_bytes > kPanel ? window > kPanelsWindow : of_a_panel >= kFew && window > kOnePanelWindow;
 }
 
 template <typename T>

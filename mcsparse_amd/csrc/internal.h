@@ -552,6 +552,8 @@ void launch_spmm_strip_fill(hipStream_t stream, idx_t m, idx_t nnz, idx_t base, 
 bool spmm_strip_schedule_fits(idx_t m, idx_t nnz, uint32_t stride, uint32_t blocks);
 // Any row-major op(B) of at least five 128-bit vectors a row, wherever its rows and those of C begin.
 bool spmm_strips_usable(const SpmmArgs& a, size_t value_bytes);
+// Rows of op(B) begin and end at whole 16-byte vectors: else its kernel reads them from any element, at a third line to a load.
+bool spmm_strips_whole_vectors(const SpmmArgs& a, size_t value_bytes);
 // How many wavefronts such a product is.
 uint64_t spmm_strip_wavefronts(const SpmmArgs& a, uint32_t stride, size_t value_bytes);
 template <typename T>

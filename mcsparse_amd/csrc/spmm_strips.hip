@@ -611,10 +611,6 @@ __global__ __launch_bounds__(kStripBlock, 3) void spmm_strips_kernel(idx_t m, id
 
 // The strip schedule inside the region spmm_schedule_layout describes: the offsets where the merged lists keep
 // theirs, the blocks from the start of the entries' place, the order of the groups at its end.
-bool whole_vectors(const SpmmArgs& a, size_t value_bytes) {
-    const int64_t wide = static_cast<int64_t>(16 / value_bytes);
-    return reinterpret_cast<uintptr_t>(a.B) % 16 == 0 && a.ldb % wide == 0 && a.n % wide == 0;
-}
 struct Carved {
     uint32_t* block_ptr;
     StripCounters* counters;
@@ -638,6 +634,11 @@ bool spmm_strips_usable(const SpmmArgs& a, size_t value_bytes) {
     // at least five 128-bit vectors per row, as for the blocks over eight rows
     return a.b_row_major && a.n >= 4 * static_cast<int64_t>(16 / value_bytes) + 1 && a.k <= kSpmmMaxScheduledColumns &&
            a.m < (idx_t(1) << 31);
+}
+
+bool spmm_strips_whole_vectors(const SpmmArgs& a, size_t value_bytes) {
+    const int64_t wide = static_cast<int64_t>(16 / value_bytes);
+    return reinterpret_cast<uintptr_t>(a.B) % 16 == 0 && a.ldb % wide == 0 && a.n % wide == 0;
 }
 
 uint64_t spmm_strip_wavefronts(const SpmmArgs& a, uint32_t stride, size_t value_bytes) {
@@ -713,7 +714,7 @@ void launch_spmm_strips(hipStream_t stream, const SpmmArgs& a, const void* sched
                            c.order, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta, xcd_chunk, xcds, a.k, a.nnz, total_blocks);
     };
     auto launch = [&](auto wide_c, auto staged_c) {
-        if (whole_vectors(a, sizeof(T))) launch_kind(wide_c, staged_c, std::false_type{});
+        if (spmm_strips_whole_vectors(a, sizeof(T))) launch_kind(wide_c, staged_c, std::false_type{});
         else launch_kind(wide_c, staged_c, std::true_type{});
     };
     if (narrow_offsets(a, sizeof(T))) {

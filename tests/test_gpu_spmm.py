@@ -542,6 +542,16 @@ def test_strips_of_lines_that_are_no_whole_number_of_strips(torch_gpu, handle, o
           prepare_for_row_major_c=True)
 
 
+@pytest.mark.parametrize("line,dtype,n,pad_b,kernel", [(64, np.float32, 128, 0, 4), (64, np.float32, 128, 1, 1), (64, np.float32, 128, 2, 1),
+                                                       (64, np.float64, 64, 1, 1), (64, np.float64, 64, 2, 4), (40, np.float32, 64, 3, 1),
+                                                       (76, np.float32, 64, 1, 4), (76, np.float64, 33, 0, 4)])
+def test_strips_are_left_where_rows_begin_at_any_element(torch_gpu, handle, oracle, line, dtype, n, pad_b, kernel):
+    """Whole lines.  What counts is where the rows of op(B) begin, not how many columns they have: with an odd leading dimension the
+    kernel without a schedule is the faster one for few rows of A."""
+    a = wl.stencil_27pt(line, dtype=dtype)
+    check(torch_gpu, handle, oracle, a, n, 1.0, 0.0, preprocess=True, expect_schedule=4, pad_b=pad_b, expect_kernel=kernel)
+
+
 @pytest.mark.parametrize("line", [51, 53, 54])
 @pytest.mark.parametrize("dtype,n", [(np.float32, 17), (np.float32, 18), (np.float32, 20), (np.float32, 31), (np.float32, 32),
                                      (np.float64, 9), (np.float64, 10), (np.float64, 15), (np.float64, 16)])
