@@ -1224,26 +1224,28 @@ mcsparseStatus_t mcsparseSpMM_bufferSize(mcsparseHandle_t handle, mcsparseOperat
 // structure of A alone; the values of A may change freely.
 namespace {
 
-// The distance, in rows, at which the strips of a strip schedule would lie for this matrix, or 0: the smallest
-// distance between the beginnings of two runs of consecutive diagonals in the middle row that is a whole number of
-// strips and leaves the matrix at least eight such stretches (a 27-point stencil on a grid of lines of 128 points
+// The distances, in rows, at which the strips of a strip schedule might lie for this matrix, or 0: the smallest
+// distance between the beginnings of two runs of consecutive diagonals in the middle row that a schedule can be built with
+// (spmm_strip_stride_usable), and the smallest that is a whole number of strips (a 27-point stencil on a grid of lines of 128 points
 // has runs of three diagonals 128 apart).  Reads the row back: blocks.
-uint32_t strip_stride_of_middle_row(hipStream_t stream, idx_t m, idx_t base, const idx_t* row_ptr, const idx_t* col) {
+struct StripStrides {
+    uint32_t smallest = 0, whole = 0;
+};
+void strip_strides_of_middle_row(hipStream_t stream, idx_t m, idx_t base, const idx_t* row_ptr, const idx_t* col, StripStrides* strides) {
     constexpr idx_t kMostLooked = 256;
     const idx_t row = m / 2;
     idx_t ends[2] = {0, 0};
     if (hipMemcpyAsync(ends, row_ptr + row, sizeof(ends), hipMemcpyDeviceToHost, stream) != hipSuccess ||
         hipStreamSynchronize(stream) != hipSuccess)
-        return 0;
-    if (ends[1] < ends[0] || ends[0] < base) return 0;
+        return;
+    if (ends[1] < ends[0] || ends[0] < base) return;
     const idx_t count = ends[1] - ends[0];
-    if (count < 2 || count > kMostLooked) return 0;
+    if (count < 2 || count > kMostLooked) return;
     idx_t cols[kMostLooked];
     if (hipMemcpyAsync(cols, col + (ends[0] - base), count * sizeof(idx_t), hipMemcpyDeviceToHost, stream) != hipSuccess ||
         hipStreamSynchronize(stream) != hipSuccess)
-        return 0;
+        return;
     std::sort(cols, cols + count);
-    uint32_t best = 0;
     idx_t run_start = cols[0];
     for (idx_t i = 1; i < count; ++i) {
         if (cols[i] <= cols[i - 1] + 1) continue;  // the run goes on (or a duplicate)
@@ -1251,9 +1253,10 @@ uint32_t strip_stride_of_middle_row(hipStream_t stream, idx_t m, idx_t base, con
         run_start = cols[i];
         if (gap > 0xffffffffull) continue;
         const uint32_t stride = static_cast<uint32_t>(gap);
-        if (mcsp::spmm_strip_stride_usable(m, stride) && (best == 0 || stride < best)) best = stride;
+        if (!mcsp::spmm_strip_stride_usable(m, stride)) continue;
+        if (strides->smallest == 0 || stride < strides->smallest) strides->smallest = stride;
+        if (stride % mcsp::kSpmmStripRows == 0 && (strides->whole == 0 || stride < strides->whole)) strides->whole = stride;
     }
-    return best;
 }
 
 // The schedule of mcsparseSpMM_preprocess, of whichever kind suits; matA->schedule says which.  ia: the matrix's 32-bit arrays.
@@ -1306,31 +1309,55 @@ mcsparseStatus_t build_spmm_schedule(mcsparseHandle_t handle, mcsparseSpMatDescr
             s.odd_blocks = static_cast<uint32_t>(counters[3] >> 32);
             const bool lines_cut = static_cast<uint64_t>(s.odd_blocks) * 16 > blocks;
             const bool strips_suit = (row_bytes > 128 || (lines_cut && m >= kNarrowStripRows)) && matC->order == MCSPARSE_ORDER_ROW;
-            const uint32_t stride = !strips_suit ? 0u
-                                                 : strip_stride_of_middle_row(handle->stream, m, static_cast<idx_t>(matA->idxBase),
-                                                                              ia.rows, ia.cols);
-            if (stride != 0) {
+            StripStrides strides;
+            if (strips_suit)
+                strip_strides_of_middle_row(handle->stream, m, static_cast<idx_t>(matA->idxBase), ia.rows, ia.cols, &strides);
+            // Covers the matrix in strips `stride` apart and says what came of it.
+            struct Cover {
+                uint32_t stride = 0, blocks = 0;
+                unsigned long long counters[3] = {0, 0, 0};  // span sum, rows of op(B) loaded, longest strip
+                bool pays = false;
+            };
+            auto cover = [&](uint32_t stride, Cover* c) {
+                c->stride = stride;
                 mcsp::launch_spmm_strip_count(handle->stream, m, nnz, static_cast<idx_t>(matA->idxBase), stride, ia.rows,
                                               ia.cols, externalBuffer);
-                const uint64_t strip_groups = mcsp::spmm_strip_groups(m, stride);
-                uint32_t strip_blocks = 0;
-                unsigned long long strip_counters[3] = {0, 0, 0};  // span sum, rows of op(B) loaded, longest strip
-                const char* strip_total = static_cast<const char*>(externalBuffer) + l.group_ptr + strip_groups * sizeof(uint32_t);
-                if (hipMemcpyAsync(&strip_blocks, strip_total, sizeof(strip_blocks), hipMemcpyDeviceToHost, handle->stream) != hipSuccess ||
-                    hipMemcpyAsync(strip_counters, span_slot, sizeof(strip_counters), hipMemcpyDeviceToHost, handle->stream) != hipSuccess ||
+                const char* strip_total = static_cast<const char*>(externalBuffer) + l.group_ptr +
+                                          mcsp::spmm_strip_groups(m, stride) * sizeof(uint32_t);
+                if (hipMemcpyAsync(&c->blocks, strip_total, sizeof(c->blocks), hipMemcpyDeviceToHost, handle->stream) != hipSuccess ||
+                    hipMemcpyAsync(c->counters, span_slot, sizeof(c->counters), hipMemcpyDeviceToHost, handle->stream) != hipSuccess ||
                     hipStreamSynchronize(handle->stream) != hipSuccess)
-                    return to_public_status(MCSP_STATUS_INTERNAL_ERROR);
+                    return false;
                 // (and its strips' values fit the copies in LDS: read where they lie, 16 rows' values cost more than they save)
-                if (strip_blocks != 0 && strip_counters[1] * 5 <= counters[1] * 4 &&
-                    (strip_counters[2] & 0xffffffffull) <= mcsp::kSpmmStripStagedValues &&
-                    mcsp::spmm_strip_schedule_fits(m, nnz, stride, strip_blocks)) {
-                    mcsp::launch_spmm_strip_fill(handle->stream, m, nnz, static_cast<idx_t>(matA->idxBase), stride, ia.rows,
+                c->pays = c->blocks != 0 && c->counters[1] * 5 <= counters[1] * 4 &&
+                          (c->counters[2] & 0xffffffffull) <= mcsp::kSpmmStripStagedValues &&
+                          mcsp::spmm_strip_schedule_fits(m, nnz, stride, c->blocks);
+                return true;
+            };
+            if (strides.smallest != 0) {
+                Cover best, other;
+                if (!cover(strides.smallest, &best)) return to_public_status(MCSP_STATUS_INTERNAL_ERROR);
+                // the other one where this does not pay, or leaves more than a sixteenth of its strips' rows empty
+                constexpr uint32_t kRows = mcsp::kSpmmStripRows;
+                const uint32_t empty = (best.stride + kRows - 1) / kRows * kRows - best.stride;
+                if (strides.whole != 0 && strides.whole != best.stride && (!best.pays || empty * 16 > best.stride)) {
+                    if (!cover(strides.whole, &other)) return to_public_status(MCSP_STATUS_INTERNAL_ERROR);
+                    if (other.pays && (!best.pays || other.counters[1] <= best.counters[1])) {
+                        best = other;
+                    } else if (best.pays) {  // its offsets are counted again (the region is shared)
+                        mcsp::launch_spmm_strip_count(handle->stream, m, nnz, static_cast<idx_t>(matA->idxBase), best.stride, ia.rows,
+                                                      ia.cols, externalBuffer);
+                    }
+                }
+                if (best.pays) {
+                    const uint64_t strip_groups = mcsp::spmm_strip_groups(m, best.stride);
+                    mcsp::launch_spmm_strip_fill(handle->stream, m, nnz, static_cast<idx_t>(matA->idxBase), best.stride, ia.rows,
                                                  ia.cols, externalBuffer);
-                    s.entries = strip_blocks;
-                    s.mean_span = strip_groups != 0 ? strip_counters[0] / strip_groups : 0;
+                    s.entries = best.blocks;
+                    s.mean_span = strip_groups != 0 ? best.counters[0] / strip_groups : 0;
                     s.blocks = true;
-                    s.stride = stride;
-                    s.longest_group = static_cast<uint32_t>(strip_counters[2] & 0xffffffffull);
+                    s.stride = best.stride;
+                    s.longest_group = static_cast<uint32_t>(best.counters[2] & 0xffffffffull);
                     s.useful = true;
                     s.valid = true;
                     return MCSPARSE_STATUS_SUCCESS;

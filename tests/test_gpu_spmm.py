@@ -317,6 +317,12 @@ def columns_from_blocks(ptr, words, m):
     return rows
 
 
+def read_strip_stride(buf, m):
+    """The stride of a strip schedule as it lies in the buffer, among the counters."""
+    at = (4 * ((m + 3) // 4 + 1) + 127) // 128 * 128 + 24
+    return int(buf[at:at + 4].cpu().numpy().view(np.uint32)[0])
+
+
 def read_strip_blocks(torch, buf, m):
     """The strip schedule as it lies in the buffer: the stride among the counters, offsets per group, 16-byte blocks."""
     def align(x):
@@ -407,6 +413,35 @@ def test_blocks_cover_every_nonzero_once_and_in_storage_order(torch_gpu, handle,
     for r in range(a.m):
         want = (a.col[a.ptr[r] - a.base:a.ptr[r + 1] - a.base].astype(np.int64) - a.base).tolist()
         assert got[r] == want, (r, got[r], want)
+
+
+@pytest.mark.parametrize("runs,stride", [((-128, 0, 11, 128), 128), ((-22, -11, 0, 11, 22, 150), 11)])
+def test_strips_lie_where_they_share_most(torch_gpu, handle, oracle, runs, stride):
+    """Runs of three diagonals, from 2^17 rows on: the smallest distance between two, 11, is no whole number of strips.  Strips that
+    far apart share less than a fifth of the rows of op(B), strips 128 apart more; or the other way round."""
+    torch = torch_gpu
+    m, n = (1 << 17) + 5, 64
+    col = np.arange(m)[:, None] + np.concatenate([np.arange(r, r + 3) for r in runs])
+    kept = (col >= 0) & (col < m)
+    ptr = np.concatenate([[0], np.cumsum(kept.sum(1))]).astype(np.int32)
+    rng = np.random.default_rng(3)
+    a = wl.Csr(m, m, ptr, col[kept].astype(np.int32), rng.uniform(-1, 1, int(ptr[-1])).astype(np.float32))
+    B = rng.uniform(-1, 1, (m, n)).astype(np.float32)
+    d_ptr, d_col, d_val, d_B = dev(torch, a.ptr), dev(torch, a.col), dev(torch, a.val), dev(torch, B)
+    d_C = torch.zeros((m, n), dtype=torch.float32, device="cuda")
+    mat = api.SpMat(m, m, a.nnz, d_ptr, d_col, d_val)
+    mB, mC = api.DnMat(m, n, n, d_B), api.DnMat(m, n, n, d_C)
+    st, size = api.spmm_buffer_size(handle, api.OP_N, api.OP_N, 1.0, mat, mB, 0.0, mC, api.R_32F)
+    buf = torch.zeros(size, dtype=torch.uint8, device="cuda")
+    assert api.spmm_preprocess(handle, api.OP_N, api.OP_N, 1.0, mat, mB, 0.0, mC, api.R_32F, buf) == 0
+    assert mat.spmm_schedule()[0] == 4
+    assert read_strip_stride(buf, m) == stride
+    mat.set_spmm_schedule(1)
+    assert api.spmm(handle, api.OP_N, api.OP_N, 1.0, mat, mB, 0.0, mC, api.R_32F, buf) == 0
+    torch.cuda.synchronize()
+    assert mat.spmm_kernel() == 4
+    c_ref, bound = oracle.spmm(m, n, 0, a.ptr, a.col, a.val, 1.0, 0.0, B.ravel(), n, True, None, n, True)
+    assert_within(d_C.cpu().numpy(), c_ref, bound, np.float32)
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
