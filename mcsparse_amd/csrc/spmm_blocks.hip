@@ -31,8 +31,7 @@ struct BlockCounters {
     unsigned long long loads;     // rows of op(B) all blocks load together
     unsigned int longest_group;   // most nonzeros in one group that has blocks
     unsigned int most_blocks;     // of one group
-    unsigned int odd_groups;      // with twice the blocks of a group near them, or more
-    unsigned int odd_blocks;      // of these
+    unsigned long long odd;       // groups with twice the blocks that are usual near them, or more; << 32 the blocks of these
 };
 
 __global__ void zero_block_counters_kernel(BlockCounters* c) {
@@ -40,8 +39,7 @@ __global__ void zero_block_counters_kernel(BlockCounters* c) {
     c->loads = 0;
     c->longest_group = 0;
     c->most_blocks = 0;
-    c->odd_groups = 0;
-    c->odd_blocks = 0;
+    c->odd = 0;
 }
 
 // One thread covers the nonzeros of one group of K rows with blocks.  It merges the rows by the key
@@ -187,28 +185,8 @@ __global__ __launch_bounds__(kWave) void block_cover_kernel(idx_t m, idx_t base,
     if (!FILL) {
         if (group <= groups) block_ptr[group] = count;  // slot `groups` receives the total after the scan
         unsigned long long span = count != 0 ? last_col - first_col : 0;
-        // A group is odd that has twice as many blocks as the wavefront's first quarter: three quarters of the groups may hold a
-        // grid line's end before these count as the rule.
-        uint32_t rank = 0;
-#pragma unroll
-        for (int j = 0; j < kWave; ++j) {
-            const uint32_t other = __builtin_amdgcn_readlane(count, j);
-            rank += other != 0 && (other < count || (other == count && static_cast<uint32_t>(j) < threadIdx.x)) ? 1u : 0u;
-        }
-        const uint32_t with_blocks = __popcll(__ballot(count != 0));
-        const unsigned long long first_quarter = __ballot(count != 0 && rank == with_blocks / 4);
-        uint32_t odd_blocks = 0;
-        unsigned long long odd = 0;
-        if (first_quarter != 0) {
-            const uint32_t usual = __builtin_amdgcn_readlane(count, __builtin_ctzll(first_quarter));
-            odd = __ballot(count >= 2 * usual);
-            odd_blocks = count >= 2 * usual ? count : 0;
-        }
-        uint32_t most = count;
 #pragma unroll
         for (int off = kWave / 2; off > 0; off >>= 1) {
-            most = max(most, static_cast<uint32_t>(__shfl_xor(static_cast<int>(most), off, kWave)));
-            odd_blocks += __shfl_xor(odd_blocks, off, kWave);
             span += __shfl_xor(span, off, kWave);
             loads += __shfl_xor(loads, off, kWave);
             group_nnz = max(group_nnz, static_cast<uint32_t>(__shfl_xor(static_cast<int>(group_nnz), off, kWave)));
@@ -217,13 +195,52 @@ __global__ __launch_bounds__(kWave) void block_cover_kernel(idx_t m, idx_t base,
             if (span != 0) atomicAdd(&counters->span_sum, span);
             if (loads != 0) atomicAdd(&counters->loads, loads);
             if (group_nnz != 0) atomicMax(&counters->longest_group, group_nnz);
-            if (most != 0) atomicMax(&counters->most_blocks, most);
-            if (odd != 0) {
-                atomicAdd(&counters->odd_groups, static_cast<unsigned int>(__popcll(odd)));
-                atomicAdd(&counters->odd_blocks, odd_blocks);
-            }
         }
     }
+}
+
+// What the blocks of the groups say before they are summed up: the most of one group, and the groups that are odd, with twice as
+// many as is usual, or more.  Usual: the least of sixteen groups, and of the four such numbers of a wavefront the largest (a line of a
+// grid, or a group of fewer nonzeros, ends in some of the sixteen).  A kernel of its own: in the cover, whose every wavefront adds to
+// the counters' line (5 ns each), it was 27 us of 232 on a million rows.
+constexpr int kOddBlock = 1024;
+__global__ __launch_bounds__(kOddBlock) void odd_groups_kernel(uint64_t groups, const uint32_t* __restrict__ counts,
+                                                               BlockCounters* __restrict__ counters) {
+    constexpr int kWaves = kOddBlock / kWave;
+    __shared__ uint32_t s_most[kWaves], s_odd[kWaves], s_odd_blocks[kWaves];
+    const uint64_t group = static_cast<uint64_t>(blockIdx.x) * kOddBlock + threadIdx.x;
+    const uint32_t count = group < groups ? counts[group] : 0;
+    auto of_lane = [](uint32_t v, int off) { return static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), off, kWave)); };
+    uint32_t usual = count != 0 ? count : 0xffffffffu;
+#pragma unroll
+    for (int off = 1; off < 16; off <<= 1) usual = min(usual, of_lane(usual, off));
+    if (usual == 0xffffffffu) usual = 0;
+#pragma unroll
+    for (int off = 16; off < kWave; off <<= 1) usual = max(usual, of_lane(usual, off));
+    const bool odd = usual != 0 && count >= 2 * usual;
+    uint32_t most = count, odd_blocks = odd ? count : 0;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        most = max(most, of_lane(most, off));
+        odd_blocks += of_lane(odd_blocks, off);
+    }
+    const uint32_t wave = threadIdx.x / kWave, odd_groups = __popcll(__ballot(odd));
+    if (lane_id() == 0) {
+        s_most[wave] = most;
+        s_odd[wave] = odd_groups;
+        s_odd_blocks[wave] = odd_blocks;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    unsigned long long sum = 0;
+    most = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+        most = max(most, s_most[w]);
+        sum += s_odd[w] | static_cast<unsigned long long>(s_odd_blocks[w]) << 32;
+    }
+    if (most != 0) atomicMax(&counters->most_blocks, most);
+    if (sum != 0) atomicAdd(&counters->odd, sum);
 }
 
 // The lane groups of a wavefront walk their block lists in lockstep: a wavefront whose groups hold different
@@ -678,6 +695,8 @@ void launch_spmm_block_count(hipStream_t stream, idx_t m, idx_t nnz, idx_t base,
     hipLaunchKernelGGL(zero_block_counters_kernel, dim3(1), dim3(1), 0, stream, c.counters);
     hipLaunchKernelGGL((block_cover_kernel<false>), grid, dim3(kWave), 0, stream, m, base, row_ptr, col, c.block_ptr,
                        c.blocks, c.counters);
+    hipLaunchKernelGGL(odd_groups_kernel, dim3(static_cast<uint32_t>((slots + kOddBlock - 1) / kOddBlock)), dim3(kOddBlock), 0, stream,
+                       slots - 1, c.block_ptr, c.counters);
     launch_exclusive_scan_u32(stream, c.block_ptr, slots, c.scan_ws);
 }
 
