@@ -15,23 +15,78 @@ namespace {
 
 using namespace spmm_detail;
 
+// Where rows differ much in length (the matrix has rows above kSpmmLongRow, which are not taken here), a row of more than kTogether
+// nonzeros is the whole wavefront's, its groups on neighbouring stretches of it: walked by one group,
+// four or eight rows of op(B) at a time, the longest of them outlast the launch.  Power-law rows, microseconds a call before and
+// so: 16 fp32 columns, 100 K rows 69 and 49, 400 K 142 and 123, a million 313 and 293, 2.5 M 863 and 839; 12 fp64 columns, 100 K
+// 65 and 57, a million 427 and 415 (150 K rows, 16 fp32 columns, with limits of 4, 8 and 16 times LR 55, 53 and 54).  Eight lanes
+// of fp32 get there faster, and the code beside the loop costs them more than it gives (32 columns, 100 K rows 69 and 67, 200 K
+// 91 and 92, a million 348 and 351, 2.5 M 1006 and 1019); with sixteen lanes the limit is the least length of a row taken apart.
+template <int LR>
+constexpr idx_t kTogether = 16 * LR;
+template <typename T, int LR>
+constexpr bool kTakenTogether = LR == 4 || (LR == 8 && sizeof(T) == 8);
+static_assert(kTogether<8> < kSpmmLongCutLeast, "rows that are not taken apart");
+// The rows of more than kTogether<LR> among a wavefront's 64 from row0 on, of which lane i has the i-th, my_start to my_end; mine: it is
+// to be taken.  For whole wavefronts.
+template <typename T, int LR, int V>
+__device__ __forceinline__ void rows_together(bool mine, idx_t my_start, idx_t my_end, uint64_t row0, idx_t base,
+                                              const idx_t* __restrict__ col, const T* __restrict__ val, const char* __restrict__ B_bytes,
+                                              uint32_t lane_off, uint32_t ldb_bytes, T* __restrict__ C, int64_t ldc, bool c_row_major,
+                                              T alpha, T beta, const LaneColumns& own) {
+    const uint32_t wave_lane = threadIdx.x % kWave, lane = wave_lane % LR, group = wave_lane / LR;
+    for (unsigned long long together = __ballot(mine && my_end - my_start > kTogether<LR>); together != 0; together &= together - 1) {  // whole wavefront
+        const uint32_t r = __builtin_ctzll(together);
+        const idx_t begin = __builtin_amdgcn_readlane(my_start, r), end = __builtin_amdgcn_readlane(my_end, r);
+        T acc[V];
+#pragma unroll
+        for (int i = 0; i < V; ++i) acc[i] = T(0);
+        row_times_b<T, LR, V, false, true>(begin + group * LR, end, lane, base, col, val, B_bytes, lane_off, ldb_bytes, acc, kWave);
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+#pragma unroll
+            for (int off = LR; off < kWave; off <<= 1) acc[i] += __shfl_xor(acc[i], off, kWave);
+        }
+        if (group == 0 && own.any) store_c<T, V>(C, ldc, c_row_major, row0 + r, own.first, acc, alpha, beta, own.skip);
+    }
+}
+
 // op(B) row-major.  LR lanes per row of A, V adjacent columns per lane; blockIdx.y walks the
 // column panels of LR*V columns.  V > 1 requires n >= V, which the launcher checks; RAGGED: n need not be a multiple of
 // V.  Eight wavefronts per SIMD are asked for outright: left alone, the scheduler draws the batches of sixteen lanes
 // together into 102 registers instead of 59, four wavefronts (27-point stencil 128^3, 64 fp32 columns: 636 -> 707 us).
 // Not in fp64, where five or six wavefronts do better (16 columns 420 us, 439 with eight; 32 columns 657 and 677).
-template <typename T, int LR, int V, bool WIDE, bool RAGGED>
+//
+// TOGETHER: a call that does not know whether there are long rows (COO, CSC, a captured one) for a width whose longer rows are wavefronts'
+// where there are; the first `beside` workgroups take these, so that a row's sum is the same by every way to the product.  (As a launch of
+// its own: COO, 1000 and 100 K rows of 16, 16 fp32 columns 21.4 and 37.9 us, 18.5 and 37.0 so; 100 K power-law rows 58 and 46.)
+template <typename T, int LR, int V, bool WIDE, bool RAGGED, bool TOGETHER>
 __global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 8 : 1) void spmm_rowb_kernel(idx_t m, idx_t n, idx_t base,
                                                            const idx_t* __restrict__ row_ptr,
                                                            const idx_t* __restrict__ col, const T* __restrict__ val,
                                                            const T* __restrict__ B, int64_t ldb, T* __restrict__ C,
                                                            int64_t ldc, bool c_row_major, T alpha, T beta,
                                                            idx_t long_row, const uint32_t* __restrict__ apart,
-                                                           uint32_t xcd_chunk, uint32_t xcds) {
+                                                           uint32_t beside, uint32_t xcd_chunk, uint32_t xcds) {
     typedef typename ByteOffset<WIDE>::type off_t;
     constexpr int kRowsPerBlock = kBlock / LR;
     const idx_t lane = threadIdx.x % LR;
-    const uint64_t row = xcd_position(blockIdx.x, xcd_chunk, xcds) * kRowsPerBlock + threadIdx.x / LR;
+    if constexpr (TOGETHER) {
+        if (blockIdx.x < beside) {  // whole workgroup
+            if (*apart == 0) return;
+            const LaneColumns own = lane_columns<V, RAGGED>((static_cast<uint64_t>(blockIdx.y) * LR + lane) * V, n);
+            for (uint64_t row0 = (static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x) / kWave * kWave; row0 < m;
+                 row0 += static_cast<uint64_t>(beside) * kBlock) {  // whole wavefront
+                const uint64_t mine = row0 + threadIdx.x % kWave, at = min(mine, static_cast<uint64_t>(m) - 1);
+                const idx_t start = row_ptr[at] - base, end = row_ptr[at + 1] - base;
+                rows_together<T, LR, V>(mine < m && end - start <= long_row, start, end, row0, base, col, val,
+                                        reinterpret_cast<const char*>(B), static_cast<uint32_t>(own.first * sizeof(T)),
+                                        static_cast<uint32_t>(ldb * sizeof(T)), C, ldc, c_row_major, alpha, beta, own);
+            }
+            return;
+        }
+    }
+    const uint64_t row = xcd_position(TOGETHER ? blockIdx.x - beside : blockIdx.x, xcd_chunk, xcds) * kRowsPerBlock + threadIdx.x / LR;
     if (row >= m) return;  // whole lane groups
     // Lanes past the last column still fetch their share of the row's nonzeros for the group;
     // they compute on the first columns and store nothing.
@@ -42,7 +97,8 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 8 : 1) void sp
     const idx_t end = row_ptr[row + 1] - base;
     // long_row != 0: rows with more nonzeros are the work of the kernels in spmm_long.hip, C included, unless *apart is
     // zero (null: known not to be)
-    if (long_row != 0 && end - start > long_row && (apart == nullptr || *apart != 0)) return;  // whole lane groups
+    const idx_t longest = TOGETHER ? kTogether<LR> : long_row;
+    if (longest != 0 && end - start > longest && (apart == nullptr || *apart != 0)) return;  // whole lane groups
     T acc[V];
 #pragma unroll
     for (int i = 0; i < V; ++i) acc[i] = T(0);
@@ -59,31 +115,14 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 8 : 1) void sp
 // rows, and most rows, of one or two nonzeros, are three dependent trips to memory by themselves.  Here a wavefront has
 // kTurnRows neighbouring rows: a group that is through with one takes the next, the long ones first, and the nonzeros of what a group
 // is at next, the next LR of its row or the first of another, are asked for behind the rows of op(B) of the present ones.
-//
-// A row of more than kTogether nonzeros is the whole wavefront's, its groups on neighbouring stretches of it: walked by one group,
-// four or eight rows of op(B) at a time, the longest of them outlast the launch.  Power-law rows, microseconds a call before and
-// so: 16 fp32 columns, 100 K rows 69 and 49, 400 K 142 and 123, a million 313 and 293, 2.5 M 863 and 839; 12 fp64 columns, 100 K
-// 65 and 57, a million 427 and 415 (150 K rows, 16 fp32 columns, with limits of 4, 8 and 16 times LR 55, 53 and 54).  Eight lanes
-// of fp32 get there faster, and the code beside the loop costs them more than it gives (32 columns, 100 K rows 69 and 67, 200 K
-// 91 and 92, a million 348 and 351, 2.5 M 1006 and 1019); with sixteen lanes the limit is the least length of a row taken apart.
 constexpr int kTurnRows = kWave;
-template <int LR>
-constexpr idx_t kTogether = 16 * LR;
-template <typename T, int LR>
-constexpr bool kTakenTogether = LR == 4 || (LR == 8 && sizeof(T) == 8);
-static_assert(kTogether<8> < kSpmmLongCutLeast, "rows that are not taken apart");
-// BESIDE: another kernel has taken the rows of up to kTogether<LR>, and all of them unless *apart says that there are long rows.
-template <typename T, int LR, int V, bool RAGGED, bool BESIDE>
+template <typename T, int LR, int V, bool RAGGED>
 __global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 7 : 1) void spmm_rowb_turns_kernel(idx_t m, idx_t n, idx_t nnz, idx_t base,
                                                                  const idx_t* __restrict__ row_ptr,
                                                                  const idx_t* __restrict__ col, const T* __restrict__ val,
                                                                  const T* __restrict__ B, int64_t ldb, T* __restrict__ C,
                                                                  int64_t ldc, bool c_row_major, T alpha, T beta,
-                                                                 idx_t long_row, const uint32_t* __restrict__ apart,
-                                                                 const BoundsWork cut) {
-    if constexpr (BESIDE) {
-        if (*apart == 0) return;  // all workgroups
-    }
+                                                                 idx_t long_row, const BoundsWork cut) {
     if (blockIdx.x < cut.blocks) {  // whole workgroup
         cut_pieces(cut, base, nnz, row_ptr, col);
         return;
@@ -100,23 +139,8 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 7 : 1) void sp
     const idx_t my_start = row_ptr[my_row] - base, my_end = row_ptr[my_row + 1] - base;
     const uint32_t length = my_end - my_start;
     const bool mine = row0 + wave_lane < m && length <= long_row, live = mine && (!kTakenTogether<T, LR> || length <= kTogether<LR>);
-    if constexpr (kTakenTogether<T, LR>) {
-        for (unsigned long long together = __ballot(mine && length > kTogether<LR>); together != 0; together &= together - 1) {  // whole wavefront
-            const uint32_t r = __builtin_ctzll(together);
-            const idx_t begin = __builtin_amdgcn_readlane(my_start, r), end = __builtin_amdgcn_readlane(my_end, r);
-            T acc[V];
-#pragma unroll
-            for (int i = 0; i < V; ++i) acc[i] = T(0);
-            row_times_b<T, LR, V, false, true>(begin + group * LR, end, lane, base, col, val, B_bytes, lane_off, ldb_bytes, acc, kWave);
-#pragma unroll
-            for (int i = 0; i < V; ++i) {
-#pragma unroll
-                for (int off = LR; off < kWave; off <<= 1) acc[i] += __shfl_xor(acc[i], off, kWave);
-            }
-            if (group == 0 && own.any) store_c<T, V>(C, ldc, c_row_major, row0 + r, own.first, acc, alpha, beta, own.skip);
-        }
-        if constexpr (BESIDE) return;
-    }
+    if constexpr (kTakenTogether<T, LR>)
+        rows_together<T, LR, V>(mine, my_start, my_end, row0, base, col, val, B_bytes, lane_off, ldb_bytes, C, ldc, c_row_major, alpha, beta, own);
     const unsigned long long first = __ballot(live && length > 4 * LR), second = __ballot(live && length <= 4 * LR);
     auto below = [&](unsigned long long mask) {
         return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u));
@@ -895,36 +919,38 @@ void launch_rowb(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     const T* val = static_cast<const T*>(a.val);
     const T* B = static_cast<const T*>(a.B);
     T* C = static_cast<T*>(a.C);
-    // A call that does not know whether there are long rows leaves those that the kernel for turns gives to whole wavefronts to it,
-    // so that a row's sum is the same by every way to the product.
-    const bool in_turns = takes_rows_in_turns<T, LR>(a, true), beside = kTakenTogether<T, LR> && takes_rows_in_turns<T, LR>(a, false);
-    auto launch = [&](auto wide, auto ragged) {
-        hipLaunchKernelGGL((spmm_rowb_kernel<T, LR, V, decltype(wide)::value, decltype(ragged)::value>), grid, dim3(kBlock), 0,
-                           stream, a.m, a.n, a.base, a.row_ptr, a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta,
-                           beside ? kTogether<LR> : a.long_row, a.long_apart, chunk, xcds);
+    auto launch = [&](auto wide, auto ragged, auto together, uint32_t beside) {
+        const dim3 all(grid.x + beside, grid.y);
+        hipLaunchKernelGGL((spmm_rowb_kernel<T, LR, V, decltype(wide)::value, decltype(ragged)::value, decltype(together)::value>), all,
+                           dim3(kBlock), 0, stream, a.m, a.n, a.base, a.row_ptr, a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta,
+                           a.long_row, a.long_apart, beside, chunk, xcds);
     };
     auto launch_offsets = [&](auto ragged) {
-        if (narrow_offsets(a, sizeof(T))) launch(std::false_type{}, ragged);
-        else launch(std::true_type{}, ragged);
+        if constexpr (kTakenTogether<T, LR>) {
+            if (takes_rows_in_turns<T, LR>(a, false)) {
+                // (a whole number for every XCD, which leaves the others' order as it is)
+                constexpr uint64_t kMost = 1024;
+                const uint64_t needed = min((static_cast<uint64_t>(a.m) + kBlock - 1) / kBlock, kMost);
+                launch(std::false_type{}, ragged, std::true_type{}, static_cast<uint32_t>((needed + xcds - 1) / xcds * xcds));
+                return;
+            }
+        }
+        if (narrow_offsets(a, sizeof(T))) launch(std::false_type{}, ragged, std::false_type{}, 0);
+        else launch(std::true_type{}, ragged, std::false_type{}, 0);
     };
     if constexpr (LR <= 16) {
-        if (in_turns || beside) {
+        if (takes_rows_in_turns<T, LR>(a, true)) {
             constexpr uint32_t kRowsPerBlock = kBlock / kWave * kTurnRows;
-            const BoundsWork none = {0, {nullptr, 0, 0, 0, 0}, nullptr, nullptr, 0};
-            const BoundsWork cut = in_turns ? spmm_long_bounds(a, sizeof(T)) : none;
+            const BoundsWork cut = spmm_long_bounds(a, sizeof(T));
             const dim3 turns_grid(cut.blocks + (a.m + kRowsPerBlock - 1) / kRowsPerBlock, static_cast<uint32_t>(panels));
-            auto turns = [&](auto ragged, auto other) {
-                hipLaunchKernelGGL((spmm_rowb_turns_kernel<T, LR, V, decltype(ragged)::value, decltype(other)::value>), turns_grid,
-                                   dim3(kBlock), 0, stream, a.m, a.n, a.nnz, a.base, a.row_ptr, a.col, val, B, a.ldb, C, a.ldc,
-                                   a.c_row_major, alpha, beta, a.long_row, a.long_apart, cut);
+            auto turns = [&](auto ragged) {
+                hipLaunchKernelGGL((spmm_rowb_turns_kernel<T, LR, V, decltype(ragged)::value>), turns_grid, dim3(kBlock), 0, stream,
+                                   a.m, a.n, a.nnz, a.base, a.row_ptr, a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta,
+                                   a.long_row, cut);
             };
-            auto turns_of = [&](auto other) {
-                if (a.n % V != 0) turns(std::true_type{}, other);
-                else turns(std::false_type{}, other);
-            };
-            if (in_turns) turns_of(std::false_type{});
-            else if constexpr (kTakenTogether<T, LR>) turns_of(std::true_type{});
-            if (in_turns) return;
+            if (a.n % V != 0) turns(std::true_type{});
+            else turns(std::false_type{});
+            return;
         }
     }
     if constexpr (V > 1) {

@@ -339,3 +339,39 @@ def test_rows_taken_by_a_whole_wavefront(torch_gpu, handle, oracle, dtype, n):
         torch.cuda.synchronize()
         products.append(C.cpu().numpy())
     assert np.array_equal(products[0], products[1])
+
+
+def launches_of(torch, call):
+    """How many launches a call is, from a graph that has captured it."""
+    import ctypes
+    with open("/proc/self/maps") as maps:
+        runtime = ctypes.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph, stream=call[0]):
+        assert call[1]() == 0
+    nodes = ctypes.c_size_t()
+    assert runtime.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(nodes)) == 0
+    return nodes.value
+
+
+@pytest.mark.parametrize("dtype,narrow,wide", [(np.float32, 16, 32), (np.float64, 16, 32), (np.float64, 8, 32)])
+def test_rows_of_wavefronts_cost_no_launch_of_their_own(torch_gpu, dtype, narrow, wide):
+    """A call that does not know whether there are long rows (COO): as many launches where rows are taken by whole wavefronts as
+    for wider operands, whose rows never are."""
+    torch = torch_gpu
+    side = torch.cuda.Stream()
+    handle = api.Handle(stream=side.cuda_stream)
+    a = wl.random_ragged(3000, 2000, 16, dtype=dtype, seed=1)
+    rows = dev(torch, np.repeat(np.arange(a.m, dtype=np.int32), np.diff(a.ptr)))
+    col, val = dev(torch, a.col), dev(torch, a.val)
+    counts = []
+    for n in (narrow, wide):
+        mat = api.SpMat(a.m, a.n, a.nnz, rows, col, val, fmt=api.FORMAT_COO)
+        B, C = (torch.zeros((k, n), dtype=val.dtype, device="cuda") for k in (a.n, a.m))
+        call = (handle, api.OP_N, api.OP_N, 1.0, mat, api.DnMat(a.n, n, n, B), 0.0, api.DnMat(a.m, n, n, C), api.maca_type(np.dtype(dtype)))
+        st, size = api.spmm_buffer_size(*call)
+        assert st == 0
+        buf = torch.empty(size, dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        counts.append(launches_of(torch, (side, lambda: api.spmm(*call, buf))))
+    assert counts[0] == counts[1] > 0, counts
