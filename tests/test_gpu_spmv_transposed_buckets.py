@@ -135,6 +135,28 @@ def test_alg2_repeats_its_bits_and_both_agree(torch_gpu, handle, oracle):
         assert_within(got, y_ref, bound, np.float32, what="bucketed products")
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("ask", ["algorithm", "handle"])
+def test_bits_repeat_where_asked_for_with_more_columns(torch_gpu, oracle, dtype, ask):
+    """From 2^22 to 18.8 million columns the default takes the products by bucket too, and its last bits may differ from run to
+    run; they do not under MCSPARSE_SPMV_CSR_ALG2, nor with a handle that has been asked for it."""
+    handle = api.Handle(stream=torch_gpu.cuda.current_stream().cuda_stream)
+    if ask == "handle":
+        handle.set_spmv_deterministic(True)
+    alg = api.SPMV_CSR_ALG2 if ask == "algorithm" else api.SPMV_ALG_DEFAULT
+    a = wl.power_law(m=60000, n=5000011, max_len=20000, dtype=dtype)
+    a.col[::3] = a.col[0]  # sums of many products, in which an order would show
+    rng = np.random.default_rng(33)
+    x, y = rng.uniform(-1, 1, a.m).astype(dtype), rng.uniform(-1, 1, a.n).astype(dtype)
+    y_ref, bound = oracle.spmv(True, a.m, a.n, a.base, a.ptr, a.col, a.val, 1.5, 0.5, x, y)
+    runs = run(torch_gpu, handle, a, x, y, 1.5, 0.5, alg=alg, repeats=4)
+    assert all(np.array_equal(runs[0], other) for other in runs[1:])
+    assert_within(runs[0], y_ref, bound, dtype, what="sorted products")
+    handle.set_spmv_deterministic(False)
+    assert_within(run(torch_gpu, handle, a, x, y, 1.5, 0.5), y_ref, bound, dtype, what="bucketed products")
+    handle.destroy()
+
+
 # ---- few columns, many nonzeros in each: no sort at all, copies of y in LDS ----
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
@@ -207,6 +229,28 @@ def test_crowded_buckets_exact_on_integers(torch_gpu, handle, dtype, rows, per_r
     for base in (0, 1):
         got = run(torch_gpu, handle, a.with_base(base), x, y, 2.0, 1.0)
         assert np.array_equal(got.astype(np.float64), want), (shape, rows, base)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [6000011, 18432 * 1024])
+@pytest.mark.parametrize("shape", ["one_bucket", "third_in_one", "last_bucket"])
+def test_crowded_buckets_of_many_columns_exact_on_integers(torch_gpu, handle, dtype, n, shape):
+    """1024 buckets: a crowded one is dealt out, the last one has fewer columns than the others."""
+    rows, per_row, width = 400000, 12, (n - 1 >> 10) + 1
+    rng = np.random.default_rng(n + len(shape))
+    nnz = rows * per_row
+    last = (n - 1) // width * width
+    if shape == "one_bucket":
+        col = rng.integers(700 * width, 701 * width, nnz)
+    elif shape == "third_in_one":
+        col = np.where(rng.random(nnz) < 0.33, rng.integers(0, width, nnz), rng.integers(0, n, nnz))
+    else:
+        col = rng.integers(last, n, nnz)
+    a = wl.Csr(rows, n, np.arange(rows + 1) * per_row, col, np.zeros(nnz, dtype))
+    x, y = integer_valued(a, 6)
+    want = 2 * np.bincount(col, weights=a.val.astype(np.float64) * np.repeat(x.astype(np.float64), per_row), minlength=n) + y
+    got = run(torch_gpu, handle, a, x, y, 2.0, 1.0)
+    assert np.array_equal(got.astype(np.float64), want), (shape, n)
 
 
 @pytest.mark.parametrize("preprocess", [False, True])
