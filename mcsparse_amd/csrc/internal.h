@@ -439,14 +439,17 @@ struct SpmmArgs {
 //  - a second launch for what is left of a row behind the last panel: 4 us, and for every nonzero its column, value and a line of
 //    op(B).  100 K rows of 16 evenly spread columns, fp32, 130, 160, 192, 390 columns: whole 134, 138, 167, 424 us, in panels 170, 144,
 //    188, 464; rows of 1, 2, 4, 6, 8, 192 columns: 0.59, 0.68, 0.84, 1.02, 1.10 of the time.  More than half a panel left idles lanes on
-//    top: 194 columns 0.78, 0.85, 1.02, 1.15, 1.19; stencil, 20 K rows, 193 columns 30 and 36 us;
+//    top: 194 columns 0.78, 0.85, 1.02, 1.15, 1.19; stencils, 20 K, 128 K, 198 K, a million rows, 200 columns 30 and 35, 159 and 149, 246 and 213,
+//    1443 and 1476 us (fp64, 100 columns, whole vectors, which whole rows are a fifth slower with: 35 and 35, 196 and 155, 305 and 227, 1768
+//    and 1534);
 //  - a line of op(B) fetched twice where a panel ends inside one: 100 K rows of 16, 256 columns, leading dimension 256: 232 and 234,
 //    257: 259 and 290 (rows of two: 0.84 of the time);
 //  - the longest row twice, and with half the lanes: rows of up to 1000 by Zipf's law, 20 K, 100 K, 300 K, a million of them, 256 fp32
 //    columns 48 and 70, 145 and 170, 410 and 427, 1543 and 1393; of up to 128 23.9 and 24.7, 89 and 84.  So it is to be a 4096th of the
 //    nonzeros at most, which also leaves matrices of few rows whole (729 of a stencil 5.0 and 5.5 us).
-// whole_lines: rows of op(B) begin at multiples of 128 bytes.
-constexpr bool spmm_takes_panels(uint64_t row_bytes, uint64_t m, uint64_t nnz, uint64_t longest_row, bool shared_rows, bool whole_lines) {
+// whole_lines: rows of op(B) begin at multiples of 128 bytes; f64_vectors: they are whole vectors of two doubles.
+constexpr bool spmm_takes_panels(uint64_t row_bytes, uint64_t m, uint64_t nnz, uint64_t longest_row, bool shared_rows, bool whole_lines,
+                                 bool f64_vectors) {
     constexpr uint64_t kPanel = 512, kLaunchRows = 16384, kManyRows = 1 << 19;
     if (row_bytes <= kPanel || longest_row == 0 || nnz / 4096 < longest_row) return false;
     const uint64_t whole = row_bytes / kPanel, rest = row_bytes % kPanel;
@@ -455,6 +458,7 @@ constexpr bool spmm_takes_panels(uint64_t row_bytes, uint64_t m, uint64_t nnz, u
     if (rest == 0) return shared_rows || short_rows || whole_lines;
     if (m < kLaunchRows) return false;
     if ((shared_rows && whole >= 2) || nnz / 2 <= m) return true;
+    if (shared_rows && m >= 4 * kLaunchRows && (f64_vectors || m < kManyRows)) return true;
     if (shared_rows || short_rows) return rest <= kPanel / 2;
     return (whole >= 2 && rest == kPanel / 2 && whole_lines) || (whole == 2 && rest <= kPanel / 4);
 }

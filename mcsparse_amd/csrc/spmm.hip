@@ -987,13 +987,14 @@ template <typename T, int V>
 SpmmKernel launch_rowb_v(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     const uint64_t lanes_needed = (static_cast<uint64_t>(a.n) + V - 1) / V;
     const bool whole_lines = (reinterpret_cast<uintptr_t>(a.B) | static_cast<uintptr_t>(a.ldb * sizeof(T))) % 128 == 0;
+    const bool f64_vectors = sizeof(T) == 8 && V > 1 && ((reinterpret_cast<uintptr_t>(a.B) | static_cast<uintptr_t>(a.ldb * sizeof(T))) % 16 == 0 && a.n % V == 0);
     if (lanes_needed <= 1) launch_narrow<T, V, 1>(stream, a, alpha, beta);
     else if (lanes_needed <= 2) launch_narrow<T, V, 2>(stream, a, alpha, beta);
     else if (lanes_needed <= 4) launch_rowb<T, 4, V>(stream, a, alpha, beta);  // measured faster than four column lanes above
     else if (lanes_needed <= 8) launch_rowb<T, 8, V>(stream, a, alpha, beta);
     else if (lanes_needed <= 16) launch_rowb<T, 16, V>(stream, a, alpha, beta);
     else if (lanes_needed <= 32) launch_rowb<T, 32, V>(stream, a, alpha, beta);
-    else if (V == 1 || a.long_row != 0 || !spmm_takes_panels(a.n * sizeof(T), a.m, a.nnz, a.longest_row, a.shared_rows, whole_lines))
+    else if (V == 1 || a.long_row != 0 || !spmm_takes_panels(a.n * sizeof(T), a.m, a.nnz, a.longest_row, a.shared_rows, whole_lines, f64_vectors))
         launch_rowb<T, 64, V>(stream, a, alpha, beta);
     else {
         launch_panels<T, V>(stream, a, alpha, beta);
