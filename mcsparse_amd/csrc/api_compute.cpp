@@ -565,7 +565,7 @@ bool schedule_pays(const SpmmSchedule& s, const mcsp::SpmmArgs& a, size_t value_
         if (us < s.most_blocks * (everywhere ? 4.0 : 1.5)) return false;
         // Wavefronts with groups of different blocks run them one after the other: 27-point stencils whose lines end inside groups,
         // which takes a fifth to a quarter of the blocks (97 x 61 x 97 and 127 x 127 x 60, 128 fp32 columns 378 and 345, 686 and 578).
-        // Of many short rows the kernel without a schedule has to write as much: a million of 5 and 15 diagonals, one group in 20, 243
+        // Of many short rows the kernel without a schedule has as much to write: a million of 5 and 15 diagonals, one group in 20, 243
         // and 309, 337 and 427.
         constexpr idx_t kManyRows = 1 << 19;
         const bool short_rows = a.m >= kManyRows && a.nnz / 16 <= a.m;
@@ -587,16 +587,24 @@ bool schedule_pays(const SpmmSchedule& s, const mcsp::SpmmArgs& a, size_t value_
     // 61 x 55 x 59, fp32, 64 and 128 columns, 3100 and 6200 wavefronts, 65 and 62, 104 and 107; 150 x 150 x 12, 64 columns, 4400
     // wavefronts, 11 MB: 65 and 102.
     constexpr uint64_t kL2 = 4 << 20;
-    if (mcsp::spmm_strips_whole_vectors(a, value_bytes))
-        return s.stride % mcsp::kSpmmStripRows == 0 || wavefronts >= kTwiceFull || window > kL2;
-    // Rows that begin or end at any element, by the rows of A alone (a panel more is as much more work for both): 76^3, 6900 wavefronts, 64
+    if (s.stride % mcsp::kSpmmStripRows == 0 && mcsp::spmm_strips_whole_vectors(a, value_bytes)) return true;
+    const bool whole_lines = (reinterpret_cast<uintptr_t>(a.B) | static_cast<uintptr_t>(a.ldb) * value_bytes) % 128 == 0;
+    // (and wide rows that are no whole number of 512 bytes, for which the kernel without a schedule is slow: 51^3, 90 and 100 fp64 columns
+    // 129 and 151, 151 and 212)
+    if (whole_lines || (row_bytes > 512 && row_bytes % 512 != 0)) return wavefronts >= kTwiceFull || window > kL2;
+    // Rows that begin inside a line cost the strips a third line to a load.  By the rows of A alone (a panel more is as much more work for
+    // both), and fewer where the kernel without a schedule has many lanes idle: 45 x 90 x 90, 6100 wavefronts, 70, 80, 100, 112 columns 168 and
+    // 191, 171 and 180, 210 and 189, 202 and 192; 33 x 100 x 100 and 50 x 65 x 93, 5600 and 4700 wavefronts, 70 columns 153 and 172, 140 and 161; 76^3, 6900 wavefronts, 64
     // and 128 fp32 columns 103 and 150, 261 and 295; 64^3, 4100 wavefronts, 75 and 62, 175 and 128; 60 x 56 x 60, 64 fp64 columns 133 and 117.
     // Fewer where the rows of op(B) that a group reads have left the L2s: 100 x 100 x 20, 3100 wavefronts, 5.0 MB, 64 columns 52 and 65, 10
     // MB, 128 columns 118 and 159; 120 x 120 x 12, 2700 wavefronts, 7.4 MB, 32 fp64 columns 58 and 53, 15 MB, 64 columns 109 and 126; 72^3,
     // 5800 wavefronts, 5.5 MB, 128 fp32 columns 221 and 203.
-    constexpr uint64_t kPanel = 256, kFew = 3072, kOnePanelWindow = 4500000, kPanelsWindow = 8000000;
+    constexpr uint64_t kPanel = 256, kFew = 3072, kOnePanelWindow = 4500000, kPanelsWindow = 8000000, kLanesIdle = 4608, kFewer = 5500;
     const uint64_t of_a_panel = wavefronts / ((row_bytes + kPanel - 1) / kPanel);
-    if (of_a_panel >= kTwiceFull) return true;
+    const bool lanes_idle = row_bytes > kPanel && row_bytes <= kPanel + 128;  // of 32 to a row
+    if (of_a_panel >= (lanes_idle ? kLanesIdle : row_bytes <= kPanel || value_bytes == 8 ? kFewer : kTwiceFull)) return true;
+    // (two panels of whole vectors, the second one short: 61 x 55 x 59, 3200 wavefronts, 34 and 40 fp64 columns 100 and 110, 108 and 108)
+    if (lanes_idle && of_a_panel >= kFew && mcsp::spmm_strips_whole_vectors(a, value_bytes)) return true;
     return row_bytes > kPanel ? window > kPanelsWindow : of_a_panel >= kFew && window > kOnePanelWindow;
 }
 
@@ -1248,6 +1256,7 @@ namespace {
 // has runs of three diagonals 128 apart).  Reads the row back: blocks.
 struct StripStrides {
     uint32_t smallest = 0, whole = 0;
+    uint32_t row_span = 0;  // between that row's first and last column
 };
 void strip_strides_of_middle_row(hipStream_t stream, idx_t m, idx_t base, const idx_t* row_ptr, const idx_t* col, StripStrides* strides) {
     constexpr idx_t kMostLooked = 256;
@@ -1264,6 +1273,7 @@ void strip_strides_of_middle_row(hipStream_t stream, idx_t m, idx_t base, const 
         hipStreamSynchronize(stream) != hipSuccess)
         return;
     std::sort(cols, cols + count);
+    strides->row_span = cols[count - 1] - cols[0];
     idx_t run_start = cols[0];
     for (idx_t i = 1; i < count; ++i) {
         if (cols[i] <= cols[i - 1] + 1) continue;  // the run goes on (or a duplicate)
@@ -1353,19 +1363,24 @@ mcsparseStatus_t build_spmm_schedule(mcsparseHandle_t handle, mcsparseSpMatDescr
                 return true;
             };
             if (strides.smallest != 0) {
-                Cover best, other;
-                if (!cover(strides.smallest, &best)) return to_public_status(MCSP_STATUS_INTERNAL_ERROR);
-                // the other one where this does not pay, or leaves more than a sixteenth of its strips' rows empty
-                constexpr uint32_t kRows = mcsp::kSpmmStripRows;
-                const uint32_t empty = (best.stride + kRows - 1) / kRows * kRows - best.stride;
-                if (strides.whole != 0 && strides.whole != best.stride && (!best.pays || empty * 16 > best.stride)) {
-                    if (!cover(strides.whole, &other)) return to_public_status(MCSP_STATUS_INTERNAL_ERROR);
-                    if (other.pays && (!best.pays || other.counters[1] <= best.counters[1])) {
-                        best = other;
-                    } else if (best.pays) {  // its offsets are counted again (the region is shared)
-                        mcsp::launch_spmm_strip_count(handle->stream, m, nnz, static_cast<idx_t>(matA->idxBase), best.stride, ia.rows,
-                                                      ia.cols, externalBuffer);
-                    }
+                // Where both are there (a grid of odd lines, rows of one plane and of the next line of the one before it): strips the
+                // smallest distance apart load the fewest rows of op(B), those of the other are all of one length and its groups
+                // faster as long as the rows that they read, some five planes of a grid, are not too many for the L2s.  Smallest and whole, 64
+                // fp32 columns: 47 x 125 x 64 (7.5 MB) 126 and 82 us, 142 x 75 x 48 (13.6) 112 and 102, 149 x 149 x 12 (28) 62 and 82; 96 columns:
+                // 118 x 65 x 58 (14.7) 195 and 157, 142 x 75 x 48 (20) 207 and 220; 128 columns: 47 x 125 x 64 (15) 163 and 145, 118 x 65 x 58
+                // (19.6) 192 and 242.  Rows of less than 192 bytes (fp64: up to 192) leave lanes idle, and the smallest is faster where it would
+                // be used: 36 columns 142 x 75 x 48 85 and 97, 146 x 99 x 40 90 and 101, but 47 x 125 x 64 104 and 79.
+                // Of few rows only wide ones: 30 x 89 x 52, 36, 100 and 128 columns 38 and 48, 75 and 83, 83 and 73.
+                constexpr idx_t kSmallestUsed = 6144 * 64, kWholeUsed = 1 << 18;
+                const uint64_t most_window = row_bytes <= 256 ? 20000000 : 15500000;
+                const uint64_t window = (3ull * strides.whole + strides.row_span) * static_cast<uint64_t>(row_bytes);
+                const bool lanes_idle = row_bytes < (vb == 4 ? 192 : 193);
+                const bool whole_first = window <= most_window && (m >= kWholeUsed || row_bytes >= 512) && (!lanes_idle || m < kSmallestUsed);
+                Cover best;
+                for (const bool whole : {whole_first, !whole_first}) {
+                    const uint32_t stride = whole ? strides.whole : strides.smallest;
+                    if (stride == 0 || best.pays || stride == best.stride) continue;
+                    if (!cover(stride, &best)) return to_public_status(MCSP_STATUS_INTERNAL_ERROR);
                 }
                 if (best.pays) {
                     const uint64_t strip_groups = mcsp::spmm_strip_groups(m, best.stride);

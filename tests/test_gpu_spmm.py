@@ -415,17 +415,27 @@ def test_blocks_cover_every_nonzero_once_and_in_storage_order(torch_gpu, handle,
         assert got[r] == want, (r, got[r], want)
 
 
-@pytest.mark.parametrize("runs,stride", [((-128, 0, 11, 128), 128), ((-22, -11, 0, 11, 22, 150), 11)])
-def test_strips_lie_where_they_share_most(torch_gpu, handle, oracle, runs, stride):
-    """Runs of three diagonals, from 2^17 rows on: the smallest distance between two, 11, is no whole number of strips.  Strips that
-    far apart share less than a fifth of the rows of op(B), strips 128 apart more; or the other way round."""
-    torch = torch_gpu
-    m, n = (1 << 17) + 5, 64
+def matrix_of_runs(runs):
+    """Runs of three diagonals."""
+    m = (1 << 17) + 5
     col = np.arange(m)[:, None] + np.concatenate([np.arange(r, r + 3) for r in runs])
     kept = (col >= 0) & (col < m)
     ptr = np.concatenate([[0], np.cumsum(kept.sum(1))]).astype(np.int32)
+    return wl.Csr(m, m, ptr, col[kept].astype(np.int32), np.random.default_rng(3).uniform(-1, 1, int(ptr[-1])).astype(np.float32))
+
+
+@pytest.mark.parametrize("what,n,stride", [((-128, 0, 11, 128), 64, 128), ((-22, -11, 0, 11, 22, 150), 64, 11),
+                                           ((-11, 0, 11, 2000, 4000, 6000, 8000), 64, 2000),
+                                           ("41x41x80", 64, 41), ("41x41x80", 128, 1640), ("63x65x66", 64, 4032), ("63x65x66", 36, 4032), ("263x265x8", 64, 263)])
+def test_which_of_two_distances_strips_lie_apart(torch_gpu, handle, oracle, what, n, stride):
+    """From 2^17 rows on: the smallest distance between two runs of diagonals is no whole number of strips, another one is.
+    Where strips of one of them share less than a fifth of the rows of op(B) the other is taken; where both share more (grids), the
+    whole number, unless there are few rows or its groups read too much of op(B) for the L2s."""
+    from test_gpu_spmv_diagonals import BOX, grid
+    torch = torch_gpu
+    a = grid(tuple(int(side) for side in what.split("x")), BOX, np.float32, 3) if isinstance(what, str) else matrix_of_runs(what)
+    m = a.m
     rng = np.random.default_rng(3)
-    a = wl.Csr(m, m, ptr, col[kept].astype(np.int32), rng.uniform(-1, 1, int(ptr[-1])).astype(np.float32))
     B = rng.uniform(-1, 1, (m, n)).astype(np.float32)
     d_ptr, d_col, d_val, d_B = dev(torch, a.ptr), dev(torch, a.col), dev(torch, a.val), dev(torch, B)
     d_C = torch.zeros((m, n), dtype=torch.float32, device="cuda")
