@@ -15,40 +15,75 @@ namespace {
 
 using namespace spmm_detail;
 
-// Where rows differ much in length (the matrix has rows above kSpmmLongRow, which are not taken here), a row of more than kTogether
-// nonzeros is the whole wavefront's, its groups on neighbouring stretches of it: walked by one group,
-// four or eight rows of op(B) at a time, the longest of them outlast the launch.  Power-law rows, microseconds a call before and
-// so: 16 fp32 columns, 100 K rows 69 and 49, 400 K 142 and 123, a million 313 and 293, 2.5 M 863 and 839; 12 fp64 columns, 100 K
-// 65 and 57, a million 427 and 415 (150 K rows, 16 fp32 columns, with limits of 4, 8 and 16 times LR 55, 53 and 54).  Eight lanes
-// of fp32 get there faster, and the code beside the loop costs them more than it gives (32 columns, 100 K rows 69 and 67, 200 K
-// 91 and 92, a million 348 and 351, 2.5 M 1006 and 1019); with sixteen lanes the limit is the least length of a row taken apart.
+// Where rows differ much in length (the matrix has rows above kSpmmLongRow, which are not taken here), a row of more than
+// together_from() nonzeros is taken by 1/kAtOnce of a wavefront, its groups on neighbouring stretches of it: walked by one group,
+// four or eight rows of op(B) at a time, the longest of them outlast the launch.  Power-law rows, microseconds a call walked so and
+// now: 16 fp32 columns, 100 K rows 67 and 41, 400 K 137 and 115, a million 296 and 280; 12 fp64 columns, 100 K 62 and 51, a million
+// 405 and 393.  Eight lanes of fp32 get there faster, and the code beside the loop costs them more than it gives (32 columns, 100 K
+// rows 69 and 67, 200 K 91 and 92, a million 348 and 351, 2.5 M 1006 and 1019); with sixteen lanes the limit is the least length of
+// a row taken apart.
+//
+// A row far above the mean is one of few; rows of about the mean are most of them, and better off with a group each.  20 K rows of
+// 70, 140 and 256 nonzeros and one of 3000, 16 fp32 columns: walked 46, 100 and 135, limit 16 * LR 86, 118 and 141, now 43, 90 and
+// 128.  (Over 240 matrices of sizes, shares and lengths like these, the time against that of walked rows: a limit of four means
+// 0.89 and at worst 1.8, six 0.90 and 1.19, eight 0.90 and 1.19, each with one row at a time to a wavefront; six with four 0.88 and
+// 1.10.)
+constexpr uint64_t kTogetherMeans = 6;
+constexpr uint32_t kAtOnce = 4;
 template <int LR>
-constexpr idx_t kTogether = 16 * LR;
+idx_t together_from(idx_t m, idx_t nnz) {
+    return static_cast<idx_t>(std::max<uint64_t>(16 * LR, std::min<uint64_t>(kTogetherMeans * (static_cast<uint64_t>(nnz) / m + 1), kSpmmLongRow)));
+}
 template <typename T, int LR>
 constexpr bool kTakenTogether = LR == 4 || (LR == 8 && sizeof(T) == 8);
-static_assert(kTogether<8> < kSpmmLongCutLeast, "rows that are not taken apart");
-// The rows of more than kTogether<LR> among a wavefront's 64 from row0 on, of which lane i has the i-th, my_start to my_end; mine: it is
-// to be taken.  For whole wavefronts.
-template <typename T, int LR, int V>
-__device__ __forceinline__ void rows_together(bool mine, idx_t my_start, idx_t my_end, uint64_t row0, idx_t base,
-                                              const idx_t* __restrict__ col, const T* __restrict__ val, const char* __restrict__ B_bytes,
-                                              uint32_t lane_off, uint32_t ldb_bytes, T* __restrict__ C, int64_t ldc, bool c_row_major,
-                                              T alpha, T beta, const LaneColumns& own) {
-    const uint32_t wave_lane = threadIdx.x % kWave, lane = wave_lane % LR, group = wave_lane / LR;
-    for (unsigned long long together = __ballot(mine && my_end - my_start > kTogether<LR>); together != 0; together &= together - 1) {  // whole wavefront
-        const uint32_t r = __builtin_ctzll(together);
-        const idx_t begin = __builtin_amdgcn_readlane(my_start, r), end = __builtin_amdgcn_readlane(my_end, r);
-        T acc[V];
+// The rows of more than `least` and up to long_row nonzeros, by workgroup `block` of `blocks`.  A wavefront's 64 rows are 16 stretches
+// of four from all over the matrix: long rows that lie together go to many wavefronts.  100 K power-law rows sorted by their length,
+// 16 fp32 columns: walked 191, 64 adjacent rows to a wavefront 183, now 73; COO 79, 202 and 50.
+template <typename T, int LR, int V, bool RAGGED>
+__device__ __forceinline__ void rows_together(uint32_t block, uint32_t blocks, idx_t least, idx_t long_row, idx_t m, idx_t n, idx_t base,
+                                              const idx_t* __restrict__ row_ptr, const idx_t* __restrict__ col,
+                                              const T* __restrict__ val, const T* __restrict__ B, uint32_t ldb_bytes,
+                                              T* __restrict__ C, int64_t ldc, bool c_row_major, T alpha, T beta) {
+    constexpr uint32_t kNeighbours = 4;
+    constexpr int kLanes = kWave / kAtOnce;  // to a row
+    static_assert(kLanes % LR == 0);
+    const uint32_t wave_lane = threadIdx.x % kWave, lane = wave_lane % LR, part = wave_lane / kLanes, group = wave_lane % kLanes / LR;
+    const uint64_t waves = static_cast<uint64_t>(blocks) * (kBlock / kWave), wave = static_cast<uint64_t>(block) * (kBlock / kWave) + threadIdx.x / kWave;
+    const LaneColumns own = lane_columns<V, RAGGED>((static_cast<uint64_t>(blockIdx.y) * LR + lane) * V, n);
+    for (uint64_t row0 = 0; row0 < m; row0 += waves * kWave) {  // whole wavefront
+        const uint64_t mine = row0 + wave_lane / kNeighbours * (waves * kNeighbours) + wave * kNeighbours + wave_lane % kNeighbours;
+        const uint32_t my_row = static_cast<uint32_t>(min(mine, static_cast<uint64_t>(m) - 1));
+        const idx_t my_start = row_ptr[my_row] - base, my_end = row_ptr[my_row + 1] - base, length = my_end - my_start;
+        for (unsigned long long left = __ballot(mine < m && length > least && length <= long_row); left != 0;) {
+            // the kAtOnce next rows, one to each part of the wavefront
+            uint32_t r = kWave;
 #pragma unroll
-        for (int i = 0; i < V; ++i) acc[i] = T(0);
-        row_times_b<T, LR, V, false, true>(begin + group * LR, end, lane, base, col, val, B_bytes, lane_off, ldb_bytes, acc, kWave);
+            for (uint32_t k = 0; k < kAtOnce; ++k) {
+                if (part == k && left != 0) r = __builtin_ctzll(left);
+                left &= left - 1;
+            }
+            const bool have = r < kWave;
+            const uint32_t row = __shfl(my_row, r % kWave);  // (by all lanes: the one that has it may be of a part without a row)
+            const idx_t begin = __shfl(my_start, r % kWave), its_end = __shfl(my_end, r % kWave), end = have ? its_end : begin;
+            T acc[V];
 #pragma unroll
-        for (int i = 0; i < V; ++i) {
+            for (int i = 0; i < V; ++i) acc[i] = T(0);
+            row_times_b<T, LR, V, false, true>(begin + group * LR, end, lane, base, col, val, reinterpret_cast<const char*>(B),
+                                               static_cast<uint32_t>(own.first * sizeof(T)), ldb_bytes, acc, kLanes);
 #pragma unroll
-            for (int off = LR; off < kWave; off <<= 1) acc[i] += __shfl_xor(acc[i], off, kWave);
+            for (int i = 0; i < V; ++i) {
+#pragma unroll
+                for (int off = LR; off < kLanes; off <<= 1) acc[i] += __shfl_xor(acc[i], off, kWave);
+            }
+            if (group == 0 && have && own.any) store_c<T, V>(C, ldc, c_row_major, row, own.first, acc, alpha, beta, own.skip);
         }
-        if (group == 0 && own.any) store_c<T, V>(C, ldc, c_row_major, row0 + r, own.first, acc, alpha, beta, own.skip);
     }
+}
+// Workgroups of them, a whole number for every XCD, which leaves the others' order as it is.
+uint32_t together_blocks(idx_t m, uint32_t xcds) {
+    constexpr uint64_t kMost = 1024;
+    const uint64_t needed = std::min((static_cast<uint64_t>(m) + kBlock - 1) / kBlock, kMost);
+    return static_cast<uint32_t>((needed + xcds - 1) / xcds * xcds);
 }
 
 // op(B) row-major.  LR lanes per row of A, V adjacent columns per lane; blockIdx.y walks the
@@ -57,8 +92,8 @@ __device__ __forceinline__ void rows_together(bool mine, idx_t my_start, idx_t m
 // together into 102 registers instead of 59, four wavefronts (27-point stencil 128^3, 64 fp32 columns: 636 -> 707 us).
 // Not in fp64, where five or six wavefronts do better (16 columns 420 us, 439 with eight; 32 columns 657 and 677).
 //
-// TOGETHER: a call that does not know whether there are long rows (COO, CSC, a captured one) for a width whose longer rows are wavefronts'
-// where there are; the first `beside` workgroups take these, so that a row's sum is the same by every way to the product.  (As a launch of
+// TOGETHER: a call that does not know whether there are long rows (COO, CSC, a captured one) for a width whose longer rows are taken by
+// parts of wavefronts where there are; the first `beside` workgroups take these, so that a row's sum is the same by every way to the product.  (As a launch of
 // its own: COO, 1000 and 100 K rows of 16, 16 fp32 columns 21.4 and 37.9 us, 18.5 and 37.0 so; 100 K power-law rows 58 and 46.)
 template <typename T, int LR, int V, bool WIDE, bool RAGGED, bool TOGETHER>
 __global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 8 : 1) void spmm_rowb_kernel(idx_t m, idx_t n, idx_t base,
@@ -67,22 +102,15 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 8 : 1) void sp
                                                            const T* __restrict__ B, int64_t ldb, T* __restrict__ C,
                                                            int64_t ldc, bool c_row_major, T alpha, T beta,
                                                            idx_t long_row, const uint32_t* __restrict__ apart,
-                                                           uint32_t beside, uint32_t xcd_chunk, uint32_t xcds) {
+                                                           idx_t together, uint32_t beside, uint32_t xcd_chunk, uint32_t xcds) {
     typedef typename ByteOffset<WIDE>::type off_t;
     constexpr int kRowsPerBlock = kBlock / LR;
     const idx_t lane = threadIdx.x % LR;
     if constexpr (TOGETHER) {
         if (blockIdx.x < beside) {  // whole workgroup
-            if (*apart == 0) return;
-            const LaneColumns own = lane_columns<V, RAGGED>((static_cast<uint64_t>(blockIdx.y) * LR + lane) * V, n);
-            for (uint64_t row0 = (static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x) / kWave * kWave; row0 < m;
-                 row0 += static_cast<uint64_t>(beside) * kBlock) {  // whole wavefront
-                const uint64_t mine = row0 + threadIdx.x % kWave, at = min(mine, static_cast<uint64_t>(m) - 1);
-                const idx_t start = row_ptr[at] - base, end = row_ptr[at + 1] - base;
-                rows_together<T, LR, V>(mine < m && end - start <= long_row, start, end, row0, base, col, val,
-                                        reinterpret_cast<const char*>(B), static_cast<uint32_t>(own.first * sizeof(T)),
-                                        static_cast<uint32_t>(ldb * sizeof(T)), C, ldc, c_row_major, alpha, beta, own);
-            }
+            if (*apart != 0)
+                rows_together<T, LR, V, RAGGED>(blockIdx.x, beside, together, long_row, m, n, base, row_ptr, col, val, B,
+                                                static_cast<uint32_t>(ldb * sizeof(T)), C, ldc, c_row_major, alpha, beta);
             return;
         }
     }
@@ -97,7 +125,7 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 8 : 1) void sp
     const idx_t end = row_ptr[row + 1] - base;
     // long_row != 0: rows with more nonzeros are the work of the kernels in spmm_long.hip, C included, unless *apart is
     // zero (null: known not to be)
-    const idx_t longest = TOGETHER ? kTogether<LR> : long_row;
+    const idx_t longest = TOGETHER ? together : long_row;
     if (longest != 0 && end - start > longest && (apart == nullptr || *apart != 0)) return;  // whole lane groups
     T acc[V];
 #pragma unroll
@@ -122,14 +150,22 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 7 : 1) void sp
                                                                  const idx_t* __restrict__ col, const T* __restrict__ val,
                                                                  const T* __restrict__ B, int64_t ldb, T* __restrict__ C,
                                                                  int64_t ldc, bool c_row_major, T alpha, T beta,
-                                                                 idx_t long_row, const BoundsWork cut) {
+                                                                 idx_t long_row, idx_t together, uint32_t beside, const BoundsWork cut) {
     if (blockIdx.x < cut.blocks) {  // whole workgroup
         cut_pieces(cut, base, nnz, row_ptr, col);
         return;
     }
+    const uint32_t block = blockIdx.x - cut.blocks;
+    if constexpr (kTakenTogether<T, LR>) {
+        if (block < beside) {  // whole workgroup
+            rows_together<T, LR, V, RAGGED>(block, beside, together, long_row, m, n, base, row_ptr, col, val, B,
+                                            static_cast<uint32_t>(ldb * sizeof(T)), C, ldc, c_row_major, alpha, beta);
+            return;
+        }
+    }
     constexpr int kBatch = LR < 8 ? LR : 8;  // rows of op(B) in flight per lane
     const uint32_t wave_lane = threadIdx.x % kWave, lane = wave_lane % LR, group = wave_lane / LR;
-    const uint64_t row0 = (static_cast<uint64_t>(blockIdx.x - cut.blocks) * (kBlock / kWave) + threadIdx.x / kWave) * kTurnRows;
+    const uint64_t row0 = (static_cast<uint64_t>(block - beside) * (kBlock / kWave) + threadIdx.x / kWave) * kTurnRows;
     if (row0 >= m) return;  // whole wavefront
     const LaneColumns own = lane_columns<V, RAGGED>((static_cast<uint64_t>(blockIdx.y) * LR + lane) * V, n);
     const uint32_t lane_off = static_cast<uint32_t>(own.first * sizeof(T)), ldb_bytes = static_cast<uint32_t>(ldb * sizeof(T));
@@ -138,9 +174,7 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 4 && LR <= 16 ? 7 : 1) void sp
     const uint32_t my_row = static_cast<uint32_t>(min(row0 + wave_lane, static_cast<uint64_t>(m) - 1));
     const idx_t my_start = row_ptr[my_row] - base, my_end = row_ptr[my_row + 1] - base;
     const uint32_t length = my_end - my_start;
-    const bool mine = row0 + wave_lane < m && length <= long_row, live = mine && (!kTakenTogether<T, LR> || length <= kTogether<LR>);
-    if constexpr (kTakenTogether<T, LR>)
-        rows_together<T, LR, V>(mine, my_start, my_end, row0, base, col, val, B_bytes, lane_off, ldb_bytes, C, ldc, c_row_major, alpha, beta, own);
+    const bool live = row0 + wave_lane < m && length <= (beside != 0 ? together : long_row);
     const unsigned long long first = __ballot(live && length > 4 * LR), second = __ballot(live && length <= 4 * LR);
     auto below = [&](unsigned long long mask) {
         return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u));
@@ -919,19 +953,17 @@ void launch_rowb(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
     const T* val = static_cast<const T*>(a.val);
     const T* B = static_cast<const T*>(a.B);
     T* C = static_cast<T*>(a.C);
+    const idx_t from = a.nnz != 0 ? together_from<LR>(a.m, a.nnz) : 0;
     auto launch = [&](auto wide, auto ragged, auto together, uint32_t beside) {
         const dim3 all(grid.x + beside, grid.y);
         hipLaunchKernelGGL((spmm_rowb_kernel<T, LR, V, decltype(wide)::value, decltype(ragged)::value, decltype(together)::value>), all,
                            dim3(kBlock), 0, stream, a.m, a.n, a.base, a.row_ptr, a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta,
-                           a.long_row, a.long_apart, beside, chunk, xcds);
+                           a.long_row, a.long_apart, from, beside, chunk, xcds);
     };
     auto launch_offsets = [&](auto ragged) {
         if constexpr (kTakenTogether<T, LR>) {
-            if (takes_rows_in_turns<T, LR>(a, false)) {
-                // (a whole number for every XCD, which leaves the others' order as it is)
-                constexpr uint64_t kMost = 1024;
-                const uint64_t needed = min((static_cast<uint64_t>(a.m) + kBlock - 1) / kBlock, kMost);
-                launch(std::false_type{}, ragged, std::true_type{}, static_cast<uint32_t>((needed + xcds - 1) / xcds * xcds));
+            if (takes_rows_in_turns<T, LR>(a, false) && from < a.long_row) {
+                launch(std::false_type{}, ragged, std::true_type{}, together_blocks(a.m, xcds));
                 return;
             }
         }
@@ -942,11 +974,12 @@ void launch_rowb(hipStream_t stream, const SpmmArgs& a, T alpha, T beta) {
         if (takes_rows_in_turns<T, LR>(a, true)) {
             constexpr uint32_t kRowsPerBlock = kBlock / kWave * kTurnRows;
             const BoundsWork cut = spmm_long_bounds(a, sizeof(T));
-            const dim3 turns_grid(cut.blocks + (a.m + kRowsPerBlock - 1) / kRowsPerBlock, static_cast<uint32_t>(panels));
+            const uint32_t beside = kTakenTogether<T, LR> && from < a.long_row ? together_blocks(a.m, xcds) : 0;
+            const dim3 turns_grid(cut.blocks + beside + (a.m + kRowsPerBlock - 1) / kRowsPerBlock, static_cast<uint32_t>(panels));
             auto turns = [&](auto ragged) {
                 hipLaunchKernelGGL((spmm_rowb_turns_kernel<T, LR, V, decltype(ragged)::value>), turns_grid, dim3(kBlock), 0, stream,
                                    a.m, a.n, a.nnz, a.base, a.row_ptr, a.col, val, B, a.ldb, C, a.ldc, a.c_row_major, alpha, beta,
-                                   a.long_row, cut);
+                                   a.long_row, from, beside, cut);
             };
             if (a.n % V != 0) turns(std::true_type{});
             else turns(std::false_type{});
