@@ -59,15 +59,22 @@ __device__ __forceinline__ uint32_t tile_of_block(uint32_t tiles, uint32_t xcds)
     return (blockIdx.x % xcds) * per_xcd + blockIdx.x / xcds;
 }
 
-// The order of buckets over the workgroups: XCDs take kNeighbours in turn.  (A contiguous range of them each, as for tiles, leaves
-// XCDs without work where the number of keys is no power of two and the last buckets are empty, or where the keys are not evenly
-// spread: 22 M nonzeros in 1.2 M columns, a call of csr2csc 325 us, and 269 so; 11.5 M in 700 K 168 and 151; index sort of 10 M
-// triples in 2^20 rows 280 and 216.  Neighbours meet on the lines at the ends of their runs, for which 2, 4, 8 and 16 of them do:
-// 270, 269, 269, 269, and 60, 59, 59, 59 for 4 M nonzeros in 300 K columns, 68 before.)
+// The order of buckets over the workgroups: XCDs take kNeighbours in turn or, if `range` is not 0, that many each.  (A contiguous
+// range of them each, as for tiles, leaves XCDs without work where the number of keys is no power of two and the last buckets are
+// empty, or where the keys are not evenly spread: 22 M nonzeros in 1.2 M columns, a call of csr2csc 325 us, and 269 in turn; 11.5 M
+// in 700 K 168 and 151; index sort of 10 M triples in 2^20 rows 280 and 216.  Neighbours meet on the lines at the ends of their
+// runs, for which 2, 4, 8 and 16 of them do: 270, 269, 269, 269, and 60, 59, 59, 59 for 4 M nonzeros in 300 K columns, 68 before.)
 constexpr uint32_t kNeighbours = 8;
-__device__ __forceinline__ uint32_t bucket_of_block(uint32_t xcds) {
-    const uint32_t per_round = xcds * kNeighbours, place = blockIdx.x % per_round;
-    return blockIdx.x - place + place % xcds * kNeighbours + place / xcds;
+// Few entries stay in the L2s from one step to the next.  A range of the buckets that have keys then finds in its own XCD's L2
+// what the tiles of that part of a banded matrix left there: csr2csc of a million nonzeros in 65536 columns 29.4 us, in turn
+// 31.9 (fp64 31.4 and 35.1), in 80 K columns 29.5 and 31.8 (fp64 33.3 and 35.6), of 1.4 M in 200 K 36.2 and 38.9.  Nonzeros from
+// everywhere lose up to 3 % by it (33.5 and 32.4 us in 65536 columns).  2.4 M in 2^18 columns 46.9 and 47.6 (fp64 55.1 and 54.7;
+// power-law columns 105 and 102), 3.5 M in 2^17 48.1 and 47.7.
+constexpr uint32_t kEntriesThatStay = 1u << 21;
+__device__ __forceinline__ uint32_t bucket_of_block(uint32_t range, uint32_t xcds) {
+    const uint32_t turn = blockIdx.x / xcds, xcd = blockIdx.x - turn * xcds;
+    if (range != 0) return turn < range ? xcd * range + turn : blockIdx.x;
+    return turn / kNeighbours * kNeighbours * xcds + xcd * kNeighbours + turn % kNeighbours;
 }
 
 enum EntryKind : int { kPlain = 0, kCsr = 1, kProducts = 2 };
@@ -1003,11 +1010,11 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 || (MANY && !packed_entries
                                                                                       const uint32_t* __restrict__ aux_in,
                                                                                       const void* __restrict__ vals_in,
                                                                                       SortOutput out, uint32_t buckets,
-                                                                                      uint32_t xcds) {
+                                                                                      uint32_t range, uint32_t xcds) {
     constexpr int kUsualItems = kBucketItems * 2 / 3, kFewItems = kBucketItems / 3;
     constexpr int kMoreItems = MANY && packed_entries<Key>() ? kBucketItems * 3 / 4 : kUsualItems;
     __shared__ BucketLds s;
-    const uint32_t sub = bucket_of_block(xcds);
+    const uint32_t sub = bucket_of_block(range, xcds);
     if (sub >= buckets) return;  // whole workgroup
     const uint32_t tid = threadIdx.x;
     const uint32_t first = t.sub_first[sub], count = t.sub_first[sub + 1] - first;
@@ -1568,12 +1575,14 @@ void launch_sort(hipStream_t stream, EntrySource in, const SortShape& s, const S
         vals = w + l.vals2;
     }
     const uint32_t buckets = 1u << (s.d1 + s.d2);
-    const uint32_t per_round = xcds * kNeighbours;
+    // (what a contiguous range is of: the buckets that have keys, which the sorts by two keys don't tell)
+    const uint32_t used = ((out.key_count - 1) >> s.d3) + 1, range = !kMany && in.count <= kEntriesThatStay ? (used + xcds - 1) / xcds : 0;
+    const uint32_t per_round = xcds * (range != 0 ? range : kNeighbours);
     const dim3 grid((buckets + per_round - 1) / per_round * per_round);
     auto sort = [&](auto key) {
         typedef decltype(key) Key;
         hipLaunchKernelGGL((bucket_sort_kernel<VB, Key, kMany>), grid, dim3(kBucketThreads), 0, stream, t,
-                           static_cast<const Key*>(keys), aux, vals, out, buckets, xcds);
+                           static_cast<const Key*>(keys), aux, vals, out, buckets, range, xcds);
         if (in.count > kBucketRoom)  // else no bucket is larger than that
             hipLaunchKernelGGL((oversize_kernel<VB, Key, kMany>), dim3(kOversizeGrid), dim3(kBucketThreads), 0, stream, t,
                                static_cast<const Key*>(keys), aux, vals, out);
