@@ -17,8 +17,8 @@ constexpr int kBlock = 256;
 // One workgroup per bucket of neighbouring columns: the sums of the bucket's columns live in LDS as
 // doubles (fp32 products are widened: ds_add_f64 runs at four times the rate of ds_add_f32 on this chip), and every
 // column of the bucket is written at the end, with or without products.
-// BUCKETS: rows of the table of runs.  With 1024 of them (more than 4.7 M columns) a run is 8 entries instead of 32 and a
-// third of a tile's places may be padding, but a sort by the columns takes three times as long.
+// BUCKETS: rows of the table of runs.  With 1024 of them (more than 4.7 M columns) a run is 8 entries instead of 32 and
+// 3072 of a tile's 11264 places may be padding (tiles of 4096 entries: 3072 of 7168), but a sort by the columns takes three times as long.
 constexpr int kBucketBlock = 1024;
 
 // Which part of which bucket a workgroup takes.  A bucket whose pairs number more than twice `share` (the mean of
