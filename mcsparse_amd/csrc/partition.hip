@@ -1057,6 +1057,11 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 || (MANY && !packed_entries
 // spread is not known on the host, where the choice is made, and evenly spread ones gain as much (10 M: 481 and 330 us);
 // so does csr2csc under any spread.
 constexpr uint32_t kOversizeGrid = 512;
+// Up to that many workgroups may look more often than 512: waits are what a phase of few chunks takes.  By Zipf's law, with the long
+// waits and with the short ones: csr2csc of 20 K nonzeros 48.4 and 46.1 us, 160 K 55.8 and 53.6, 1.05 M 68.5 and 67.2; index sorts of
+// 10 K triples 96.6 and 89, 300 K 132 and 124, a million 149 and 145.  Of more chunks: csr2csc of 3.5 M 101 and 103, index sort of
+// 4.8 M 434 and 450.  (With 128 for 256 csr2csc of 1.05 M 69, of 1.4 M 77.6 for 74.5; with 384 as with 256.)
+constexpr uint32_t kFewOversizeChunks = 256;
 
 struct OversizeChunk {
     uint32_t listed_at, bucket, first, entries;  // first: place of the bucket's first entry in the output
@@ -1161,8 +1166,10 @@ __global__ __launch_bounds__(kBucketThreads, VB == 8 ? 2 : 4) void oversize_kern
         const word_t* between_vals = static_cast<const word_t*>(t.oversize_vals[(p + 1) % 2]);
         if (tid == 0) {
             for (uint32_t idle = 0; phase != 0 && load_shared(&t.oversize->done[phase - 1]) < all_chunks; ++idle) {
-                // (hundreds of workgroups may be waiting: some 3 us, then 6)
-                for (uint32_t n = 0; n < (1u << min(idle, 1u)); ++n) __builtin_amdgcn_s_sleep(100);
+                if (all_chunks <= kFewOversizeChunks)
+                    for (uint32_t n = 0; n < (1u << min(idle, 2u)); ++n) __builtin_amdgcn_s_sleep(32);  // some 1, 2, 4 us
+                else
+                    for (uint32_t n = 0; n < (1u << min(idle, 1u)); ++n) __builtin_amdgcn_s_sleep(100);  // some 3, 6 us
             }
             s_ticket = take_chunk(t, phase);
         }
